@@ -1,0 +1,788 @@
+"""The work that a user of this framework has it do, as cases that can be timed and compared: generations and prompts of the flat families (one stream, several
+rows of a running batch) and engine steps of the layered designs (ragged prompts, single decoded tokens), in the storage types that they are served in.
+
+  listed()                  the cases, each with what it stands for beside it
+  draw(rng)                 one more case of the same ranges
+  prepare(case, seed)       model (random weights), prompts and the tokens that are fed: what a program holds before the call
+  run(state)                one pass through the public entry points (tinygpt_amd.ffi.Model, tinygpt_amd.serving.SlotEngine)
+  exact(case, seed)         the same outputs in 64-bit torch arithmetic, whole sequences at a time, written from the designs' equations
+  work(case), tolerance(case)
+
+A pass is one generation or one serving session from an empty cache: the prompts in, then `steps` further tokens.  The layered cases feed given tokens (a step
+of SlotEngine that wants logits, the form a trace replay and a scoring client use) except the `greedy` ones, which run the library's own decode loop.  Greedy
+tokens are kept apart by a few loud rows in an untied output head, so that rounding does not choose them.
+"""
+import math
+import zlib
+
+import numpy as np
+import torch
+
+from tinygpt_amd.desc import LayerDesc, ModelDesc, StackDesc, known_desc
+from tinygpt_amd.ffi import GREEDY, Model, SamplerCfg
+from tinygpt_amd.serving import SlotEngine
+
+VOCAB = 32000                     # of the layered models
+LOUD, LOUD_SCALE = 4, 64.0        # rows of an untied head that win every greedy choice, and as many mirrored ones
+SAMPLED = dict(temperature=0.8, top_p=0.9)
+TORCH = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}
+
+
+def listed():
+    return [
+        # the first thing anybody runs: the smallest model in 32 bits, a short prompt, 32 greedy tokens
+        dict(name="gpt2-chat-fp32", model="gpt2", dtype="fp32", seqs=1, prompt=24, ragged=False, steps=32, mode="greedy"),
+        # a chat turn of a small model with the command line's default sampler
+        dict(name="qwen-chat-sampled", model="qwen2.5-0.5b", dtype="bf16", seqs=1, prompt=133, ragged=False, steps=48, mode="sampled"),
+        # reading one short prompt (classification, a time to first token): no decoding at all
+        dict(name="qwen3-prompt", model="qwen3-0.6b", dtype="bf16", seqs=1, prompt=509, ragged=False, steps=0, mode="greedy"),
+        # the headline workload: a 2048-token prompt, then one stream decoded
+        dict(name="llama-long-prompt", model="llama-3.2-1b", dtype="bf16", seqs=1, prompt=2048, ragged=False, steps=64, mode="greedy"),
+        # a running batch whose rows were refilled one by one with prompts of different lengths
+        dict(name="llama-rows-fp16", model="llama-3.2-1b", dtype="fp16", seqs=16, prompt=300, ragged=True, steps=24, mode="greedy"),
+        # the layered designs: ragged prompts of a few requests joining in one step, then tokens of all of them
+        dict(name="zakusun-serve", model="zakusun", width=1024, layers=8, dtype="bf16", seqs=4, prompt=1100, ragged=True, steps=12, mode="forced"),
+        # one long prompt of a wide mixture-of-experts design
+        dict(name="modepel-prompt", model="modepel", width=2048, layers=4, dtype="bf16", seqs=1, prompt=2048, ragged=False, steps=6, mode="forced"),
+        # an interactive turn: a short question, one stream of tokens from the library's decode loop (launches and latency)
+        dict(name="vitudra-chat", model="vitudra", width=1024, layers=8, dtype="bf16", seqs=1, prompt=47, ragged=False, steps=48, mode="greedy"),
+        # one long prompt of the same design at the larger width
+        dict(name="vitudra-prompt", model="vitudra", width=2048, layers=8, dtype="bf16", seqs=1, prompt=2048, ragged=False, steps=4, mode="greedy"),
+        # half storage: two medium requests
+        dict(name="zaluvik-serve-fp16", model="zaluvik", width=1024, layers=6, dtype="fp16", seqs=2, prompt=1500, ragged=True, steps=8, mode="forced"),
+        # throughput: several documents read in one step
+        dict(name="nusovik-documents", model="nusovik", width=2048, layers=8, dtype="bf16", seqs=8, prompt=2048, ragged=True, steps=4, mode="greedy"),
+        # many short requests decoding together
+        dict(name="keronex-batch", model="keronex", width=1024, layers=8, dtype="bf16", seqs=16, prompt=160, ragged=True, steps=24, mode="forced"),
+    ]
+
+
+def draw(rng):
+    def size(lo, hi):
+        return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+    model = rng.choice(["gpt2", "qwen2.5-0.5b", "qwen3-0.6b", "llama-3.2-1b", "zakusun", "modepel", "vitudra", "vitudra", "zaluvik", "nusovik", "keronex"])
+    if model in FLAT:
+        seqs = rng.choice([1, 1, 1, 2, 5, 16]) if model != "gpt2" else rng.choice([1, 3])
+        c = dict(model=model, dtype="fp32" if model == "gpt2" else rng.choice(["bf16", "bf16", "fp16"]), seqs=seqs, prompt=size(12, 700 if model == "gpt2" else 2048 if seqs == 1 else 400),
+                 ragged=seqs > 1, steps=rng.choice([0, size(4, 48)]))
+        c["mode"] = "sampled" if model == "qwen2.5-0.5b" and c["steps"] and seqs == 1 else "greedy"
+        return c
+    width = rng.choice([1024, 1024, 2048])
+    layers = 6 if model == "zaluvik" else rng.randint(4, 8) if width == 1024 else rng.randint(3, 4)
+    seqs = rng.choice([1, 1, 2, 4, 7, 16])
+    return dict(model=model, width=width, layers=layers, dtype=rng.choice(["bf16", "bf16", "fp16"]), seqs=seqs, prompt=size(20, max(200, 4096 // seqs if seqs > 1 else 2048)),
+                ragged=seqs > 1, steps=size(2, 24), mode="greedy" if model in ("vitudra", "nusovik") else "forced")
+
+
+FLAT = ("gpt2", "qwen2.5-0.5b", "qwen3-0.6b", "llama-3.2-1b")
+
+
+def lengths(case):
+    """the prompts' lengths: spread between a third and the whole of `prompt`, odd ones among them; from the sizes alone, so that work() knows them"""
+    n, p = case["seqs"], case["prompt"]
+    if not case["ragged"]:
+        return [p] * n
+    return [max(3, p - (2 * p // 3) * i // max(1, n - 1) - (i % 3 if i else 0)) for i in range(n)]
+
+
+# ---- the models ----------------------------------------------------------------------------------------------------------------------------
+def flat_desc(case):
+    d = known_desc(case["model"], case["dtype"], case["seqs"])
+    d.max_ctx = min(d.max_ctx, 4096)
+    if case["model"] == "llama-3.2-1b":      # greedy tokens that rounding cannot choose: an untied head with loud rows
+        d.tied = False
+    return d
+
+
+def stack_layers(case):
+    W, n = case["width"], case["layers"]
+    experts, top, ff = (16, 4, 2048) if W >= 2048 else (8, 2, 1536)
+    head = dict(heads=W // 128, kv_heads=max(1, W // 512), dim=128, vdim=128)
+    out = []
+    for i in range(n):
+        m = case["model"]
+        if m == "zakusun":
+            out.append(LayerDesc(mixer="latent_attention", heads=W // 128, dim=128, vdim=128, kv_rank=W // 4, scale=128 ** -0.5, mlp="moe", experts=experts, top=top, ff=ff, limit=7.0))
+            continue
+        if m == "modepel":
+            if i % 3 == 0:
+                l = LayerDesc(mixer="mlstm", heads=W // 256, dim=128, vdim=256, gate_cap=15.0)
+            else:
+                l = LayerDesc(mixer="attention", rot_dims=64, rot_base=500000.0, scale=128 ** -0.5, v_mix=True, **head)
+            if i == 0:
+                l.mlp, l.ff = "dense", top * ff
+            else:
+                l.mlp, l.experts, l.identity, l.top, l.ff, l.groups, l.groups_keep, l.router_scale, l.shared_ff = "moe", experts, 4, top, ff, 4, 2, 1.5, ff
+        elif m == "vitudra":
+            if i % 3 == 0:
+                l = LayerDesc(mixer="wkv", heads=W // 64, kv_heads=W // 64, dim=64, vdim=64, decay_rank=64)
+            elif i % 3 == 1:
+                l = LayerDesc(mixer="parallel", scale=128 ** -0.5, rot_dims=32, rot_base=10000.0, rot_pairs=True, rot_factor=4.0, softcap=30.0, mask="chunk", mask_size=1024,
+                              d_heads=W // 128, d_kv_heads=max(1, W // 256), d_dim=128, d_vdim=128, conv_taps=4, left_scale=0.7, right_scale=1.1, **head)
+            else:
+                l = LayerDesc(mixer="attention", scale=128 ** -0.5, mask="window", mask_size=1024, dist_bias=True, q_temp_coef=0.2, q_temp_every=128,
+                              kv_from=i - 3 if i % 6 == 5 else None, **head)
+            l.mlp, l.ff = "dense", top * ff
+        elif m == "zaluvik":
+            if i in (2, 4):
+                l = LayerDesc(mixer="latent_attention", heads=W // 128, dim=128, vdim=128, kv_rank=W // 4 - 64, rot_dim=64, rot_dims=64, rot_base=500000.0, scale=192 ** -0.5,
+                              mask="window", mask_size=1024, gate_kind="head")
+            else:
+                l = LayerDesc(mixer="attention", scale=0.09, mask="window", mask_size=1024, qk_norm=True, score_fn="sigmoid", head_mix=True, gate_kind="channel", **head)
+            if i % 2 == 0:
+                l.mlp, l.ff, l.ff_act = "dense", top * ff, "gelu"
+            else:
+                l.mlp, l.experts, l.top, l.ff, l.groups, l.groups_keep, l.shared_ff = "moe", experts, top, ff, 4, 2, ff
+                l.router_fn, l.group_score, l.router_norm = "sigmoid", "top2", True
+        elif m == "nusovik":
+            if i % 2 == 0:
+                l = LayerDesc(mixer="mamba1", inner=2 * W, d_dim=16, dt_rank=W // 16, conv_taps=4)
+            else:
+                l = LayerDesc(mixer="parallel", scale=128 ** -0.5, mask="chunk", mask_size=1024, qk_norm="weighted", v_is_k=True, head_sink=True, gate_kind="head", bias_max=1024,
+                              bias_buckets=32, right_kind="ssd", d_heads=2 * W // 64, d_kv_heads=max(1, W // 1024), d_dim=128, d_vdim=64, conv_taps=4, part_norms=max(1, W // 1024),
+                              left_scale=0.7, right_scale=0.9, mlp="dense", ff=top * ff, ff_act="relu2", **head)
+        else:
+            if i % 3 == 0:
+                l = LayerDesc(mixer="channel_delta", heads=W // 128, kv_heads=max(1, W // 256), dim=128, vdim=128, conv_taps=4, decay_rank=128, gate_rank=128)
+            elif i % 3 == 1:
+                H = W // 256
+                l = LayerDesc(mixer="retention", heads=H, kv_heads=H, dim=128, vdim=256, rot_dims=128, rot_base=10000.0, decays=tuple(1.0 - 2.0 ** (-5 - h % 8) for h in range(H)))
+            else:
+                l = LayerDesc(mixer="attention", heads=W // 128, kv_heads=max(1, W // 512), dim=64, vdim=128, maps=2, diff=0.4, scale=64 ** -0.5, rot_dims=64, rot_base=500000.0)
+            if i == 0:
+                l.mlp, l.ff, l.ff_act = "dense", top * ff, "gelu_tanh_gated"
+            else:
+                l.mlp, l.experts, l.top, l.ff, l.shared_ff, l.router_fn, l.router_in, l.expert_act = "moe", experts, top, ff, ff, "sigmoid", True, "relu2"
+            if i == 7:
+                l.weights_of = 1
+        out.append(l)
+    return out
+
+
+def stack_desc(case):
+    ctx = max(lengths(case)) + case["steps"] + 8
+    more = {"zakusun": dict(norm_groups=2, norm_eps=1e-6, canon_taps=4), "modepel": {}, "vitudra": dict(residual_mult=0.5), "nusovik": dict(embed_scale=2.0),
+            "zaluvik": dict(residual_mult=0.5, embed_scale=3.0, loop_start=1, loop_stop=3, loop_times=2),
+            "keronex": dict(embed_scale=2.0, streams=4, bigram_buckets=4093, bigram_before=31, bigram_cur=7)}[case["model"]]
+    more.setdefault("norm_eps", 1e-5)
+    pages = sum(-(-(n + case["steps"] + 1) // 64) for n in lengths(case))
+    return StackDesc(family=case["model"], width=case["width"], vocab=VOCAB, layers=stack_layers(case), compute_dtype=case["dtype"], max_seqs=case["seqs"], max_ctx=ctx,
+                     budget_tokens=64 * pages, name=case["model"], **more)
+
+
+# how a tensor that is no projection is spread: (leaf or name suffix, kind, a, b); projections are normal with deviation 1 / sqrt(inputs)
+SPREAD = [("mix.sink", "normal", 0, 1), (".dwa", "mean", 0.2, 0), (".canon1", "normal", 0, 0.4), (".canon2", "normal", 0, 0.4), (".router.b", "normal", 0, 1), (".router", "proj", 3, 0),
+          ("norm1b", "uniform", 0.3, 0.8), ("norm2b", "uniform", 0.3, 0.8), (".vmix", "uniform", 0.2, 0.6), (".act", "uniform", -1, 1), (".correction", "uniform", -0.02, 0.02),
+          ("mix.f.b", "uniform", 1, 4), ("mix.i.b", "uniform", -2, 1), (".conv", "normal", 0, 0.6), (".mix.u", "normal", 0, 0.5), (".w2", "proj", 3, 0), (".w0", "uniform", -3, 0.3),
+          (".A_log", "uniform", -2.5, 0.3), (".dt_bias", "uniform", -2, 0.5), ("dt.b", "uniform", -2, 0.5), (".talk", "eye", 0.4, 0), (".pb", "uniform", -2, 1), (".rel", "normal", 0, 1),
+          (".sink", "uniform", -1, 2), (".D", "uniform", 0.3, 1.5), (".in", "uniform", 0.1, 0.4), (".out", "uniform", 0.5, 1.5), ("hc1.mix", "eye", 0.15, 0), ("hc2.mix", "eye", 0.15, 0),
+          ("lq1", "normal", 0, 0.3), ("lq2", "normal", 0, 0.3), ("lk1", "normal", 0, 0.3), ("lk2", "normal", 0, 0.3), (".b", "normal", 0, 0.2), (".bias", "normal", 0, 0.1)]
+
+
+def weights(case, desc, seed):
+    """(name, tensor in the storage type on the GPU) of every tensor of the checkpoint, from the seed alone"""
+    dt, offset = TORCH[case["dtype"]], case["model"] in ("vitudra", "keronex")
+    for name, shape in desc.tensor_shapes().items():
+        gen = torch.Generator("cuda").manual_seed((seed * 1000003 + zlib.crc32(name.encode())) % (1 << 62))
+        normal = lambda: torch.randn(shape, generator=gen, device="cuda")              # noqa: E731
+        uniform = lambda a, b: torch.rand(shape, generator=gen, device="cuda") * (b - a) + a      # noqa: E731
+        leaf = name.split(".")[-1]
+        rule = next((r for r in SPREAD if name.endswith(r[0])), None)
+        if name in ("embed", "bigram") or "wte" in name or "wpe" in name or "embed_tokens" in name:
+            v = normal() * (1.0 if name in ("embed", "bigram") and case["model"] not in ("zakusun", "zaluvik") else 0.5)
+        elif leaf in ("in",) and len(shape) == 2:                                        # projections of that name, not the streams' weights
+            v = normal() / math.sqrt(shape[-1] if name != "loop.in" else shape[-1] / 2)
+        elif ".mu." in name:
+            v = uniform(0, 1)
+        elif rule is not None and not (len(shape) == 2 and leaf in ("b", "norm")):
+            _, kind, a, b = rule
+            v = (normal() * b + a if kind == "normal" else uniform(a, b) if kind == "uniform" else normal() * a / math.sqrt(shape[-1]) if kind == "proj"
+                 else torch.eye(shape[0], device="cuda") + normal() * a if kind == "eye" else normal() * a + 1.0 / shape[0])
+        elif "norm" in leaf or "norm" in name.split(".")[-2:][0] or ".ln_" in name or name.startswith("ln_"):
+            v = uniform(-0.3, 0.3) if offset and (leaf == "norm1" or leaf == "norm2" or name == "final.norm") else uniform(0.7, 1.3)
+        elif len(shape) == 2:
+            fan = shape[0] if case["model"] == "gpt2" else shape[-1]                     # that family stores its projections inputs first
+            v = normal() / math.sqrt(fan)
+        else:
+            v = normal() * 0.3
+        v = v.to(dt)
+        if name in ("head", "lm_head.weight"):
+            rows = loud_rows(seed, shape[0])
+            v[rows[:LOUD]] *= LOUD_SCALE
+            v[rows[LOUD:]] = -v[rows[:LOUD]]
+        yield name, v
+
+
+def loud_rows(seed, vocab):
+    return torch.from_numpy(np.random.default_rng(seed + 77).choice(vocab, 2 * LOUD, replace=False)).cuda()
+
+
+def as_numpy(t):
+    t = t.cpu()
+    return t.view(torch.int16).numpy().view(np.uint16) if t.dtype == torch.bfloat16 else t.numpy()
+
+
+def tokens_of(case, vocab, seed):
+    """(prompts, tokens fed after them [steps][seqs])"""
+    rng = np.random.default_rng(seed)
+    prompts = [rng.integers(0, vocab, n, dtype=np.int64) for n in lengths(case)]
+    return prompts, rng.integers(0, vocab, (case["steps"], case["seqs"]), dtype=np.int64)
+
+
+# ---- one pass ------------------------------------------------------------------------------------------------------------------------------
+def prepare(case, seed):
+    if case["model"] in FLAT:
+        desc = flat_desc(case)
+        model = Model(desc)
+        for name, t in weights(case, desc, seed):
+            model.upload(name, as_numpy(t))
+        model.finalize()
+        engine = None
+    else:
+        desc = stack_desc(case)
+        engine = SlotEngine(desc=desc, tensors={n: as_numpy(t) for n, t in weights(case, desc, seed)})
+        model = engine.model
+    prompts, fed = tokens_of(case, desc.vocab, seed)
+    return dict(case=case, model=model, engine=engine, prompts=prompts, fed=fed, cfg=SamplerCfg(**SAMPLED) if case["mode"] == "sampled" else GREEDY)
+
+
+def run(s):
+    m, engine, case, prompts = s["model"], s["engine"], s["case"], s["prompts"]
+    n = len(prompts)
+    if engine is None:
+        m.reset_cache()
+        if n == 1:
+            m.forward(prompts[0])
+        else:
+            for i, p in enumerate(prompts):
+                m.forward_row(i, p)
+        first = m.logits(rounded=False)
+        if not case["steps"]:
+            return {"first": first}
+        m.sample(s["cfg"], seed=11)
+        toks = m.decode(case["steps"], s["cfg"], seed=11)
+        return {"first": first, "tokens": toks, "last": m.logits(rounded=False)}
+    end = [0]
+    entries = []
+    for i, p in enumerate(prompts):
+        end.append(end[-1] + len(p))
+        entries.append((i, p, [len(p) - 1]))
+    first = engine.step(entries)
+    if case["mode"] == "forced":
+        out = {"first": first}
+        for t, row in enumerate(s["fed"]):
+            out["step%02d" % t] = engine.step([(i, row[i:i + 1], [0]) for i in range(n)])
+    else:
+        m.sample(GREEDY)
+        toks = m.decode(case["steps"], GREEDY)
+        out = {"first": first, "tokens": toks, "last": m.logits(rounded=False)}
+    for i in range(n):
+        engine.release(i)
+    return out
+
+
+# ---- the same in 64 bits -------------------------------------------------------------------------------------------------------------------
+def rms(x, eps):
+    return x / torch.sqrt((x * x).mean(-1, keepdim=True) + eps)
+
+
+def layer_norm(x, w, b, eps):
+    x = x - x.mean(-1, keepdim=True)
+    return x / torch.sqrt((x * x).mean(-1, keepdim=True) + eps) * w + b
+
+
+def silu(z):
+    return z * torch.sigmoid(z)
+
+
+def gelu_tanh(z):
+    return 0.5 * z * (1 + torch.tanh(math.sqrt(2 / math.pi) * (z + 0.044715 * z ** 3)))
+
+
+def angles(T, dims, base, factor=1.0):
+    f = base ** (-2.0 * torch.arange(dims // 2, dtype=torch.float64, device="cuda") / dims) / factor
+    return torch.arange(T, dtype=torch.float64, device="cuda")[:, None] * f
+
+
+def turn(x, a, dims, pairs=False):
+    """x [T][heads][D]: its first `dims` channels turned by the angles a [T][dims / 2], channel i with i + dims / 2 (pairs: 2i with 2i + 1)"""
+    c, s = torch.cos(a)[:, None], torch.sin(a)[:, None]
+    out = x.clone()
+    u, v = (x[..., 0:dims:2], x[..., 1:dims:2]) if pairs else (x[..., :dims // 2], x[..., dims // 2:dims])
+    if pairs:
+        out[..., 0:dims:2], out[..., 1:dims:2] = u * c - v * s, v * c + u * s
+    else:
+        out[..., :dims // 2], out[..., dims // 2:dims] = u * c - v * s, v * c + u * s
+    return out
+
+
+def seen(T, kind, size):
+    i = torch.arange(T, device="cuda")
+    d = i[:, None] - i[None]
+    ok = d >= 0
+    return ok & (d < size) if kind == "window" else ok & (i[:, None] // size == i[None] // size) if kind == "chunk" else ok
+
+
+def attend(q, k, v, ok, scale, sink=None, softcap=0.0, bias=None):
+    """q [T][H][D], k [T][G][D], v [T][G][E]; bias(h) is added to head h's scores, sink[h] is one more score without a value"""
+    H, G = q.shape[1], k.shape[1]
+    out = []
+    for h in range(H):
+        g = h // (H // G)
+        z = q[:, h] @ k[:, g].T * scale
+        if softcap:
+            z = softcap * torch.tanh(z / softcap)
+        if bias is not None:
+            z = z + bias(h)
+        z = z.masked_fill(~ok, -math.inf)
+        top = z.amax(1, keepdim=True)
+        if sink is not None:
+            top = torch.clamp(top, min=float(sink[h]))
+        p = torch.exp(z - top)
+        den = p.sum(1, keepdim=True) + (torch.exp(float(sink[h]) - top) if sink is not None else 0)
+        out.append(p @ v[:, g] / den)
+    return torch.stack(out, 1)
+
+
+def conv(x, w, b=None):
+    """causal depth-wise filter over the tokens, the last tap on the current one"""
+    taps = w.shape[1]
+    out = torch.zeros_like(x) if b is None else b.expand_as(x).clone()
+    for j in range(taps):
+        back = taps - 1 - j
+        out[back:] += x[:len(x) - back] * w[:, j] if back < len(x) else 0
+    return out
+
+
+def by_expert(h, sel, wts, expert):
+    """sum over a token's chosen experts; expert(e, rows, weights)"""
+    out = torch.zeros_like(h)
+    for e in torch.unique(sel).tolist():
+        t, j = (sel == e).nonzero(as_tuple=True)
+        out.index_add_(0, t, expert(e, h[t], wts[t, j][:, None]))
+    return out
+
+
+def grouped_choice(score, top, groups, keep, best_two):
+    T, n = score.shape
+    g = score.view(T, groups, n // groups)
+    gs = g.topk(2, -1).values.sum(-1) if best_two else g.amax(-1)
+    ok = torch.zeros(T, groups, dtype=torch.bool, device="cuda").scatter_(1, gs.topk(keep, -1).indices, True)
+    return score.masked_fill(~ok.repeat_interleave(n // groups, 1), -math.inf).topk(top, -1).indices
+
+
+class Exact:
+    """one model in 64 bits; cached keys, values and latents are rounded to the storage type as every implementation stores them"""
+
+    def __init__(self, case, seed):
+        self.case = case
+        self.desc = flat_desc(case) if case["model"] in FLAT else stack_desc(case)
+        self.w = dict(weights(case, self.desc, seed))
+        self.store = TORCH[case["dtype"]]
+
+    def __getitem__(self, name):
+        return self.w[name].double()
+
+    def has(self, name):
+        return name in self.w
+
+    def kept(self, x):
+        return x.to(self.store).double()
+
+    def lin(self, x, name):
+        return x @ self[name].T
+
+    def logits(self, ids, rows=slice(-1, None)):
+        self.rows, ids = rows, torch.as_tensor(ids, device="cuda")      # the positions whose logits are wanted
+        if self.case["model"] in FLAT:
+            return self.gpt2(ids) if self.case["model"] == "gpt2" else self.llama(ids)
+        return getattr(self, self.case["model"])(ids)
+
+    # -- flat families
+    def gpt2(self, ids):
+        d, T = self.desc, len(ids)
+        x = self["wte.weight"][ids] + self["wpe.weight"][:T]
+        ok = seen(T, None, 0)
+        for i in range(d.layers):
+            p = "h.%d." % i
+            h = layer_norm(x, self[p + "ln_1.weight"], self[p + "ln_1.bias"], d.norm_eps)
+            q, k, v = (h @ self[p + "attn.c_attn.weight"] + self[p + "attn.c_attn.bias"]).view(T, 3, d.heads, d.head_dim).unbind(1)
+            o = attend(q, self.kept(k), self.kept(v), ok, d.head_dim ** -0.5).reshape(T, -1)
+            x = x + o @ self[p + "attn.c_proj.weight"] + self[p + "attn.c_proj.bias"]
+            h = layer_norm(x, self[p + "ln_2.weight"], self[p + "ln_2.bias"], d.norm_eps)
+            x = x + gelu_tanh(h @ self[p + "mlp.c_fc.weight"] + self[p + "mlp.c_fc.bias"]) @ self[p + "mlp.c_proj.weight"] + self[p + "mlp.c_proj.bias"]
+        return layer_norm(x[self.rows], self["ln_f.weight"], self["ln_f.bias"], d.norm_eps) @ self["wte.weight"].T
+
+    def llama(self, ids):
+        d, T = self.desc, len(ids)
+        a = angles(1, d.head_dim, d.rope_theta)
+        f = d.rope_theta ** (-2.0 * torch.arange(d.head_dim // 2, dtype=torch.float64, device="cuda") / d.head_dim)
+        if d.rope_factor:
+            wave = 2 * math.pi / f
+            mid = (d.rope_orig_ctx / wave - d.rope_low_freq) / (d.rope_high_freq - d.rope_low_freq)
+            f = torch.where(wave < d.rope_orig_ctx / d.rope_high_freq, f, torch.where(wave > d.rope_orig_ctx / d.rope_low_freq, f / d.rope_factor, (1 - mid) * f / d.rope_factor + mid * f))
+        a = torch.arange(T, dtype=torch.float64, device="cuda")[:, None] * f
+        x, ok = self["model.embed_tokens.weight"][ids], seen(T, None, 0)
+        for i in range(d.layers):
+            p, t = "model.layers.%d." % i, "model.layers.%d.self_attn." % i
+            h = rms(x, d.norm_eps) * self[p + "input_layernorm.weight"]
+            q, k, v = (self.lin(h, t + n + "_proj.weight") + (self[t + n + "_proj.bias"] if d.qkv_bias else 0) for n in "qkv")
+            q, k, v = (y.reshape(T, -1, d.head_dim) for y in (q, k, v))
+            if d.qk_norm:
+                q, k = rms(q, d.norm_eps) * self[t + "q_norm.weight"], rms(k, d.norm_eps) * self[t + "k_norm.weight"]
+            q, k = turn(q, a, d.head_dim), turn(k, a, d.head_dim)
+            x = x + self.lin(attend(q, self.kept(k), self.kept(v), ok, d.head_dim ** -0.5).reshape(T, -1), t + "o_proj.weight")
+            h = rms(x, d.norm_eps) * self[p + "post_attention_layernorm.weight"]
+            x = x + self.lin(silu(self.lin(h, p + "mlp.gate_proj.weight")) * self.lin(h, p + "mlp.up_proj.weight"), p + "mlp.down_proj.weight")
+        h = rms(x[self.rows], d.norm_eps) * self["model.norm.weight"]
+        return self.lin(h, "model.embed_tokens.weight" if d.tied else "lm_head.weight")
+
+    # -- layered designs
+    def sinusoids(self, T):
+        a = angles(T, self.desc.width, 10000.0)
+        return torch.stack([torch.sin(a), torch.cos(a)], -1).reshape(T, -1)
+
+    def zakusun(self, ids):
+        d, T = self.desc, len(ids)
+        x = self["embed"][ids] + self.sinusoids(T)
+        norm = lambda v, n: rms(v.view(len(v), d.norm_groups, -1), d.norm_eps).reshape(len(v), -1) * self[n]      # noqa: E731
+        results, ok = [x], seen(T, None, 0)
+        for i, l in enumerate(d.layers):
+            p, q_ = "l%d." % i, "l%d.mix." % i
+            h = norm(x, p + "norm1")
+            h = h + conv(h, self[p + "canon1"])
+            c = self.kept(rms(self.lin(h, q_ + "dkv"), d.norm_eps) * self[q_ + "dkv.norm"])
+            q, k, v = self.lin(h, q_ + "q").view(T, -1, l.dim), self.lin(c, q_ + "uk").view(T, -1, l.dim), self.lin(c, q_ + "uv").view(T, -1, l.vdim)
+            o = attend(q, k, v, ok, l.scale, sink=self[q_ + "sink"]).reshape(T, -1)
+            x = x + self.lin(o * torch.sigmoid(self.lin(h, q_ + "g")), q_ + "o")
+            h = norm(x, p + "norm2")
+            h = h + conv(h, self[p + "canon2"])
+            z, sel = (self.lin(h, p + "mlp.router") + self[p + "mlp.router.b"]).topk(l.top, -1)
+
+            def expert(e, rows, wt):
+                g = torch.clamp(self.lin(rows, p + "mlp.e%d.gate" % e), max=l.limit)
+                u = torch.clamp(self.lin(rows, p + "mlp.e%d.up" % e), -l.limit, l.limit)
+                return wt * self.lin(g * torch.sigmoid(1.702 * g) * (u + 1), p + "mlp.e%d.down" % e)
+            x = x + by_expert(h, sel, torch.softmax(z, -1), expert)
+            results.append(x)
+            x = sum(a * r for a, r in zip(self[p + "dwa"], results))
+        return self.lin(norm(x[self.rows], "final.norm"), "embed")
+
+    def gated_expert(self, rows, p):
+        return self.lin(silu(self.lin(rows, p + "gate")) * self.lin(rows, p + "up"), p + "down")
+
+    def modepel(self, ids):
+        d, T, eps = self.desc, len(ids), self.desc.norm_eps
+        x, first, ok = self["embed"][ids], None, seen(T, None, 0)
+        for i, l in enumerate(d.layers):
+            p, m = "l%d." % i, "l%d.mix." % i
+            h = rms(x, eps) * self[p + "norm1"]
+            if l.mixer == "attention":
+                q, k, v = (self.lin(h, m + n) + self[m + n + ".b"] for n in "qkv")
+                if first is None:
+                    first = v
+                else:
+                    v = (1 - self[m + "vmix"]) * v + self[m + "vmix"] * first
+                a = angles(T, l.rot_dims, l.rot_base)
+                q, k = (turn(y.view(T, -1, l.dim), a, l.rot_dims) for y in (q, k))
+                o = attend(q, self.kept(k), self.kept(v.view(T, -1, l.vdim)), ok, l.scale, sink=[0.0] * l.heads).reshape(T, -1)
+                y = self.lin(o * torch.sigmoid(self.lin(h, m + "g")), m + "o")
+            else:
+                H, D, cap = l.heads, l.dim, l.gate_cap
+                q, k, v = (self.lin(h, m + n).view(T, H, -1) for n in "qkv")
+                q = q * D ** -0.5
+                ig = cap * torch.tanh((self.lin(h, m + "i") + self[m + "i.b"]) / cap)
+                fg = torch.nn.functional.logsigmoid(cap * torch.tanh((self.lin(h, m + "f") + self[m + "f.b"]) / cap))
+                S, n, mx = x.new_zeros(H, D, l.vdim), x.new_zeros(H, D), x.new_zeros(H)
+                o = torch.empty(T, H, l.vdim, dtype=torch.float64, device="cuda")
+                for t in range(T):
+                    new = torch.maximum(fg[t] + mx, ig[t])
+                    keep, take = torch.exp(fg[t] + mx - new)[:, None], torch.exp(ig[t] - new)[:, None] * k[t]
+                    mx = new
+                    S = keep[..., None] * S + take[..., None] * v[t][:, None]
+                    n = keep * n + take
+                    den = torch.maximum((n * q[t]).sum(-1).abs(), torch.exp(-mx)) + 1e-6
+                    o[t] = (q[t][:, None] @ S)[:, 0] / den[:, None]
+                y = self.lin(rms(o, eps).reshape(T, -1) * self[m + "norm"] * torch.sigmoid(self.lin(h, m + "g")), m + "o")
+            x = x + rms(y, eps) * self[p + "norm1b"]
+            h, f = rms(x, eps) * self[p + "norm2"], p + "mlp."
+            if l.mlp == "dense":
+                z, c = self.lin(h, f + "up"), self[f + "act"]
+                y = self.lin(c[0] * rms(z, eps) + c[1] * rms(z * z, eps) + c[2] * rms(z ** 3, eps) + c[3], f + "down")
+            else:
+                s = torch.softmax(self.lin(h, f + "router"), -1)
+                sel = grouped_choice(s + self[f + "correction"], l.top, l.groups, l.groups_keep, False)
+                y = by_expert(h, sel, s.gather(1, sel) * l.router_scale, lambda e, r, wt: wt * (r if e >= l.experts else self.gated_expert(r, f + "e%d." % e)))
+                y = y + torch.sigmoid(self.lin(h, f + "shared.sg")) * self.gated_expert(h, f + "shared.")
+            x = x + rms(y, eps) * self[p + "norm2b"]
+        return self.lin(rms(x[self.rows], eps) * self["final.norm"], "head")
+
+    def vitudra(self, ids):
+        d, T, eps = self.desc, len(ids), self.desc.norm_eps
+        x, cache = self["embed"][ids], {}
+        for i, l in enumerate(d.layers):
+            p, m = "l%d." % i, "l%d.mix." % i
+            h = rms(x, eps) * (1 + self[p + "norm1"])
+            ok = seen(T, l.mask, l.mask_size)
+            if l.mixer == "attention":
+                q = self.lin(h, m + "q").view(T, -1, l.dim)
+                if l.kv_from is None:
+                    cache[i] = tuple(self.kept(self.lin(h, m + n)).view(T, l.kv_heads, -1) for n in "kv")
+                k, v = cache[i if l.kv_from is None else l.kv_from]
+                pos = torch.arange(T, dtype=torch.float64, device="cuda")
+                q = q * (1 + l.q_temp_coef * torch.log(torch.floor((pos + 1) / l.q_temp_every) + 1))[:, None, None]
+                far = pos[:, None] - pos[None]
+                y = self.lin(attend(q, k, v, ok, l.scale, bias=lambda hd: -2.0 ** (-8.0 * (hd + 1) / l.heads) * far).reshape(T, -1), m + "o")
+            elif l.mixer == "wkv":
+                H, D = l.heads, l.dim
+                prev = torch.cat([torch.zeros_like(h[:1]), h[:-1]])
+                mix = {n: h + (prev - h) * self[m + "mu." + n] for n in "rkvgw"}
+                r, k, v = (self.lin(mix[n], m + n).view(T, H, D) for n in "rkv")
+                w = torch.exp(-torch.exp(self.lin(torch.tanh(self.lin(mix["w"], m + "w1")), m + "w2") + self[m + "w0"])).view(T, H, D)
+                u, S = self[m + "u"], x.new_zeros(H, D, D)
+                o = torch.empty(T, H, D, dtype=torch.float64, device="cuda")
+                for t in range(T):
+                    kv = k[t][..., None] * v[t][:, None]
+                    o[t] = (r[t][:, None] @ (S + u[..., None] * kv))[:, 0]
+                    S = w[t][..., None] * S + kv
+                y = self.lin(rms(o, eps).reshape(T, -1) * self[m + "norm"] * silu(self.lin(mix["g"], m + "g")), m + "o")
+            else:
+                a = angles(T, l.rot_dims, l.rot_base, l.rot_factor)
+                q, k, v = (self.lin(h, m + "left." + n).view(T, -1, l.dim) for n in "qkv")
+                q, k = turn(q, a, l.rot_dims, True), turn(k, a, l.rot_dims, True)
+                left = self.lin(attend(q, self.kept(k), self.kept(v), ok, l.scale, softcap=l.softcap).reshape(T, -1), m + "left.o")
+                m += "right."
+                g = torch.exp(-torch.exp(self[m + "A_log"]) * torch.nn.functional.softplus(self.lin(h, m + "a") + self[m + "dt_bias"]))[..., None]
+                o = self.delta(h, m, l.d_heads, l.d_kv_heads, l.d_dim, l.d_vdim, g)
+                o = rms(o, eps) * self[m + "norm"] * silu(self.lin(h, m + "g")).view(T, l.d_heads, -1)
+                y = l.left_scale * left + l.right_scale * self.lin(o.reshape(T, -1), m + "o")
+            x = x + d.residual_mult * (y + self.gated_expert(h, p + "mlp."))
+        return self.lin(rms(x[self.rows], eps) * (1 + self["final.norm"]), "head")
+
+    def delta(self, h, m, H, G, D, E, g):
+        """delta rule over [T][H][D or 1] decays g"""
+        T = len(h)
+        q, k, v = (silu(conv(self.lin(h, m + n), self[m + n + ".conv"])) for n in "qkv")
+        unit = lambda y: y / torch.sqrt((y * y).sum(-1, keepdim=True) + 1e-6)      # noqa: E731
+        q, k = (unit(y.view(T, G, D)).repeat_interleave(H // G, 1) for y in (q, k))
+        q, v, beta = q * D ** -0.5, v.view(T, H, E), torch.sigmoid(self.lin(h, m + "b"))
+        S, o = h.new_zeros(H, D, E), torch.empty(T, H, E, dtype=torch.float64, device="cuda")
+        for t in range(T):
+            S = g[t][..., None] * S
+            S = S + k[t][..., None] * (beta[t][:, None] * (v[t] - (k[t][:, None] @ S)[:, 0]))[:, None]
+            o[t] = (q[t][:, None] @ S)[:, 0]
+        return o
+
+    def zaluvik(self, ids):
+        d, T, eps = self.desc, len(ids), self.desc.norm_eps
+        ln = lambda v, n: layer_norm(v, self[n], self[n + ".b"], eps)      # noqa: E731
+        x = x0 = self["embed"][ids] * d.embed_scale
+        began = False
+        for i in d.layer_runs():
+            if i == d.loop_start:
+                x = self.lin(torch.cat([x, x0], -1), "loop.in")
+            l, p, m = d.layers[i], "l%d." % i, "l%d.mix." % i
+            h, ok = ln(x, p + "norm1"), seen(T, l.mask, l.mask_size)
+            if l.mixer == "attention":
+                H, G = l.heads, l.kv_heads
+                q, k = rms(self.lin(h, m + "q").view(T, H, -1), eps), self.kept(rms(self.lin(h, m + "k").view(T, G, -1), eps))
+                v, talk, pb = self.kept(self.lin(h, m + "v")).view(T, G, -1), self[m + "talk"], self[m + "pb"]
+                o = torch.zeros(T, H, l.vdim, dtype=torch.float64, device="cuda")
+                for a in range(H):      # the weights of one head go to every head's sum
+                    wt = torch.sigmoid(q[:, a] @ k[:, a // (H // G)].T * l.scale + pb[a]) * ok
+                    for b in range(G):
+                        o[:, b * (H // G):(b + 1) * (H // G)] += (wt @ v[:, b])[:, None] * talk[b * (H // G):(b + 1) * (H // G), a][None, :, None]
+                y = self.lin(o.reshape(T, -1) * torch.sigmoid(self.lin(h, m + "g")), m + "o")
+            else:
+                R, D = l.kv_rank, l.dim
+                q, c, a = self.lin(h, m + "q").view(T, l.heads, -1), self.lin(h, m + "dkv"), angles(T, l.rot_dims, l.rot_base)
+                q = torch.cat([q[..., :D], turn(q[..., D:], a, l.rot_dims)], -1)
+                kr = self.kept(turn(c[:, None, R:], a, l.rot_dims)).expand(T, l.heads, -1)
+                c = self.kept(rms(c[:, :R], eps) * self[m + "dkv.norm"])
+                k = torch.cat([self.lin(c, m + "uk").view(T, l.heads, -1), kr], -1)
+                o = attend(q, k, self.lin(c, m + "uv").view(T, l.heads, -1), ok, l.scale)
+                y = self.lin((o * torch.sigmoid(self.lin(h, m + "g"))[..., None]).reshape(T, -1), m + "o")
+            x = x + d.residual_mult * ln(y, p + "norm1b")
+            h, f = ln(x, p + "norm2"), p + "mlp."
+            if l.mlp == "dense":
+                z = self.lin(h, f + "up")
+                y = self.lin(0.5 * z * (1 + torch.erf(z / math.sqrt(2))), f + "down")
+            else:
+                s = torch.sigmoid(self.lin(h, f + "router"))
+                sel = grouped_choice(s, l.top, l.groups, l.groups_keep, True)
+                wt = s.gather(1, sel)
+                y = by_expert(h, sel, wt / (wt.sum(-1, keepdim=True) + 1e-20), lambda e, r, a: a * self.gated_expert(r, f + "e%d." % e)) + self.gated_expert(h, f + "shared.")
+            x = x + d.residual_mult * ln(y, p + "norm2b")
+        return self.lin(ln(x[self.rows], "final.norm"), "embed")
+
+    def nusovik(self, ids):
+        d, T, eps = self.desc, len(ids), self.desc.norm_eps
+        x = self["embed"][ids] * d.embed_scale + self.sinusoids(T)
+        for i, l in enumerate(d.layers):
+            p, m = "l%d." % i, "l%d.mix." % i
+            if l.mixer == "mamba1":
+                I, N, R = l.inner, l.d_dim, l.dt_rank
+                u, z = self.lin(x, m + "in").split(I, -1)
+                u = silu(conv(u, self[m + "conv"], self[m + "conv.b"]))
+                r = self.lin(u, m + "x")
+                dt = torch.nn.functional.softplus(self.lin(r[:, :R], m + "dt") + self[m + "dt.b"])
+                A, B, C = -torch.exp(self[m + "A_log"]), r[:, R:R + N], r[:, R + N:]
+                S, y = x.new_zeros(I, N), torch.empty(T, I, dtype=torch.float64, device="cuda")
+                for t in range(T):
+                    S = torch.exp(dt[t][:, None] * A) * S + (dt[t] * u[t])[:, None] * B[t]
+                    y[t] = S @ C[t]
+                y = self.lin((y + self[m + "D"] * u) * silu(z), m + "o")
+            else:
+                a = m + "left."
+                q, k = ((self.lin(x, a + n) + self[a + n + ".b"]).view(T, -1, l.dim) for n in "qk")
+                v = self.kept(k)
+                q, k = rms(q, eps) * self[a + "q.norm"], self.kept(rms(k, eps) * self[a + "k.norm"])
+                B = l.bias_buckets
+                n = torch.arange(T, device="cuda")
+                log = torch.log(n.clamp(min=1) / (B // 2)) / math.log(l.bias_max / (B // 2)) * (B - B // 2)
+                row = torch.where(n < B // 2, n, torch.clamp(B // 2 + torch.floor(log.double() + 1e-9).long(), max=B - 1))
+                rel, far = self[a + "rel"], row[(n[:, None] - n[None]).clamp(min=0)]
+                o = attend(q, k, v, seen(T, l.mask, l.mask_size), l.scale, sink=self[a + "sink"], bias=lambda h: rel[far, h])
+                y = l.left_scale * self.lin((o * torch.sigmoid(self.lin(x, a + "g"))[..., None]).reshape(T, -1), a + "o")
+                a, H, E, N, G = m + "right.", l.d_heads, l.d_vdim, l.d_dim, l.d_kv_heads
+                I = H * E
+                r = self.lin(x, a + "in")
+                u = silu(conv(r[:, I:2 * I + 2 * G * N], self[a + "conv"], self[a + "conv.b"]))
+                dt = torch.nn.functional.softplus(r[:, 2 * I + 2 * G * N:] + self[a + "dt_bias"])
+                keep = torch.exp(-torch.exp(self[a + "A_log"]) * dt)
+                xs, B, C = u[:, :I].view(T, H, E), u[:, I:I + G * N].view(T, G, N).repeat_interleave(H // G, 1), u[:, I + G * N:].view(T, G, N).repeat_interleave(H // G, 1)
+                S, s = x.new_zeros(H, N, E), torch.empty(T, H, E, dtype=torch.float64, device="cuda")
+                for t in range(T):
+                    S = keep[t][:, None, None] * S + (dt[t][:, None] * B[t])[..., None] * xs[t][:, None]
+                    s[t] = (C[t][:, None] @ S)[:, 0]
+                s = ((s + self[a + "D"][:, None] * xs).reshape(T, I) * silu(r[:, :I])).view(T, l.part_norms, -1)
+                y = y + l.right_scale * self.lin(rms(s, eps).reshape(T, I) * self[a + "norm"], a + "o")
+            x = x + rms(y, eps) * self[p + "norm1"]
+            if l.mlp:
+                x = x + rms(self.lin(torch.relu(self.lin(x, p + "mlp.up")) ** 2, p + "mlp.down"), eps) * self[p + "norm2"]
+        return self.lin(rms(x[self.rows], eps) * self["final.norm"], "head")
+
+    def keronex(self, ids):
+        d, T, eps = self.desc, len(ids), self.desc.norm_eps
+        e = self["embed"][ids] * d.embed_scale
+        pair = torch.full((T,), d.bigram_buckets, device="cuda")
+        pair[1:] = (ids[:-1] * d.bigram_before + ids[1:] * d.bigram_cur) % d.bigram_buckets
+        xs, ok = (e + self["bigram"][pair])[None].repeat(d.streams, 1, 1), seen(T, None, 0)
+        norm = lambda v, n: rms(v, eps) * (1 + self[n])      # noqa: E731
+
+        def sublayer(xs, hc, name, f):
+            y = f(norm(torch.einsum("s,stw->tw", self[hc + ".in"], xs), name))
+            return torch.einsum("sk,stw->ktw", self[hc + ".mix"], xs) + self[hc + ".out"][:, None, None] * y
+        relu2 = lambda rows, p, wt=1.0: self.lin(torch.relu(self.lin(wt * rows, p + "up")) ** 2, p + "down")      # noqa: E731
+        for i, l in enumerate(d.layers):
+            p = "l%d." % (i if l.weights_of is None else l.weights_of)
+            m, f, H = p + "mix.", p + "mlp.", l.heads
+
+            def mixer(h):
+                if l.mixer == "retention":
+                    a = angles(T, l.rot_dims, l.rot_base)
+                    q, k = (turn(self.lin(h, m + n).view(T, H, -1), a, l.rot_dims) for n in "qk")
+                    k, v = k * l.dim ** -0.5, self.lin(h, m + "v").view(T, H, -1)
+                    keep = torch.tensor(np.float32(l.decays), device="cuda").double()[:, None, None]
+                    S, o = h.new_zeros(H, l.dim, l.vdim), torch.empty(T, H, l.vdim, dtype=torch.float64, device="cuda")
+                    for t in range(T):
+                        S = keep * S + k[t][..., None] * v[t][:, None]
+                        o[t] = (q[t][:, None] @ S)[:, 0]
+                    return self.lin(rms(o, eps).reshape(T, -1) * silu(self.lin(h, m + "g")), m + "o")
+                if l.mixer == "attention":
+                    a = angles(T, l.rot_dims, l.rot_base)
+                    q, k = turn(self.lin(h, m + "q").view(T, -1, l.dim), a, l.rot_dims), self.kept(turn(self.lin(h, m + "k").view(T, -1, l.dim), a, l.rot_dims))
+                    v = self.kept(self.lin(h, m + "v")).view(T, l.kv_heads, -1)
+                    lam = torch.exp((self[m + "lq1"] * self[m + "lk1"]).sum()) - torch.exp((self[m + "lq2"] * self[m + "lk2"]).sum()) + float(np.float32(l.diff))
+                    o = attend(q[:, 0::2], k[:, 0::2], v, ok, l.scale) - lam * attend(q[:, 1::2], k[:, 1::2], v, ok, l.scale)
+                    return self.lin((rms(o, eps) * (1 - float(np.float32(l.diff)))).reshape(T, -1), m + "o")
+                g = torch.nn.functional.softplus(self.lin(self.lin(h, m + "a1"), m + "a2") + self[m + "dt_bias"]).view(T, H, -1)
+                o = self.delta(h, m, H, l.kv_heads, l.dim, l.vdim, torch.exp(-torch.exp(self[m + "A_log"])[:, None] * g))
+                return self.lin((rms(o, eps) * self[m + "norm"]).reshape(T, -1) * torch.sigmoid(self.lin(self.lin(h, m + "g1"), m + "g2")), m + "o")
+
+            def feed(h):
+                if l.mlp == "dense":
+                    return self.lin(gelu_tanh(self.lin(h, f + "gate")) * self.lin(h, f + "up"), f + "down")
+                s, sel = torch.sigmoid(self.lin(h, f + "router")).topk(l.top, -1)
+                return by_expert(h, sel, s, lambda e, r, wt: relu2(r, f + "e%d." % e, wt)) + relu2(h, f + "shared.")
+            xs = sublayer(xs, p + "hc1", p + "norm1", mixer)
+            xs = sublayer(xs, p + "hc2", p + "norm2", feed)
+        return self.lin(norm(xs.sum(0)[self.rows], "final.norm"), "head")
+
+
+def exact(case, seed):
+    # a prompt of a design with recurrent layers is walked token by token, and a greedy token costs a walk over its whole sequence
+    flat, lens = case["model"] in FLAT, lengths(case)
+    walk = sum(lens) * (1.0e-5 if flat else 1.0e-4 * case["layers"])
+    if walk > 18:
+        return None
+    m = Exact(case, seed)
+    prompts, fed = tokens_of(case, m.desc.vocab, seed)
+    steps = case["steps"]
+    if case["mode"] == "forced":      # one walk over prompt and fed tokens, the logits behind every fed token taken from it
+        per = [m.logits(list(p) + [int(fed[t][i]) for t in range(steps)], slice(len(p) - 1, None)).cpu() for i, p in enumerate(prompts)]
+        return {"first" if t == 0 else "step%02d" % (t - 1): torch.stack([x[t] for x in per]) for t in range(steps + 1)}
+    out = {"first": torch.cat([m.logits(p) for p in prompts]).cpu()}
+    if not steps:
+        return out
+    # tokens that a draw or a rounding may choose have no exact value
+    if case["mode"] == "sampled" or walk * (1 + steps) > 18 or (flat and m.desc.tied and case["dtype"] != "fp32"):
+        return dict(out, tokens=None, last=None)
+    seqs, last, toks = [list(p) for p in prompts], out["first"], []
+    for t in range(steps + 1):
+        for s, row in zip(seqs, last):
+            s.append(int(row.argmax()))
+        if t:
+            toks.append([s[-1] for s in seqs])
+        if t < steps:
+            last = torch.cat([m.logits(s) for s in seqs]).cpu()
+    return dict(out, tokens=torch.tensor(toks), last=last)
+
+
+# ---- what a pass cannot do without ---------------------------------------------------------------------------------------------------------
+def work(case):
+    """every step reads each matrix it needs once (of the experts: as many as its tokens are expected to choose), reads the cached keys and values of its requests
+    and writes its logits; two operations for each weight and token, and those of the attention's and the recurrences' own products"""
+    es, lens, steps = TORCH[case["dtype"]].itemsize, lengths(case), case["steps"]
+    desc = flat_desc(case) if case["model"] in FLAT else stack_desc(case)
+    count = lambda names: sum(math.prod(s) for n, s in names)      # noqa: E731
+    shapes = list(desc.tensor_shapes().items())
+    table = [(n, s) for n, s in shapes if n in ("embed", "bigram", "wte.weight", "wpe.weight", "model.embed_tokens.weight")]
+    head = math.prod(next((s for n, s in shapes if n in ("head", "lm_head.weight")), (desc.vocab, desc.hidden)))
+    expert = [(n, s) for n, s in shapes if ".mlp.e" in n]
+    plain = count(shapes) - count(table) - count(expert) - (head if any(n in ("head", "lm_head.weight") for n, _ in shapes) else 0)
+    bytes_, flops = 0.0, 0.0
+    layers = desc.layers if case["model"] not in FLAT else []
+    runs = [layers[i] for i in desc.layer_runs()] if layers else []
+    moe = next((l for l in layers if l.mlp == "moe"), None)
+    for k in range(steps + 1):
+        toks = sum(lens) if k == 0 else len(lens)
+        chosen = 0.0 if moe is None else count(expert) * (1 - (1 - moe.top / moe.experts) ** toks)
+        bytes_ += es * (plain + chosen + head) + 4.0 * len(lens) * desc.vocab
+        active = plain + (0 if moe is None else count(expert) * moe.top / moe.experts)
+        flops += 2.0 * toks * active + 2.0 * len(lens) * head
+        for n in lens:
+            rows, ctx = (n, (n + 1) / 2) if k == 0 else (1, n + k)
+            if not layers:
+                flops += 4.0 * desc.layers * desc.q_dim * rows * ctx
+                bytes_ += es * 2.0 * desc.layers * desc.kv_dim * (n + k)
+            for l in runs:
+                if l.mixer in ("attention", "latent_attention") or (l.mixer == "parallel"):
+                    c, held = (min(ctx, l.mask_size), min(n + k, l.mask_size)) if l.mask else (ctx, n + k)
+                    flops += 2.0 * l.maps * l.heads * (l.dim + l.rot_dim + l.vdim) * rows * c
+                    bytes_ += es * held * (l.kv_rank + l.rot_dim if l.mixer == "latent_attention" else l.kv_heads * (l.maps * l.dim + l.vdim))
+                state = {"mlstm": l.heads * l.dim * l.vdim, "wkv": l.heads * l.dim * l.vdim, "retention": l.heads * l.dim * l.vdim, "channel_delta": l.heads * l.dim * l.vdim,
+                         "parallel": l.d_heads * l.d_dim * l.d_vdim, "mamba1": l.inner * l.d_dim}.get(l.mixer, 0)
+                flops += 6.0 * rows * state
+                bytes_ += (8.0 if k else 4.0) * state
+    return {"bytes": float(bytes_), "flops": float(flops)}
+
+
+def tolerance(case):
+    # fp32 storage rounds nothing: sums in another order (5e-7 off 64 bits, measured).  16-bit storage rounds keys, values and latents once into the cache, and two
+    # correct implementations differ where a rounding falls on the other side: up to 1e-3 off 64 bits, measured over these ranges (24 layers of 16-bit rows); a
+    # router's near tie may also hand a token to another expert.
+    if case["dtype"] == "fp32":
+        return {"rel": 4e-6, "max": 4e-4, "differ": 0.0}
+    return {"rel": 0.01 if case["model"] in ("zakusun", "modepel", "zaluvik", "keronex") else 0.004, "max": 0.2, "differ": 0.01}
