@@ -41,7 +41,7 @@ def listed():
         # a running batch whose rows were refilled one by one with prompts of different lengths
         dict(name="llama-rows-fp16", model="llama-3.2-1b", dtype="fp16", seqs=16, prompt=300, ragged=True, steps=24, mode="greedy"),
         # the layered designs: ragged prompts of a few requests joining in one step, then tokens of all of them
-        dict(name="zakusun-serve", model="zakusun", width=1024, layers=8, dtype="bf16", seqs=4, prompt=1100, ragged=True, steps=12, mode="forced"),
+        dict(name="zakusun-serve", model="zakusun", width=1024, layers=8, dtype="bf16", seqs=4, prompt=900, ragged=True, steps=12, mode="forced"),
         # one long prompt of a wide mixture-of-experts design
         dict(name="modepel-prompt", model="modepel", width=2048, layers=4, dtype="bf16", seqs=1, prompt=2048, ragged=False, steps=6, mode="forced"),
         # an interactive turn: a short question, one stream of tokens from the library's decode loop (launches and latency)
@@ -197,6 +197,7 @@ def weights(case, desc, seed):
             v = uniform(0, 1)
         elif rule is not None and not (len(shape) == 2 and leaf in ("b", "norm")):
             _, kind, a, b = rule
+            a = 1.0 if leaf == "router" and case["model"] in ("keronex", "zaluvik") else a      # (sigmoid scores: three deviations would press them against one)
             v = (normal() * b + a if kind == "normal" else uniform(a, b) if kind == "uniform" else normal() * a / math.sqrt(shape[-1]) if kind == "proj"
                  else torch.eye(shape[0], device="cuda") + normal() * a if kind == "eye" else normal() * a + 1.0 / shape[0])
         elif "norm" in leaf or "norm" in name.split(".")[-2:][0] or ".ln_" in name or name.startswith("ln_"):
@@ -204,6 +205,8 @@ def weights(case, desc, seed):
         elif len(shape) == 2:
             fan = shape[0] if case["model"] == "gpt2" else shape[-1]                     # that family stores its projections inputs first
             v = normal() / math.sqrt(fan)
+            if ".mlp.e" in name and leaf == "down":      # one expert of several adds a part to a stream that the rest has built: two that score alike are no coin that turns the result
+                v = v * 0.3
         else:
             v = normal() * 0.3
         v = v.to(dt)
