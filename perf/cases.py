@@ -182,39 +182,65 @@ SPREAD = [("mix.sink", "normal", 0, 1), (".dwa", "mean", 0.2, 0), (".canon1", "n
 
 def weights(case, desc, seed):
     """(name, tensor in the storage type on the GPU) of every tensor of the checkpoint, from the seed alone"""
-    dt, offset = TORCH[case["dtype"]], case["model"] in ("vitudra", "keronex")
-    for name, shape in desc.tensor_shapes().items():
-        gen = torch.Generator("cuda").manual_seed((seed * 1000003 + zlib.crc32(name.encode())) % (1 << 62))
-        normal = lambda: torch.randn(shape, generator=gen, device="cuda")              # noqa: E731
-        uniform = lambda a, b: torch.rand(shape, generator=gen, device="cuda") * (b - a) + a      # noqa: E731
-        leaf = name.split(".")[-1]
-        rule = next((r for r in SPREAD if name.endswith(r[0])), None)
-        if name in ("embed", "bigram") or "wte" in name or "wpe" in name or "embed_tokens" in name:
-            v = normal() * (1.0 if name in ("embed", "bigram") and case["model"] not in ("zakusun", "zaluvik") else 0.5)
-        elif leaf in ("in",) and len(shape) == 2:                                        # projections of that name, not the streams' weights
-            v = normal() / math.sqrt(shape[-1] if name != "loop.in" else shape[-1] / 2)
-        elif ".mu." in name:
-            v = uniform(0, 1)
-        elif rule is not None and not (len(shape) == 2 and leaf in ("b", "norm")):
-            _, kind, a, b = rule
-            a = 1.0 if leaf == "router" and case["model"] in ("keronex", "zaluvik") else a      # (sigmoid scores: three deviations would press them against one)
-            v = (normal() * b + a if kind == "normal" else uniform(a, b) if kind == "uniform" else normal() * a / math.sqrt(shape[-1]) if kind == "proj"
-                 else torch.eye(shape[0], device="cuda") + normal() * a if kind == "eye" else normal() * a + 1.0 / shape[0])
-        elif "norm" in leaf or "norm" in name.split(".")[-2:][0] or ".ln_" in name or name.startswith("ln_"):
-            v = uniform(-0.3, 0.3) if offset and (leaf == "norm1" or leaf == "norm2" or name == "final.norm") else uniform(0.7, 1.3)
-        elif len(shape) == 2:
-            fan = shape[0] if case["model"] == "gpt2" else shape[-1]                     # that family stores its projections inputs first
-            v = normal() / math.sqrt(fan)
-            if ".mlp.e" in name and leaf == "down":      # one expert of several adds a part to a stream that the rest has built: two that score alike are no coin that turns the result
-                v = v * 0.3
-        else:
-            v = normal() * 0.3
-        v = v.to(dt)
+    shapes = desc.tensor_shapes()
+    for name, shape in shapes.items():
+        v = one_tensor(case, name, shape, seed)
+        if name == "embed":
+            for i, l in enumerate(desc.layers):
+                if "l%d.mlp.router" % i in shapes:
+                    v += preferences(case, l, shapes["l%d.mlp.router" % i], "l%d.mlp.router" % i, v, seed)
+        v = v.to(TORCH[case["dtype"]])
         if name in ("head", "lm_head.weight"):
             rows = loud_rows(seed, shape[0])
             v[rows[:LOUD]] *= LOUD_SCALE
             v[rows[LOUD:]] = -v[rows[:LOUD]]
         yield name, v
+
+
+def generator(seed, name):
+    return torch.Generator("cuda").manual_seed((seed * 1000003 + zlib.crc32(name.encode())) % (1 << 62))
+
+
+def preferences(case, l, shape, name, embed, seed):
+    """what a trained router knows of a token: a part of its embedding along the rows of a few experts (of as many groups as may be kept), so that the choice of an
+    expert is no near tie that the last bit of a sum decides"""
+    rows = one_tensor(case, name, shape, seed)[:l.experts + l.identity]
+    rows = rows / rows.norm(dim=1, keepdim=True)
+    groups, keep = (l.groups, l.groups_keep) if l.groups > 1 else (1, 1)
+    per, gen = len(rows) // groups, generator(seed, name + ".tokens")
+    kept = torch.rand(len(embed), groups, generator=gen, device="cuda").topk(keep, 1).indices
+    out = torch.zeros_like(embed)
+    for g in range(keep):
+        of = torch.rand(len(embed), per, generator=gen, device="cuda").topk(max(1, l.top // keep), 1).indices
+        for j in range(of.shape[1]):
+            out += rows[kept[:, g] * per + of[:, j]]
+    return out * (8.0 * float(embed[:64].std()))
+
+
+def one_tensor(case, name, shape, seed):
+    gen, offset = generator(seed, name), case["model"] in ("vitudra", "keronex")
+    normal = lambda: torch.randn(shape, generator=gen, device="cuda")              # noqa: E731
+    uniform = lambda a, b: torch.rand(shape, generator=gen, device="cuda") * (b - a) + a      # noqa: E731
+    leaf = name.split(".")[-1]
+    rule = next((r for r in SPREAD if name.endswith(r[0])), None)
+    if name in ("embed", "bigram") or "wte" in name or "wpe" in name or "embed_tokens" in name:
+        return normal() * (1.0 if name in ("embed", "bigram") and case["model"] not in ("zakusun", "zaluvik") else 0.5)
+    if leaf in ("in",) and len(shape) == 2:                                          # projections of that name, not the streams' weights
+        return normal() / math.sqrt(shape[-1] if name != "loop.in" else shape[-1] / 2)
+    if ".mu." in name:
+        return uniform(0, 1)
+    if rule is not None and not (len(shape) == 2 and leaf in ("b", "norm")):
+        _, kind, a, b = rule
+        a = 1.0 if leaf == "router" and case["model"] in ("keronex", "zaluvik") else a      # (sigmoid scores: three deviations would press them against one)
+        return (normal() * b + a if kind == "normal" else uniform(a, b) if kind == "uniform" else normal() * a / math.sqrt(shape[-1]) if kind == "proj"
+                else torch.eye(shape[0], device="cuda") + normal() * a if kind == "eye" else normal() * a + 1.0 / shape[0])
+    if "norm" in leaf or "norm" in name.split(".")[-2:][0] or ".ln_" in name or name.startswith("ln_"):
+        return uniform(-0.3, 0.3) if offset and (leaf == "norm1" or leaf == "norm2" or name == "final.norm") else uniform(0.7, 1.3)
+    if len(shape) == 2:
+        fan = shape[0] if case["model"] == "gpt2" else shape[-1]                     # that family stores its projections inputs first
+        # one expert of several adds a part to a stream that the rest has built
+        return normal() / math.sqrt(fan) * (0.3 if ".mlp.e" in name and leaf == "down" else 1.0)
+    return normal() * 0.3
 
 
 def loud_rows(seed, vocab):
