@@ -67,6 +67,19 @@ __device__ __forceinline__ float gelu_tanh(float z) { return 0.5f * z * (1.0f + 
 // the product of a gated feed-forward's two halves: silu or (act SG_ACT_GELU_TANH) the tanh gelu of the gate
 __device__ __forceinline__ float gate_mul(const StackGemmArgs& a, float gate, float up) { return a.act == SG_ACT_GELU_TANH ? gelu_tanh(gate) * up : silu_mul(gate, up); }
 
+// one output of a product: the epilogue on the accumulated sum v (dual products: v of the first matrix, v2 of the second) of grouped / batched row m and column n
+template <int EPI>
+__device__ __forceinline__ void sg_finish(const StackGemmArgs& a, int z, int m, int n, float v, float v2) {
+  const size_t crow = a.c_rows ? (size_t)a.c_rows[m] : (size_t)m;
+  float* cp = a.C + crow * a.ldc + (size_t)z * a.c_zoff + n;
+  if constexpr (EPI == SG_STORE) *cp = store_value(a, a.in_w ? v * a.in_w[a.in_rows[m]] : v, (size_t)z * a.c_zoff + n, n);
+  else if constexpr (EPI == SG_ADD) *cp = fmaf(v, a.scale, *cp);
+  else if constexpr (EPI == SG_GATE) *cp = v / (1.0f + expf(-a.G[crow * a.ldg + a.g_col0 + (a.g_per_z ? (size_t)z : (size_t)z * a.c_zoff + n)]));
+  else if constexpr (EPI == SG_EXPERT_ACT) *cp = expert_act(v, v2, a.limit);
+  else if constexpr (EPI == SG_SILU_MUL) *cp = gate_mul(a, v, v2);
+  else *cp = v * a.rw[crow];
+}
+
 template <int DT, int EPI, bool DUAL, int WT, bool VEC>
 __global__ __launch_bounds__(256) void stack_gemm_kernel(const StackGemmArgs a) {
   constexpr bool F32 = DT == DT_F32;
@@ -242,20 +255,10 @@ __global__ __launch_bounds__(256) void stack_gemm_kernel(const StackGemmArgs a) 
     for (int r = 0; r < 16; r++) {
       const int m = mbase + wm * (32 * WT) + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
       if (m >= mend) continue;
-      const size_t crow = a.c_rows ? (size_t)a.c_rows[m] : (size_t)m;
-      float* cp = a.C + crow * a.ldc + (size_t)z * a.c_zoff;
-      const float in_w = EPI == SG_STORE && a.in_w ? a.in_w[a.in_rows[m]] : 1.f;
 #pragma unroll
       for (int j = 0; j < WT; j++) {
         const int n = n0 + wn * (32 * WT) + j * 32 + (lane & 31);
-        if (n >= a.N) continue;
-        const float v = acc[0][i][j][r];
-        if constexpr (EPI == SG_STORE) cp[n] = store_value(a, a.in_w ? v * in_w : v, (size_t)z * a.c_zoff + n, n);
-        else if constexpr (EPI == SG_ADD) cp[n] = fmaf(v, a.scale, cp[n]);
-        else if constexpr (EPI == SG_GATE) cp[n] = v / (1.0f + expf(-a.G[crow * a.ldg + a.g_col0 + (a.g_per_z ? (size_t)z : (size_t)z * a.c_zoff + n)]));
-        else if constexpr (EPI == SG_EXPERT_ACT) cp[n] = expert_act(v, acc[NB - 1][i][j][r], a.limit);
-        else if constexpr (EPI == SG_SILU_MUL) cp[n] = gate_mul(a, v, acc[NB - 1][i][j][r]);
-        else cp[n] = v * a.rw[crow];
+        if (n < a.N) sg_finish<EPI>(a, z, m, n, acc[0][i][j][r], acc[NB - 1][i][j][r]);
       }
     }
 }
@@ -270,22 +273,17 @@ constexpr size_t stack_gemm_lds() {
 
 namespace tgx {
 
-// output columns per wave of the few-row kernel (four for eight-row tiles was measured slower: 16 rows x 8 layers at width 2048 6.6k -> 6.2k tokens/s)
-constexpr int stack_gemv_cols(int, bool) { return 2; }
+constexpr int STACK_GEMV_COLS = 2;      // output columns per wave
 
-// ---- the same products for a FEW rows (decode steps): a weight-streaming kernel.  One wave per pair of output columns: every lane takes 8 weights of each
+// ---- the same products for ONE or TWO rows (decode steps): a weight-streaming kernel.  One wave per pair of output columns: every lane takes 8 weights of each
 // column per pass (one 16-byte load for the 16-bit dtypes) against the 8 activations of up to MR rows, fp32 FMA chains, one cross-lane sum per (row, column)
-// at the end.  Same argument block, batching (blockIdx.z), grouping (tile list with tiles of MR rows) and epilogues as stack_gemm_kernel; the activations
+// at the end.  Same argument block, batching (blockIdx.z) and epilogues as stack_gemm_kernel; the activations
 // enter in fp32 (rounded to the storage dtype first under option act.round16).  Needs the vector-load alignment (K a multiple of 8).
 template <int DT, int EPI, bool DUAL, int MR>
 __global__ __launch_bounds__(256) void stack_gemv_kernel(const StackGemmArgs a) {
-  constexpr int NC = stack_gemv_cols(MR, DUAL), NB = DUAL ? 2 : 1;
+  constexpr int NC = STACK_GEMV_COLS, NB = DUAL ? 2 : 1;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  int z, mbase, mend;
-  if (a.z_off) {
-    if ((int)blockIdx.y >= *a.n_tiles) return;
-    z = a.tile_z[blockIdx.y]; mbase = a.tile_m0[blockIdx.y]; mend = min(a.z_off[z + 1], mbase + MR);
-  } else { z = blockIdx.z; mbase = blockIdx.y * MR; mend = min(a.M, mbase + MR); }
+  const int z = blockIdx.z, mbase = blockIdx.y * MR, mend = min(a.M, mbase + MR);
   const int n0 = (blockIdx.x * 4 + wv) * NC;
   if (n0 >= a.N) return;
   const float* Ab = a.A + (size_t)z * a.a_zoff;
@@ -336,27 +334,15 @@ __global__ __launch_bounds__(256) void stack_gemv_kernel(const StackGemmArgs a) 
     for (int j = 0; j < NC; j++)
 #pragma unroll
       for (int r = 0; r < MR; r++) acc[b][j][r] = wave_sum(acc[b][j][r]);
-  if (lane != 0) return;
+  // one output a lane, so that the epilogues' loads (bias, gate, the stream itself) are one round trip and not one after the other
+  float v = acc[0][0][0], v2 = acc[NB - 1][0][0];
 #pragma unroll
-  for (int r = 0; r < MR; r++) {
-    const int m = mbase + r;
-    if (m >= mend) break;
-    const size_t crow = a.c_rows ? (size_t)a.c_rows[m] : (size_t)m;
-    float* cp = a.C + crow * a.ldc + (size_t)z * a.c_zoff;
-    const float in_w = EPI == SG_STORE && a.in_w ? a.in_w[a.in_rows[m]] : 1.f;
+  for (int r = 0; r < MR; r++)
 #pragma unroll
-    for (int j = 0; j < NC; j++) {
-      const int n = n0 + j;
-      if (n >= a.N) break;
-      const float v = acc[0][j][r];
-      if constexpr (EPI == SG_STORE) cp[n] = store_value(a, a.in_w ? v * in_w : v, (size_t)z * a.c_zoff + n, n);
-      else if constexpr (EPI == SG_ADD) cp[n] = fmaf(v, a.scale, cp[n]);
-      else if constexpr (EPI == SG_GATE) cp[n] = v / (1.0f + expf(-a.G[crow * a.ldg + a.g_col0 + (a.g_per_z ? (size_t)z : (size_t)z * a.c_zoff + n)]));
-      else if constexpr (EPI == SG_EXPERT_ACT) cp[n] = expert_act(v, acc[NB - 1][j][r], a.limit);
-      else if constexpr (EPI == SG_SILU_MUL) cp[n] = gate_mul(a, v, acc[NB - 1][j][r]);
-      else cp[n] = v * a.rw[crow];
-    }
-  }
+    for (int j = 0; j < NC; j++)
+      if (lane == r * NC + j) { v = acc[0][j][r]; v2 = acc[NB - 1][j][r]; }
+  const int m = mbase + lane / NC, n = n0 + lane % NC;
+  if (lane < MR * NC && m < mend && n < a.N) sg_finish<EPI>(a, z, m, n, v, v2);
 }
 
 }  // namespace tgx

@@ -147,6 +147,11 @@ void launch_gqa_mfma(tgx_ctx* c, const tgx::StepMeta& m, const tgx::GqaMfmaArgs&
 void launch_mix_mfma(tgx_ctx* c, const tgx::StepMeta& m, const tgx::MixMfmaArgs& a, dim3 grid);      // kernels/stack_mix_mfma.h
 size_t mix_mfma_wg_lds(int heads, int kv_heads);      // LDS bytes of one of its workgroups
 
+// stack_few.hip
+namespace tgx { struct StackGemmArgs; }
+int stack_few_init(tgx_ctx* c);
+void launch_stack_few(tgx_ctx* c, const tgx::StackGemmArgs& a, int epi, int nz, int grouped_tiles, int dt);
+
 // stack_ssd.hip
 bool ssd_mfma_shapes_ok(int heads, int groups, int N, int E, long long ld);
 size_t ssd_gram_elems(int T, int S, int groups);

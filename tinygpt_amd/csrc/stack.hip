@@ -76,16 +76,15 @@ void launch_gemm_t(tgx_ctx* c, const tgx::StackGemmArgs& a, dim3 grid1, dim3 gri
 }
 template <int DT, int EPI, bool DUAL>
 void launch_gemv_t(tgx_ctx* c, const tgx::StackGemmArgs& a, dim3 grid, int mr) {
-  switch (mr) {
-    case 1: hipLaunchKernelGGL((tgx::stack_gemv_kernel<DT, EPI, DUAL, 1>), grid, dim3(256), 0, c->stream, a); break;
-    case 2: hipLaunchKernelGGL((tgx::stack_gemv_kernel<DT, EPI, DUAL, 2>), grid, dim3(256), 0, c->stream, a); break;
-    case 4: hipLaunchKernelGGL((tgx::stack_gemv_kernel<DT, EPI, DUAL, 4>), grid, dim3(256), 0, c->stream, a); break;
-    default: hipLaunchKernelGGL((tgx::stack_gemv_kernel<DT, EPI, DUAL, 8>), grid, dim3(256), 0, c->stream, a); break;
-  }
+  if (mr == 1) hipLaunchKernelGGL((tgx::stack_gemv_kernel<DT, EPI, DUAL, 1>), grid, dim3(256), 0, c->stream, a);
+  else hipLaunchKernelGGL((tgx::stack_gemv_kernel<DT, EPI, DUAL, 2>), grid, dim3(256), 0, c->stream, a);
 }
 // rows per tile of a grouped product's plan (moe_plan_kernel tile_m): steps of few (token, expert) pairs stream the experts through the few-row kernel
-constexpr int GROUPED_FEW_PAIRS = 128, GROUPED_FEW_ROWS = 4, FEW_ROWS_MAX = 16;
-constexpr int FEW_COLS_ANY_ROWS = 64;      // a matrix of so few rows (the router's) is streamed per eight-row tile whatever the step's size: the 64-wide matrix-core tiles would stand mostly empty
+constexpr int GROUPED_FEW_PAIRS = 128, GROUPED_FEW_ROWS = 16, FEW_ROWS_MAX = 64;
+// the vector kernel serves one and two rows (1024 x 1024, two rows: 4.4 us against 5.4; 3072 x 1024 gate and up: 6.8 against 7.7; four rows 6.0 against 5.5), stack_few_kernel
+// three to 64 and the grouped tiles (47 rows, 1024 x 3072: 25 us against 38 on 64-wide tiles)
+constexpr int GEMV_ROWS_MAX = 2;
+constexpr int FEW_COLS_ANY_ROWS = 64;      // a matrix of so few rows (the router's) takes the few-row kernel whatever the step's size: the 64-wide matrix-core tiles would stand mostly empty
 // (both products of the layer must be able to take it: their contraction lengths, the width and the expert width, in whole 8-element slices)
 int grouped_tile_rows(const tgx_ctx* c, int pairs, int width, int ff) {
   return c->stack->gemv && pairs <= GROUPED_FEW_PAIRS && width % 8 == 0 && ff % 8 == 0 ? GROUPED_FEW_ROWS : 64;
@@ -105,10 +104,11 @@ void launch_gemm(tgx_ctx* c, tgx::StackGemmArgs a, int epi, int nz, int grouped_
   // few rows: the weight-streaming kernel (its loads take whole 8-element slices)
   const bool few = sm->gemv && vec && a.K % 8 == 0 && a.ldb % 8 == 0 && a.b_zstride % 8 == 0 && (a.z_off ? grouped_tile == GROUPED_FEW_ROWS : (a.M <= FEW_ROWS_MAX || a.N <= FEW_COLS_ANY_ROWS));
   if (a.z_off && grouped_tile == GROUPED_FEW_ROWS && !few) { c->launch_fault = "grouped product: the plan was made for the few-row kernel, which these operands cannot take"; return; }
+  if (few && (a.z_off || a.M > GEMV_ROWS_MAX)) { launch_stack_few(c, a, epi, nz, a.z_off ? grouped_rows / GROUPED_FEW_ROWS + std::min(groups, grouped_rows) : 0, dt); return; }
   if (few) {
-    const int mr = a.z_off ? GROUPED_FEW_ROWS : (a.M <= 1 ? 1 : a.M <= 2 ? 2 : a.M <= 4 ? 4 : 8);
-    const int cols = 4 * tgx::stack_gemv_cols(mr, dual);      // per workgroup
-    const dim3 grid((a.N + cols - 1) / cols, a.z_off ? grouped_rows / mr + groups : (a.M + mr - 1) / mr, a.z_off ? 1 : nz);
+    const int mr = a.M <= 1 ? 1 : 2;
+    const int cols = 4 * tgx::STACK_GEMV_COLS;      // per workgroup
+    const dim3 grid((a.N + cols - 1) / cols, (a.M + mr - 1) / mr, nz);
     TGX_DT_SWITCH(dt,
       switch (epi) {
         case tgx::SG_STORE: launch_gemv_t<DT, tgx::SG_STORE, false>(c, a, grid, mr); break;
@@ -124,7 +124,7 @@ void launch_gemm(tgx_ctx* c, tgx::StackGemmArgs a, int epi, int nz, int grouped_
   dim3 g1, g2;
   if (a.z_off) {      // grouped: the tile list is built for 64-row tiles
     wt = 1;
-    g1 = dim3((a.N + 63) / 64, grouped_rows / 64 + groups, 1);
+    g1 = dim3((a.N + 63) / 64, grouped_rows / 64 + std::min(groups, grouped_rows), 1);
   } else {
     g1 = dim3((a.N + 63) / 64, (a.M + 63) / 64, nz);
     g2 = dim3((a.N + 127) / 128, (a.M + 127) / 128, nz);
@@ -2456,7 +2456,7 @@ int stack_create(const tgx_stack_desc* desc, const tgx_layer_desc* layers, int d
 
   const size_t W = (size_t)d.width, es = c->esz;
   int rc;
-  if ((rc = dev_alloc(c, &c->embed, (size_t)d.vocab * W * es)) || (rc = dev_alloc(c, &sm->final_norm, 2 * W))) return rc;      // (weight, and a bias where the norm has one)
+  if ((rc = stack_few_init(c)) || (rc = dev_alloc(c, &c->embed, (size_t)d.vocab * W * es)) || (rc = dev_alloc(c, &sm->final_norm, 2 * W))) return rc;      // (weight, and a bias where the norm has one)
   sm->missing.insert("embed"); sm->missing.insert("final.norm");
   sm->L.resize((size_t)d.layers);
   if (sandwich) return create_sandwich_layers(c, layers);
