@@ -53,3 +53,51 @@ def test_rows_of_a_step_in_half_storage(slots, dtype, bound):
     for i in range(0, slots, max(1, slots // 5)):
         want = both(one, t, seqs[i:i + 1])[0]
         assert np.abs(got[i] - want).max() / np.abs(want).max() < bound, (slots, dtype, i)
+
+
+# ---- prompts: the line kernels against the register-staged tiles ---------------------------------------------------------------------------
+# Both forms multiply the same two 16-bit terms of an activation by the same stored weights; only the order of fp32 sums differs (5e-7 measured per product, 1e-4 allowed
+# through two layers and a recurrence).  The wkv model caches nothing, so nothing rounds on the way; the expert model's cached latents may round to the other neighbour.
+def wkv_model(W, ff, dtype, T):
+    layers = [LayerDesc(mixer="wkv", heads=W // 64, kv_heads=W // 64, dim=64, vdim=64, decay_rank=64, mlp="dense", ff=ff) for _ in range(2)]
+    return StackDesc(family="vitudra", width=W, vocab=101, compute_dtype=dtype, max_seqs=1, max_ctx=T, budget_tokens=T, norm_eps=1e-5, residual_mult=0.5, layers=layers)
+
+
+def on_and_off(d, tensors, ids, want, options=()):
+    eng = SlotEngine(desc=d, tensors={k: np.asarray(v, np.float32) for k, v in tensors.items()})
+    for o in options:
+        eng.model.set_option(*o)
+    out = []
+    for on in (1, 0):
+        eng.model.set_option("stack.line", on)
+        out.append(eng.step([("p", ids, want)], ["p"]))
+    eng.close()
+    return out
+
+
+# (T 2177: 18 row tiles of 128, the last of one row; 4161: 256-row tiles, the last of 65; ff 1088 = 17 x 64: column tiles that end inside; width 320: five steps of K)
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("W,ff,T", [(320, 1088, 2177), (320, 1088, 4161), (256, 1024, 2048), (320, 64, 8200)])
+def test_prompt_products_of_a_model_that_caches_nothing(W, ff, T, dtype):
+    import vitudra_oracle as vo
+    d = wkv_model(W, ff, dtype, T)
+    rng = np.random.default_rng(T)
+    cfg = dict(width=W, vocab=101, layers=[dict(type="wkv", mixer=dict(heads=W // 64, dim=64), mlp=dict(ff=ff))] * 2)
+    t = vo.random_tensors(cfg, 3, decay_rank=64)
+    want = sorted({0, 1, 63, 64, 127, 128, 255, 256, T // 2, T - 66, T - 2, T - 1})
+    on, off = on_and_off(d, t, rng.integers(0, d.vocab, T), want)
+    assert np.isfinite(on).all() and np.abs(on - off).max() / np.abs(off).max() < 1e-4, (W, ff, T, dtype)
+    one, _ = on_and_off(d, t, rng.integers(0, d.vocab, T), want, [("act.round16", 1)])      # a single term: both forms round the same inputs, which differ in their last bits
+    assert np.isfinite(one).all()
+
+
+@pytest.mark.parametrize("dtype,bound", [("bf16", 2.0 ** -7), ("fp16", 2.0 ** -10)])
+@pytest.mark.parametrize("T,experts,top,ff", [(2100, 5, 2, 192), (4000, 3, 3, 1024), (1537, 9, 4, 320)])
+def test_prompt_products_of_experts(T, experts, top, ff, dtype, bound):
+    layers = [LayerDesc(heads=4, dim=64, vdim=64, kv_rank=128, scale=0.125, mlp="moe", experts=experts, top=top, ff=ff, limit=7.0) for _ in range(2)]
+    d = StackDesc(width=256, vocab=101, canon_taps=3, norm_groups=2, norm_eps=1e-6, max_seqs=1, max_ctx=T, budget_tokens=T, compute_dtype=dtype, layers=layers)
+    t = so.random_tensors(d, T)
+    on, off = on_and_off(d, t, np.random.default_rng(T).integers(0, d.vocab, T), [0, 127, 128, T // 2, T - 1])
+    # (a near tie of the router may send a token to another expert: the other rows hold)
+    rows = np.abs(on - off).max(1) / np.abs(off).max()
+    assert np.isfinite(on).all() and np.sort(rows)[-2] < bound, (T, dtype, rows)

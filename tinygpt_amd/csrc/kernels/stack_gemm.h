@@ -40,6 +40,9 @@ struct StackGemmArgs {
   int g_per_z;                                   //          one gate per batch member z (a head): sigmoid(G[row][g_col0 + z])
   const float* rw;             // SG_ROWSCALE: C = acc * rw[c row]
   int terms;                   // 16-bit storage: 2 = hi + lo, 1 = hi only
+  // stack_line.h: the activations, or the outputs, as lines of two 16-bit terms [row][K / 32][hi 32 | lo 32] in the place of A, or of C (nullptr: fp32)
+  const unsigned short* At; unsigned short* Ct;
+  int a_count;                 // gathered products (a_rows): rows of A
 };
 
 // an expert's activation: g = min(gate, limit), u = clamp(up, -limit, limit); g * sigmoid(1.702 g) * (u + 1)
@@ -67,17 +70,22 @@ __device__ __forceinline__ float gelu_tanh(float z) { return 0.5f * z * (1.0f + 
 // the product of a gated feed-forward's two halves: silu or (act SG_ACT_GELU_TANH) the tanh gelu of the gate
 __device__ __forceinline__ float gate_mul(const StackGemmArgs& a, float gate, float up) { return a.act == SG_ACT_GELU_TANH ? gelu_tanh(gate) * up : silu_mul(gate, up); }
 
-// one output of a product: the epilogue on the accumulated sum v (dual products: v of the first matrix, v2 of the second) of grouped / batched row m and column n
+// the epilogue on the accumulated sum v (dual products: v of the first matrix, v2 of the second) of grouped / batched row m, row crow and column n of C; old: what C holds (SG_ADD)
+template <int EPI>
+__device__ __forceinline__ float sg_value(const StackGemmArgs& a, int z, int m, size_t crow, int n, float v, float v2, float old) {
+  if constexpr (EPI == SG_STORE) return store_value(a, a.in_w ? v * a.in_w[a.in_rows[m]] : v, (size_t)z * a.c_zoff + n, n);
+  else if constexpr (EPI == SG_ADD) return fmaf(v, a.scale, old);
+  else if constexpr (EPI == SG_GATE) return v / (1.0f + expf(-a.G[crow * a.ldg + a.g_col0 + (a.g_per_z ? (size_t)z : (size_t)z * a.c_zoff + n)]));
+  else if constexpr (EPI == SG_EXPERT_ACT) return expert_act(v, v2, a.limit);
+  else if constexpr (EPI == SG_SILU_MUL) return gate_mul(a, v, v2);
+  else return v * a.rw[crow];
+}
+// one output of a product
 template <int EPI>
 __device__ __forceinline__ void sg_finish(const StackGemmArgs& a, int z, int m, int n, float v, float v2) {
   const size_t crow = a.c_rows ? (size_t)a.c_rows[m] : (size_t)m;
   float* cp = a.C + crow * a.ldc + (size_t)z * a.c_zoff + n;
-  if constexpr (EPI == SG_STORE) *cp = store_value(a, a.in_w ? v * a.in_w[a.in_rows[m]] : v, (size_t)z * a.c_zoff + n, n);
-  else if constexpr (EPI == SG_ADD) *cp = fmaf(v, a.scale, *cp);
-  else if constexpr (EPI == SG_GATE) *cp = v / (1.0f + expf(-a.G[crow * a.ldg + a.g_col0 + (a.g_per_z ? (size_t)z : (size_t)z * a.c_zoff + n)]));
-  else if constexpr (EPI == SG_EXPERT_ACT) *cp = expert_act(v, v2, a.limit);
-  else if constexpr (EPI == SG_SILU_MUL) *cp = gate_mul(a, v, v2);
-  else *cp = v * a.rw[crow];
+  *cp = sg_value<EPI>(a, z, m, crow, n, v, v2, EPI == SG_ADD ? *cp : 0.f);
 }
 
 template <int DT, int EPI, bool DUAL, int WT, bool VEC>

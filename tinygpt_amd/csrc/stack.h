@@ -128,6 +128,8 @@ struct StackModel {
   float* zr = nullptr;                 // [T][experts] router products
   float *selw = nullptr, *yh = nullptr, *yd = nullptr, *xn = nullptr, *lg = nullptr, *part = nullptr;
   size_t part_elems = 0;
+  unsigned short *terms = nullptr, *terms2 = nullptr;      // prompt products: the activations as lines of two 16-bit terms, and a feed-forward's hidden values (grown to the largest product seen)
+  size_t terms_elems = 0, terms2_elems = 0;
   int *sel = nullptr, *moe_off = nullptr, *perm = nullptr, *ptok = nullptr, *tile_e = nullptr, *tile_m0 = nullptr, *n_tiles = nullptr;
   int max_in = 0, max_hr = 0, max_hv = 0, max_top = 0, max_ff = 0, max_E = 0, max_rank = 0;
   int attn_split_min_keys = 2048;      // option attn.split_min: steps of few tokens split a sequence's keys between workgroups from this context on
@@ -137,6 +139,8 @@ struct StackModel {
   int mlstm_narrow = -1;               // option mlstm.narrow: the matrix-memory scan's columns per wave (1: eight, 0: sixteen, -1: by the step's entries and heads)
   int ssd_min = 64;                    // option ssd.min: portions from this many tokens on take the blocked form of the scalar-decay recurrence (0: never)
   int mix_groups = 0;                  // option attn.mix_groups: key / value heads per workgroup of the matrix-core sigmoid attention: 1; 2 where their accumulators fit, whatever the grid; 0: 2 while the halved grid fills the chip
+  std::set<const void*> lds_kernels;   // kernels that may take the whole LDS of a compute unit on this context's device
+  int line = 1;                        // option stack.line: 0 keeps prompts' products on the register-staged tiles
   int gemm_wt = 0;                     // option stack.gemm_wt: force the product's tile (1: 64 x 64, 2: 128 x 128); 0 = by the number of tiles
 };
 
@@ -147,10 +151,17 @@ void launch_gqa_mfma(tgx_ctx* c, const tgx::StepMeta& m, const tgx::GqaMfmaArgs&
 void launch_mix_mfma(tgx_ctx* c, const tgx::StepMeta& m, const tgx::MixMfmaArgs& a, dim3 grid);      // kernels/stack_mix_mfma.h
 size_t mix_mfma_wg_lds(int heads, int kv_heads);      // LDS bytes of one of its workgroups
 
+// stack.hip: lets a kernel take `bytes` of dynamic LDS (asked of the runtime once per kernel and context, and only beyond the 64 KB that every kernel has); false: launch_fault is set
+bool stack_allow_lds(tgx_ctx* c, const void* kernel, size_t bytes);
 // stack_few.hip
 namespace tgx { struct StackGemmArgs; }
-int stack_few_init(tgx_ctx* c);
 void launch_stack_few(tgx_ctx* c, const tgx::StackGemmArgs& a, int epi, int nz, int grouped_tiles, int dt);
+
+// stack_line.hip
+int stack_line_tile(const tgx_ctx* c, long long M, long long N, bool dual, int nz);      // 256 or 128 rows a tile; 0: the product is too small for such tiles
+int stack_line_tile_grouped(const tgx_ctx* c, long long pairs, int groups, long long N);
+void launch_split_terms(tgx_ctx* c, const float* a, long long lda, int rows, int cols, unsigned short* out);
+void launch_stack_line(tgx_ctx* c, const tgx::StackGemmArgs& g, int epi, int nz, int tile, int row_tiles, const unsigned short* terms, long long ldt);
 
 // stack_ssd.hip
 bool ssd_mfma_shapes_ok(int heads, int groups, int N, int E, long long ld);

@@ -85,9 +85,35 @@ constexpr int GROUPED_FEW_PAIRS = 128, GROUPED_FEW_ROWS = 16, FEW_ROWS_MAX = 64;
 // three to 64 and the grouped tiles (47 rows, 1024 x 3072: 25 us against 38 on 64-wide tiles)
 constexpr int GEMV_ROWS_MAX = 2;
 constexpr int FEW_COLS_ANY_ROWS = 64;      // a matrix of so few rows (the router's) takes the few-row kernel whatever the step's size: the 64-wide matrix-core tiles would stand mostly empty
-// (both products of the layer must be able to take it: their contraction lengths, the width and the expert width, in whole 8-element slices)
-int grouped_tile_rows(const tgx_ctx* c, int pairs, int width, int ff) {
-  return c->stack->gemv && pairs <= GROUPED_FEW_PAIRS && width % 8 == 0 && ff % 8 == 0 ? GROUPED_FEW_ROWS : 64;
+// workspace of the line kernels; false: no memory for it (the register-staged tiles need none)
+bool ensure_terms(tgx_ctx* c, unsigned short*& p, size_t& have, size_t elems) {
+  if (elems <= have) return true;
+  if (hipStreamSynchronize(c->stream) != hipSuccess) return false;
+  if (p) (void)hipFree(p);
+  p = nullptr; have = 0;
+  if (hipMalloc((void**)&p, elems * 2) != hipSuccess) { (void)hipGetLastError(); p = nullptr; return false; }
+  have = elems;
+  return true;
+}
+// tiles of the two grouped products of an expert layer (both must be able to take them: their contraction lengths are the width and the expert width).  np: (token, expert)
+// pairs, E: experts, up_n: columns of the first product (gate and up together)
+int grouped_tile_rows(tgx_ctx* c, int np, int width, int ff, int E, int T, int up_n) {
+  StackModel* sm = c->stack;
+  if (sm->gemv && np <= GROUPED_FEW_PAIRS && width % 8 == 0 && ff % 8 == 0) return GROUPED_FEW_ROWS;
+  if (sm->line && c->dt != tgx::DT_F32 && width % 64 == 0 && ff % 64 == 0 && E > 0) {
+    const int tile = stack_line_tile_grouped(c, np, E, up_n);
+    if (tile && ensure_terms(c, sm->terms, sm->terms_elems, (size_t)T * 2 * width) && ensure_terms(c, sm->terms2, sm->terms2_elems, (size_t)np * 2 * ff)) return tile;
+  }
+  return 64;
+}
+// whether a plain or batched product takes the line kernels, and on which tiles (0: no)
+int line_tile(const tgx_ctx* c, const tgx::StackGemmArgs& a, int epi, int nz, int dt) {
+  const StackModel* sm = c->stack;
+  if (!sm->line || sm->gemm_wt || dt == tgx::DT_F32 || a.z_off || a.K % 64 || a.ldb % 8 || a.b_zstride % 8 || (uintptr_t)a.B % 16 || (a.B2 && (uintptr_t)a.B2 % 16)) return 0;
+  if (!a.At && (a.lda % 4 || (uintptr_t)a.A % 16)) return 0;
+  if (nz > 1 && (a.a_zoff % 32 || a.K < 256)) return 0;      // (per-head products of one head's width: two or four steps of K do not fill the ring)
+  if (a.M <= FEW_ROWS_MAX || a.N <= FEW_COLS_ANY_ROWS) return 0;
+  return stack_line_tile(c, a.M, a.N, tgx::sg_dual(epi), nz);
 }
 
 // nz: batched products (blockIdx.z); grouped products pass the number of their rows and groups (the device-side tile list says how many tiles are real)
@@ -97,6 +123,16 @@ void launch_gemm(tgx_ctx* c, tgx::StackGemmArgs a, int epi, int nz, int grouped_
   if (a.M <= 0 && !a.z_off) return;
   if (a.N <= 0 || a.K <= 0) return;
   a.terms = c->act16 ? 1 : 2;
+  const int tile = a.z_off ? (grouped_tile >= 128 ? grouped_tile : 0) : line_tile(c, a, epi, nz, dt);
+  if (tile) {
+    const int cols = a.K + a.a_zoff * (nz - 1), rows = a.a_rows ? a.a_count : a.M;
+    if (!a.At && ensure_terms(c, c->stack->terms, c->stack->terms_elems, (size_t)rows * 2 * cols)) {
+      launch_split_terms(c, a.A, a.lda, rows, cols, c->stack->terms);
+      a.At = c->stack->terms;
+    }
+    if (a.At) { launch_stack_line(c, a, epi, nz, tile, a.z_off ? grouped_rows / tile + std::min(groups, grouped_rows) : (a.M + tile - 1) / tile, a.At, 2LL * cols); return; }
+    if (a.z_off) { c->launch_fault = "grouped product: no workspace for the tiles its plan was made for"; return; }
+  }
   const int kq = dt == tgx::DT_F32 ? 4 : 8;
   const bool vec = a.K % kq == 0 && a.ldb % kq == 0 && a.b_zstride % kq == 0 && a.lda % 4 == 0 && a.a_zoff % 4 == 0 && ((uintptr_t)a.A % 16 == 0) && ((uintptr_t)a.B % 16 == 0) &&
                    (!a.B2 || (uintptr_t)a.B2 % 16 == 0);
@@ -140,6 +176,23 @@ void launch_gemm(tgx_ctx* c, tgx::StackGemmArgs a, int epi, int nz, int grouped_
       case tgx::SG_SILU_MUL: launch_gemm_t<DT, tgx::SG_SILU_MUL, true>(c, a, g1, g2, wt, vec); break;
       default: if (dual) launch_gemm_t<DT, tgx::SG_EXPERT_ACT, true>(c, a, g1, g2, wt, vec); break;
     })
+}
+
+// a sublayer's last product: yd = A . W^T
+tgx::StackGemmArgs sublayer_product(const tgx_ctx* c, const float* A, int K, const ebyte* Wm, int T) {
+  const StackModel* sm = c->stack;
+  tgx::StackGemmArgs g{};
+  g.A = A; g.lda = K; g.B = Wm; g.ldb = K; g.C = sm->yd; g.ldc = sm->d.width; g.M = T; g.N = sm->d.width; g.K = K; g.scale = 1.f;
+  return g;
+}
+// the two products of a feed-forward, the second on the first one's outputs (up.C = down.A, row for row): where both take the line kernels the hidden values go from one to
+// the other as lines of terms, and their fp32 form is neither written nor read
+void launch_ff(tgx_ctx* c, tgx::StackGemmArgs up, int epi_up, tgx::StackGemmArgs down, int epi_down, int np = 0, int groups = 0, int tile = 64) {
+  StackModel* sm = c->stack;
+  const bool line = up.N == down.K && up.ldc == up.N && (up.z_off ? tile >= 128 : line_tile(c, up, epi_up, 1, c->dt) && line_tile(c, down, epi_down, 1, c->dt));
+  if (line && ensure_terms(c, sm->terms, sm->terms_elems, (size_t)(up.a_rows ? up.a_count : up.M) * 2 * up.K) && ensure_terms(c, sm->terms2, sm->terms2_elems, (size_t)up.M * 2 * up.N)) { up.Ct = sm->terms2; down.At = sm->terms2; }
+  launch_gemm(c, up, epi_up, 1, np, groups, tile);
+  launch_gemm(c, down, epi_down, 1, np, groups, tile);
 }
 
 template <int DT, bool SPLIT>
@@ -314,19 +367,19 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
       hipLaunchKernelGGL(tgx::router_topk_kernel, dim3(T), dim3(64), 0, c->stream, ra);
       const int np = T * top;
       tgx::MoePlanArgs pa{};
-      pa.sel = sm->sel; pa.n_pairs = np; pa.E = ld.experts; pa.top = top; pa.tile_m = grouped_tile_rows(c, np, W, ld.ff);
+      pa.sel = sm->sel; pa.n_pairs = np; pa.E = ld.experts; pa.top = top; pa.tile_m = grouped_tile_rows(c, np, W, ld.ff, ld.experts, T, 2 * ld.ff);
       pa.off = sm->moe_off; pa.perm = sm->perm; pa.tok = sm->ptok; pa.tile_e = sm->tile_e; pa.tile_m0 = sm->tile_m0; pa.n_tiles = sm->n_tiles;
       hipLaunchKernelGGL(tgx::moe_plan_kernel, dim3(1), dim3(1024), 0, c->stream, pa);
       // yh[n] = act(gate_e . a[tok(n)], up_e . a[tok(n)]) over the pairs grouped by expert
       g = tgx::StackGemmArgs{};
-      g.A = sm->a; g.lda = W; g.a_rows = sm->ptok; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff;
+      g.A = sm->a; g.lda = W; g.a_rows = sm->ptok; g.a_count = T; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff;
       g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = ld.ff; g.K = W; g.limit = ld.limit;
-      launch_gemm(c, g, tgx::SG_EXPERT_ACT, 1, np, ld.experts, pa.tile_m);
       // yd[pair] = router weight * (down_e . yh[n])
+      const tgx::StackGemmArgs gu = g;
       g = tgx::StackGemmArgs{};
       g.A = sm->yh; g.lda = ld.ff; g.B = w.w_down; g.ldb = ld.ff; g.b_zstride = (long long)W * ld.ff; g.C = sm->yd; g.ldc = W; g.c_rows = sm->perm;
       g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = W; g.K = ld.ff; g.rw = sm->selw;
-      launch_gemm(c, g, tgx::SG_ROWSCALE, 1, np, ld.experts, pa.tile_m);
+      launch_ff(c, gu, tgx::SG_EXPERT_ACT, g, tgx::SG_ROWSCALE, np, ld.experts, pa.tile_m);
     }
     tgx::CombineDepthArgs cd{};
     cd.x = sm->x; cd.y = sm->yd; cd.xs = sm->xs; cd.slot_stride = slot_stride; cd.dw = w.dwa; cd.W = W; cd.top = top; cd.n_res = li + 2;
@@ -540,26 +593,26 @@ void run_choice_experts(tgx_ctx* c, StackLayerW& w, const float* hin, int T) {
   const int np = T * top;
   if (ld.experts > 0) {
     tgx::MoePlanArgs pa{};
-    pa.sel = sm->sel; pa.n_pairs = np; pa.E = E; pa.top = top; pa.tile_m = grouped_tile_rows(c, np, W, ld.ff); pa.E_tiles = ld.experts;
+    pa.sel = sm->sel; pa.n_pairs = np; pa.E = E; pa.top = top; pa.tile_m = grouped_tile_rows(c, np, W, ld.ff, E, T, 2 * ld.ff); pa.E_tiles = ld.experts;
     pa.off = sm->moe_off; pa.perm = sm->perm; pa.tok = sm->ptok; pa.tile_e = sm->tile_e; pa.tile_m0 = sm->tile_m0; pa.n_tiles = sm->n_tiles;
     hipLaunchKernelGGL(tgx::moe_plan_kernel, dim3(1), dim3(1024), 0, c->stream, pa);
     g = tgx::StackGemmArgs{};
-    g.A = hin; g.lda = W; g.a_rows = sm->ptok; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff;
+    g.A = hin; g.lda = W; g.a_rows = sm->ptok; g.a_count = T; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff;
     g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = ld.ff; g.K = W;
-    launch_gemm(c, g, tgx::SG_SILU_MUL, 1, np, E, pa.tile_m);
+    const tgx::StackGemmArgs gu = g;
     g = tgx::StackGemmArgs{};
     g.A = sm->yh; g.lda = ld.ff; g.B = w.w_down; g.ldb = ld.ff; g.b_zstride = (long long)W * ld.ff; g.C = sm->yd; g.ldc = W; g.c_rows = sm->perm;
     g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = W; g.K = ld.ff; g.rw = sm->selw;
-    launch_gemm(c, g, tgx::SG_ROWSCALE, 1, np, E, pa.tile_m);
+    launch_ff(c, gu, tgx::SG_SILU_MUL, g, tgx::SG_ROWSCALE, np, E, pa.tile_m);
   }
   if (ld.shared_ff > 0) {
     float* hsh = sm->yh + (size_t)np * std::max(1, ld.ff);
     g = tgx::StackGemmArgs{};
     g.A = hin; g.lda = W; g.B = w.ws_gate; g.B2 = w.ws_up; g.ldb = W; g.C = hsh; g.ldc = ld.shared_ff; g.M = T; g.N = ld.shared_ff; g.K = W;
-    launch_gemm(c, g, tgx::SG_SILU_MUL, 1);
+    const tgx::StackGemmArgs gu = g;
     g = tgx::StackGemmArgs{};
     g.A = hsh; g.lda = ld.shared_ff; g.B = w.ws_down; g.ldb = ld.shared_ff; g.C = sm->ysh; g.ldc = W; g.M = T; g.N = W; g.K = ld.shared_ff; g.rw = sm->sgw;
-    launch_gemm(c, g, tgx::SG_ROWSCALE, 1);
+    launch_ff(c, gu, tgx::SG_SILU_MUL, g, tgx::SG_ROWSCALE);
   }
 }
 
@@ -598,12 +651,13 @@ int run_layers_sandwich(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_ke
 
 // ---- parallel-sublayer designs (Vitudra): per layer  h = norm(x);  x += mult * (mixer(h) + ff(h)).  Every sublayer's last product adds its share to the
 // stream in its epilogue (mult, and the half's weight in a parallel mixer, as the product's scale), so no combine launch is needed.
-void add_to_stream(tgx_ctx* c, const float* A, int K, const ebyte* Wm, int T, float scale) {
-  StackModel* sm = c->stack;
+tgx::StackGemmArgs to_stream(const tgx_ctx* c, const float* A, int K, const ebyte* Wm, int T, float scale) {
+  const StackModel* sm = c->stack;
   tgx::StackGemmArgs g{};
   g.A = A; g.lda = K; g.B = Wm; g.ldb = K; g.C = sm->x; g.ldc = sm->d.width; g.M = T; g.N = sm->d.width; g.K = K; g.scale = scale;
-  launch_gemm(c, g, tgx::SG_ADD, 1);
+  return g;
 }
+void add_to_stream(tgx_ctx* c, const float* A, int K, const ebyte* Wm, int T, float scale) { launch_gemm(c, to_stream(c, A, K, Wm, T, scale), tgx::SG_ADD, 1); }
 
 void launch_rec_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs& a, int kind, int S) {
   const dim3 grid(S, a.heads, (a.vdim + tgx::REC_COLS - 1) / tgx::REC_COLS);
@@ -722,8 +776,7 @@ int run_layers_joint(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys,
     if (ld.mlp == TGX_MLP_DENSE) {      // x += mult * down(silu(gate h) * (up h))
       tgx::StackGemmArgs g{};
       g.A = sm->a; g.lda = W; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.C = sm->yh; g.ldc = ld.ff; g.M = T; g.N = ld.ff; g.K = W;
-      launch_gemm(c, g, tgx::SG_SILU_MUL, 1);
-      add_to_stream(c, sm->yh, ld.ff, w.w_down, T, sm->d.residual_mult);
+      launch_ff(c, g, tgx::SG_SILU_MUL, to_stream(c, sm->yh, ld.ff, w.w_down, T, sm->d.residual_mult), tgx::SG_ADD);
     }
   }
   return TGX_OK;
@@ -909,10 +962,7 @@ void run_affine_ff(tgx_ctx* c, StackLayerW& w, int T) {
   tgx::StackGemmArgs g{};
   if (ld.mlp == TGX_MLP_DENSE) {      // down(act(up h))
     g.A = sm->a; g.lda = W; g.B = w.w_up; g.ldb = W; g.C = sm->yh; g.ldc = ld.ff; g.M = T; g.N = ld.ff; g.K = W; g.scale = 1.f; g.act = ld.ff_act == 1 ? tgx::SG_ACT_GELU : tgx::SG_ACT_NONE;
-    launch_gemm(c, g, tgx::SG_STORE, 1);
-    g = tgx::StackGemmArgs{};
-    g.A = sm->yh; g.lda = ld.ff; g.B = w.w_down; g.ldb = ld.ff; g.C = sm->yd; g.ldc = W; g.M = T; g.N = W; g.K = ld.ff; g.scale = 1.f;
-    launch_gemm(c, g, tgx::SG_STORE, 1);
+    launch_ff(c, g, tgx::SG_STORE, sublayer_product(c, sm->yh, ld.ff, w.w_down, T), tgx::SG_STORE);
     return;
   }
   const int E = ld.experts, top = ld.top, np = T * top;
@@ -924,25 +974,25 @@ void run_affine_ff(tgx_ctx* c, StackLayerW& w, int T) {
   ra.sigmoid_scores = ld.router_fn == 1; ra.group_top2 = ld.group_score == 1; ra.normalise = ld.router_norm;
   hipLaunchKernelGGL(tgx::router_group_kernel, dim3(T), dim3(64), 0, c->stream, ra);
   tgx::MoePlanArgs pa{};
-  pa.sel = sm->sel; pa.n_pairs = np; pa.E = E; pa.top = top; pa.tile_m = grouped_tile_rows(c, np, W, ld.ff); pa.E_tiles = E;
+  pa.sel = sm->sel; pa.n_pairs = np; pa.E = E; pa.top = top; pa.tile_m = grouped_tile_rows(c, np, W, ld.ff, E, T, 2 * ld.ff); pa.E_tiles = E;
   pa.off = sm->moe_off; pa.perm = sm->perm; pa.tok = sm->ptok; pa.tile_e = sm->tile_e; pa.tile_m0 = sm->tile_m0; pa.n_tiles = sm->n_tiles;
   hipLaunchKernelGGL(tgx::moe_plan_kernel, dim3(1), dim3(1024), 0, c->stream, pa);
   g = tgx::StackGemmArgs{};
-  g.A = sm->a; g.lda = W; g.a_rows = sm->ptok; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff;
+  g.A = sm->a; g.lda = W; g.a_rows = sm->ptok; g.a_count = T; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff;
   g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = ld.ff; g.K = W;
-  launch_gemm(c, g, tgx::SG_SILU_MUL, 1, np, E, pa.tile_m);
+  const tgx::StackGemmArgs gu = g;
   g = tgx::StackGemmArgs{};
   g.A = sm->yh; g.lda = ld.ff; g.B = w.w_down; g.ldb = ld.ff; g.b_zstride = (long long)W * ld.ff; g.C = sm->yd; g.ldc = W; g.c_rows = sm->perm;
   g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = W; g.K = ld.ff; g.rw = sm->selw;
-  launch_gemm(c, g, tgx::SG_ROWSCALE, 1, np, E, pa.tile_m);
+  launch_ff(c, gu, tgx::SG_SILU_MUL, g, tgx::SG_ROWSCALE, np, E, pa.tile_m);
   if (ld.shared_ff > 0) {      // the shared expert runs for every token, without a gate of its own
     float* hsh = sm->yh + (size_t)np * std::max(1, ld.ff);
     g = tgx::StackGemmArgs{};
     g.A = sm->a; g.lda = W; g.B = w.ws_gate; g.B2 = w.ws_up; g.ldb = W; g.C = hsh; g.ldc = ld.shared_ff; g.M = T; g.N = ld.shared_ff; g.K = W;
-    launch_gemm(c, g, tgx::SG_SILU_MUL, 1);
+    const tgx::StackGemmArgs gs = g;
     g = tgx::StackGemmArgs{};
     g.A = hsh; g.lda = ld.shared_ff; g.B = w.ws_down; g.ldb = ld.shared_ff; g.C = sm->ysh; g.ldc = W; g.M = T; g.N = W; g.K = ld.shared_ff; g.scale = 1.f;
-    launch_gemm(c, g, tgx::SG_STORE, 1);
+    launch_ff(c, gs, tgx::SG_SILU_MUL, g, tgx::SG_STORE);
   }
 }
 
@@ -1185,12 +1235,7 @@ int check_affine_desc(const tgx_stack_desc& d, const tgx_layer_desc* layers) {
 int pad4(int n) { return (n + 3) & ~3; }      // row strides of buffers whose rows are read in vectors of four
 
 // y = A . W^T into the sublayers' output rows
-void sublayer_out(tgx_ctx* c, const float* A, int K, const ebyte* Wm, int T) {
-  StackModel* sm = c->stack;
-  tgx::StackGemmArgs g{};
-  g.A = A; g.lda = K; g.B = Wm; g.ldb = K; g.C = sm->yd; g.ldc = sm->d.width; g.M = T; g.N = sm->d.width; g.K = K; g.scale = 1.f;
-  launch_gemm(c, g, tgx::SG_STORE, 1);
-}
+void sublayer_out(tgx_ctx* c, const float* A, int K, const ebyte* Wm, int T) { launch_gemm(c, sublayer_product(c, A, K, Wm, T), tgx::SG_STORE, 1); }
 void post_norm_add(tgx_ctx* c, const float* w, int T) {
   StackModel* sm = c->stack;
   tgx::PostNormArgs a{};
@@ -1302,8 +1347,7 @@ int run_layers_post(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys, 
     if (ld.mlp != TGX_MLP_DENSE) continue;
     tgx::StackGemmArgs g{};      // down(max(up x, 0)^2)
     g.A = sm->x; g.lda = W; g.B = w.w_up; g.ldb = W; g.C = sm->yh; g.ldc = ld.ff; g.M = T; g.N = ld.ff; g.K = W; g.scale = 1.f; g.act = tgx::SG_ACT_RELU2;
-    launch_gemm(c, g, tgx::SG_STORE, 1);
-    sublayer_out(c, sm->yh, ld.ff, w.w_down, T);
+    launch_ff(c, g, tgx::SG_STORE, sublayer_product(c, sm->yh, ld.ff, w.w_down, T), tgx::SG_STORE);
     post_norm_add(c, w.norm2, T);
   }
   return TGX_OK;
@@ -1586,7 +1630,7 @@ void run_channel_delta(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T
 // the shared expert's product takes the wide tiles by itself.)
 bool shared_rides(const tgx_ctx* c, const StackLayerW& w, int T) {
   const int np = T * (w.d.top + 1);
-  return w.shared_slot && np <= GROUPED_FEW_PAIRS && grouped_tile_rows(c, np, c->stack->d.width, w.d.ff) == GROUPED_FEW_ROWS;
+  return w.shared_slot && np <= GROUPED_FEW_PAIRS && c->stack->gemv && c->stack->d.width % 8 == 0 && w.d.ff % 8 == 0;      // (the plan's tiles of few rows)
 }
 // the feed-forward into yd (one row per token, or a row per choice for experts) and ysh (the shared expert's row, unless it rides among the choices)
 void run_hyper_ff(tgx_ctx* c, StackLayerW& w, int T) {
@@ -1596,8 +1640,7 @@ void run_hyper_ff(tgx_ctx* c, StackLayerW& w, int T) {
   tgx::StackGemmArgs g{};
   if (ld.mlp == TGX_MLP_DENSE) {      // down(gelu(gate h) * (up h))
     g.A = sm->a; g.lda = W; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.C = sm->yh; g.ldc = ld.ff; g.M = T; g.N = ld.ff; g.K = W; g.act = tgx::SG_ACT_GELU_TANH;
-    launch_gemm(c, g, tgx::SG_SILU_MUL, 1);
-    sublayer_out(c, sm->yh, ld.ff, w.w_down, T);
+    launch_ff(c, g, tgx::SG_SILU_MUL, sublayer_product(c, sm->yh, ld.ff, w.w_down, T), tgx::SG_STORE);
     return;
   }
   const int ride = shared_rides(c, w, T) ? 1 : 0, E = ld.experts + ride, top = ld.top + ride, np = T * top;
@@ -1607,26 +1650,26 @@ void run_hyper_ff(tgx_ctx* c, StackLayerW& w, int T) {
   ra.z = sm->zr; ra.ldz = ld.experts; ra.sel = sm->sel; ra.selw = sm->selw; ra.E = ld.experts; ra.top = ld.top; ra.shared = ride; ra.groups = 1; ra.keep = 1; ra.scale = 1.f; ra.sigmoid_scores = ld.router_fn == 1; ra.normalise = ld.router_norm;
   hipLaunchKernelGGL(tgx::router_group_kernel, dim3(T), dim3(64), 0, c->stream, ra);
   tgx::MoePlanArgs pa{};
-  pa.sel = sm->sel; pa.n_pairs = np; pa.E = E; pa.top = top; pa.tile_m = grouped_tile_rows(c, np, W, ld.ff); pa.E_tiles = E;
+  pa.sel = sm->sel; pa.n_pairs = np; pa.E = E; pa.top = top; pa.tile_m = grouped_tile_rows(c, np, W, ld.ff, E, T, ld.ff); pa.E_tiles = E;
   pa.off = sm->moe_off; pa.perm = sm->perm; pa.tok = sm->ptok; pa.tile_e = sm->tile_e; pa.tile_m0 = sm->tile_m0; pa.n_tiles = sm->n_tiles;
   hipLaunchKernelGGL(tgx::moe_plan_kernel, dim3(1), dim3(1024), 0, c->stream, pa);
   // yh[n] = max(up_e (w h), 0)^2 over the pairs grouped by expert: up_e is linear, so the weight multiplies its product
   g = tgx::StackGemmArgs{};
-  g.A = sm->a; g.lda = W; g.a_rows = sm->ptok; g.B = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff; g.scale = 1.f; g.act = tgx::SG_ACT_RELU2;
+  g.A = sm->a; g.lda = W; g.a_rows = sm->ptok; g.a_count = T; g.B = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff; g.scale = 1.f; g.act = tgx::SG_ACT_RELU2;
   g.in_w = sm->selw; g.in_rows = sm->perm; g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = ld.ff; g.K = W;
-  launch_gemm(c, g, tgx::SG_STORE, 1, np, E, pa.tile_m);
+  const tgx::StackGemmArgs gu = g;
   g = tgx::StackGemmArgs{};
   g.A = sm->yh; g.lda = ld.ff; g.B = w.w_down; g.ldb = ld.ff; g.b_zstride = (long long)W * ld.ff; g.C = sm->yd; g.ldc = W; g.c_rows = sm->perm; g.scale = 1.f;
   g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = W; g.K = ld.ff;
-  launch_gemm(c, g, tgx::SG_STORE, 1, np, E, pa.tile_m);
+  launch_ff(c, gu, tgx::SG_STORE, g, tgx::SG_STORE, np, E, pa.tile_m);
   if (ld.shared_ff > 0 && !ride) {
     float* hsh = sm->yh + (((size_t)np * ld.ff + 3) & ~(size_t)3);
     g = tgx::StackGemmArgs{};
     g.A = sm->a; g.lda = W; g.B = w.ws_up; g.ldb = W; g.C = hsh; g.ldc = ld.shared_ff; g.M = T; g.N = ld.shared_ff; g.K = W; g.scale = 1.f; g.act = tgx::SG_ACT_RELU2;
-    launch_gemm(c, g, tgx::SG_STORE, 1);
+    const tgx::StackGemmArgs gs = g;
     g = tgx::StackGemmArgs{};
     g.A = hsh; g.lda = ld.shared_ff; g.B = w.ws_down; g.ldb = ld.shared_ff; g.C = sm->ysh; g.ldc = W; g.M = T; g.N = W; g.K = ld.shared_ff; g.scale = 1.f;
-    launch_gemm(c, g, tgx::SG_STORE, 1);
+    launch_ff(c, gs, tgx::SG_STORE, g, tgx::SG_STORE);
   }
 }
 
@@ -2348,6 +2391,13 @@ int upload_joint(tgx_ctx* c, const char* name, const void* host, const int64_t* 
 }  // namespace
 
 // ================================================================================================================================================
+bool stack_allow_lds(tgx_ctx* c, const void* kernel, size_t bytes) {
+  if (bytes <= 64 * 1024 || c->stack->lds_kernels.count(kernel)) return true;
+  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) { (void)hipGetLastError(); c->launch_fault = "the device does not grant a product's LDS"; return false; }
+  c->stack->lds_kernels.insert(kernel);
+  return true;
+}
+
 int stack_create(const tgx_stack_desc* desc, const tgx_layer_desc* layers, int device_ordinal, tgx_ctx** out_ctx) {
   if (!desc || !layers || !out_ctx) return set_err(nullptr, TGX_ERR_INVALID, "null argument");
   *out_ctx = nullptr;
@@ -2456,7 +2506,7 @@ int stack_create(const tgx_stack_desc* desc, const tgx_layer_desc* layers, int d
 
   const size_t W = (size_t)d.width, es = c->esz;
   int rc;
-  if ((rc = stack_few_init(c)) || (rc = dev_alloc(c, &c->embed, (size_t)d.vocab * W * es)) || (rc = dev_alloc(c, &sm->final_norm, 2 * W))) return rc;      // (weight, and a bias where the norm has one)
+  if ((rc = dev_alloc(c, &c->embed, (size_t)d.vocab * W * es)) || (rc = dev_alloc(c, &sm->final_norm, 2 * W))) return rc;      // (weight, and a bias where the norm has one)
   sm->missing.insert("embed"); sm->missing.insert("final.norm");
   sm->L.resize((size_t)d.layers);
   if (sandwich) return create_sandwich_layers(c, layers);
@@ -2779,7 +2829,7 @@ void stack_destroy(tgx_ctx* c) {
   fr(sm->mixed); fr(sm->lora); fr(sm->rec_in);
   fr(sm->head); fr(sm->norm_g); fr(sm->a2); fr(sm->ytmp); fr(sm->ysh); fr(sm->sgw); fr(sm->vfirst); fr(sm->hs);
   fr(sm->final_norm); fr(sm->freq); fr(sm->tbl_dev); fr(sm->meta_dev); fr(sm->x); fr(sm->xs); fr(sm->a); fr(sm->proj); fr(sm->ql); fr(sm->lat); fr(sm->o); fr(sm->selw);
-  fr(sm->yh); fr(sm->yd); fr(sm->xn); fr(sm->lg); fr(sm->part); fr(sm->zr); fr(sm->sel); fr(sm->moe_off); fr(sm->perm); fr(sm->ptok); fr(sm->tile_e); fr(sm->tile_m0); fr(sm->n_tiles);
+  fr(sm->yh); fr(sm->yd); fr(sm->xn); fr(sm->lg); fr(sm->part); fr(sm->terms); fr(sm->terms2); fr(sm->zr); fr(sm->sel); fr(sm->moe_off); fr(sm->perm); fr(sm->ptok); fr(sm->tile_e); fr(sm->tile_m0); fr(sm->n_tiles);
   if (sm->tbl_host) (void)hipHostFree(sm->tbl_host);
   if (sm->meta_host) (void)hipHostFree(sm->meta_host);
   if (sm->meta_ev) (void)hipEventDestroy(sm->meta_ev);

@@ -20,7 +20,9 @@ void launch_few_mb(tgx_ctx* c, const tgx::StackGemmArgs& a, dim3 grid) {
   while (nw > 1 && nw > steps) nw /= 2;
   int depth = wgs >= 4LL * c->num_cus || nw >= steps ? 1 : 2;
   while (tgx::few_lds_bytes<DT, DUAL, MB>(nw, depth) > LDS_BYTES) { if (depth > 1) depth--; else nw /= 2; }
-  hipLaunchKernelGGL((tgx::stack_few_kernel<DT, EPI, DUAL, MB>), grid, dim3(64 * nw), (tgx::few_lds_bytes<DT, DUAL, MB>(nw, depth)), c->stream, a, depth);
+  const size_t lds = tgx::few_lds_bytes<DT, DUAL, MB>(nw, depth);
+  if (!stack_allow_lds(c, (const void*)&tgx::stack_few_kernel<DT, EPI, DUAL, MB>, lds)) return;
+  hipLaunchKernelGGL((tgx::stack_few_kernel<DT, EPI, DUAL, MB>), grid, dim3(64 * nw), lds, c->stream, a, depth);
 }
 template <int DT, int EPI, bool DUAL>
 void launch_few_t(tgx_ctx* c, const tgx::StackGemmArgs& a, dim3 grid, int mb) {
@@ -30,28 +32,7 @@ void launch_few_t(tgx_ctx* c, const tgx::StackGemmArgs& a, dim3 grid, int mb) {
     default: launch_few_mb<DT, EPI, DUAL, 4>(c, a, grid); break;
   }
 }
-template <int DT, int EPI, bool DUAL>
-hipError_t allow_lds_t() {
-  const void* k[3] = {(const void*)&tgx::stack_few_kernel<DT, EPI, DUAL, 1>, (const void*)&tgx::stack_few_kernel<DT, EPI, DUAL, 2>, (const void*)&tgx::stack_few_kernel<DT, EPI, DUAL, 4>};
-  for (const void* p : k) { const hipError_t e = hipFuncSetAttribute(p, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BYTES); if (e != hipSuccess) return e; }
-  return hipSuccess;
-}
-template <int DT>
-hipError_t allow_lds_dt() {
-  for (const hipError_t e : {allow_lds_t<DT, tgx::SG_STORE, false>(), allow_lds_t<DT, tgx::SG_ADD, false>(), allow_lds_t<DT, tgx::SG_GATE, false>(), allow_lds_t<DT, tgx::SG_ROWSCALE, false>(),
-                             allow_lds_t<DT, tgx::SG_SILU_MUL, true>(), allow_lds_t<DT, tgx::SG_EXPERT_ACT, true>()})
-    if (e != hipSuccess) return e;
-  return hipSuccess;
-}
 }  // namespace
-
-// once per context, on its device: a workgroup of these kernels may take the whole LDS of a compute unit
-int stack_few_init(tgx_ctx* c) {
-  HIP_OK(c, (allow_lds_dt<tgx::DT_F32>()));      // (the router's products are fp32 in every storage mode)
-  if (c->dt == tgx::DT_BF16) HIP_OK(c, (allow_lds_dt<tgx::DT_BF16>()));
-  if (c->dt == tgx::DT_F16) HIP_OK(c, (allow_lds_dt<tgx::DT_F16>()));
-  return TGX_OK;
-}
 
 // grouped_tiles: upper bound of the tile list of a grouped product (a.z_off), 0 for plain and batched ones
 void launch_stack_few(tgx_ctx* c, const tgx::StackGemmArgs& a, int epi, int nz, int grouped_tiles, int dt) {
