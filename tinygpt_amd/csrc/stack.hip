@@ -310,7 +310,7 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
       ma.q = sm->ql; ma.pool = w.pool; ma.poolT = w.poolT; ma.sink = w.sink; ma.out = sm->lat; ma.rank = R; ma.heads = H; ma.terms = c->act16 ? 1 : 2;
       const int tiles = (max_count * H + 31) / 32;
       int nsplit = 1;
-      if (max_keys >= sm->attn_split_min_keys && (long long)tiles * S < c->num_cus) {
+      if (max_keys >= sm->latent_split_min_keys && (long long)tiles * S < c->num_cus) {
         nsplit = (int)std::min<long long>(64, (2LL * c->num_cus) / ((long long)tiles * S));
         const int per = std::max(64, ((max_keys + nsplit - 1) / nsplit + 31) / 32 * 32);      // two key tiles per workgroup at least
         nsplit = (max_keys + per - 1) / per;
@@ -487,7 +487,7 @@ int run_gqa_core(tgx_ctx* c, const tgx::StepMeta& m, const GqaSpec& sp_, int T, 
   aa.mask_kind = sp.mask_kind; aa.mask_size = sp.mask_size; aa.softcap = sp.softcap; aa.dist_bias = sp.dist_bias;
   aa.sinks = sp.sinks; aa.dist_tab = sp.dist; aa.dist_len = sp.dist_len; aa.gate_per_head = sp.gate_per_head; aa.out_scale = sp.out_scale;
   int nsplit = 1;
-  if (span >= sm->gqa_split_min_keys && (long long)T * H < 2LL * c->num_cus) {      // few (token, head) pairs and a long context: the keys are divided between workgroups
+  if (span >= sm->gqa_lane_split_min_keys && (long long)T * H < 2LL * c->num_cus) {      // few (token, head) pairs and a long context: the keys are divided between workgroups
     nsplit = (int)std::min<long long>(64, (4LL * c->num_cus) / ((long long)T * H));
     const int per = std::max(256, ((span + nsplit - 1) / nsplit + 63) / 64 * 64);
     nsplit = (span + per - 1) / per;
@@ -910,7 +910,7 @@ int run_affine_latent(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, const 
     ma.q = sm->ql; ma.pool = run.pool; ma.poolT = run.poolT; ma.sink = nullptr; ma.out = sm->lat; ma.rank = RR; ma.heads = H; ma.terms = c->act16 ? 1 : 2;
     ma.mask_kind = ld.mask_kind; ma.mask_size = ld.mask_size;
     const int tiles = (max_count * H + 31) / 32;
-    if (span >= std::min(sm->attn_split_min_keys, 256) && (long long)tiles * S < c->num_cus) {
+    if (span >= sm->latent_split_min_keys && (long long)tiles * S < c->num_cus) {
       nsplit = (int)std::min<long long>(64, (2LL * c->num_cus) / ((long long)tiles * S));
       const int per = std::max(64, ((span + nsplit - 1) / nsplit + 31) / 32 * 32);      // two key tiles per workgroup at least
       nsplit = (span + per - 1) / per;
