@@ -101,3 +101,21 @@ def test_prompt_products_of_experts(T, experts, top, ff, dtype, bound):
     # (a near tie of the router may send a token to another expert: the other rows hold)
     rows = np.abs(on - off).max(1) / np.abs(off).max()
     assert np.isfinite(on).all() and np.sort(rows)[-2] < bound, (T, dtype, rows)
+
+
+@pytest.mark.parametrize("vocab", [53, 96, 1028, 1030])
+def test_wanted_logits_reach_their_slots(vocab):
+    """a step's last wanted logits are its slots' current logits (bit for bit) and their argmax is what the greedy pick starts from; slots whose last place is not wanted keep theirs"""
+    d = StackDesc(width=72, vocab=vocab, canon_taps=2, norm_groups=2, norm_eps=1e-6, max_seqs=5, max_ctx=64, budget_tokens=320, compute_dtype="fp32",
+                  layers=[LayerDesc(heads=2, dim=8, vdim=8, kv_rank=8, scale=0.35, mlp=None)])
+    eng = SlotEngine(desc=d, tensors={k: v.astype(np.float32) for k, v in so.random_tensors(d, vocab).items()})
+    ids = np.random.default_rng(vocab).integers(0, vocab, 64)
+    first = eng.step([(i, ids[5 * i:5 * i + 3 + i], [2 + i]) for i in range(4)])
+    slot = [eng.slot_of[i] for i in range(4)]
+    assert (eng.model.logits(rounded=False)[slot] == first).all()
+    assert [eng.model.sample_row(s) for s in slot] == first.argmax(1).tolist()
+    second = eng.step([(2, ids[:3], [0, 2]), (0, ids[3:5], [0]), (3, ids[5:6], [0])])      # request 0's last place is not wanted
+    now = eng.model.logits(rounded=False)
+    assert (now[slot[2]] == second[1]).all() and (now[slot[3]] == second[3]).all() and (now[slot[0]] == first[0]).all() and (now[slot[1]] == first[1]).all()
+    assert eng.model.sample_row(slot[2]) == int(second[1].argmax()) and eng.model.sample_row(slot[3]) == int(second[3].argmax())
+    eng.close()

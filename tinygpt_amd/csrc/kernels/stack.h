@@ -441,4 +441,42 @@ __global__ void stack_advance_kernel(int* tok_pos, int* ent_par, int* tok_par, i
   if (i < S) { tok_pos[i] += 1; ent_par[i] ^= 1; tok_par[i] ^= 1; }
 }
 
+// ---- a step's wanted logits into their slots: row i of src (nullptr: already in the slot) becomes the current logits of slot rows[i] (-1: of none), and the per-workgroup
+// argmax partials that the greedy pick and the sampler start from are left beside it, n_part of them (those without a workgroup of their own take the reduction's identity).
+// One launch for all rows: a copy and an argmax launch each were 16 x (3 + 3) us of a 1 ms step of sixteen requests.
+__global__ __launch_bounds__(256) void slot_logits_kernel(const float* src, const int* rows, float* slots, int V, float* part_val, int* part_idx, int n_part) {
+  __shared__ float sv[4];
+  __shared__ int si[4];
+  const int row = rows[blockIdx.y];
+  if (row < 0) return;
+  float* dst = slots + (size_t)row * V;
+  const float* lg = src ? src + (size_t)blockIdx.y * V : dst;
+  float bv = -INFINITY; int bi = 0x7fffffff;
+  auto take = [&](float v, int i) { if (v > bv || (v == bv && i < bi)) { bv = v; bi = i; } };
+  if ((V & 3) == 0)
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < (V >> 2); i += gridDim.x * 256) {
+      const f32x4 v = reinterpret_cast<const f32x4*>(lg)[i];
+      if (src) reinterpret_cast<f32x4*>(dst)[i] = v;
+#pragma unroll
+      for (int j = 0; j < 4; j++) take(v[j], 4 * i + j);
+    }
+  else
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < V; i += gridDim.x * 256) {
+      const float v = lg[i];
+      if (src) dst[i] = v;
+      take(v, i);
+    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) { const float v = __shfl_xor(bv, o, 64); const int i = __shfl_xor(bi, o, 64); take(v, i); }
+  if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = bv; si[threadIdx.x >> 6] = bi; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 4; w++) take(sv[w], si[w]);
+    part_val[(size_t)row * n_part + blockIdx.x] = bv; part_idx[(size_t)row * n_part + blockIdx.x] = bi;
+  }
+  for (int p = (int)gridDim.x + (int)blockIdx.x * 256 + (int)threadIdx.x; p < n_part; p += (int)gridDim.x * 256) {
+    part_val[(size_t)row * n_part + p] = -INFINITY; part_idx[(size_t)row * n_part + p] = 0x7fffffff;
+  }
+}
+
 }  // namespace tgx

@@ -2044,6 +2044,12 @@ void run_logits(tgx_ctx* c, const int* want_dev, int nw, float* C, const int* c_
   launch_gemm(c, g, tgx::SG_STORE, 1);
 }
 
+// n rows of logits into the slots rows_dev names, with their argmax partials (src nullptr: the logits stand there already)
+void launch_slot_logits(tgx_ctx* c, const float* src, const int* rows_dev, int n) {
+  const int V = c->d.vocab, gx = std::min(c->lm_grid, std::max(1, (V / 4 + 255) / 256));
+  hipLaunchKernelGGL(tgx::slot_logits_kernel, dim3(gx, n), dim3(256), 0, c->stream, src, rows_dev, c->slab_logits, V, c->slab_part_val, c->slab_part_idx, c->lm_grid);
+}
+
 // pages for `tokens` tokens of a slot; the caller has checked that enough are free
 void assign_pages(StackModel* sm, int row, long long tokens) {
   const int need = (int)((tokens + sm->page - 1) / sm->page);
@@ -2893,22 +2899,17 @@ int stack_step(tgx_ctx* c, int S, const int32_t* rows, const int32_t* counts, co
     }
   }
   for (int i = 0; i < n_want; i++) {
-    hp.want[i] = want[i]; hp.want_row[i] = 0;
+    hp.want[i] = want[i]; hp.want_row[i] = -1;
     for (int e = 0; e < S; e++) if (want[i] == hp.ent_start[e] + counts[e] - 1) last_want[(size_t)e] = i;
   }
+  bool slots = false;      // the slots' current logits: what tgx_sample_row / tgx_read_logits see
+  for (int e = 0; e < S; e++) if (last_want[(size_t)e] >= 0) { hp.want_row[last_want[(size_t)e]] = rows[e]; slots = true; }
   if ((rc = push_tables(c)) || (rc = push_meta(c, hp.n))) return rc;
   if ((rc = run_layers(c, dp, (int)T, S, max_keys, max_count))) return rc;
   if (n_want > 0) {
     run_logits(c, dp.want, n_want, sm->lg, nullptr);
+    if (slots) { launch_slot_logits(c, sm->lg, dp.want_row, n_want); c->have_logits = true; }
     HIP_OK(c, hipMemcpyAsync(out_logits, sm->lg, (size_t)n_want * d.vocab * 4, hipMemcpyDeviceToHost, c->stream));
-  }
-  for (int e = 0; e < S; e++) {
-    const int r = rows[e];
-    if (last_want[(size_t)e] >= 0) {      // the slot's current logits: what tgx_sample_row / tgx_read_logits see
-      HIP_OK(c, hipMemcpyAsync(c->rows[(size_t)r].logits, sm->lg + (size_t)last_want[(size_t)e] * d.vocab, (size_t)d.vocab * 4, hipMemcpyDeviceToDevice, c->stream));
-      launch_argmax_partials(c, c->rows[(size_t)r].logits, d.vocab, c->rows[(size_t)r].part_val, c->rows[(size_t)r].part_idx);
-      c->have_logits = true;
-    }
   }
   HIP_OK(c, hipGetLastError());
   HIP_OK(c, hipStreamSynchronize(c->stream));
@@ -2968,7 +2969,7 @@ int stack_decode(tgx_ctx* c, const tgx_sampler_cfg& cfg, uint64_t seed, int n) {
     hipLaunchKernelGGL(tgx::stack_gather_tok_kernel, dim3((S + 63) / 64), dim3(64), 0, c->stream, dp.tok_id, dp.ent_row, c->slab_tok, S);
     if ((rc = run_layers(c, dp, S, S, max_keys + s + 1, 1))) return rc;
     run_logits(c, dp.want, S, c->slab_logits, dp.want_row);
-    for (int r : live) launch_argmax_partials(c, c->rows[(size_t)r].logits, d.vocab, c->rows[(size_t)r].part_val, c->rows[(size_t)r].part_idx);
+    launch_slot_logits(c, nullptr, dp.want_row, S);
     launch_sample(c, 0, c->batch, cfg, /*advance_pos=*/true, /*log_step=*/true);
     hipLaunchKernelGGL(tgx::stack_advance_kernel, dim3((S + 63) / 64), dim3(64), 0, c->stream, dp.tok_pos, dp.ent_par, dp.tok_par, S);
     c->steps_issued++;
