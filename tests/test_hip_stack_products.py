@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import stack_oracle as so
+import test_hip_vitudra as tv
 from tinygpt_amd.desc import LayerDesc, StackDesc
 from tinygpt_amd.serving import SlotEngine
 
@@ -119,3 +120,19 @@ def test_wanted_logits_reach_their_slots(vocab):
     assert (now[slot[2]] == second[1]).all() and (now[slot[3]] == second[3]).all() and (now[slot[0]] == first[0]).all() and (now[slot[1]] == first[1]).all()
     assert eng.model.sample_row(slot[2]) == int(second[1].argmax()) and eng.model.sample_row(slot[3]) == int(second[3].argmax())
     eng.close()
+
+
+# ---- the recurrences' scan: sixteen row groups (few workgroups, rows in vectors of four), eight, and rows of any length number by number; 64 rows a group and their
+# remainders.  fp32 storage against the plain oracle: fp32 sums over at most 196 rows and 64 steps; 1e-4 of the largest logit as in the design's own tests.
+@pytest.mark.parametrize("dim", [4, 12, 36, 60, 64, 68, 100, 128, 132, 196, 6, 70, 129])
+@pytest.mark.parametrize("entries", [1, 40])
+def test_scan_of_the_recurrences(dim, entries):
+    cfg = tv.config([tv.wkv(heads=2, dim=dim), tv.par(right={"heads": 4, "kv_heads": 2, "dim": dim, "vdim": 36})], width=20)
+    eng, w = tv.engine(cfg, seed=dim, max_seqs=entries, max_ctx=128, budget_tokens=64 * entries)
+    seqs = [tv.tokens(cfg, 64 - i, seed=i) for i in range(entries)]
+    got = [eng.step([(i, s[:24], [23]) for i, s in enumerate(seqs)]), eng.step([(i, s[24:], [len(s) - 25]) for i, s in enumerate(seqs)])]
+    eng.close()
+    for i in {0, entries // 2}:
+        want = tv.want_of(cfg, w, seqs[i])
+        for at, part in ((23, got[0]), (-1, got[1])):
+            assert np.abs(part[i] - want[at]).max() / np.abs(want).max() < 1e-4, (dim, entries, i, at)

@@ -116,10 +116,14 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(StepMeta m, DeltaPrepAr
   if ((int)threadIdx.x < n) o[c0 + threadIdx.x] = mine * r;
 }
 
-// ---- the recurrences.  One workgroup per (entry, head, 32 value columns) walks the entry's tokens in order, TB at a time: the block's per-key-channel
+// ---- the recurrences.  One workgroup per (entry, head, 256 / RG value columns) walks the entry's tokens in order, TB at a time: the block's per-key-channel
 // inputs (up to three vectors of `dim`) and the workgroup's value columns are staged in LDS (the next block's travel in registers meanwhile), then every
-// lane updates its DPER rows of its column with no barrier inside the block: a wave owns 8 columns, its lanes = 8 columns x 8 row groups (the row groups
-// of a column are adjacent lanes), 8 DPER >= dim.  Sums over the key channels cross the row groups on the lane crossbar.
+// lane updates its DPER rows of its column with no barrier inside the block: a wave's lanes = 64 / RG columns x RG row groups (the row groups of a column are
+// adjacent lanes), RG DPER >= dim.  Sums over the key channels cross the row groups on the lane crossbar.
+// What bounds a prompt is the instructions that one wave issues per token (64 multiply-adds and some fifty others for the delta rule at eight groups of sixteen rows; with the
+// stores, crossbar steps, staging and LDS reads taken out the multiply-adds alone are 345 of 630 us for 2048 tokens).  Sixteen groups halve a lane's rows and double the workgroups,
+// which is right while the step leaves compute units idle; eight issue fewer instructions in all.  2048 tokens, delta rule of 16 heads of 128 x 128: 632 us at
+// eight row groups staged number by number, 578 staged in vectors of four, 469 at sixteen; channel decays 688 / 604 / 505, wkv of 32 heads of 64 x 64 419 / 409 / 330.
 enum { REC_WKV = 0, REC_DELTA = 1, REC_SSD = 2, REC_CDELTA = 3 };
 struct RecScanArgs {
   const float* a; long long lda;     // per token and key head [dim]: the read vector (wkv: r, delta: q, ssd: C)
@@ -134,11 +138,11 @@ struct RecScanArgs {
   float* out; long long ldo;         // [T][heads * vdim]
   int heads, kv_heads, dim, vdim;
 };
-constexpr int REC_RG = 8, REC_COLS = 4 * (64 / REC_RG);      // row groups per column; columns per workgroup
-template <int DPER, int KIND>
+constexpr int rec_cols(int rg) { return 4 * (64 / rg); }      // columns per workgroup
+template <int DPER, int KIND, int RG, bool VEC>
 __global__ __launch_bounds__(256) void rec_scan_kernel(StepMeta m, RecScanArgs a) {
-  constexpr int RG = REC_RG, CW = 64 / RG, CB = REC_COLS, LP = DPER + 4, DP = RG * DPER, TB = DP <= 128 ? 16 : 8;      // LP: a row group's LDS stride (the groups' reads fall into different banks)
-  constexpr int NQ = TB * DP / 256, NV = (TB * CB + 255) / 256, NA = KIND == REC_WKV || KIND == REC_CDELTA ? 3 : 2;
+  constexpr int CW = 64 / RG, CB = rec_cols(RG), LP = RG == 16 && DPER == 4 ? 4 : DPER + 4, DP = RG * DPER, TB = DP <= 128 ? 16 : 8;      // LP: a row group's LDS stride (the groups' reads fall into different banks)
+  constexpr int Q4 = TB * DP / 4, NQ = (Q4 + 255) / 256, NV = (TB * CB + 255) / 256, NA = KIND == REC_WKV || KIND == REC_CDELTA ? 3 : 2;
   __shared__ __attribute__((aligned(16))) float s_in[NA][TB][RG * LP];      // [0]: the read vector, [1]: k, [2]: the decay
   __shared__ float s_v[TB][CB], s_b[TB], s_g[TB];
   const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, rg = lane % RG, cl = lane / RG;
@@ -158,16 +162,25 @@ __global__ __launch_bounds__(256) void rec_scan_kernel(StepMeta m, RecScanArgs a
   }
   const float* src[3] = {a.a, a.k, a.w};
   const long long lds[3] = {a.lda, a.ldk, a.ldw};
-  float rin[NA][NQ], rv[NV], rb = 0.f, rgt = 0.f;
+  f32x4 rin[NA][NQ];
+  float rv[NV], rb = 0.f, rgt = 0.f;
   auto fetch = [&](int t0) {
     const int nb = min(TB, cnt - t0);
 #pragma unroll
-    for (int u = 0; u < NQ; u++) {
-      const int i = tid + 256 * u, t = i / DP, d = i - t * DP;
-      const bool on = t < nb && d < a.dim;
-      const size_t tok = (size_t)(start + t0 + min(t, nb - 1));
+    for (int u = 0; u < NQ; u++) {      // (rows past the entry's end repeat its last one and are never used)
+      const int i = tid + 256 * u, t = min(i / (DP / 4), TB - 1), d = 4 * (i % (DP / 4));
+      const size_t tok = (size_t)(start + min(t0 + t, cnt - 1));
 #pragma unroll
-      for (int s = 0; s < NA; s++) rin[s][u] = on ? src[s][tok * lds[s] + (size_t)(KIND == REC_CDELTA && s == 2 ? h : kh) * a.dim + d] : 0.f;
+      for (int s = 0; s < NA; s++) {
+        const float* p = src[s] + tok * lds[s] + (size_t)(KIND == REC_CDELTA && s == 2 ? h : kh) * a.dim;
+        if constexpr (VEC) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(p + min(d, a.dim - 4));
+#pragma unroll
+          for (int c = 0; c < 4; c++) rin[s][u][c] = d < a.dim ? v[c] : 0.f;
+        } else
+#pragma unroll
+          for (int c = 0; c < 4; c++) { const float v = p[min(d + c, a.dim - 1)]; rin[s][u][c] = d + c < a.dim ? v : 0.f; }
+      }
     }
 #pragma unroll
     for (int u = 0; u < NV; u++) {
@@ -186,9 +199,9 @@ __global__ __launch_bounds__(256) void rec_scan_kernel(StepMeta m, RecScanArgs a
     __syncthreads();                                       // the block before has been read
 #pragma unroll
     for (int u = 0; u < NQ; u++) {
-      const int i = tid + 256 * u, t = i / DP, d = i - t * DP, at = (d / DPER) * LP + d % DPER;
+      const int i = tid + 256 * u, t = i / (DP / 4), d = 4 * (i - t * (DP / 4)), at = (d / DPER) * LP + d % DPER;
 #pragma unroll
-      for (int s = 0; s < NA; s++) s_in[s][t][at] = rin[s][u];
+      for (int s = 0; s < NA; s++) if (i < Q4) *reinterpret_cast<f32x4*>(&s_in[s][t][at]) = rin[s][u];
     }
 #pragma unroll
     for (int u = 0; u < NV; u++) { const int i = tid + 256 * u; if (i < TB * CB) s_v[i / CB][i % CB] = rv[u]; }

@@ -660,14 +660,25 @@ tgx::StackGemmArgs to_stream(const tgx_ctx* c, const float* A, int K, const ebyt
 void add_to_stream(tgx_ctx* c, const float* A, int K, const ebyte* Wm, int T, float scale) { launch_gemm(c, to_stream(c, A, K, Wm, T, scale), tgx::SG_ADD, 1); }
 
 void launch_rec_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs& a, int kind, int S) {
-  const dim3 grid(S, a.heads, (a.vdim + tgx::REC_COLS - 1) / tgx::REC_COLS);
-  const int dper = (a.dim + tgx::REC_RG - 1) / tgx::REC_RG;      // rows per lane
+  const bool vec = a.dim % 4 == 0 && a.lda % 4 == 0 && a.ldk % 4 == 0 && (uintptr_t)a.a % 16 == 0 && (uintptr_t)a.k % 16 == 0 && (!a.w || (a.ldw % 4 == 0 && (uintptr_t)a.w % 16 == 0));
+  // sixteen row groups per column while their workgroups, of sixteen columns, leave a compute unit with two at most: one prompt of 16 heads of 128 (kernels/stack_rec.h), a few
+  // requests; a full chip issues fewer instructions with eight
+  auto cols = [&](int rg) { return (a.vdim + tgx::rec_cols(rg) - 1) / tgx::rec_cols(rg); };
+  const bool wide = vec && a.dim <= 256 && (long long)S * a.heads * cols(16) <= 2LL * c->num_cus;
+  const int rg = wide ? 16 : 8, dper = (a.dim + rg - 1) / rg;      // rows per lane
+  const dim3 grid(S, a.heads, cols(rg));
   auto go = [&](auto K) {
     constexpr int KIND = decltype(K)::value;
-    if (dper <= 4) hipLaunchKernelGGL((tgx::rec_scan_kernel<4, KIND>), grid, dim3(256), 0, c->stream, m, a);
-    else if (dper <= 8) hipLaunchKernelGGL((tgx::rec_scan_kernel<8, KIND>), grid, dim3(256), 0, c->stream, m, a);
-    else if (dper <= 16) hipLaunchKernelGGL((tgx::rec_scan_kernel<16, KIND>), grid, dim3(256), 0, c->stream, m, a);
-    else hipLaunchKernelGGL((tgx::rec_scan_kernel<32, KIND>), grid, dim3(256), 0, c->stream, m, a);
+    auto rows = [&](auto D) {
+      constexpr int DPER = decltype(D)::value;
+      if constexpr (DPER <= 16) if (wide) { hipLaunchKernelGGL((tgx::rec_scan_kernel<DPER, KIND, 16, true>), grid, dim3(256), 0, c->stream, m, a); return; }
+      if (vec) hipLaunchKernelGGL((tgx::rec_scan_kernel<DPER, KIND, 8, true>), grid, dim3(256), 0, c->stream, m, a);
+      else hipLaunchKernelGGL((tgx::rec_scan_kernel<DPER, KIND, 8, false>), grid, dim3(256), 0, c->stream, m, a);
+    };
+    if (dper <= 4) rows(std::integral_constant<int, 4>{});
+    else if (dper <= 8) rows(std::integral_constant<int, 8>{});
+    else if (dper <= 16) rows(std::integral_constant<int, 16>{});
+    else rows(std::integral_constant<int, 32>{});
   };
   if (kind == tgx::REC_WKV) go(std::integral_constant<int, tgx::REC_WKV>{});
   else if (kind == tgx::REC_CDELTA) go(std::integral_constant<int, tgx::REC_CDELTA>{});
