@@ -487,17 +487,19 @@ __global__ __launch_bounds__(256) void mlstm_scan_kernel(StepMeta m, MlstmArgs a
 
 // out[t][h][c] = hs / sqrt(mean_c(hs^2) + eps) * w[h * w_hstride + c] * gate, gate = sigmoid(z) or silu(z) of the pre-activation z (w_hstride 0: one
 // weight vector for all heads; w nullptr: none).  One wave per (token, head): the seam behind every recurrent mixer (mLSTM, wkv, gated delta rule, retention).
-struct HeadNormGateArgs { const float* hs; long long ldh; const float* w; int w_hstride; const float* gate; long long ldg; int silu_gate; float* out; long long ldo; int vdim; float eps; };
+struct HeadNormGateArgs { const float* hs; long long ldh; const float* w; int w_hstride; const float* gate; long long ldg; int silu_gate; float* out; long long ldo; int vdim; float eps;
+                          const float* norm; long long ldnorm; const float* floor; long long ldfloor; float scale; };      // norm: hs enters as hs scale / (max(|norm scale|, floor) + 1e-6), both per token and head
 __global__ __launch_bounds__(64) void head_norm_gate_kernel(HeadNormGateArgs a) {
   const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
   const float* r = a.hs + (size_t)t * a.ldh + (size_t)h * a.vdim;
+  const float f = a.norm ? a.scale / (fmaxf(fabsf(a.norm[(size_t)t * a.ldnorm + h] * a.scale), a.floor[(size_t)t * a.ldfloor + h]) + 1e-6f) : 1.f;
   float ss = 0.f;
-  for (int c = lane; c < a.vdim; c += 64) ss = fmaf(r[c], r[c], ss);
+  for (int c = lane; c < a.vdim; c += 64) { const float v = r[c] * f; ss = fmaf(v, v, ss); }
   ss = wave_sum(ss);
   const float rinv = 1.0f / sqrtf(ss / (float)a.vdim + a.eps);
   for (int c = lane; c < a.vdim; c += 64) {
     const float g = a.gate[(size_t)t * a.ldg + (size_t)h * a.vdim + c], sg = 1.0f / (1.0f + expf(-g));
-    a.out[(size_t)t * a.ldo + (size_t)h * a.vdim + c] = r[c] * rinv * (a.w ? a.w[(size_t)h * a.w_hstride + c] : 1.0f) * (a.silu_gate ? g * sg : sg);
+    a.out[(size_t)t * a.ldo + (size_t)h * a.vdim + c] = r[c] * f * rinv * (a.w ? a.w[(size_t)h * a.w_hstride + c] : 1.0f) * (a.silu_gate ? g * sg : sg);
   }
 }
 

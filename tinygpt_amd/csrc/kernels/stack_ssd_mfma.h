@@ -14,13 +14,18 @@ namespace tgx {
 
 constexpr int SSD_BLOCK = 64;
 struct SsdArgs {
-  const float* row; long long ld;      // per token [x (heads E) | B (groups N) | C (groups N) | dt (heads) | decay (heads) | log decay (heads)]
-  int heads, groups, N, E;             // N and heads E multiples of 4
+  const float* row; long long ld;      // per token x (heads E), B and C (groups N each) from columns x0, b0 and c0
+  int x0, b0, c0;                      // b0 and c0 multiples of 4
+  const float* gates; long long ldgate;      // per token and head: dt from column dt_col, the logarithm of the decay from column log_col
+  int dt_col, log_col;
+  int heads, groups, N, E;             // N a multiple of 4
   float* gram;                         // [blocks][groups][64][64]
-  const float* fixed; float dt0;       // [2][heads] decays and their logarithms that hold for every token, with dt0 as every token's dt (the rows then end behind C; nullptr: per token)
+  const float* fixed; float dt0;       // [2][heads] decays and their logarithms that hold for every token, with dt0 as every token's dt (nullptr: per token, from gates)
   const float* skip;                   // [heads] (nullptr: none)
   float* S;                            // [slots][heads][N][E]
   float* out; long long ldo;           // [T][heads E]
+  float* norm_S; size_t norm_buf;      // a second state N_t = g_t N_(t-1) + dt_t B_t, the sum that a matrix memory divides by: [2][slots][heads][N], norm_buf between the two (nullptr: none)
+  float* norm_out; long long ldn;      // N_t . C_t: [T][heads]
 };
 // the first block of an entry in `gram`: entries never share a block
 __device__ __forceinline__ int ssd_first_block(int start, int e) { return start / SSD_BLOCK + e; }
@@ -35,8 +40,8 @@ __global__ __launch_bounds__(256) void ssd_gram_kernel(StepMeta m, SsdArgs a) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, half = lane >> 5, l31 = lane & 31, it = wv >> 1, jt = wv & 1;
   if (jt > it) return;
   const int i = b * Q + 32 * it + l31, j = b * Q + 32 * jt + l31;
-  const float* cr = a.row + (size_t)(start + min(i, cnt - 1)) * a.ld + (size_t)a.heads * a.E + (size_t)(a.groups + g) * a.N;
-  const float* br = a.row + (size_t)(start + min(j, cnt - 1)) * a.ld + (size_t)a.heads * a.E + (size_t)g * a.N;
+  const float* cr = a.row + (size_t)(start + min(i, cnt - 1)) * a.ld + a.c0 + (size_t)g * a.N;
+  const float* br = a.row + (size_t)(start + min(j, cnt - 1)) * a.ld + a.b0 + (size_t)g * a.N;
   f32x16 acc;
 #pragma unroll
   for (int r = 0; r < 16; r++) acc[r] = 0.f;
@@ -59,7 +64,8 @@ __global__ __launch_bounds__(256) void ssd_gram_kernel(StepMeta m, SsdArgs a) {
 // Operands travel straight from memory to registers (every wave reads its own state rows only): B of a block is asked for at the block's start and used at its end,
 // C and the Gram rows of the next block replace the present ones as soon as these are used up, so nothing is held twice.  Rows past the
 // entry's end are clamped to its last one (what is read there twice meets dt = 0 or is not stored).
-template <int NW>
+// NORM: the grid's last z index carries the second state: the recurrence with x = 1 in one column.
+template <int NW, bool NORM = false>
 __global__ __launch_bounds__(256, NW == 1 ? 2 : 1) void ssd_block_kernel(StepMeta m, SsdArgs a) {
   constexpr int Q = SSD_BLOCK;
   constexpr double LOG2E = 1.4426950408889634;
@@ -70,23 +76,33 @@ __global__ __launch_bounds__(256, NW == 1 ? 2 : 1) void ssd_block_kernel(StepMet
   const int e = blockIdx.x, h = blockIdx.y, e0 = blockIdx.z * 32, tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), half = lane >> 5, l31 = lane & 31;
   const int start = m.ent_start[e], cnt = m.ent_count[e], slot = m.ent_row[e], grp = h / (a.heads / a.groups);
   const bool fresh = m.tok_pos[start] == 0;
-  const int ld = (int)a.ld, oX = h * a.E + e0, oB = a.heads * a.E + grp * a.N, oC = oB + a.groups * a.N, oD = a.heads * a.E + 2 * a.groups * a.N + h, oL = oD + 2 * a.heads;
+  const bool ones = NORM && blockIdx.z + 1 == gridDim.z;
+  const int ld = (int)a.ld, ldg = (int)a.ldgate, oX = a.x0 + h * a.E + e0, oB = a.b0 + grp * a.N, oC = a.c0 + grp * a.N;
   const float* base = a.row + (size_t)start * ld;
+  const float* gbase = a.gates + (size_t)start * ldg + h;
   const float* gram = a.gram + ((size_t)ssd_first_block(start, e) * a.groups + grp) * (Q * Q);
   float* Sg = a.S + ((size_t)slot * a.heads + h) * (size_t)a.N * a.E;
-  const bool colok = e0 + l31 < a.E;
+  const bool colok = ones ? l31 == 0 : e0 + l31 < a.E;
   const int xcol = colok ? l31 : 0, n0 = 32 * wv * NW;
+  const size_t sn = ones ? 1 : a.E, sc = ones ? 0 : e0 + l31;
+  float* Snew = Sg;
+  if (ones) {
+    const int par = m.ent_par[e];
+    const size_t at = ((size_t)slot * a.heads + h) * a.N;
+    Sg = a.norm_S + (size_t)par * a.norm_buf + at; Snew = a.norm_S + (size_t)(par ^ 1) * a.norm_buf + at;
+  }
   f32x16 S[NW];
 #pragma unroll
   for (int w = 0; w < NW; w++)
 #pragma unroll
     for (int r = 0; r < 16; r++) {
       const int n = n0 + 32 * w + (r & 3) + 8 * (r >> 2) + 4 * half;
-      S[w][r] = (!fresh && n < a.N && colok) ? Sg[(size_t)n * a.E + e0 + l31] : 0.f;
+      S[w][r] = (!fresh && n < a.N && colok) ? Sg[n * sn + sc] : 0.f;
     }
   auto at = [](const float* p, unsigned int bytes) -> const float* { return reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + bytes); };
   // byte offset of row t0 + k of a block with `left` rows, clamped to its last one (ld < 2^21 floats: the factors fit 24 bits); the constant k stays out of registers
-  auto row_off = [&](int t0, int k, int left) -> unsigned int { return (unsigned int)(4 * (__mul24(t0, ld) + __mul24(min(k, left - 1 - t0), ld))); };
+  auto row_at = [](int t0, int k, int left, int ld) -> unsigned int { return (unsigned int)(4 * (__mul24(t0, ld) + __mul24(min(k, left - 1 - t0), ld))); };
+  auto row_off = [&](int t0, int k, int left) -> unsigned int { return row_at(t0, k, left, ld); };
   float B[NW][32], x[8], dt = 0.f, la = 0.f;      // B[n][j]: j = kk + 32 half
   f32x4 C[NW][2][4], G[2][2];                     // C[i][n]: four channels at a time; the Gram rows of this wave's sixteen keys j = 16 wv + 8 half + 0 .. 7
   // (what stands in state rows beyond N is finite and meets a factor of zero)
@@ -125,8 +141,8 @@ __global__ __launch_bounds__(256, NW == 1 ? 2 : 1) void ssd_block_kernel(StepMet
     const float* p = base + (size_t)b * Q * ld;
     const int left = cnt - b * Q;
 #pragma unroll
-    for (int u = 0; u < 8; u++) x[u] = *at(p, row_off(tid >> 5, 8 * u, left) + 4 * (oX + xcol));
-    if (wv == 0 && !a.fixed) { const unsigned int off = row_off(lane, 0, left); dt = *at(p + oD, off); la = *at(p + oL, off); }
+    for (int u = 0; u < 8; u++) x[u] = ones ? 1.f : *at(p, row_off(tid >> 5, 8 * u, left) + 4 * (oX + xcol));
+    if (wv == 0 && !a.fixed) { const float* g = gbase + (size_t)b * Q * ldg; const unsigned int off = row_at(lane, 0, left, ldg); dt = *at(g + a.dt_col, off); la = *at(g + a.log_col, off); }
   };
   auto stage = [&](int b) {
     const int buf = b & 1, left = cnt - b * Q;
@@ -217,7 +233,7 @@ __global__ __launch_bounds__(256, NW == 1 ? 2 : 1) void ssd_block_kernel(StepMet
     for (int u = 0; u < 8; u++) {
       const int t = (tid >> 5) + 8 * u;
       if (t0 + t < cnt && colok)
-        a.out[(size_t)(start + t0 + t) * a.ldo + oX + l31] = fmaf(Dh, s_x[buf][t][l31], s_part[0][t][l31] + s_part[1][t][l31] + s_part[2][t][l31] + s_part[3][t][l31]);
+        *(ones ? a.norm_out + (size_t)(start + t0 + t) * a.ldn + h : a.out + (size_t)(start + t0 + t) * a.ldo + h * a.E + e0 + l31) = fmaf(Dh, s_x[buf][t][l31], s_part[0][t][l31] + s_part[1][t][l31] + s_part[2][t][l31] + s_part[3][t][l31]);
     }
   }
 #pragma unroll
@@ -225,8 +241,60 @@ __global__ __launch_bounds__(256, NW == 1 ? 2 : 1) void ssd_block_kernel(StepMet
 #pragma unroll
     for (int r = 0; r < 16; r++) {
       const int n = n0 + 32 * w + (r & 3) + 8 * (r >> 2) + 4 * half;
-      if (n < a.N && colok) Sg[(size_t)n * a.E + e0 + l31] = S[w][r];
+      if (n < a.N && colok) Snew[n * sn + sc] = S[w][r];
     }
+}
+
+// The gates of a matrix memory in that form.  With the running maximum m_t = max(f_t + m_(t-1), i_t) of the log gates, the memory decays by exp(f_t + m_(t-1) - m_t), takes
+// k v^T by exp(i_t - m_t), and divides by at least exp(-m_t).  A token is the map m -> max(f + m, i), and such maps compose to maps of the same form, so a scan over lanes,
+// waves and portions of 1024 tokens gives every m_t from sums of the f alone (no difference of two long sums).  Grid: (entries, heads).
+struct GateScanArgs {
+  const float* proj; long long ldp; int i0, f0;      // the columns of the log gates
+  float* mx; size_t mx_buf;                          // [2][slots][heads]
+  float* gates; int heads;                           // [T][take (heads) | log decay (heads) | exp(-m) (heads)]
+};
+template <int TPT = 4>      // tokens of a thread
+__global__ __launch_bounds__(256) void gate_scan_kernel(StepMeta m, GateScanArgs a) {
+  __shared__ float s_f[2][4], s_m[2][4];
+  const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int start = m.ent_start[e], cnt = m.ent_count[e], row = m.ent_row[e], par = m.ent_par[e];
+  float carry = m.tok_pos[start] == 0 ? 0.f : a.mx[(size_t)par * a.mx_buf + (size_t)row * a.heads + h];
+  for (int t0 = 0, p = 0; t0 < cnt; t0 += 256 * TPT, p ^= 1) {
+    float f[TPT], ig[TPT];
+#pragma unroll
+    for (int u = 0; u < TPT; u++) {      // (past the end m -> max(0 + m, -inf))
+      const int t = t0 + TPT * tid + u;
+      const float* r = a.proj + (size_t)(start + min(t, cnt - 1)) * a.ldp;
+      const float fv = r[a.f0 + h], iv = r[a.i0 + h];
+      f[u] = t < cnt ? fv : 0.f; ig[u] = t < cnt ? iv : -INFINITY;
+    }
+    float F = f[0], M = ig[0];
+#pragma unroll
+    for (int u = 1; u < TPT; u++) { M = fmaxf(M + f[u], ig[u]); F += f[u]; }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const float pf = __shfl_up(F, o, 64), pm = __shfl_up(M, o, 64);
+      if (lane >= o) { M = fmaxf(pm + F, M); F += pf; }
+    }
+    if (lane == 63) { s_f[p][wv] = F; s_m[p][wv] = M; }
+    const float bf = __shfl_up(F, 1, 64), bm = __shfl_up(M, 1, 64);      // the map of the lanes before
+    __syncthreads();      // (two buffers: the next portion's sums are written before all have read these)
+    float before = carry;
+#pragma unroll
+    for (int w = 0; w < 4; w++) { if (w < wv) before = fmaxf(before + s_f[p][w], s_m[p][w]); carry = fmaxf(carry + s_f[p][w], s_m[p][w]); }
+    if (lane > 0) before = fmaxf(before + bf, bm);
+#pragma unroll
+    for (int u = 0; u < TPT; u++) {
+      const int t = t0 + TPT * tid + u;
+      const float now = fmaxf(before + f[u], ig[u]);
+      if (t < cnt) {
+        float* o = a.gates + (size_t)(start + t) * 3 * a.heads + h;
+        o[0] = expf(ig[u] - now); o[a.heads] = f[u] + before - now; o[2 * a.heads] = expf(-now);
+      }
+      before = now;
+    }
+  }
+  if (tid == 0) a.mx[(size_t)(par ^ 1) * a.mx_buf + (size_t)row * a.heads + h] = carry;
 }
 
 }  // namespace tgx

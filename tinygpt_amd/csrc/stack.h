@@ -149,7 +149,7 @@ struct StackModel {
 };
 
 // stack_gqa.hip
-namespace tgx { struct StepMeta; struct GqaMfmaArgs; struct MixMfmaArgs; struct SsdArgs; }
+namespace tgx { struct StepMeta; struct GqaMfmaArgs; struct MixMfmaArgs; struct SsdArgs; struct GateScanArgs; }
 bool gqa_mfma_shapes_ok(int dt, int dim, int vdim, int page_shift, long long ldq);
 void launch_gqa_mfma(tgx_ctx* c, const tgx::StepMeta& m, const tgx::GqaMfmaArgs& a, dim3 grid, bool split);
 void launch_mix_mfma(tgx_ctx* c, const tgx::StepMeta& m, const tgx::MixMfmaArgs& a, dim3 grid);      // kernels/stack_mix_mfma.h
@@ -171,6 +171,7 @@ void launch_stack_line(tgx_ctx* c, const tgx::StackGemmArgs& g, int epi, int nz,
 bool ssd_mfma_shapes_ok(int heads, int groups, int N, int E, long long ld);
 size_t ssd_gram_elems(int T, int S, int groups);
 void launch_ssd_mfma(tgx_ctx* c, const tgx::StepMeta& m, const tgx::SsdArgs& a, int S, int max_count);
+void launch_gate_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::GateScanArgs& a, int S);
 
 int stack_create(const tgx_stack_desc* desc, const tgx_layer_desc* layers, int device_ordinal, tgx_ctx** out_ctx);
 int stack_upload(tgx_ctx* c, const char* name, const void* host, const int64_t* shape, int nd, int src_dtype);

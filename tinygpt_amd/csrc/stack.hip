@@ -25,6 +25,7 @@
 int upload_param_ext(tgx_ctx* c, ebyte* dst, const void* host, int64_t n, int src_dtype);      // abi.hip
 
 namespace {
+int pad4(int n) { return (n + 3) & ~3; }      // row strides of buffers whose rows are read in vectors of four
 
 float half_bits_to_f32(uint16_t h) {
   const uint32_t s = (h >> 15) & 1, e = (h >> 10) & 0x1f, m = h & 0x3ff;
@@ -527,38 +528,54 @@ int run_attention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, const floa
   return TGX_OK;
 }
 
-int run_mlstm(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, const float* hin, int T, int S) {
+int run_mlstm(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, const float* hin, int T, int S, int max_count) {
   StackModel* sm = c->stack;
   const tgx_layer_desc& ld = w.d;
-  const int W = sm->d.width, H = ld.heads, qd = H * ld.dim, vd = H * ld.vdim, nin = 2 * qd + 2 * vd + 2 * H;
+  const int W = sm->d.width, H = ld.heads, qd = H * ld.dim, vd = H * ld.vdim, nin = 2 * qd + 2 * vd + 2 * H, ldp = pad4(nin);
   // [q | k | v | gate | i | f] = h . w_in^T (+ the gate biases); i and f through the soft cap (and the log sigmoid) in the product's epilogue
   tgx::StackGemmArgs g{};
-  g.A = hin; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = nin; g.M = T; g.N = nin; g.K = W; g.scale = 1.f; g.bias = w.b_in;
+  g.A = hin; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = ldp; g.M = T; g.N = nin; g.K = W; g.scale = 1.f; g.bias = w.b_in;
   g.gate_col0 = 2 * qd + 2 * vd; g.gate_heads = H; g.gate_cap = ld.gate_cap;      // the two gate rows leave the product as log gates
   launch_gemm(c, g, tgx::SG_STORE, 1);
-  tgx::MlstmArgs ma{};
-  ma.proj = sm->proj; ma.ldp = nin; ma.heads = H; ma.dim = ld.dim; ma.vdim = ld.vdim; ma.qscale = 1.0f / sqrtf((float)ld.dim);
-  ma.S = w.mS; ma.n = w.mn; ma.mx = w.mm; ma.n_buf = (size_t)sm->d.max_seqs * H * ld.dim; ma.mx_buf = (size_t)sm->d.max_seqs * H;
-  ma.hs = sm->hs; ma.ldh = vd;
-  // columns per wave: 16, or 8 (twice the workgroups, half the rows per lane) while the step's entries and heads leave most of the chip idle
-  const bool narrow = ld.dim <= 256 && (sm->mlstm_narrow >= 0 ? sm->mlstm_narrow != 0 : (long long)S * H * ((ld.vdim + 63) / 64) * 2 <= c->num_cus);
-  if (narrow) {
-    const dim3 grid(S, H, (ld.vdim + 31) / 32);
-    const int dper = (ld.dim + 7) / 8;
-    if (dper <= 8) hipLaunchKernelGGL((tgx::mlstm_scan_kernel<8, 8>), grid, dim3(256), 0, c->stream, m, ma);
-    else if (dper <= 16) hipLaunchKernelGGL((tgx::mlstm_scan_kernel<16, 8>), grid, dim3(256), 0, c->stream, m, ma);
-    else hipLaunchKernelGGL((tgx::mlstm_scan_kernel<32, 8>), grid, dim3(256), 0, c->stream, m, ma);
-  } else {
-    const dim3 grid(S, H, (ld.vdim + 63) / 64);
-    const int dper = (ld.dim + 3) / 4;      // rows per lane: four row groups share a column
-    if (dper <= 8) hipLaunchKernelGGL((tgx::mlstm_scan_kernel<8, 16>), grid, dim3(256), 0, c->stream, m, ma);
-    else if (dper <= 16) hipLaunchKernelGGL((tgx::mlstm_scan_kernel<16, 16>), grid, dim3(256), 0, c->stream, m, ma);
-    else if (dper <= 32) hipLaunchKernelGGL((tgx::mlstm_scan_kernel<32, 16>), grid, dim3(256), 0, c->stream, m, ma);
-    else if (dper <= 64) hipLaunchKernelGGL((tgx::mlstm_scan_kernel<64, 16>), grid, dim3(256), 0, c->stream, m, ma);
-    else hipLaunchKernelGGL((tgx::mlstm_scan_kernel<128, 16>), grid, dim3(256), 0, c->stream, m, ma);
-  }
   tgx::HeadNormGateArgs oa{};
-  oa.hs = sm->hs; oa.ldh = vd; oa.w = w.head_w; oa.w_hstride = ld.vdim; oa.gate = sm->proj + 2 * qd + vd; oa.ldg = nin; oa.out = sm->o; oa.ldo = vd; oa.vdim = ld.vdim; oa.eps = sm->d.norm_eps;
+  // portions: the recurrence with its maximum taken out is a scalar-decay recurrence and runs in blocks of 64 tokens (kernels/stack_ssd_mfma.h): from 64 tokens,
+  // as the other families (a layer of 8 heads of 128 x 256, one prompt: 32 tokens 82 us by the scan and 86 in blocks, 64 tokens 115 and 107, 256 240 and 173, 1024 596 and 295)
+  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && (2 * qd) % 4 == 0) {
+    const size_t gram = ssd_gram_elems(T, S, H);
+    int rc = ensure_part(c, gram + (size_t)T * 4 * H);
+    if (rc) return rc;
+    tgx::GateScanArgs ga{};
+    ga.proj = sm->proj; ga.ldp = ldp; ga.i0 = 2 * qd + 2 * vd; ga.f0 = ga.i0 + H; ga.mx = w.mm; ga.mx_buf = (size_t)sm->d.max_seqs * H; ga.gates = sm->part + gram; ga.heads = H;
+    launch_gate_scan(c, m, ga, S);
+    tgx::SsdArgs da{};
+    da.row = sm->proj; da.ld = ldp; da.x0 = 2 * qd; da.b0 = qd; da.c0 = 0; da.gates = ga.gates; da.ldgate = 3 * H; da.dt_col = 0; da.log_col = H; da.heads = H; da.groups = H; da.N = ld.dim; da.E = ld.vdim;
+    da.gram = sm->part; da.S = w.mS; da.out = sm->hs; da.ldo = vd; da.norm_S = w.mn; da.norm_buf = (size_t)sm->d.max_seqs * H * ld.dim; da.norm_out = ga.gates + (size_t)T * 3 * H; da.ldn = H;
+    launch_ssd_mfma(c, m, da, S, max_count);
+    oa.norm = da.norm_out; oa.ldnorm = H; oa.floor = ga.gates + 2 * H; oa.ldfloor = 3 * H; oa.scale = 1.0f / sqrtf((float)ld.dim);
+  } else {
+    tgx::MlstmArgs ma{};
+    ma.proj = sm->proj; ma.ldp = ldp; ma.heads = H; ma.dim = ld.dim; ma.vdim = ld.vdim; ma.qscale = 1.0f / sqrtf((float)ld.dim);
+    ma.S = w.mS; ma.n = w.mn; ma.mx = w.mm; ma.n_buf = (size_t)sm->d.max_seqs * H * ld.dim; ma.mx_buf = (size_t)sm->d.max_seqs * H;
+    ma.hs = sm->hs; ma.ldh = vd;
+    // columns per wave: 16, or 8 (twice the workgroups, half the rows per lane) while the step's entries and heads leave most of the chip idle
+    const bool narrow = ld.dim <= 256 && (sm->mlstm_narrow >= 0 ? sm->mlstm_narrow != 0 : (long long)S * H * ((ld.vdim + 63) / 64) * 2 <= c->num_cus);
+    if (narrow) {
+      const dim3 grid(S, H, (ld.vdim + 31) / 32);
+      const int dper = (ld.dim + 7) / 8;
+      if (dper <= 8) hipLaunchKernelGGL((tgx::mlstm_scan_kernel<8, 8>), grid, dim3(256), 0, c->stream, m, ma);
+      else if (dper <= 16) hipLaunchKernelGGL((tgx::mlstm_scan_kernel<16, 8>), grid, dim3(256), 0, c->stream, m, ma);
+      else hipLaunchKernelGGL((tgx::mlstm_scan_kernel<32, 8>), grid, dim3(256), 0, c->stream, m, ma);
+    } else {
+      const dim3 grid(S, H, (ld.vdim + 63) / 64);
+      const int dper = (ld.dim + 3) / 4;      // rows per lane: four row groups share a column
+      if (dper <= 8) hipLaunchKernelGGL((tgx::mlstm_scan_kernel<8, 16>), grid, dim3(256), 0, c->stream, m, ma);
+      else if (dper <= 16) hipLaunchKernelGGL((tgx::mlstm_scan_kernel<16, 16>), grid, dim3(256), 0, c->stream, m, ma);
+      else if (dper <= 32) hipLaunchKernelGGL((tgx::mlstm_scan_kernel<32, 16>), grid, dim3(256), 0, c->stream, m, ma);
+      else if (dper <= 64) hipLaunchKernelGGL((tgx::mlstm_scan_kernel<64, 16>), grid, dim3(256), 0, c->stream, m, ma);
+      else hipLaunchKernelGGL((tgx::mlstm_scan_kernel<128, 16>), grid, dim3(256), 0, c->stream, m, ma);
+    }
+  }
+  oa.hs = sm->hs; oa.ldh = vd; oa.w = w.head_w; oa.w_hstride = ld.vdim; oa.gate = sm->proj + 2 * qd + vd; oa.ldg = ldp; oa.out = sm->o; oa.ldo = vd; oa.vdim = ld.vdim; oa.eps = sm->d.norm_eps;
   hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, H), dim3(64), 0, c->stream, oa);
   g = tgx::StackGemmArgs{};
   g.A = sm->o; g.lda = vd; g.B = w.w_o; g.ldb = vd; g.C = sm->yd; g.ldc = W; g.M = T; g.N = W; g.K = vd; g.scale = 1.f;
@@ -629,7 +646,7 @@ int run_layers_sandwich(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_ke
     const tgx_layer_desc& ld = w.d;
     const float* ng = sm->norm_g + 4 * (size_t)li;
     const float* next_layer = li + 1 < L ? ng + 4 : nullptr;
-    int rc = ld.mixer == TGX_MIXER_ATTENTION ? run_attention(c, m, w, hin, T, S, max_keys, max_count) : run_mlstm(c, m, w, hin, T, S);
+    int rc = ld.mixer == TGX_MIXER_ATTENTION ? run_attention(c, m, w, hin, T, S, max_keys, max_count) : run_mlstm(c, m, w, hin, T, S, max_count);
     if (rc) return rc;
     tgx::SandwichArgs sa{};
     sa.x = sm->x; sa.y = sm->yd; sa.top = 1; sa.ytmp = sm->ytmp; sa.g_post = ng + 1; sa.g_next = ld.mlp != TGX_MLP_NONE ? ng + 2 : next_layer; sa.out = hout; sa.W = W; sa.eps = eps;
@@ -1243,7 +1260,6 @@ int check_affine_desc(const tgx_stack_desc& d, const tgx_layer_desc* layers) {
 }
 
 // ---- output-norm designs (Nusovik): per layer  x += norm1(mixer(x))  and  x += norm2(ff(x)); the sublayers read the stream itself.
-int pad4(int n) { return (n + 3) & ~3; }      // row strides of buffers whose rows are read in vectors of four
 
 // y = A . W^T into the sublayers' output rows
 void sublayer_out(tgx_ctx* c, const float* A, int K, const ebyte* Wm, int T) { launch_gemm(c, sublayer_product(c, A, K, Wm, T), tgx::SG_STORE, 1); }
@@ -1333,7 +1349,7 @@ int run_ssm_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, 
   if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(rH, ld.d_kv_heads, ld.d_dim, ld.d_vdim, ldr)) {
     if ((rc = ensure_part(c, ssd_gram_elems(T, S, ld.d_kv_heads)))) return rc;
     tgx::SsdArgs da{};
-    da.row = sm->rec_in; da.ld = ldr; da.heads = rH; da.groups = ld.d_kv_heads; da.N = ld.d_dim; da.E = ld.d_vdim; da.gram = sm->part; da.skip = w.d_skip; da.S = w.mS; da.out = sm->hs; da.ldo = I;
+    da.row = sm->rec_in; da.ld = ldr; da.b0 = I; da.c0 = I + gn; da.gates = sm->rec_in; da.ldgate = ldr; da.dt_col = C; da.log_col = C + 2 * rH; da.heads = rH; da.groups = ld.d_kv_heads; da.N = ld.d_dim; da.E = ld.d_vdim; da.gram = sm->part; da.skip = w.d_skip; da.S = w.mS; da.out = sm->hs; da.ldo = I;
     launch_ssd_mfma(c, m, da, S, max_count);
   } else launch_rec_scan(c, m, ra, tgx::REC_SSD, S);
   tgx::PartNormArgs pa{};
@@ -1583,7 +1599,7 @@ int run_retention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int
     int rc = ensure_part(c, ssd_gram_elems(T, S, H));
     if (rc) return rc;
     tgx::SsdArgs da{};
-    da.row = sm->proj; da.ld = ldp; da.heads = H; da.groups = H; da.N = ld.dim; da.E = ld.vdim; da.gram = sm->part; da.fixed = w.decays; da.dt0 = kscale; da.S = w.mS; da.out = sm->hs; da.ldo = vd;
+    da.row = sm->proj; da.ld = ldp; da.b0 = vd; da.c0 = vd + qd; da.heads = H; da.groups = H; da.N = ld.dim; da.E = ld.vdim; da.gram = sm->part; da.fixed = w.decays; da.dt0 = kscale; da.S = w.mS; da.out = sm->hs; da.ldo = vd;
     launch_ssd_mfma(c, m, da, S, max_count);
   } else {
     tgx::RecScanArgs ra{};
@@ -2146,7 +2162,7 @@ int create_sandwich_layers(tgx_ctx* c, const tgx_layer_desc* layers) {
     }
     if ((rc = dev_alloc(c, &w.w_in, nin * W * es)) || (rc = dev_alloc(c, &w.b_in, nin)) || (rc = dev_alloc(c, &w.w_o, W * vd * es))) return rc;
     HIP_OK(c, hipMemset(w.b_in, 0, nin * 4));
-    sm->max_in = std::max(sm->max_in, (int)nin); sm->max_hv = std::max(sm->max_hv, (int)vd);
+    sm->max_in = std::max(sm->max_in, pad4((int)nin)); sm->max_hv = std::max(sm->max_hv, (int)vd);
     if (l.mlp == TGX_MLP_NONE) continue;
     for (const char* n : {"norm2", "norm2b"}) sm->missing.insert(p + n);
     if (l.mlp == TGX_MLP_DENSE) {
