@@ -6,7 +6,9 @@ round to the other neighbour (2^-9 for bf16, 2^-12 for fp16) where two sums of t
 import numpy as np
 import pytest
 
+import modepel_oracle as mo
 import stack_oracle as so
+import test_hip_modepel as tm
 import test_hip_vitudra as tv
 from tinygpt_amd.desc import LayerDesc, StackDesc
 from tinygpt_amd.serving import SlotEngine
@@ -136,3 +138,21 @@ def test_scan_of_the_recurrences(dim, entries):
         want = tv.want_of(cfg, w, seqs[i])
         for at, part in ((23, got[0]), (-1, got[1])):
             assert np.abs(part[i] - want[at]).max() / np.abs(want).max() < 1e-4, (dim, entries, i, at)
+
+
+# ---- matrix memories in blocks (portions from 64 tokens): remainders of a block, of a portion of the gate scan (1024 tokens), of the state's and the values' tiles; then a
+# second portion and single tokens that carry both states on.  fp32 storage against the plain oracle: fp32 sums over at most 256 channels and 64 tokens, an order of
+# magnitude below the 1e-4 of the largest logit that the design's own tests allow.
+@pytest.mark.parametrize("dim,vdim", [(4, 8), (32, 33), (36, 32), (132, 6), (256, 40)])
+@pytest.mark.parametrize("n", [64, 65, 127, 192, 1023, 1025, 2050])
+def test_matrix_memory_in_blocks(n, dim, vdim):
+    cfg = tm.config([tm.rec(heads=3, dim=dim, vdim=vdim), tm.rec(heads=2, dim=dim, vdim=vdim, gate_cap=4.0)], width=20)
+    eng, w = tm.engine(cfg, seed=n, max_seqs=2, max_ctx=4096, budget_tokens=8192)
+    tok = [np.random.default_rng(n + i).integers(0, cfg["vocab"], n + 70).tolist() for i in range(2)]
+    at = sorted({0, 63, n // 2, n - 1})
+    got = [eng.step([(0, tok[0][:n], at), (1, tok[1][:3], [2])]), eng.step([(1, tok[1][3:n], [n - 4]), (0, tok[0][n:n + 68], [67])]),
+           eng.step([(0, tok[0][n + 68:n + 69], [0]), (1, tok[1][n:n + 1], [0])])]
+    eng.close()
+    want = [mo.forward(cfg, w, t[:n + 69])[0] for t in tok]
+    for i, rows, pos in ((0, got[0][:len(at)], at), (1, got[0][len(at):], [2]), (1, got[1][:1], [n - 1]), (0, got[1][1:], [n + 67]), (0, got[2][:1], [n + 68]), (1, got[2][1:], [n])):
+        assert np.abs(rows - want[i][pos]).max() / np.abs(want[i]).max() < 1e-4, (n, dim, vdim, i, pos)
