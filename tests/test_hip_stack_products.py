@@ -10,6 +10,7 @@ import modepel_oracle as mo
 import stack_oracle as so
 import test_hip_modepel as tm
 import test_hip_vitudra as tv
+import test_hip_zaluvik as tz
 from tinygpt_amd.desc import LayerDesc, StackDesc
 from tinygpt_amd.serving import SlotEngine
 
@@ -156,3 +157,31 @@ def test_matrix_memory_in_blocks(n, dim, vdim):
     want = [mo.forward(cfg, w, t[:n + 69])[0] for t in tok]
     for i, rows, pos in ((0, got[0][:len(at)], at), (1, got[0][len(at):], [2]), (1, got[1][:1], [n - 1]), (0, got[1][1:], [n + 67]), (0, got[2][:1], [n + 68]), (1, got[2][1:], [n])):
         assert np.abs(rows - want[i][pos]).max() / np.abs(want[i]).max() < 1e-4, (n, dim, vdim, i, pos)
+
+
+# ---- seams and norms: rows of one, two and four vectors a thread, widths that are no multiple of four, and widths past the registers; taps by number and by name.
+# fp32 storage against the plain oracles of the designs: fp32 sums over at most 4100 channels, 1e-4 of the largest logit as in the designs' own tests.
+@pytest.mark.parametrize("width", [1024, 1028, 1030, 2044, 2052, 4096, 4100])
+@pytest.mark.parametrize("design", ["modepel", "zaluvik", "vitudra"])
+def test_seams_of_wide_rows(design, width):
+    t, layers = {"modepel": (tm, [tm.rec(tm.moe()), tm.attn(tm.dense())]), "zaluvik": (tz, [tz.attn(tz.moe()), tz.lat(tz.dense())]), "vitudra": (tv, [tv.wkv(tv.ff()), tv.attn()])}[design]
+    cfg = t.config(layers, width=width)
+    eng, w = t.engine(cfg, seed=width)
+    toks = t.tokens(cfg, 5, seed=width)
+    got = t.run_whole(eng, "a", toks)
+    eng.close()
+    t.check(got, t.want_of(cfg, w, toks), "fp32", f"{design} {width}")
+
+
+@pytest.mark.parametrize("width,groups", [(1024, 2), (1032, 6), (1036, 7), (1030, 5)])
+@pytest.mark.parametrize("taps", [1, 2, 4, 5, 8])
+def test_norm_and_convolution_of_wide_rows(taps, width, groups):
+    layers = [LayerDesc(heads=3, dim=8, vdim=8, kv_rank=24, scale=0.35, mlp="moe", experts=5, top=2, ff=24, limit=1.5)]
+    d = StackDesc(width=width, vocab=53, canon_taps=taps, norm_groups=groups, norm_eps=1e-6, max_seqs=2, max_ctx=64, budget_tokens=128, compute_dtype="fp32", layers=layers)
+    t = so.random_tensors(d, taps)
+    toks = np.random.default_rng(taps).integers(0, 53, 14).tolist()
+    eng = SlotEngine(desc=d, tensors={k: v.astype(np.float32) for k, v in t.items()})
+    got = np.concatenate([eng.step([("a", toks[lo:hi], list(range(hi - lo)))]) for lo, hi in ((0, 2), (2, 3), (3, 12), (12, 14))])
+    eng.close()
+    want = so.forward(d, t, toks)
+    assert np.abs(got - want).max() / np.abs(want).max() < 1e-4, (taps, width)

@@ -33,6 +33,39 @@ __global__ __launch_bounds__(256) void sinusoid_embed_kernel(StepMeta m, const e
   }
 }
 
+// ---- a token's row kept in the registers of a workgroup of 256 between the passes of a seam: vectors k < ROW_REG of four channels each, 4 tid + 1024 k + u with V4
+// (widths that are multiples of four), tid + 1024 k + 256 u otherwise.  Channels past the width read as zero; loads past it repeat the row's end.
+constexpr int ROW_REG = 4;      // widths up to 4096
+template <bool V4>
+__device__ __forceinline__ int row_channel(int k, int u) { return V4 ? 4 * (int)threadIdx.x + 1024 * k + u : (int)threadIdx.x + 1024 * k + 256 * u; }
+template <bool V4>
+__device__ __forceinline__ f32x4 row_load(const float* p, int k, int W) {
+  f32x4 r = {0.f, 0.f, 0.f, 0.f};
+  if (1024 * k >= W) return r;      // (uniform)
+  if constexpr (V4) {
+    const int c = row_channel<true>(k, 0);
+    const f32x4 v = *reinterpret_cast<const f32x4*>(p + min(c, W - 4));
+    if (c < W) r = v;
+  } else
+#pragma unroll
+    for (int u = 0; u < 4; u++) { const int c = row_channel<false>(k, u); const float v = p[min(c, W - 1)]; r[u] = c < W ? v : 0.f; }
+  return r;
+}
+template <bool V4>
+__device__ __forceinline__ void row_store(float* p, int k, int W, f32x4 v) {
+  if constexpr (V4) { const int c = row_channel<true>(k, 0); if (c < W) *reinterpret_cast<f32x4*>(p + c) = v; }
+  else
+#pragma unroll
+    for (int u = 0; u < 4; u++) { const int c = row_channel<false>(k, u); if (c < W) p[c] = v[u]; }
+}
+// the sum over a workgroup of 256 with one barrier: every call of a kernel has its own four numbers of LDS
+__device__ __forceinline__ float block_sum_once(float v, float* own4) {
+  v = group_sum<64>(v);
+  if ((threadIdx.x & 63) == 0) own4[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return own4[0] + own4[1] + own4[2] + own4[3];
+}
+
 // ---- grouped RMS norm + input convolution.  One workgroup per token.  hn_r = x_r / rms_group(x_r) * w for the token and its taps - 1 predecessors
 // (rows of this step where the entry holds them, the slot's state otherwise, zero before the sequence's start);
 // out = hn_t + sum_j cw[:, j] * hn_(t - taps + 1 + j).  The state (the last taps - 1 normed rows of the slot) is double-buffered per slot: this
@@ -48,31 +81,35 @@ struct NormConvArgs {
   int W, groups, taps;
   float eps;
 };
+// TAPS: 4 and 1 have the filter's size at compile time (its taps arrive four a load and stand in registers by number); 0: any.  The row and its predecessors are asked for
+// before the sums of squares, whose barrier they cross in flight (four taps, 1024 channels: 7.4 -> 3.2 us for a few rows, 43 -> 17 for some 2400, which selecting taps by number bounded).
+template <int TAPS>
 __global__ __launch_bounds__(256) void norm_conv_kernel(StepMeta m, NormConvArgs a) {
   __shared__ float s_rinv[CONV_MAX_TAPS][NORM_MAX_GROUPS];
   const int t = blockIdx.x, i = m.tok_idx[t], cnt = m.tok_cnt[t], pos = m.tok_pos[t];
   const int row = m.tok_row[t], par = m.tok_par[t];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int gw = a.W / a.groups, nb = a.taps - 1;
-  // 1 / rms of every (row back, group) pair that lives in this step: one wave per pair, lanes over the group's channels
-  for (int it = wv; it < a.taps * a.groups; it += 4) {
-    const int d = it / a.groups, g = it - d * a.groups;
-    if (d > i) continue;                                  // wave-uniform: that row comes from the state (already normed) or lies before the start
-    const float* xr = a.x + (size_t)(t - d) * a.W + (size_t)g * gw;
-    float ss = 0.f;
-    if ((a.W & 3) == 0 && (gw & 3) == 0)
-      for (int c = 4 * lane; c < gw; c += 256) { const f32x4 v = *reinterpret_cast<const f32x4*>(xr + c); ss = fmaf(v[0], v[0], ss); ss = fmaf(v[1], v[1], ss); ss = fmaf(v[2], v[2], ss); ss = fmaf(v[3], v[3], ss); }
-    else
-      for (int c = lane; c < gw; c += 64) ss = fmaf(xr[c], xr[c], ss);
-    ss = wave_sum(ss);
-    if (lane == 0) s_rinv[d][g] = 1.0f / sqrtf(ss / (float)gw + a.eps);
-  }
-  __syncthreads();
+  const int gw = a.W / a.groups, taps = TAPS > 0 ? TAPS : a.taps, nb = taps - 1;
   // (the two state buffers, the stream and the output never overlap: without the qualifiers every state store would order the loads behind it)
   const float* __restrict__ st_old = a.state ? a.state + (size_t)par * a.state_buf + (size_t)row * nb * a.W : nullptr;
   float* __restrict__ st_new = a.state ? a.state + (size_t)(par ^ 1) * a.state_buf + (size_t)row * nb * a.W : nullptr;
   const float* __restrict__ xin = a.x;
   float* __restrict__ outp = a.out;
+  // 1 / rms of every (row back, group) pair that lives in this step: one wave per pair, lanes over the group's channels
+  auto sums = [&] {
+    for (int it = wv; it < taps * a.groups; it += 4) {
+      const int d = it / a.groups, g = it - d * a.groups;
+      if (d > i) continue;                                  // wave-uniform: that row comes from the state (already normed) or lies before the start
+      const float* xr = a.x + (size_t)(t - d) * a.W + (size_t)g * gw;
+      float ss = 0.f;
+      if ((a.W & 3) == 0 && (gw & 3) == 0)
+        for (int c = 4 * lane; c < gw; c += 256) { const f32x4 v = *reinterpret_cast<const f32x4*>(xr + c); ss = fmaf(v[0], v[0], ss); ss = fmaf(v[1], v[1], ss); ss = fmaf(v[2], v[2], ss); ss = fmaf(v[3], v[3], ss); }
+      else
+        for (int c = lane; c < gw; c += 64) ss = fmaf(xr[c], xr[c], ss);
+      ss = wave_sum(ss);
+      if (lane == 0) s_rinv[d][g] = 1.0f / sqrtf(ss / (float)gw + a.eps);
+    }
+  };
   // channel c of the token: the normed row, the filter over it and its predecessors, the new state
   auto channel = [&](int c, float xv, float w, const float* cw) -> float {
     const int g = c / gw;
@@ -98,40 +135,53 @@ __global__ __launch_bounds__(256) void norm_conv_kernel(StepMeta m, NormConvArgs
   if ((a.W & 3) == 0 && (gw & 3) == 0) {
     // four channels per thread.  Every load is issued unconditionally (where the row back comes from — this step, the state, nowhere — is uniform over the
     // workgroup and only selects the address): one memory round trip instead of one per tap
-#pragma unroll 2
-    for (int c = 4 * threadIdx.x; c < a.W; c += 1024) {
-      const int g = c / gw;
-      const f32x4 xv = *reinterpret_cast<const f32x4*>(xin + (size_t)t * a.W + c), wv4 = *reinterpret_cast<const f32x4*>(a.nw + c);
-      f32x4 hv[CONV_MAX_TAPS];
-      float cwv[4][CONV_MAX_TAPS];
+    constexpr int MT = TAPS > 0 ? TAPS : CONV_MAX_TAPS;
+    f32x4 hv[MT], wv4, cwv[4][(MT + 3) / 4];
+    auto fetch = [&](int c) {
+      wv4 = *reinterpret_cast<const f32x4*>(a.nw + c);
 #pragma unroll
-      for (int d = 1; d < CONV_MAX_TAPS; d++) {
+      for (int d = 0; d < MT; d++) {
         if (d > nb) continue;
-        const bool inrow = d <= i, ok = inrow || pos - d >= 0;
-        const float* p = inrow ? xin + (size_t)(t - d) * a.W + c : (ok ? st_old + (size_t)(nb - (d - i)) * a.W + c : xin + (size_t)t * a.W + c);
-        const f32x4 v = *reinterpret_cast<const f32x4*>(p);
-        const float sc = inrow ? s_rinv[d][g] : (ok ? 1.f : 0.f);
-#pragma unroll
-        for (int k = 0; k < 4; k++) hv[d][k] = inrow ? v[k] * sc * wv4[k] : v[k] * sc;
+        const float* p = d <= i ? xin + (size_t)(t - d) * a.W + c : (pos - d >= 0 ? st_old + (size_t)(nb - (d - i)) * a.W + c : xin + (size_t)t * a.W + c);
+        hv[d] = *reinterpret_cast<const f32x4*>(p);
       }
       if (a.cw) {
 #pragma unroll
-        for (int k = 0; k < 4; k++)
+        for (int k = 0; k < 4; k++) {
+          if constexpr (TAPS == 4) cwv[k][0] = *reinterpret_cast<const f32x4*>(a.cw + 4 * (size_t)(c + k));
+          else
 #pragma unroll
-          for (int j = 0; j < CONV_MAX_TAPS; j++) cwv[k][j] = j < a.taps ? a.cw[(size_t)(c + k) * a.taps + j] : 0.f;
+            for (int j = 0; j < MT; j++) cwv[k][j / 4][j % 4] = j < taps ? a.cw[(size_t)(c + k) * taps + j] : 0.f;
+        }
       }
-      f32x4 o;
+    };
+    int c = 4 * threadIdx.x;
+    if (c < a.W) fetch(c);
+    __builtin_amdgcn_sched_barrier(0);
+    sums();
+    __syncthreads();
+    for (; c < a.W;) {
+      const int g = c / gw;
 #pragma unroll
-      for (int k = 0; k < 4; k++) { hv[0][k] = xv[k] * s_rinv[0][g] * wv4[k]; o[k] = hv[0][k]; }
+      for (int d = 0; d < MT; d++) {
+        if (d > nb) continue;
+        const bool inrow = d <= i;
+        const float sc = inrow ? s_rinv[d][g] : (pos - d >= 0 ? 1.f : 0.f);
+#pragma unroll
+        for (int k = 0; k < 4; k++) hv[d][k] = inrow ? hv[d][k] * sc * wv4[k] : hv[d][k] * sc;
+      }
+      f32x4 o = hv[0];
       if (a.cw) {
 #pragma unroll
-        for (int d = 0; d < CONV_MAX_TAPS; d++) {
+        for (int d = 0; d < MT; d++) {
           if (d > nb) continue;
 #pragma unroll
           for (int k = 0; k < 4; k++) {
             float wsel = 0.f;                                // filter tap nb - d of channel c + k
+            if constexpr (TAPS > 0) wsel = cwv[k][(TAPS - 1 - d) / 4][(TAPS - 1 - d) % 4];
+            else
 #pragma unroll
-            for (int j = 0; j < CONV_MAX_TAPS; j++) wsel = (j == nb - d) ? cwv[k][j] : wsel;
+              for (int j = 0; j < MT; j++) wsel = (j == nb - d) ? cwv[k][j / 4][j % 4] : wsel;
             o[k] = fmaf(wsel, hv[d][k], o[k]);
           }
         }
@@ -139,7 +189,7 @@ __global__ __launch_bounds__(256) void norm_conv_kernel(StepMeta m, NormConvArgs
         if (sl >= 0) *reinterpret_cast<f32x4*>(st_new + (size_t)sl * a.W + c) = hv[0];
         if (i == 0) {
 #pragma unroll
-          for (int d = 1; d < CONV_MAX_TAPS; d++) {          // an entry shorter than the state keeps the tail of the old one: old row d back -> slot nb - cnt - d
+          for (int d = 1; d < MT; d++) {          // an entry shorter than the state keeps the tail of the old one: old row d back -> slot nb - cnt - d
             if (d > nb) continue;
             const int kk = nb - cnt - d;
             if (kk >= 0) *reinterpret_cast<f32x4*>(st_new + (size_t)kk * a.W + c) = hv[d];
@@ -147,9 +197,13 @@ __global__ __launch_bounds__(256) void norm_conv_kernel(StepMeta m, NormConvArgs
         }
       }
       *reinterpret_cast<f32x4*>(outp + (size_t)t * a.W + c) = o;
+      c += 1024;
+      if (c < a.W) fetch(c);
     }
   } else {
-    for (int c = threadIdx.x; c < a.W; c += 256) outp[(size_t)t * a.W + c] = channel(c, xin[(size_t)t * a.W + c], a.nw[c], a.cw ? a.cw + (size_t)c * a.taps : nullptr);
+    sums();
+    __syncthreads();
+    for (int c = threadIdx.x; c < a.W; c += 256) outp[(size_t)t * a.W + c] = channel(c, xin[(size_t)t * a.W + c], a.nw[c], a.cw ? a.cw + (size_t)c * taps : nullptr);
   }
 }
 

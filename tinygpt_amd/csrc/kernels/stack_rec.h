@@ -21,11 +21,28 @@ namespace tgx {
 __global__ __launch_bounds__(256) void offset_norm_kernel(const float* x, const int* rows, const float* w, float offset, float* out, int W, float eps) {
   __shared__ float s4[4];
   const float* xr = x + (size_t)(rows ? rows[blockIdx.x] : blockIdx.x) * W;
+  float* o = out + (size_t)blockIdx.x * W;
   float ss = 0.f;
+  if ((W & 3) == 0 && W <= 1024 * ROW_REG) {      // (the weights are on their way before the sum)
+    f32x4 v[ROW_REG], wv[ROW_REG];
+#pragma unroll
+    for (int k = 0; k < ROW_REG; k++) { v[k] = row_load<true>(xr, k, W); wv[k] = row_load<true>(w, k, W); }
+#pragma unroll
+    for (int k = 0; k < ROW_REG; k++)
+#pragma unroll
+      for (int u = 0; u < 4; u++) ss = fmaf(v[k][u], v[k][u], ss);
+    const float r = 1.0f / sqrtf(block_sum_once(ss, s4) / (float)W + eps);
+#pragma unroll
+    for (int k = 0; k < ROW_REG; k++) {
+      for (int u = 0; u < 4; u++) v[k][u] = v[k][u] * r * (offset + wv[k][u]);
+      row_store<true>(o, k, W, v[k]);
+    }
+    return;
+  }
   for (int c = threadIdx.x; c < W; c += 256) ss = fmaf(xr[c], xr[c], ss);
   ss = block_sum_256(ss, s4);
   const float r = 1.0f / sqrtf(ss / (float)W + eps);
-  for (int c = threadIdx.x; c < W; c += 256) out[(size_t)blockIdx.x * W + c] = xr[c] * r * (offset + w[c]);
+  for (int c = threadIdx.x; c < W; c += 256) o[c] = xr[c] * r * (offset + w[c]);
 }
 
 // ---- token shift.  One thread per (token, channel): out[t][s] = h_t + (h_(t-1) - h_t) * mu[s] for the n mixes; h_(t-1) is the row before in the entry,

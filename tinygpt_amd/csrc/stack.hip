@@ -26,6 +26,13 @@ int upload_param_ext(tgx_ctx* c, ebyte* dst, const void* host, int64_t n, int sr
 
 namespace {
 int pad4(int n) { return (n + 3) & ~3; }      // row strides of buffers whose rows are read in vectors of four
+// a seam's kernel with as many vectors of four a thread as its width needs (kernels/stack.h, ROW_REG)
+template <class F>
+void launch_seam(int W, F go) {
+  if (W <= 1024) go(std::integral_constant<int, 1>{});
+  else if (W <= 2048) go(std::integral_constant<int, 2>{});
+  else go(std::integral_constant<int, 4>{});
+}
 
 float half_bits_to_f32(uint16_t h) {
   const uint32_t s = (h >> 15) & 1, e = (h >> 10) & 0x1f, m = h & 0x3ff;
@@ -275,6 +282,12 @@ int ensure_part(tgx_ctx* c, size_t elems) {
   return TGX_OK;
 }
 
+void launch_norm_conv(tgx_ctx* c, const tgx::StepMeta& m, const tgx::NormConvArgs& a, int T) {
+  if (a.taps == 4) hipLaunchKernelGGL(tgx::norm_conv_kernel<4>, dim3(T), dim3(256), 0, c->stream, m, a);
+  else if (a.taps == 1) hipLaunchKernelGGL(tgx::norm_conv_kernel<1>, dim3(T), dim3(256), 0, c->stream, m, a);
+  else hipLaunchKernelGGL(tgx::norm_conv_kernel<0>, dim3(T), dim3(256), 0, c->stream, m, a);
+}
+
 // the layers of one step; meta is on the device.  max_keys: the longest context any token of the step attends (host knowledge; picks the attention form)
 int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys, int max_count) {
   StackModel* sm = c->stack;
@@ -290,7 +303,7 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
     tgx::NormConvArgs nc{};
     nc.x = sm->x; nc.nw = w.norm1; nc.cw = w.canon1; nc.out = sm->a; nc.state = nb > 0 ? w.conv_state : nullptr; nc.state_buf = st_buf;
     nc.W = W; nc.groups = sm->d.norm_groups; nc.taps = sm->d.canon_taps; nc.eps = sm->d.norm_eps;
-    hipLaunchKernelGGL(tgx::norm_conv_kernel, dim3(T), dim3(256), 0, c->stream, m, nc);
+    launch_norm_conv(c, m, nc, T);
     // [q | latent | gate] = a . w_in^T
     tgx::StackGemmArgs g{};
     g.A = sm->a; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = nin; g.M = T; g.N = nin; g.K = W; g.scale = 1.f;
@@ -358,7 +371,7 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
     if (ld.mlp == TGX_MLP_MOE) {
       top = ld.top;
       nc.nw = w.norm2; nc.cw = w.canon2; nc.state = nb > 0 ? w.conv_state + 2 * st_buf : nullptr;
-      hipLaunchKernelGGL(tgx::norm_conv_kernel, dim3(T), dim3(256), 0, c->stream, m, nc);
+      launch_norm_conv(c, m, nc, T);
       // router: fp32 weights, fp32 products (nothing is rounded), then bias, top-k and the softmax over the chosen
       g = tgx::StackGemmArgs{};
       g.A = sm->a; g.lda = W; g.B = w.w_router; g.ldb = W; g.C = sm->zr; g.ldc = ld.experts; g.M = T; g.N = ld.experts; g.K = W; g.scale = 1.f;
@@ -650,7 +663,7 @@ int run_layers_sandwich(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_ke
     if (rc) return rc;
     tgx::SandwichArgs sa{};
     sa.x = sm->x; sa.y = sm->yd; sa.top = 1; sa.ytmp = sm->ytmp; sa.g_post = ng + 1; sa.g_next = ld.mlp != TGX_MLP_NONE ? ng + 2 : next_layer; sa.out = hout; sa.W = W; sa.eps = eps;
-    hipLaunchKernelGGL(tgx::sandwich_kernel, dim3(T), dim3(256), 0, c->stream, sa);
+    launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::sandwich_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa); });
     std::swap(hin, hout);
     if (ld.mlp == TGX_MLP_NONE) continue;
     sa = tgx::SandwichArgs{};
@@ -660,7 +673,7 @@ int run_layers_sandwich(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_ke
       run_choice_experts(c, w, hin, T);
       sa.top = ld.top; sa.sel = sm->sel; sa.selw = sm->selw; sa.n_real = ld.experts; sa.h = hin; sa.ysh = ld.shared_ff > 0 ? sm->ysh : nullptr;
     }
-    hipLaunchKernelGGL(tgx::sandwich_kernel, dim3(T), dim3(256), 0, c->stream, sa);
+    launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::sandwich_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa); });
     std::swap(hin, hout);
   }
   return TGX_OK;
@@ -1055,7 +1068,7 @@ int run_layers_affine(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
     sa.x = sm->x; sa.y = sm->yd; sa.top = 1; sa.ytmp = sm->ytmp; sa.w_post = ln + 2 * (size_t)W; sa.b_post = ln + 3 * (size_t)W; sa.mult = mult; sa.out = sm->a; sa.W = W; sa.eps = eps;
     if (ld.mlp != TGX_MLP_NONE) { sa.w_next = ln + 4 * (size_t)W; sa.b_next = ln + 5 * (size_t)W; }
     else if (next_ln) { sa.w_next = next_ln; sa.b_next = next_ln + W; }
-    hipLaunchKernelGGL(tgx::affine_seam_kernel, dim3(T), dim3(256), 0, c->stream, sa);
+    launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::affine_seam_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa); });
     normed = sa.w_next != nullptr;
     if (ld.mlp == TGX_MLP_NONE) continue;
     run_affine_ff(c, w, T);
@@ -1063,7 +1076,7 @@ int run_layers_affine(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
     sa.x = sm->x; sa.y = sm->yd; sa.top = ld.mlp == TGX_MLP_MOE ? ld.top : 1; sa.ysh = ld.mlp == TGX_MLP_MOE && ld.shared_ff > 0 ? sm->ysh : nullptr; sa.ytmp = sm->ytmp;
     sa.w_post = ln + 6 * (size_t)W; sa.b_post = ln + 7 * (size_t)W; sa.mult = mult; sa.out = sm->a; sa.W = W; sa.eps = eps;
     if (next_ln) { sa.w_next = next_ln; sa.b_next = next_ln + W; }
-    hipLaunchKernelGGL(tgx::affine_seam_kernel, dim3(T), dim3(256), 0, c->stream, sa);
+    launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::affine_seam_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa); });
     normed = sa.w_next != nullptr;
   }
   return TGX_OK;
