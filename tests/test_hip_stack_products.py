@@ -185,3 +185,25 @@ def test_norm_and_convolution_of_wide_rows(taps, width, groups):
     eng.close()
     want = so.forward(d, t, toks)
     assert np.abs(got - want).max() / np.abs(want).max() < 1e-4, (taps, width)
+
+
+# ---- layers whose mixer and feed-forward share a decode step's launches (one and two rows, whole slices of eight): against the plain oracle, fp32 sums over at most 320
+# channels (1e-4 of the largest logit as in the design's own tests), and against the same step with each product launched by itself.
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("width,ffn,dim", [(64, 40, 8), (72, 1096, 24), (520, 24, 16)])
+@pytest.mark.parametrize("rows", [1, 2, 3])
+def test_merged_products_of_a_step(rows, width, ffn, dim, dtype):
+    layers = [tv.wkv(tv.ff(ffn), heads=4, dim=dim), tv.par(tv.ff(ffn), left={"heads": 4, "kv_heads": 2, "dim": dim, "vdim": dim + 8, "rot": {"base": 300.0, "dims": 4}}, right={"heads": 4, "kv_heads": 2, "dim": dim, "vdim": 8}),
+              tv.attn(tv.ff(ffn), heads=4, kv_heads=2, dim=dim, vdim=dim), tv.attn(), tv.wkv()]
+    cfg = tv.config(layers, width=width)
+    eng, w = tv.engine(cfg, dtype, seed=width)
+    toks = [tv.tokens(cfg, 6, seed=i) for i in range(rows)]
+    out = []
+    for on in (1, 0):
+        eng.model.set_option("stack.gemv", on)
+        out.append(np.stack([eng.step([((on, i), [toks[i][t]], [0]) for i in range(rows)], [(on, i) for i in range(rows)] if t == 5 else []) for t in range(6)], 1))
+    eng.close()
+    for i in range(rows):
+        want = tv.want_of(cfg, w, toks[i])
+        tv.check(out[0][i], want, "fp32" if dtype == "fp32" else "bf16", f"{rows} rows, row {i}")
+        tv.check(out[1][i], want, "fp32" if dtype == "fp32" else "bf16", f"{rows} rows, row {i}, apart")

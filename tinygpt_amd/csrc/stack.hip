@@ -124,6 +124,11 @@ int line_tile(const tgx_ctx* c, const tgx::StackGemmArgs& a, int epi, int nz, in
   return stack_line_tile(c, a.M, a.N, tgx::sg_dual(epi), nz);
 }
 
+// operands that the weight-streaming kernels' loads take: whole 8-element slices
+bool slices_ok(const tgx::StackGemmArgs& a) {
+  return a.K % 8 == 0 && a.ldb % 8 == 0 && a.b_zstride % 8 == 0 && a.lda % 4 == 0 && a.a_zoff % 4 == 0 && (uintptr_t)a.A % 16 == 0 && (uintptr_t)a.B % 16 == 0 && (!a.B2 || (uintptr_t)a.B2 % 16 == 0);
+}
+
 // nz: batched products (blockIdx.z); grouped products pass the number of their rows and groups (the device-side tile list says how many tiles are real)
 void launch_gemm(tgx_ctx* c, tgx::StackGemmArgs a, int epi, int nz, int grouped_rows = 0, int groups = 0, int grouped_tile = 64, int dt = -1) {
   const StackModel* sm = c->stack;
@@ -145,8 +150,8 @@ void launch_gemm(tgx_ctx* c, tgx::StackGemmArgs a, int epi, int nz, int grouped_
   const bool vec = a.K % kq == 0 && a.ldb % kq == 0 && a.b_zstride % kq == 0 && a.lda % 4 == 0 && a.a_zoff % 4 == 0 && ((uintptr_t)a.A % 16 == 0) && ((uintptr_t)a.B % 16 == 0) &&
                    (!a.B2 || (uintptr_t)a.B2 % 16 == 0);
   const bool dual = tgx::sg_dual(epi);
-  // few rows: the weight-streaming kernel (its loads take whole 8-element slices)
-  const bool few = sm->gemv && vec && a.K % 8 == 0 && a.ldb % 8 == 0 && a.b_zstride % 8 == 0 && (a.z_off ? grouped_tile == GROUPED_FEW_ROWS : (a.M <= FEW_ROWS_MAX || a.N <= FEW_COLS_ANY_ROWS));
+  // few rows: the weight-streaming kernels
+  const bool few = sm->gemv && slices_ok(a) && (a.z_off ? grouped_tile == GROUPED_FEW_ROWS : (a.M <= FEW_ROWS_MAX || a.N <= FEW_COLS_ANY_ROWS));
   if (a.z_off && grouped_tile == GROUPED_FEW_ROWS && !few) { c->launch_fault = "grouped product: the plan was made for the few-row kernel, which these operands cannot take"; return; }
   if (few && (a.z_off || a.M > GEMV_ROWS_MAX)) { launch_stack_few(c, a, epi, nz, a.z_off ? grouped_rows / GROUPED_FEW_ROWS + std::min(groups, grouped_rows) : 0, dt); return; }
   if (few) {
@@ -687,7 +692,41 @@ tgx::StackGemmArgs to_stream(const tgx_ctx* c, const float* A, int K, const ebyt
   g.A = A; g.lda = K; g.B = Wm; g.ldb = K; g.C = sm->x; g.ldc = sm->d.width; g.M = T; g.N = sm->d.width; g.K = K; g.scale = scale;
   return g;
 }
-void add_to_stream(tgx_ctx* c, const float* A, int K, const ebyte* Wm, int T, float scale) { launch_gemm(c, to_stream(c, A, K, Wm, T, scale), tgx::SG_ADD, 1); }
+// One layer's products of one or two rows, collected where its mixer and its feed-forward are independent chains from one input into one stream (kernels/stack_gemm.h):
+// the feed-forward's first product leaves with the mixer's, and everything that the stream takes is added by one launch at the layer's end.  Other steps launch each
+// product where it stands.
+struct JointLayer {
+  bool merged = false;
+  tgx::StackGemmArgs up{};       // the feed-forward's first product (merged layers)
+  tgx::StackGemvSum sum{};
+  int n_sum = 0;
+  int blocks(int N) const { return (N + 4 * tgx::STACK_GEMV_COLS - 1) / (4 * tgx::STACK_GEMV_COLS); }
+  // the mixer's first product (batched by nz) and, where it has one, a second that does not need it
+  void first(tgx_ctx* c, const tgx::StackGemmArgs& p0, int nz, const tgx::StackGemmArgs* p1 = nullptr) {
+    if (!merged) { launch_gemm(c, p0, tgx::SG_STORE, nz); if (p1) launch_gemm(c, *p1, tgx::SG_STORE, 1); return; }
+    tgx::StackGemvGroup g{};
+    g.p0 = p0; g.up = up; g.z0 = nz; g.blocks0 = blocks(p0.N);
+    if (p1) { g.p1 = *p1; g.blocks1 = blocks(p1->N); }
+    g.p0.terms = g.p1.terms = g.up.terms = c->act16 ? 1 : 2;
+    const dim3 grid(g.blocks0 * nz + g.blocks1 + blocks(up.N));
+    TGX_DT_SWITCH(c->dt,
+      if (p0.M == 1) hipLaunchKernelGGL((tgx::stack_gemv_group_kernel<DT, 1>), grid, dim3(256), 0, c->stream, g);
+      else hipLaunchKernelGGL((tgx::stack_gemv_group_kernel<DT, 2>), grid, dim3(256), 0, c->stream, g);)
+  }
+  // x += A . Wm^T * scale
+  void add(tgx_ctx* c, const tgx::StackGemmArgs& p) { if (merged) sum.p[n_sum++] = p; else launch_gemm(c, p, tgx::SG_ADD, 1); }
+  void finish(tgx_ctx* c) {
+    if (!n_sum) return;
+    for (int s = 0; s < n_sum; s++) sum.p[s].terms = c->act16 ? 1 : 2;
+    const dim3 grid((sum.p[0].N + tgx::STACK_GEMV_COLS - 1) / tgx::STACK_GEMV_COLS);
+    TGX_DT_SWITCH(c->dt,
+      auto go = [&](auto NS) {
+        if (sum.p[0].M == 1) hipLaunchKernelGGL((tgx::stack_gemv_sum_kernel<DT, decltype(NS)::value, 1>), grid, dim3(256), 0, c->stream, sum);
+        else hipLaunchKernelGGL((tgx::stack_gemv_sum_kernel<DT, decltype(NS)::value, 2>), grid, dim3(256), 0, c->stream, sum);
+      };
+      if (n_sum == 2) go(std::integral_constant<int, 2>{}); else go(std::integral_constant<int, 3>{});)
+  }
+};
 
 void launch_rec_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs& a, int kind, int S) {
   const bool vec = a.dim % 4 == 0 && a.lda % 4 == 0 && a.ldk % 4 == 0 && (uintptr_t)a.a % 16 == 0 && (uintptr_t)a.k % 16 == 0 && (!a.w || (a.ldw % 4 == 0 && (uintptr_t)a.w % 16 == 0));
@@ -716,14 +755,14 @@ void launch_rec_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs&
   else go(std::integral_constant<int, tgx::REC_DELTA>{});
 }
 
-int run_joint_attention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int S, int max_keys, int max_count) {
+int run_joint_attention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer& jl, int T, int S, int max_keys, int max_count) {
   StackModel* sm = c->stack;
   const tgx_layer_desc& ld = w.d;
   const bool shared = w.kv_src >= 0;
   const int W = sm->d.width, H = ld.heads, G = ld.kv_heads, qd = H * ld.dim, vd = H * ld.vdim, nin = qd + (shared ? 0 : G * (ld.dim + ld.vdim));
   tgx::StackGemmArgs g{};
   g.A = sm->a; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = nin; g.M = T; g.N = nin; g.K = W; g.scale = 1.f;
-  launch_gemm(c, g, tgx::SG_STORE, 1);
+  jl.first(c, g, 1);
   GqaSpec sp{};
   sp.proj = sm->proj; sp.ldp = nin; sp.heads = H; sp.kv_heads = G; sp.dim = ld.dim; sp.vdim = ld.vdim; sp.rot_dims = ld.rot_dims; sp.rot_pairs = ld.rot_pairs;
   sp.cs = w.rot >= 0 ? sm->rot[(size_t)w.rot].cs : nullptr; sp.poolK = w.pool; sp.poolV = w.poolV; sp.poolVT = w.poolVT; sp.append = !shared;
@@ -731,11 +770,11 @@ int run_joint_attention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int 
   sp.q_temp_coef = ld.q_temp_coef; sp.q_temp_every = ld.q_temp_every; sp.out = sm->o; sp.ldo = vd;
   int rc = run_gqa_core(c, m, sp, T, S, max_keys, max_count);
   if (rc) return rc;
-  add_to_stream(c, sm->o, vd, w.w_o, T, sm->d.residual_mult);
+  jl.add(c, to_stream(c, sm->o, vd, w.w_o, T, sm->d.residual_mult));
   return TGX_OK;
 }
 
-void run_wkv(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int S) {
+void run_wkv(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer& jl, int T, int S) {
   StackModel* sm = c->stack;
   const tgx_layer_desc& ld = w.d;
   const int W = sm->d.width, H = ld.heads, HD = H * ld.dim, R = ld.decay_rank;
@@ -746,10 +785,10 @@ void run_wkv(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int S) {
   tgx::StackGemmArgs g{};
   g.A = sm->mixed; g.lda = 5LL * W; g.a_zoff = W; g.B = w.w_in; g.ldb = W; g.b_zstride = (long long)HD * W; g.C = sm->proj; g.ldc = 5LL * HD; g.c_zoff = HD;
   g.M = T; g.N = HD; g.K = W; g.scale = 1.f;
-  launch_gemm(c, g, tgx::SG_STORE, 4);
+  const tgx::StackGemmArgs rkvg = g;
   g = tgx::StackGemmArgs{};
   g.A = sm->mixed + 4 * (size_t)W; g.lda = 5LL * W; g.B = w.w_w1; g.ldb = W; g.C = sm->lora; g.ldc = R; g.M = T; g.N = R; g.K = W; g.scale = 1.f; g.act = tgx::SG_ACT_TANH;
-  launch_gemm(c, g, tgx::SG_STORE, 1);
+  jl.first(c, rkvg, 4, &g);
   g = tgx::StackGemmArgs{};
   g.A = sm->lora; g.lda = R; g.B = w.w_w2; g.ldb = R; g.C = sm->proj + 4 * (size_t)HD; g.ldc = 5LL * HD; g.M = T; g.N = HD; g.K = R; g.scale = 1.f; g.bias = w.w0; g.act = tgx::SG_ACT_DECAY;
   launch_gemm(c, g, tgx::SG_STORE, 1);
@@ -761,10 +800,10 @@ void run_wkv(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int S) {
   oa.hs = sm->hs; oa.ldh = HD; oa.w = w.head_w; oa.w_hstride = ld.dim; oa.gate = sm->proj + 3 * (size_t)HD; oa.ldg = 5LL * HD; oa.silu_gate = 1; oa.out = sm->o; oa.ldo = HD; oa.vdim = ld.dim;
   oa.eps = sm->d.norm_eps;
   hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, H), dim3(64), 0, c->stream, oa);
-  add_to_stream(c, sm->o, HD, w.w_o, T, sm->d.residual_mult);
+  jl.add(c, to_stream(c, sm->o, HD, w.w_o, T, sm->d.residual_mult));
 }
 
-int run_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int S, int max_keys, int max_count) {
+int run_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer& jl, int T, int S, int max_keys, int max_count) {
   StackModel* sm = c->stack;
   const tgx_layer_desc& ld = w.d;
   const int W = sm->d.width, H = ld.heads, G = ld.kv_heads, lq = H * ld.dim, lkv = G * (ld.dim + ld.vdim), lvd = H * ld.vdim;
@@ -772,7 +811,7 @@ int run_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int 
   // [left q | k | v | right q | k | v | b | a | g] = h . w_in^T: both halves read the same input
   tgx::StackGemmArgs g{};
   g.A = sm->a; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = nin; g.M = T; g.N = nin; g.K = W; g.scale = 1.f;
-  launch_gemm(c, g, tgx::SG_STORE, 1);
+  jl.first(c, g, 1);
   GqaSpec sp{};
   sp.proj = sm->proj; sp.ldp = nin; sp.heads = H; sp.kv_heads = G; sp.dim = ld.dim; sp.vdim = ld.vdim; sp.rot_dims = ld.rot_dims; sp.rot_pairs = ld.rot_pairs;
   sp.cs = w.rot >= 0 ? sm->rot[(size_t)w.rot].cs : nullptr; sp.poolK = w.pool; sp.poolV = w.poolV; sp.poolVT = w.poolVT; sp.append = true;
@@ -780,7 +819,9 @@ int run_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int 
   sp.q_temp_coef = ld.q_temp_coef; sp.q_temp_every = ld.q_temp_every; sp.out = sm->o; sp.ldo = lvd;
   int rc = run_gqa_core(c, m, sp, T, S, max_keys, max_count);
   if (rc) return rc;
-  add_to_stream(c, sm->o, lvd, w.w_o, T, sm->d.residual_mult * ld.left_scale);
+  jl.add(c, to_stream(c, sm->o, lvd, w.w_o, T, sm->d.residual_mult * ld.left_scale));
+  // (the left half's outputs stay until the layer's sum)
+  float* ro = sm->o + (jl.merged ? GEMV_ROWS_MAX * (size_t)sm->max_hv : 0);
   // the right half: rec_in row = [q | k | v | beta | decay]
   const int ldr = rC + 2 * rH, nb = ld.conv_taps - 1;
   tgx::DeltaPrepArgs dp{};
@@ -793,10 +834,10 @@ int run_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int 
   ra.beta = sm->rec_in + rC; ra.g = sm->rec_in + rC + rH; ra.ldg = ldr; ra.S = w.mS; ra.out = sm->hs; ra.ldo = rvd; ra.heads = rH; ra.kv_heads = rG; ra.dim = ld.d_dim; ra.vdim = ld.d_vdim;
   launch_rec_scan(c, m, ra, tgx::REC_DELTA, S);
   tgx::HeadNormGateArgs oa{};
-  oa.hs = sm->hs; oa.ldh = rvd; oa.w = w.head_w; oa.w_hstride = 0; oa.gate = sm->proj + lq + lkv + rC + 2 * rH; oa.ldg = nin; oa.silu_gate = 1; oa.out = sm->o; oa.ldo = rvd; oa.vdim = ld.d_vdim;
+  oa.hs = sm->hs; oa.ldh = rvd; oa.w = w.head_w; oa.w_hstride = 0; oa.gate = sm->proj + lq + lkv + rC + 2 * rH; oa.ldg = nin; oa.silu_gate = 1; oa.out = ro; oa.ldo = rvd; oa.vdim = ld.d_vdim;
   oa.eps = sm->d.norm_eps;
   hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, rH), dim3(64), 0, c->stream, oa);
-  add_to_stream(c, sm->o, rvd, w.w_o2, T, sm->d.residual_mult * ld.right_scale);
+  jl.add(c, to_stream(c, ro, rvd, w.w_o2, T, sm->d.residual_mult * ld.right_scale));
   return TGX_OK;
 }
 
@@ -810,14 +851,24 @@ int run_layers_joint(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys,
     const tgx_layer_desc& ld = w.d;
     hipLaunchKernelGGL(tgx::offset_norm_kernel, dim3(T), dim3(256), 0, c->stream, sm->x, nullptr, w.norm1, 1.0f, sm->a, W, sm->d.norm_eps);
     int rc = TGX_OK;
-    if (ld.mixer == TGX_MIXER_ATTENTION) rc = run_joint_attention(c, m, w, T, S, max_keys, max_count);
-    else if (ld.mixer == TGX_MIXER_WKV) run_wkv(c, m, w, T, S);
-    else rc = run_parallel(c, m, w, T, S, max_keys, max_count);
-    if (rc) return rc;
+    JointLayer jl;
+    tgx::StackGemmArgs g{};
     if (ld.mlp == TGX_MLP_DENSE) {      // x += mult * down(silu(gate h) * (up h))
-      tgx::StackGemmArgs g{};
       g.A = sm->a; g.lda = W; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.C = sm->yh; g.ldc = ld.ff; g.M = T; g.N = ld.ff; g.K = W;
-      launch_ff(c, g, tgx::SG_SILU_MUL, to_stream(c, sm->yh, ld.ff, w.w_down, T, sm->d.residual_mult), tgx::SG_ADD);
+      jl.up = g;
+      // every product that joins a launch must take the weight-streaming kernel by itself (one or two rows, whole slices)
+      const int outs[] = {ld.heads * (ld.mixer == TGX_MIXER_WKV ? ld.dim : ld.vdim), ld.mixer == TGX_MIXER_PARALLEL ? ld.d_heads * ld.d_vdim : 0, ld.ff, W, ld.mixer == TGX_MIXER_PARALLEL ? sm->max_hv : 0};
+      jl.merged = sm->gemv && T <= GEMV_ROWS_MAX;
+      for (int k : outs) jl.merged = jl.merged && k % 8 == 0;
+    }
+    if (ld.mixer == TGX_MIXER_ATTENTION) rc = run_joint_attention(c, m, w, jl, T, S, max_keys, max_count);
+    else if (ld.mixer == TGX_MIXER_WKV) run_wkv(c, m, w, jl, T, S);
+    else rc = run_parallel(c, m, w, jl, T, S, max_keys, max_count);
+    if (rc) return rc;
+    if (ld.mlp == TGX_MLP_DENSE) {
+      const tgx::StackGemmArgs down = to_stream(c, sm->yh, ld.ff, w.w_down, T, sm->d.residual_mult);
+      if (jl.merged) { jl.add(c, down); jl.finish(c); }
+      else launch_ff(c, g, tgx::SG_SILU_MUL, down, tgx::SG_ADD);
     }
   }
   return TGX_OK;
