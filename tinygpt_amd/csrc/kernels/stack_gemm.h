@@ -285,14 +285,14 @@ constexpr int STACK_GEMV_COLS = 2;      // output columns per wave
 
 // ---- the same products for ONE or TWO rows (decode steps): a weight-streaming kernel.  One wave per pair of output columns: every lane takes 8 weights of each
 // column per pass (one 16-byte load for the 16-bit dtypes) against the 8 activations of up to MR rows, fp32 FMA chains, one cross-lane sum per (row, column)
-// at the end.  Same argument block, batching (blockIdx.z) and epilogues as stack_gemm_kernel; the activations
+// at the end.  KSPLIT: the four waves divide the slices of one pair of columns (their sums meet in LDS): four times the workgroups.  Same argument block, batching (blockIdx.z) and epilogues as stack_gemm_kernel; the activations
 // enter in fp32 (rounded to the storage dtype first under option act.round16).  Needs the vector-load alignment (K a multiple of 8).
-template <int DT, int EPI, bool DUAL, int MR>
+template <int DT, int EPI, bool DUAL, int MR, bool KSPLIT = false>
 __device__ __forceinline__ void stack_gemv_body(const StackGemmArgs& a, int bx, int by, int z) {
   constexpr int NC = STACK_GEMV_COLS, NB = DUAL ? 2 : 1;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int mbase = by * MR, mend = min(a.M, mbase + MR);
-  const int n0 = (bx * 4 + wv) * NC;
+  const int n0 = (KSPLIT ? bx : bx * 4 + wv) * NC;
   if (n0 >= a.N) return;
   const float* Ab = a.A + (size_t)z * a.a_zoff;
   const float* arow[MR];
@@ -313,8 +313,8 @@ __device__ __forceinline__ void stack_gemv_body(const StackGemmArgs& a, int bx, 
       for (int r = 0; r < MR; r++) acc[b][j][r] = 0.f;
   const int round16 = a.terms == 1;
   const int nsl = a.K >> 3;                               // 8-element slices of a row
-  for (int s0 = lane; s0 < nsl; s0 += 128) {              // two slices per lane and pass: twice the loads in flight
-    const int s1 = s0 + 64;
+  for (int s0 = KSPLIT ? 64 * wv + lane : lane; s0 < nsl; s0 += KSPLIT ? 512 : 128) {              // two slices per lane and pass: twice the loads in flight
+    const int s1 = s0 + (KSPLIT ? 256 : 64);
     const bool two = s1 < nsl;
     Slice8<DT> w0[NB][NC], w1[NB][NC];
 #pragma unroll
@@ -342,6 +342,23 @@ __device__ __forceinline__ void stack_gemv_body(const StackGemmArgs& a, int bx, 
     for (int j = 0; j < NC; j++)
 #pragma unroll
       for (int r = 0; r < MR; r++) acc[b][j][r] = wave_sum(acc[b][j][r]);
+  if constexpr (KSPLIT) {
+    __shared__ float s_part[4][NB * NC * MR];
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int j = 0; j < NC; j++)
+#pragma unroll
+        for (int r = 0; r < MR; r++) if (lane == 0) s_part[wv][(b * NC + j) * MR + r] = acc[b][j][r];
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int j = 0; j < NC; j++)
+#pragma unroll
+        for (int r = 0; r < MR; r++) { const int at = (b * NC + j) * MR + r; acc[b][j][r] = s_part[0][at] + s_part[1][at] + s_part[2][at] + s_part[3][at]; }
+    if (wv) return;
+  }
   // one output a lane, so that the epilogues' loads (bias, gate, the stream itself) are one round trip and not one after the other
   float v = acc[0][0][0], v2 = acc[NB - 1][0][0];
 #pragma unroll
@@ -352,8 +369,8 @@ __device__ __forceinline__ void stack_gemv_body(const StackGemmArgs& a, int bx, 
   const int m = mbase + lane / NC, n = n0 + lane % NC;
   if (lane < MR * NC && m < mend && n < a.N) sg_finish<EPI>(a, z, m, n, v, v2);
 }
-template <int DT, int EPI, bool DUAL, int MR>
-__global__ __launch_bounds__(256) void stack_gemv_kernel(const StackGemmArgs a) { stack_gemv_body<DT, EPI, DUAL, MR>(a, blockIdx.x, blockIdx.y, blockIdx.z); }
+template <int DT, int EPI, bool DUAL, int MR, bool KSPLIT>
+__global__ __launch_bounds__(256) void stack_gemv_kernel(const StackGemmArgs a) { stack_gemv_body<DT, EPI, DUAL, MR, KSPLIT>(a, blockIdx.x, blockIdx.y, blockIdx.z); }
 
 // ---- a layer whose mixer and feed-forward read the same input and add to the same stream.  A decode step is bound by its launches (1024 x 1024 streams 2 MB in 0.4 us and
 // takes 2.6), so the products that stand at the same place of the two chains share one:

@@ -83,9 +83,11 @@ void launch_gemm_t(tgx_ctx* c, const tgx::StackGemmArgs& a, dim3 grid1, dim3 gri
   else { if (vec) go(std::integral_constant<int, 2>{}, std::true_type{}); else go(std::integral_constant<int, 2>{}, std::false_type{}); }
 }
 template <int DT, int EPI, bool DUAL>
-void launch_gemv_t(tgx_ctx* c, const tgx::StackGemmArgs& a, dim3 grid, int mr) {
-  if (mr == 1) hipLaunchKernelGGL((tgx::stack_gemv_kernel<DT, EPI, DUAL, 1>), grid, dim3(256), 0, c->stream, a);
-  else hipLaunchKernelGGL((tgx::stack_gemv_kernel<DT, EPI, DUAL, 2>), grid, dim3(256), 0, c->stream, a);
+void launch_gemv_t(tgx_ctx* c, const tgx::StackGemmArgs& a, dim3 grid, int mr, bool ksplit) {
+  auto go = [&](auto R, auto S) { hipLaunchKernelGGL((tgx::stack_gemv_kernel<DT, EPI, DUAL, decltype(R)::value, decltype(S)::value>), grid, dim3(256), 0, c->stream, a); };
+  if (mr == 1) { if (ksplit) go(std::integral_constant<int, 1>{}, std::true_type{}); else go(std::integral_constant<int, 1>{}, std::false_type{}); }
+  else if (ksplit) go(std::integral_constant<int, 2>{}, std::true_type{});
+  else go(std::integral_constant<int, 2>{}, std::false_type{});
 }
 // rows per tile of a grouped product's plan (moe_plan_kernel tile_m): steps of few (token, expert) pairs stream the experts through the few-row kernel
 constexpr int GROUPED_FEW_PAIRS = 128, GROUPED_FEW_ROWS = 16, FEW_ROWS_MAX = 64;
@@ -129,6 +131,11 @@ bool slices_ok(const tgx::StackGemmArgs& a) {
   return a.K % 8 == 0 && a.ldb % 8 == 0 && a.b_zstride % 8 == 0 && a.lda % 4 == 0 && a.a_zoff % 4 == 0 && (uintptr_t)a.A % 16 == 0 && (uintptr_t)a.B % 16 == 0 && (!a.B2 || (uintptr_t)a.B2 % 16 == 0);
 }
 
+// whether the four waves of a workgroup divide the slices of two columns instead of taking two columns each: while the
+// columns alone leave a compute unit with fewer than two workgroups and there are slices to divide (the products of a step of two rows at a width of 1024: 6.0 us each on average
+// undivided, 5.0 divided; products of more columns already stream at memory's rate)
+bool gemv_ksplit(const tgx_ctx* c, const tgx::StackGemmArgs& a, int nz) { return a.K >= 512 && (long long)((a.N + 7) / 8) * nz < 2LL * c->num_cus; }
+
 // nz: batched products (blockIdx.z); grouped products pass the number of their rows and groups (the device-side tile list says how many tiles are real)
 void launch_gemm(tgx_ctx* c, tgx::StackGemmArgs a, int epi, int nz, int grouped_rows = 0, int groups = 0, int grouped_tile = 64, int dt = -1) {
   const StackModel* sm = c->stack;
@@ -156,16 +163,17 @@ void launch_gemm(tgx_ctx* c, tgx::StackGemmArgs a, int epi, int nz, int grouped_
   if (few && (a.z_off || a.M > GEMV_ROWS_MAX)) { launch_stack_few(c, a, epi, nz, a.z_off ? grouped_rows / GROUPED_FEW_ROWS + std::min(groups, grouped_rows) : 0, dt); return; }
   if (few) {
     const int mr = a.M <= 1 ? 1 : 2;
-    const int cols = 4 * tgx::STACK_GEMV_COLS;      // per workgroup
+    const bool ksplit = gemv_ksplit(c, a, nz);
+    const int cols = (ksplit ? 1 : 4) * tgx::STACK_GEMV_COLS;      // per workgroup
     const dim3 grid((a.N + cols - 1) / cols, (a.M + mr - 1) / mr, nz);
     TGX_DT_SWITCH(dt,
       switch (epi) {
-        case tgx::SG_STORE: launch_gemv_t<DT, tgx::SG_STORE, false>(c, a, grid, mr); break;
-        case tgx::SG_ADD: launch_gemv_t<DT, tgx::SG_ADD, false>(c, a, grid, mr); break;
-        case tgx::SG_GATE: launch_gemv_t<DT, tgx::SG_GATE, false>(c, a, grid, mr); break;
-        case tgx::SG_ROWSCALE: launch_gemv_t<DT, tgx::SG_ROWSCALE, false>(c, a, grid, mr); break;
-        case tgx::SG_SILU_MUL: launch_gemv_t<DT, tgx::SG_SILU_MUL, true>(c, a, grid, mr); break;
-        default: if (dual) launch_gemv_t<DT, tgx::SG_EXPERT_ACT, true>(c, a, grid, mr); break;
+        case tgx::SG_STORE: launch_gemv_t<DT, tgx::SG_STORE, false>(c, a, grid, mr, ksplit); break;
+        case tgx::SG_ADD: launch_gemv_t<DT, tgx::SG_ADD, false>(c, a, grid, mr, ksplit); break;
+        case tgx::SG_GATE: launch_gemv_t<DT, tgx::SG_GATE, false>(c, a, grid, mr, ksplit); break;
+        case tgx::SG_ROWSCALE: launch_gemv_t<DT, tgx::SG_ROWSCALE, false>(c, a, grid, mr, ksplit); break;
+        case tgx::SG_SILU_MUL: launch_gemv_t<DT, tgx::SG_SILU_MUL, true>(c, a, grid, mr, ksplit); break;
+        default: if (dual) launch_gemv_t<DT, tgx::SG_EXPERT_ACT, true>(c, a, grid, mr, ksplit); break;
       })
     return;
   }
