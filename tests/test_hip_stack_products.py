@@ -207,3 +207,31 @@ def test_merged_products_of_a_step(rows, width, ffn, dim, dtype):
         want = tv.want_of(cfg, w, toks[i])
         tv.check(out[0][i], want, "fp32" if dtype == "fp32" else "bf16", f"{rows} rows, row {i}")
         tv.check(out[1][i], want, "fp32" if dtype == "fp32" else "bf16", f"{rows} rows, row {i}, apart")
+
+
+# ---- choice kernels that take the router's products themselves (up to 64 rows and 64 products): widths around a wave's 256 channels a load, expert counts around the four
+# of a wave's pass, beside the step of one row more that takes the general products.  fp32 storage against the plain oracles: 1e-4 of the largest logit as above.
+@pytest.mark.parametrize("width", [8, 252, 260, 1028])
+@pytest.mark.parametrize("experts,identity", [(3, 1), (13, 2), (62, 2), (63, 3)])
+@pytest.mark.parametrize("rows", [1, 64, 65])
+def test_router_products_in_the_choice(rows, experts, identity, width):
+    cfg = tm.config([tm.attn(tm.moe(experts=experts, identity=identity, top=3, count=1, keep=1))], width=width)
+    eng, w = tm.engine(cfg, seed=experts + width)
+    toks = tm.tokens(cfg, rows, seed=rows)
+    got = tm.run_whole(eng, "a", toks)
+    eng.close()
+    tm.check(got, tm.want_of(cfg, w, toks), "fp32", f"{rows} rows")
+
+
+@pytest.mark.parametrize("experts", [2, 5, 16, 17, 64, 65])
+@pytest.mark.parametrize("rows", [1, 63, 64, 65])
+def test_router_products_in_the_biased_choice(rows, experts):
+    layers = [LayerDesc(heads=3, dim=8, vdim=8, kv_rank=24, scale=0.35, mlp="moe", experts=experts, top=2, ff=24, limit=1.5)]
+    d = StackDesc(width=76, vocab=53, canon_taps=2, norm_groups=2, norm_eps=1e-6, max_seqs=2, max_ctx=128, budget_tokens=256, compute_dtype="fp32", layers=layers)
+    t = so.random_tensors(d, experts)
+    toks = np.random.default_rng(rows).integers(0, 53, rows).tolist()
+    eng = SlotEngine(desc=d, tensors={k: v.astype(np.float32) for k, v in t.items()})
+    got = eng.step([("a", toks, list(range(rows)))])
+    eng.close()
+    want = so.forward(d, t, toks)
+    assert np.abs(got - want).max() / np.abs(want).max() < 1e-4, (rows, experts)

@@ -360,8 +360,69 @@ __global__ __launch_bounds__(256) void latent_attn_merge_kernel(LatentAttnArgs a
   }
 }
 
-// ---- router: the `top` largest of z + b (z = Wr h, an fp32 product of fp32 weights; ties: the lower index), weights = softmax over them.  One wave per token.
+// LDS that one wave writes and reads: its accesses stay in program order
+__device__ __forceinline__ void wave_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); }
+
+// ---- the products of a router for one token, w [n][K] . h [K] in fp32, by a workgroup of four waves into LDS.  A step of few tokens is bound by its launches (16 tokens of
+// 1024 channels, 8 experts: 5.5 us for the products and 4.4 for the choice behind them, 4.2 together), so its choice kernels take the products themselves.
+struct RouterInput { const float* h; long long ldh; const float* w; int n, K; };      // h nullptr: the products are given
+constexpr int ROUTER_FUSED_MAX = 64;      // products a choice kernel takes itself
+__device__ __forceinline__ void router_products(const RouterInput& in, int t, float* s_z) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const float* h = in.h + (size_t)t * in.ldh;
+  for (int e0 = 4 * wv; e0 < in.n; e0 += 16) {
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 4 * lane; k0 < in.K; k0 += 1024) {      // every load of 1024 channels and four products in flight at once; loads past the end repeat it and are dropped
+      f32x4 x[4], w[4][4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int k = min(k0 + 256 * i, in.K - 4);
+        x[i] = *reinterpret_cast<const f32x4*>(h + k);
+#pragma unroll
+        for (int j = 0; j < 4; j++) w[i][j] = *reinterpret_cast<const f32x4*>(in.w + (size_t)min(e0 + j, in.n - 1) * in.K + k);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const bool on = k0 + 256 * i < in.K;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+#pragma unroll
+          for (int j = 0; j < 4; j++) acc[j] = on ? fmaf(x[i][u], w[i][j][u], acc[j]) : acc[j];
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) { const float v = wave_sum(acc[j]); if (lane == 0 && e0 + j < in.n) s_z[e0 + j] = v; }
+  }
+  __syncthreads();
+}
+
+// the largest of s[0 .. n) and its index (ties: the lower; 0x7fffffff where all are -inf), in every lane of the wave.  ONE: n <= 64, a number per lane: the
+// maximum alone crosses the lanes and a ballot finds its first holder
+template <bool ONE>
+__device__ __forceinline__ int wave_pick(const float* s, int n, float& bv) {
+  const int lane = threadIdx.x & 63;
+  if constexpr (ONE) {
+    const float v = lane < n ? s[lane] : -INFINITY;
+    bv = group_max<64>(v);
+    const unsigned long long mask = __ballot(v == bv && v > -INFINITY);
+    return mask ? (int)__builtin_ctzll(mask) : 0x7fffffff;
+  }
+  int bi = 0x7fffffff;
+  bv = -INFINITY;
+  for (int e = lane; e < n; e += 64) { const float v = s[e]; if (v > bv) { bv = v; bi = e; } }
+  for (int o = 32; o > 0; o >>= 1) {
+    const float ov = __shfl_xor(bv, o, 64); const int oi = __shfl_xor(bi, o, 64);
+    if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
+  }
+  return bi;
+}
+
+// ---- router: the `top` largest of z + b (z = Wr h, an fp32 product of fp32 weights; ties: the lower index), weights = softmax over them.  One wave per token (and three
+// more for its products where `in` gives them).
 struct RouterArgs {
+  RouterInput in;
   const float* z;        // [T][E] router products
   const float* br;       // [E]
   int* sel;              // [T][top]
@@ -369,30 +430,30 @@ struct RouterArgs {
   int E, top;
 };
 constexpr int ROUTER_MAX_E = 1024, ROUTER_MAX_TOP = 64;
-__global__ __launch_bounds__(64) void router_topk_kernel(RouterArgs a) {
+template <bool PRODUCT>
+__global__ __launch_bounds__(PRODUCT ? 256 : 64) void router_topk_kernel(RouterArgs a) {
   __shared__ float s_z[ROUTER_MAX_E];
   __shared__ float s_v[ROUTER_MAX_TOP];
   __shared__ int s_i[ROUTER_MAX_TOP];
   const int t = blockIdx.x, lane = threadIdx.x;
   // every lane owns the logits e = lane, lane + 64, ...: it alone writes, reads and retires them, so the loop needs no barrier; the butterfly leaves each
   // pick in all lanes, lane 0 keeps the list
-  for (int e = lane; e < a.E; e += 64) s_z[e] = a.z[(size_t)t * a.E + e] + a.br[e];
+  if constexpr (PRODUCT) {
+    router_products(a.in, t, s_z);
+    if (lane >= 64) return;      // (no barrier below)
+    for (int e = lane; e < a.E; e += 64) s_z[e] += a.br[e];
+  } else for (int e = lane; e < a.E; e += 64) s_z[e] = a.z[(size_t)t * a.E + e] + a.br[e];
   for (int k = 0; k < a.top; k++) {
-    float bv = -INFINITY; int bi = 0x7fffffff;
-    for (int e = lane; e < a.E; e += 64) { const float v = s_z[e]; if (v > bv) { bv = v; bi = e; } }
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64); const int oi = __shfl_xor(bi, o, 64);
-      if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-    }
+    float bv;
+    const int bi = wave_pick<PRODUCT>(s_z, a.E, bv);
     if (bi < a.E && (bi & 63) == lane) s_z[bi] = -INFINITY;
     if (lane == 0) { s_v[k] = bv; s_i[k] = bi < a.E ? bi : 0; }
   }
-  if (lane == 0) {
-    const float mx = s_v[0];            // the first pick is the largest
-    float den = 0.f;
-    for (int k = 0; k < a.top; k++) den += expf(s_v[k] - mx);
-    for (int k = 0; k < a.top; k++) { a.sel[(size_t)t * a.top + k] = s_i[k]; a.selw[(size_t)t * a.top + k] = expf(s_v[k] - mx) / den; }
-  }
+  wave_fence();
+  const float mx = s_v[0];            // the first pick is the largest
+  float den = 0.f;
+  for (int k = 0; k < a.top; k++) den += expf(s_v[k] - mx);
+  for (int k = lane; k < a.top; k += 64) { a.sel[(size_t)t * a.top + k] = s_i[k]; a.selw[(size_t)t * a.top + k] = expf(s_v[k] - mx) / den; }
 }
 
 // ---- plan of the grouped expert products: pairs i = t * top + k grouped by expert.  One workgroup.

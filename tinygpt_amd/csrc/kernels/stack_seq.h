@@ -555,6 +555,7 @@ __global__ __launch_bounds__(64) void head_norm_gate_kernel(HeadNormGateArgs a) 
 // Variants: sigmoid_scores: s = sigmoid(z) instead of the softmax (corr may be nullptr: no correction); group_top2: a group counts as the sum of its two
 // largest choice scores; normalise: the chosen weights are divided by their sum + 1e-20 (before the scale).
 struct RouterGroupArgs {
+  RouterInput in;
   const float* z; int ldz;
   const float* corr;         // [E]
   int* sel; float* selw;     // [T][top]
@@ -564,10 +565,17 @@ struct RouterGroupArgs {
   int sigmoid_scores, group_top2, normalise;
   int shared;                // 1: every token has one more choice behind its top: expert E with weight 1 (a shared expert that rides among the routed ones)
 };
-__global__ __launch_bounds__(64) void router_group_kernel(RouterGroupArgs a) {
-  __shared__ float s_s[ROUTER_MAX_E], s_c[ROUTER_MAX_E], s_g[ROUTER_MAX_E];
+template <bool PRODUCT>
+__global__ __launch_bounds__(PRODUCT ? 256 : 64) void router_group_kernel(RouterGroupArgs a) {
+  constexpr int ME = PRODUCT ? ROUTER_FUSED_MAX : ROUTER_MAX_E;
+  __shared__ float s_s[ME], s_c[ME], s_g[ME], s_z[PRODUCT ? ME : 1], s_pw[ROUTER_MAX_TOP];
+  __shared__ int s_pick[ROUTER_MAX_TOP];
   const int t = blockIdx.x, lane = threadIdx.x, stride = a.top + a.shared;
-  const float* z = a.z + (size_t)t * a.ldz;
+  const float* z = s_z;
+  if constexpr (PRODUCT) {
+    router_products(a.in, t, s_z);
+    if (threadIdx.x >= 64) return;      // one wave chooses: its barriers below are its own
+  } else z = a.z + (size_t)t * a.ldz;
   if (a.sigmoid_scores) {
     for (int e = lane; e < a.E; e += 64) { s_s[e] = 1.0f / (1.0f + expf(-z[e])); s_c[e] = a.corr ? s_s[e] + a.corr[e] : s_s[e]; }
   } else {
@@ -579,7 +587,7 @@ __global__ __launch_bounds__(64) void router_group_kernel(RouterGroupArgs a) {
     den = wave_sum(den);
     for (int e = lane; e < a.E; e += 64) { s_s[e] = s_s[e] / den; s_c[e] = a.corr ? s_s[e] + a.corr[e] : s_s[e]; }
   }
-  __syncthreads();
+  wave_fence();
   if (a.groups > 1) {
     const int per = a.E / a.groups;
     for (int g = lane; g < a.groups; g += 64) {
@@ -587,7 +595,7 @@ __global__ __launch_bounds__(64) void router_group_kernel(RouterGroupArgs a) {
       for (int e = g * per; e < (g + 1) * per; e++) { const float v = s_c[e]; if (v > b) { b2 = b; b = v; } else b2 = fmaxf(b2, v); }
       s_g[g] = a.group_top2 && per > 1 ? b + b2 : b;
     }
-    __syncthreads();
+    wave_fence();
     // the `keep` best groups, one pick per round; a kept group is marked by +inf, the others end as dropped
     for (int k = 0; k < a.keep; k++) {
       float bv = -INFINITY; int bi = 0x7fffffff;
@@ -598,31 +606,23 @@ __global__ __launch_bounds__(64) void router_group_kernel(RouterGroupArgs a) {
       }
       if (bi < a.groups && (bi & 63) == lane) s_g[bi] = INFINITY;
     }
-    __syncthreads();
+    wave_fence();
     for (int e = lane; e < a.E; e += 64) if (s_g[e / per] != INFINITY) s_c[e] = -INFINITY;
-    __syncthreads();
+    wave_fence();
   }
+  float sum = 0.f;      // in choice order
   for (int k = 0; k < a.top; k++) {
-    float bv = -INFINITY; int bi = 0x7fffffff;
-    for (int e = lane; e < a.E; e += 64) { const float v = s_c[e]; if (v > bv) { bv = v; bi = e; } }
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64); const int oi = __shfl_xor(bi, o, 64);
-      if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-    }
+    float bv;
+    const int bi = wave_pick<PRODUCT>(s_c, a.E, bv), pick = bi < a.E ? bi : 0;
     if (bi < a.E && (bi & 63) == lane) s_c[bi] = -INFINITY;
-    if (lane == 0) {
-      const int pick = bi < a.E ? bi : 0;
-      a.sel[(size_t)t * stride + k] = pick;
-      a.selw[(size_t)t * stride + k] = bi < a.E ? s_s[pick] * a.scale : 0.f;
-    }
+    const float v = bi < a.E ? s_s[pick] * a.scale : 0.f;
+    sum += v;
+    if (lane == 0) { s_pick[k] = pick; s_pw[k] = v; }
   }
+  wave_fence();
+  const float inv = a.normalise ? a.scale / (sum + 1e-20f * a.scale) : 1.f;
+  for (int k = lane; k < a.top; k += 64) { a.sel[(size_t)t * stride + k] = s_pick[k]; a.selw[(size_t)t * stride + k] = a.normalise ? s_pw[k] * inv : s_pw[k]; }
   if (a.shared && lane == 0) { a.sel[(size_t)t * stride + a.top] = a.E; a.selw[(size_t)t * stride + a.top] = 1.f; }
-  if (a.normalise && lane == 0) {      // in choice order
-    float sum = 0.f;
-    for (int k = 0; k < a.top; k++) sum += a.selw[(size_t)t * stride + k];
-    const float inv = a.scale / (sum + 1e-20f * a.scale);
-    for (int k = 0; k < a.top; k++) a.selw[(size_t)t * stride + k] *= inv;
-  }
   if (a.sgw && lane == 0) a.sgw[t] = 1.0f / (1.0f + expf(-z[a.E]));
 }
 

@@ -216,6 +216,17 @@ void launch_ff(tgx_ctx* c, tgx::StackGemmArgs up, int epi_up, tgx::StackGemmArgs
   launch_gemm(c, down, epi_down, 1, np, groups, tile);
 }
 
+// a router's products on the rows h: true: the choice kernel takes them itself (steps of few tokens); false: they stand in zr
+bool route(tgx_ctx* c, tgx::RouterInput& in, const float* h, const float* wr, int n, int T) {
+  StackModel* sm = c->stack;
+  const int W = sm->d.width;
+  if (sm->gemv && T <= FEW_ROWS_MAX && n <= tgx::ROUTER_FUSED_MAX && W % 4 == 0) { in.h = h; in.ldh = W; in.w = wr; in.n = n; in.K = W; return true; }
+  tgx::StackGemmArgs g{};
+  g.A = h; g.lda = W; g.B = wr; g.ldb = W; g.C = sm->zr; g.ldc = n; g.M = T; g.N = n; g.K = W; g.scale = 1.f;
+  launch_gemm(c, g, tgx::SG_STORE, 1, 0, 0, 64, tgx::DT_F32);
+  return false;
+}
+
 template <int DT, bool SPLIT>
 void launch_attn_t(tgx_ctx* c, const tgx::StepMeta& m, const tgx::LatentAttnArgs& a, dim3 grid) {
   const size_t lds = (size_t)4 * a.rank * 4;
@@ -386,12 +397,10 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
       nc.nw = w.norm2; nc.cw = w.canon2; nc.state = nb > 0 ? w.conv_state + 2 * st_buf : nullptr;
       launch_norm_conv(c, m, nc, T);
       // router: fp32 weights, fp32 products (nothing is rounded), then bias, top-k and the softmax over the chosen
-      g = tgx::StackGemmArgs{};
-      g.A = sm->a; g.lda = W; g.B = w.w_router; g.ldb = W; g.C = sm->zr; g.ldc = ld.experts; g.M = T; g.N = ld.experts; g.K = W; g.scale = 1.f;
-      launch_gemm(c, g, tgx::SG_STORE, 1, 0, 0, 64, tgx::DT_F32);
       tgx::RouterArgs ra{};
       ra.z = sm->zr; ra.br = w.b_router; ra.sel = sm->sel; ra.selw = sm->selw; ra.E = ld.experts; ra.top = top;
-      hipLaunchKernelGGL(tgx::router_topk_kernel, dim3(T), dim3(64), 0, c->stream, ra);
+      if (route(c, ra.in, sm->a, w.w_router, ld.experts, T)) hipLaunchKernelGGL(tgx::router_topk_kernel<true>, dim3(T), dim3(256), 0, c->stream, ra);
+      else hipLaunchKernelGGL(tgx::router_topk_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
       const int np = T * top;
       tgx::MoePlanArgs pa{};
       pa.sel = sm->sel; pa.n_pairs = np; pa.E = ld.experts; pa.top = top; pa.tile_m = grouped_tile_rows(c, np, W, ld.ff, ld.experts, T, 2 * ld.ff);
@@ -627,12 +636,11 @@ void run_choice_experts(tgx_ctx* c, StackLayerW& w, const float* hin, int T) {
   const tgx_layer_desc& ld = w.d;
   const int W = sm->d.width, E = ld.experts + ld.identity, top = ld.top, nz = E + (ld.shared_ff > 0 ? 1 : 0);
   tgx::StackGemmArgs g{};
-  g.A = hin; g.lda = W; g.B = w.w_router; g.ldb = W; g.C = sm->zr; g.ldc = nz; g.M = T; g.N = nz; g.K = W; g.scale = 1.f;
-  launch_gemm(c, g, tgx::SG_STORE, 1, 0, 0, 64, tgx::DT_F32);
   tgx::RouterGroupArgs ra{};
   ra.z = sm->zr; ra.ldz = nz; ra.corr = w.b_router; ra.sel = sm->sel; ra.selw = sm->selw; ra.sgw = ld.shared_ff > 0 ? sm->sgw : nullptr;
   ra.E = E; ra.top = top; ra.groups = ld.groups; ra.keep = ld.groups_keep; ra.scale = ld.router_scale;
-  hipLaunchKernelGGL(tgx::router_group_kernel, dim3(T), dim3(64), 0, c->stream, ra);
+  if (route(c, ra.in, hin, w.w_router, nz, T)) hipLaunchKernelGGL(tgx::router_group_kernel<true>, dim3(T), dim3(256), 0, c->stream, ra);
+  else hipLaunchKernelGGL(tgx::router_group_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
   const int np = T * top;
   if (ld.experts > 0) {
     tgx::MoePlanArgs pa{};
@@ -1066,13 +1074,12 @@ void run_affine_ff(tgx_ctx* c, StackLayerW& w, int T) {
     return;
   }
   const int E = ld.experts, top = ld.top, np = T * top;
-  g.A = sm->a; g.lda = W; g.B = w.w_router; g.ldb = W; g.C = sm->zr; g.ldc = E; g.M = T; g.N = E; g.K = W; g.scale = 1.f;
-  launch_gemm(c, g, tgx::SG_STORE, 1, 0, 0, 64, tgx::DT_F32);
   tgx::RouterGroupArgs ra{};
   ra.z = sm->zr; ra.ldz = E; ra.corr = nullptr; ra.sel = sm->sel; ra.selw = sm->selw; ra.sgw = nullptr;
   ra.E = E; ra.top = top; ra.groups = ld.groups; ra.keep = ld.groups_keep; ra.scale = 1.f;
   ra.sigmoid_scores = ld.router_fn == 1; ra.group_top2 = ld.group_score == 1; ra.normalise = ld.router_norm;
-  hipLaunchKernelGGL(tgx::router_group_kernel, dim3(T), dim3(64), 0, c->stream, ra);
+  if (route(c, ra.in, sm->a, w.w_router, E, T)) hipLaunchKernelGGL(tgx::router_group_kernel<true>, dim3(T), dim3(256), 0, c->stream, ra);
+  else hipLaunchKernelGGL(tgx::router_group_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
   tgx::MoePlanArgs pa{};
   pa.sel = sm->sel; pa.n_pairs = np; pa.E = E; pa.top = top; pa.tile_m = grouped_tile_rows(c, np, W, ld.ff, E, T, 2 * ld.ff); pa.E_tiles = E;
   pa.off = sm->moe_off; pa.perm = sm->perm; pa.tok = sm->ptok; pa.tile_e = sm->tile_e; pa.tile_m0 = sm->tile_m0; pa.n_tiles = sm->n_tiles;
@@ -1743,11 +1750,10 @@ void run_hyper_ff(tgx_ctx* c, StackLayerW& w, int T) {
     return;
   }
   const int ride = shared_rides(c, w, T) ? 1 : 0, E = ld.experts + ride, top = ld.top + ride, np = T * top;
-  g.A = sm->a; g.lda = W; g.B = w.w_router; g.ldb = W; g.C = sm->zr; g.ldc = ld.experts; g.M = T; g.N = ld.experts; g.K = W; g.scale = 1.f;
-  launch_gemm(c, g, tgx::SG_STORE, 1, 0, 0, 64, tgx::DT_F32);
   tgx::RouterGroupArgs ra{};
   ra.z = sm->zr; ra.ldz = ld.experts; ra.sel = sm->sel; ra.selw = sm->selw; ra.E = ld.experts; ra.top = ld.top; ra.shared = ride; ra.groups = 1; ra.keep = 1; ra.scale = 1.f; ra.sigmoid_scores = ld.router_fn == 1; ra.normalise = ld.router_norm;
-  hipLaunchKernelGGL(tgx::router_group_kernel, dim3(T), dim3(64), 0, c->stream, ra);
+  if (route(c, ra.in, sm->a, w.w_router, ld.experts, T)) hipLaunchKernelGGL(tgx::router_group_kernel<true>, dim3(T), dim3(256), 0, c->stream, ra);
+  else hipLaunchKernelGGL(tgx::router_group_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
   tgx::MoePlanArgs pa{};
   pa.sel = sm->sel; pa.n_pairs = np; pa.E = E; pa.top = top; pa.tile_m = grouped_tile_rows(c, np, W, ld.ff, E, T, ld.ff); pa.E_tiles = E;
   pa.off = sm->moe_off; pa.perm = sm->perm; pa.tok = sm->ptok; pa.tile_e = sm->tile_e; pa.tile_m0 = sm->tile_m0; pa.n_tiles = sm->n_tiles;
