@@ -534,18 +534,39 @@ __global__ __launch_bounds__(256) void mlstm_scan_kernel(StepMeta m, MlstmArgs a
 // weight vector for all heads; w nullptr: none).  One wave per (token, head): the seam behind every recurrent mixer (mLSTM, wkv, gated delta rule, retention).
 struct HeadNormGateArgs { const float* hs; long long ldh; const float* w; int w_hstride; const float* gate; long long ldg; int silu_gate; float* out; long long ldo; int vdim; float eps;
                           const float* norm; long long ldnorm; const float* floor; long long ldfloor; float scale; };      // norm: hs enters as hs scale / (max(|norm scale|, floor) + 1e-6), both per token and head
+// Up to 256 channels a head the wave holds its row, and the gate and weight are on their way before the sum (a decoded
+// stream's launches 3.0 -> 2.6 us, those of 16 requests 4.2 -> 3.4).
 __global__ __launch_bounds__(64) void head_norm_gate_kernel(HeadNormGateArgs a) {
+  constexpr int NR = 4;
   const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
   const float* r = a.hs + (size_t)t * a.ldh + (size_t)h * a.vdim;
+  const float* gr = a.gate + (size_t)t * a.ldg + (size_t)h * a.vdim;
+  const float* w = a.w ? a.w + (size_t)h * a.w_hstride : nullptr;
+  float* o = a.out + (size_t)t * a.ldo + (size_t)h * a.vdim;
+  const bool held = a.vdim <= 64 * NR;
+  float v[NR], g[NR], wv[NR];
+  if (held)
+#pragma unroll
+    for (int k = 0; k < NR; k++) {
+      const int c = min(lane + 64 * k, a.vdim - 1);
+      v[k] = g[k] = 0.f; wv[k] = 1.f;
+      if (64 * k < a.vdim) { v[k] = r[c]; g[k] = gr[c]; if (w) wv[k] = w[c]; }      // (uniform)
+    }
   const float f = a.norm ? a.scale / (fmaxf(fabsf(a.norm[(size_t)t * a.ldnorm + h] * a.scale), a.floor[(size_t)t * a.ldfloor + h]) + 1e-6f) : 1.f;
+  auto gated = [&](float z) -> float { const float sg = 1.0f / (1.0f + expf(-z)); return a.silu_gate ? z * sg : sg; };
   float ss = 0.f;
-  for (int c = lane; c < a.vdim; c += 64) { const float v = r[c] * f; ss = fmaf(v, v, ss); }
+  if (held) {
+#pragma unroll
+    for (int k = 0; k < NR; k++) if (lane + 64 * k < a.vdim) { v[k] *= f; ss = fmaf(v[k], v[k], ss); }
+  } else
+    for (int c = lane; c < a.vdim; c += 64) { const float x = r[c] * f; ss = fmaf(x, x, ss); }
   ss = wave_sum(ss);
   const float rinv = 1.0f / sqrtf(ss / (float)a.vdim + a.eps);
-  for (int c = lane; c < a.vdim; c += 64) {
-    const float g = a.gate[(size_t)t * a.ldg + (size_t)h * a.vdim + c], sg = 1.0f / (1.0f + expf(-g));
-    a.out[(size_t)t * a.ldo + (size_t)h * a.vdim + c] = r[c] * f * rinv * (a.w ? a.w[(size_t)h * a.w_hstride + c] : 1.0f) * (a.silu_gate ? g * sg : sg);
-  }
+  if (held) {
+#pragma unroll
+    for (int k = 0; k < NR; k++) if (lane + 64 * k < a.vdim) o[lane + 64 * k] = v[k] * rinv * wv[k] * gated(g[k]);
+  } else
+    for (int c = lane; c < a.vdim; c += 64) o[c] = r[c] * f * rinv * (w ? w[c] : 1.0f) * gated(gr[c]);
 }
 
 // ---- grouped-choice router.  z [T][ldz]: the E router products of a token (fp32 product of fp32 weights), then the shared expert's gate product where
