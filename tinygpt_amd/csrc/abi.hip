@@ -911,6 +911,7 @@ int tgx_reset_cache(tgx_ctx* c) {
     c->batch = 0; c->past = 0;
     std::fill(c->row_idle.begin(), c->row_idle.end(), 0);
     c->have_logits = c->have_token = false;
+    c->poisoned = false;
     return TGX_OK;
   }
   for (auto& r : c->rows) HIP_OK(c, hipMemsetAsync(r.pos, 0, 4, c->stream));
@@ -1079,6 +1080,7 @@ int tgx_step_ragged(tgx_ctx* c, int n_entries, const int32_t* rows, const int32_
   if (!c) return TGX_ERR_INVALID;
   if (!c->stack) return set_err(c, TGX_ERR_UNSUPPORTED, "tgx_step_ragged serves layered models (tgx_create_stack); this family steps through tgx_forward_row / tgx_decode");
   if (!c->finalized) return set_err(c, TGX_ERR_STATE, "step before finalize");
+  if (c->poisoned) return set_err(c, TGX_ERR_STATE, "an earlier pass failed half-way: call tgx_reset_cache first");
   return stack_step(c, n_entries, rows, counts, ids, n_want, want, out_logits);
 }
 
@@ -1251,6 +1253,7 @@ int tgx_set_option(tgx_ctx* c, const char* key, int value) {
     if (!strcmp(key, "ssd.min")) { c->stack->ssd_min = value < 0 ? 0 : value; return TGX_OK; }      // tokens of a portion from which the scalar-decay recurrence runs in blocks on the matrix cores (0: never)
     if (!strcmp(key, "stack.gemv")) { c->stack->gemv = value != 0; return TGX_OK; }      // 0: products of few rows on the matrix-core tiles too
     if (!strcmp(key, "stack.line")) { c->stack->line = value != 0; return TGX_OK; }      // 0: prompts' products on the register-staged tiles
+    if (!strcmp(key, "debug.refuse_lds")) { c->stack->refuse_lds = value; return TGX_OK; }
     if (!strcmp(key, "stack.gemm_wt")) { if (value < 0 || value > 2) return set_err(c, TGX_ERR_INVALID, "stack.gemm_wt: 0, 1 or 2"); c->stack->gemm_wt = value; return TGX_OK; }
     return set_err(c, TGX_ERR_INVALID, "unknown option %s for a layered model", key);
   }

@@ -2503,6 +2503,7 @@ int upload_joint(tgx_ctx* c, const char* name, const void* host, const int64_t* 
 
 // ================================================================================================================================================
 bool stack_allow_lds(tgx_ctx* c, const void* kernel, size_t bytes) {
+  if (c->stack->refuse_lds > 0 && --c->stack->refuse_lds == 0) { c->launch_fault = "a product's LDS was refused (option debug.refuse_lds)"; return false; }
   if (bytes <= 64 * 1024 || c->stack->lds_kernels.count(kernel)) return true;
   if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) { (void)hipGetLastError(); c->launch_fault = "the device does not grant a product's LDS"; return false; }
   c->stack->lds_kernels.insert(kernel);
@@ -2963,6 +2964,15 @@ int stack_reset_row(tgx_ctx* c, int row) {
   return TGX_OK;
 }
 
+// the end of a step whose kernels were not all issued: those that were have moved caches and recurrent states, so nothing of it stays in flight and the context refuses every
+// pass until tgx_reset_cache
+static int half_way(tgx_ctx* c, int rc) {
+  (void)hipStreamSynchronize(c->stream);
+  c->poisoned = true;
+  LAUNCH_OK(c);
+  return rc;
+}
+
 int stack_step(tgx_ctx* c, int S, const int32_t* rows, const int32_t* counts, const int64_t* ids, int n_want, const int32_t* want, float* out_logits) {
   StackModel* sm = c->stack;
   const tgx_stack_desc& d = sm->d;
@@ -3010,15 +3020,15 @@ int stack_step(tgx_ctx* c, int S, const int32_t* rows, const int32_t* counts, co
   bool slots = false;      // the slots' current logits: what tgx_sample_row / tgx_read_logits see
   for (int e = 0; e < S; e++) if (last_want[(size_t)e] >= 0) { hp.want_row[last_want[(size_t)e]] = rows[e]; slots = true; }
   if ((rc = push_tables(c)) || (rc = push_meta(c, hp.n))) return rc;
-  if ((rc = run_layers(c, dp, (int)T, S, max_keys, max_count))) return rc;
+  if ((rc = run_layers(c, dp, (int)T, S, max_keys, max_count))) return half_way(c, rc);
   if (n_want > 0) {
     run_logits(c, dp.want, n_want, sm->lg, nullptr);
     if (slots) { launch_slot_logits(c, sm->lg, dp.want_row, n_want); c->have_logits = true; }
     HIP_OK(c, hipMemcpyAsync(out_logits, sm->lg, (size_t)n_want * d.vocab * 4, hipMemcpyDeviceToHost, c->stream));
   }
   HIP_OK(c, hipGetLastError());
+  if (c->launch_fault) return half_way(c, TGX_OK);
   HIP_OK(c, hipStreamSynchronize(c->stream));
-  LAUNCH_OK(c);
   for (int e = 0; e < S; e++) {
     const int r = rows[e];
     c->row_past[(size_t)r] += counts[e];
@@ -3072,12 +3082,13 @@ int stack_decode(tgx_ctx* c, const tgx_sampler_cfg& cfg, uint64_t seed, int n) {
   c->have_probs = !is_greedy(&cfg);
   for (int s = 0; s < n; s++) {
     hipLaunchKernelGGL(tgx::stack_gather_tok_kernel, dim3((S + 63) / 64), dim3(64), 0, c->stream, dp.tok_id, dp.ent_row, c->slab_tok, S);
-    if ((rc = run_layers(c, dp, S, S, max_keys + s + 1, 1))) return rc;
+    if ((rc = run_layers(c, dp, S, S, max_keys + s + 1, 1))) return half_way(c, rc);
     run_logits(c, dp.want, S, c->slab_logits, dp.want_row);
     launch_slot_logits(c, nullptr, dp.want_row, S);
     launch_sample(c, 0, c->batch, cfg, /*advance_pos=*/true, /*log_step=*/true);
     hipLaunchKernelGGL(tgx::stack_advance_kernel, dim3((S + 63) / 64), dim3(64), 0, c->stream, dp.tok_pos, dp.ent_par, dp.tok_par, S);
     c->steps_issued++;
+    if (c->launch_fault) return half_way(c, TGX_OK);
   }
   HIP_OK(c, hipGetLastError());
   for (int r : live) { c->row_past[(size_t)r] += n; if (n & 1) sm->row_par[(size_t)r] ^= 1; }
