@@ -1,9 +1,16 @@
-"""Layered models where something runs out: a step that cannot issue one of its kernels."""
+"""Layered models where something runs out: a step that cannot issue one of its kernels, no scratch for the forms that divide or block their work."""
 import numpy as np
 import pytest
 
 import stack_oracle as so
-from test_hip_stack_products import desc
+import test_hip_keronex as tk
+import test_hip_modepel as tm
+import test_hip_nusovik as tn
+import test_hip_stack as ts
+import test_hip_vitudra as tv
+import test_hip_zaluvik as tz
+import vitudra_oracle as vo
+from test_hip_stack_products import desc, wkv_model
 from tinygpt_amd.ffi import TgxError
 from tinygpt_amd.serving import SlotEngine
 
@@ -46,3 +53,86 @@ def test_a_step_that_cannot_issue_a_kernel_fails_and_a_reset_goes_on(how, nth):
     again = begin()
     eng.close()
     assert (again[0] == whole[0]).all() and (again[1] == whole[1]).all()
+
+
+# ---- scratch ------------------------------------------------------------------------------------------------------------------------------
+def layered(design, dtype):
+    """an engine whose prompt takes the blocked recurrence and whose decoding can divide its keys (16-bit storage: on the matrix cores)"""
+    if design == "zakusun":
+        return ts.engine(ts.small_desc(dtype, width=64, layers=[ts.plain_layer(heads=4, dim=8, vdim=8, kv_rank=128, scale=1.5), ts.moe_layer(heads=4, kv_rank=128, dim=4)]), 1)[0]
+    head = dict(heads=4, kv_heads=2, dim=64, vdim=64)
+    if design == "modepel":
+        return tm.engine(tm.config([tm.rec(heads=2, dim=32, vdim=36), tm.attn(tm.moe(), rot={"dims": 32, "base": 10000.0}, scale=0.15, **head)], width=64), dtype)[0]
+    if design == "vitudra":
+        return tv.engine(tv.config([tv.attn(mask=None, **head), tv.par()], width=64), dtype)[0]
+    if design == "zaluvik":
+        return tz.engine(tz.config([tz.attn(mask={"size": 400}, **head), tz.lat(heads=4, dim=16, rot_dim=16, vdim=16, kv_rank=112, mask={"size": 400})], width=64, loop=None), dtype)[0]
+    if design == "nusovik":
+        return tn.engine(tn.config([tn.mamba(), tn.par(left=dict(mask={"size": 300}, **head))], width=64), dtype)[0]
+    return tk.engine(tk.config([tk.ret(dim=8, vdim=12), tk.attn(**head)], width=64), dtype)[0]
+
+
+def prompt_and_tokens(eng, rid, n=600, steps=3):
+    ids = np.random.default_rng(9).integers(0, eng.desc.vocab, n + steps)
+    out = [eng.step([(rid, ids[:n], [0, 63, n - 1])])]
+    out += [eng.step([(rid, ids[n + t:n + t + 1], [0])]) for t in range(steps)]
+    eng.release(rid)
+    return np.concatenate(out)
+
+
+# Without scratch every layer takes the form that needs none: the same kernels as with the forms switched off, bit for bit.  Against the forms that use it: 1e-4 in fp32, where
+# only sums are ordered otherwise; in bf16 a cached row may round to the other neighbour (2^-8), and a near tie of a router sends a token elsewhere.
+@pytest.mark.parametrize("design", ["zakusun", "modepel", "vitudra", "zaluvik", "nusovik", "keronex"])
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+def test_no_memory_for_scratch(design, dtype):
+    eng = layered(design, dtype)
+    m = eng.model
+    m.set_option("attn.split_min", 64)
+    with_scratch = prompt_and_tokens(eng, "a")
+    m.set_option("stack.ws_max", 0)
+    without = prompt_and_tokens(eng, "b")
+    m.set_option("stack.ws_max", -1)
+    assert (prompt_and_tokens(eng, "c") == with_scratch).all()
+    m.set_option("ssd.min", 0)
+    m.set_option("attn.split_min", 1 << 30)
+    off = prompt_and_tokens(eng, "d")
+    eng.close()
+    if design != "zaluvik":      # (its sigmoid attention divides from 128 keys whatever the option says)
+        assert (without == off).all()
+    assert not (without == with_scratch).all()
+    err = np.abs(without - with_scratch).max(1) / np.abs(with_scratch).max()
+    assert np.sort(err)[-2 if dtype == "bf16" else -1] < (1e-4 if dtype == "fp32" else 2.0 ** -6), err
+
+
+@pytest.mark.parametrize("limit", [0, 4096])      # none; enough for the split of the width's products (2177 x 320 rows of two terms), not of the feed-forward's hidden values
+def test_no_memory_for_the_terms_of_a_prompt(limit):
+    W, ff, T = 320, 1088, 2177
+    d = wkv_model(W, ff, "bf16", T)
+    cfg = dict(width=W, vocab=101, layers=[dict(type="wkv", mixer=dict(heads=W // 64, dim=64), mlp=dict(ff=ff))] * 2)
+    eng = SlotEngine(desc=d, tensors={k: np.asarray(v, np.float32) for k, v in vo.random_tensors(cfg, 3, decay_rank=64).items()})
+    ids, want = np.random.default_rng(1).integers(0, d.vocab, T), [0, 127, T // 2, T - 1]
+    eng.model.set_option("stack.ws_max", limit)
+    got = eng.step([("a", ids, want)], ["a"])
+    eng.model.set_option("stack.ws_max", -1)
+    eng.model.set_option("stack.line", 0)
+    off = eng.step([("b", ids, want)], ["b"])
+    eng.close()
+    assert (got == off).all() if limit == 0 else np.abs(got - off).max() / np.abs(off).max() < 1e-4      # (the bound of test_prompt_products_of_a_model_that_caches_nothing)
+
+
+@pytest.mark.parametrize("limit", [0, 1024, 8192])
+def test_no_memory_for_the_terms_of_experts(limit):
+    from tinygpt_amd.desc import LayerDesc, StackDesc
+    T = 2100
+    layers = [LayerDesc(heads=4, dim=64, vdim=64, kv_rank=128, scale=0.125, mlp="moe", experts=5, top=2, ff=192, limit=7.0) for _ in range(2)]
+    d = StackDesc(width=256, vocab=101, canon_taps=3, norm_groups=2, norm_eps=1e-6, max_seqs=1, max_ctx=T, budget_tokens=T, compute_dtype="bf16", layers=layers)
+    eng = SlotEngine(desc=d, tensors={k: v.astype(np.float32) for k, v in so.random_tensors(d, T).items()})
+    ids, want = np.random.default_rng(T).integers(0, d.vocab, T), list(range(0, T, 50))
+    eng.model.set_option("stack.ws_max", limit)
+    got = eng.step([("a", ids, want)], ["a"])
+    eng.model.set_option("stack.ws_max", -1)
+    eng.model.set_option("stack.line", 0)
+    off = eng.step([("b", ids, want)], ["b"])
+    eng.close()
+    rows = np.abs(got - off).max(1) / np.abs(off).max()
+    assert (got == off).all() if limit == 0 else np.isfinite(got).all() and np.sort(rows)[-4] < 2.0 ** -7, rows      # (a near tie of the router may send a token to another expert)

@@ -144,6 +144,7 @@ struct StackModel {
   int ssd_min = 64;                    // option ssd.min: portions from this many tokens on take the blocked form of the scalar-decay recurrence (0: never)
   int mix_groups = 0;                  // option attn.mix_groups: key / value heads per workgroup of the matrix-core sigmoid attention: 1; 2 where their accumulators fit, whatever the grid; 0: 2 while the halved grid fills the chip
   std::set<const void*> lds_kernels;   // kernels that may take the whole LDS of a compute unit on this context's device
+  int ws_max = -1;                     // option stack.ws_max: most KiB of each of part, terms and terms2 (-1: as memory allows); products, attention and recurrences that would need more take their forms without scratch
   int refuse_lds = 0;                  // option debug.refuse_lds: the n-th product from now that asks for its LDS is refused it, as a device could (tests of a step that fails half-way)
   int line = 1;                        // option stack.line: 0 keeps prompts' products on the register-staged tiles
   int gemm_wt = 0;                     // option stack.gemm_wt: force the product's tile (1: 64 x 64, 2: 128 x 128); 0 = by the number of tiles

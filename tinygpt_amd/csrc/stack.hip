@@ -95,16 +95,21 @@ constexpr int GROUPED_FEW_PAIRS = 128, GROUPED_FEW_ROWS = 16, FEW_ROWS_MAX = 64;
 // three to 64 and the grouped tiles (47 rows, 1024 x 3072: 25 us against 38 on 64-wide tiles)
 constexpr int GEMV_ROWS_MAX = 2;
 constexpr int FEW_COLS_ANY_ROWS = 64;      // a matrix of so few rows (the router's) takes the few-row kernel whatever the step's size: the 64-wide matrix-core tiles would stand mostly empty
-// workspace of the line kernels; false: no memory for it (the register-staged tiles need none)
-bool ensure_terms(tgx_ctx* c, unsigned short*& p, size_t& have, size_t elems) {
+// scratch of the forms that divide, block or split their work, grown to the largest seen; false: there is no memory for it, or option stack.ws_max forbids it, and the caller
+// takes the form that needs none
+template <class E>
+bool ensure_scratch(tgx_ctx* c, E*& p, size_t& have, size_t elems) {
+  const long long most = c->stack->ws_max;
+  if (most >= 0 && elems * sizeof(E) > (size_t)most * 1024) return false;
   if (elems <= have) return true;
   if (hipStreamSynchronize(c->stream) != hipSuccess) return false;
   if (p) (void)hipFree(p);
   p = nullptr; have = 0;
-  if (hipMalloc((void**)&p, elems * 2) != hipSuccess) { (void)hipGetLastError(); p = nullptr; return false; }
+  if (hipMalloc((void**)&p, elems * sizeof(E)) != hipSuccess) { (void)hipGetLastError(); p = nullptr; return false; }
   have = elems;
   return true;
 }
+bool ensure_part(tgx_ctx* c, size_t elems) { return ensure_scratch(c, c->stack->part, c->stack->part_elems, elems); }
 // tiles of the two grouped products of an expert layer (both must be able to take them: their contraction lengths are the width and the expert width).  np: (token, expert)
 // pairs, E: experts, up_n: columns of the first product (gate and up together)
 int grouped_tile_rows(tgx_ctx* c, int np, int width, int ff, int E, int T, int up_n) {
@@ -112,7 +117,7 @@ int grouped_tile_rows(tgx_ctx* c, int np, int width, int ff, int E, int T, int u
   if (sm->gemv && np <= GROUPED_FEW_PAIRS && width % 8 == 0 && ff % 8 == 0) return GROUPED_FEW_ROWS;
   if (sm->line && c->dt != tgx::DT_F32 && width % 64 == 0 && ff % 64 == 0 && E > 0) {
     const int tile = stack_line_tile_grouped(c, np, E, up_n);
-    if (tile && ensure_terms(c, sm->terms, sm->terms_elems, (size_t)T * 2 * width) && ensure_terms(c, sm->terms2, sm->terms2_elems, (size_t)np * 2 * ff)) return tile;
+    if (tile && ensure_scratch(c, sm->terms, sm->terms_elems, (size_t)T * 2 * width) && ensure_scratch(c, sm->terms2, sm->terms2_elems, (size_t)np * 2 * ff)) return tile;
   }
   return 64;
 }
@@ -146,7 +151,7 @@ void launch_gemm(tgx_ctx* c, tgx::StackGemmArgs a, int epi, int nz, int grouped_
   const int tile = a.z_off ? (grouped_tile >= 128 ? grouped_tile : 0) : line_tile(c, a, epi, nz, dt);
   if (tile) {
     const int cols = a.K + a.a_zoff * (nz - 1), rows = a.a_rows ? a.a_count : a.M;
-    if (!a.At && ensure_terms(c, c->stack->terms, c->stack->terms_elems, (size_t)rows * 2 * cols)) {
+    if (!a.At && ensure_scratch(c, c->stack->terms, c->stack->terms_elems, (size_t)rows * 2 * cols)) {
       launch_split_terms(c, a.A, a.lda, rows, cols, c->stack->terms);
       a.At = c->stack->terms;
     }
@@ -211,7 +216,7 @@ tgx::StackGemmArgs sublayer_product(const tgx_ctx* c, const float* A, int K, con
 void launch_ff(tgx_ctx* c, tgx::StackGemmArgs up, int epi_up, tgx::StackGemmArgs down, int epi_down, int np = 0, int groups = 0, int tile = 64) {
   StackModel* sm = c->stack;
   const bool line = up.N == down.K && up.ldc == up.N && (up.z_off ? tile >= 128 : line_tile(c, up, epi_up, 1, c->dt) && line_tile(c, down, epi_down, 1, c->dt));
-  if (line && ensure_terms(c, sm->terms, sm->terms_elems, (size_t)(up.a_rows ? up.a_count : up.M) * 2 * up.K) && ensure_terms(c, sm->terms2, sm->terms2_elems, (size_t)up.M * 2 * up.N)) { up.Ct = sm->terms2; down.At = sm->terms2; }
+  if (line && ensure_scratch(c, sm->terms, sm->terms_elems, (size_t)(up.a_rows ? up.a_count : up.M) * 2 * up.K) && ensure_scratch(c, sm->terms2, sm->terms2_elems, (size_t)up.M * 2 * up.N)) { up.Ct = sm->terms2; down.At = sm->terms2; }
   launch_gemm(c, up, epi_up, 1, np, groups, tile);
   launch_gemm(c, down, epi_down, 1, np, groups, tile);
 }
@@ -294,18 +299,6 @@ int ensure_ws(tgx_ctx* c, int T) {
   return TGX_OK;
 }
 
-int ensure_part(tgx_ctx* c, size_t elems) {
-  StackModel* sm = c->stack;
-  if (elems <= sm->part_elems) return TGX_OK;
-  HIP_OK(c, hipStreamSynchronize(c->stream));
-  if (sm->part) (void)hipFree(sm->part);
-  sm->part = nullptr; sm->part_elems = 0;
-  int rc = dev_alloc(c, &sm->part, elems);
-  if (rc) return rc;
-  sm->part_elems = elems;
-  return TGX_OK;
-}
-
 void launch_norm_conv(tgx_ctx* c, const tgx::StepMeta& m, const tgx::NormConvArgs& a, int T) {
   if (a.taps == 4) hipLaunchKernelGGL(tgx::norm_conv_kernel<4>, dim3(T), dim3(256), 0, c->stream, m, a);
   else if (a.taps == 1) hipLaunchKernelGGL(tgx::norm_conv_kernel<1>, dim3(T), dim3(256), 0, c->stream, m, a);
@@ -354,9 +347,7 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
         nsplit = (max_keys + per - 1) / per;
         ma.keys_per = per;
       }
-      if (nsplit > 1) {
-        int rc = ensure_part(c, (size_t)T * H * nsplit * (size_t)(R + 2));
-        if (rc) return rc;
+      if (nsplit > 1 && ensure_part(c, (size_t)T * H * nsplit * (size_t)(R + 2))) {
         ma.part = sm->part; ma.nsplit = nsplit;
         aa.part = sm->part; aa.nsplit = nsplit;
         if (c->dt == tgx::DT_F16) launch_attn_mfma_t<tgx::DT_F16, true>(c, m, ma, dim3(tiles, S, nsplit)); else launch_attn_mfma_t<tgx::DT_BF16, true>(c, m, ma, dim3(tiles, S, nsplit));
@@ -372,9 +363,7 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
       nsplit = (max_keys + per - 1) / per;
       aa.keys_per = per;
     }
-    if (nsplit > 1) {
-      int rc = ensure_part(c, (size_t)T * H * nsplit * (size_t)(R + 2));
-      if (rc) return rc;
+    if (nsplit > 1 && ensure_part(c, (size_t)T * H * nsplit * (size_t)(R + 2))) {
       aa.part = sm->part; aa.nsplit = nsplit;
       TGX_DT_SWITCH(c->dt, (launch_attn_t<DT, true>(c, m, aa, dim3(T, H, nsplit))))
       hipLaunchKernelGGL(tgx::latent_attn_merge_kernel, dim3(T, H), dim3(256), 0, c->stream, aa);
@@ -502,9 +491,7 @@ int run_gqa_core(tgx_ctx* c, const tgx::StepMeta& m, const GqaSpec& sp_, int T, 
       nsplit = (span + per - 1) / per;
       ma.keys_per = per;
     }
-    if (nsplit > 1) {
-      int rc = ensure_part(c, (size_t)T * H * nsplit * (size_t)(sp.vdim + 2));
-      if (rc) return rc;
+    if (nsplit > 1 && ensure_part(c, (size_t)T * H * nsplit * (size_t)(sp.vdim + 2))) {
       ma.part = sm->part; ma.nsplit = nsplit;
       launch_gqa_mfma(c, m, ma, dim3(tiles, S * G, nsplit), true);
       tgx::GqaAttnArgs mg{};
@@ -529,9 +516,7 @@ int run_gqa_core(tgx_ctx* c, const tgx::StepMeta& m, const GqaSpec& sp_, int T, 
     nsplit = (span + per - 1) / per;
     aa.keys_per = per;
   }
-  if (nsplit > 1) {
-    int rc = ensure_part(c, (size_t)T * H * nsplit * (size_t)(sp.vdim + 2));
-    if (rc) return rc;
+  if (nsplit > 1 && ensure_part(c, (size_t)T * H * nsplit * (size_t)(sp.vdim + 2))) {
     aa.part = sm->part; aa.nsplit = nsplit;
     TGX_DT_SWITCH(c->dt, (launch_gqa_t<DT, true>(c, m, aa, dim3(T, H, nsplit))))
     merge(aa);
@@ -575,10 +560,8 @@ int run_mlstm(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, const float* h
   tgx::HeadNormGateArgs oa{};
   // portions: the recurrence with its maximum taken out is a scalar-decay recurrence and runs in blocks of 64 tokens (kernels/stack_ssd_mfma.h): from 64 tokens,
   // as the other families (a layer of 8 heads of 128 x 256, one prompt: 32 tokens 82 us by the scan and 86 in blocks, 64 tokens 115 and 107, 256 240 and 173, 1024 596 and 295)
-  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && (2 * qd) % 4 == 0) {
-    const size_t gram = ssd_gram_elems(T, S, H);
-    int rc = ensure_part(c, gram + (size_t)T * 4 * H);
-    if (rc) return rc;
+  const size_t gram = ssd_gram_elems(T, S, H);
+  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && ensure_part(c, gram + (size_t)T * 4 * H)) {
     tgx::GateScanArgs ga{};
     ga.proj = sm->proj; ga.ldp = ldp; ga.i0 = 2 * qd + 2 * vd; ga.f0 = ga.i0 + H; ga.mx = w.mm; ga.mx_buf = (size_t)sm->d.max_seqs * H; ga.gates = sm->part + gram; ga.heads = H;
     launch_gate_scan(c, m, ga, S);
@@ -970,11 +953,9 @@ int run_affine_attention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, con
     const int per = std::max(32, ((span + nsplit - 1) / nsplit + 31) / 32 * 32);
     nsplit = (span + per - 1) / per;
     aa.keys_per = per;
-    aa.kt = std::min(aa.kt, per);
   }
-  if (nsplit > 1) {
-    int rc = ensure_part(c, (size_t)T * nsplit * (size_t)vd);
-    if (rc) return rc;
+  if (nsplit > 1 && ensure_part(c, (size_t)T * nsplit * (size_t)vd)) {
+    aa.kt = std::min(aa.kt, aa.keys_per);
     aa.part = sm->part; aa.nsplit = nsplit;
     TGX_DT_SWITCH(c->dt, (launch_mix_attn_t<DT, true>(c, m, aa, dim3(T, nsplit), lds, vec)))
     hipLaunchKernelGGL(tgx::sigmoid_mix_merge_kernel, dim3(T, std::min(8, (vd + 255) / 256)), dim3(256), 0, c->stream, aa);
@@ -1024,9 +1005,7 @@ int run_affine_latent(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, const 
       nsplit = (span + per - 1) / per;
       ma.keys_per = per;
     }
-    if (nsplit > 1) {
-      int rc = ensure_part(c, (size_t)T * H * nsplit * (size_t)(RR + 2));
-      if (rc) return rc;
+    if (nsplit > 1 && ensure_part(c, (size_t)T * H * nsplit * (size_t)(RR + 2))) {
       ma.part = sm->part; ma.nsplit = nsplit;
       aa.part = sm->part; aa.nsplit = nsplit;
       if (c->dt == tgx::DT_F16) launch_attn_mfma_t<tgx::DT_F16, true>(c, m, ma, dim3(tiles, S, nsplit)); else launch_attn_mfma_t<tgx::DT_BF16, true>(c, m, ma, dim3(tiles, S, nsplit));
@@ -1041,9 +1020,7 @@ int run_affine_latent(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, const 
     nsplit = (span + per - 1) / per;
     aa.keys_per = per;
   }
-  if (nsplit > 1) {
-    int rc = ensure_part(c, (size_t)T * H * nsplit * (size_t)(RR + 2));
-    if (rc) return rc;
+  if (nsplit > 1 && ensure_part(c, (size_t)T * H * nsplit * (size_t)(RR + 2))) {
     aa.part = sm->part; aa.nsplit = nsplit;
     TGX_DT_SWITCH(c->dt, (launch_attn_t<DT, true>(c, m, aa, dim3(T, H, nsplit))))
     hipLaunchKernelGGL(tgx::latent_attn_merge_kernel, dim3(T, H), dim3(256), 0, c->stream, aa);
@@ -1425,8 +1402,7 @@ int run_ssm_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, 
   tgx::RecScanArgs ra{};
   ra.a = sm->rec_in + I + gn; ra.lda = ldr; ra.k = sm->rec_in + I; ra.ldk = ldr; ra.v = sm->rec_in; ra.ldv = ldr; ra.beta = sm->rec_in + C; ra.g = sm->rec_in + C + rH; ra.ldg = ldr;
   ra.skip = w.d_skip; ra.S = w.mS; ra.out = sm->hs; ra.ldo = I; ra.heads = rH; ra.kv_heads = ld.d_kv_heads; ra.dim = ld.d_dim; ra.vdim = ld.d_vdim;
-  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(rH, ld.d_kv_heads, ld.d_dim, ld.d_vdim, ldr)) {
-    if ((rc = ensure_part(c, ssd_gram_elems(T, S, ld.d_kv_heads)))) return rc;
+  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(rH, ld.d_kv_heads, ld.d_dim, ld.d_vdim, ldr) && ensure_part(c, ssd_gram_elems(T, S, ld.d_kv_heads))) {
     tgx::SsdArgs da{};
     da.row = sm->rec_in; da.ld = ldr; da.b0 = I; da.c0 = I + gn; da.gates = sm->rec_in; da.ldgate = ldr; da.dt_col = C; da.log_col = C + 2 * rH; da.heads = rH; da.groups = ld.d_kv_heads; da.N = ld.d_dim; da.E = ld.d_vdim; da.gram = sm->part; da.skip = w.d_skip; da.S = w.mS; da.out = sm->hs; da.ldo = I;
     launch_ssd_mfma(c, m, da, S, max_count);
@@ -1674,9 +1650,7 @@ int run_retention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int
     TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::gqa_append_kernel<DT>, dim3(T), dim3(256), 0, c->stream, m, ap))
   }
   const float kscale = 1.0f / sqrtf((float)ld.dim);      // the keys' factor, applied to k v^T
-  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp)) {
-    int rc = ensure_part(c, ssd_gram_elems(T, S, H));
-    if (rc) return rc;
+  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && ensure_part(c, ssd_gram_elems(T, S, H))) {
     tgx::SsdArgs da{};
     da.row = sm->proj; da.ld = ldp; da.b0 = vd; da.c0 = vd + qd; da.heads = H; da.groups = H; da.N = ld.dim; da.E = ld.vdim; da.gram = sm->part; da.fixed = w.decays; da.dt0 = kscale; da.S = w.mS; da.out = sm->hs; da.ldo = vd;
     launch_ssd_mfma(c, m, da, S, max_count);
