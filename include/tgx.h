@@ -492,7 +492,7 @@ TGX_API int tgx_set_logits(tgx_ctx* ctx, const float* logits, int batch);
  *                  key / value heads per workgroup of the matrix-core sigmoid attention (1; 2 = two where their accumulators fit; 0 = two while the halved grid fills the chip);
  *                  tokens of a portion from which a scalar-decay recurrence runs in blocks on the matrix cores (0 = never)
  *   "stack.ws_max" (layered models) most KiB of each scratch buffer that divided keys, blocked recurrences and prompts' products ask for (-1: as memory allows); what would need more,
- *                  or finds no memory, takes its form without scratch
+ *                  or finds no memory, takes its form without scratch; tgx_get_option "stack.ws_grown" = how often the context has allocated them
  *   "debug.refuse_lds"  (layered models, tests) the n-th product from now that asks for its LDS is refused it: its step fails half-way, TGX_ERR_UNSUPPORTED
  *   "debug.*"      experiment switches (tools/gemv_dissect.py, tools/attn_dissect.py; live only in a -DTGX_DISSECT=1 build) */
 TGX_API int tgx_set_option(tgx_ctx* ctx, const char* key, int value);

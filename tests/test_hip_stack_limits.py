@@ -104,9 +104,9 @@ def test_no_memory_for_scratch(design, dtype):
     assert np.sort(err)[-2 if dtype == "bf16" else -1] < (1e-4 if dtype == "fp32" else 2.0 ** -6), err
 
 
-@pytest.mark.parametrize("limit", [0, 4096])      # none; enough for the split of the width's products (2177 x 320 rows of two terms), not of the feed-forward's hidden values
+@pytest.mark.parametrize("limit", [0, 8192])      # none; enough for the split of the width's products (4161 x 320 rows of two terms), not of the feed-forward's hidden values
 def test_no_memory_for_the_terms_of_a_prompt(limit):
-    W, ff, T = 320, 1088, 2177
+    W, ff, T = 320, 1088, 4161
     d = wkv_model(W, ff, "bf16", T)
     cfg = dict(width=W, vocab=101, layers=[dict(type="wkv", mixer=dict(heads=W // 64, dim=64), mlp=dict(ff=ff))] * 2)
     eng = SlotEngine(desc=d, tensors={k: np.asarray(v, np.float32) for k, v in vo.random_tensors(cfg, 3, decay_rank=64).items()})
@@ -136,3 +136,34 @@ def test_no_memory_for_the_terms_of_experts(limit):
     eng.close()
     rows = np.abs(got - off).max(1) / np.abs(off).max()
     assert (got == off).all() if limit == 0 else np.isfinite(got).all() and np.sort(rows)[-4] < 2.0 ** -7, rows      # (a near tie of the router may send a token to another expert)
+
+
+@pytest.mark.parametrize("design", ["zakusun", "modepel", "vitudra", "zaluvik", "nusovik", "keronex"])
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+def test_decoding_allocates_nothing(design, dtype):
+    """a context's first step of single tokens takes what such steps can come to need: none of 640 further keys, nor more requests beside the first, stops for an allocation"""
+    eng = layered(design, dtype)
+    m = eng.model
+    m.set_option("attn.split_min", 64)
+    ids = np.random.default_rng(2).integers(0, eng.desc.vocab, 700)
+    eng.step([("a", ids[:59], [58])])
+    eng.step([("a", ids[59:60], [0])])
+    grown = m.get_option("stack.ws_grown")
+    assert grown == 1
+    for t in range(60, 700):
+        eng.step([("a", ids[t:t + 1], [0])] + [(r, ids[t:t + 1], []) for r, since in (("b", 300), ("c", 420), ("d", 421)) if t >= since])
+    assert m.get_option("stack.ws_grown") == grown
+    eng.close()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+def test_a_prompt_allocates_its_scratch_once(dtype):
+    W, ff, T = 320, 1088, 4161
+    d = wkv_model(W, ff, dtype, T)
+    cfg = dict(width=W, vocab=101, layers=[dict(type="wkv", mixer=dict(heads=W // 64, dim=64), mlp=dict(ff=ff))] * 2)
+    eng = SlotEngine(desc=d, tensors={k: np.asarray(v, np.float32) for k, v in vo.random_tensors(cfg, 3, decay_rank=64).items()})
+    ids = np.random.default_rng(1).integers(0, d.vocab, T)
+    for n, grown in ((T, 2), (T - 1, 2), (900, 2)):      # the products' terms and the hidden rows'
+        eng.step([("a", ids[:n], [n - 1])], ["a"])
+        assert eng.model.get_option("stack.ws_grown") == grown
+    eng.close()

@@ -1228,6 +1228,7 @@ int tgx_get_option(const tgx_ctx* c, const char* key, int* out_value) {
     if (!strcmp(key, "kv.free_tokens")) { *out_value = stack_free_tokens(c); return TGX_OK; }
     if (!strcmp(key, "kv.page_tokens")) { *out_value = c->stack->page; return TGX_OK; }
     if (!strcmp(key, "act.round16")) { *out_value = c->act16; return TGX_OK; }
+    if (!strcmp(key, "stack.ws_grown")) { *out_value = c->stack->ws_grown; return TGX_OK; }
     if (!strcmp(key, "attn.split_min")) { *out_value = c->stack->attn_split_min_keys; return TGX_OK; }
     return TGX_ERR_INVALID;
   }

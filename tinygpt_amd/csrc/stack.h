@@ -144,6 +144,9 @@ struct StackModel {
   int ssd_min = 64;                    // option ssd.min: portions from this many tokens on take the blocked form of the scalar-decay recurrence (0: never)
   int mix_groups = 0;                  // option attn.mix_groups: key / value heads per workgroup of the matrix-core sigmoid attention: 1; 2 where their accumulators fit, whatever the grid; 0: 2 while the halved grid fills the chip
   std::set<const void*> lds_kernels;   // kernels that may take the whole LDS of a compute unit on this context's device
+  size_t part_ask = 0, terms_cols = 0, terms2_cols = 0;      // what part can come to hold for divided keys; elements of one term that a token's row of terms and terms2 can come to hold (scratch_sizes)
+  size_t ws_refused = SIZE_MAX;        // bytes that this step has asked for in vain
+  int ws_grown = 0;                    // tgx_get_option stack.ws_grown: how often part, terms and terms2 were allocated
   int ws_max = -1;                     // option stack.ws_max: most KiB of each of part, terms and terms2 (-1: as memory allows); products, attention and recurrences that would need more take their forms without scratch
   int refuse_lds = 0;                  // option debug.refuse_lds: the n-th product from now that asks for its LDS is refused it, as a device could (tests of a step that fails half-way)
   int line = 1;                        // option stack.line: 0 keeps prompts' products on the register-staged tiles

@@ -95,21 +95,50 @@ constexpr int GROUPED_FEW_PAIRS = 128, GROUPED_FEW_ROWS = 16, FEW_ROWS_MAX = 64;
 // three to 64 and the grouped tiles (47 rows, 1024 x 3072: 25 us against 38 on 64-wide tiles)
 constexpr int GEMV_ROWS_MAX = 2;
 constexpr int FEW_COLS_ANY_ROWS = 64;      // a matrix of so few rows (the router's) takes the few-row kernel whatever the step's size: the 64-wide matrix-core tiles would stand mostly empty
-// scratch of the forms that divide, block or split their work, grown to the largest seen; false: there is no memory for it, or option stack.ws_max forbids it, and the caller
-// takes the form that needs none
+// Scratch of the forms that divide, block or split their work: at least `need` elements.  false: there is no memory for them, or option stack.ws_max forbids it, and the caller
+// takes the form that needs none; what stood before stays.  A buffer grows to `ask`, what this context's steps of as many tokens can come to need, so that a decode does not
+// stop for an allocation at every 64th key nor a first prompt at every wider product; to `need` where memory does not allow that.
 template <class E>
-bool ensure_scratch(tgx_ctx* c, E*& p, size_t& have, size_t elems) {
-  const long long most = c->stack->ws_max;
-  if (most >= 0 && elems * sizeof(E) > (size_t)most * 1024) return false;
-  if (elems <= have) return true;
+bool ensure_scratch(tgx_ctx* c, E*& p, size_t& have, size_t need, size_t ask) {
+  StackModel* sm = c->stack;
+  const size_t most = sm->ws_max >= 0 ? (size_t)sm->ws_max * 1024 / sizeof(E) : SIZE_MAX;
+  if (need > most) return false;
+  if (need <= have) return true;
+  if (need * sizeof(E) >= sm->ws_refused) return false;      // (in this step)
   if (hipStreamSynchronize(c->stream) != hipSuccess) return false;
+  ask = std::min(std::max(ask, need), most);
+  E* q = nullptr;
+  auto take = [&](size_t n) { if (hipMalloc((void**)&q, n * sizeof(E)) == hipSuccess) return true; (void)hipGetLastError(); q = nullptr; return false; };
+  size_t got = ask;
+  bool ok = take(got);
+  if (!ok) ok = take(got = need);
+  if (p && !ok) { (void)hipFree(p); p = nullptr; ok = take(got); }      // (the two do not fit side by side)
+  if (!ok) {
+    sm->ws_refused = need * sizeof(E);
+    if (!p && have > 0) { if (take(have)) p = q; else have = 0; }
+    return false;
+  }
   if (p) (void)hipFree(p);
-  p = nullptr; have = 0;
-  if (hipMalloc((void**)&p, elems * sizeof(E)) != hipSuccess) { (void)hipGetLastError(); p = nullptr; return false; }
-  have = elems;
+  p = q; have = got; sm->ws_grown++;
   return true;
 }
-bool ensure_part(tgx_ctx* c, size_t elems) { return ensure_scratch(c, c->stack->part, c->stack->part_elems, elems); }
+bool ensure_part(tgx_ctx* c, size_t need, size_t ask = 0) { StackModel* sm = c->stack; return ensure_scratch(c, sm->part, sm->part_elems, need, std::max(ask, sm->part_ask)); }
+bool ensure_terms(tgx_ctx* c, size_t need) { StackModel* sm = c->stack; return ensure_scratch(c, sm->terms, sm->terms_elems, need, 2 * (size_t)sm->cap_tokens * sm->terms_cols); }
+bool ensure_terms2(tgx_ctx* c, size_t need) { StackModel* sm = c->stack; return ensure_scratch(c, sm->terms2, sm->terms2_elems, need, 2 * (size_t)sm->cap_tokens * sm->terms2_cols); }
+// what those buffers can come to hold: the sums of the divided keys of any step (tiles of up to 32 rows on twice as many workgroups as there are compute units, a value or
+// latent row and two numbers each; or a token's outputs, heads in a row), and a token's widest product input and hidden row
+void scratch_sizes(tgx_ctx* c) {
+  StackModel* sm = c->stack;
+  int cols = std::max({sm->d.width * (sm->affine ? 2 : 1), sm->max_hv, sm->max_hr});
+  for (const StackLayerW& w : sm->L) {
+    const tgx_layer_desc& l = w.d;
+    const size_t row = (size_t)std::max(l.kv_rank + l.rot_dim, l.vdim) + 2;
+    if (sm->affine || w.pool) sm->part_ask = std::max(sm->part_ask, 2 * (size_t)c->num_cus * std::max(32 * row, (size_t)l.heads * l.vdim));
+    cols = std::max(cols, l.mixer == TGX_MIXER_WKV ? 4 * sm->d.width : 0);      // (one split of four of the token shift's five mixes)
+    sm->terms2_cols = std::max(sm->terms2_cols, (size_t)(l.mlp == TGX_MLP_MOE ? std::max(l.top * l.ff, l.shared_ff) : l.ff));
+  }
+  sm->terms_cols = (size_t)cols;
+}
 // tiles of the two grouped products of an expert layer (both must be able to take them: their contraction lengths are the width and the expert width).  np: (token, expert)
 // pairs, E: experts, up_n: columns of the first product (gate and up together)
 int grouped_tile_rows(tgx_ctx* c, int np, int width, int ff, int E, int T, int up_n) {
@@ -117,7 +146,7 @@ int grouped_tile_rows(tgx_ctx* c, int np, int width, int ff, int E, int T, int u
   if (sm->gemv && np <= GROUPED_FEW_PAIRS && width % 8 == 0 && ff % 8 == 0) return GROUPED_FEW_ROWS;
   if (sm->line && c->dt != tgx::DT_F32 && width % 64 == 0 && ff % 64 == 0 && E > 0) {
     const int tile = stack_line_tile_grouped(c, np, E, up_n);
-    if (tile && ensure_scratch(c, sm->terms, sm->terms_elems, (size_t)T * 2 * width) && ensure_scratch(c, sm->terms2, sm->terms2_elems, (size_t)np * 2 * ff)) return tile;
+    if (tile && ensure_terms(c, (size_t)T * 2 * width) && ensure_terms2(c, (size_t)np * 2 * ff)) return tile;
   }
   return 64;
 }
@@ -151,7 +180,7 @@ void launch_gemm(tgx_ctx* c, tgx::StackGemmArgs a, int epi, int nz, int grouped_
   const int tile = a.z_off ? (grouped_tile >= 128 ? grouped_tile : 0) : line_tile(c, a, epi, nz, dt);
   if (tile) {
     const int cols = a.K + a.a_zoff * (nz - 1), rows = a.a_rows ? a.a_count : a.M;
-    if (!a.At && ensure_scratch(c, c->stack->terms, c->stack->terms_elems, (size_t)rows * 2 * cols)) {
+    if (!a.At && ensure_terms(c, (size_t)rows * 2 * cols)) {
       launch_split_terms(c, a.A, a.lda, rows, cols, c->stack->terms);
       a.At = c->stack->terms;
     }
@@ -216,7 +245,7 @@ tgx::StackGemmArgs sublayer_product(const tgx_ctx* c, const float* A, int K, con
 void launch_ff(tgx_ctx* c, tgx::StackGemmArgs up, int epi_up, tgx::StackGemmArgs down, int epi_down, int np = 0, int groups = 0, int tile = 64) {
   StackModel* sm = c->stack;
   const bool line = up.N == down.K && up.ldc == up.N && (up.z_off ? tile >= 128 : line_tile(c, up, epi_up, 1, c->dt) && line_tile(c, down, epi_down, 1, c->dt));
-  if (line && ensure_scratch(c, sm->terms, sm->terms_elems, (size_t)(up.a_rows ? up.a_count : up.M) * 2 * up.K) && ensure_scratch(c, sm->terms2, sm->terms2_elems, (size_t)up.M * 2 * up.N)) { up.Ct = sm->terms2; down.At = sm->terms2; }
+  if (line && ensure_terms(c, (size_t)(up.a_rows ? up.a_count : up.M) * 2 * up.K) && ensure_terms2(c, (size_t)up.M * 2 * up.N)) { up.Ct = sm->terms2; down.At = sm->terms2; }
   launch_gemm(c, up, epi_up, 1, np, groups, tile);
   launch_gemm(c, down, epi_down, 1, np, groups, tile);
 }
@@ -296,6 +325,7 @@ int ensure_ws(tgx_ctx* c, int T) {
   if ((rc = dev_alloc(c, &sm->meta_dev, sm->meta_cap))) return rc;
   HIP_OK(c, hipHostMalloc((void**)&sm->meta_host, sm->meta_cap * 4, hipHostMallocDefault));
   sm->cap_tokens = cap;
+  if (sm->terms_cols == 0) scratch_sizes(c);
   return TGX_OK;
 }
 
@@ -303,6 +333,12 @@ void launch_norm_conv(tgx_ctx* c, const tgx::StepMeta& m, const tgx::NormConvArg
   if (a.taps == 4) hipLaunchKernelGGL(tgx::norm_conv_kernel<4>, dim3(T), dim3(256), 0, c->stream, m, a);
   else if (a.taps == 1) hipLaunchKernelGGL(tgx::norm_conv_kernel<1>, dim3(T), dim3(256), 0, c->stream, m, a);
   else hipLaunchKernelGGL(tgx::norm_conv_kernel<0>, dim3(T), dim3(256), 0, c->stream, m, a);
+}
+
+// a step of single tokens: the contexts that its kind will come to divide
+void reserve_part(tgx_ctx* c) {
+  StackModel* sm = c->stack;
+  if (sm->part_ask > 0 && sm->d.max_ctx >= 128) (void)ensure_part(c, sm->part_ask);
 }
 
 // the layers of one step; meta is on the device.  max_keys: the longest context any token of the step attends (host knowledge; picks the attention form)
@@ -561,7 +597,7 @@ int run_mlstm(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, const float* h
   // portions: the recurrence with its maximum taken out is a scalar-decay recurrence and runs in blocks of 64 tokens (kernels/stack_ssd_mfma.h): from 64 tokens,
   // as the other families (a layer of 8 heads of 128 x 256, one prompt: 32 tokens 82 us by the scan and 86 in blocks, 64 tokens 115 and 107, 256 240 and 173, 1024 596 and 295)
   const size_t gram = ssd_gram_elems(T, S, H);
-  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && ensure_part(c, gram + (size_t)T * 4 * H)) {
+  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && ensure_part(c, gram + (size_t)T * 4 * H, ssd_gram_elems(sm->cap_tokens, sm->d.max_seqs, H) + (size_t)sm->cap_tokens * 4 * H)) {
     tgx::GateScanArgs ga{};
     ga.proj = sm->proj; ga.ldp = ldp; ga.i0 = 2 * qd + 2 * vd; ga.f0 = ga.i0 + H; ga.mx = w.mm; ga.mx_buf = (size_t)sm->d.max_seqs * H; ga.gates = sm->part + gram; ga.heads = H;
     launch_gate_scan(c, m, ga, S);
@@ -1402,7 +1438,7 @@ int run_ssm_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, 
   tgx::RecScanArgs ra{};
   ra.a = sm->rec_in + I + gn; ra.lda = ldr; ra.k = sm->rec_in + I; ra.ldk = ldr; ra.v = sm->rec_in; ra.ldv = ldr; ra.beta = sm->rec_in + C; ra.g = sm->rec_in + C + rH; ra.ldg = ldr;
   ra.skip = w.d_skip; ra.S = w.mS; ra.out = sm->hs; ra.ldo = I; ra.heads = rH; ra.kv_heads = ld.d_kv_heads; ra.dim = ld.d_dim; ra.vdim = ld.d_vdim;
-  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(rH, ld.d_kv_heads, ld.d_dim, ld.d_vdim, ldr) && ensure_part(c, ssd_gram_elems(T, S, ld.d_kv_heads))) {
+  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(rH, ld.d_kv_heads, ld.d_dim, ld.d_vdim, ldr) && ensure_part(c, ssd_gram_elems(T, S, ld.d_kv_heads), ssd_gram_elems(sm->cap_tokens, sm->d.max_seqs, ld.d_kv_heads))) {
     tgx::SsdArgs da{};
     da.row = sm->rec_in; da.ld = ldr; da.b0 = I; da.c0 = I + gn; da.gates = sm->rec_in; da.ldgate = ldr; da.dt_col = C; da.log_col = C + 2 * rH; da.heads = rH; da.groups = ld.d_kv_heads; da.N = ld.d_dim; da.E = ld.d_vdim; da.gram = sm->part; da.skip = w.d_skip; da.S = w.mS; da.out = sm->hs; da.ldo = I;
     launch_ssd_mfma(c, m, da, S, max_count);
@@ -1650,7 +1686,7 @@ int run_retention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int
     TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::gqa_append_kernel<DT>, dim3(T), dim3(256), 0, c->stream, m, ap))
   }
   const float kscale = 1.0f / sqrtf((float)ld.dim);      // the keys' factor, applied to k v^T
-  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && ensure_part(c, ssd_gram_elems(T, S, H))) {
+  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && ensure_part(c, ssd_gram_elems(T, S, H), ssd_gram_elems(sm->cap_tokens, sm->d.max_seqs, H))) {
     tgx::SsdArgs da{};
     da.row = sm->proj; da.ld = ldp; da.b0 = vd; da.c0 = vd + qd; da.heads = H; da.groups = H; da.N = ld.dim; da.E = ld.vdim; da.gram = sm->part; da.fixed = w.decays; da.dt0 = kscale; da.S = w.mS; da.out = sm->hs; da.ldo = vd;
     launch_ssd_mfma(c, m, da, S, max_count);
@@ -2973,7 +3009,9 @@ int stack_step(tgx_ctx* c, int S, const int32_t* rows, const int32_t* counts, co
     return set_err(c, TGX_ERR_CONTEXT, "latent pool exhausted: the step needs %lld more pages of %d tokens, %zu free of %d", need_pages, sm->page, sm->free_pages.size(), sm->n_pages);
   HIP_OK(c, hipSetDevice(c->device));
   int rc;
+  sm->ws_refused = SIZE_MAX;
   if ((rc = ensure_ws(c, (int)std::max<long long>(T, n_want)))) return rc;
+  if (max_count == 1) reserve_part(c);
   if ((rc = meta_host_free(c))) return rc;
   const MetaPtrs hp = meta_layout(sm->meta_host, (int)T, S, n_want), dp = meta_layout(sm->meta_dev, (int)T, S, n_want);
   std::vector<int> last_want((size_t)S, -1);
@@ -3042,7 +3080,9 @@ int stack_decode(tgx_ctx* c, const tgx_sampler_cfg& cfg, uint64_t seed, int n) {
   }
   const int S = (int)live.size();
   int rc;
+  sm->ws_refused = SIZE_MAX;
   if ((rc = ensure_ws(c, S)) || (rc = meta_host_free(c))) return rc;
+  reserve_part(c);
   const MetaPtrs hp = meta_layout(sm->meta_host, S, S, S), dp = meta_layout(sm->meta_dev, S, S, S);
   for (int e = 0; e < S; e++) {
     const int r = live[(size_t)e];
