@@ -55,6 +55,29 @@ def test_a_step_that_cannot_issue_a_kernel_fails_and_a_reset_goes_on(how, nth):
     assert (again[0] == whole[0]).all() and (again[1] == whole[1]).all()
 
 
+# ---- options ----
+@pytest.mark.parametrize("dtype,latent,gqa", [("fp32", 2048, 1024), ("bf16", 128, 128)])
+def test_the_threshold_read_is_the_one_in_force(dtype, latent, gqa):
+    """a caller that reads the option and writes the value back leaves steps as they were: 200 keys are divided on the matrix cores and not on the lane kernels"""
+    eng = layered("zakusun", dtype)
+    m = eng.model
+    get = lambda: (m.get_option("attn.split_min"), m.get_option("attn.gqa_split_min"))      # noqa: E731
+    assert get() == (latent, gqa)
+    before = prompt_and_tokens(eng, "a", 200)
+    m.set_option("attn.split_min", m.get_option("attn.split_min"))
+    assert (prompt_and_tokens(eng, "b", 200) == before).all()
+    m.set_option("attn.split_min", 1 << 30)
+    assert get() == (1 << 30, 1 << 30) and (prompt_and_tokens(eng, "c", 200) == before).all() == (dtype == "fp32")
+    m.set_option("attn.split_min", -1)
+    m.set_option("attn.gqa_split_min", 77)
+    assert get() == (latent, 77)
+    m.set_option("attn.gqa_split_min", -1)
+    assert get() == (latent, gqa) and (prompt_and_tokens(eng, "d", 200) == before).all()
+    m.set_option("attn.mfma", 0)
+    assert get() == (2048, 1024)
+    eng.close()
+
+
 # ---- scratch ------------------------------------------------------------------------------------------------------------------------------
 def layered(design, dtype):
     """an engine whose prompt takes the blocked recurrence and whose decoding can divide its keys (16-bit storage: on the matrix cores)"""

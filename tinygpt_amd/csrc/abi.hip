@@ -1229,7 +1229,8 @@ int tgx_get_option(const tgx_ctx* c, const char* key, int* out_value) {
     if (!strcmp(key, "kv.page_tokens")) { *out_value = c->stack->page; return TGX_OK; }
     if (!strcmp(key, "act.round16")) { *out_value = c->act16; return TGX_OK; }
     if (!strcmp(key, "stack.ws_grown")) { *out_value = c->stack->ws_grown; return TGX_OK; }
-    if (!strcmp(key, "attn.split_min")) { *out_value = c->stack->attn_split_min_keys; return TGX_OK; }
+    if (!strcmp(key, "attn.split_min")) { *out_value = c->stack->on_matrix_cores() ? c->stack->latent_split_min_keys : c->stack->attn_split_min_keys; return TGX_OK; }
+    if (!strcmp(key, "attn.gqa_split_min")) { *out_value = c->stack->on_matrix_cores() ? c->stack->gqa_split_min_keys : c->stack->gqa_lane_split_min_keys; return TGX_OK; }
     return TGX_ERR_INVALID;
   }
   if (!strcmp(key, "attn.direct_limit")) { *out_value = (int)std::min<long long>(direct_limit(c, c->batch, true), INT_MAX); return TGX_OK; }
@@ -1246,8 +1247,8 @@ int tgx_set_option(tgx_ctx* c, const char* key, int value) {
   static const char* cls_names[TGX_KERNEL_COUNT] = {"qkv", "attn", "oproj", "gateup", "down", "lmhead"};
   if (c->stack) {      // layered models: "act.round16" as for the other families; "attn.split_min" = context from which steps of few tokens divide a sequence's keys
     if (!strcmp(key, "act.round16")) { c->act16 = value != 0; return TGX_OK; }      // between workgroups; "stack.gemm_wt" forces the product tile (1 / 2, 0 = automatic)
-    if (!strcmp(key, "attn.split_min")) { StackModel* s = c->stack; s->attn_split_min_keys = s->latent_split_min_keys = s->gqa_split_min_keys = s->gqa_lane_split_min_keys = value; return TGX_OK; }
-    if (!strcmp(key, "attn.gqa_split_min")) { c->stack->gqa_split_min_keys = c->stack->gqa_lane_split_min_keys = value; return TGX_OK; }
+    if (!strcmp(key, "attn.split_min")) { c->stack->set_split_min(value); return TGX_OK; }
+    if (!strcmp(key, "attn.gqa_split_min")) { c->stack->set_gqa_split_min(value); return TGX_OK; }
     if (!strcmp(key, "attn.mfma")) { c->stack->attn_mfma = value != 0; return TGX_OK; }      // 0: the lane-per-channel attention kernels for every layer
     if (!strcmp(key, "mlstm.narrow")) { c->stack->mlstm_narrow = value < 0 ? -1 : (value != 0); return TGX_OK; }      // the matrix-memory scan's column split (-1: automatic)
     if (!strcmp(key, "attn.mix_groups")) { c->stack->mix_groups = value == 1 || value == 2 ? value : 0; return TGX_OK; }      // key / value heads per workgroup of the matrix-core sigmoid attention: 1, 2 (where they fit, whatever the grid), 0 = by the grid

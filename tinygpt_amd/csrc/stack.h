@@ -133,11 +133,20 @@ struct StackModel {
   int *sel = nullptr, *moe_off = nullptr, *perm = nullptr, *ptok = nullptr, *tile_e = nullptr, *tile_m0 = nullptr, *n_tiles = nullptr;
   int max_in = 0, max_hr = 0, max_hv = 0, max_top = 0, max_ff = 0, max_E = 0, max_rank = 0;
   // Steps of few tokens split a sequence's keys between workgroups from these contexts on (option attn.split_min sets all four, attn.gqa_split_min the grouped-query ones, which
-  // count the keys that a workgroup would walk: a mask's span).  Matrix-core kernels: an undivided workgroup walks its keys tile by tile, 1.3 us for 32 latent rows, 0.9 us for 64
+  // count the keys that a workgroup would walk: a mask's span; a negative value brings these defaults back).  Matrix-core kernels: an undivided workgroup walks its keys tile by tile, 1.3 us for 32 latent rows, 0.9 us for 64
   // keys; a merge costs 4 to 5 us and a divided walk two tiles.  A decoded token's step at width 1024 and six layers, undivided -> divided: latent attention, four requests at 96 /
   // 160 / 256 / 1000 keys 627 -> 630, 646 -> 628, 675 -> 632, 872 -> 648 us; grouped-query, sixteen requests 691 -> 688, 702 -> 687, 704 -> 687, 786 -> 695
-  int latent_split_min_keys = 128, gqa_split_min_keys = 128;
-  int attn_split_min_keys = 2048, gqa_lane_split_min_keys = 1024;      // ... lane kernels
+  static constexpr int MFMA_SPLIT_MIN = 128, LATENT_LANE_SPLIT_MIN = 2048, GQA_LANE_SPLIT_MIN = 1024;
+  int latent_split_min_keys = MFMA_SPLIT_MIN, gqa_split_min_keys = MFMA_SPLIT_MIN;
+  int attn_split_min_keys = LATENT_LANE_SPLIT_MIN, gqa_lane_split_min_keys = GQA_LANE_SPLIT_MIN;      // ... lane kernels
+  void set_gqa_split_min(int keys) { gqa_split_min_keys = keys < 0 ? MFMA_SPLIT_MIN : keys; gqa_lane_split_min_keys = keys < 0 ? GQA_LANE_SPLIT_MIN : keys; }
+  void set_split_min(int keys) { set_gqa_split_min(keys); latent_split_min_keys = keys < 0 ? MFMA_SPLIT_MIN : keys; attn_split_min_keys = keys < 0 ? LATENT_LANE_SPLIT_MIN : keys; }
+  bool on_matrix_cores() const {      // whether any attention layer runs there
+    if (!attn_mfma) return false;
+    for (const auto& w : L) if (w.poolT || w.poolVT) return true;
+    for (const auto& r : runs) if (r.poolT) return true;
+    return false;
+  }
   int attn_mfma = 1;                   // option attn.mfma: 0 keeps every layer on the lane-per-channel attention kernels
   int gemv = 1;                        // option stack.gemv: 0 sends products of few rows through the matrix-core tiles as well
   int mlstm_narrow = -1;               // option mlstm.narrow: the matrix-memory scan's columns per wave (1: eight, 0: sixteen, -1: by the step's entries and heads)
