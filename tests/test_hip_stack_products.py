@@ -159,6 +159,25 @@ def test_matrix_memory_in_blocks(n, dim, vdim):
         assert np.abs(rows - want[i][pos]).max() / np.abs(want[i]).max() < 1e-4, (n, dim, vdim, i, pos)
 
 
+# The blocks' error against 64 bits is no larger than the scan's.  Geometric means over 16 models, fp32 storage: with one sum over a row's channels in the blocks' key products it
+# was 1.02 times (128 channels) and 1.06 times (256) the scan's, with eight sums 0.96 (standard errors 0.005 and 0.013).
+@pytest.mark.parametrize("heads,dim,vdim,n", [(2, 128, 64, 700), (1, 256, 256, 500)])
+def test_matrix_memory_in_blocks_is_as_exact_as_the_scan(heads, dim, vdim, n):
+    cfg = tm.config([tm.rec(heads=heads, dim=dim, vdim=vdim), tm.rec(heads=heads, dim=dim, vdim=vdim)], width=64)
+    ratios = []
+    for seed in range(16):
+        eng, w = tm.engine(cfg, seed=seed, max_ctx=4096, budget_tokens=4096)
+        ids = np.random.default_rng(seed).integers(0, cfg["vocab"], n).tolist()
+        want = mo.forward(cfg, w, ids)[0]
+        err = []
+        for least in (64, 0):
+            eng.model.set_option("ssd.min", least)
+            err.append(np.linalg.norm(eng.step([("p", ids, list(range(n)))], ["p"]) - want))
+        eng.close()
+        ratios.append(err[0] / err[1])
+    assert np.exp(np.log(ratios).mean()) <= 1.0, ratios
+
+
 # ---- seams and norms: rows of one, two and four vectors a thread, widths that are no multiple of four, and widths past the registers; taps by number and by name.
 # fp32 storage against the plain oracles of the designs: fp32 sums over at most 4100 channels, 1e-4 of the largest logit as in the designs' own tests.
 @pytest.mark.parametrize("width", [1024, 1028, 1030, 2044, 2052, 4096, 4100])

@@ -32,7 +32,9 @@ struct SsdArgs {
 __device__ __forceinline__ int ssd_first_block(int start, int e) { return start / SSD_BLOCK + e; }
 
 // G[i][j] = C_i . B_j, one 32 x 32 tile per wave (the tile above the diagonal is never read).  A lane holds one row of either operand: four consecutive channels per
-// load, channel 8 q + 4 (lane / 32) + u as the two contraction slots of step 4 q + u.  Grid: (blocks of the longest entry, groups, entries).
+// load, channel 8 q + 4 (lane / 32) + u as the two contraction slots of step 4 q + u.  Eight sums run side by side and meet in pairs, as the scan's eight row groups do: one sum
+// over all channels was most of a block's error (a matrix memory of 128 / 256 channels, against 64 bits: 1.9 / 2.2 times the scan's error with one sum, 1.0 with eight).
+// Grid: (blocks of the longest entry, groups, entries).
 template <int Q = SSD_BLOCK>
 __global__ __launch_bounds__(256) void ssd_gram_kernel(StepMeta m, SsdArgs a) {
   const int b = blockIdx.x, g = blockIdx.y, e = blockIdx.z, cnt = m.ent_count[e], start = m.ent_start[e];
@@ -43,19 +45,27 @@ __global__ __launch_bounds__(256) void ssd_gram_kernel(StepMeta m, SsdArgs a) {
   const int i = b * Q + 32 * it + l31, j = b * Q + 32 * jt + l31;
   const float* cr = a.row + (size_t)(start + min(i, cnt - 1)) * a.ld + a.c0 + (size_t)g * a.N;
   const float* br = a.row + (size_t)(start + min(j, cnt - 1)) * a.ld + a.b0 + (size_t)g * a.N;
-  f32x16 acc;
+  f32x16 acc[8];
 #pragma unroll
-  for (int r = 0; r < 16; r++) acc[r] = 0.f;
-  for (int q = 0; q < (a.N + 7) / 8; q++) {
-    const int n = 8 * q + 4 * half;
-    const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-    const f32x4 cv = n < a.N ? *reinterpret_cast<const f32x4*>(cr + n) : z, bv = n < a.N ? *reinterpret_cast<const f32x4*>(br + n) : z;
+  for (int k = 0; k < 8; k++)
 #pragma unroll
-    for (int u = 0; u < 4; u++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(cv[u], bv[u], acc, 0, 0, 0);
-  }
+    for (int r = 0; r < 16; r++) acc[k][r] = 0.f;
+  for (int q0 = 0; q0 < (a.N + 7) / 8; q0 += 2)
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const int n = 8 * (q0 + k) + 4 * half;
+      const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+      const f32x4 cv = n < a.N ? *reinterpret_cast<const f32x4*>(cr + n) : z, bv = n < a.N ? *reinterpret_cast<const f32x4*>(br + n) : z;
+#pragma unroll
+      for (int u = 0; u < 4; u++) acc[4 * k + u] = __builtin_amdgcn_mfma_f32_32x32x2f32(cv[u], bv[u], acc[4 * k + u], 0, 0, 0);
+    }
+#pragma unroll
+  for (int k = 4; k > 0; k /= 2)
+#pragma unroll
+    for (int j2 = 0; j2 < k; j2++) acc[j2] += acc[j2 + k];
   float* G = a.gram + ((size_t)(ssd_first_block(start, e) + b) * a.groups + g) * (Q * Q);
 #pragma unroll
-  for (int r = 0; r < 16; r++) G[(32 * it + (r & 3) + 8 * (r >> 2) + 4 * half) * Q + 32 * jt + l31] = acc[r];
+  for (int r = 0; r < 16; r++) G[(32 * it + (r & 3) + 8 * (r >> 2) + 4 * half) * Q + 32 * jt + l31] = acc[0][r];
 }
 
 // NW: 32-row tiles of the state per wave (4 NW 32 >= N).  Wave w owns the state rows n of its tiles and 32 columns, in the accumulator layout: register r of a lane is
@@ -248,7 +258,9 @@ __global__ __launch_bounds__(256, NW == 1 ? 2 : 1) void ssd_block_kernel(StepMet
 
 // The gates of a matrix memory in that form.  With the running maximum m_t = max(f_t + m_(t-1), i_t) of the log gates, the memory decays by exp(f_t + m_(t-1) - m_t), takes
 // k v^T by exp(i_t - m_t), and divides by at least exp(-m_t).  A token is the map m -> max(f + m, i), and such maps compose to maps of the same form, so a scan over lanes,
-// waves and portions of 1024 tokens gives every m_t from sums of the f alone (no difference of two long sums).  2048 tokens, 8 heads of 128 x 256: token by token 940 us a layer,
+// waves and portions of 1024 tokens gives every m_t from sums of the f alone (no difference of two long sums).  The maxima are kept in double: a thread takes the maximum
+// before its tokens from the composed maps and its neighbour's from its own steps, and in fp32 the two differed by a rounding, which is a factor on the whole memory.  The
+// maximum that the entry leaves is an fp32 number, so its last token's is rounded to that before its gates are made.  2048 tokens, 8 heads of 128 x 256: token by token 940 us a layer,
 // bound by each token's dependent step; 207 in blocks, a chain of 32 on 72 workgroups.  Grid: (entries, heads).
 struct GateScanArgs {
   const float* proj; long long ldp; int i0, f0;      // the columns of the log gates
@@ -257,12 +269,12 @@ struct GateScanArgs {
 };
 template <int TPT = 4>      // tokens of a thread
 __global__ __launch_bounds__(256) void gate_scan_kernel(StepMeta m, GateScanArgs a) {
-  __shared__ float s_f[2][4], s_m[2][4];
+  __shared__ double s_f[2][4], s_m[2][4];
   const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int start = m.ent_start[e], cnt = m.ent_count[e], row = m.ent_row[e], par = m.ent_par[e];
-  float carry = m.tok_pos[start] == 0 ? 0.f : a.mx[(size_t)par * a.mx_buf + (size_t)row * a.heads + h];
+  double carry = m.tok_pos[start] == 0 ? 0.f : a.mx[(size_t)par * a.mx_buf + (size_t)row * a.heads + h];
   for (int t0 = 0, p = 0; t0 < cnt; t0 += 256 * TPT, p ^= 1) {
-    float f[TPT], ig[TPT];
+    double f[TPT], ig[TPT];
 #pragma unroll
     for (int u = 0; u < TPT; u++) {      // (past the end m -> max(0 + m, -inf))
       const int t = t0 + TPT * tid + u;
@@ -270,33 +282,35 @@ __global__ __launch_bounds__(256) void gate_scan_kernel(StepMeta m, GateScanArgs
       const float fv = r[a.f0 + h], iv = r[a.i0 + h];
       f[u] = t < cnt ? fv : 0.f; ig[u] = t < cnt ? iv : -INFINITY;
     }
-    float F = f[0], M = ig[0];
+    double F = f[0], M = ig[0];
 #pragma unroll
-    for (int u = 1; u < TPT; u++) { M = fmaxf(M + f[u], ig[u]); F += f[u]; }
+    for (int u = 1; u < TPT; u++) { M = fmax(M + f[u], ig[u]); F += f[u]; }
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-      const float pf = __shfl_up(F, o, 64), pm = __shfl_up(M, o, 64);
-      if (lane >= o) { M = fmaxf(pm + F, M); F += pf; }
+      const double pf = __shfl_up(F, o, 64), pm = __shfl_up(M, o, 64);
+      if (lane >= o) { M = fmax(pm + F, M); F += pf; }
     }
     if (lane == 63) { s_f[p][wv] = F; s_m[p][wv] = M; }
-    const float bf = __shfl_up(F, 1, 64), bm = __shfl_up(M, 1, 64);      // the map of the lanes before
+    const double bf = __shfl_up(F, 1, 64), bm = __shfl_up(M, 1, 64);      // the map of the lanes before
     __syncthreads();      // (two buffers: the next portion's sums are written before all have read these)
-    float before = carry;
+    double before = carry;
 #pragma unroll
-    for (int w = 0; w < 4; w++) { if (w < wv) before = fmaxf(before + s_f[p][w], s_m[p][w]); carry = fmaxf(carry + s_f[p][w], s_m[p][w]); }
-    if (lane > 0) before = fmaxf(before + bf, bm);
+    for (int w = 0; w < 4; w++) { if (w < wv) before = fmax(before + s_f[p][w], s_m[p][w]); carry = fmax(carry + s_f[p][w], s_m[p][w]); }
+    if (lane > 0) before = fmax(before + bf, bm);
 #pragma unroll
     for (int u = 0; u < TPT; u++) {
       const int t = t0 + TPT * tid + u;
-      const float now = fmaxf(before + f[u], ig[u]);
+      double now = fmax(before + f[u], ig[u]);
+      if (t == cnt - 1) now = (float)now;
       if (t < cnt) {
         float* o = a.gates + (size_t)(start + t) * 3 * a.heads + h;
-        o[0] = expf(ig[u] - now); o[a.heads] = f[u] + before - now; o[2 * a.heads] = expf(-now);
+        const float mf = (float)now;
+        o[0] = expf((float)(ig[u] - now)); o[a.heads] = (float)(f[u] + before - now); o[2 * a.heads] = expf(-mf) * (1.0f + (float)(mf - now));      // exp(-now), now = mf + what its rounding left
       }
       before = now;
     }
   }
-  if (tid == 0) a.mx[(size_t)(par ^ 1) * a.mx_buf + (size_t)row * a.heads + h] = carry;
+  if (tid == 0) a.mx[(size_t)(par ^ 1) * a.mx_buf + (size_t)row * a.heads + h] = (float)carry;
 }
 
 }  // namespace tgx
