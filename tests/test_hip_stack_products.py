@@ -59,6 +59,26 @@ def test_rows_of_a_step_in_half_storage(slots, dtype, bound):
         assert np.abs(got[i] - want).max() / np.abs(want).max() < bound, (slots, dtype, i)
 
 
+# The few-row kernel's sums are as exact as the vector kernel's: sixteen rows together against one at a time, fp32 storage, a model that caches nothing, geometric means of the
+# errors' ratio over ten models.  1.41 (standard error 0.05) with one chain over a wave's share of K, 1.05 (0.12) with a chain a level; the bound lies between.
+def test_few_rows_are_as_exact_as_one():
+    import vitudra_oracle as vo
+    W, ff, rows, ratios = 1024, 512, 16, []
+    for seed in range(10):
+        cfg = dict(width=W, vocab=101, norm=dict(eps=1e-5), residual_mult=0.5, layers=[dict(type="wkv", mixer=dict(heads=W // 64, dim=64), mlp=dict(kind="dense", ff=ff))])
+        t = vo.random_tensors(cfg, seed, decay_rank=64)
+        d = StackDesc(family="vitudra", width=W, vocab=101, compute_dtype="fp32", max_seqs=rows, max_ctx=64, budget_tokens=64 * rows, norm_eps=1e-5, residual_mult=0.5,
+                      layers=[LayerDesc(mixer="wkv", heads=W // 64, kv_heads=W // 64, dim=64, vdim=64, decay_rank=64, mlp="dense", ff=ff)])
+        eng = SlotEngine(desc=d, tensors={k: np.asarray(v, np.float32) for k, v in t.items()})
+        ids = np.random.default_rng(seed).permutation(101)[:rows]
+        want = np.stack([vo.forward(cfg, t, [int(i)])[0] for i in ids])
+        many = eng.step([(i, [x], [0]) for i, x in enumerate(ids)], range(rows))
+        one = np.concatenate([eng.step([(0, [x], [0])], [0]) for x in ids])
+        eng.close()
+        ratios.append(np.linalg.norm(many - want) / np.linalg.norm(one - want))
+    assert np.exp(np.log(ratios).mean()) < 1.25, ratios
+
+
 # ---- prompts: the line kernels against the register-staged tiles ---------------------------------------------------------------------------
 # Both forms multiply the same two 16-bit terms of an activation by the same stored weights; only the order of fp32 sums differs (5e-7 measured per product, 1e-4 allowed
 # through two layers and a recurrence).  The wkv model caches nothing, so nothing rounds on the way; the expert model's cached latents may round to the other neighbour.

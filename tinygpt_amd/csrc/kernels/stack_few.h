@@ -5,9 +5,11 @@
 // activation row through L2 for every two columns — eight rows of 4 KB for 4 KB of weights — and streamed the weights again for every tile of four or eight rows.
 // Here a workgroup owns SIXTEEN columns and up to 64 rows, so an activation byte serves eight times as many weights and a weight byte is read once for all rows.  The
 // products are v_mfma_f32_16x16x4_f32 on the stored weights widened to 32 bits and the activations as they are: nothing is rounded or split, as in the vector form
-// (at sixteen rows the 32-bit rate costs less than the stream: 0.6 us for 3072 x 1024 on the whole chip).
+// (at sixteen rows the 32-bit rate costs less than the stream: 0.6 us for 3072 x 1024 on the whole chip).  Products are summed in runs of 32 (a half step), the runs of a step,
+// the steps of a wave and the waves in chains of their own (fp32 logits of two layers of 1024 / 8192 channels against 64 bits, four / sixteen rows: 1.25 / 1.17 times the vector
+// form's error with one chain over a wave's whole share of K, 0.95 / 0.97 so).
 //
-// The waves of a workgroup divide K in steps of 64 and have nothing to do with each other until their sums meet in LDS, in wave order (fixed: results do not depend on
+// The waves of a workgroup divide K in steps of 64 and have nothing to do with each other until their sums meet in LDS, in a fixed order (results do not depend on
 // timing).  A step arrives by LDS-DMA in the wave's own ring: straight loads in the matrix operand's layout put sixteen rows under sixteen neighbouring lanes, one
 // address lookup a lane — 26 us for 32000 x 1024 however many were in flight; a DMA piece covers whole lines (eight weight rows of 128 bytes, four activation rows of 256).
 // LDS image: 16-byte chunk c of row r in slot c ^ (r & 7), applied on the global side and in the fragment reads (as in gemm_dma.h).
@@ -85,17 +87,27 @@ __global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_kernel(const
         dma_1k(k < a.K ? (const void*)(xsrc[i][p] + k) : (const void*)&few_zeros, dst);
       }
   };
-  f32x4 acc[2][NB][MB];                                             // one set per half step: two chains of products in flight
+  // a step's sums, one set per half step (two chains of products in flight), are added to the wave's when the next step's operands have landed
+  f32x4 acc[NB][MB], part[2][NB][MB];
 #pragma unroll
-  for (int h = 0; h < 2; h++)
+  for (int b = 0; b < NB; b++)
+#pragma unroll
+    for (int i = 0; i < MB; i++) acc[b][i] = part[0][b][i] = part[1][b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto collect = [&] {
 #pragma unroll
     for (int b = 0; b < NB; b++)
 #pragma unroll
-      for (int i = 0; i < MB; i++) acc[h][b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < MB; i++) acc[b][i] += part[0][b][i] + part[1][b][i];
+  };
   auto product = [&](int slot, auto R16) {                          // R16: activations rounded to the storage type first (option act.round16)
     const unsigned char* st = ring + slot * STEP;
+    collect();
 #pragma unroll
     for (int h = 0; h < 2; h++) {
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int i = 0; i < MB; i++) part[h][b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
       const int sl = 4 * h + q;                                     // this lane's slice of the step
       float w[NB][8];
 #pragma unroll
@@ -116,7 +128,7 @@ __global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_kernel(const
         for (int e = 0; e < 8; e++) {
           const float v = e < 4 ? x0[e & 3] : x1[e & 3], x = R16.value ? round_storage_if<DT>(v, 1) : v;
 #pragma unroll
-          for (int b = 0; b < NB; b++) acc[h][b][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, w[b][e], acc[h][b][i], 0, 0, 0);
+          for (int b = 0; b < NB; b++) part[h][b][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, w[b][e], part[h][b][i], 0, 0, 0);
         }
       }
     }
@@ -137,6 +149,7 @@ __global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_kernel(const
     slot = slot + 1 == depth ? 0 : slot + 1;
   }
 
+  collect();
   __syncthreads();                                                  // every wave is done with its ring
   float* red = reinterpret_cast<float*>(few_lds);                   // [waves][NB * MB * 4][64]
 #pragma unroll
@@ -144,7 +157,7 @@ __global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_kernel(const
 #pragma unroll
     for (int i = 0; i < MB; i++)
 #pragma unroll
-      for (int r = 0; r < 4; r++) red[((wv * NB + b) * MB * 4 + i * 4 + r) * 64 + lane] = acc[0][b][i][r] + acc[1][b][i][r];
+      for (int r = 0; r < 4; r++) red[((wv * NB + b) * MB * 4 + i * 4 + r) * 64 + lane] = acc[b][i][r];
   __syncthreads();
   // C layout of the 16 x 16 product: column = lane & 15, row = 4 (lane >> 4) + r
   for (int o = threadIdx.x; o < MB * 256; o += blockDim.x) {
@@ -153,8 +166,12 @@ __global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_kernel(const
     float v[NB];
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-      v[b] = red[(b * MB * 4 + ir) * 64 + l];
-      for (int w = 1; w < nw; w++) v[b] += red[((w * NB + b) * MB * 4 + ir) * 64 + l];
+      float t[few_max_waves(MB)], s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < few_max_waves(MB); w++) t[w] = red[((min(w, nw - 1) * NB + b) * MB * 4 + ir) * 64 + l];      // (all on their way at once)
+#pragma unroll
+      for (int w = 0; w < few_max_waves(MB); w++) s[w & 3] += w < nw ? t[w] : 0.f;
+      v[b] = (s[0] + s[1]) + (s[2] + s[3]);
     }
     sg_finish<EPI>(a, z, m, n, v[0], v[NB - 1]);
   }
