@@ -87,16 +87,28 @@ def wkv_model(W, ff, dtype, T):
     return StackDesc(family="vitudra", width=W, vocab=101, compute_dtype=dtype, max_seqs=1, max_ctx=T, budget_tokens=T, norm_eps=1e-5, residual_mult=0.5, layers=layers)
 
 
-def on_and_off(d, tensors, ids, want, options=()):
-    eng = SlotEngine(desc=d, tensors={k: np.asarray(v, np.float32) for k, v in tensors.items()})
-    for o in options:
-        eng.model.set_option(*o)
-    out = []
-    for on in (1, 0):
-        eng.model.set_option("stack.line", on)
-        out.append(eng.step([("p", ids, want)], ["p"]))
+# What the second terms are worth: without them (act.round16) a row of logits moves by 1.5e-4 (wkv; experts 3e-5) in fp16 and ten times that in bf16 at least.  With them the two
+# forms differ by fp32 sums and by second terms that round to the other neighbour, 2^-17 of an activation in bf16 and 2^-23 in fp16: a median row by 2.5e-6 and 2.8e-7 at most
+# (measured), 2^-16 and 2^-20 allowed.  Single terms round the same inputs, which differ in their last bits, so their roundings part from layer to layer and only the distance that
+# they bring can be compared: that of one form's median row against the other's (0.92 to 1.07 measured), two thirds to three halves.
+MEDIAN = {"bf16": 2.0 ** -16, "fp16": 2.0 ** -20}
+
+
+def on_and_off(eng, ids, want, dtype):
+    """a prompt's logits by the line kernels and by the tiles, both terms of an activation; single terms are compared on the way"""
+    out = {}
+    for one in (0, 1):
+        eng.model.set_option("act.round16", one)
+        for line in (1, 0):
+            eng.model.set_option("stack.line", line)
+            out[line, one] = eng.step([("p", ids, want)], ["p"]).astype(np.float64)
     eng.close()
-    return out
+    assert all(np.isfinite(x).all() for x in out.values())
+    away = lambda x, y: np.median(np.abs(out[x] - out[y]).max(1) / np.abs(out[y]).max())      # noqa: E731
+    assert 0 < away((1, 0), (0, 0)) < MEDIAN[dtype], away((1, 0), (0, 0))
+    ratio = away((1, 1), (1, 0)) / away((0, 1), (0, 0))
+    assert 2 / 3 < ratio < 3 / 2, ratio
+    return out[1, 0], out[0, 0]
 
 
 # (T 2177: 18 row tiles of 128, the last of one row; 4161: 256-row tiles, the last of 65; ff 1088 = 17 x 64: column tiles that end inside; width 320: five steps of K)
@@ -109,22 +121,35 @@ def test_prompt_products_of_a_model_that_caches_nothing(W, ff, T, dtype):
     cfg = dict(width=W, vocab=101, layers=[dict(type="wkv", mixer=dict(heads=W // 64, dim=64), mlp=dict(ff=ff))] * 2)
     t = vo.random_tensors(cfg, 3, decay_rank=64)
     want = sorted({0, 1, 63, 64, 127, 128, 255, 256, T // 2, T - 66, T - 2, T - 1})
-    on, off = on_and_off(d, t, rng.integers(0, d.vocab, T), want)
-    assert np.isfinite(on).all() and np.abs(on - off).max() / np.abs(off).max() < 1e-4, (W, ff, T, dtype)
-    one, _ = on_and_off(d, t, rng.integers(0, d.vocab, T), want, [("act.round16", 1)])      # a single term: both forms round the same inputs, which differ in their last bits
-    assert np.isfinite(one).all()
+    eng = SlotEngine(desc=d, tensors={k: np.asarray(v, np.float32) for k, v in t.items()})
+    on, off = on_and_off(eng, rng.integers(0, d.vocab, T), want, dtype)
+    assert np.abs(on - off).max() / np.abs(off).max() < 1e-4, (W, ff, T, dtype)
 
 
+# a near tie of the router may send a token to another expert, and a cached latent may round to the other neighbour: one row in sixteen may go beyond the bound of such a step
 @pytest.mark.parametrize("dtype,bound", [("bf16", 2.0 ** -7), ("fp16", 2.0 ** -10)])
-@pytest.mark.parametrize("T,experts,top,ff", [(2100, 5, 2, 192), (4000, 3, 3, 1024), (1537, 9, 4, 320)])
-def test_prompt_products_of_experts(T, experts, top, ff, dtype, bound):
-    layers = [LayerDesc(heads=4, dim=64, vdim=64, kv_rank=128, scale=0.125, mlp="moe", experts=experts, top=top, ff=ff, limit=7.0) for _ in range(2)]
+@pytest.mark.parametrize("T,experts,top,ff,kv_rank", [(2100, 5, 2, 192, 128), (4000, 3, 3, 1024, 128), (1537, 9, 4, 320, 128), (2100, 5, 2, 192, 256), (4100, 3, 2, 512, 320)])
+def test_prompt_products_of_experts(T, experts, top, ff, kv_rank, dtype, bound):
+    """kv_rank from 256 on: the gated products of every head's latents take the line kernels too"""
+    layers = [LayerDesc(heads=4, dim=64, vdim=64, kv_rank=kv_rank, scale=0.125, mlp="moe", experts=experts, top=top, ff=ff, limit=7.0) for _ in range(2)]
     d = StackDesc(width=256, vocab=101, canon_taps=3, norm_groups=2, norm_eps=1e-6, max_seqs=1, max_ctx=T, budget_tokens=T, compute_dtype=dtype, layers=layers)
-    t = so.random_tensors(d, T)
-    on, off = on_and_off(d, t, np.random.default_rng(T).integers(0, d.vocab, T), [0, 127, 128, T // 2, T - 1])
-    # (a near tie of the router may send a token to another expert: the other rows hold)
+    eng = SlotEngine(desc=d, tensors={k: v.astype(np.float32) for k, v in so.random_tensors(d, T).items()})
+    on, off = on_and_off(eng, np.random.default_rng(T).integers(0, d.vocab, T), sorted({*range(0, T, 33), 127, 128, T // 2, T - 1}), dtype)
     rows = np.abs(on - off).max(1) / np.abs(off).max()
-    assert np.isfinite(on).all() and np.sort(rows)[-2] < bound, (T, dtype, rows)
+    assert np.quantile(rows, 15 / 16) < bound, (T, dtype, rows)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("T,experts,top,ff,shared", [(1100, 4, 2, 512, 512), (2100, 9, 3, 320, 64), (1500, 3, 1, 1024, 0)])
+def test_prompt_products_of_experts_weighted_at_their_input(T, experts, top, ff, shared, dtype):
+    """gathered products with a weight a row and an activation in the epilogue; retention caches nothing, so only a router's near tie goes beyond 1e-4"""
+    import test_hip_keronex as tk
+    layer = tk.ret(tk.moe(experts, top, ff, shared), heads=4, dim=32, vdim=64, decay=[0.875, 0.99, 0.5, 0.9])
+    cfg = tk.config([layer, layer], width=256)
+    eng, _ = tk.engine(cfg, dtype, max_seqs=1, max_ctx=T, budget_tokens=T + 64)
+    on, off = on_and_off(eng, np.array(tk.tokens(cfg, T)), sorted({*range(0, T, 17), 127, 128, T - 1}), dtype)
+    rows = np.abs(on - off).max(1) / np.abs(off).max()
+    assert np.quantile(rows, 15 / 16) < 1e-4, (T, dtype, rows)
 
 
 @pytest.mark.parametrize("vocab", [53, 96, 1028, 1030])
