@@ -11,6 +11,7 @@ import test_hip_vitudra as tv
 import test_hip_zaluvik as tz
 import vitudra_oracle as vo
 from test_hip_stack_products import desc, wkv_model
+from tinygpt_amd.desc import LayerDesc, StackDesc
 from tinygpt_amd.ffi import TgxError
 from tinygpt_amd.serving import SlotEngine
 
@@ -53,6 +54,23 @@ def test_a_step_that_cannot_issue_a_kernel_fails_and_a_reset_goes_on(how, nth):
     again = begin()
     eng.close()
     assert (again[0] == whole[0]).all() and (again[1] == whole[1]).all()
+
+
+def test_a_step_too_large_for_memory_leaves_the_context_usable():
+    """200000 rows of a million logits: the workspace's last buffers cannot be had, and neither those that stood nor the failed request are taken for granted afterwards"""
+    T = 200_000
+    d = StackDesc(width=8, vocab=1_000_000, canon_taps=2, norm_groups=2, norm_eps=1e-6, max_seqs=2, max_ctx=T, budget_tokens=T + 128, compute_dtype="bf16",
+                  layers=[LayerDesc(heads=1, dim=8, vdim=8, kv_rank=8, scale=0.35, mlp=None)])
+    eng = SlotEngine(desc=d, tensors={k: v.astype(np.float32) for k, v in so.random_tensors(d, 1).items()})
+    ids = np.random.default_rng(1).integers(0, d.vocab, T)
+    before = eng.step([("a", ids[:5], [1, 4])])
+    with pytest.raises(TgxError, match="memory"):
+        eng.step([("b", ids, [T - 1])])
+    eng.release("b")
+    assert (eng.step([("c", ids[:5], [1, 4])]) == before).all()
+    both = eng.step([("a", ids[5:6], [0]), ("c", ids[5:6], [0])])
+    assert np.isfinite(both).all() and (both[0] == both[1]).all()
+    eng.close()
 
 
 # ---- options ----
@@ -145,7 +163,6 @@ def test_no_memory_for_the_terms_of_a_prompt(limit):
 
 @pytest.mark.parametrize("limit", [0, 1024, 8192])
 def test_no_memory_for_the_terms_of_experts(limit):
-    from tinygpt_amd.desc import LayerDesc, StackDesc
     T = 2100
     layers = [LayerDesc(heads=4, dim=64, vdim=64, kv_rank=128, scale=0.125, mlp="moe", experts=5, top=2, ff=192, limit=7.0) for _ in range(2)]
     d = StackDesc(width=256, vocab=101, canon_taps=3, norm_groups=2, norm_eps=1e-6, max_seqs=1, max_ctx=T, budget_tokens=T, compute_dtype="bf16", layers=layers)

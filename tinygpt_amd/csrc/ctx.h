@@ -285,7 +285,12 @@ int set_err(tgx_ctx* c, int code, const char* fmt, ...);
 
 template <typename T>
 int dev_alloc(tgx_ctx* c, T** p, size_t n) {
-  HIP_OK(c, hipMalloc((void**)p, n * sizeof(T)));
+  const hipError_t e = hipMalloc((void**)p, n * sizeof(T));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();      // (a later pass asks for its own launches' errors)
+    *p = nullptr;
+    return set_err(c, TGX_ERR_DEVICE, "%zu bytes of device memory: %s", n * sizeof(T), hipGetErrorString(e));
+  }
   return TGX_OK;
 }
 

@@ -292,6 +292,7 @@ int ensure_ws(tgx_ctx* c, int T) {
   StackModel* sm = c->stack;
   if (T <= sm->cap_tokens) return TGX_OK;
   HIP_OK(c, hipStreamSynchronize(c->stream));
+  sm->cap_tokens = 0;      // (until all of it stands: where memory runs out on the way, the next step starts over)
   auto fr = [](auto*& p) { if (p) (void)hipFree(p); p = nullptr; };
   fr(sm->x); fr(sm->xs); fr(sm->a); fr(sm->proj); fr(sm->ql); fr(sm->lat); fr(sm->o); fr(sm->selw); fr(sm->yh); fr(sm->yd); fr(sm->xn); fr(sm->lg);
   fr(sm->sel); fr(sm->perm); fr(sm->ptok); fr(sm->tile_e); fr(sm->tile_m0); fr(sm->meta_dev); fr(sm->zr);
