@@ -82,7 +82,8 @@ struct NormConvArgs {
   float eps;
 };
 // TAPS: 4 and 1 have the filter's size at compile time (its taps arrive four a load and stand in registers by number); 0: any.  The row and its predecessors are asked for
-// before the sums of squares, whose barrier they cross in flight (four taps, 1024 channels: 7.4 -> 3.2 us for a few rows, 43 -> 17 for some 2400, which selecting taps by number bounded).
+// before the sums of squares, whose barrier they cross in flight (four taps, 1024 channels: the median launch of four decoded rows 8.0 -> 3.8 us,
+// some 2400 rows 45 -> 15; selecting taps by number bounded it).
 template <int TAPS>
 __global__ __launch_bounds__(256) void norm_conv_kernel(StepMeta m, NormConvArgs a) {
   __shared__ float s_rinv[CONV_MAX_TAPS][NORM_MAX_GROUPS];
@@ -364,7 +365,8 @@ __global__ __launch_bounds__(256) void latent_attn_merge_kernel(LatentAttnArgs a
 __device__ __forceinline__ void wave_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); }
 
 // ---- the products of a router for one token, w [n][K] . h [K] in fp32, by a workgroup of four waves into LDS.  A step of few tokens is bound by its launches (16 tokens of
-// 1024 channels, 8 experts: 5.5 us for the products and 4.4 for the choice behind them, 4.2 together), so its choice kernels take the products themselves.
+// 1024 channels, 8 experts: 5.5 us for the products and 4.4 for the choice behind them, 4.4 together; one token of 2048 channels, 20 experts: 4.7 and 6.8, 11.1 together), so its
+// choice kernels take the products themselves.
 struct RouterInput { const float* h; long long ldh; const float* w; int n, K; };      // h nullptr: the products are given
 constexpr int ROUTER_FUSED_MAX = 64;      // products a choice kernel takes itself
 __device__ __forceinline__ void router_products(const RouterInput& in, int t, float* s_z) {
