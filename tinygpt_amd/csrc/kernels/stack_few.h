@@ -163,16 +163,18 @@ __global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_kernel(const
   for (int o = threadIdx.x; o < MB * 256; o += blockDim.x) {
     const int l = o & 63, ir = o >> 6, m = mbase + (ir >> 2) * 16 + 4 * (l >> 4) + (ir & 3), n = n0 + (l & 15);
     if (m >= mend || n >= a.N) continue;
+    auto total = [&](auto WAVES, int b) {                           // (all on their way at once)
+      constexpr int W = decltype(WAVES)::value;
+      float t[W], s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < W; w++) t[w] = red[((min(w, nw - 1) * NB + b) * MB * 4 + ir) * 64 + l];
+#pragma unroll
+      for (int w = 0; w < W; w++) s[w & 3] += w < nw ? t[w] : 0.f;
+      return (s[0] + s[1]) + (s[2] + s[3]);
+    };
     float v[NB];
 #pragma unroll
-    for (int b = 0; b < NB; b++) {
-      float t[few_max_waves(MB)], s[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int w = 0; w < few_max_waves(MB); w++) t[w] = red[((min(w, nw - 1) * NB + b) * MB * 4 + ir) * 64 + l];      // (all on their way at once)
-#pragma unroll
-      for (int w = 0; w < few_max_waves(MB); w++) s[w & 3] += w < nw ? t[w] : 0.f;
-      v[b] = (s[0] + s[1]) + (s[2] + s[3]);
-    }
+    for (int b = 0; b < NB; b++) v[b] = nw <= 4 ? total(std::integral_constant<int, 4>{}, b) : nw <= 8 ? total(std::integral_constant<int, 8>{}, b) : total(std::integral_constant<int, few_max_waves(MB)>{}, b);
     sg_finish<EPI>(a, z, m, n, v[0], v[NB - 1]);
   }
 }
