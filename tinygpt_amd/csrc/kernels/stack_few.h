@@ -174,7 +174,11 @@ __global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_kernel(const
     };
     float v[NB];
 #pragma unroll
-    for (int b = 0; b < NB; b++) v[b] = nw <= 4 ? total(std::integral_constant<int, 4>{}, b) : nw <= 8 ? total(std::integral_constant<int, 8>{}, b) : total(std::integral_constant<int, few_max_waves(MB)>{}, b);
+    for (int b = 0; b < NB; b++)
+      v[b] = nw == 1   ? total(std::integral_constant<int, 1>{}, b)
+             : nw <= 4 ? total(std::integral_constant<int, 4>{}, b)
+             : nw <= 8 ? total(std::integral_constant<int, 8>{}, b)
+                       : total(std::integral_constant<int, few_max_waves(MB)>{}, b);
     sg_finish<EPI>(a, z, m, n, v[0], v[NB - 1]);
   }
 }
