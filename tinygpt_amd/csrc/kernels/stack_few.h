@@ -16,7 +16,7 @@
 // The host picks waves and ring depth so that narrow matrices (N / 16 workgroups) have as much of K in flight at once as LDS holds.
 // Any M, N; K a multiple of 8, 16-byte aligned rows (launch_gemm's condition).
 //
-// Measured against the vector form (us, medians of a step's launches, bf16): sixteen rows 2 x 3072 x 1024 19.0 -> 9.0, 32000 x 1024 82 -> 24; eight rows 2 x 8192 x 2048 35 -> 20,
+// Measured against the vector form (us, medians of a step's launches, bf16): sixteen rows 2 x 3072 x 1024 19.0 -> 8.5, 32000 x 1024 82 -> 24; eight rows 2 x 8192 x 2048 35 -> 20,
 // 2048 x 8192 26 -> 14; four rows 2 x 8192 x 2048 22.7 -> 19.8 (3.4 TB/s), 2048 x 8192 13.0 -> 14.2; against the 64-wide tiles, 47 rows: 2 x 3072 x 1024 27 -> 17, 1024 x 3072 42 -> 20.
 #pragma once
 #include "gemm_dma.h"

@@ -94,7 +94,7 @@ constexpr int GROUPED_FEW_PAIRS = 128, GROUPED_FEW_ROWS = 16, FEW_ROWS_MAX = 64;
 // the vector kernel serves one and two rows (1024 x 1024, two rows: 4.4 us against 5.4; 3072 x 1024 gate and up: 6.8 against 7.7; four rows 6.0 against 5.5), stack_few_kernel
 // three to 64 and the grouped tiles.  Where the line at 64 rows lies, us of the few-row kernel against the 64-wide tiles at 64 rows, bf16: 1024 x 3072 20 / 42, 2048 x 8192 39 / 92,
 // 2 x 3072 x 1024 17.5 / 26, four of 2048 x 2048 42 / 45; products whose tiles fill the chip are the faster ones on the tiles, in two 16-bit terms where the few-row kernel rounds
-// nothing: 2 x 8192 x 2048 70 / 47, 32000 x 1024 73 / 30 (fp32 storage 84 / 100, 79 / 58).  A step takes the few-row kernel for all of them: four layers of 2048 channels and 8192
+// nothing: 2 x 8192 x 2048 69 / 47, 32000 x 1024 72 / 29 (fp32 storage 84 / 100, 79 / 58).  A step takes the few-row kernel for all of them: four layers of 2048 channels and 8192
 // hidden ones, 33 / 64 rows, 1050 / 1150 us against 1490 / 1610, 1085 with the products that fill the chip on tiles, whose logits are twice as far from 64 bits (9.5e-5 against 4.9e-5)
 constexpr int GEMV_ROWS_MAX = 2;
 constexpr int FEW_COLS_ANY_ROWS = 64;      // a matrix of so few rows (the router's) takes the few-row kernel whatever the step's size: the 64-wide matrix-core tiles would stand mostly empty
