@@ -224,6 +224,9 @@ __device__ __forceinline__ float round_storage_mode(float v, int mode) {
   return mode == 1 ? rb : (mode == 2 ? rh : v);
 }
 
+// LDS that one wave writes and reads: its accesses stay in program order
+__device__ __forceinline__ void wave_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); }
+
 // Block-wide sum over 256 threads (4 waves) through a 4-float LDS scratch; every thread gets the result.
 __device__ __forceinline__ float block_sum_256(float v, float* scratch4) {
   v = group_sum<64>(v);

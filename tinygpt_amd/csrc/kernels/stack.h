@@ -361,9 +361,6 @@ __global__ __launch_bounds__(256) void latent_attn_merge_kernel(LatentAttnArgs a
   }
 }
 
-// LDS that one wave writes and reads: its accesses stay in program order
-__device__ __forceinline__ void wave_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); }
-
 // ---- the products of a router for one token, w [n][K] . h [K] in fp32, by a workgroup of four waves into LDS.  A step of few tokens is bound by its launches (16 tokens of
 // 1024 channels, 8 experts: 5.5 us for the products and 4.4 for the choice behind them, 4.4 together; one token of 2048 channels, 20 experts: 4.7 and 6.8, 11.1 together), so its
 // choice kernels take the products themselves.

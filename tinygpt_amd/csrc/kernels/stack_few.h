@@ -1,5 +1,5 @@
-// stack_few.h — the products of layered models (stack_gemm.h) for A FEW rows: 3 to 64 activation rows, the tiles of sixteen rows of a grouped product with few
-// (token, expert) pairs, and matrices of so few rows (a router's) that 64-wide tiles would stand empty.
+// stack_few.h — the products of layered models (stack_gemm.h) for A FEW rows: 3 to 64 activation rows, and matrices of so few rows (a router's) that 64-wide tiles
+// would stand empty.
 //
 // What bounds it: the weights cross once, so the stream of weight bytes is the floor; the vector form (stack_gemv_kernel, two columns a wave) instead moved every
 // activation row through L2 for every two columns — eight rows of 4 KB for 4 KB of weights — and streamed the weights again for every tile of four or eight rows.
@@ -43,11 +43,7 @@ __global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_kernel(const
   extern __shared__ __attribute__((aligned(1024))) unsigned char few_lds[];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
   const int li = lane & 15, q = lane >> 4;                          // row (column) of the operands, quarter of a half step's k
-  int z, mbase, mend;
-  if (a.z_off) {
-    if ((int)blockIdx.y >= *a.n_tiles) return;
-    z = a.tile_z[blockIdx.y]; mbase = a.tile_m0[blockIdx.y]; mend = min(a.z_off[z + 1], mbase + 16 * MB);
-  } else { z = blockIdx.z; mbase = blockIdx.y * 16 * MB; mend = min(a.M, mbase + 16 * MB); }
+  const int z = blockIdx.z, mbase = blockIdx.y * 16 * MB, mend = min(a.M, mbase + 16 * MB);
   const int n0 = blockIdx.x * 16, steps = (a.K + 63) >> 6;
   unsigned char* ring = few_lds + (size_t)wv * depth * STEP;
   const unsigned ring_lds = (unsigned)(size_t)ring;

@@ -16,6 +16,7 @@ namespace tgx {
 
 enum { SG_ACT_NONE = 0, SG_ACT_TANH = 1, SG_ACT_DECAY = 2, SG_ACT_GELU = 3, SG_ACT_SOFTPLUS = 4, SG_ACT_RELU2 = 5, SG_ACT_HEAD_DECAY = 6, SG_ACT_GELU_TANH = 7 };
 enum { SG_STORE = 0, SG_ADD = 1, SG_GATE = 2, SG_EXPERT_ACT = 3, SG_ROWSCALE = 4, SG_SILU_MUL = 5 };
+constexpr int ROWS_MAX_PAIRS = 128;      // stack_rows.h: pairs whose choices a workgroup reads
 constexpr bool sg_dual(int epi) { return epi == SG_EXPERT_ACT || epi == SG_SILU_MUL; }
 struct StackGemmArgs {
   const float* A; long long lda; int a_zoff;
@@ -31,7 +32,7 @@ struct StackGemmArgs {
                                //           exp(-exp(a_log[n / head_cols]) ln(1 + e^v)) (a decay per channel whose rate has a factor per head)
                                // SG_SILU_MUL: SG_ACT_GELU_TANH takes the tanh form of gelu instead of silu
   const float* a_log; int head_cols;
-  const float* in_w; const int* in_rows;         // SG_STORE: row m's product is first multiplied by in_w[in_rows[m]] (a router weight on its expert's input; nullptr: none)
+  const float* in_w; const int* in_rows;         // SG_STORE: row m's product is first multiplied by in_w[in_rows[m]] (in_rows nullptr: in_w[m]; a router weight on its expert's input; in_w nullptr: none)
   const float* bias;           // SG_STORE: [N] per z (column z * c_zoff + n), nullptr: none
   int gate_col0, gate_heads;   // SG_STORE: columns [gate_col0, + gate_heads) leave as log input gates cap tanh(v / cap), the next gate_heads columns as log forget gates
   float gate_cap;              //           logsigmoid(cap tanh(v / cap)) (the two gate rows of a matrix-memory layer's input product); gate_heads 0: none
@@ -43,6 +44,8 @@ struct StackGemmArgs {
   // stack_line.h: the activations, or the outputs, as lines of two 16-bit terms [row][K / 32][hi 32 | lo 32] in the place of A, or of C (nullptr: fp32)
   const unsigned short* At; unsigned short* Ct;
   int a_count;                 // gathered products (a_rows): rows of A
+  // stack_rows.h: the choices of a step's pairs (an expert each; those from `experts` on have no product); pair p reads row p / pairs_per_row of A and writes row p of C
+  const int* sel; int n_pairs, experts, pairs_per_row, tokens;
 };
 
 // an expert's activation: g = min(gate, limit), u = clamp(up, -limit, limit); g * sigmoid(1.702 g) * (u + 1)
@@ -73,7 +76,7 @@ __device__ __forceinline__ float gate_mul(const StackGemmArgs& a, float gate, fl
 // the epilogue on the accumulated sum v (dual products: v of the first matrix, v2 of the second) of grouped / batched row m, row crow and column n of C; old: what C holds (SG_ADD)
 template <int EPI>
 __device__ __forceinline__ float sg_value(const StackGemmArgs& a, int z, int m, size_t crow, int n, float v, float v2, float old) {
-  if constexpr (EPI == SG_STORE) return store_value(a, a.in_w ? v * a.in_w[a.in_rows[m]] : v, (size_t)z * a.c_zoff + n, n);
+  if constexpr (EPI == SG_STORE) return store_value(a, a.in_w ? v * a.in_w[a.in_rows ? a.in_rows[m] : m] : v, (size_t)z * a.c_zoff + n, n);
   else if constexpr (EPI == SG_ADD) return fmaf(v, a.scale, old);
   else if constexpr (EPI == SG_GATE) return v / (1.0f + expf(-a.G[crow * a.ldg + a.g_col0 + (a.g_per_z ? (size_t)z : (size_t)z * a.c_zoff + n)]));
   else if constexpr (EPI == SG_EXPERT_ACT) return expert_act(v, v2, a.limit);

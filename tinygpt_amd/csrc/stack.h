@@ -173,7 +173,9 @@ size_t mix_mfma_wg_lds(int heads, int kv_heads);      // LDS bytes of one of its
 bool stack_allow_lds(tgx_ctx* c, const void* kernel, size_t bytes);
 // stack_few.hip
 namespace tgx { struct StackGemmArgs; }
-void launch_stack_few(tgx_ctx* c, const tgx::StackGemmArgs& a, int epi, int nz, int grouped_tiles, int dt);
+void launch_stack_few(tgx_ctx* c, const tgx::StackGemmArgs& a, int epi, int nz, int dt);
+// stack_rows.hip
+void launch_stack_rows(tgx_ctx* c, const tgx::StackGemmArgs& a, int epi, int dt);
 
 // stack_line.hip
 int stack_line_tile(const tgx_ctx* c, long long M, long long N, bool dual, int nz);      // 256 or 128 rows a tile; 0: the product is too small for such tiles

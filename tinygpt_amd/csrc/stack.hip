@@ -89,10 +89,10 @@ void launch_gemv_t(tgx_ctx* c, const tgx::StackGemmArgs& a, dim3 grid, int mr, b
   else if (ksplit) go(std::integral_constant<int, 2>{}, std::true_type{});
   else go(std::integral_constant<int, 2>{}, std::false_type{});
 }
-// rows per tile of a grouped product's plan (moe_plan_kernel tile_m): steps of few (token, expert) pairs stream the experts through the few-row kernel
-constexpr int GROUPED_FEW_PAIRS = 128, GROUPED_FEW_ROWS = 16, FEW_ROWS_MAX = 64;
+// steps of up to so many (token, expert) pairs take the experts' products without a plan (stack_rows_kernel); products of up to so many rows the few-row kernel
+constexpr int GROUPED_FEW_PAIRS = tgx::ROWS_MAX_PAIRS, FEW_ROWS_MAX = 64;
 // the vector kernel serves one and two rows (1024 x 1024, two rows: 4.4 us against 5.4; 3072 x 1024 gate and up: 6.8 against 7.7; four rows 6.0 against 5.5), stack_few_kernel
-// three to 64 and the grouped tiles.  Where the line at 64 rows lies, us of the few-row kernel against the 64-wide tiles at 64 rows, bf16: 1024 x 3072 20 / 42, 2048 x 8192 39 / 92,
+// three to 64.  Where the line at 64 rows lies, us of the few-row kernel against the 64-wide tiles at 64 rows, bf16: 1024 x 3072 20 / 42, 2048 x 8192 39 / 92,
 // 2 x 3072 x 1024 17.5 / 26, four of 2048 x 2048 42 / 45; products whose tiles fill the chip are the faster ones on the tiles, in two 16-bit terms where the few-row kernel rounds
 // nothing: 2 x 8192 x 2048 69 / 47, 32000 x 1024 72 / 29 (fp32 storage 84 / 100, 79 / 58).  A step takes the few-row kernel for all of them: four layers of 2048 channels and 8192
 // hidden ones, 33 / 64 rows, 1050 / 1150 us against 1490 / 1610, 1085 with the products that fill the chip on tiles, whose logits are twice as far from 64 bits (9.5e-5 against 4.9e-5)
@@ -142,11 +142,11 @@ void scratch_sizes(tgx_ctx* c) {
   }
   sm->terms_cols = (size_t)cols;
 }
-// tiles of the two grouped products of an expert layer (both must be able to take them: their contraction lengths are the width and the expert width).  np: (token, expert)
-// pairs, E: experts, up_n: columns of the first product (gate and up together)
+// rows per tile of the two grouped products of an expert layer's plan (both must be able to take them: their contraction lengths are the width and the expert width); 0: no plan,
+// the pairs' kernel.  np: (token, expert) pairs, E: experts, up_n: columns of the first product (gate and up together)
 int grouped_tile_rows(tgx_ctx* c, int np, int width, int ff, int E, int T, int up_n) {
   StackModel* sm = c->stack;
-  if (sm->gemv && np <= GROUPED_FEW_PAIRS && width % 8 == 0 && ff % 8 == 0) return GROUPED_FEW_ROWS;
+  if (sm->gemv && np <= GROUPED_FEW_PAIRS && width % 8 == 0 && ff % 8 == 0) return 0;
   if (sm->line && c->dt != tgx::DT_F32 && width % 64 == 0 && ff % 64 == 0 && E > 0) {
     const int tile = stack_line_tile_grouped(c, np, E, up_n);
     if (tile && ensure_terms(c, (size_t)T * 2 * width) && ensure_terms2(c, (size_t)np * 2 * ff)) return tile;
@@ -180,6 +180,11 @@ void launch_gemm(tgx_ctx* c, tgx::StackGemmArgs a, int epi, int nz, int grouped_
   if (a.M <= 0 && !a.z_off) return;
   if (a.N <= 0 || a.K <= 0) return;
   a.terms = c->act16 ? 1 : 2;
+  if (a.sel) {
+    if (slices_ok(a)) launch_stack_rows(c, a, epi, dt);
+    else c->launch_fault = "grouped product: operands that the pairs' kernel cannot take";
+    return;
+  }
   const int tile = a.z_off ? (grouped_tile >= 128 ? grouped_tile : 0) : line_tile(c, a, epi, nz, dt);
   if (tile) {
     const int cols = a.K + a.a_zoff * (nz - 1), rows = a.a_rows ? a.a_count : a.M;
@@ -195,9 +200,8 @@ void launch_gemm(tgx_ctx* c, tgx::StackGemmArgs a, int epi, int nz, int grouped_
                    (!a.B2 || (uintptr_t)a.B2 % 16 == 0);
   const bool dual = tgx::sg_dual(epi);
   // few rows: the weight-streaming kernels
-  const bool few = sm->gemv && slices_ok(a) && (a.z_off ? grouped_tile == GROUPED_FEW_ROWS : (a.M <= FEW_ROWS_MAX || a.N <= FEW_COLS_ANY_ROWS));
-  if (a.z_off && grouped_tile == GROUPED_FEW_ROWS && !few) { c->launch_fault = "grouped product: the plan was made for the few-row kernel, which these operands cannot take"; return; }
-  if (few && (a.z_off || a.M > GEMV_ROWS_MAX)) { launch_stack_few(c, a, epi, nz, a.z_off ? grouped_rows / GROUPED_FEW_ROWS + std::min(groups, grouped_rows) : 0, dt); return; }
+  const bool few = sm->gemv && slices_ok(a) && !a.z_off && (a.M <= FEW_ROWS_MAX || a.N <= FEW_COLS_ANY_ROWS);
+  if (few && a.M > GEMV_ROWS_MAX) { launch_stack_few(c, a, epi, nz, dt); return; }
   if (few) {
     const int mr = a.M <= 1 ? 1 : 2;
     const bool ksplit = gemv_ksplit(c, a, nz);
@@ -251,6 +255,28 @@ void launch_ff(tgx_ctx* c, tgx::StackGemmArgs up, int epi_up, tgx::StackGemmArgs
   if (line && ensure_terms(c, (size_t)(up.a_rows ? up.a_count : up.M) * 2 * up.K) && ensure_terms2(c, (size_t)up.M * 2 * up.N)) { up.Ct = sm->terms2; down.At = sm->terms2; }
   launch_gemm(c, up, epi_up, 1, np, groups, tile);
   launch_gemm(c, down, epi_down, 1, np, groups, tile);
+}
+
+// an expert layer's two products over the step's pairs: up on the rows of h, down on its outputs, a row of yd per pair.  E: experts that the choices name, E_tiles: those that
+// have products (the others' outputs are identities)
+void launch_experts(tgx_ctx* c, tgx::StackGemmArgs up, int epi_up, tgx::StackGemmArgs down, int epi_down, int T, int top, int E, int E_tiles) {
+  StackModel* sm = c->stack;
+  const int np = T * top, tile = grouped_tile_rows(c, np, up.K, up.N, E, T, tgx::sg_dual(epi_up) ? 2 * up.N : up.N);
+  up.M = down.M = np;
+  if (!tile) {
+    up.sel = down.sel = sm->sel; up.n_pairs = down.n_pairs = np; up.experts = down.experts = E_tiles; up.tokens = down.tokens = T; up.pairs_per_row = top; down.pairs_per_row = 1;
+    launch_gemm(c, up, epi_up, 1);
+    launch_gemm(c, down, epi_down, 1);
+    return;
+  }
+  tgx::MoePlanArgs pa{};
+  pa.sel = sm->sel; pa.n_pairs = np; pa.E = E; pa.top = top; pa.tile_m = tile; pa.E_tiles = E_tiles;
+  pa.off = sm->moe_off; pa.perm = sm->perm; pa.tok = sm->ptok; pa.tile_e = sm->tile_e; pa.tile_m0 = sm->tile_m0; pa.n_tiles = sm->n_tiles;
+  hipLaunchKernelGGL(tgx::moe_plan_kernel, dim3(1), dim3(1024), 0, c->stream, pa);
+  up.a_rows = sm->ptok; up.a_count = T; down.c_rows = sm->perm;
+  if (up.in_w) up.in_rows = sm->perm;
+  for (tgx::StackGemmArgs* g : {&up, &down}) { g->z_off = sm->moe_off; g->tile_z = sm->tile_e; g->tile_m0 = sm->tile_m0; g->n_tiles = sm->n_tiles; }
+  launch_ff(c, up, epi_up, down, epi_down, np, E, tile);
 }
 
 // a router's products on the rows h: true: the choice kernel takes them itself (steps of few tokens); false: they stand in zr
@@ -322,8 +348,8 @@ int ensure_ws(tgx_ctx* c, int T) {
     const size_t np = std::max<size_t>(n * (size_t)sm->max_top, sm->hyper ? GROUPED_FEW_PAIRS : 0);      // (a shared expert that rides among the choices: at most that many pairs)
     if ((rc = dev_alloc(c, &sm->zr, n * (size_t)(sm->max_E + 1))) || (rc = dev_alloc(c, &sm->selw, np)) || (rc = dev_alloc(c, &sm->sel, np)) || (rc = dev_alloc(c, &sm->perm, np)) || (rc = dev_alloc(c, &sm->ptok, np)) ||
         (rc = dev_alloc(c, &sm->yh, np * (size_t)sm->max_ff + n * (size_t)sm->max_sff)) || (rc = dev_alloc(c, &sm->yd, np * W)) ||
-        (rc = dev_alloc(c, &sm->tile_e, std::max<size_t>(np / 64, GROUPED_FEW_PAIRS / GROUPED_FEW_ROWS) + (size_t)sm->max_E + 1)) ||
-        (rc = dev_alloc(c, &sm->tile_m0, std::max<size_t>(np / 64, GROUPED_FEW_PAIRS / GROUPED_FEW_ROWS) + (size_t)sm->max_E + 1))) return rc;
+        (rc = dev_alloc(c, &sm->tile_e, np / 64 + (size_t)sm->max_E + 1)) ||
+        (rc = dev_alloc(c, &sm->tile_m0, np / 64 + (size_t)sm->max_E + 1))) return rc;
   }
   sm->meta_cap = (size_t)9 * n + (size_t)4 * sm->d.max_seqs;
   if ((rc = dev_alloc(c, &sm->meta_dev, sm->meta_cap))) return rc;
@@ -430,21 +456,13 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
       ra.z = sm->zr; ra.br = w.b_router; ra.sel = sm->sel; ra.selw = sm->selw; ra.E = ld.experts; ra.top = top;
       if (route(c, ra.in, sm->a, w.w_router, ld.experts, T)) hipLaunchKernelGGL(tgx::router_topk_kernel<true>, dim3(T), dim3(256), 0, c->stream, ra);
       else hipLaunchKernelGGL(tgx::router_topk_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
-      const int np = T * top;
-      tgx::MoePlanArgs pa{};
-      pa.sel = sm->sel; pa.n_pairs = np; pa.E = ld.experts; pa.top = top; pa.tile_m = grouped_tile_rows(c, np, W, ld.ff, ld.experts, T, 2 * ld.ff);
-      pa.off = sm->moe_off; pa.perm = sm->perm; pa.tok = sm->ptok; pa.tile_e = sm->tile_e; pa.tile_m0 = sm->tile_m0; pa.n_tiles = sm->n_tiles;
-      hipLaunchKernelGGL(tgx::moe_plan_kernel, dim3(1), dim3(1024), 0, c->stream, pa);
-      // yh[n] = act(gate_e . a[tok(n)], up_e . a[tok(n)]) over the pairs grouped by expert
+      // yh[pair] = act(gate_e . a[token], up_e . a[token]), yd[pair] = router weight * (down_e . yh[pair])
       g = tgx::StackGemmArgs{};
-      g.A = sm->a; g.lda = W; g.a_rows = sm->ptok; g.a_count = T; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff;
-      g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = ld.ff; g.K = W; g.limit = ld.limit;
-      // yd[pair] = router weight * (down_e . yh[n])
+      g.A = sm->a; g.lda = W; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff; g.N = ld.ff; g.K = W; g.limit = ld.limit;
       const tgx::StackGemmArgs gu = g;
       g = tgx::StackGemmArgs{};
-      g.A = sm->yh; g.lda = ld.ff; g.B = w.w_down; g.ldb = ld.ff; g.b_zstride = (long long)W * ld.ff; g.C = sm->yd; g.ldc = W; g.c_rows = sm->perm;
-      g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = W; g.K = ld.ff; g.rw = sm->selw;
-      launch_ff(c, gu, tgx::SG_EXPERT_ACT, g, tgx::SG_ROWSCALE, np, ld.experts, pa.tile_m);
+      g.A = sm->yh; g.lda = ld.ff; g.B = w.w_down; g.ldb = ld.ff; g.b_zstride = (long long)W * ld.ff; g.C = sm->yd; g.ldc = W; g.N = W; g.K = ld.ff; g.rw = sm->selw;
+      launch_experts(c, gu, tgx::SG_EXPERT_ACT, g, tgx::SG_ROWSCALE, T, top, ld.experts, ld.experts);
     }
     tgx::CombineDepthArgs cd{};
     cd.x = sm->x; cd.y = sm->yd; cd.xs = sm->xs; cd.slot_stride = slot_stride; cd.dw = w.dwa; cd.W = W; cd.top = top; cd.n_res = li + 2;
@@ -666,18 +684,12 @@ void run_choice_experts(tgx_ctx* c, StackLayerW& w, const float* hin, int T) {
   else hipLaunchKernelGGL(tgx::router_group_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
   const int np = T * top;
   if (ld.experts > 0) {
-    tgx::MoePlanArgs pa{};
-    pa.sel = sm->sel; pa.n_pairs = np; pa.E = E; pa.top = top; pa.tile_m = grouped_tile_rows(c, np, W, ld.ff, E, T, 2 * ld.ff); pa.E_tiles = ld.experts;
-    pa.off = sm->moe_off; pa.perm = sm->perm; pa.tok = sm->ptok; pa.tile_e = sm->tile_e; pa.tile_m0 = sm->tile_m0; pa.n_tiles = sm->n_tiles;
-    hipLaunchKernelGGL(tgx::moe_plan_kernel, dim3(1), dim3(1024), 0, c->stream, pa);
     g = tgx::StackGemmArgs{};
-    g.A = hin; g.lda = W; g.a_rows = sm->ptok; g.a_count = T; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff;
-    g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = ld.ff; g.K = W;
+    g.A = hin; g.lda = W; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff; g.N = ld.ff; g.K = W;
     const tgx::StackGemmArgs gu = g;
     g = tgx::StackGemmArgs{};
-    g.A = sm->yh; g.lda = ld.ff; g.B = w.w_down; g.ldb = ld.ff; g.b_zstride = (long long)W * ld.ff; g.C = sm->yd; g.ldc = W; g.c_rows = sm->perm;
-    g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = W; g.K = ld.ff; g.rw = sm->selw;
-    launch_ff(c, gu, tgx::SG_SILU_MUL, g, tgx::SG_ROWSCALE, np, E, pa.tile_m);
+    g.A = sm->yh; g.lda = ld.ff; g.B = w.w_down; g.ldb = ld.ff; g.b_zstride = (long long)W * ld.ff; g.C = sm->yd; g.ldc = W; g.N = W; g.K = ld.ff; g.rw = sm->selw;
+    launch_experts(c, gu, tgx::SG_SILU_MUL, g, tgx::SG_ROWSCALE, T, top, E, ld.experts);
   }
   if (ld.shared_ff > 0) {
     float* hsh = sm->yh + (size_t)np * std::max(1, ld.ff);
@@ -1097,18 +1109,12 @@ void run_affine_ff(tgx_ctx* c, StackLayerW& w, int T) {
   ra.sigmoid_scores = ld.router_fn == 1; ra.group_top2 = ld.group_score == 1; ra.normalise = ld.router_norm;
   if (route(c, ra.in, sm->a, w.w_router, E, T)) hipLaunchKernelGGL(tgx::router_group_kernel<true>, dim3(T), dim3(256), 0, c->stream, ra);
   else hipLaunchKernelGGL(tgx::router_group_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
-  tgx::MoePlanArgs pa{};
-  pa.sel = sm->sel; pa.n_pairs = np; pa.E = E; pa.top = top; pa.tile_m = grouped_tile_rows(c, np, W, ld.ff, E, T, 2 * ld.ff); pa.E_tiles = E;
-  pa.off = sm->moe_off; pa.perm = sm->perm; pa.tok = sm->ptok; pa.tile_e = sm->tile_e; pa.tile_m0 = sm->tile_m0; pa.n_tiles = sm->n_tiles;
-  hipLaunchKernelGGL(tgx::moe_plan_kernel, dim3(1), dim3(1024), 0, c->stream, pa);
   g = tgx::StackGemmArgs{};
-  g.A = sm->a; g.lda = W; g.a_rows = sm->ptok; g.a_count = T; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff;
-  g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = ld.ff; g.K = W;
+  g.A = sm->a; g.lda = W; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff; g.N = ld.ff; g.K = W;
   const tgx::StackGemmArgs gu = g;
   g = tgx::StackGemmArgs{};
-  g.A = sm->yh; g.lda = ld.ff; g.B = w.w_down; g.ldb = ld.ff; g.b_zstride = (long long)W * ld.ff; g.C = sm->yd; g.ldc = W; g.c_rows = sm->perm;
-  g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = W; g.K = ld.ff; g.rw = sm->selw;
-  launch_ff(c, gu, tgx::SG_SILU_MUL, g, tgx::SG_ROWSCALE, np, E, pa.tile_m);
+  g.A = sm->yh; g.lda = ld.ff; g.B = w.w_down; g.ldb = ld.ff; g.b_zstride = (long long)W * ld.ff; g.C = sm->yd; g.ldc = W; g.N = W; g.K = ld.ff; g.rw = sm->selw;
+  launch_experts(c, gu, tgx::SG_SILU_MUL, g, tgx::SG_ROWSCALE, T, top, E, E);
   if (ld.shared_ff > 0) {      // the shared expert runs for every token, without a gate of its own
     float* hsh = sm->yh + (size_t)np * std::max(1, ld.ff);
     g = tgx::StackGemmArgs{};
@@ -1750,7 +1756,7 @@ void run_channel_delta(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T
 // the shared expert's product takes the wide tiles by itself.)
 bool shared_rides(const tgx_ctx* c, const StackLayerW& w, int T) {
   const int np = T * (w.d.top + 1);
-  return w.shared_slot && np <= GROUPED_FEW_PAIRS && c->stack->gemv && c->stack->d.width % 8 == 0 && w.d.ff % 8 == 0;      // (the plan's tiles of few rows)
+  return w.shared_slot && np <= GROUPED_FEW_PAIRS && c->stack->gemv && c->stack->d.width % 8 == 0 && w.d.ff % 8 == 0;      // (the pairs' kernel)
 }
 // the feed-forward into yd (one row per token, or a row per choice for experts) and ysh (the shared expert's row, unless it rides among the choices)
 void run_hyper_ff(tgx_ctx* c, StackLayerW& w, int T) {
@@ -1768,19 +1774,13 @@ void run_hyper_ff(tgx_ctx* c, StackLayerW& w, int T) {
   ra.z = sm->zr; ra.ldz = ld.experts; ra.sel = sm->sel; ra.selw = sm->selw; ra.E = ld.experts; ra.top = ld.top; ra.shared = ride; ra.groups = 1; ra.keep = 1; ra.scale = 1.f; ra.sigmoid_scores = ld.router_fn == 1; ra.normalise = ld.router_norm;
   if (route(c, ra.in, sm->a, w.w_router, ld.experts, T)) hipLaunchKernelGGL(tgx::router_group_kernel<true>, dim3(T), dim3(256), 0, c->stream, ra);
   else hipLaunchKernelGGL(tgx::router_group_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
-  tgx::MoePlanArgs pa{};
-  pa.sel = sm->sel; pa.n_pairs = np; pa.E = E; pa.top = top; pa.tile_m = grouped_tile_rows(c, np, W, ld.ff, E, T, ld.ff); pa.E_tiles = E;
-  pa.off = sm->moe_off; pa.perm = sm->perm; pa.tok = sm->ptok; pa.tile_e = sm->tile_e; pa.tile_m0 = sm->tile_m0; pa.n_tiles = sm->n_tiles;
-  hipLaunchKernelGGL(tgx::moe_plan_kernel, dim3(1), dim3(1024), 0, c->stream, pa);
-  // yh[n] = max(up_e (w h), 0)^2 over the pairs grouped by expert: up_e is linear, so the weight multiplies its product
+  // yh[pair] = max(up_e (w h), 0)^2: up_e is linear, so the weight multiplies its product
   g = tgx::StackGemmArgs{};
-  g.A = sm->a; g.lda = W; g.a_rows = sm->ptok; g.a_count = T; g.B = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff; g.scale = 1.f; g.act = tgx::SG_ACT_RELU2;
-  g.in_w = sm->selw; g.in_rows = sm->perm; g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = ld.ff; g.K = W;
+  g.A = sm->a; g.lda = W; g.B = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff; g.scale = 1.f; g.act = tgx::SG_ACT_RELU2; g.in_w = sm->selw; g.N = ld.ff; g.K = W;
   const tgx::StackGemmArgs gu = g;
   g = tgx::StackGemmArgs{};
-  g.A = sm->yh; g.lda = ld.ff; g.B = w.w_down; g.ldb = ld.ff; g.b_zstride = (long long)W * ld.ff; g.C = sm->yd; g.ldc = W; g.c_rows = sm->perm; g.scale = 1.f;
-  g.z_off = sm->moe_off; g.tile_z = sm->tile_e; g.tile_m0 = sm->tile_m0; g.n_tiles = sm->n_tiles; g.M = np; g.N = W; g.K = ld.ff;
-  launch_ff(c, gu, tgx::SG_STORE, g, tgx::SG_STORE, np, E, pa.tile_m);
+  g.A = sm->yh; g.lda = ld.ff; g.B = w.w_down; g.ldb = ld.ff; g.b_zstride = (long long)W * ld.ff; g.C = sm->yd; g.ldc = W; g.scale = 1.f; g.N = W; g.K = ld.ff;
+  launch_experts(c, gu, tgx::SG_STORE, g, tgx::SG_STORE, T, top, E, E);
   if (ld.shared_ff > 0 && !ride) {
     float* hsh = sm->yh + (((size_t)np * ld.ff + 3) & ~(size_t)3);
     g = tgx::StackGemmArgs{};
