@@ -5,6 +5,7 @@
 // entered by one thread only: examples/inference/main.cpp, server/HttpServer.cpp:118-163).
 // There is NO CPU path in this library: every entry point either runs on the GPU or returns an error.
 #include <climits>
+#include <cstring>
 #include "ctx.h"
 #include "stack.h"
 
@@ -64,6 +65,40 @@ inline uint16_t host_f32_to_half(float f) {   // round-to-nearest-even, subnorma
   return (uint16_t)(sign | h);
 }
 
+}  // namespace
+
+// Results for the caller: by way of pinned halves of 1 MB, one on its way while the other is taken out.  A copy straight into memory that is not pinned stages or locks it inside the
+// runtime: 128 KB 60 us, 512 KB 28 to 214, 2 MB 110, 8 MB in one piece 475; so 13, 28, 89 and 330 (halves of 512 KB: 105 and 390; of 4 MB: 108 and 373).
+int copy_to_host(tgx_ctx* c, void* dst, const void* src, size_t bytes) {
+  constexpr size_t HALF = 1 << 20;
+  if (!c->stage) {
+    for (auto& e : c->stage_ev) if (!e) HIP_OK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (hipHostMalloc((void**)&c->stage, 2 * HALF, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      c->stage = nullptr;
+      HIP_OK(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
+      HIP_OK(c, hipStreamSynchronize(c->stream));
+      return TGX_OK;
+    }
+  }
+  size_t sent = 0, got = 0;
+  for (unsigned in = 0, out = 0; got < bytes; out++) {
+    for (; sent < bytes && in - out < 2; in++) {
+      const size_t n = std::min(HALF, bytes - sent);
+      HIP_OK(c, hipMemcpyAsync(c->stage + (in & 1) * HALF, (const char*)src + sent, n, hipMemcpyDeviceToHost, c->stream));
+      if (bytes > HALF) HIP_OK(c, hipEventRecord(c->stage_ev[in & 1], c->stream));
+      sent += n;
+    }
+    if (bytes > HALF) HIP_OK(c, hipEventSynchronize(c->stage_ev[out & 1]));
+    else HIP_OK(c, hipStreamSynchronize(c->stream));
+    const size_t n = std::min(HALF, bytes - got);
+    std::memcpy((char*)dst + got, c->stage + (out & 1) * HALF, n);
+    got += n;
+  }
+  return TGX_OK;
+}
+
+namespace {
 // host -> device copy with conversion to the compute dtype (== model().to(dtype), ModelLoader.cpp:84):
 // widening is exact, narrowing rounds to nearest even once.
 int upload_param(tgx_ctx* c, ebyte* dst, const void* host, int64_t n, int src_dtype) {
@@ -728,6 +763,8 @@ void tgx_destroy(tgx_ctx* c) {
   fr(c->slab_x); fr(c->slab_q); fr(c->slab_kraw); fr(c->slab_attn); fr(c->slab_h); fr(c->slab_logits); fr(c->slab_probs);
   fr(c->slab_part_val); fr(c->slab_part_idx); fr(c->slab_attn_part); fr(c->slab_tok); fr(c->slab_pos); fr(c->slab_prompt); fr(c->slab_k); fr(c->slab_v);
   if (c->host_ring) (void)hipHostFree(c->host_ring);
+  if (c->stage) (void)hipHostFree(c->stage);
+  for (auto& e : c->stage_ev) if (e) (void)hipEventDestroy(e);
   for (auto& e : c->ticket_ev) if (e) (void)hipEventDestroy(e);
   for (auto& e : c->prof.ev) if (e) (void)hipEventDestroy(e);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -815,9 +852,9 @@ int tgx_read_logits(tgx_ctx* c, float* out, int rounded) {
   if (!c || !out) return TGX_ERR_INVALID;
   if (!c->have_logits) return set_err(c, TGX_ERR_STATE, "no logits: call tgx_forward/tgx_decode first");
   HIP_OK(c, hipSetDevice(c->device));
-  HIP_OK(c, hipStreamSynchronize(c->stream));
   const size_t V = (size_t)c->d.vocab;
-  for (int b = 0; b < c->batch; b++) HIP_OK(c, hipMemcpy(out + b * V, c->rows[(size_t)b].logits, V * 4, hipMemcpyDeviceToHost));
+  int rc = copy_to_host(c, out, c->slab_logits, (size_t)c->batch * V * 4);
+  if (rc) return rc;
   if (rounded && c->dt != tgx::DT_F32)
     for (size_t i = 0; i < V * (size_t)c->batch; i++)
       out[i] = c->dt == tgx::DT_BF16 ? host_bf16_to_f32(host_f32_to_bf16(out[i])) : host_half_to_f32(host_f32_to_half(out[i]));
@@ -839,14 +876,14 @@ int tgx_sample(tgx_ctx* c, const tgx_sampler_cfg* cfg, uint64_t seed, int64_t* o
   note_sampled(c, 0, c->batch, *cfg);
   launch_sample(c, 0, c->batch, *cfg, /*advance_pos=*/false, /*log_step=*/false);
   HIP_OK(c, hipGetLastError());
-  HIP_OK(c, hipStreamSynchronize(c->stream));
+  std::vector<int> toks((size_t)c->batch);
+  int rc = copy_to_host(c, toks.data(), c->slab_tok, toks.size() * 4);
+  if (rc) return rc;
   for (int b = 0; b < c->batch; b++) {
-    int t = 0;
-    HIP_OK(c, hipMemcpy(&t, c->rows[(size_t)b].tok, 4, hipMemcpyDeviceToHost));
-    if (out_ids) out_ids[b] = t;
-    if (b == 0) c->last_sampled0 = t;
+    if (out_ids) out_ids[b] = toks[(size_t)b];
     c->row_tok[(size_t)b] = 1;
   }
+  if (!toks.empty()) c->last_sampled0 = toks[0];
   c->have_token = true;
   return TGX_OK;
 }
@@ -867,10 +904,8 @@ int tgx_decode(tgx_ctx* c, const tgx_sampler_cfg* cfg, uint64_t seed, int n_step
     std::vector<int> tmp((size_t)n_steps * B);
     const int64_t s0 = start % c->log_cap;
     const int64_t first = (s0 + n_steps <= c->log_cap) ? n_steps : c->log_cap - s0;
-    HIP_OK(c, hipMemcpyAsync(tmp.data(), c->tok_log + (size_t)s0 * B, (size_t)first * B * 4, hipMemcpyDeviceToHost, c->stream));
-    if (first < n_steps)
-      HIP_OK(c, hipMemcpyAsync(tmp.data() + (size_t)first * B, c->tok_log, (size_t)(n_steps - first) * B * 4, hipMemcpyDeviceToHost, c->stream));
-    HIP_OK(c, hipStreamSynchronize(c->stream));
+    if ((rc = copy_to_host(c, tmp.data(), c->tok_log + (size_t)s0 * B, (size_t)first * B * 4))) return rc;
+    if (first < n_steps && (rc = copy_to_host(c, tmp.data() + (size_t)first * B, c->tok_log, (size_t)(n_steps - first) * B * 4))) return rc;
     for (size_t i = 0; i < tmp.size(); i++) out_ids[i] = tmp[i];
     c->last_sampled0 = tmp[(size_t)(n_steps - 1) * B];
   }
@@ -1057,9 +1092,9 @@ int tgx_sample_row(tgx_ctx* c, int row, const tgx_sampler_cfg* cfg, uint64_t see
   note_sampled(c, row, 1, *cfg);
   launch_sample(c, row, 1, *cfg, /*advance_pos=*/false, /*log_step=*/false);
   HIP_OK(c, hipGetLastError());
-  HIP_OK(c, hipStreamSynchronize(c->stream));
   int t = 0;
-  HIP_OK(c, hipMemcpy(&t, c->rows[(size_t)row].tok, 4, hipMemcpyDeviceToHost));
+  int rc = copy_to_host(c, &t, c->rows[(size_t)row].tok, 4);
+  if (rc) return rc;
   if (out_id) *out_id = t;
   if (row == 0) c->last_sampled0 = t;
   c->row_tok[(size_t)row] = 1;
@@ -1195,9 +1230,7 @@ int tgx_read_probs(tgx_ctx* c, float* out) {
     else HIP_OK(c, hipMemsetAsync(c->rows[(size_t)b].probs, 0, V * 4, c->stream));
   }
   HIP_OK(c, hipGetLastError());
-  HIP_OK(c, hipStreamSynchronize(c->stream));
-  for (int b = 0; b < c->batch; b++) HIP_OK(c, hipMemcpy(out + b * V, c->rows[(size_t)b].probs, V * 4, hipMemcpyDeviceToHost));
-  return TGX_OK;
+  return copy_to_host(c, out, c->slab_probs, (size_t)c->batch * V * 4);
 }
 
 int tgx_set_logits(tgx_ctx* c, const float* logits, int batch) {

@@ -120,6 +120,9 @@ struct tgx_ctx {
   int log_cap = 0;
   int* host_ring = nullptr;  // pinned host ring [HOST_RING][rows]
   int* host_ring_dev = nullptr;
+  // pinned halves that results pass through on their way to the caller's memory (copy_to_host; allocated by its first call)
+  char* stage = nullptr;
+  hipEvent_t stage_ev[2] = {};
   int64_t steps_issued = 0;
   hipEvent_t ticket_ev[MAX_TICKET_EVENTS] = {};
   int32_t last_sampled0 = -1;
@@ -298,6 +301,7 @@ namespace tgx { struct AttnArgs; struct FinalizeArgs; struct AttnPrefillArgs; st
 
 // ---- abi.hip
 void drop_step_graphs(tgx_ctx* c);
+int copy_to_host(tgx_ctx* c, void* dst, const void* src, size_t bytes);      // device memory to any host memory behind what the stream holds; there when it returns
 int kv_ensure_blocks(tgx_ctx* c, int row, long long tokens);       // paged KV: row `row` may hold `tokens` tokens after this (assigns blocks, updates the device table, stream-ordered)
 bool is_greedy(const tgx_sampler_cfg* s);   // Sampler.cpp:15-21
 // ---- decode.hip (kernels/gemv.h, kernels/oproj_sliced.h)

@@ -3040,11 +3040,11 @@ int stack_step(tgx_ctx* c, int S, const int32_t* rows, const int32_t* counts, co
   if (n_want > 0) {
     run_logits(c, dp.want, n_want, sm->lg, nullptr);
     if (slots) { launch_slot_logits(c, sm->lg, dp.want_row, n_want); c->have_logits = true; }
-    HIP_OK(c, hipMemcpyAsync(out_logits, sm->lg, (size_t)n_want * d.vocab * 4, hipMemcpyDeviceToHost, c->stream));
   }
   HIP_OK(c, hipGetLastError());
   if (c->launch_fault) return half_way(c, TGX_OK);
-  HIP_OK(c, hipStreamSynchronize(c->stream));
+  if (n_want == 0) HIP_OK(c, hipStreamSynchronize(c->stream));
+  else if ((rc = copy_to_host(c, out_logits, sm->lg, (size_t)n_want * d.vocab * 4))) return rc;
   for (int e = 0; e < S; e++) {
     const int r = rows[e];
     c->row_past[(size_t)r] += counts[e];
