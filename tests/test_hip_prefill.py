@@ -225,3 +225,20 @@ def test_down_on_wide_tiles_matches_the_square_tiles(name, S, dtype):
     np.testing.assert_array_equal(outs[1][0], outs[2][0])
 
 
+
+
+# query blocks of 64 (workgroups below a chip): the last block of one, 63 and 64 rows, keys that end at and beside a pair of tiles; gate_up whole below a chip of tiles; more than
+# four slabs for the N = hidden products.  Bound: the two schedules differ by roundings of the cached keys and values, as above
+@pytest.mark.parametrize("name", ["qwen3-0.6b", "qwen2.5-0.5b"])
+@pytest.mark.parametrize("S,dtype", [(129, "bf16"), (191, "bf16"), (192, "fp16"), (193, "bf16"), (255, "fp16"), (385, "bf16"), (511, "fp16")])
+def test_short_prompt_blocks_equal_steps(name, S, dtype):
+    d = copy.deepcopy(known_desc(name, dtype))
+    d.layers, d.vocab, d.max_ctx = 2, 4096, 640
+    gpu = Model(d, product_backend()).load_synthetic(17, 0.02).finalize()
+    prompt = synth.synth_prompt(d.vocab, S, 3)[None, :]
+    l1, _, _, kv1 = run(gpu, prompt, mfma=True)
+    l0, _, _, kv0 = run(gpu, prompt, mfma=False)
+    assert rel_err(l1, l0) < 1e-3
+    ulp = {"bf16": 8e-3, "fp16": 1e-3}[dtype]
+    for (k1, v1), (k0, v0) in zip(kv1, kv0):
+        assert rel_err(k1, k0) < ulp and rel_err(v1, v0) < ulp

@@ -527,21 +527,24 @@ struct AttnPrefillArgs {
 // the query sub-blocks of waves 0-3 on the ODD tiles, 0-3 take the even ones; two tiles are staged per barrier pair; the two online-softmax streams of a
 // query meet once, through LDS, after the loop ((m, l, O) merged as flash-decoding does).  One workgroup per CU instead of two, the same matrix work per CU and
 // cycle, half the chain; blocks are dispatched heaviest first (AttnPrefillArgs.heavy_first) so that the second round fills the CUs as they free up.
+// QW = waves of queries (32 each).  A short prompt's blocks of 128 queries leave most of the chip idle (509 tokens, sixteen heads: 64 workgroups, two waves a SIMD walking four
+// pairs of tiles); blocks of 64 are twice as many workgroups of four waves.
 // PAGED (round 6): the workgroup copies the part of the sequence's block table it needs (<= 1024 entries) into LDS first; a K / V row's address then takes one LDS
 // read (it does not touch the counted vmcnt waits of the tile pipeline) — a 64-key tile never straddles a 128-token page.
-template <int DT, int HD, int LA = 2, int KP = 1, bool PAGED = false>
-__global__ __launch_bounds__(256 * KP, KP == 2 ? 2 : (LA == 1 ? (HD == 64 ? 3 : 2) : 1)) void attn_prefill_kernel(const AttnPrefillArgs a) {      // head_dim 128: LA = 1 fits two waves per SIMD (LA = 2 needs 292 registers: one)
+template <int DT, int HD, int LA = 2, int KP = 1, bool PAGED = false, int QW = 4>
+__global__ __launch_bounds__(64 * QW * KP, QW < 4 ? 1 : KP == 2 ? 2 : (LA == 1 ? (HD == 64 ? 3 : 2) : 1)) void attn_prefill_kernel(const AttnPrefillArgs a) {      // head_dim 128: LA = 1 fits two waves per SIMD (LA = 2 needs 292 registers: one)
   constexpr int DIS = TGX_ATTN_DIS;
   constexpr int LQ = HD + 8;                  // 16-bit row stride of the K tile (144 / 272 B: conflict-free 16-byte fragment reads)
   constexpr int LV = HD + 32;                 // 16-bit row stride of the V tile ([key][d], 64 B more than a row: the four key rows of a transposing read fall on four bank quarters)
   constexpr int KS = HD / 16;                 // MFMA k-steps over the head dimension
   constexpr int NB = HD / 32;                 // 32-row output-dim blocks
   constexpr int CH = HD / 8;                  // 16-byte chunks per head row
-  constexpr int NCH = 64 * CH / 256;          // chunks per thread and tile
+  constexpr int GT = 64 * QW;                 // threads that stage and multiply one tile
+  constexpr int NCH = 64 * CH / GT;           // chunks per thread and tile
   constexpr float LOG2E = 1.4426950408889634f;
   constexpr int REG = 64 * LQ + 64 * LV;      // one K tile | V tile pair, 16-bit elements
   extern __shared__ __attribute__((aligned(16))) bf16_t smem[];     // KP x (K tile | V tile); the output rows (and the KP = 2 merge) pass through it at the end
-  const int tid = threadIdx.x, lane = tid & 63, wv = (tid >> 6) & 3, kp = tid >> 8, hh = lane >> 5, ql = lane & 31;      // kp: this wave's tile parity (0 when KP == 1)
+  const int tid = threadIdx.x, lane = tid & 63, wv = (tid >> 6) & (QW - 1), kp = tid / GT, hh = lane >> 5, ql = lane & 31;      // kp: this wave's tile parity (0 when KP == 1)
   bf16_t* const sK = smem + kp * REG;          // the tile this wave multiplies — and the one its thread group stages
   bf16_t* const sV = sK + 64 * LQ;
 
@@ -551,7 +554,7 @@ __global__ __launch_bounds__(256 * KP, KP == 2 ? 2 : (LA == 1 ? (HD == 64 ? 3 : 
   // the grid (which tend to share a CU) carry complementary amounts.  heavy_first: every head's last block first (linear workgroup order = dispatch order)
   const int qblk = a.heavy_first ? (int)gridDim.y - 1 - (int)blockIdx.y
                                  : ((a.qblk_mirror && h >= a.heads / 2) ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x);
-  const int q0 = qblk * 128 + wv * 32;                 // first query of this wave
+  const int q0 = qblk * 32 * QW + wv * 32;                 // first query of this wave
   const int qi = q0 + ql;                              // this lane's query
   const bool qvalid = qi < a.S;
   const int qpos = a.past + qi;
@@ -577,10 +580,10 @@ __global__ __launch_bounds__(256 * KP, KP == 2 ? 2 : (LA == 1 ? (HD == 64 ? 3 : 
 
   const bf16_t* kbase = a.k_cache + (PAGED ? (size_t)0 : (size_t)kvh * a.max_ctx * HD);
   const bf16_t* vbase = a.v_cache + (PAGED ? (size_t)0 : (size_t)kvh * a.max_ctx * HD);
-  const int wg_last_pos = a.past + min(qblk * 128 + 127, a.S - 1);   // keys beyond it are never attended by this workgroup
+  const int wg_last_pos = a.past + min(qblk * 32 * QW + 32 * QW - 1, a.S - 1);   // keys beyond it are never attended by this workgroup
   __shared__ int stbl[PAGED ? 1024 : 1];
   if constexpr (PAGED) {
-    for (int i = tid; i <= (wg_last_pos >> KV_BLOCK_SHIFT); i += 256 * KP) stbl[i] = a.blk_tbl[i];
+    for (int i = tid; i <= (wg_last_pos >> KV_BLOCK_SHIFT); i += GT * KP) stbl[i] = a.blk_tbl[i];
     __syncthreads();
   }
   auto key_off = [&](int key) -> size_t {      // element offset of a key's row from kbase / vbase
@@ -600,7 +603,7 @@ __global__ __launch_bounds__(256 * KP, KP == 2 ? 2 : (LA == 1 ? (HD == 64 ? 3 : 
   auto fetch_tile = [&](int kt, u32x4* kr, u32x4* vr) {
 #pragma unroll
     for (int i = 0; i < NCH; i++) {
-      const int c = (tid & 255) + 256 * i, row = c / CH, kc = c - row * CH;
+      const int c = (tid & (GT - 1)) + GT * i, row = c / CH, kc = c - row * CH;
       const int key = min((KP * kt + kp) * 64 + row, wg_last_pos);
       const size_t ko = key_off(key) + kc * 8;
       kr[i] = *reinterpret_cast<const u32x4*>(kbase + ko);
@@ -612,7 +615,7 @@ __global__ __launch_bounds__(256 * KP, KP == 2 ? 2 : (LA == 1 ? (HD == 64 ? 3 : 
   auto stage_tile = [&](const u32x4* kr, const u32x4* vr) {
 #pragma unroll
     for (int i = 0; i < NCH; i++) {
-      const int c = (tid & 255) + 256 * i, row = c / CH, kc = c - row * CH;
+      const int c = (tid & (GT - 1)) + GT * i, row = c / CH, kc = c - row * CH;
       const u32x4 kv = kr[i], vv = vr[i];
       *reinterpret_cast<u32x4*>(&sK[row * LQ + kc * 8]) = kv;
       *reinterpret_cast<u32x4*>(&sV[row * LV + kc * 8]) = vv;       // V stays [key][d]: the PV step reads it with the transposing LDS read
@@ -758,7 +761,7 @@ __global__ __launch_bounds__(256 * KP, KP == 2 ? 2 : (LA == 1 ? (HD == 64 ? 3 : 
   if constexpr (KP == 2) {
     // the odd-tile stream of every query joins the even-tile one: lane-to-lane (the two waves hold the same queries in the same layout)
     constexpr int NV = NB * 16 + 2;
-    static_assert(4 * NV * 64 * 4 <= KP * REG * 2, "the merge buffer exceeds the K / V tiles");
+    static_assert(QW * NV * 64 * 4 <= KP * REG * 2, "the merge buffer exceeds the K / V tiles");
     float* const mo = reinterpret_cast<float*>(smem) + (size_t)wv * NV * 64 + lane;
     if (kp == 1) {
 #pragma unroll
@@ -784,7 +787,7 @@ __global__ __launch_bounds__(256 * KP, KP == 2 ? 2 : (LA == 1 ? (HD == 64 ? 3 : 
     if (kp == 1) return;
   }
   constexpr int RS = HD + 4;                    // staged row stride in 16-bit elements
-  static_assert(4 * 32 * RS <= 64 * LQ + 64 * LV, "output staging exceeds the K / V tiles");
+  static_assert(QW * 32 * RS <= 64 * LQ + 64 * LV, "output staging exceeds the K / V tiles");
   bf16_t* const wrow = smem + wv * 32 * RS;
   const float inv_l = qvalid ? 1.0f / l_run : 0.f;
   unsigned int whi[NB * 8], wlo[NB * 8];

@@ -103,16 +103,22 @@ static void launch_gemm(tgx_ctx* c, int epi, const ebyte* B_, const ebyte* bias_
   const bool qkv_bal = (c->gemm_dma & 3) && three_terms && epi == tgx::GEMM_STORE && three_from > 0 && three_from % tgx::GBN == 0 && N > three_from && K % 64 == 0 && M >= 128;
   const int qkv_wgs = qkv_bal ? (three_from / tgx::GBN) * ((M + 127) / 128) + ((N - three_from + tgx::GBN - 1) / tgx::GBN) * ((M + 63) / 64) : 0;
   const bool qkv_nosplit = qkv_bal && c->qkv_nosplit && qkv_wgs >= c->num_cus;
-  if (c->gemm_splitk && ntiles < c->num_cus && K % tgx::GBK == 0 && !qkv_nosplit) nsplit = std::min(std::min(16, ktiles), (2 * c->num_cus + ntiles - 1) / ntiles);
+  // (the gate_up product of prompts below a chip of 128 x 128 tiles keeps them whole, on the eight-wave kernel, from a quarter of a chip on: no slabs, no reduce launch.  Whole / split,
+  //  ms per prompt: Qwen3-0.6B 133 tokens (96 tiles) 2.68 / 2.78, 256 2.98 / 3.21, 509 (192) 3.45 / 3.92; Qwen2.5-0.5B 133 (152) 2.07 / 2.27, 384 (228) 2.49 / 2.99)
+  const bool silu8 = epi == tgx::GEMM_SILU && (c->gemm_dma & 8) && K % 64 == 0 && !three_terms && 4 * ntiles >= c->num_cus;
+  if (c->gemm_splitk && ntiles < c->num_cus && K % tgx::GBK == 0 && !qkv_nosplit && !silu8) nsplit = std::min(std::min(16, ktiles), (2 * c->num_cus + ntiles - 1) / ntiles);
   // N = hidden products of a 129-1500-row prompt (round 4, option prefill.splitk_8k): their 128 x 128 tiles number less than a chip (Llama-3.2-1B S = 1024: 128 tiles on 256
-  // CUs, 84 us per product against 104 at twice the rows) — the eight-wave LDS-DMA kernel over 2-4 K slabs instead of 64-row register-staged slabs or a half-empty chip
+  // CUs, 84 us per product against 104 at twice the rows) — the eight-wave LDS-DMA kernel over 2-8 K slabs instead of 64-row register-staged slabs or a half-empty chip
   bool part_8k = false;
   if (c->gemm_splitk && c->splitk_8k && (c->gemm_dma & 8) && K % 64 == 0 && !three_terms && (epi == tgx::GEMM_RESIDUAL || epi == tgx::GEMM_STORE) && M > 128) {
     const int t128 = ((N + 127) / 128) * ((M + 127) / 128);
-    // slabs z = 2..4 that shorten the critical path: rounds of workgroups x 1 / z of the K loop against one round of whole tiles (160 tiles on 256 CUs: z = 3 -> 2 rounds of a
-    // third = 0.67; 128 tiles: z = 2 -> 0.5); taken from 0.8 down (the slabs cost a pass over z x M x N floats)
+    // slabs z = 2..8 that shorten the critical path: rounds of workgroups x 1 / z of the K loop against one round of whole tiles (160 tiles on 256 CUs: z = 3 -> 2 rounds of a
+    // third = 0.67; 128 tiles: z = 2 -> 0.5); taken from 0.8 down (the slabs cost a pass over z x M x N floats).  More than four where all of them run at once and the steps of K
+    // that they save (0.6 us each) outweigh their floats (written and read at 5 TB/s): eight / four, ms per prompt, Llama-3.2-1B 133 tokens 2.14 / 2.25, 256 2.28 / 2.39,
+    // Qwen2.5-0.5B 256 2.51 / 2.67; with eight in two rounds or for K 2048 at 509 rows and N 1024 it is slower (Qwen3-0.6B 3.53 / 3.45)
     int z = 1; double best = 0.8001;
-    for (int zz = 2; zz <= 4; zz++) {
+    for (int zz = 2; zz <= 8; zz++) {
+      if (zz > 4 && (zz * t128 > c->num_cus || K < 6.8e-4 * zz * M * N)) break;
       const double cost = (double)((zz * t128 + c->num_cus - 1) / c->num_cus) / zz;
       if (t128 < c->num_cus && cost < best - 1e-9 && K / 64 >= 4 * zz) { best = cost; z = zz; }
     }
@@ -227,7 +233,7 @@ static void launch_gemm(tgx_ctx* c, int epi, const ebyte* B_, const ebyte* bias_
     // the wide product of a prompt too short for 256 x 256 tiles (129-384 rows: 128-384 tiles of 128 x 128): the eight-wave kernel with the K step split between
     // wave pairs instead of the four-wave one (option prefill.wide_8k: Llama-3.2-1B S = 256 gate_up 61 us per layer)
     const int t128 = ((N + 127) / 128) * ((M + 127) / 128);
-    if (2 * t128 >= c->num_cus && (2 * t128 <= c->wide_8k_max * c->num_cus || ragged256)) {
+    if ((silu8 || 2 * t128 >= c->num_cus) && (2 * t128 <= c->wide_8k_max * c->num_cus || ragged256)) {
       const dim3 g8((N + 127) / 128, (M + 127) / 128), b8(512);
       const size_t lds8 = (size_t)3 * 3 * 128 * 64 * 2;
       TGX_DT16_SWITCH(c->dt, if (one_k) hipLaunchKernelGGL((tgx::gemm_dma8k_kernel<DT, tgx::GEMM_SILU, false>), g8, b8, lds8, c->stream, g); else hipLaunchKernelGGL((tgx::gemm_dma8k_kernel<DT, tgx::GEMM_SILU>), g8, b8, lds8, c->stream, g);)
@@ -320,12 +326,19 @@ void launch_attn_prefill(tgx_ctx* c, const tgx::AttnPrefillArgs& a_, bool allow_
   const bool ksplit = nqb >= 2 && (c->attn_ksplit == 2 || (c->attn_ksplit == 1 && (hd == 128 || nwg < 3 * c->num_cus)));
   // head_dim 64 with three or more workgroups per CU: the one-tile look-ahead form at three waves per SIMD (prefill.h)
   const bool lean = allow_lean && hd == 64 && nwg >= 3 * c->num_cus;
+  // below a chip of workgroups: blocks of 64 queries, twice as many of half the waves (QW = 2).  ms per prompt, 64 / 128: Qwen3-0.6B 256 tokens 2.72 / 2.82, 509 3.43 / 3.53, 1000
+  // 4.86 / 5.03, 1300 6.05 / 6.15; Llama-3.2-1B fp16 256 2.22 / 2.26, 700 4.53 / 4.57
+  const bool half = ksplit && nwg <= c->num_cus;
   a.heavy_first = ksplit ? 1 : 0;
   const dim3 gridk(a.heads, nqb), blkk(512), grid(nqb, a.heads), blk(256);
   auto go = [&](auto paged) {        // (paged KV: the same forms through the sequence's block table)
     constexpr bool P = decltype(paged)::value;
     TGX_DT16_SWITCH(c->dt,
-      if (ksplit) {
+      if (half) {
+        const dim3 gridh(a.heads, (a.S + 63) / 64);
+        if (hd == 64) hipLaunchKernelGGL((tgx::attn_prefill_kernel<DT, 64, 2, 2, P, 2>), gridh, dim3(256), 2 * lds1, c->stream, a);
+        else hipLaunchKernelGGL((tgx::attn_prefill_kernel<DT, 128, 1, 2, P, 2>), gridh, dim3(256), 2 * lds1, c->stream, a);
+      } else if (ksplit) {
         if (hd == 64) hipLaunchKernelGGL((tgx::attn_prefill_kernel<DT, 64, 2, 2, P>), gridk, blkk, 2 * lds1, c->stream, a);
         else hipLaunchKernelGGL((tgx::attn_prefill_kernel<DT, 128, 1, 2, P>), gridk, blkk, 2 * lds1, c->stream, a);
       } else if (lean) hipLaunchKernelGGL((tgx::attn_prefill_kernel<DT, 64, 1, 1, P>), grid, blk, lds1, c->stream, a);
@@ -454,6 +467,10 @@ int prefill_set_attrs(tgx_ctx* c) {
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma_qkv8_kernel<tgx::DT_F16>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (3 * 128 + 128 + 64) * 64 * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8i_kernel<tgx::DT_BF16, tgx::GEMM_SILU>), hipFuncAttributeMaxDynamicSharedMemorySize, 5 * 256 * 128));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8i_kernel<tgx::DT_F16, tgx::GEMM_SILU>), hipFuncAttributeMaxDynamicSharedMemorySize, 5 * 256 * 128));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_BF16, 128, 1, 2, false, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_BF16, 128, 1, 2, true, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_F16, 128, 1, 2, false, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_F16, 128, 1, 2, true, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_BF16, 128, 1, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_BF16, 128, 1, 2, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_F16, 128, 1, 2, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
