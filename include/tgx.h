@@ -486,7 +486,7 @@ TGX_API int tgx_set_logits(tgx_ctx* ctx, const float* logits, int batch);
  *                  tgx_reset_row / tgx_reset_cache; max_ctx stays the per-row limit.  A call that would need a block when none is free returns TGX_ERR_CONTEXT and
  *                  changes nothing (retire a row, retry).  Results are those of the unpaged cache, bit for bit on the same kernels (tests/test_hip_paged.py);
  *                  tgx_get_option "kv.free_tokens" = the unassigned blocks' worth of tokens (-1 when unpaged)
- *   "attn.split_min", "attn.gqa_split_min", "attn.mfma", "stack.gemv", "stack.line", "stack.gemm_wt", "mlstm.narrow", "attn.mix_groups", "ssd.min"  (layered models) keys a workgroup walks from which a step of few
+ *   "attn.split_min", "attn.gqa_split_min", "attn.mfma", "stack.gemv", "stack.rec_step", "stack.line", "stack.gemm_wt", "mlstm.narrow", "attn.mix_groups", "ssd.min"  (layered models) keys a workgroup walks from which a step of few
  *                  tokens divides them between workgroups (four thresholds: 128 on the matrix cores, 2048 on the lane kernels for latent rows, 1024 for grouped queries, counted in a
  *                  mask's span.  The first key sets all four, the second the grouped-query ones; a negative value brings the defaults back; tgx_get_option gives the
  *                  one in force, the matrix cores' where any layer's attention runs there);

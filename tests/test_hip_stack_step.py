@@ -1,0 +1,72 @@
+"""Single tokens through a mixer's one launch (kernels/stack_step.h): recurrences whose heads fill, exceed and fall short of the columns and row groups of a workgroup,
+convolutions of one tap to the most that the kernel takes and one more, attention over one key up to the most that it takes and past that, masks, caps, slopes, rotations and
+groups of one to four query heads.  fp32 storage against the plain oracles of the designs: fp32 sums over at most 256 channels and keys, 1e-4 of the largest logit as in the
+designs' own tests; and against the same steps in the launches that it stands for, whose sums meet in another order (1e-5: a thousand roundings of 2^-24)."""
+import numpy as np
+import pytest
+
+import test_hip_keronex as tk
+import test_hip_vitudra as tv
+
+pytestmark = pytest.mark.gpu
+
+
+def stepped(t, cfg, n, seed, first=2, **kw):
+    """three sequences: a portion of `first` tokens each, then single tokens of all of them; the last logits by the step kernels and by the launches of their own, and the oracle's"""
+    out, toks = [], [t.tokens(cfg, n, seed + i) for i in range(3)]
+    for on in (1, 0):
+        eng, w = t.engine(cfg, seed=seed, **kw)
+        eng.model.set_option("stack.rec_step", on)
+        got = [eng.step([(i, s[:first], [first - 1]) for i, s in enumerate(toks)])]
+        got += [eng.step([(i, s[j:j + 1], [0]) for i, s in enumerate(toks)]) for j in range(first, n)]
+        eng.close()
+        out.append(np.stack(got, 1))
+    assert np.abs(out[0] - out[1]).max() / np.abs(out[1]).max() < 1e-5
+    for i, s in enumerate(toks):
+        want = t.want_of(cfg, w, s)
+        assert np.abs(out[0][i] - want[first - 1:n]).max() / np.abs(want).max() < 1e-4, i
+
+
+@pytest.mark.parametrize("dim,vdim", [(4, 1), (6, 5), (8, 32), (36, 33), (64, 64), (128, 128), (132, 130), (256, 128), (40, 256), (24, 260)])
+def test_delta_rule(dim, vdim):
+    cfg = tv.config([tv.par(right=dict(dim=dim, vdim=vdim, heads=4, kv_heads=2)), tv.par(tv.ff(16), right=dict(dim=dim, vdim=vdim, heads=2, kv_heads=2, conv=2))], width=24)
+    stepped(tv, cfg, 7, dim)
+
+
+@pytest.mark.parametrize("taps", [1, 2, 3, 5, 8, 9])
+@pytest.mark.parametrize("first", [1, 2, 9])
+def test_convolution_tails(taps, first):
+    cfg = tv.config([tv.par(right=dict(conv=taps)), tv.par(right=dict(conv=taps))], width=24)
+    stepped(tv, cfg, first + 11, taps, first)
+
+
+@pytest.mark.parametrize("dim,rank", [(4, 5), (6, 16), (33, 17), (64, 64), (128, 1), (160, 40), (256, 64)])
+def test_wkv_with_its_decays(dim, rank):
+    cfg = tv.config([tv.wkv(heads=2, dim=dim), tv.wkv(tv.ff(16), heads=3, dim=dim)], width=24)
+    stepped(tv, cfg, 7, dim, decay_rank=rank)
+
+
+@pytest.mark.parametrize("dim,vdim,rot", [(8, 12, 6), (64, 64, 64), (128, 256, 128), (10, 3, 2), (20, 130, None)])
+def test_retention(dim, vdim, rot):
+    cfg = tk.config([tk.ret(dim=dim, vdim=vdim, rot={"base": 10000.0, "dims": rot} if rot else None), tk.ret(dim=dim, vdim=vdim)], width=24)
+    stepped(tk, cfg, 7, dim)
+
+
+@pytest.mark.parametrize("dim,vdim", [(8, 6), (64, 32), (128, 128), (100, 65), (4, 200)])
+def test_channel_decays(dim, vdim):
+    cfg = tk.config([tk.cd(dim=dim, vdim=vdim), tk.cd(tk.dense(16), dim=dim, vdim=vdim, conv=1)], width=24)
+    stepped(tk, cfg, 7, dim)
+
+
+@pytest.mark.parametrize("n", [1, 2, 62, 63, 64, 127, 128, 255, 256, 257])
+@pytest.mark.parametrize("shape", [dict(heads=4, kv_heads=1, dim=8, vdim=6), dict(heads=2, kv_heads=2, dim=64, vdim=64), dict(heads=3, kv_heads=1, dim=136, vdim=128), dict(heads=8, kv_heads=2, dim=256, vdim=100)])
+def test_attention_of_so_many_keys(n, shape):
+    layers = [tv.attn(mask=None, **shape), tv.attn(tv.ff(16), kv_from=0, mask=None, **shape), tv.par(tv.ff(16), left=dict(shape, mask=None, softcap=3.0, rot={"base": 300.0, "dims": 8}))]
+    cfg = tv.config(layers, width=24)
+    stepped(tv, cfg, n + 2, n, max(1, n - 1))
+
+
+@pytest.mark.parametrize("mask", [{"size": 1}, {"size": 64}, {"size": 200}, {"size": 256}, {"size": 300}])
+def test_attention_behind_masks(mask):
+    cfg = tv.config([tv.attn(mask=mask), tv.par(tv.ff(16), left=dict(mask=mask))], width=24)
+    stepped(tv, cfg, 330, mask["size"], 326)

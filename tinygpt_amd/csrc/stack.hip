@@ -16,6 +16,7 @@
 #include "kernels/stack_seq.h"
 #include "kernels/stack_gqa_mfma.h"
 #include "kernels/stack_rec.h"
+#include "kernels/stack_step.h"
 #include "kernels/stack_loop.h"
 #include "kernels/stack_mix_mfma.h"
 #include "kernels/stack_ssm.h"
@@ -504,9 +505,33 @@ struct GqaSpec {
   float lambda = 0.f, diff_eps = 0.f, diff_scale = 0.f;        // normed difference (map_difference_kernel) and map_out their own outputs on the way there
   float* map_out = nullptr;
 };
+tgx::GqaAppendArgs append_args(const StackModel* sm, const GqaSpec& sp) {
+  tgx::GqaAppendArgs ap{};
+  ap.proj = sp.proj; ap.ldp = sp.ldp; ap.heads = sp.heads; ap.kv_heads = sp.kv_heads; ap.maps = sp.maps; ap.dim = sp.dim; ap.vdim = sp.vdim; ap.rot_dims = sp.cs ? sp.rot_dims : 0;
+  ap.rot_pairs = sp.rot_pairs; ap.cs = sp.cs; ap.poolK = sp.append ? sp.poolK : nullptr; ap.poolV = sp.poolV; ap.poolVT = sp.poolVT; ap.vfirst = sm->vfirst; ap.vmode = sp.vmode; ap.lam = sp.lam;
+  ap.q_temp_coef = sp.q_temp_every > 0 ? sp.q_temp_coef : 0.f; ap.q_temp_every = sp.q_temp_every;
+  return ap;
+}
+// whether single tokens over few keys take the one-launch form (kernels/stack_step.h; the options that choose another form by hand keep theirs), and its arguments
+bool gqa_step(const StackModel* sm, const GqaSpec& sp, int max_keys, int max_count, tgx::GqaStepArgs& a) {
+  const int span = sp.mask_kind == tgx::MASK_CAUSAL ? max_keys : std::min(max_keys, sp.mask_size);
+  if (max_count != 1 || !sm->rec_step || !sm->attn_mfma || sm->gqa_split_min_keys != StackModel::MFMA_SPLIT_MIN || span > tgx::STEP_MAX_KEYS) return false;
+  if (sp.maps != 1 || sp.v_is_k || sp.sinks || sp.dist || sp.dim % 8 || sp.dim > tgx::STEP_MAX_DIM || sp.vdim > tgx::STEP_MAX_VDIM || sp.heads > tgx::STEP_MAX_GROUP * sp.kv_heads) return false;
+  a.ap = append_args(sm, sp);
+  a.gate = sp.gate; a.ldg = sp.ldg; a.gate_per_head = sp.gate_per_head; a.out = sp.out; a.ldo = sp.ldo; a.out_scale = sp.out_scale;
+  a.scale = sp.scale; a.sink = sp.sink; a.has_sink = sp.has_sink; a.mask_kind = sp.mask_kind; a.mask_size = sp.mask_size; a.softcap = sp.softcap; a.dist_bias = sp.dist_bias;
+  a.poolK = sp.poolK; a.poolV = sp.poolV;
+  return true;
+}
+
 int run_gqa_core(tgx_ctx* c, const tgx::StepMeta& m, const GqaSpec& sp_, int T, int S, int max_keys, int max_count) {
   StackModel* sm = c->stack;
   GqaSpec sp = sp_;
+  tgx::GqaStepArgs sa{};
+  if (gqa_step(sm, sp, max_keys, max_count, sa)) {
+    TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::gqa_step_kernel<DT>, dim3(S, sp.kv_heads), dim3(1024), 0, c->stream, m, sa))
+    return TGX_OK;
+  }
   if (sp.maps == 2) { sp.out = sp_.map_out; sp.ldo = (long long)sp.heads * sp.vdim; }
   auto merge = [&](const tgx::GqaAttnArgs& mg) {      // the records of a divided attention
     if (sp.maps != 2) { hipLaunchKernelGGL(tgx::gqa_attn_merge_kernel, dim3(T, sp.heads), dim3(256), 0, c->stream, mg); return; }
@@ -521,10 +546,7 @@ int run_gqa_core(tgx_ctx* c, const tgx::StepMeta& m, const GqaSpec& sp_, int T, 
     hipLaunchKernelGGL(tgx::map_difference_kernel, dim3((da.pairs + 3) / 4), dim3(256), 0, c->stream, da);
   };
   const int H = sp.heads, G = sp.kv_heads;
-  tgx::GqaAppendArgs ap{};
-  ap.proj = sp.proj; ap.ldp = sp.ldp; ap.heads = H; ap.kv_heads = G; ap.maps = sp.maps; ap.dim = sp.dim; ap.vdim = sp.vdim; ap.rot_dims = sp.cs ? sp.rot_dims : 0; ap.rot_pairs = sp.rot_pairs;
-  ap.cs = sp.cs; ap.poolK = sp.append ? sp.poolK : nullptr; ap.poolV = sp.poolV; ap.poolVT = sp.poolVT; ap.vfirst = sm->vfirst; ap.vmode = sp.vmode; ap.lam = sp.lam;
-  ap.q_temp_coef = sp.q_temp_every > 0 ? sp.q_temp_coef : 0.f; ap.q_temp_every = sp.q_temp_every;
+  const tgx::GqaAppendArgs ap = append_args(sm, sp);
   if (sp.v_is_k) {      // normed queries and keys, the keys' projections as values
     tgx::KeyValueAppendArgs ka{};
     ka.proj = sp.proj; ka.ldp = sp.ldp; ka.heads = H; ka.kv_heads = G; ka.dim = sp.dim; ka.q_norm = sp.q_norm; ka.k_norm = sp.k_norm; ka.eps = sp.qk_eps;
@@ -806,6 +828,37 @@ void launch_rec_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs&
   else go(std::integral_constant<int, tgx::REC_DELTA>{});
 }
 
+// a step of single tokens: the recurrence with what makes its inputs and finishes its outputs in one launch (kernels/stack_step.h), where the head's sizes allow; false: not launched
+struct RecStepPlan { bool ok; int log_cp, dper; };      // columns' power of two, rows per lane
+RecStepPlan rec_step_plan(const tgx_ctx* c, const tgx::RecStepArgs& a, int max_count) {
+  RecStepPlan p{false, 0, 0};
+  if (max_count != 1 || !c->stack->rec_step || a.s.dim > tgx::STEP_MAX_DIM || a.s.vdim > tgx::STEP_MAX_DIM || (a.prep && a.p.taps > tgx::STEP_MAX_TAPS)) return p;
+  while ((1 << p.log_cp) < a.s.vdim) p.log_cp++;
+  const int rg = 1024 >> p.log_cp;
+  p.dper = (a.s.dim + rg - 1) / rg;
+  p.ok = p.dper <= 32;
+  return p;
+}
+bool launch_rec_step(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecStepArgs& a, int kind, int S, int max_count) {
+  const RecStepPlan p = rec_step_plan(c, a, max_count);
+  if (!p.ok) return false;
+  const int log_cp = p.log_cp, dper = p.dper;
+  const dim3 grid(S, a.s.heads);
+  auto go = [&](auto DTc, auto K) {
+    constexpr int DT = decltype(DTc)::value, KIND = decltype(K)::value;
+    if (dper <= 4) hipLaunchKernelGGL((tgx::rec_step_kernel<DT, KIND, 4>), grid, dim3(1024), 0, c->stream, m, a, log_cp);
+    else if (dper <= 8) hipLaunchKernelGGL((tgx::rec_step_kernel<DT, KIND, 8>), grid, dim3(1024), 0, c->stream, m, a, log_cp);
+    else if (dper <= 16) hipLaunchKernelGGL((tgx::rec_step_kernel<DT, KIND, 16>), grid, dim3(1024), 0, c->stream, m, a, log_cp);
+    else hipLaunchKernelGGL((tgx::rec_step_kernel<DT, KIND, 32>), grid, dim3(1024), 0, c->stream, m, a, log_cp);
+  };
+  const std::integral_constant<int, tgx::DT_F32> any{};      // (only the low-rank decays read stored weights)
+  if (kind == tgx::REC_WKV) TGX_DT_SWITCH(c->dt, (go(std::integral_constant<int, DT>{}, std::integral_constant<int, tgx::REC_WKV>{})))
+  else if (kind == tgx::REC_CDELTA) go(any, std::integral_constant<int, tgx::REC_CDELTA>{});
+  else if (kind == tgx::REC_SSD) go(any, std::integral_constant<int, tgx::REC_SSD>{});
+  else go(any, std::integral_constant<int, tgx::REC_DELTA>{});
+  return true;
+}
+
 int run_joint_attention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer& jl, int T, int S, int max_keys, int max_count) {
   StackModel* sm = c->stack;
   const tgx_layer_desc& ld = w.d;
@@ -825,7 +878,7 @@ int run_joint_attention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, Join
   return TGX_OK;
 }
 
-void run_wkv(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer& jl, int T, int S) {
+void run_wkv(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer& jl, int T, int S, int max_count) {
   StackModel* sm = c->stack;
   const tgx_layer_desc& ld = w.d;
   const int W = sm->d.width, H = ld.heads, HD = H * ld.dim, R = ld.decay_rank;
@@ -840,17 +893,21 @@ void run_wkv(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer& jl,
   g = tgx::StackGemmArgs{};
   g.A = sm->mixed + 4 * (size_t)W; g.lda = 5LL * W; g.B = w.w_w1; g.ldb = W; g.C = sm->lora; g.ldc = R; g.M = T; g.N = R; g.K = W; g.scale = 1.f; g.act = tgx::SG_ACT_TANH;
   jl.first(c, rkvg, 4, &g);
-  g = tgx::StackGemmArgs{};
-  g.A = sm->lora; g.lda = R; g.B = w.w_w2; g.ldb = R; g.C = sm->proj + 4 * (size_t)HD; g.ldc = 5LL * HD; g.M = T; g.N = HD; g.K = R; g.scale = 1.f; g.bias = w.w0; g.act = tgx::SG_ACT_DECAY;
-  launch_gemm(c, g, tgx::SG_STORE, 1);
   tgx::RecScanArgs ra{};
   ra.a = sm->proj; ra.lda = 5LL * HD; ra.k = sm->proj + HD; ra.ldk = 5LL * HD; ra.v = sm->proj + 2 * (size_t)HD; ra.ldv = 5LL * HD; ra.w = sm->proj + 4 * (size_t)HD; ra.ldw = 5LL * HD;
   ra.u = w.ubonus; ra.S = w.mS; ra.out = sm->hs; ra.ldo = HD; ra.heads = H; ra.kv_heads = H; ra.dim = ld.dim; ra.vdim = ld.dim;
-  launch_rec_scan(c, m, ra, tgx::REC_WKV, S);
   tgx::HeadNormGateArgs oa{};
   oa.hs = sm->hs; oa.ldh = HD; oa.w = w.head_w; oa.w_hstride = ld.dim; oa.gate = sm->proj + 3 * (size_t)HD; oa.ldg = 5LL * HD; oa.silu_gate = 1; oa.out = sm->o; oa.ldo = HD; oa.vdim = ld.dim;
   oa.eps = sm->d.norm_eps;
-  hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, H), dim3(64), 0, c->stream, oa);
+  tgx::RecStepArgs st{};
+  st.s = ra; st.g = oa; st.w2 = w.w_w2; st.lora = sm->lora; st.ldlora = R; st.w0 = w.w0; st.rank = R; st.terms = c->act16 ? 1 : 2;
+  if (!launch_rec_step(c, m, st, tgx::REC_WKV, S, max_count)) {
+    g = tgx::StackGemmArgs{};
+    g.A = sm->lora; g.lda = R; g.B = w.w_w2; g.ldb = R; g.C = sm->proj + 4 * (size_t)HD; g.ldc = 5LL * HD; g.M = T; g.N = HD; g.K = R; g.scale = 1.f; g.bias = w.w0; g.act = tgx::SG_ACT_DECAY;
+    launch_gemm(c, g, tgx::SG_STORE, 1);
+    launch_rec_scan(c, m, ra, tgx::REC_WKV, S);
+    hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, H), dim3(64), 0, c->stream, oa);
+  }
   jl.add(c, to_stream(c, sm->o, HD, w.w_o, T, sm->d.residual_mult));
 }
 
@@ -868,9 +925,6 @@ int run_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer&
   sp.cs = w.rot >= 0 ? sm->rot[(size_t)w.rot].cs : nullptr; sp.poolK = w.pool; sp.poolV = w.poolV; sp.poolVT = w.poolVT; sp.append = true;
   sp.scale = ld.scale; sp.mask_kind = ld.mask_kind; sp.mask_size = ld.mask_size; sp.softcap = ld.softcap; sp.dist_bias = ld.dist_bias;
   sp.q_temp_coef = ld.q_temp_coef; sp.q_temp_every = ld.q_temp_every; sp.out = sm->o; sp.ldo = lvd;
-  int rc = run_gqa_core(c, m, sp, T, S, max_keys, max_count);
-  if (rc) return rc;
-  jl.add(c, to_stream(c, sm->o, lvd, w.w_o, T, sm->d.residual_mult * ld.left_scale));
   // (the left half's outputs stay until the layer's sum)
   float* ro = sm->o + (jl.merged ? GEMV_ROWS_MAX * (size_t)sm->max_hv : 0);
   // the right half: rec_in row = [q | k | v | beta | decay]
@@ -879,15 +933,34 @@ int run_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer&
   dp.proj = sm->proj; dp.ldp = nin; dp.col0 = lq + lkv; dp.b_col = rC; dp.cw = w.conv_w; dp.a_log = w.a_log; dp.dt_bias = w.dt_bias; dp.out = sm->rec_in; dp.ldo = ldr;
   dp.state = nb > 0 ? w.conv_state : nullptr; dp.state_buf = (size_t)sm->d.max_seqs * nb * rC; dp.heads = rH; dp.kv_heads = rG; dp.dim = ld.d_dim; dp.vdim = ld.d_vdim; dp.taps = ld.conv_taps;
   dp.q_scale = 1.0f / sqrtf((float)ld.d_dim); dp.unit_eps = 1e-6f;
-  hipLaunchKernelGGL(tgx::delta_prep_kernel, dim3(T, 2 * rG + rH + 1), dim3(256), 0, c->stream, m, dp);
   tgx::RecScanArgs ra{};
   ra.a = sm->rec_in; ra.lda = ldr; ra.k = sm->rec_in + rGD; ra.ldk = ldr; ra.v = sm->rec_in + 2 * (size_t)rGD; ra.ldv = ldr;
   ra.beta = sm->rec_in + rC; ra.g = sm->rec_in + rC + rH; ra.ldg = ldr; ra.S = w.mS; ra.out = sm->hs; ra.ldo = rvd; ra.heads = rH; ra.kv_heads = rG; ra.dim = ld.d_dim; ra.vdim = ld.d_vdim;
-  launch_rec_scan(c, m, ra, tgx::REC_DELTA, S);
   tgx::HeadNormGateArgs oa{};
   oa.hs = sm->hs; oa.ldh = rvd; oa.w = w.head_w; oa.w_hstride = 0; oa.gate = sm->proj + lq + lkv + rC + 2 * rH; oa.ldg = nin; oa.silu_gate = 1; oa.out = ro; oa.ldo = rvd; oa.vdim = ld.d_vdim;
   oa.eps = sm->d.norm_eps;
-  hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, rH), dim3(64), 0, c->stream, oa);
+  tgx::RecStepArgs st{};
+  st.s = ra; st.p = dp; st.prep = 1; st.g = oa;
+  const auto left_out = [&] { jl.add(c, to_stream(c, sm->o, lvd, w.w_o, T, sm->d.residual_mult * ld.left_scale)); };
+  const RecStepPlan sp1 = rec_step_plan(c, st, max_count);
+  tgx::GqaStepArgs sa{};
+  if (jl.merged && sp1.ok && sp1.dper <= 16 && gqa_step(sm, sp, max_keys, max_count, sa)) {      // both halves' outputs stay until the layer's sum: one launch for the two
+    const dim3 grid(S, G + rH);
+    TGX_DT_SWITCH(c->dt,
+      if (sp1.dper <= 4) hipLaunchKernelGGL((tgx::parallel_step_kernel<DT, 4>), grid, dim3(1024), 0, c->stream, m, sa, st, sp1.log_cp);
+      else if (sp1.dper <= 8) hipLaunchKernelGGL((tgx::parallel_step_kernel<DT, 8>), grid, dim3(1024), 0, c->stream, m, sa, st, sp1.log_cp);
+      else hipLaunchKernelGGL((tgx::parallel_step_kernel<DT, 16>), grid, dim3(1024), 0, c->stream, m, sa, st, sp1.log_cp);)
+    left_out();
+  } else {
+    int rc = run_gqa_core(c, m, sp, T, S, max_keys, max_count);
+    if (rc) return rc;
+    left_out();      // (unmerged layers' outputs are added here, before the right half takes their place)
+    if (!launch_rec_step(c, m, st, tgx::REC_DELTA, S, max_count)) {
+      hipLaunchKernelGGL(tgx::delta_prep_kernel, dim3(T, 2 * rG + rH + 1), dim3(256), 0, c->stream, m, dp);
+      launch_rec_scan(c, m, ra, tgx::REC_DELTA, S);
+      hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, rH), dim3(64), 0, c->stream, oa);
+    }
+  }
   jl.add(c, to_stream(c, ro, rvd, w.w_o2, T, sm->d.residual_mult * ld.right_scale));
   return TGX_OK;
 }
@@ -913,7 +986,7 @@ int run_layers_joint(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys,
       for (int k : outs) jl.merged = jl.merged && k % 8 == 0;
     }
     if (ld.mixer == TGX_MIXER_ATTENTION) rc = run_joint_attention(c, m, w, jl, T, S, max_keys, max_count);
-    else if (ld.mixer == TGX_MIXER_WKV) run_wkv(c, m, w, jl, T, S);
+    else if (ld.mixer == TGX_MIXER_WKV) run_wkv(c, m, w, jl, T, S, max_count);
     else rc = run_parallel(c, m, w, jl, T, S, max_keys, max_count);
     if (rc) return rc;
     if (ld.mlp == TGX_MLP_DENSE) {
@@ -1690,25 +1763,27 @@ int run_retention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int
   tgx::StackGemmArgs g{};
   g.A = sm->a; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = ldp; g.M = T; g.N = nin; g.K = W; g.scale = 1.f;
   launch_gemm(c, g, tgx::SG_STORE, 1);
-  if (w.rot >= 0) {      // q and k turn in place (2 H heads side by side)
-    tgx::GqaAppendArgs ap{};
-    ap.proj = sm->proj + vd; ap.ldp = ldp; ap.heads = 2 * H; ap.dim = ld.dim; ap.rot_dims = ld.rot_dims; ap.cs = sm->rot[(size_t)w.rot].cs;
-    TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::gqa_append_kernel<DT>, dim3(T), dim3(256), 0, c->stream, m, ap))
-  }
   const float kscale = 1.0f / sqrtf((float)ld.dim);      // the keys' factor, applied to k v^T
-  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && ensure_part(c, ssd_gram_elems(T, S, H), ssd_gram_elems(sm->cap_tokens, sm->d.max_seqs, H))) {
-    tgx::SsdArgs da{};
-    da.row = sm->proj; da.ld = ldp; da.b0 = vd; da.c0 = vd + qd; da.heads = H; da.groups = H; da.N = ld.dim; da.E = ld.vdim; da.gram = sm->part; da.fixed = w.decays; da.dt0 = kscale; da.S = w.mS; da.out = sm->hs; da.ldo = vd;
-    launch_ssd_mfma(c, m, da, S, max_count);
-  } else {
-    tgx::RecScanArgs ra{};
-    ra.a = sm->proj + vd + qd; ra.lda = ldp; ra.k = sm->proj + vd; ra.ldk = ldp; ra.v = sm->proj; ra.ldv = ldp; ra.fixed = w.decays; ra.beta0 = kscale; ra.S = w.mS; ra.out = sm->hs; ra.ldo = vd;
-    ra.heads = H; ra.kv_heads = H; ra.dim = ld.dim; ra.vdim = ld.vdim;
-    launch_rec_scan(c, m, ra, tgx::REC_SSD, S);
-  }
+  tgx::RecScanArgs ra{};
+  ra.a = sm->proj + vd + qd; ra.lda = ldp; ra.k = sm->proj + vd; ra.ldk = ldp; ra.v = sm->proj; ra.ldv = ldp; ra.fixed = w.decays; ra.beta0 = kscale; ra.S = w.mS; ra.out = sm->hs; ra.ldo = vd;
+  ra.heads = H; ra.kv_heads = H; ra.dim = ld.dim; ra.vdim = ld.vdim;
   tgx::HeadNormGateArgs oa{};
   oa.hs = sm->hs; oa.ldh = vd; oa.gate = sm->proj + vd + 2 * qd; oa.ldg = ldp; oa.silu_gate = 1; oa.out = sm->o; oa.ldo = vd; oa.vdim = ld.vdim; oa.eps = sm->d.norm_eps;
-  hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, H), dim3(64), 0, c->stream, oa);
+  tgx::RecStepArgs st{};
+  st.s = ra; st.g = oa; st.rot_dims = ld.rot_dims; st.cs = w.rot >= 0 ? sm->rot[(size_t)w.rot].cs : nullptr;
+  if (!launch_rec_step(c, m, st, tgx::REC_SSD, S, max_count)) {
+    if (w.rot >= 0) {      // q and k turn in place (2 H heads side by side)
+      tgx::GqaAppendArgs ap{};
+      ap.proj = sm->proj + vd; ap.ldp = ldp; ap.heads = 2 * H; ap.dim = ld.dim; ap.rot_dims = ld.rot_dims; ap.cs = sm->rot[(size_t)w.rot].cs;
+      TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::gqa_append_kernel<DT>, dim3(T), dim3(256), 0, c->stream, m, ap))
+    }
+    if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && ensure_part(c, ssd_gram_elems(T, S, H), ssd_gram_elems(sm->cap_tokens, sm->d.max_seqs, H))) {
+      tgx::SsdArgs da{};
+      da.row = sm->proj; da.ld = ldp; da.b0 = vd; da.c0 = vd + qd; da.heads = H; da.groups = H; da.N = ld.dim; da.E = ld.vdim; da.gram = sm->part; da.fixed = w.decays; da.dt0 = kscale; da.S = w.mS; da.out = sm->hs; da.ldo = vd;
+      launch_ssd_mfma(c, m, da, S, max_count);
+    } else launch_rec_scan(c, m, ra, tgx::REC_SSD, S);
+    hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, H), dim3(64), 0, c->stream, oa);
+  }
   sublayer_out(c, sm->o, vd, w.w_o, T);
   return TGX_OK;
 }
@@ -1720,7 +1795,7 @@ struct ChannelDeltaCols {
     qk = l.kv_heads * l.dim; HD = l.heads * l.dim; HE = l.heads * l.vdim; C = 2 * qk + HE; a1 = pad4(C); g1 = a1 + pad4(l.decay_rank); b = g1 + pad4(l.gate_rank); n = b + l.heads;
   }
 };
-void run_channel_delta(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int S) {
+void run_channel_delta(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int S, int max_count) {
   StackModel* sm = c->stack;
   const tgx_layer_desc& ld = w.d;
   const ChannelDeltaCols k(ld);
@@ -1741,14 +1816,18 @@ void run_channel_delta(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T
   dp.proj = sm->proj; dp.ldp = ldp; dp.b_col = k.b; dp.cw = w.conv_w; dp.out = sm->rec_in; dp.ldo = ldr; dp.state = nb > 0 ? w.conv_state : nullptr;
   dp.state_buf = (size_t)sm->d.max_seqs * nb * k.C; dp.heads = ld.heads; dp.kv_heads = ld.kv_heads; dp.dim = ld.dim; dp.vdim = ld.vdim; dp.taps = ld.conv_taps;
   dp.q_scale = 1.0f / sqrtf((float)ld.dim); dp.unit_eps = 1e-6f;
-  hipLaunchKernelGGL(tgx::delta_prep_kernel, dim3(T, 2 * ld.kv_heads + ld.heads + 1), dim3(256), 0, c->stream, m, dp);
   tgx::RecScanArgs ra{};
   ra.a = sm->rec_in; ra.lda = ldr; ra.k = sm->rec_in + k.qk; ra.ldk = ldr; ra.v = sm->rec_in + 2 * (size_t)k.qk; ra.ldv = ldr; ra.beta = sm->rec_in + k.C; ra.ldg = ldr;
   ra.w = sm->mixed; ra.ldw = k.HD; ra.S = w.mS; ra.out = sm->hs; ra.ldo = k.HE; ra.heads = ld.heads; ra.kv_heads = ld.kv_heads; ra.dim = ld.dim; ra.vdim = ld.vdim;
-  launch_rec_scan(c, m, ra, tgx::REC_CDELTA, S);
   tgx::HeadNormGateArgs oa{};
   oa.hs = sm->hs; oa.ldh = k.HE; oa.w = w.head_w; oa.w_hstride = 0; oa.gate = sm->lora; oa.ldg = k.HE; oa.out = sm->o; oa.ldo = k.HE; oa.vdim = ld.vdim; oa.eps = sm->d.norm_eps;
-  hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, ld.heads), dim3(64), 0, c->stream, oa);
+  tgx::RecStepArgs st{};
+  st.s = ra; st.p = dp; st.prep = 1; st.g = oa;
+  if (!launch_rec_step(c, m, st, tgx::REC_CDELTA, S, max_count)) {
+    hipLaunchKernelGGL(tgx::delta_prep_kernel, dim3(T, 2 * ld.kv_heads + ld.heads + 1), dim3(256), 0, c->stream, m, dp);
+    launch_rec_scan(c, m, ra, tgx::REC_CDELTA, S);
+    hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, ld.heads), dim3(64), 0, c->stream, oa);
+  }
   sublayer_out(c, sm->o, k.HE, w.w_o, T);
 }
 
@@ -1821,7 +1900,7 @@ int run_layers_hyper(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys,
     int rc = TGX_OK;
     if (ld.mixer == TGX_MIXER_ATTENTION) rc = run_two_map_attention(c, m, w, T, S, max_keys, max_count);
     else if (ld.mixer == TGX_MIXER_RETENTION) rc = run_retention(c, m, w, T, S, max_count);
-    else run_channel_delta(c, m, w, T, S);
+    else run_channel_delta(c, m, w, T, S, max_count);
     if (rc) return rc;
     const bool last = li + 1 == d.layers, ff = ld.mlp != TGX_MLP_NONE;
     const StackLayerW* nx = last ? nullptr : &sm->L[(size_t)li + 1];
