@@ -70,3 +70,19 @@ def test_attention_of_so_many_keys(n, shape):
 def test_attention_behind_masks(mask):
     cfg = tv.config([tv.attn(mask=mask), tv.par(tv.ff(16), left=dict(mask=mask))], width=24)
     stepped(tv, cfg, 330, mask["size"], 326)
+
+
+# ---- sigmoid attention of single tokens over divided keys (kernels/stack_loop.h sigmoid_mix_step_kernel): value slices that divide 256 threads evenly and not, one to four query
+# heads a key / value head, one to three of those, head counts up to sixteen, tiles of 32 keys that end inside; and shapes past its limits
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(4, 2, 8, 8), (3, 3, 16, 24), (8, 2, 128, 128), (16, 4, 64, 40), (4, 1, 120, 256), (6, 3, 24, 104), (17, 17, 8, 8), (5, 1, 8, 8), (2, 1, 12, 8)])
+@pytest.mark.parametrize("n,mask", [(130, None), (163, {"size": 100}), (300, {"size": 257})])
+def test_sigmoid_attention_of_divided_keys(heads, kv, dim, vdim, n, mask):
+    import test_hip_zaluvik as tz
+    kw = dict(heads=heads, kv_heads=kv, dim=dim, vdim=vdim, mask=mask)
+    cfg = tz.config([tz.attn(**kw), tz.attn(tz.dense(), **kw)], width=24)
+    toks = tz.tokens(cfg, n, seed=dim)
+    eng, w = tz.engine(cfg, seed=heads)
+    got = [eng.step([("a", toks[:n - 3], [n - 4])])] + [eng.step([("a", toks[j:j + 1], [0])]) for j in range(n - 3, n)]
+    eng.close()
+    want = tz.want_of(cfg, w, toks)
+    assert np.abs(np.concatenate(got) - want[n - 4:]).max() / np.abs(want).max() < 1e-4

@@ -258,6 +258,125 @@ __global__ __launch_bounds__(256) void sigmoid_mix_attn_kernel(StepMeta m, MixAt
       else a.out[(size_t)t * a.ldo + o] = a.gate ? acc[n][e] / (1.0f + expf(-a.gate[(size_t)t * a.ldg + o])) : acc[n][e];
     }
 }
+// The split form of few tokens, whose workgroups each have a tile or two: bound by the chain of their loads (a key row a thread, four slices of it on their way, then the tile's value
+// rows four at a time: 18.5 us for two tokens over 1024 keys, 64 workgroups).  Here every load of a tile of 32 keys stands at once in whole lines: four keys a wave and turn, sixteen
+// lanes a key row, for the scores; a slice of eight value channels and every KG-th key a thread for the values, whose key groups meet in LDS.  9.0 us for the same (14.2 with runtime divisions in its index arithmetic and a sigmoid per head and lane).
+// Rows of 16-byte slices, dim <= 128, at most 16 heads of at most four a key / value head, at most 256 value slices (mix_step_ok), rows of q at 16 bytes.
+constexpr int MIX_STEP_HEADS = 16, MIX_STEP_GROUP = 4, MIX_STEP_KEYS = 32;
+inline bool mix_step_ok(int heads, int kv_heads, int dim, int vdim) {
+  return dim % 8 == 0 && dim <= 128 && vdim % 8 == 0 && heads <= MIX_STEP_HEADS && heads <= MIX_STEP_GROUP * kv_heads && kv_heads * vdim <= 2048;
+}
+template <int DT>
+__global__ __launch_bounds__(256) void sigmoid_mix_step_kernel(StepMeta m, MixAttnArgs a) {
+  constexpr int KT = MIX_STEP_KEYS, MQ = MIX_STEP_GROUP;
+  __shared__ __attribute__((aligned(16))) float s_q[MIX_STEP_HEADS][128];
+  __shared__ float s_w[MIX_STEP_HEADS][KT + 1], s_w2[MIX_STEP_HEADS][KT + 1], s_t[MIX_STEP_HEADS][MIX_STEP_HEADS], s_acc[MQ * 8][256];
+  const int H = a.heads, G = a.kv_heads, qpg = H / G, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, sub = lane >> 4, ch = 8 * (lane & 15);
+  const int t = blockIdx.x, row = m.tok_row[t], pos = m.tok_pos[t], pmask = (1 << m.page_shift) - 1, kd = G * a.dim, vd = G * a.vdim;
+  int k1 = pos + 1;
+  const int k0 = min(k1, first_key(pos, a.mask_kind, a.mask_size) + (int)blockIdx.y * a.keys_per);
+  k1 = min(k1, k0 + a.keys_per);
+  const int* tbl = m.tbl + (size_t)row * m.tbl_stride;
+  auto slot_of = [&](int key) -> size_t { return ((size_t)tbl[key >> m.page_shift] << m.page_shift) + (size_t)(key & pmask); };
+  const elem_t<DT>* pk = reinterpret_cast<const elem_t<DT>*>(a.poolK);
+  const elem_t<DT>* pv = reinterpret_cast<const elem_t<DT>*>(a.poolV);
+  const int slices = vd >> 3, KG = 256 / slices, kg = tid / slices, sl = tid - kg * slices, vg = sl / (a.vdim >> 3);      // key groups; this thread's group, slice and key / value head
+  for (int h = tid >> 5; h < H; h += 8)
+    for (int c = 4 * (tid & 31); c < a.dim; c += 128) *reinterpret_cast<f32x4*>(&s_q[h][c]) = *reinterpret_cast<const f32x4*>(a.q + (size_t)t * a.ldq + (size_t)h * a.dim + c);
+  if (a.talk && (tid >> 4) < H && (tid & 15) < H) s_t[tid >> 4][tid & 15] = a.talk[(tid >> 4) * H + (tid & 15)];
+  float acc[MQ][8];
+#pragma unroll
+  for (int r = 0; r < MQ; r++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[r][e] = 0.f;
+  for (int kb = k0; kb < k1; kb += KT) {
+    const int last = k1 - 1, nk = min(KT, k1 - kb);
+    Slice8<DT> vr[4];
+    auto values = [&](int i0) {
+#pragma unroll
+      for (int u = 0; u < 4; u++) vr[u] = load_slice<DT>(pv + slot_of(min(kb + i0 + u * KG, last)) * vd + 8 * sl, 0);
+    };
+    if (kg < KG) values(kg);
+    __syncthreads();                         // queries staged; the previous tile's weights have been read
+    for (int g0 = 0; g0 < G; g0 += 2) {
+      Slice8<DT> kr[2][2];
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const elem_t<DT>* kp = pk + slot_of(min(kb + 4 * (wv + 4 * u) + sub, last)) * kd + min(ch, a.dim - 8);
+#pragma unroll
+        for (int x = 0; x < 2; x++) kr[u][x] = load_slice<DT>(kp + min(g0 + x, G - 1) * a.dim, 0);
+      }
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int x = 0; x < 2; x++) {
+          const int g = g0 + x, i = 4 * (wv + 4 * u) + sub;
+          if (g >= G) continue;
+          float k[8], sc[MQ] = {0.f, 0.f, 0.f, 0.f};
+          slice_unpack<DT>(kr[u][x], k);
+          if (ch < a.dim)
+#pragma unroll
+            for (int r = 0; r < MQ; r++) {
+              const float* q = s_q[min(g * qpg + r, H - 1)] + ch;
+              const f32x4 qa = *reinterpret_cast<const f32x4*>(q), qb = *reinterpret_cast<const f32x4*>(q + 4);
+#pragma unroll
+              for (int e = 0; e < 8; e++) sc[r] = fmaf(e < 4 ? qa[e & 3] : qb[e & 3], k[e], sc[r]);
+            }
+          float v = 0.f;                     // lane r of a key's sixteen keeps head r
+#pragma unroll
+          for (int r = 0; r < MQ; r++) { const float z = row_group_sum<16>(sc[r]); v = (lane & 15) == r ? z : v; }
+          const int h = min(g * qpg + (lane & 15), H - 1);
+          v = 1.0f / (1.0f + expf(-fmaf(v, a.scale, a.pb ? a.pb[h] : 0.f)));
+          if ((lane & 15) < qpg) s_w[h][i] = v;
+        }
+    }
+    __syncthreads();
+    if (a.talk) {
+      for (int h = tid / KT; h < H; h += 256 / KT) {
+        const int j = tid % KT;
+        float v = 0.f;
+#pragma unroll 4
+        for (int g = 0; g < H; g++) v = fmaf(s_t[h][g], s_w[g][j], v);
+        s_w2[h][j] = v;
+      }
+      __syncthreads();
+    }
+    auto weight = [&](int h, int j) { return a.talk ? s_w2[h][j] : s_w[h][j]; };
+    if (kg < KG)
+      for (int i0 = kg; i0 < nk; i0 += 4 * KG) {
+        if (i0 != kg) values(i0);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const int i = i0 + u * KG;
+          if (i >= nk) continue;
+          float f[8];
+          slice_unpack<DT>(vr[u], f);
+#pragma unroll
+          for (int r = 0; r < MQ; r++) {
+            const float w = weight(min(vg * qpg + r, H - 1), i);
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc[r][e] = fmaf(w, f[e], acc[r][e]);
+          }
+        }
+      }
+  }
+#pragma unroll
+  for (int r = 0; r < MQ; r++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) s_acc[r * 8 + e][tid] = acc[r][e];
+  __syncthreads();
+  float* part = a.part + ((size_t)t * a.nsplit + blockIdx.y) * H * a.vdim;
+  for (int c = tid; c < vd; c += 256) {      // a channel of a value row, for every head that reads it
+    const int g = c / a.vdim;
+    float v[MQ] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int k = 0; k < KG; k++)
+#pragma unroll
+      for (int r = 0; r < MQ; r++) v[r] += s_acc[r * 8 + (c & 7)][k * slices + (c >> 3)];
+#pragma unroll
+    for (int r = 0; r < MQ; r++) if (r < qpg) part[(size_t)(g * qpg + r) * a.vdim + c - g * a.vdim] = v[r];
+  }
+}
 __global__ __launch_bounds__(256) void sigmoid_mix_merge_kernel(MixAttnArgs a) {
   const size_t t = blockIdx.x;
   const int O = a.heads * a.vdim;

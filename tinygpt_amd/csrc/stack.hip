@@ -1082,7 +1082,8 @@ int run_affine_attention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, con
   if (nsplit > 1 && ensure_part(c, (size_t)T * nsplit * (size_t)vd)) {
     aa.kt = std::min(aa.kt, aa.keys_per);
     aa.part = sm->part; aa.nsplit = nsplit;
-    TGX_DT_SWITCH(c->dt, (launch_mix_attn_t<DT, true>(c, m, aa, dim3(T, nsplit), lds, vec)))
+    if (nin % 4 == 0 && tgx::mix_step_ok(H, G, ld.dim, ld.vdim)) TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::sigmoid_mix_step_kernel<DT>, dim3(T, nsplit), dim3(256), 0, c->stream, m, aa))
+    else TGX_DT_SWITCH(c->dt, (launch_mix_attn_t<DT, true>(c, m, aa, dim3(T, nsplit), lds, vec)))
     hipLaunchKernelGGL(tgx::sigmoid_mix_merge_kernel, dim3(T, std::min(8, (vd + 255) / 256)), dim3(256), 0, c->stream, aa);
   } else {
     TGX_DT_SWITCH(c->dt, (launch_mix_attn_t<DT, false>(c, m, aa, dim3(T), lds, vec)))
