@@ -85,7 +85,7 @@ struct NormConvArgs {
 // before the sums of squares, whose barrier they cross in flight (four taps, 1024 channels: the median launch of four decoded rows 8.0 -> 3.8 us,
 // some 2400 rows 45 -> 15; selecting taps by number bounded it).
 template <int TAPS>
-__global__ __launch_bounds__(256) void norm_conv_kernel(StepMeta m, NormConvArgs a) {
+__device__ __forceinline__ void norm_conv_body(StepMeta m, NormConvArgs a) {
   __shared__ float s_rinv[CONV_MAX_TAPS][NORM_MAX_GROUPS];
   const int t = blockIdx.x, i = m.tok_idx[t], cnt = m.tok_cnt[t], pos = m.tok_pos[t];
   const int row = m.tok_row[t], par = m.tok_par[t];
@@ -207,6 +207,8 @@ __global__ __launch_bounds__(256) void norm_conv_kernel(StepMeta m, NormConvArgs
     for (int c = threadIdx.x; c < a.W; c += 256) outp[(size_t)t * a.W + c] = channel(c, xin[(size_t)t * a.W + c], a.nw[c], a.cw ? a.cw + (size_t)c * taps : nullptr);
   }
 }
+template <int TAPS>
+__global__ __launch_bounds__(256) void norm_conv_kernel(StepMeta m, NormConvArgs a) { norm_conv_body<TAPS>(m, a); }
 
 // ---- latent: c = rms_norm(down-projected row) * w, stored at the token's place in the pool (storage dtype).  One wave per token.
 struct LatentAppendArgs {
@@ -430,7 +432,7 @@ struct RouterArgs {
 };
 constexpr int ROUTER_MAX_E = 1024, ROUTER_MAX_TOP = 64;
 template <bool PRODUCT>
-__global__ __launch_bounds__(PRODUCT ? 256 : 64) void router_topk_kernel(RouterArgs a) {
+__device__ __forceinline__ void router_topk_body(RouterArgs a) {
   __shared__ float s_z[ROUTER_MAX_E];
   __shared__ float s_v[ROUTER_MAX_TOP];
   __shared__ int s_i[ROUTER_MAX_TOP];
@@ -453,6 +455,15 @@ __global__ __launch_bounds__(PRODUCT ? 256 : 64) void router_topk_kernel(RouterA
   float den = 0.f;
   for (int k = 0; k < a.top; k++) den += expf(s_v[k] - mx);
   for (int k = lane; k < a.top; k += 64) { a.sel[(size_t)t * a.top + k] = s_i[k]; a.selw[(size_t)t * a.top + k] = expf(s_v[k] - mx) / den; }
+}
+template <bool PRODUCT>
+__global__ __launch_bounds__(PRODUCT ? 256 : 64) void router_topk_kernel(RouterArgs a) { router_topk_body<PRODUCT>(a); }
+// A few tokens' norm and convolution with the choice of experts behind it, whose products a workgroup takes from the row that it has just written: a launch less (one of 2.6 us at least)
+template <int TAPS>
+__global__ __launch_bounds__(256) void norm_conv_route_kernel(StepMeta m, NormConvArgs a, RouterArgs r) {
+  norm_conv_body<TAPS>(m, a);
+  __syncthreads();
+  router_topk_body<true>(r);
 }
 
 // ---- plan of the grouped expert products: pairs i = t * top + k grouped by expert.  One workgroup.
@@ -499,7 +510,7 @@ struct CombineDepthArgs {
   const float* dw;       // [n_res]
   int W, top, n_res;
 };
-__global__ __launch_bounds__(256) void combine_depth_kernel(CombineDepthArgs a) {
+__device__ __forceinline__ void combine_depth_body(CombineDepthArgs a) {
   const size_t t = blockIdx.x;
   if ((a.W & 3) == 0) {
     for (int c = 4 * threadIdx.x; c < a.W; c += 1024) {
@@ -528,6 +539,14 @@ __global__ __launch_bounds__(256) void combine_depth_kernel(CombineDepthArgs a) 
     for (int j = 0; j < a.n_res - 1; j++) s = fmaf(a.dw[j], a.xs[(size_t)j * a.slot_stride + t * a.W + c], s);
     a.x[t * a.W + c] = fmaf(a.dw[a.n_res - 1], v, s);
   }
+}
+__global__ __launch_bounds__(256) void combine_depth_kernel(CombineDepthArgs a) { combine_depth_body(a); }
+// ... and, in a step of single tokens (whose convolutions read no other row of the step), the next layer's norm and convolution of the row
+template <int TAPS>
+__global__ __launch_bounds__(256) void combine_norm_conv_kernel(StepMeta m, CombineDepthArgs c, NormConvArgs a) {
+  combine_depth_body(c);
+  __syncthreads();
+  norm_conv_body<TAPS>(m, a);
 }
 
 // ---- out[i] = grouped RMS norm of x[rows[i]] * w

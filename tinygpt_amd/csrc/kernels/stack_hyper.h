@@ -74,7 +74,7 @@ struct HyperSeamArgs {
   HyperIn in;
 };
 template <int NS>
-__global__ __launch_bounds__(256) void hyper_seam_kernel(HyperSeamArgs a) {
+__device__ __forceinline__ void hyper_seam_body(HyperSeamArgs a) {
   __shared__ float s4[4];
   const size_t t = blockIdx.x;
   float* __restrict__ xs = a.xs + t * a.n * a.W;
@@ -162,6 +162,14 @@ __global__ __launch_bounds__(256) void hyper_seam_kernel(HyperSeamArgs a) {
   ss = block_sum_256(ss, s4);
   const float r = 1.0f / sqrtf(ss / (float)a.W + a.in.eps);
   for (int c = threadIdx.x; c < a.W; c += 256) out[c] *= r * (1.0f + a.in.w_norm[c]);
+}
+template <int NS>
+__global__ __launch_bounds__(256) void hyper_seam_kernel(HyperSeamArgs a) { hyper_seam_body<NS>(a); }
+template <int NS>
+__global__ __launch_bounds__(256) void hyper_seam_route_kernel(HyperSeamArgs a, RouterGroupArgs r) {      // (as sandwich_route_kernel)
+  hyper_seam_body<NS>(a);
+  __syncthreads();
+  router_group_body<true>(r);
 }
 
 // ---- out[t][h] = d / sqrt(mean(d^2) + eps) * scale, d = o_1 - lambda o_2 of the head's two maps.  One wave per (token, head); vdim <= 64 GQA_MAX_RPL.

@@ -9,7 +9,7 @@
 //   sigmoid_mix_merge_kernel   adds up the partial sums of a window divided between workgroups, applies the output gate
 //   (kernels/stack_mix_mfma.h holds the same attention for portions of prompts on the matrix cores)
 #pragma once
-#include "stack.h"
+#include "stack_seq.h"
 
 namespace tgx {
 
@@ -112,7 +112,7 @@ __device__ __forceinline__ void affine_seam_row(const AffineSeamArgs& a, size_t 
   }
 }
 template <int NR>
-__global__ __launch_bounds__(256) void affine_seam_kernel(AffineSeamArgs a) {
+__device__ __forceinline__ void affine_seam_body(AffineSeamArgs a) {
   __shared__ float s44[4][4];
   const size_t t = blockIdx.x;
   if (a.W <= 1024 * NR) {
@@ -135,6 +135,14 @@ __global__ __launch_bounds__(256) void affine_seam_kernel(AffineSeamArgs a) {
   if (!a.w_next) return;
   row_moments_256(xt, a.W, a.eps, s4, mean, rstd);
   for (int c = threadIdx.x; c < a.W; c += 256) a.out[t * a.W + c] = fmaf((xt[c] - mean) * rstd, a.w_next[c], a.b_next[c]);
+}
+template <int NR>
+__global__ __launch_bounds__(256) void affine_seam_kernel(AffineSeamArgs a) { affine_seam_body<NR>(a); }
+template <int NR>
+__global__ __launch_bounds__(256) void affine_seam_route_kernel(AffineSeamArgs a, RouterGroupArgs r) {      // (as sandwich_route_kernel)
+  affine_seam_body<NR>(a);
+  __syncthreads();
+  router_group_body<true>(r);
 }
 
 // ---- sigmoid attention with mixed heads.  For the query token i and every key j it sees (a sliding window, a chunk, or all before it: stack_meta.h):

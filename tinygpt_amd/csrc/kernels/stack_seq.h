@@ -94,7 +94,7 @@ __device__ __forceinline__ void sandwich_row(const SandwichArgs& a, size_t t, fl
   }
 }
 template <int NR>
-__global__ __launch_bounds__(256) void sandwich_kernel(SandwichArgs a) {
+__device__ __forceinline__ void sandwich_body(SandwichArgs a) {
   __shared__ float s44[2][4];
   const size_t t = blockIdx.x;
   if (a.W <= 1024 * NR) {
@@ -128,6 +128,8 @@ __global__ __launch_bounds__(256) void sandwich_kernel(SandwichArgs a) {
   const float r2 = a.g_next[0] / sqrtf(s2 / (float)a.W + a.eps);
   for (int c = threadIdx.x; c < a.W; c += 256) a.out[t * a.W + c] = a.x[t * a.W + c] * r2;
 }
+template <int NR>
+__global__ __launch_bounds__(256) void sandwich_kernel(SandwichArgs a) { sandwich_body<NR>(a); }
 
 // ---- PolyNorm in place on z [T][F]: coef = (a, b, c, e)
 __global__ __launch_bounds__(256) void poly_norm_kernel(float* z, const float* coef, int F, float eps) {
@@ -587,7 +589,7 @@ struct RouterGroupArgs {
   int shared;                // 1: every token has one more choice behind its top: expert E with weight 1 (a shared expert that rides among the routed ones)
 };
 template <bool PRODUCT>
-__global__ __launch_bounds__(PRODUCT ? 256 : 64) void router_group_kernel(RouterGroupArgs a) {
+__device__ __forceinline__ void router_group_body(RouterGroupArgs a) {
   constexpr int ME = PRODUCT ? ROUTER_FUSED_MAX : ROUTER_MAX_E;
   __shared__ float s_s[ME], s_c[ME], s_g[ME], s_z[PRODUCT ? ME : 1], s_pw[ROUTER_MAX_TOP];
   __shared__ int s_pick[ROUTER_MAX_TOP];
@@ -645,6 +647,15 @@ __global__ __launch_bounds__(PRODUCT ? 256 : 64) void router_group_kernel(Router
   for (int k = lane; k < a.top; k += 64) { a.sel[(size_t)t * stride + k] = s_pick[k]; a.selw[(size_t)t * stride + k] = a.normalise ? s_pw[k] * inv : s_pw[k]; }
   if (a.shared && lane == 0) { a.sel[(size_t)t * stride + a.top] = a.E; a.selw[(size_t)t * stride + a.top] = 1.f; }
   if (a.sgw && lane == 0) a.sgw[t] = 1.0f / (1.0f + expf(-z[a.E]));
+}
+template <bool PRODUCT>
+__global__ __launch_bounds__(PRODUCT ? 256 : 64) void router_group_kernel(RouterGroupArgs a) { router_group_body<PRODUCT>(a); }
+// a few tokens' seam with the choice of experts behind it (as norm_conv_route_kernel)
+template <int NR>
+__global__ __launch_bounds__(256) void sandwich_route_kernel(SandwichArgs a, RouterGroupArgs r) {
+  sandwich_body<NR>(a);
+  __syncthreads();
+  router_group_body<true>(r);
 }
 
 }  // namespace tgx

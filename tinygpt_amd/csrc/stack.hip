@@ -280,11 +280,18 @@ void launch_experts(tgx_ctx* c, tgx::StackGemmArgs up, int epi_up, tgx::StackGem
   launch_ff(c, up, epi_up, down, epi_down, np, E, tile);
 }
 
-// a router's products on the rows h: true: the choice kernel takes them itself (steps of few tokens); false: they stand in zr
+// whether a router's choice kernel takes its products itself (steps of few tokens): then it rides behind the seam that writes its rows
+bool route_rides(const tgx_ctx* c, int n, int T) { return c->stack->gemv && T <= FEW_ROWS_MAX && n <= tgx::ROUTER_FUSED_MAX && c->stack->d.width % 4 == 0; }
+tgx::RouterInput router_input(const tgx_ctx* c, const float* h, const float* wr, int n) {
+  tgx::RouterInput in{};
+  in.h = h; in.ldh = in.K = c->stack->d.width; in.w = wr; in.n = n;
+  return in;
+}
+// a router's products on the rows h: true: the choice kernel takes them itself; false: they stand in zr
 bool route(tgx_ctx* c, tgx::RouterInput& in, const float* h, const float* wr, int n, int T) {
   StackModel* sm = c->stack;
   const int W = sm->d.width;
-  if (sm->gemv && T <= FEW_ROWS_MAX && n <= tgx::ROUTER_FUSED_MAX && W % 4 == 0) { in.h = h; in.ldh = W; in.w = wr; in.n = n; in.K = W; return true; }
+  if (route_rides(c, n, T)) { in = router_input(c, h, wr, n); return true; }
   tgx::StackGemmArgs g{};
   g.A = h; g.lda = W; g.B = wr; g.ldb = W; g.C = sm->zr; g.ldc = n; g.M = T; g.N = n; g.K = W; g.scale = 1.f;
   launch_gemm(c, g, tgx::SG_STORE, 1, 0, 0, 64, tgx::DT_F32);
@@ -360,10 +367,12 @@ int ensure_ws(tgx_ctx* c, int T) {
   return TGX_OK;
 }
 
-void launch_norm_conv(tgx_ctx* c, const tgx::StepMeta& m, const tgx::NormConvArgs& a, int T) {
-  if (a.taps == 4) hipLaunchKernelGGL(tgx::norm_conv_kernel<4>, dim3(T), dim3(256), 0, c->stream, m, a);
-  else if (a.taps == 1) hipLaunchKernelGGL(tgx::norm_conv_kernel<1>, dim3(T), dim3(256), 0, c->stream, m, a);
-  else hipLaunchKernelGGL(tgx::norm_conv_kernel<0>, dim3(T), dim3(256), 0, c->stream, m, a);
+// a filter's size by number where the kernels have it (kernels/stack.h)
+template <class F>
+void with_taps(int taps, F go) {
+  if (taps == 4) go(std::integral_constant<int, 4>{});
+  else if (taps == 1) go(std::integral_constant<int, 1>{});
+  else go(std::integral_constant<int, 0>{});
 }
 
 // a step of single tokens: the contexts that its kind will come to divide
@@ -379,15 +388,19 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
   const int W = sm->d.width, nslots = sm->d.max_seqs, nb = sm->d.canon_taps - 1;
   const size_t slot_stride = (size_t)sm->cap_tokens * W;
   TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::sinusoid_embed_kernel<DT>, dim3(T), dim3(256), 0, c->stream, m, reinterpret_cast<const tgx::elem_t<DT>*>(c->embed), 1.0f, sm->freq, sm->x, sm->xs, W))
+  const size_t st_buf = (size_t)nslots * nb * W;
+  auto norm_conv = [&](const StackLayerW& w, int sub) {      // in front of a layer's mixer (0) or feed-forward (1)
+    tgx::NormConvArgs nc{};
+    nc.x = sm->x; nc.nw = sub ? w.norm2 : w.norm1; nc.cw = sub ? w.canon2 : w.canon1; nc.out = sm->a; nc.state = nb > 0 ? w.conv_state + 2 * sub * st_buf : nullptr; nc.state_buf = st_buf;
+    nc.W = W; nc.groups = sm->d.norm_groups; nc.taps = sm->d.canon_taps; nc.eps = sm->d.norm_eps;
+    return nc;
+  };
+  bool normed = false;      // whether sm->a holds the layer's input (the layer before has left it there)
   for (int li = 0; li < sm->d.layers; li++) {
     StackLayerW& w = sm->L[(size_t)li];
     const tgx_layer_desc& ld = w.d;
     const int H = ld.heads, qd = H * ld.dim, R = ld.kv_rank, vd = H * ld.vdim, nin = qd + R + vd;
-    const size_t st_buf = (size_t)nslots * nb * W;
-    tgx::NormConvArgs nc{};
-    nc.x = sm->x; nc.nw = w.norm1; nc.cw = w.canon1; nc.out = sm->a; nc.state = nb > 0 ? w.conv_state : nullptr; nc.state_buf = st_buf;
-    nc.W = W; nc.groups = sm->d.norm_groups; nc.taps = sm->d.canon_taps; nc.eps = sm->d.norm_eps;
-    launch_norm_conv(c, m, nc, T);
+    if (!normed) with_taps(sm->d.canon_taps, [&](auto N) { hipLaunchKernelGGL(tgx::norm_conv_kernel<decltype(N)::value>, dim3(T), dim3(256), 0, c->stream, m, norm_conv(w, 0)); });
     // [q | latent | gate] = a . w_in^T
     tgx::StackGemmArgs g{};
     g.A = sm->a; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = nin; g.M = T; g.N = nin; g.K = W; g.scale = 1.f;
@@ -450,13 +463,17 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
     int top = 0;
     if (ld.mlp == TGX_MLP_MOE) {
       top = ld.top;
-      nc.nw = w.norm2; nc.cw = w.canon2; nc.state = nb > 0 ? w.conv_state + 2 * st_buf : nullptr;
-      launch_norm_conv(c, m, nc, T);
       // router: fp32 weights, fp32 products (nothing is rounded), then bias, top-k and the softmax over the chosen
       tgx::RouterArgs ra{};
       ra.z = sm->zr; ra.br = w.b_router; ra.sel = sm->sel; ra.selw = sm->selw; ra.E = ld.experts; ra.top = top;
-      if (route(c, ra.in, sm->a, w.w_router, ld.experts, T)) hipLaunchKernelGGL(tgx::router_topk_kernel<true>, dim3(T), dim3(256), 0, c->stream, ra);
-      else hipLaunchKernelGGL(tgx::router_topk_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
+      if (route_rides(c, ld.experts, T)) {
+        ra.in = router_input(c, sm->a, w.w_router, ld.experts);
+        with_taps(sm->d.canon_taps, [&](auto N) { hipLaunchKernelGGL(tgx::norm_conv_route_kernel<decltype(N)::value>, dim3(T), dim3(256), 0, c->stream, m, norm_conv(w, 1), ra); });
+      } else {
+        with_taps(sm->d.canon_taps, [&](auto N) { hipLaunchKernelGGL(tgx::norm_conv_kernel<decltype(N)::value>, dim3(T), dim3(256), 0, c->stream, m, norm_conv(w, 1)); });
+        (void)route(c, ra.in, sm->a, w.w_router, ld.experts, T);
+        hipLaunchKernelGGL(tgx::router_topk_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
+      }
       // yh[pair] = act(gate_e . a[token], up_e . a[token]), yd[pair] = router weight * (down_e . yh[pair])
       g = tgx::StackGemmArgs{};
       g.A = sm->a; g.lda = W; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff; g.N = ld.ff; g.K = W; g.limit = ld.limit;
@@ -467,7 +484,9 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
     }
     tgx::CombineDepthArgs cd{};
     cd.x = sm->x; cd.y = sm->yd; cd.xs = sm->xs; cd.slot_stride = slot_stride; cd.dw = w.dwa; cd.W = W; cd.top = top; cd.n_res = li + 2;
-    hipLaunchKernelGGL(tgx::combine_depth_kernel, dim3(T), dim3(256), 0, c->stream, cd);
+    normed = max_count == 1 && li + 1 < sm->d.layers;
+    if (normed) with_taps(sm->d.canon_taps, [&](auto N) { hipLaunchKernelGGL(tgx::combine_norm_conv_kernel<decltype(N)::value>, dim3(T), dim3(256), 0, c->stream, m, cd, norm_conv(sm->L[(size_t)li + 1], 0)); });
+    else hipLaunchKernelGGL(tgx::combine_depth_kernel, dim3(T), dim3(256), 0, c->stream, cd);
   }
   return TGX_OK;
 }
@@ -694,16 +713,28 @@ void run_dense_ff(tgx_ctx* c, StackLayerW& w, const float* hin, int T) {
 }
 
 // grouped-choice experts: the chosen pairs' rows land in yd (none for identity outputs), the shared expert's in ysh; the seam kernel sums them
-void run_choice_experts(tgx_ctx* c, StackLayerW& w, const float* hin, int T) {
+// products of a choice layer's router: its outputs and the shared expert's gate
+int choice_products(const tgx_layer_desc& ld) { return ld.experts + ld.identity + (ld.shared_ff > 0 ? 1 : 0); }
+tgx::RouterGroupArgs choice_router(const tgx_ctx* c, const StackLayerW& w, const float* hin) {
+  const StackModel* sm = c->stack;
+  const tgx_layer_desc& ld = w.d;
+  tgx::RouterGroupArgs ra{};
+  ra.in = router_input(c, hin, w.w_router, choice_products(ld));
+  ra.z = sm->zr; ra.ldz = choice_products(ld); ra.corr = w.b_router; ra.sel = sm->sel; ra.selw = sm->selw; ra.sgw = ld.shared_ff > 0 ? sm->sgw : nullptr;
+  ra.E = ld.experts + ld.identity; ra.top = ld.top; ra.groups = ld.groups; ra.keep = ld.groups_keep; ra.scale = ld.router_scale;
+  return ra;
+}
+// routed: the choice stands already (it rode behind the seam)
+void run_choice_experts(tgx_ctx* c, StackLayerW& w, const float* hin, int T, bool routed) {
   StackModel* sm = c->stack;
   const tgx_layer_desc& ld = w.d;
-  const int W = sm->d.width, E = ld.experts + ld.identity, top = ld.top, nz = E + (ld.shared_ff > 0 ? 1 : 0);
+  const int W = sm->d.width, E = ld.experts + ld.identity, top = ld.top;
   tgx::StackGemmArgs g{};
-  tgx::RouterGroupArgs ra{};
-  ra.z = sm->zr; ra.ldz = nz; ra.corr = w.b_router; ra.sel = sm->sel; ra.selw = sm->selw; ra.sgw = ld.shared_ff > 0 ? sm->sgw : nullptr;
-  ra.E = E; ra.top = top; ra.groups = ld.groups; ra.keep = ld.groups_keep; ra.scale = ld.router_scale;
-  if (route(c, ra.in, hin, w.w_router, nz, T)) hipLaunchKernelGGL(tgx::router_group_kernel<true>, dim3(T), dim3(256), 0, c->stream, ra);
-  else hipLaunchKernelGGL(tgx::router_group_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
+  if (!routed) {
+    tgx::RouterGroupArgs ra = choice_router(c, w, hin);
+    (void)route(c, ra.in, hin, w.w_router, choice_products(ld), T);
+    hipLaunchKernelGGL(tgx::router_group_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
+  }
   const int np = T * top;
   if (ld.experts > 0) {
     g = tgx::StackGemmArgs{};
@@ -741,14 +772,16 @@ int run_layers_sandwich(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_ke
     if (rc) return rc;
     tgx::SandwichArgs sa{};
     sa.x = sm->x; sa.y = sm->yd; sa.top = 1; sa.ytmp = sm->ytmp; sa.g_post = ng + 1; sa.g_next = ld.mlp != TGX_MLP_NONE ? ng + 2 : next_layer; sa.out = hout; sa.W = W; sa.eps = eps;
-    launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::sandwich_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa); });
+    const bool routed = ld.mlp == TGX_MLP_MOE && route_rides(c, choice_products(ld), T);
+    if (routed) launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::sandwich_route_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa, choice_router(c, w, hout)); });
+    else launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::sandwich_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa); });
     std::swap(hin, hout);
     if (ld.mlp == TGX_MLP_NONE) continue;
     sa = tgx::SandwichArgs{};
     sa.x = sm->x; sa.y = sm->yd; sa.top = 1; sa.ytmp = sm->ytmp; sa.g_post = ng + 3; sa.g_next = next_layer; sa.out = hout; sa.W = W; sa.eps = eps;
     if (ld.mlp == TGX_MLP_DENSE) run_dense_ff(c, w, hin, T);
     else {
-      run_choice_experts(c, w, hin, T);
+      run_choice_experts(c, w, hin, T, routed);
       sa.top = ld.top; sa.sel = sm->sel; sa.selw = sm->selw; sa.n_real = ld.experts; sa.h = hin; sa.ysh = ld.shared_ff > 0 ? sm->ysh : nullptr;
     }
     launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::sandwich_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa); });
@@ -1166,7 +1199,16 @@ int run_affine_latent(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, const 
 }
 
 // the feed-forward of a layer-norm design into yd (one row per token, or `top` rows per token for experts) and ysh (the shared expert's row)
-void run_affine_ff(tgx_ctx* c, StackLayerW& w, int T) {
+tgx::RouterGroupArgs affine_router(const tgx_ctx* c, const StackLayerW& w) {
+  const StackModel* sm = c->stack;
+  const tgx_layer_desc& ld = w.d;
+  tgx::RouterGroupArgs ra{};
+  ra.in = router_input(c, sm->a, w.w_router, ld.experts);
+  ra.z = sm->zr; ra.ldz = ld.experts; ra.sel = sm->sel; ra.selw = sm->selw; ra.E = ld.experts; ra.top = ld.top; ra.groups = ld.groups; ra.keep = ld.groups_keep; ra.scale = 1.f;
+  ra.sigmoid_scores = ld.router_fn == 1; ra.group_top2 = ld.group_score == 1; ra.normalise = ld.router_norm;
+  return ra;
+}
+void run_affine_ff(tgx_ctx* c, StackLayerW& w, int T, bool routed) {
   StackModel* sm = c->stack;
   const tgx_layer_desc& ld = w.d;
   const int W = sm->d.width;
@@ -1177,12 +1219,11 @@ void run_affine_ff(tgx_ctx* c, StackLayerW& w, int T) {
     return;
   }
   const int E = ld.experts, top = ld.top, np = T * top;
-  tgx::RouterGroupArgs ra{};
-  ra.z = sm->zr; ra.ldz = E; ra.corr = nullptr; ra.sel = sm->sel; ra.selw = sm->selw; ra.sgw = nullptr;
-  ra.E = E; ra.top = top; ra.groups = ld.groups; ra.keep = ld.groups_keep; ra.scale = 1.f;
-  ra.sigmoid_scores = ld.router_fn == 1; ra.group_top2 = ld.group_score == 1; ra.normalise = ld.router_norm;
-  if (route(c, ra.in, sm->a, w.w_router, E, T)) hipLaunchKernelGGL(tgx::router_group_kernel<true>, dim3(T), dim3(256), 0, c->stream, ra);
-  else hipLaunchKernelGGL(tgx::router_group_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
+  if (!routed) {
+    tgx::RouterGroupArgs ra = affine_router(c, w);
+    (void)route(c, ra.in, sm->a, w.w_router, E, T);
+    hipLaunchKernelGGL(tgx::router_group_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
+  }
   g = tgx::StackGemmArgs{};
   g.A = sm->a; g.lda = W; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff; g.N = ld.ff; g.K = W;
   const tgx::StackGemmArgs gu = g;
@@ -1231,10 +1272,12 @@ int run_layers_affine(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
     sa.x = sm->x; sa.y = sm->yd; sa.top = 1; sa.ytmp = sm->ytmp; sa.w_post = ln + 2 * (size_t)W; sa.b_post = ln + 3 * (size_t)W; sa.mult = mult; sa.out = sm->a; sa.W = W; sa.eps = eps;
     if (ld.mlp != TGX_MLP_NONE) { sa.w_next = ln + 4 * (size_t)W; sa.b_next = ln + 5 * (size_t)W; }
     else if (next_ln) { sa.w_next = next_ln; sa.b_next = next_ln + W; }
-    launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::affine_seam_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa); });
+    const bool routed = ld.mlp == TGX_MLP_MOE && route_rides(c, ld.experts, T);
+    if (routed) launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::affine_seam_route_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa, affine_router(c, w)); });
+    else launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::affine_seam_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa); });
     normed = sa.w_next != nullptr;
     if (ld.mlp == TGX_MLP_NONE) continue;
-    run_affine_ff(c, w, T);
+    run_affine_ff(c, w, T, routed);
     sa = tgx::AffineSeamArgs{};
     sa.x = sm->x; sa.y = sm->yd; sa.top = ld.mlp == TGX_MLP_MOE ? ld.top : 1; sa.ysh = ld.mlp == TGX_MLP_MOE && ld.shared_ff > 0 ? sm->ysh : nullptr; sa.ytmp = sm->ytmp;
     sa.w_post = ln + 6 * (size_t)W; sa.b_post = ln + 7 * (size_t)W; sa.mult = mult; sa.out = sm->a; sa.W = W; sa.eps = eps;
@@ -1838,6 +1881,16 @@ bool shared_rides(const tgx_ctx* c, const StackLayerW& w, int T) {
   const int np = T * (w.d.top + 1);
   return w.shared_slot && np <= GROUPED_FEW_PAIRS && c->stack->gemv && c->stack->d.width % 8 == 0 && w.d.ff % 8 == 0;      // (the pairs' kernel)
 }
+tgx::RouterGroupArgs hyper_router(const tgx_ctx* c, const StackLayerW& w, int T) {
+  const StackModel* sm = c->stack;
+  const tgx_layer_desc& ld = w.d;
+  tgx::RouterGroupArgs ra{};
+  ra.in = router_input(c, sm->a, w.w_router, ld.experts);
+  ra.z = sm->zr; ra.ldz = ld.experts; ra.sel = sm->sel; ra.selw = sm->selw; ra.E = ld.experts; ra.top = ld.top; ra.shared = shared_rides(c, w, T) ? 1 : 0; ra.groups = 1; ra.keep = 1; ra.scale = 1.f;
+  ra.sigmoid_scores = ld.router_fn == 1; ra.normalise = ld.router_norm;
+  return ra;
+}
+bool hyper_route_rides(const tgx_ctx* c, const StackLayerW& w, int T) { return w.d.mlp == TGX_MLP_MOE && route_rides(c, w.d.experts, T); }
 // the feed-forward into yd (one row per token, or a row per choice for experts) and ysh (the shared expert's row, unless it rides among the choices)
 void run_hyper_ff(tgx_ctx* c, StackLayerW& w, int T) {
   StackModel* sm = c->stack;
@@ -1850,10 +1903,11 @@ void run_hyper_ff(tgx_ctx* c, StackLayerW& w, int T) {
     return;
   }
   const int ride = shared_rides(c, w, T) ? 1 : 0, E = ld.experts + ride, top = ld.top + ride, np = T * top;
-  tgx::RouterGroupArgs ra{};
-  ra.z = sm->zr; ra.ldz = ld.experts; ra.sel = sm->sel; ra.selw = sm->selw; ra.E = ld.experts; ra.top = ld.top; ra.shared = ride; ra.groups = 1; ra.keep = 1; ra.scale = 1.f; ra.sigmoid_scores = ld.router_fn == 1; ra.normalise = ld.router_norm;
-  if (route(c, ra.in, sm->a, w.w_router, ld.experts, T)) hipLaunchKernelGGL(tgx::router_group_kernel<true>, dim3(T), dim3(256), 0, c->stream, ra);
-  else hipLaunchKernelGGL(tgx::router_group_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
+  if (!hyper_route_rides(c, w, T)) {      // (else the choice stands already)
+    tgx::RouterGroupArgs ra = hyper_router(c, w, T);
+    (void)route(c, ra.in, sm->a, w.w_router, ld.experts, T);
+    hipLaunchKernelGGL(tgx::router_group_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
+  }
   // yh[pair] = max(up_e (w h), 0)^2: up_e is linear, so the weight multiplies its product
   g = tgx::StackGemmArgs{};
   g.A = sm->a; g.lda = W; g.B = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff; g.scale = 1.f; g.act = tgx::SG_ACT_RELU2; g.in_w = sm->selw; g.N = ld.ff; g.K = W;
@@ -1879,11 +1933,17 @@ void hyper_seam(tgx_ctx* c, const StackLayerW& w, int sub, const float* next_in,
   tgx::HyperSeamArgs sa{};
   sa.xs = sm->xs; sa.y = sm->yd; sa.top = top; sa.ysh = shared ? sm->ysh : nullptr; sa.w_out = hc + n; sa.mix = hc + 2 * n; sa.n = n; sa.W = sm->d.width;
   sa.in.w_in = next_in; sa.in.w_norm = next_norm; sa.in.out = next_in ? sm->a : sm->x; sa.in.eps = sm->d.norm_eps;
-  if (n <= 1) hipLaunchKernelGGL(tgx::hyper_seam_kernel<1>, dim3(T), dim3(256), 0, c->stream, sa);
-  else if (n <= 2) hipLaunchKernelGGL(tgx::hyper_seam_kernel<2>, dim3(T), dim3(256), 0, c->stream, sa);
-  else if (n <= 4) hipLaunchKernelGGL(tgx::hyper_seam_kernel<4>, dim3(T), dim3(256), 0, c->stream, sa);
-  else if (n <= 8) hipLaunchKernelGGL(tgx::hyper_seam_kernel<8>, dim3(T), dim3(256), 0, c->stream, sa);
-  else hipLaunchKernelGGL(tgx::hyper_seam_kernel<16>, dim3(T), dim3(256), 0, c->stream, sa);
+  const bool routed = sub == 0 && hyper_route_rides(c, w, T);      // (the feed-forward's input: the choice of experts rides behind)
+  auto go = [&](auto NS) {
+    constexpr int N = decltype(NS)::value;
+    if (routed) hipLaunchKernelGGL(tgx::hyper_seam_route_kernel<N>, dim3(T), dim3(256), 0, c->stream, sa, hyper_router(c, w, T));
+    else hipLaunchKernelGGL(tgx::hyper_seam_kernel<N>, dim3(T), dim3(256), 0, c->stream, sa);
+  };
+  if (n <= 1) go(std::integral_constant<int, 1>{});
+  else if (n <= 2) go(std::integral_constant<int, 2>{});
+  else if (n <= 4) go(std::integral_constant<int, 4>{});
+  else if (n <= 8) go(std::integral_constant<int, 8>{});
+  else go(std::integral_constant<int, 16>{});
 }
 
 int run_layers_hyper(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys, int max_count) {
