@@ -86,3 +86,19 @@ def test_sigmoid_attention_of_divided_keys(heads, kv, dim, vdim, n, mask):
     eng.close()
     want = tz.want_of(cfg, w, toks)
     assert np.abs(np.concatenate(got) - want[n - 4:]).max() / np.abs(want).max() < 1e-4
+
+
+# ---- the scan over portions: blocks of sixteen and eight tokens, one and two turns of eight, sixteen and thirty-two row groups, odd ends of each; then single tokens carry on
+@pytest.mark.parametrize("dim,vdim,entries", [(128, 36, 1), (100, 20, 1), (64, 17, 1), (192, 24, 1), (32, 40, 24), (128, 64, 24), (30, 6, 2)])
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 15, 16, 17, 24, 33])
+def test_scan_over_portions(dim, vdim, entries, n):
+    cfg = tv.config([tv.par(right=dict(dim=dim, vdim=vdim, heads=4, kv_heads=2)), tv.wkv(heads=2, dim=dim)], width=20)
+    eng, w = tv.engine(cfg, seed=dim, max_seqs=entries, max_ctx=128, budget_tokens=64 * entries)
+    toks = [tv.tokens(cfg, n + 3, seed=i) for i in range(entries)]
+    got = [eng.step([(i, s[:max(1, n - i % 3)], [max(1, n - i % 3) - 1]) for i, s in enumerate(toks)])]
+    got.append(eng.step([(i, s[max(1, n - i % 3):], [len(s) - max(1, n - i % 3) - 1]) for i, s in enumerate(toks)]))
+    eng.close()
+    for i in {0, entries // 2}:
+        want = tv.want_of(cfg, w, toks[i])
+        for at, part in ((max(1, n - i % 3) - 1, got[0]), (n + 2, got[1])):
+            assert np.abs(part[i] - want[at]).max() / np.abs(want).max() < 1e-4, (n, i, at)

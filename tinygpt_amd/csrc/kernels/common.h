@@ -196,14 +196,18 @@ __device__ __forceinline__ float group_max(float v) {
   return v;
 }
 
-// Sum over aligned groups of 4, 8 or 16 adjacent lanes on the DPP crossbar; every lane of the group gets the sum.
+// Sum over aligned groups of 4, 8, 16 or 32 adjacent lanes on the DPP crossbar; every lane of the group gets the sum.
 template <int WIDTH>
 __device__ __forceinline__ float row_group_sum(float v) {
-  static_assert(WIDTH == 4 || WIDTH == 8 || WIDTH == 16, "row_group_sum: 4, 8 or 16 lanes");
+  static_assert(WIDTH == 4 || WIDTH == 8 || WIDTH == 16 || WIDTH == 32, "row_group_sum: 4, 8, 16 or 32 lanes");
   v += dpp_mov<0xB1, 0xf>(v);    // quad_perm:[1,0,3,2]
   v += dpp_mov<0x4E, 0xf>(v);    // quad_perm:[2,3,0,1]
   if (WIDTH >= 8) v += dpp_mov<0x141, 0xf>(v);   // row_half_mirror
-  if (WIDTH == 16) v += dpp_mov<0x140, 0xf>(v);   // row_mirror
+  if (WIDTH >= 16) v += dpp_mov<0x140, 0xf>(v);   // row_mirror
+  if constexpr (WIDTH == 32) {                     // rows 0 and 1, 2 and 3: each gets the other's
+    const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
   return v;
 }
 

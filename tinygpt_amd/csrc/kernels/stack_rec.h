@@ -137,10 +137,11 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(StepMeta m, DeltaPrepAr
 // inputs (up to three vectors of `dim`) and the workgroup's value columns are staged in LDS (the next block's travel in registers meanwhile), then every
 // lane updates its DPER rows of its column with no barrier inside the block: a wave's lanes = 64 / RG columns x RG row groups (the row groups of a column are
 // adjacent lanes), RG DPER >= dim.  Sums over the key channels cross the row groups on the lane crossbar.
-// What bounds a prompt is the instructions that one wave issues per token (64 multiply-adds and some fifty others for the delta rule at eight groups of sixteen rows; with the
-// stores, crossbar steps, staging and LDS reads taken out the multiply-adds alone are 345 of 630 us for 2048 tokens).  Sixteen groups halve a lane's rows and double the workgroups,
-// which is right while the step leaves compute units idle; eight issue fewer instructions in all.  2048 tokens, delta rule of 16 heads of 128 x 128: 632 us at
-// eight row groups staged number by number, 578 staged in vectors of four, 469 at sixteen; channel decays 688 / 604 / 505, wkv of 32 heads of 64 x 64 419 / 409 / 330.
+// What bounds a prompt is the instructions that one wave issues per token, four cycles each, and the waits between dependent ones where a SIMD has a single wave.  So a step that
+// leaves compute units idle spreads a column over more row groups (sixteen, or thirty-two of four rows: twice the workgroups of half the rows), a full chip takes eight, which issue
+// fewer instructions in all; two tokens go without a branch between them, so that the one's sum over the groups lies under the other's arithmetic; and a column's outputs are kept by its
+// row groups, a token each, and leave in one store for as many tokens as there are groups.  2048 tokens, delta rule of 16 heads of 128 x 128: 632 us at eight row groups staged number
+// by number, 578 staged in vectors of four, 470 at sixteen with a store a token, 340 at thirty-two and stores by the block; wkv of 32 heads of 64 x 64 419, 409, 335, 257 (sixteen groups).
 enum { REC_WKV = 0, REC_DELTA = 1, REC_SSD = 2, REC_CDELTA = 3 };
 struct RecScanArgs {
   const float* a; long long lda;     // per token and key head [dim]: the read vector (wkv: r, delta: q, ssd: C)
@@ -158,7 +159,7 @@ struct RecScanArgs {
 constexpr int rec_cols(int rg) { return 4 * (64 / rg); }      // columns per workgroup
 template <int DPER, int KIND, int RG, bool VEC>
 __global__ __launch_bounds__(256) void rec_scan_kernel(StepMeta m, RecScanArgs a) {
-  constexpr int CW = 64 / RG, CB = rec_cols(RG), LP = RG == 16 && DPER == 4 ? 4 : DPER + 4, DP = RG * DPER, TB = DP <= 128 ? 16 : 8;      // LP: a row group's LDS stride (the groups' reads fall into different banks)
+  constexpr int CW = 64 / RG, CB = rec_cols(RG), LP = RG >= 16 && DPER == 4 ? 4 : DPER + 4, DP = RG * DPER, TB = DP <= 128 ? 16 : 8;      // LP: a row group's LDS stride (the groups' reads fall into different banks)
   constexpr int Q4 = TB * DP / 4, NQ = (Q4 + 255) / 256, NV = (TB * CB + 255) / 256, NA = KIND == REC_WKV || KIND == REC_CDELTA ? 3 : 2;
   __shared__ __attribute__((aligned(16))) float s_in[NA][TB][RG * LP];      // [0]: the read vector, [1]: k, [2]: the decay
   __shared__ float s_v[TB][CB], s_b[TB], s_g[TB];
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(256) void rec_scan_kernel(StepMeta m, RecScanArgs a
       k.v = s_v[t][jl];
       if (KIND != REC_WKV) { k.g = s_g[t]; k.b = s_b[t]; }
     };
-    auto advance = [&](const Tok& k, int t) {
+    auto advance = [&](const Tok& k) -> float {
       float po = 0.f;
       if (KIND == REC_WKV) {
 #pragma unroll
@@ -260,15 +261,30 @@ __global__ __launch_bounds__(256) void rec_scan_kernel(StepMeta m, RecScanArgs a
       }
       po = row_group_sum<RG>(po);
       if (KIND == REC_SSD) po = fmaf(skip, k.v, po);
-      if (rg == 0 && col) a.out[(size_t)(start + t0 + t) * a.ldo + (size_t)h * a.vdim + j] = po;
+      return po;
     };
+    // Every row group of a column ends with a token's output: group r keeps that of token r (of as many tokens as there are groups), so a column's tokens leave in one store.
+    // Two tokens a turn without a branch between them: the one's sum over the groups lies under the other's arithmetic.
+    constexpr int FL = RG < TB ? RG : TB;
     Tok ka, kb;
     take(ka, 0);
-    for (int t = 0; t < nb; t += 2) {
-      take(kb, min(t + 1, TB - 1));
-      advance(ka, t);
-      take(ka, min(t + 2, TB - 1));
-      if (t + 1 < nb) advance(kb, t + 1);
+    for (int s0 = 0; s0 < nb; s0 += FL) {
+      const int n = min(FL, nb - s0);
+      float keep = 0.f;
+      int t = 0;
+      for (; t + 1 < n; t += 2) {
+        take(kb, s0 + t + 1);
+        const float o0 = advance(ka);
+        take(ka, min(s0 + t + 2, TB - 1));
+        const float o1 = advance(kb);
+        keep = rg == t ? o0 : rg == t + 1 ? o1 : keep;
+      }
+      if (t < n) {
+        const float o0 = advance(ka);
+        take(ka, min(s0 + t + 1, TB - 1));
+        keep = rg == t ? o0 : keep;
+      }
+      if (rg < n && col) a.out[(size_t)(start + t0 + s0 + rg) * a.ldo + (size_t)h * a.vdim + j] = keep;
     }
   }
 #pragma unroll

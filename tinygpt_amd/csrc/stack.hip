@@ -837,15 +837,18 @@ struct JointLayer {
 void launch_rec_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs& a, int kind, int S) {
   const bool vec = a.dim % 4 == 0 && a.lda % 4 == 0 && a.ldk % 4 == 0 && (uintptr_t)a.a % 16 == 0 && (uintptr_t)a.k % 16 == 0 && (!a.w || (a.ldw % 4 == 0 && (uintptr_t)a.w % 16 == 0));
   // sixteen row groups per column while their workgroups, of sixteen columns, leave a compute unit with two at most: one prompt of 16 heads of 128 (kernels/stack_rec.h), a few
-  // requests; a full chip issues fewer instructions with eight
+  // requests; thirty-two, of four rows, while there is a compute unit for each of theirs (one prompt of 16 heads of 128 x 128: 340 us against sixteen's 400 for 2048 tokens; a SIMD
+  // with two of their waves would issue more than with one of sixteen groups'); a full chip issues fewer instructions with eight
   auto cols = [&](int rg) { return (a.vdim + tgx::rec_cols(rg) - 1) / tgx::rec_cols(rg); };
   const bool wide = vec && a.dim <= 256 && (long long)S * a.heads * cols(16) <= 2LL * c->num_cus;
-  const int rg = wide ? 16 : 8, dper = (a.dim + rg - 1) / rg;      // rows per lane
+  const bool widest = wide && a.dim > 64 && a.dim <= 128 && (long long)S * a.heads * cols(32) <= c->num_cus;
+  const int rg = widest ? 32 : wide ? 16 : 8, dper = (a.dim + rg - 1) / rg;      // rows per lane
   const dim3 grid(S, a.heads, cols(rg));
   auto go = [&](auto K) {
     constexpr int KIND = decltype(K)::value;
     auto rows = [&](auto D) {
       constexpr int DPER = decltype(D)::value;
+      if constexpr (DPER == 4) if (widest) { hipLaunchKernelGGL((tgx::rec_scan_kernel<DPER, KIND, 32, true>), grid, dim3(256), 0, c->stream, m, a); return; }
       if constexpr (DPER <= 16) if (wide) { hipLaunchKernelGGL((tgx::rec_scan_kernel<DPER, KIND, 16, true>), grid, dim3(256), 0, c->stream, m, a); return; }
       if (vec) hipLaunchKernelGGL((tgx::rec_scan_kernel<DPER, KIND, 8, true>), grid, dim3(256), 0, c->stream, m, a);
       else hipLaunchKernelGGL((tgx::rec_scan_kernel<DPER, KIND, 8, false>), grid, dim3(256), 0, c->stream, m, a);
