@@ -102,3 +102,23 @@ def test_scan_over_portions(dim, vdim, entries, n):
         want = tv.want_of(cfg, w, toks[i])
         for at, part in ((max(1, n - i % 3) - 1, got[0]), (n + 2, got[1])):
             assert np.abs(part[i] - want[at]).max() / np.abs(want).max() < 1e-4, (n, i, at)
+
+
+# ---- sigmoid attention of prompts over divided keys (two to four shares while the tiles leave half of the chip idle), against the undivided lane kernels: the same bf16 weights and
+# cached rows, bound of the design's own comparison of the two
+@pytest.mark.parametrize("shape", [dict(heads=4, kv_heads=2, dim=32, vdim=64), dict(heads=2, kv_heads=1, dim=16, vdim=32)])
+@pytest.mark.parametrize("size", [None, 513, 770, 1100])
+def test_sigmoid_attention_of_prompts_over_divided_keys(shape, size):
+    import test_hip_zaluvik as tz
+    mask = {"size": size} if size else None
+    cfg = tz.config([tz.attn(tz.dense(), mask=mask, scale=2.0, **shape), tz.attn(mask=mask, scale=2.0, **shape)], width=64, loop=None)
+    toks = [tz.tokens(cfg, n, seed=n) for n in (1201, 530)]
+    out = []
+    for on in (1, 0):
+        eng, _ = tz.engine(cfg, "bf16", seed=3, max_ctx=2048, budget_tokens=4096)
+        eng.model.set_option("attn.mfma", on)
+        o = [eng.step([("a", toks[0][:640], [0, 511, 512, 639]), ("b", toks[1], [0, 31, 32, 529])])]
+        o.append(eng.step([("a", toks[0][640:], [0, 31, 300, 560])]))
+        eng.close()
+        out.append(np.concatenate(o))
+    assert np.abs(out[0] - out[1]).max() / np.abs(out[1]).max() < 1e-3

@@ -29,6 +29,9 @@ struct MixMfmaArgs {
   int heads, kv_heads, dim, vdim, terms;
   float scale;
   int mask_kind, mask_size;
+  // divided keys: blockIdx.z = key / value head group * nsplit + share; a share takes keys_per (a multiple of 32) keys from the tile's first on and leaves its sums in
+  // part [T][nsplit][heads * vdim] for sigmoid_mix_merge_kernel (nothing is normalised: shares are added).  nsplit 1: undivided
+  float* part = nullptr; int nsplit = 1, keys_per = 0;
 };
 constexpr int MIXM_LDW = 32;            // floats per row of a weight tile in LDS
 // qpg: the query heads a workgroup sums values for (NG * QPG)
@@ -46,14 +49,15 @@ __global__ __launch_bounds__(256) void sigmoid_mix_mfma_kernel(StepMeta m, MixMf
   bf16_t* s_pl = s_ph + NH * 32 * 40;
   float* s_t = reinterpret_cast<float*>(s_pl + NH * 32 * 40);                    // [NH][H]: the rows of the mixing matrix for this workgroup's heads
   float* s_pb = s_t + NH * H;                                                   // [H], in units of log 2 like the scores
-  const int e = blockIdx.y, c0 = blockIdx.z * NG;      // key / value heads c0 .. c0 + NG - 1 (those that exist)
+  const int e = blockIdx.y, zs = blockIdx.z % a.nsplit, c0 = blockIdx.z / a.nsplit * NG;      // key / value heads c0 .. c0 + NG - 1 (those that exist)
   const int cnt = m.ent_count[e], start = m.ent_start[e], slot = m.ent_row[e];
   const int t0 = blockIdx.x * 32;
   if (t0 >= cnt) return;
   const int past = m.tok_pos[start];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, half = lane >> 5, l31 = lane & 31;
-  const int kmax = past + min(t0 + 31, cnt - 1) + 1;
-  const int k0 = first_key(past + t0, a.mask_kind, a.mask_size) & ~31;
+  int kmax = past + min(t0 + 31, cnt - 1) + 1;
+  int k0 = first_key(past + t0, a.mask_kind, a.mask_size) & ~31;
+  if (a.nsplit > 1) { k0 += zs * a.keys_per; kmax = min(kmax, k0 + a.keys_per); }
   const int page = 1 << m.page_shift, kd = a.kv_heads * a.dim, vd = a.kv_heads * a.vdim, qd = H * a.dim;
   const bf16_t* poolK = reinterpret_cast<const bf16_t*>(a.poolK);
   const bf16_t* poolVT = reinterpret_cast<const bf16_t*>(a.poolVT);
@@ -210,7 +214,8 @@ __global__ __launch_bounds__(256) void sigmoid_mix_mfma_kernel(StepMeta m, MixMf
       const int ri = (r & 3) + 8 * (r >> 2) + 4 * half;
       if (t0 + ri >= cnt || c0 * QPG + hq >= H) continue;
       const size_t tk = (size_t)start + t0 + ri, o = (size_t)(c0 * QPG + hq) * a.vdim + 32 * wv + l31;
-      a.out[tk * a.ldo + o] = a.gate ? acc[hq][r] / (1.0f + expf(-a.gate[tk * a.ldg + o])) : acc[hq][r];
+      if (a.nsplit > 1) a.part[(tk * a.nsplit + zs) * (size_t)H * a.vdim + o] = acc[hq][r];
+      else a.out[tk * a.ldo + o] = a.gate ? acc[hq][r] / (1.0f + expf(-a.gate[tk * a.ldg + o])) : acc[hq][r];
     }
 }
 

@@ -73,7 +73,7 @@ void launch_mix_mfma(tgx_ctx* c, const tgx::StepMeta& m, const tgx::MixMfmaArgs&
   const int qpg = a.heads / a.kv_heads;
   int ng = mix_groups_per_wg(a.heads, a.kv_heads, a.dim, c->stack->mix_groups);
   if (ng == 2 && c->stack->mix_groups != 2 && (long long)grid.x * grid.y * ((a.kv_heads + 1) / 2) < c->num_cus) ng = 1;      // sharing the scores halves the workgroups: only while they still fill the chip
-  grid.z = (a.kv_heads + ng - 1) / ng;
+  grid.z = (a.kv_heads + ng - 1) / ng * a.nsplit;
   TGX_DT16_SWITCH(c->dt,
     if (qpg == 1) { if (ng == 2) launch_mix_q<DT, 1, 2>(c, m, a, grid); else launch_mix_q<DT, 1, 1>(c, m, a, grid); }
     else if (qpg == 2) { if (ng == 2) launch_mix_q<DT, 2, 2>(c, m, a, grid); else launch_mix_q<DT, 2, 1>(c, m, a, grid); }
