@@ -122,3 +122,35 @@ def test_sigmoid_attention_of_prompts_over_divided_keys(shape, size):
         eng.close()
         out.append(np.concatenate(o))
     assert np.abs(out[0] - out[1]).max() / np.abs(out[1]).max() < 1e-3
+
+
+# ---- products in one launch beside what does not need them: a channel-delta layer's low-rank pair (equal inner lengths; outputs of equal and of different widths; unequal lengths
+# stand apart) and a latent layer's append beside its queries, rows around the sixteen, 32 and 64 of an operand and past the last
+@pytest.mark.parametrize("ranks", [(8, 8), (72, 72), (16, 8)])
+@pytest.mark.parametrize("dim,vdim", [(16, 16), (8, 24), (40, 8)])
+@pytest.mark.parametrize("rows", [3, 16, 17, 33, 64, 65])
+def test_low_rank_pair(rows, dim, vdim, ranks):
+    cfg = tk.config([tk.cd(dim=dim, vdim=vdim)], width=24)
+    eng, w = tk.engine(cfg, seed=rows, ranks=ranks)
+    toks = tk.tokens(cfg, rows, seed=dim)
+    got = tk.run_whole(eng, "a", toks)
+    eng.close()
+    tk.check(got, tk.want_of(cfg, w, toks), "fp32", f"{rows} rows")
+
+
+@pytest.mark.parametrize("kv_rank,dim,heads", [(24, 8, 3), (72, 16, 2), (16, 40, 5)])
+@pytest.mark.parametrize("slots", [2, 3, 16, 17])
+def test_latents_beside_their_queries(slots, kv_rank, dim, heads):
+    import stack_oracle as so
+    from tinygpt_amd.desc import LayerDesc, StackDesc
+    from tinygpt_amd.serving import SlotEngine
+    layers = [LayerDesc(heads=heads, dim=dim, vdim=8, kv_rank=kv_rank, scale=0.35, mlp="moe", experts=5, top=2, ff=24, limit=1.5) for _ in range(3)]
+    d = StackDesc(width=72, vocab=53, canon_taps=4, norm_groups=2, norm_eps=1e-6, max_seqs=slots, max_ctx=64, budget_tokens=64 * slots, compute_dtype="fp32", layers=layers)
+    t = so.random_tensors(d, slots)
+    seqs = np.random.default_rng(slots).integers(0, 53, (slots, 5))
+    eng = SlotEngine(desc=d, tensors={k: v.astype(np.float32) for k, v in t.items()})
+    got = np.stack([eng.step([(i, [s[j]], [0]) for i, s in enumerate(seqs)]) for j in range(5)], 1)
+    eng.close()
+    for i in {0, slots // 2, slots - 1}:
+        want = so.forward(d, t, seqs[i].tolist())
+        assert np.abs(got[i] - want).max() / np.abs(want).max() < 1e-4, (slots, i)

@@ -226,9 +226,9 @@ struct LatentAppendArgs {
   float* ql;
 };
 template <int DT>
-__global__ __launch_bounds__(256) void latent_append_kernel(StepMeta m, LatentAppendArgs a) {
+__device__ __forceinline__ void latent_append_body(const StepMeta& m, const LatentAppendArgs& a, const int t) {
   // one wave, or several (each sums the squares for itself, the stores are dealt to all threads)
-  const int t = blockIdx.x, lane = threadIdx.x & 63, pos = m.tok_pos[t], nth = blockDim.x;
+  const int lane = threadIdx.x & 63, pos = m.tok_pos[t], nth = blockDim.x;
   const float* s = a.src + (size_t)t * a.lds + a.col0;
   float ss = 0.f;
   for (int c = lane; c < a.rank; c += 64) ss = fmaf(s[c], s[c], ss);
@@ -262,6 +262,8 @@ __global__ __launch_bounds__(256) void latent_append_kernel(StepMeta m, LatentAp
     } else a.ql[(size_t)t * a.heads * row_w + (size_t)(vec - 1) * row_w + a.rank + ch] = v * a.qscale;
   }
 }
+template <int DT>
+__global__ __launch_bounds__(256) void latent_append_kernel(StepMeta m, LatentAppendArgs a) { latent_append_body<DT>(m, a, blockIdx.x); }
 
 // ---- latent attention, one workgroup per (token, head): the four waves take every fourth key, lanes hold rank / 64 latent channels each.
 // Scores are fp32 dot products of the latent-space query (score scale folded in) with the cached latents; the softmax denominator also holds
@@ -569,9 +571,9 @@ __global__ void stack_gather_tok_kernel(int* tok_id, const int* ent_row, const i
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < S) tok_id[i] = slab_tok[ent_row[i]];
 }
-__global__ void stack_advance_kernel(int* tok_pos, int* ent_par, int* tok_par, int S) {      // one token per entry: token i is entry i
+__global__ void stack_advance_kernel(int* tok_id, const int* ent_row, const int* slab_tok, int* tok_pos, int* ent_par, int* tok_par, int S) {      // one token per entry: token i is entry i; the next step's token with it
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < S) { tok_pos[i] += 1; ent_par[i] ^= 1; tok_par[i] ^= 1; }
+  if (i < S) { tok_id[i] = slab_tok[ent_row[i]]; tok_pos[i] += 1; ent_par[i] ^= 1; tok_par[i] ^= 1; }
 }
 
 // ---- a step's wanted logits into their slots: row i of src (nullptr: already in the slot) becomes the current logits of slot rows[i] (-1: of none), and the per-workgroup

@@ -37,14 +37,15 @@ template <int DT, bool DUAL, int MB> constexpr size_t few_lds_bytes(int waves, i
 __device__ const u32x4 few_zeros = {0u, 0u, 0u, 0u};
 
 template <int DT, int EPI, bool DUAL, int MB>
-__global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_kernel(const StackGemmArgs a, const int depth) {
+__device__ __forceinline__ void stack_few_body(const StackGemmArgs& a, const int depth, const int z) {
   constexpr int NB = DUAL ? 2 : 1, WP = DT == DT_F32 ? 4 : 2;       // 1-KB pieces of a step's weight rows (per matrix)
   constexpr int PIECES = NB * WP + MB * 4, STEP = few_step_bytes<DT, DUAL, MB>();
   extern __shared__ __attribute__((aligned(1024))) unsigned char few_lds[];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
   const int li = lane & 15, q = lane >> 4;                          // row (column) of the operands, quarter of a half step's k
-  const int z = blockIdx.z, mbase = blockIdx.y * 16 * MB, mend = min(a.M, mbase + 16 * MB);
+  const int mbase = blockIdx.y * 16 * MB, mend = min(a.M, mbase + 16 * MB);
   const int n0 = blockIdx.x * 16, steps = (a.K + 63) >> 6;
+  if (n0 >= a.N) return;                                            // (the narrower product of a pair)
   unsigned char* ring = few_lds + (size_t)wv * depth * STEP;
   const unsigned ring_lds = (unsigned)(size_t)ring;
 
@@ -177,6 +178,32 @@ __global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_kernel(const
                        : total(std::integral_constant<int, few_max_waves(MB)>{}, b);
     sg_finish<EPI>(a, z, m, n, v[0], v[NB - 1]);
   }
+}
+
+template <int DT, int EPI, bool DUAL, int MB>
+__global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_kernel(const StackGemmArgs a, const int depth) { stack_few_body<DT, EPI, DUAL, MB>(a, depth, blockIdx.z); }
+// two products that do not need each other, of the same rows and contraction length, in one launch: blockIdx.z chooses (the low-rank pair of a channel-delta layer, sixteen rows of
+// 1024 x 128 each: 4.7 us and 4.7, 5.7 together)
+template <int DT, int MB>
+__global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_pair_kernel(const StackGemmArgs a, const StackGemmArgs b, const int depth) {
+  if (blockIdx.z == 0) stack_few_body<DT, SG_STORE, false, MB>(a, depth, 0);
+  else stack_few_body<DT, SG_STORE, false, MB>(b, depth, 0);
+}
+
+// Waves and ring depth: some eight waves a compute unit (2048 on the chip) and four a workgroup at least, never more than K has steps; two steps of each in flight, one
+// where the launch has a thousand workgroups that cover for each other.  Measured, us at waves / depth 4/1, 4/2, 8/1, 8/2, 16/1: sixteen rows 1024 x 1024 (64 workgroups):
+// 6.7, 5.9, 5.6, 5.6, 5.5; eight rows 2048 x 8192 (128): 36.6, 22.7, 23.3, 18.5, 18.8; 4096 x 2048 (256): 12.8, 9.3, 9.8, 8.8, 9.3; 8192 x 2048 (512): 15.1, 13.0, 14.0, 15.5,
+// 15.7; sixteen rows 24576 x 1024 (1536): 16.8, 17.7, 18.1, 26.7, 26.8
+struct FewPlan { int nw, depth; size_t lds; };
+template <int DT, bool DUAL, int MB>
+inline FewPlan few_plan(int num_cus, long long wgs, int K) {
+  const int steps = (K + 63) / 64;
+  FewPlan p{4, 1, 0};
+  while (p.nw < few_max_waves(MB) && wgs * p.nw < 8LL * num_cus) p.nw *= 2;
+  while (p.nw > 1 && p.nw > steps) p.nw /= 2;
+  p.depth = wgs >= 4LL * num_cus || p.nw >= steps ? 1 : 2;
+  while ((p.lds = few_lds_bytes<DT, DUAL, MB>(p.nw, p.depth)) > 160 * 1024) { if (p.depth > 1) p.depth--; else p.nw /= 2; }
+  return p;
 }
 
 }  // namespace tgx

@@ -17,11 +17,22 @@
 #include "kernels/stack_gqa_mfma.h"
 #include "kernels/stack_rec.h"
 #include "kernels/stack_step.h"
+#include "kernels/stack_few.h"
 #include "kernels/stack_loop.h"
 #include "kernels/stack_mix_mfma.h"
 #include "kernels/stack_ssm.h"
 #include "kernels/stack_ssd_mfma.h"
 #include "kernels/stack_hyper.h"
+
+namespace tgx {
+// A few tokens: the latents into the pool beside the queries into latent space (a product batched over the heads, kernels/stack_few.h): neither needs the other, attention needs both.
+// Four tokens, 8 heads of 256 x 128: 4.5 us and 4.4, 4.6 together.
+template <int DT>
+__global__ __launch_bounds__(64 * few_max_waves(1)) void latent_append_queries_kernel(StepMeta m, LatentAppendArgs la, StackGemmArgs a, const int depth, const int heads) {
+  if ((int)blockIdx.z < heads) stack_few_body<DT, SG_STORE, false, 1>(a, depth, blockIdx.z);
+  else for (int t = blockIdx.x; t < m.T; t += gridDim.x) latent_append_body<DT>(m, la, t);
+}
+}  // namespace tgx
 
 int upload_param_ext(tgx_ctx* c, ebyte* dst, const void* host, int64_t n, int src_dtype);      // abi.hip
 
@@ -407,12 +418,20 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
     launch_gemm(c, g, tgx::SG_STORE, 1);
     tgx::LatentAppendArgs la{};
     la.src = sm->proj; la.lds = nin; la.col0 = qd; la.nw = w.lat_norm; la.pool = w.pool; la.poolT = w.poolT; la.rank = R; la.eps = sm->d.norm_eps;
-    TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::latent_append_kernel<DT>, dim3(T), dim3(64), 0, c->stream, m, la))
     // queries into latent space, head by head: ql[t][h] = scale * q[t][h] . ukT[h]^T
     g = tgx::StackGemmArgs{};
     g.A = sm->proj; g.lda = nin; g.a_zoff = ld.dim; g.B = w.w_ukT; g.ldb = ld.dim; g.b_zstride = (long long)R * ld.dim; g.C = sm->ql; g.ldc = (long long)H * R; g.c_zoff = R;
     g.M = T; g.N = R; g.K = ld.dim; g.scale = ld.scale;
-    launch_gemm(c, g, tgx::SG_STORE, H);
+    if (sm->gemv && T > GEMV_ROWS_MAX && T <= 16 && slices_ok(g)) {
+      g.terms = c->act16 ? 1 : 2;
+      const dim3 grid((R + 15) / 16, 1, H + 1);
+      TGX_DT_SWITCH(c->dt,
+        const tgx::FewPlan p = tgx::few_plan<DT, false, 1>(c->num_cus, (long long)grid.x * H, g.K);
+        if (stack_allow_lds(c, (const void*)&tgx::latent_append_queries_kernel<DT>, p.lds)) hipLaunchKernelGGL(tgx::latent_append_queries_kernel<DT>, grid, dim3(64 * p.nw), p.lds, c->stream, m, la, g, p.depth, H);)
+    } else {
+      TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::latent_append_kernel<DT>, dim3(T), dim3(64), 0, c->stream, m, la))
+      launch_gemm(c, g, tgx::SG_STORE, H);
+    }
     tgx::LatentAttnArgs aa{};
     aa.q = sm->ql; aa.ldq = (long long)H * R; aa.pool = w.pool; aa.sink = w.sink; aa.out = sm->lat; aa.ldo = (long long)H * R; aa.rank = R; aa.heads = H;
     if (w.poolT && sm->attn_mfma) {
@@ -1869,10 +1888,16 @@ void run_channel_delta(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T
   g = tgx::StackGemmArgs{};
   g.A = sm->proj + k.a1; g.lda = ldp; g.B = w.w_w2; g.ldb = ld.decay_rank; g.C = sm->mixed; g.ldc = k.HD; g.M = T; g.N = k.HD; g.K = ld.decay_rank; g.scale = 1.f; g.bias = w.dt_bias;
   g.act = tgx::SG_ACT_HEAD_DECAY; g.a_log = w.a_log; g.head_cols = ld.dim;
-  launch_gemm(c, g, tgx::SG_STORE, 1);
+  tgx::StackGemmArgs gd = g;
   g = tgx::StackGemmArgs{};
   g.A = sm->proj + k.g1; g.lda = ldp; g.B = w.w_g2; g.ldb = ld.gate_rank; g.C = sm->lora; g.ldc = k.HE; g.M = T; g.N = k.HE; g.K = ld.gate_rank; g.scale = 1.f;
-  launch_gemm(c, g, tgx::SG_STORE, 1);
+  if (sm->gemv && T > GEMV_ROWS_MAX && T <= FEW_ROWS_MAX && gd.K == g.K && slices_ok(gd) && slices_ok(g)) {
+    gd.terms = g.terms = c->act16 ? 1 : 2;
+    launch_stack_few_pair(c, gd, g, c->dt);
+  } else {
+    launch_gemm(c, gd, tgx::SG_STORE, 1);
+    launch_gemm(c, g, tgx::SG_STORE, 1);
+  }
   // rec_in row = [q | k | v | beta]
   tgx::DeltaPrepArgs dp{};
   dp.proj = sm->proj; dp.ldp = ldp; dp.b_col = k.b; dp.cw = w.conv_w; dp.out = sm->rec_in; dp.ldo = ldr; dp.state = nb > 0 ? w.conv_state : nullptr;
@@ -3257,12 +3282,12 @@ int stack_decode(tgx_ctx* c, const tgx_sampler_cfg& cfg, uint64_t seed, int n) {
   for (int b = 0; b < c->batch; b++) { c->row_probs_cfg[(size_t)b] = cfg; c->row_probs_ok[(size_t)b] = is_greedy(&cfg) ? 0 : 1; }
   c->have_probs = !is_greedy(&cfg);
   for (int s = 0; s < n; s++) {
-    hipLaunchKernelGGL(tgx::stack_gather_tok_kernel, dim3((S + 63) / 64), dim3(64), 0, c->stream, dp.tok_id, dp.ent_row, c->slab_tok, S);
+    if (s == 0) hipLaunchKernelGGL(tgx::stack_gather_tok_kernel, dim3((S + 63) / 64), dim3(64), 0, c->stream, dp.tok_id, dp.ent_row, c->slab_tok, S);
     if ((rc = run_layers(c, dp, S, S, max_keys + s + 1, 1))) return half_way(c, rc);
     run_logits(c, dp.want, S, c->slab_logits, dp.want_row);
     launch_slot_logits(c, nullptr, dp.want_row, S);
     launch_sample(c, 0, c->batch, cfg, /*advance_pos=*/true, /*log_step=*/true);
-    hipLaunchKernelGGL(tgx::stack_advance_kernel, dim3((S + 63) / 64), dim3(64), 0, c->stream, dp.tok_pos, dp.ent_par, dp.tok_par, S);
+    hipLaunchKernelGGL(tgx::stack_advance_kernel, dim3((S + 63) / 64), dim3(64), 0, c->stream, dp.tok_id, dp.ent_row, c->slab_tok, dp.tok_pos, dp.ent_par, dp.tok_par, S);
     c->steps_issued++;
     if (c->launch_fault) return half_way(c, TGX_OK);
   }

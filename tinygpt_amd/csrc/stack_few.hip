@@ -5,24 +5,17 @@
 #include "kernels/stack_few.h"
 
 namespace {
-constexpr size_t LDS_BYTES = 160 * 1024;
-
 template <int DT, int EPI, bool DUAL, int MB>
 void launch_few_mb(tgx_ctx* c, const tgx::StackGemmArgs& a, dim3 grid) {
-  // Waves and ring depth: some eight waves a compute unit (2048 on the chip) and four a workgroup at least, never more than K has steps; two steps of each in flight, one
-  // where the launch has a thousand workgroups that cover for each other.  Measured, us at waves / depth 4/1, 4/2, 8/1, 8/2, 16/1: sixteen rows 1024 x 1024 (64 workgroups):
-  // 6.7, 5.9, 5.6, 5.6, 5.5; eight rows 2048 x 8192 (128): 36.6, 22.7, 23.3, 18.5, 18.8; 4096 x 2048 (256): 12.8, 9.3, 9.8, 8.8, 9.3; 8192 x 2048 (512): 15.1, 13.0, 14.0, 15.5,
-  // 15.7; sixteen rows 24576 x 1024 (1536): 16.8, 17.7, 18.1, 26.7, 26.8
-  const long long wgs = (long long)grid.x * grid.y * grid.z;
-  const int steps = (a.K + 63) / 64;
-  int nw = 4;
-  while (nw < tgx::few_max_waves(MB) && wgs * nw < 8LL * c->num_cus) nw *= 2;
-  while (nw > 1 && nw > steps) nw /= 2;
-  int depth = wgs >= 4LL * c->num_cus || nw >= steps ? 1 : 2;
-  while (tgx::few_lds_bytes<DT, DUAL, MB>(nw, depth) > LDS_BYTES) { if (depth > 1) depth--; else nw /= 2; }
-  const size_t lds = tgx::few_lds_bytes<DT, DUAL, MB>(nw, depth);
-  if (!stack_allow_lds(c, (const void*)&tgx::stack_few_kernel<DT, EPI, DUAL, MB>, lds)) return;
-  hipLaunchKernelGGL((tgx::stack_few_kernel<DT, EPI, DUAL, MB>), grid, dim3(64 * nw), lds, c->stream, a, depth);
+  const tgx::FewPlan p = tgx::few_plan<DT, DUAL, MB>(c->num_cus, (long long)grid.x * grid.y * grid.z, a.K);
+  if (!stack_allow_lds(c, (const void*)&tgx::stack_few_kernel<DT, EPI, DUAL, MB>, p.lds)) return;
+  hipLaunchKernelGGL((tgx::stack_few_kernel<DT, EPI, DUAL, MB>), grid, dim3(64 * p.nw), p.lds, c->stream, a, p.depth);
+}
+template <int DT, int MB>
+void launch_few_pair_mb(tgx_ctx* c, const tgx::StackGemmArgs& a, const tgx::StackGemmArgs& b, dim3 grid) {
+  const tgx::FewPlan p = tgx::few_plan<DT, false, MB>(c->num_cus, (long long)grid.x * grid.y * grid.z, a.K);
+  if (!stack_allow_lds(c, (const void*)&tgx::stack_few_pair_kernel<DT, MB>, p.lds)) return;
+  hipLaunchKernelGGL((tgx::stack_few_pair_kernel<DT, MB>), grid, dim3(64 * p.nw), p.lds, c->stream, a, b, p.depth);
 }
 template <int DT, int EPI, bool DUAL>
 void launch_few_t(tgx_ctx* c, const tgx::StackGemmArgs& a, dim3 grid, int mb) {
@@ -33,6 +26,16 @@ void launch_few_t(tgx_ctx* c, const tgx::StackGemmArgs& a, dim3 grid, int mb) {
   }
 }
 }  // namespace
+
+// two stored products of up to 64 rows, the same for both, and of one contraction length
+void launch_stack_few_pair(tgx_ctx* c, const tgx::StackGemmArgs& a, const tgx::StackGemmArgs& b, int dt) {
+  const int mb = a.M <= 16 ? 1 : a.M <= 32 ? 2 : 4;
+  const dim3 grid((std::max(a.N, b.N) + 15) / 16, 1, 2);
+  TGX_DT_SWITCH(dt,
+    if (mb == 1) launch_few_pair_mb<DT, 1>(c, a, b, grid);
+    else if (mb == 2) launch_few_pair_mb<DT, 2>(c, a, b, grid);
+    else launch_few_pair_mb<DT, 4>(c, a, b, grid);)
+}
 
 void launch_stack_few(tgx_ctx* c, const tgx::StackGemmArgs& a, int epi, int nz, int dt) {
   // sixteen-row operands: all rows of a step in one workgroup up to 64 (the weights cross once); many rows of a narrow matrix (a router's) in sixteens, which spreads
