@@ -490,7 +490,8 @@ TGX_API int tgx_set_logits(tgx_ctx* ctx, const float* logits, int batch);
  *                  tokens divides them between workgroups (four thresholds: 128 on the matrix cores, 2048 on the lane kernels for latent rows, 1024 for grouped queries, counted in a
  *                  mask's span.  The first key sets all four, the second the grouped-query ones; a negative value brings the defaults back; tgx_get_option gives the
  *                  one in force, the matrix cores' where any layer's attention runs there);
- *                  0 = lane attention kernels only; 0 = few-row products on the matrix-core tiles too; 0 = prompts' products on the register-staged tiles; forced product tile; the mLSTM scan's column split;
+ *                  0 = lane attention kernels only; 0 = few-row products on the matrix-core tiles too; 0 = a single token's recurrence or attention over few keys in the launches of a longer portion;
+ *                  0 = prompts' products on the register-staged tiles; forced product tile; the mLSTM scan's column split;
  *                  key / value heads per workgroup of the matrix-core sigmoid attention (1; 2 = two where their accumulators fit; 0 = two while the halved grid fills the chip);
  *                  tokens of a portion from which a scalar-decay recurrence runs in blocks on the matrix cores (0 = never)
  *   "stack.ws_max" (layered models) most KiB of each scratch buffer that divided keys, blocked recurrences and prompts' products ask for (-1: as memory allows); what would need more,

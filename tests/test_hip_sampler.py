@@ -142,3 +142,19 @@ def test_staged_sampler_many_workgroups_vs_oracle(V, oracle_lib):
                         np.testing.assert_allclose(probs[row], want, rtol=5e-5, atol=1e-9)
                         assert int(a[row]) == int(b[row])
                     assert probs[row][int(a[row])] > 0
+
+
+@pytest.mark.parametrize("vocab", [65536, 65537])
+def test_results_of_several_pinned_halves(vocab):
+    """Logits of less than one pinned half of 1 MB, of exactly one and two, and of several with a rest, as they were given, twice."""
+    from tinygpt_amd.ffi import Model, product_backend
+    cfg, _ = load_golden("llama_tiny")
+    m = Model(desc_from_hf_config(dict(cfg, vocab_size=vocab), "bf16", max_batch=13), product_backend()).load_synthetic(7, 0.05).finalize()
+    rng = np.random.default_rng(vocab)
+    for rows in (1, 4, 5, 8, 9, 13):
+        want = rng.standard_normal((rows, vocab), dtype=np.float32)
+        m.set_logits(want)
+        for _ in range(2):
+            np.testing.assert_array_equal(m.logits(rounded=False), want)
+        np.testing.assert_array_equal(m.sample(), want.argmax(1))
+    m.close()

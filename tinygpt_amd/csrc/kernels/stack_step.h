@@ -206,7 +206,7 @@ __global__ __launch_bounds__(1024) void rec_step_kernel(StepMeta m, RecStepArgs 
 //   softmax  a wave per query head, base 2, as in gqa_attn_mfma_kernel (cap, distance slope, sink, mask)
 //   values   a key per wave at a time, a lane's channels of all query heads; the waves' sums meet in LDS
 // Queries and probabilities stay fp32 (the matrix forms take them as two 16-bit terms).
-// Measured, us: one stream of 50 to 95 keys, two key / value heads of 128 x 128 8.4 (append 3.0, undivided walk 7.9); beside a delta rule in one launch 9.1 (7.4 of the rule's own).
+// Measured, us: one stream of 50 to 95 keys, two key / value heads of 128 x 128 7.9 (append 3.0, undivided walk 7.9; 8.4 with the columns of a row found by divisions); beside a delta rule in one launch 9.0 (7.4 of the rule's own).
 constexpr int STEP_MAX_KEYS = 256, STEP_MAX_GROUP = 4, STEP_MAX_VDIM = 128;
 struct GqaStepArgs {
   GqaAppendArgs ap;          // the token's row (maps 1, no q_hi, no qk_unit_eps)
@@ -256,24 +256,25 @@ __device__ __forceinline__ void gqa_step_body(const StepMeta& m, const GqaStepAr
   // the token's queries (score scale and log2 e folded in), key and value
   const bool capped = a.softcap > 0.f;
   const float temp = ap.q_temp_coef != 0.f ? fmaf(ap.q_temp_coef, logf((float)((pos + 1) / ap.q_temp_every) + 1.0f), 1.0f) : 1.0f, qscale = capped ? a.scale : a.scale * LOG2E;
-  for (int i = tid; i < (Gq + 1) * dim; i += 1024) {
-    const int r = i / dim, c = i - r * dim;
-    if (r == Gq && !fresh_key) break;
-    const float* u = prow + (r < Gq ? (size_t)(g * Gq + r) * dim : (size_t)ap.heads * dim + (size_t)g * dim);
-    float v = u[c];
-    if (c < ap.rot_dims) {
-      const int half = ap.rot_dims >> 1, p = ap.rot_pairs ? c >> 1 : c < half ? c : c - half;
-      const bool first = ap.rot_pairs ? (c & 1) == 0 : c < half;
-      const float cs = ap.cs[((size_t)pos * half + p) * 2], sn = ap.cs[((size_t)pos * half + p) * 2 + 1], o = u[ap.rot_pairs ? c ^ 1 : first ? c + half : c - half];
-      v = first ? __fsub_rn(__fmul_rn(v, cs), __fmul_rn(o, sn)) : __fadd_rn(__fmul_rn(v, cs), __fmul_rn(o, sn));
+  const int nq = Gq + (fresh_key ? 1 : 0);
+  if (wv < 2 * nq)                                                 // two waves a row
+    for (int c = lane + 64 * (wv & 1); c < dim; c += 128) {
+      const int r = wv >> 1;
+      const float* u = prow + (r < Gq ? (size_t)(g * Gq + r) * dim : (size_t)ap.heads * dim + (size_t)g * dim);
+      float v = u[c];
+      if (c < ap.rot_dims) {
+        const int half = ap.rot_dims >> 1, p = ap.rot_pairs ? c >> 1 : c < half ? c : c - half;
+        const bool first = ap.rot_pairs ? (c & 1) == 0 : c < half;
+        const float cs = ap.cs[((size_t)pos * half + p) * 2], sn = ap.cs[((size_t)pos * half + p) * 2 + 1], o = u[ap.rot_pairs ? c ^ 1 : first ? c + half : c - half];
+        v = first ? __fsub_rn(__fmul_rn(v, cs), __fmul_rn(o, sn)) : __fadd_rn(__fmul_rn(v, cs), __fmul_rn(o, sn));
+      }
+      if (r < Gq) s_qr[r][c] = v * temp * qscale;
+      else {
+        const elem_t<DT> k = f32_to_elem<DT>(v);
+        reinterpret_cast<elem_t<DT>*>(ap.poolK)[(((size_t)tbl[pos >> m.page_shift] << m.page_shift) + (size_t)(pos & pmask)) * kd + (size_t)g * dim + c] = k;
+        s_kn[c] = elem_to_f32<DT>(k);
+      }
     }
-    if (r < Gq) s_qr[r][c] = v * temp * qscale;
-    else {
-      const elem_t<DT> k = f32_to_elem<DT>(v);
-      reinterpret_cast<elem_t<DT>*>(ap.poolK)[(((size_t)tbl[pos >> m.page_shift] << m.page_shift) + (size_t)(pos & pmask)) * kd + (size_t)g * dim + c] = k;
-      s_kn[c] = elem_to_f32<DT>(k);
-    }
-  }
   if (fresh_key && tid < vdim) {
     const size_t at = (size_t)e * vd + (size_t)g * vdim + tid;
     float v = prow[(size_t)ap.heads * dim + kd + (size_t)g * vdim + tid];
@@ -355,8 +356,8 @@ __device__ __forceinline__ void gqa_step_body(const StepMeta& m, const GqaStepAr
 #pragma unroll
     for (int c = 0; c < 2; c++) if (lane + 64 * c < STEP_MAX_VDIM) s_acc[wv][r][lane + 64 * c] = acc[r][c];
   __syncthreads();
-  for (int i = tid; i < Gq * vdim; i += 1024) {
-    const int r = i / vdim, c = i - r * vdim;
+  const int r = tid >> 7, c = tid & 127;                           // (STEP_MAX_VDIM columns a head)
+  if (r < Gq && c < vdim) {
     const size_t hc = (size_t)(g * Gq + r) * vdim + c;
     float t[16];
 #pragma unroll
