@@ -319,3 +319,25 @@ def test_products_of_pairs(rows, experts, top, width, ff):
     eng.close()
     want = so.forward(d, t, toks)
     assert np.abs(got - want).max() / np.abs(want).max() < 1e-4, (rows, experts, width)
+
+
+# ---- norms that write the next products' terms themselves: the same two terms as the split in front of each product, so the same bits.  A limit on scratch that holds every product's
+# own terms and hidden rows, but not a norm's lines beside them, leaves the split.  (T 4161: 33 row tiles, the last of one row; widths of one line, five and sixteen)
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("width", [64, 320, 1024])
+@pytest.mark.parametrize("design", ["vitudra", "nusovik"])
+def test_terms_of_a_norm(design, width, dtype):
+    import test_hip_nusovik as tn
+    T, ff = 4161, 1344
+    heads = dict(heads=8, kv_heads=4, dim=32, vdim=32)
+    half = dict(heads=4, kv_heads=2, dim=32, vdim=32)
+    t, layers = {"vitudra": (tv, [tv.par(tv.ff(ff), left=heads, right=half), tv.wkv(tv.ff(ff), heads=2, dim=32), tv.attn(tv.ff(ff), **heads), tv.attn()]),
+                 "nusovik": (tn, [tn.mamba(tn.ff(ff), inner=256), tn.par(tn.ff(ff), left=heads, right=dict(heads=4, state=32, vdim=32)), tn.par(left=heads), tn.mamba(inner=256)])}[design]
+    cfg = t.config(layers, width=width)
+    eng, _ = t.engine(cfg, dtype, max_seqs=1, max_ctx=T, budget_tokens=T + 64)
+    ids, want, got = np.array(t.tokens(cfg, T)), [0, 63, 64, 127, 128, 2000, T - 2, T - 1], []
+    for limit in (T * 4 * (max(ff, 4 * width) + width // 2) // 1024, -1):
+        eng.model.set_option("stack.ws_max", limit)
+        got.append(eng.step([("p", ids, want)], ["p"]))
+    eng.close()
+    assert np.isfinite(got[0]).all() and (got[0] == got[1]).all()

@@ -57,6 +57,13 @@ template <int DT> __device__ __forceinline__ elem_t<DT> f32_to_elem(float f) {  
   else if constexpr (DT == DT_F16) return f32_to_f16_bits(f);
   else return f;
 }
+// x = hi + lo with hi = round16(x), lo = round16(x - hi) in the 16-bit storage dtype DT (bf16: 16 significant bits in two
+// terms; fp16: 22, with an absolute floor of 2^-25 where lo goes subnormal)
+template <int DT>
+__device__ __forceinline__ void split16(float x, bf16_t& hi, bf16_t& lo) {
+  hi = f32_to_elem<DT>(x);
+  lo = f32_to_elem<DT>(x - elem_to_f32<DT>(hi));
+}
 // two adjacent 16-bit elements packed in one dword -> fp32
 template <int DT> __device__ __forceinline__ float pair_lo(unsigned int u) {
   if constexpr (DT == DT_BF16) return bf16_lo(u); else return f16_bits_to_f32((unsigned short)(u & 0xffffu));

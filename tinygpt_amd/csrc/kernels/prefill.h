@@ -32,14 +32,6 @@ __device__ __forceinline__ f32x16 mfma16(bf16x8 a, bf16x8 b, f32x16 c) {
   else return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// x = hi + lo with hi = round16(x), lo = round16(x - hi) in the 16-bit storage dtype DT (bf16: 16 significant bits in two
-// terms; fp16: 22, with an absolute floor of 2^-25 where lo goes subnormal)
-template <int DT>
-__device__ __forceinline__ void split16(float x, bf16_t& hi, bf16_t& lo) {
-  hi = f32_to_elem<DT>(x);
-  lo = f32_to_elem<DT>(x - elem_to_f32<DT>(hi));
-}
-
 // silu(g) * u and gelu_new(v) = v * sigmoid(2 y) with the hardware exp2 / rcp (1 ulp each, ~2e-7 relative).  The MFMA prefill epilogues run them
 // for every output element — with expf + an IEEE division (~35 instructions) the epilogue of a 256 x 256 tile issued as many instructions as
 // its whole K loop; the value is rounded to two 16-bit terms (2^-17) right after.

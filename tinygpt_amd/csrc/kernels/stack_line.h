@@ -2,7 +2,7 @@
 //
 // What bounded them: stack_gemm_kernel brings every operand byte through registers (fp32 activations split into two 16-bit terms by every column tile again) with two
 // barriers a step, on 64 x 64 or 128 x 128 tiles: 0.65 PFLOP/s executed on 11264 x 8192 x 2048, where the flat families' kernels reach 1.2.  Here the activations are split
-// ONCE into lines [row][K / 32][32 first terms | 32 second terms] (split_terms_kernel, or the epilogue of the product in front), so that the two terms of a k32 block are one
+// ONCE into lines [row][K / 32][32 first terms | 32 second terms] (split_terms_kernel, the norm in front, or the epilogue of the product in front), so that the two terms of a k32 block are one
 // line, weights come as whole k64 lines, and the tiles are those of gemm_dma.h:
 //   256 x 256, eight waves of 64 x 128, a ring of five 32-KB units (gemm_dma8i_kernel's schedule): products that fill the chip with such tiles
 //   128 x 128, eight waves = two row halves x the four k16 steps of a stage, a ring of three 48-KB stages (gemm_dma8k_kernel's): the others

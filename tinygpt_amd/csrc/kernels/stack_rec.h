@@ -18,7 +18,7 @@
 namespace tgx {
 
 // out[i] = x[rows ? rows[i] : i] / sqrt(mean(row^2) + eps) * (offset + w)
-__global__ __launch_bounds__(256) void offset_norm_kernel(const float* x, const int* rows, const float* w, float offset, float* out, int W, float eps) {
+__global__ __launch_bounds__(256) void offset_norm_kernel(const float* x, const int* rows, const float* w, float offset, float* out, int W, float eps, RowTerms terms) {
   __shared__ float s4[4];
   const float* xr = x + (size_t)(rows ? rows[blockIdx.x] : blockIdx.x) * W;
   float* o = out + (size_t)blockIdx.x * W;
@@ -36,6 +36,7 @@ __global__ __launch_bounds__(256) void offset_norm_kernel(const float* x, const 
     for (int k = 0; k < ROW_REG; k++) {
       for (int u = 0; u < 4; u++) v[k][u] = v[k][u] * r * (offset + wv[k][u]);
       row_store<true>(o, k, W, v[k]);
+      if (terms.out) row_store_terms(terms, blockIdx.x, k, W, v[k]);
     }
     return;
   }

@@ -648,8 +648,7 @@ __device__ __forceinline__ void router_group_body(RouterGroupArgs a) {
   if (a.shared && lane == 0) { a.sel[(size_t)t * stride + a.top] = a.E; a.selw[(size_t)t * stride + a.top] = 1.f; }
   if (a.sgw && lane == 0) a.sgw[t] = 1.0f / (1.0f + expf(-z[a.E]));
 }
-template <bool PRODUCT>
-__global__ __launch_bounds__(PRODUCT ? 256 : 64) void router_group_kernel(RouterGroupArgs a) { router_group_body<PRODUCT>(a); }
+__global__ __launch_bounds__(64) void router_group_kernel(RouterGroupArgs a) { router_group_body<false>(a); }
 // a few tokens' seam with the choice of experts behind it (as norm_conv_route_kernel)
 template <int NR>
 __global__ __launch_bounds__(256) void sandwich_route_kernel(SandwichArgs a, RouterGroupArgs r) {

@@ -13,7 +13,7 @@
 namespace tgx {
 
 // ---- x[t] += y[t] / sqrt(mean(y[t]^2) + eps) * w.  One workgroup per token; widths up to 256 * 4 * POST_REG (in whole vectors of four) stay in registers.
-struct PostNormArgs { float* x; const float* y; const float* w; int W; float eps; };
+struct PostNormArgs { float* x; const float* y; const float* w; int W; float eps; RowTerms terms; };
 constexpr int POST_REG = 4;
 __global__ __launch_bounds__(256) void post_norm_add_kernel(PostNormArgs a) {
   __shared__ float s4[4];
@@ -43,6 +43,7 @@ __global__ __launch_bounds__(256) void post_norm_add_kernel(PostNormArgs a) {
 #pragma unroll
       for (int u = 0; u < 4; u++) xv[k][u] = fmaf(v[k][u] * r, wv[k][u], xv[k][u]);
       *reinterpret_cast<f32x4*>(x + c) = xv[k];
+      if (a.terms.out) row_store_terms(a.terms, t, k, a.W, xv[k]);
     }
     return;
   }

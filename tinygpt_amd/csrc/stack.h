@@ -130,12 +130,14 @@ struct StackModel {
   size_t part_elems = 0;
   unsigned short *terms = nullptr, *terms2 = nullptr;      // prompt products: the activations as lines of two 16-bit terms, and a feed-forward's hidden values (grown to the largest product seen)
   size_t terms_elems = 0, terms2_elems = 0;
+  const unsigned short* in_terms = nullptr; size_t in_terms_elems = 0;      // the rows that the last norm wrote as such lines, at the start of terms (nullptr: it did not; norms in front of such products set it anew)
   int *sel = nullptr, *moe_off = nullptr, *perm = nullptr, *ptok = nullptr, *tile_e = nullptr, *tile_m0 = nullptr, *n_tiles = nullptr;
   int max_in = 0, max_hr = 0, max_hv = 0, max_top = 0, max_ff = 0, max_E = 0, max_rank = 0;
   // Steps of few tokens split a sequence's keys between workgroups from these contexts on (option attn.split_min sets all four, attn.gqa_split_min the grouped-query ones, which
   // count the keys that a workgroup would walk: a mask's span; a negative value brings these defaults back).  Matrix-core kernels: an undivided workgroup walks its keys tile by tile, 1.3 us for 32 latent rows, 0.9 us for 64
   // keys; a merge costs 4 to 5 us and a divided walk two tiles.  A decoded token's step at width 1024 and six layers, undivided -> divided: latent attention, four requests at 96 /
-  // 160 / 256 / 1000 keys 627 -> 630, 646 -> 628, 675 -> 632, 872 -> 648 us; grouped-query, sixteen requests 691 -> 688, 702 -> 687, 704 -> 687, 786 -> 695
+  // 160 / 256 / 1000 keys 627 -> 630, 646 -> 628, 675 -> 632, 872 -> 648 us; grouped-query, sixteen requests 691 -> 688, 702 -> 687, 704 -> 687, 786 -> 695 (where gqa_step_kernel does
+  // not take the step: single tokens of up to 256 keys, kernels/stack_step.h)
   static constexpr int MFMA_SPLIT_MIN = 128, LATENT_LANE_SPLIT_MIN = 2048, GQA_LANE_SPLIT_MIN = 1024;
   int latent_split_min_keys = MFMA_SPLIT_MIN, gqa_split_min_keys = MFMA_SPLIT_MIN;
   int attn_split_min_keys = LATENT_LANE_SPLIT_MIN, gqa_lane_split_min_keys = GQA_LANE_SPLIT_MIN;      // ... lane kernels
@@ -155,6 +157,7 @@ struct StackModel {
   int mix_groups = 0;                  // option attn.mix_groups: key / value heads per workgroup of the matrix-core sigmoid attention: 1; 2 where their accumulators fit, whatever the grid; 0: 2 while the halved grid fills the chip
   std::set<const void*> lds_kernels;   // kernels that may take the whole LDS of a compute unit on this context's device
   size_t part_ask = 0, terms_cols = 0, terms2_cols = 0;      // what part can come to hold for divided keys; elements of one term that a token's row of terms and terms2 can come to hold (scratch_sizes)
+  size_t terms_most = 0;               // ... of any product's input, whichever form it takes
   size_t ws_refused = SIZE_MAX;        // bytes that this step has asked for in vain
   int ws_grown = 0;                    // tgx_get_option stack.ws_grown: how often part, terms and terms2 were allocated
   int ws_max = -1;                     // option stack.ws_max: most KiB of each of part, terms and terms2 (-1: as memory allows); products, attention and recurrences that would need more take their forms without scratch

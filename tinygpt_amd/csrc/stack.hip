@@ -4,8 +4,8 @@
 // One step = T tokens of S entries (a portion of a prompt, or one decoded token, per sequence slot).  Per layer:
 //   norm_conv (norm1, canon1) -> one product for [queries | latent | gate] -> latent norm + pool append -> queries into latent space (per head)
 //   -> latent attention over the pool -> value up-projection with the sigmoid gate in its epilogue -> output product added to the stream
-//   -> norm_conv (norm2, canon2) -> router top-k -> grouped expert products (gate / up with the activation, down with the router weight)
-//   -> combine + depth average.
+//   -> norm_conv (norm2, canon2) -> router top-k (few tokens: in the same launch) -> expert products (gate / up with the activation, down with the router weight)
+//   -> combine + depth average (single tokens: the next layer's norm1 and canon1 behind it).
 // Attention reads every key from the pool — also the keys of the step's own tokens, appended before it runs — so a position's result does not depend
 // on how its sequence was cut into steps.  The residual stream, norms, scores and the router are fp32; the matrices and the pool are in the storage dtype.
 #include "stack.h"
@@ -138,21 +138,28 @@ bool ensure_scratch(tgx_ctx* c, E*& p, size_t& have, size_t need, size_t ask) {
   return true;
 }
 bool ensure_part(tgx_ctx* c, size_t need, size_t ask = 0) { StackModel* sm = c->stack; return ensure_scratch(c, sm->part, sm->part_elems, need, std::max(ask, sm->part_ask)); }
-bool ensure_terms(tgx_ctx* c, size_t need) { StackModel* sm = c->stack; return ensure_scratch(c, sm->terms, sm->terms_elems, need, 2 * (size_t)sm->cap_tokens * sm->terms_cols); }
+// (behind a norm's lines; the buffer does not grow while these stand in it: norm_terms asked for all that the step can come to need)
+bool ensure_terms(tgx_ctx* c, size_t need) {
+  StackModel* sm = c->stack;
+  if (sm->in_terms) return sm->in_terms_elems + need <= sm->terms_elems;
+  return ensure_scratch(c, sm->terms, sm->terms_elems, need, 2 * (size_t)sm->cap_tokens * (sm->joint || sm->post ? sm->terms_most + sm->d.width : sm->terms_cols));
+}
 bool ensure_terms2(tgx_ctx* c, size_t need) { StackModel* sm = c->stack; return ensure_scratch(c, sm->terms2, sm->terms2_elems, need, 2 * (size_t)sm->cap_tokens * sm->terms2_cols); }
 // what those buffers can come to hold: the sums of the divided keys of any step (tiles of up to 32 rows on twice as many workgroups as there are compute units, a value or
 // latent row and two numbers each; or a token's outputs, heads in a row), and a token's widest product input and hidden row
 void scratch_sizes(tgx_ctx* c) {
   StackModel* sm = c->stack;
-  int cols = std::max({sm->d.width * (sm->affine ? 2 : 1), sm->max_hv, sm->max_hr});
+  int cols = std::max({sm->d.width * (sm->affine ? 2 : 1), sm->max_hv, sm->max_hr}), most = 0;
   for (const StackLayerW& w : sm->L) {
     const tgx_layer_desc& l = w.d;
     const size_t row = (size_t)std::max(l.kv_rank + l.rot_dim, l.vdim) + 2;
     if (sm->affine || w.pool) sm->part_ask = std::max(sm->part_ask, 2 * (size_t)c->num_cus * std::max(32 * row, (size_t)l.heads * l.vdim));
     cols = std::max(cols, l.mixer == TGX_MIXER_WKV ? 4 * sm->d.width : 0);      // (one split of four of the token shift's five mixes)
+    most = std::max({most, l.heads * std::max(l.dim, l.kv_rank), l.heads * l.vdim + l.d_heads * l.d_vdim, l.inner, l.ff, l.shared_ff, l.decay_rank, l.gate_rank, l.dt_rank});
     sm->terms2_cols = std::max(sm->terms2_cols, (size_t)(l.mlp == TGX_MLP_MOE ? std::max(l.top * l.ff, l.shared_ff) : l.ff));
   }
   sm->terms_cols = (size_t)cols;
+  sm->terms_most = (size_t)std::max(cols, most);
 }
 // rows per tile of the two grouped products of an expert layer's plan (both must be able to take them: their contraction lengths are the width and the expert width); 0: no plan,
 // the pairs' kernel.  np: (token, expert) pairs, E: experts, up_n: columns of the first product (gate and up together)
@@ -173,6 +180,23 @@ int line_tile(const tgx_ctx* c, const tgx::StackGemmArgs& a, int epi, int nz, in
   if (nz > 1 && (a.a_zoff % 32 || a.K < 256)) return 0;      // (per-head products of one head's width: two or four steps of K do not fill the ring)
   if (a.M <= FEW_ROWS_MAX || a.N <= FEW_COLS_ANY_ROWS) return 0;
   return stack_line_tile(c, a.M, a.N, tgx::sg_dual(epi), nz);
+}
+
+// whether the norm in front of a product of T rows of the stream, N columns (of each matrix of a dual one), writes its rows as terms too, and where: the product takes the line kernels
+// and the row stays in the norm's registers.  Passes in turn on one card, with a split in front of every product / so: a 2048-token Vitudra prompt, whose norm feeds two products,
+// 9735 / 9462 us (splits 30 of 8.4 us / 17, norms 8.4 / 9.6), eight Nusovik documents 29774 / 29317; Modepel's seams, whose products share rows only in front of experts, 6623 / 6622:
+// they keep the split
+tgx::RowTerms norm_terms(tgx_ctx* c, int T, int N, bool dual) {
+  StackModel* sm = c->stack;
+  const int W = sm->d.width;
+  sm->in_terms = nullptr;
+  tgx::RowTerms t{};
+  if (!sm->line || sm->gemm_wt || c->dt == tgx::DT_F32 || W % 64 || W > 1024 * tgx::ROW_REG || T <= FEW_ROWS_MAX) return t;
+  if (N <= FEW_COLS_ANY_ROWS || !stack_line_tile(c, T, N, dual, 1)) return t;
+  if (!ensure_terms(c, 2 * (size_t)T * (sm->terms_most + W))) return t;
+  t.out = sm->terms; t.half = c->dt == tgx::DT_F16; t.one_term = c->act16 ? 1 : 0;
+  sm->in_terms = sm->terms; sm->in_terms_elems = 2 * (size_t)T * W;
+  return t;
 }
 
 // operands that the weight-streaming kernels' loads take: whole 8-element slices
@@ -201,8 +225,9 @@ void launch_gemm(tgx_ctx* c, tgx::StackGemmArgs a, int epi, int nz, int grouped_
   if (tile) {
     const int cols = a.K + a.a_zoff * (nz - 1), rows = a.a_rows ? a.a_count : a.M;
     if (!a.At && ensure_terms(c, (size_t)rows * 2 * cols)) {
-      launch_split_terms(c, a.A, a.lda, rows, cols, c->stack->terms);
-      a.At = c->stack->terms;
+      unsigned short* at = sm->terms + (sm->in_terms ? sm->in_terms_elems : 0);
+      launch_split_terms(c, a.A, a.lda, rows, cols, at);
+      a.At = at;
     }
     if (a.At) { launch_stack_line(c, a, epi, nz, tile, a.z_off ? grouped_rows / tile + std::min(groups, grouped_rows) : (a.M + tile - 1) / tile, a.At, 2LL * cols); return; }
     if (a.z_off) { c->launch_fault = "grouped product: no workspace for the tiles its plan was made for"; return; }
@@ -491,7 +516,7 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
       } else {
         with_taps(sm->d.canon_taps, [&](auto N) { hipLaunchKernelGGL(tgx::norm_conv_kernel<decltype(N)::value>, dim3(T), dim3(256), 0, c->stream, m, norm_conv(w, 1)); });
         (void)route(c, ra.in, sm->a, w.w_router, ld.experts, T);
-        hipLaunchKernelGGL(tgx::router_topk_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
+        hipLaunchKernelGGL(tgx::router_topk_kernel, dim3(T), dim3(64), 0, c->stream, ra);
       }
       // yh[pair] = act(gate_e . a[token], up_e . a[token]), yd[pair] = router weight * (down_e . yh[pair])
       g = tgx::StackGemmArgs{};
@@ -752,7 +777,7 @@ void run_choice_experts(tgx_ctx* c, StackLayerW& w, const float* hin, int T, boo
   if (!routed) {
     tgx::RouterGroupArgs ra = choice_router(c, w, hin);
     (void)route(c, ra.in, hin, w.w_router, choice_products(ld), T);
-    hipLaunchKernelGGL(tgx::router_group_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
+    hipLaunchKernelGGL(tgx::router_group_kernel, dim3(T), dim3(64), 0, c->stream, ra);
   }
   const int np = T * top;
   if (ld.experts > 0) {
@@ -920,7 +945,7 @@ int run_joint_attention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, Join
   const bool shared = w.kv_src >= 0;
   const int W = sm->d.width, H = ld.heads, G = ld.kv_heads, qd = H * ld.dim, vd = H * ld.vdim, nin = qd + (shared ? 0 : G * (ld.dim + ld.vdim));
   tgx::StackGemmArgs g{};
-  g.A = sm->a; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = nin; g.M = T; g.N = nin; g.K = W; g.scale = 1.f;
+  g.A = sm->a; g.At = sm->in_terms; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = nin; g.M = T; g.N = nin; g.K = W; g.scale = 1.f;
   jl.first(c, g, 1);
   GqaSpec sp{};
   sp.proj = sm->proj; sp.ldp = nin; sp.heads = H; sp.kv_heads = G; sp.dim = ld.dim; sp.vdim = ld.vdim; sp.rot_dims = ld.rot_dims; sp.rot_pairs = ld.rot_pairs;
@@ -973,7 +998,7 @@ int run_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer&
   const int rH = ld.d_heads, rG = ld.d_kv_heads, rGD = rG * ld.d_dim, rvd = rH * ld.d_vdim, rC = 2 * rGD + rvd, nin = lq + lkv + rC + 2 * rH + rvd;
   // [left q | k | v | right q | k | v | b | a | g] = h . w_in^T: both halves read the same input
   tgx::StackGemmArgs g{};
-  g.A = sm->a; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = nin; g.M = T; g.N = nin; g.K = W; g.scale = 1.f;
+  g.A = sm->a; g.At = sm->in_terms; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = nin; g.M = T; g.N = nin; g.K = W; g.scale = 1.f;
   jl.first(c, g, 1);
   GqaSpec sp{};
   sp.proj = sm->proj; sp.ldp = nin; sp.heads = H; sp.kv_heads = G; sp.dim = ld.dim; sp.vdim = ld.vdim; sp.rot_dims = ld.rot_dims; sp.rot_pairs = ld.rot_pairs;
@@ -1028,12 +1053,14 @@ int run_layers_joint(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys,
   for (int li = 0; li < sm->d.layers; li++) {
     StackLayerW& w = sm->L[(size_t)li];
     const tgx_layer_desc& ld = w.d;
-    hipLaunchKernelGGL(tgx::offset_norm_kernel, dim3(T), dim3(256), 0, c->stream, sm->x, nullptr, w.norm1, 1.0f, sm->a, W, sm->d.norm_eps);
+    sm->in_terms = nullptr;
+    const tgx::RowTerms terms = ld.mlp == TGX_MLP_DENSE ? norm_terms(c, T, ld.ff, true) : tgx::RowTerms{};      // (the feed-forward's first product, the mixer's where it reads these rows)
+    hipLaunchKernelGGL(tgx::offset_norm_kernel, dim3(T), dim3(256), 0, c->stream, sm->x, nullptr, w.norm1, 1.0f, sm->a, W, sm->d.norm_eps, terms);
     int rc = TGX_OK;
     JointLayer jl;
     tgx::StackGemmArgs g{};
     if (ld.mlp == TGX_MLP_DENSE) {      // x += mult * down(silu(gate h) * (up h))
-      g.A = sm->a; g.lda = W; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.C = sm->yh; g.ldc = ld.ff; g.M = T; g.N = ld.ff; g.K = W;
+      g.A = sm->a; g.At = sm->in_terms; g.lda = W; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.C = sm->yh; g.ldc = ld.ff; g.M = T; g.N = ld.ff; g.K = W;
       jl.up = g;
       // every product that joins a launch must take the weight-streaming kernel by itself (one or two rows, whole slices)
       const int outs[] = {ld.heads * (ld.mixer == TGX_MIXER_WKV ? ld.dim : ld.vdim), ld.mixer == TGX_MIXER_PARALLEL ? ld.d_heads * ld.d_vdim : 0, ld.ff, W, ld.mixer == TGX_MIXER_PARALLEL ? sm->max_hv : 0};
@@ -1050,6 +1077,7 @@ int run_layers_joint(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys,
       else launch_ff(c, g, tgx::SG_SILU_MUL, down, tgx::SG_ADD);
     }
   }
+  sm->in_terms = nullptr;
   return TGX_OK;
 }
 
@@ -1259,7 +1287,7 @@ void run_affine_ff(tgx_ctx* c, StackLayerW& w, int T, bool routed) {
   if (!routed) {
     tgx::RouterGroupArgs ra = affine_router(c, w);
     (void)route(c, ra.in, sm->a, w.w_router, E, T);
-    hipLaunchKernelGGL(tgx::router_group_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
+    hipLaunchKernelGGL(tgx::router_group_kernel, dim3(T), dim3(64), 0, c->stream, ra);
   }
   g = tgx::StackGemmArgs{};
   g.A = sm->a; g.lda = W; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.b_zstride = (long long)ld.ff * W; g.C = sm->yh; g.ldc = ld.ff; g.N = ld.ff; g.K = W;
@@ -1519,10 +1547,10 @@ int check_affine_desc(const tgx_stack_desc& d, const tgx_layer_desc* layers) {
 
 // y = A . W^T into the sublayers' output rows
 void sublayer_out(tgx_ctx* c, const float* A, int K, const ebyte* Wm, int T) { launch_gemm(c, sublayer_product(c, A, K, Wm, T), tgx::SG_STORE, 1); }
-void post_norm_add(tgx_ctx* c, const float* w, int T) {
+void post_norm_add(tgx_ctx* c, const float* w, int T, const tgx::RowTerms& terms) {
   StackModel* sm = c->stack;
   tgx::PostNormArgs a{};
-  a.x = sm->x; a.y = sm->yd; a.w = w; a.W = sm->d.width; a.eps = sm->d.norm_eps;
+  a.x = sm->x; a.y = sm->yd; a.w = w; a.W = sm->d.width; a.eps = sm->d.norm_eps; a.terms = terms;
   hipLaunchKernelGGL(tgx::post_norm_add_kernel, dim3(T), dim3(256), 0, c->stream, a);
 }
 void launch_conv_silu(tgx_ctx* c, const tgx::StepMeta& m, tgx::ConvSiluArgs a, int T) {
@@ -1557,7 +1585,7 @@ void run_mamba1(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int S
   const int W = sm->d.width, I = ld.inner, N = ld.d_dim, R = ld.dt_rank, ldq = pad4(R + 2 * N), nb = ld.conv_taps - 1;
   // [x | z] = h . w_in^T
   tgx::StackGemmArgs g{};
-  g.A = sm->x; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = 2LL * I; g.M = T; g.N = 2 * I; g.K = W; g.scale = 1.f;
+  g.A = sm->x; g.At = sm->in_terms; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = 2LL * I; g.M = T; g.N = 2 * I; g.K = W; g.scale = 1.f;
   launch_gemm(c, g, tgx::SG_STORE, 1);
   tgx::ConvSiluArgs ca{};
   ca.proj = sm->proj; ca.ldp = 2LL * I; ca.cw = w.conv_w; ca.cb = w.conv_b; ca.out = sm->rec_in; ca.ldo = I; ca.state = nb > 0 ? w.conv_state : nullptr;
@@ -1584,7 +1612,7 @@ int run_ssm_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, 
   const int rH = ld.d_heads, I = rH * ld.d_vdim, gn = ld.d_kv_heads * ld.d_dim, C = I + 2 * gn, r0 = lq + lk, nin = r0 + I + C + rH + H, ldp = pad4(nin), ldo = lvd + I, nb = ld.conv_taps - 1;
   // [left q | k | right z | x | B | C | dt | left gate] = h . w_in^T (+ the biases of q and k): both halves read the same input
   tgx::StackGemmArgs g{};
-  g.A = sm->x; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = ldp; g.M = T; g.N = nin; g.K = W; g.scale = 1.f; g.bias = w.b_in;
+  g.A = sm->x; g.At = sm->in_terms; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = ldp; g.M = T; g.N = nin; g.K = W; g.scale = 1.f; g.bias = w.b_in;
   launch_gemm(c, g, tgx::SG_STORE, 1);
   GqaSpec sp{};
   sp.proj = sm->proj; sp.ldp = ldp; sp.heads = H; sp.kv_heads = G; sp.dim = ld.dim; sp.vdim = ld.vdim; sp.poolK = w.pool; sp.poolV = w.poolV; sp.poolVT = w.poolVT; sp.append = true;
@@ -1620,17 +1648,24 @@ int run_layers_post(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys, 
   const int W = sm->d.width;
   TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::sinusoid_embed_kernel<DT>, dim3(T), dim3(256), 0, c->stream, m, reinterpret_cast<const tgx::elem_t<DT>*>(c->embed), sm->d.embed_scale, sm->freq,
                                           sm->x, (float*)nullptr, W))
+  sm->in_terms = nullptr;
+  auto next_terms = [&](int li) {      // of the rows that the next mixer's first product reads
+    sm->in_terms = nullptr;
+    if (li >= sm->d.layers) return tgx::RowTerms{};
+    const tgx_layer_desc& ld = sm->L[(size_t)li].d;
+    return norm_terms(c, T, 2 * (ld.mixer == TGX_MIXER_MAMBA1 ? ld.inner : ld.d_heads * ld.d_vdim), false);      // (a parallel mixer's has more columns)
+  };
   for (int li = 0; li < sm->d.layers; li++) {
     StackLayerW& w = sm->L[(size_t)li];
     const tgx_layer_desc& ld = w.d;
     if (ld.mixer == TGX_MIXER_MAMBA1) run_mamba1(c, m, w, T, S);
     else { int rc = run_ssm_parallel(c, m, w, T, S, max_keys, max_count); if (rc) return rc; }
-    post_norm_add(c, w.norm1, T);
+    post_norm_add(c, w.norm1, T, ld.mlp == TGX_MLP_DENSE ? norm_terms(c, T, ld.ff, false) : next_terms(li + 1));
     if (ld.mlp != TGX_MLP_DENSE) continue;
     tgx::StackGemmArgs g{};      // down(max(up x, 0)^2)
-    g.A = sm->x; g.lda = W; g.B = w.w_up; g.ldb = W; g.C = sm->yh; g.ldc = ld.ff; g.M = T; g.N = ld.ff; g.K = W; g.scale = 1.f; g.act = tgx::SG_ACT_RELU2;
+    g.A = sm->x; g.At = sm->in_terms; g.lda = W; g.B = w.w_up; g.ldb = W; g.C = sm->yh; g.ldc = ld.ff; g.M = T; g.N = ld.ff; g.K = W; g.scale = 1.f; g.act = tgx::SG_ACT_RELU2;
     launch_ff(c, g, tgx::SG_STORE, sublayer_product(c, sm->yh, ld.ff, w.w_down, T), tgx::SG_STORE);
-    post_norm_add(c, w.norm2, T);
+    post_norm_add(c, w.norm2, T, next_terms(li + 1));
   }
   return TGX_OK;
 }
@@ -1949,7 +1984,7 @@ void run_hyper_ff(tgx_ctx* c, StackLayerW& w, int T) {
   if (!hyper_route_rides(c, w, T)) {      // (else the choice stands already)
     tgx::RouterGroupArgs ra = hyper_router(c, w, T);
     (void)route(c, ra.in, sm->a, w.w_router, ld.experts, T);
-    hipLaunchKernelGGL(tgx::router_group_kernel<false>, dim3(T), dim3(64), 0, c->stream, ra);
+    hipLaunchKernelGGL(tgx::router_group_kernel, dim3(T), dim3(64), 0, c->stream, ra);
   }
   // yh[pair] = max(up_e (w h), 0)^2: up_e is linear, so the weight multiplies its product
   g = tgx::StackGemmArgs{};
@@ -2338,7 +2373,7 @@ void run_logits(tgx_ctx* c, const int* want_dev, int nw, float* C, const int* c_
   StackModel* sm = c->stack;
   const int W = sm->d.width, V = sm->d.vocab;
   if (sm->affine) hipLaunchKernelGGL(tgx::layer_norm_rows_kernel, dim3(nw), dim3(256), 0, c->stream, sm->x, want_dev, sm->final_norm, sm->final_norm + W, sm->xn, W, sm->d.norm_eps);
-  else if (sm->joint || sm->post || sm->hyper) hipLaunchKernelGGL(tgx::offset_norm_kernel, dim3(nw), dim3(256), 0, c->stream, sm->x, want_dev, sm->final_norm, sm->joint || sm->hyper ? 1.0f : 0.0f, sm->xn, W, sm->d.norm_eps);
+  else if (sm->joint || sm->post || sm->hyper) hipLaunchKernelGGL(tgx::offset_norm_kernel, dim3(nw), dim3(256), 0, c->stream, sm->x, want_dev, sm->final_norm, sm->joint || sm->hyper ? 1.0f : 0.0f, sm->xn, W, sm->d.norm_eps, tgx::RowTerms{});
   else if (sm->sandwich) hipLaunchKernelGGL(tgx::scalar_norm_kernel, dim3(nw), dim3(256), 0, c->stream, sm->x, want_dev, sm->norm_g + 4 * (size_t)sm->d.layers, sm->xn, W, sm->d.norm_eps);
   else hipLaunchKernelGGL(tgx::final_norm_rows_kernel, dim3(nw), dim3(256), 0, c->stream, sm->x, want_dev, sm->final_norm, sm->xn, W, sm->d.norm_groups, sm->d.norm_eps);
   tgx::StackGemmArgs g{};
