@@ -242,3 +242,18 @@ def test_short_prompt_blocks_equal_steps(name, S, dtype):
     ulp = {"bf16": 8e-3, "fp16": 1e-3}[dtype]
     for (k1, v1), (k0, v0) in zip(kv1, kv0):
         assert rel_err(k1, k0) < ulp and rel_err(v1, v0) < ulp
+
+
+# N = hidden products whose steps of 64 do not fill six or seven slabs (25 and 29 steps; tests/test_prefill_plan.py has the rule): the counts that do are taken.  Bound as above
+@pytest.mark.parametrize("heads,S,dtype", [(25, 129, "bf16"), (25, 245, "fp16"), (29, 200, "bf16"), (29, 131, "fp16")])
+def test_products_that_fill_no_six_slabs(heads, S, dtype):
+    d = copy.deepcopy(known_desc("llama-3.2-1b", dtype))
+    d.hidden, d.heads, d.kv_heads, d.inter, d.layers, d.vocab, d.max_ctx = 64 * heads, heads, 5 if heads == 25 else heads, 64 * heads, 2, 2048, 264
+    gpu = Model(d, product_backend()).load_synthetic(19, 0.02).finalize()
+    prompt = synth.synth_prompt(d.vocab, S, 5)[None, :]
+    l1, _, _, kv1 = run(gpu, prompt, mfma=True)
+    l0, _, _, kv0 = run(gpu, prompt, mfma=False)
+    assert rel_err(l1, l0) < 1e-3
+    ulp = {"bf16": 8e-3, "fp16": 1e-3}[dtype]
+    for (k1, v1), (k0, v0) in zip(kv1, kv0):
+        assert rel_err(k1, k0) < ulp and rel_err(v1, v0) < ulp

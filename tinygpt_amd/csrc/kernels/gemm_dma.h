@@ -677,8 +677,10 @@ __global__ __launch_bounds__(512) void gemm_dma8k_kernel(const GemmArgs a) {
   };
 
   const int nk = (k_end - k_begin) / DBK;
+  if (EPI != GEMM_PARTIAL || nk > 0) {      // (a slab without K would read past the rows, into LDS that the sums below go through: nothing waits for its pieces)
 #pragma unroll
-  for (int q = 0; q < 6; q++) issue_piece(q, 0, 0);
+    for (int q = 0; q < 6; q++) issue_piece(q, 0, 0);
+  }
   if (nk > 1) {
 #pragma unroll
     for (int q = 0; q < 6; q++) issue_piece(q, DBK, 1);

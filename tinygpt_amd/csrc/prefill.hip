@@ -1,6 +1,7 @@
 // prefill.hip — the batched prefill of the MI355X shim for 16-bit storage (kernels/prefill.h, gemm_dma.h): every product of S prompt positions on the
 // matrix cores, causal flash attention, RoPE + cache append.  == CausalLM::forward on [B,S] ids with an empty cache (GPTModel.h:51-56)
 #include "ctx.h"
+#include "prefill_plan.h"
 #include <type_traits>
 #include "kernels/prefill.h"
 #include "kernels/gemm_dma.h"
@@ -111,17 +112,7 @@ static void launch_gemm(tgx_ctx* c, int epi, const ebyte* B_, const ebyte* bias_
   // CUs, 84 us per product against 104 at twice the rows) — the eight-wave LDS-DMA kernel over 2-8 K slabs instead of 64-row register-staged slabs or a half-empty chip
   bool part_8k = false;
   if (c->gemm_splitk && c->splitk_8k && (c->gemm_dma & 8) && K % 64 == 0 && !three_terms && (epi == tgx::GEMM_RESIDUAL || epi == tgx::GEMM_STORE) && M > 128) {
-    const int t128 = ((N + 127) / 128) * ((M + 127) / 128);
-    // slabs z = 2..8 that shorten the critical path: rounds of workgroups x 1 / z of the K loop against one round of whole tiles (160 tiles on 256 CUs: z = 3 -> 2 rounds of a
-    // third = 0.67; 128 tiles: z = 2 -> 0.5); taken from 0.8 down (the slabs cost a pass over z x M x N floats).  More than four where all of them run at once and the steps of K
-    // that they save (0.6 us each) outweigh their floats (written and read at 5 TB/s): eight / four, ms per prompt, Llama-3.2-1B 133 tokens 2.14 / 2.25, 256 2.28 / 2.39,
-    // Qwen2.5-0.5B 256 2.51 / 2.67; with eight in two rounds or for K 2048 at 509 rows and N 1024 it is slower (Qwen3-0.6B 3.53 / 3.45)
-    int z = 1; double best = 0.8001;
-    for (int zz = 2; zz <= 8; zz++) {
-      if (zz > 4 && (zz * t128 > c->num_cus || K < 6.8e-4 * zz * M * N)) break;
-      const double cost = (double)((zz * t128 + c->num_cus - 1) / c->num_cus) / zz;
-      if (t128 < c->num_cus && cost < best - 1e-9 && K / 64 >= 4 * zz) { best = cost; z = zz; }
-    }
+    const int z = tgx::eight_wave_slabs(M, N, K, c->num_cus);
     if (z >= 2) { part_8k = true; nsplit = z; }
   }
   // K >> N (`down`) on 128 x 256 tiles x 2 K slabs: a third fewer operand lines per output than the 128 x 128 kernel, which waits for them (kernels/gemm_dma.h
@@ -170,7 +161,7 @@ static void launch_gemm(tgx_ctx* c, int epi, const ebyte* B_, const ebyte* bias_
   }
   if (nsplit > 1) {
     g.part = c->ws_part; g.nsplit = nsplit; g.interleave = epi == tgx::GEMM_SILU ? 1 : 0;
-    g.k_per = part_8k ? ((K / 64 + nsplit - 1) / nsplit) * 64 : ((ktiles + nsplit - 1) / nsplit) * tgx::GBK;
+    g.k_per = part_8k ? tgx::slab_steps(K, nsplit) * 64 : ((ktiles + nsplit - 1) / nsplit) * tgx::GBK;
     const dim3 gz(grid.x, grid.y, nsplit);
     const size_t nout = (size_t)M * (epi == tgx::GEMM_SILU ? N / 2 : N);
     const dim3 rg((unsigned)((nout + 255) / 256));

@@ -1,0 +1,27 @@
+// prefill_plan.h — how a prompt's products are cut, as plain arithmetic on their sizes (no HIP: tests/test_prefill_plan.py goes through it on the CPU).
+#pragma once
+
+namespace tgx {
+
+// K (a multiple of 64) in z slabs: steps of 64 in each but the last, and whether the last one has any.  (Rounding up can leave none for it: 25 steps in six slabs are five of five.)
+inline int slab_steps(int K, int z) { return (K / 64 + z - 1) / z; }
+inline bool slabs_hold_k(int K, int z) { return (z - 1) * slab_steps(K, z) < K / 64; }
+
+// Slabs of an N = hidden product on the eight-wave 128 x 128 kernel (1: whole).  Slabs z = 2..8 that shorten the critical path: rounds of workgroups x 1 / z of the K loop against one
+// round of whole tiles (160 tiles on 256 CUs: z = 3 -> 2 rounds of a third = 0.67; 128 tiles: z = 2 -> 0.5); taken from 0.8 down (the slabs cost a pass over z x M x N floats).  More
+// than four where all of them run at once and the steps of K that they save (0.6 us each) outweigh their floats (written and read at 5 TB/s): eight / four, ms per prompt,
+// Llama-3.2-1B 133 tokens 2.14 / 2.25, 256 2.28 / 2.39, Qwen2.5-0.5B 256 2.51 / 2.67; with eight in two rounds or for K 2048 at 509 rows and N 1024 it is slower
+// (Qwen3-0.6B 3.53 / 3.45).  Every slab has four steps on average and one at least.
+inline int eight_wave_slabs(int M, int N, int K, int num_cus) {
+  const int tiles = ((N + 127) / 128) * ((M + 127) / 128);
+  int z = 1;
+  double best = 0.8001;
+  for (int zz = 2; zz <= 8 && tiles < num_cus; zz++) {
+    if (zz > 4 && (zz * tiles > num_cus || K < 6.8e-4 * zz * M * N)) break;
+    const double cost = (double)((zz * tiles + num_cus - 1) / num_cus) / zz;
+    if (cost < best - 1e-9 && K / 64 >= 4 * zz && slabs_hold_k(K, zz)) { best = cost; z = zz; }
+  }
+  return z;
+}
+
+}  // namespace tgx
