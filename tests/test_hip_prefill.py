@@ -257,3 +257,21 @@ def test_products_that_fill_no_six_slabs(heads, S, dtype):
     ulp = {"bf16": 8e-3, "fp16": 1e-3}[dtype]
     for (k1, v1), (k0, v0) in zip(kv1, kv0):
         assert rel_err(k1, k0) < ulp and rel_err(v1, v0) < ulp
+
+
+# gate_up on both sides of the rule that keeps it whole (tests/test_prefill_plan.py): 65 to 128 rows and half a chip of tiles (slabs), 65 rows and more tiles (whole), and the slabs that
+# a low prefill.wide_8k_max asks for.  One layer: the same products and epilogue in another summation order
+@pytest.mark.parametrize("name,S,dtype", [("llama-3.2-3b", 100, "bf16"), ("llama-3.2-3b", 128, "fp16"), ("mistral-7b-v0.3", 65, "bf16"), ("mistral-7b-v0.3", 128, "fp16"), ("qwen3-1.7b", 129, "bf16"), ("qwen3-0.6b", 257, "fp16")])
+def test_gate_up_whole_equals_slabs(name, S, dtype):
+    d = copy.deepcopy(known_desc(name, dtype))
+    d.layers, d.vocab, d.max_ctx = 1, 4096, S + 16
+    m = Model(d, product_backend()).load_synthetic(1234, 0.02).finalize()
+    prompt = synth.synth_prompt(d.vocab, S, 81)[None, :]
+    outs = []
+    for most in (8, 0, 8):
+        m.set_option("prefill.wide_8k_max", most)
+        m.reset_cache(); m.forward(prompt)
+        outs.append((m.logits(rounded=False).copy(), m.sample(GREEDY).copy()))
+    assert rel_err(outs[1][0], outs[0][0]) < 2e-5, rel_err(outs[1][0], outs[0][0])
+    np.testing.assert_array_equal(outs[1][1], outs[0][1])
+    np.testing.assert_array_equal(outs[2][0], outs[0][0])

@@ -19,6 +19,7 @@ extern "C" int empty_slab(int cus, int k_lo, int k_hi, int* out) {
       }
   return 0;
 }
+extern "C" int whole(int m, int n, int k, int cus, int most) { return tgx::gate_up_whole(m, n, k, cus, most); }
 extern "C" int slabs(int m, int n, int k, int cus) { return tgx::eight_wave_slabs(m, n, k, cus); }
 extern "C" int steps(int k, int z) { return tgx::slab_steps(k, z); }
 """
@@ -46,3 +47,19 @@ def test_slabs_of_products(plan, rows, columns, K, slabs):
     z = plan.slabs(rows, columns, K, 256)
     assert z == slabs
     assert (z - 1) * plan.steps(K, z) < K // 64 <= z * plan.steps(K, z)
+
+
+# (rows, tiles of 128 columns, K): a short K from a quarter of a chip of 256 on, any from more than half a chip on; never at rows that the slabs' 64-row tiles fit
+@pytest.mark.parametrize("rows,column_tiles,K,whole", [(133, 48, 1024, 1), (129, 32, 1024, 1), (129, 31, 1024, 0), (129, 32, 1088, 0), (128, 64, 1024, 0), (128, 129, 1024, 1), (133, 76, 896, 1),
+                                                       (509, 48, 1024, 1), (100, 128, 3072, 0), (129, 64, 3072, 0), (129, 65, 3072, 1), (65, 224, 4096, 1), (64, 224, 4096, 0), (100, 256, 3072, 0), (300, 96, 1024, 0)])
+def test_gate_up_whole(plan, rows, column_tiles, K, whole):
+    assert plan.whole(rows, 128 * column_tiles, K, 256, 8) == whole
+    assert plan.whole(rows, 128 * column_tiles - 2, K, 256, 8) == whole
+
+
+def test_gate_up_is_whole_only_where_the_eight_wave_kernel_takes_it(plan):
+    """the product is left without slabs for that kernel alone (prefill.wide_8k_max: its tiles in half-chips)"""
+    for most in (0, 1, 2, 8):
+        for tiles in range(1, 300):
+            assert not (plan.whole(100, 128 * tiles, 512, 256, most) and 2 * tiles > most * 256)
+    assert not plan.whole(133, 128 * 48, 1024, 256, 0) and plan.whole(133, 128 * 48, 1024, 256, 1)

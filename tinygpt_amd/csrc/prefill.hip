@@ -104,9 +104,7 @@ static void launch_gemm(tgx_ctx* c, int epi, const ebyte* B_, const ebyte* bias_
   const bool qkv_bal = (c->gemm_dma & 3) && three_terms && epi == tgx::GEMM_STORE && three_from > 0 && three_from % tgx::GBN == 0 && N > three_from && K % 64 == 0 && M >= 128;
   const int qkv_wgs = qkv_bal ? (three_from / tgx::GBN) * ((M + 127) / 128) + ((N - three_from + tgx::GBN - 1) / tgx::GBN) * ((M + 63) / 64) : 0;
   const bool qkv_nosplit = qkv_bal && c->qkv_nosplit && qkv_wgs >= c->num_cus;
-  // (the gate_up product of prompts below a chip of 128 x 128 tiles keeps them whole, on the eight-wave kernel, from a quarter of a chip on: no slabs, no reduce launch.  Whole / split,
-  //  ms per prompt: Qwen3-0.6B 133 tokens (96 tiles) 2.68 / 2.78, 256 2.98 / 3.21, 509 (192) 3.45 / 3.92; Qwen2.5-0.5B 133 (152) 2.07 / 2.27, 384 (228) 2.49 / 2.99)
-  const bool silu8 = epi == tgx::GEMM_SILU && (c->gemm_dma & 8) && K % 64 == 0 && !three_terms && 4 * ntiles >= c->num_cus;
+  const bool silu8 = epi == tgx::GEMM_SILU && (c->gemm_dma & 8) && K % 64 == 0 && !three_terms && tgx::gate_up_whole(M, N, K, c->num_cus, c->wide_8k_max);      // (whole: no slabs, no reduce launch)
   if (c->gemm_splitk && ntiles < c->num_cus && K % tgx::GBK == 0 && !qkv_nosplit && !silu8) nsplit = std::min(std::min(16, ktiles), (2 * c->num_cus + ntiles - 1) / ntiles);
   // N = hidden products of a 129-1500-row prompt (round 4, option prefill.splitk_8k): their 128 x 128 tiles number less than a chip (Llama-3.2-1B S = 1024: 128 tiles on 256
   // CUs, 84 us per product against 104 at twice the rows) — the eight-wave LDS-DMA kernel over 2-8 K slabs instead of 64-row register-staged slabs or a half-empty chip

@@ -24,4 +24,16 @@ inline int eight_wave_slabs(int M, int N, int K, int num_cus) {
   return z;
 }
 
+// Whether the gate_up product (N columns, below a chip of 128 x 128 tiles) of a prompt stays whole on the eight-wave kernel instead of K slabs with a launch that sums them.  most: the
+// half-chips of tiles up to which that kernel is taken (option prefill.wide_8k_max).  A whole product is a chain of K / 64 steps of 0.6 us, so a short K keeps it from a quarter of a
+// chip of tiles on, a longer one from half a chip on, where slabs would go into another round.  Whole / split, ms per prompt: Qwen3-0.6B (K 1024) 133 tokens (96 tiles) 2.68 / 2.78, 256
+// 2.98 / 3.21, 509 (192) 3.45 / 3.92; Qwen2.5-0.5B 133 (152) 2.07 / 2.27, 384 (228) 2.49 / 2.99.  Whole less split, us a layer: K 512 and 1024, 129 to 512 rows, 64 to 240 tiles -0.7 to
+// -21; K 2048, 129 to 512 rows, 64 tiles +5 to +7, 96 -4 to +2, 128 -3 to 0, 144 to 240 -14 to -28; K 2560, 3072 and 4096, 65 to 200 rows, 64 tiles +14 to +21, 96 -2 to +2, 128 +1 to
+// +7, 152 -8 to -18, 192 -17 to -33, 224 -20 to -37.  Up to 64 rows the slabs have tiles of 64 rows and nothing of it is padding.
+inline bool gate_up_whole(int M, int N, int K, int num_cus, int most) {
+  const long long tiles = (long long)((N + 127) / 128) * ((M + 127) / 128);
+  if (M <= 64 || tiles >= num_cus || 2 * tiles > (long long)most * num_cus) return false;
+  return K <= 1024 && M > 128 ? 4 * tiles >= num_cus : 2 * tiles > num_cus;
+}
+
 }  // namespace tgx
