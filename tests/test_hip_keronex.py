@@ -412,9 +412,9 @@ def test_a_router_weight_stands_in_front_of_the_square():
 
 
 @pytest.mark.parametrize("dtype", ["fp32", "bf16"])
-@pytest.mark.parametrize("n", [2, 21, 31, 32, 33, 42, 43, 70])
+@pytest.mark.parametrize("n", [2, 9, 10, 20, 21, 31, 32, 33, 42, 43, 70])
 def test_a_shared_expert_of_the_routed_size(n, dtype):
-    """steps of few pairs take the shared expert as one more choice, longer ones compute it by itself: portions on both sides of the border (128 pairs)"""
+    """steps of few pairs take the shared expert as one more choice, longer ones compute it by itself: portions on both sides of the border (128 pairs), and of the one between the pairs' kernel and planned tiles (six rows an expert)"""
     cfg = config([ret(moe(5, 3, 16, 16)), cd(moe(9, 2, 24, 24))])
     toks = tokens(cfg, n + 4, seed=n)
     w = ko.random_tensors(cfg, 13)

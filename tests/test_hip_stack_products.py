@@ -305,10 +305,11 @@ def test_router_products_in_the_biased_choice(rows, experts):
 
 
 # ---- products over a step's (token, expert) pairs (up to 128): fewer pairs than experts and more, experts of one to 64 rows (tiles of four and eight), contraction lengths around
-# the chunk of 128 and below it, column counts that end inside a workgroup's; one pair more than 128 takes the planned tiles.  fp32 storage against the plain oracle: fp32 sums over
+# the chunk of 128 and below it, column counts that end inside a workgroup's; more than six rows an expert on average take a plan and tiles of sixteen rows, one pair more than 128
+# the other planned tiles.  fp32 storage against the plain oracle: fp32 sums over
 # at most 1032 terms, 1e-4 of the largest logit as above.
 @pytest.mark.parametrize("width,ff", [(8, 24), (136, 8), (1032, 520), (264, 1032)])
-@pytest.mark.parametrize("rows,experts,top", [(1, 12, 3), (1, 2, 2), (9, 40, 2), (64, 3, 2), (25, 5, 5), (65, 3, 2), (33, 2, 1)])
+@pytest.mark.parametrize("rows,experts,top", [(1, 12, 3), (1, 2, 2), (9, 40, 2), (64, 3, 2), (25, 5, 5), (65, 3, 2), (33, 2, 1), (24, 8, 2), (25, 8, 2), (64, 11, 1), (64, 22, 2), (65, 22, 2)])
 def test_products_of_pairs(rows, experts, top, width, ff):
     layers = [LayerDesc(heads=3, dim=8, vdim=8, kv_rank=24, scale=0.35, mlp="moe", experts=experts, top=top, ff=ff, limit=1.5) for _ in range(2)]
     d = StackDesc(width=width, vocab=53, canon_taps=2, norm_groups=2, norm_eps=1e-6, max_seqs=2, max_ctx=128, budget_tokens=256, compute_dtype="fp32", layers=layers)

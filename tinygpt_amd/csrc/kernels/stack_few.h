@@ -1,5 +1,5 @@
-// stack_few.h — the products of layered models (stack_gemm.h) for A FEW rows: 3 to 64 activation rows, and matrices of so few rows (a router's) that 64-wide tiles
-// would stand empty.
+// stack_few.h — the products of layered models (stack_gemm.h) for A FEW rows: 3 to 64 activation rows, the tiles of sixteen rows of a grouped product with few
+// (token, expert) pairs, and matrices of so few rows (a router's) that 64-wide tiles would stand empty.
 //
 // What bounds it: the weights cross once, so the stream of weight bytes is the floor; the vector form (stack_gemv_kernel, two columns a wave) instead moved every
 // activation row through L2 for every two columns — eight rows of 4 KB for 4 KB of weights — and streamed the weights again for every tile of four or eight rows.
@@ -37,13 +37,12 @@ template <int DT, bool DUAL, int MB> constexpr size_t few_lds_bytes(int waves, i
 __device__ const u32x4 few_zeros = {0u, 0u, 0u, 0u};
 
 template <int DT, int EPI, bool DUAL, int MB>
-__device__ __forceinline__ void stack_few_body(const StackGemmArgs& a, const int depth, const int z) {
+__device__ __forceinline__ void stack_few_body(const StackGemmArgs& a, const int depth, const int z, const int mbase, const int mend) {
   constexpr int NB = DUAL ? 2 : 1, WP = DT == DT_F32 ? 4 : 2;       // 1-KB pieces of a step's weight rows (per matrix)
   constexpr int PIECES = NB * WP + MB * 4, STEP = few_step_bytes<DT, DUAL, MB>();
   extern __shared__ __attribute__((aligned(1024))) unsigned char few_lds[];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
   const int li = lane & 15, q = lane >> 4;                          // row (column) of the operands, quarter of a half step's k
-  const int mbase = blockIdx.y * 16 * MB, mend = min(a.M, mbase + 16 * MB);
   const int n0 = blockIdx.x * 16, steps = (a.K + 63) >> 6;
   if (n0 >= a.N) return;                                            // (the narrower product of a pair)
   unsigned char* ring = few_lds + (size_t)wv * depth * STEP;
@@ -181,13 +180,20 @@ __device__ __forceinline__ void stack_few_body(const StackGemmArgs& a, const int
 }
 
 template <int DT, int EPI, bool DUAL, int MB>
-__global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_kernel(const StackGemmArgs a, const int depth) { stack_few_body<DT, EPI, DUAL, MB>(a, depth, blockIdx.z); }
+__global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_kernel(const StackGemmArgs a, const int depth) {
+  int z = blockIdx.z, m0 = blockIdx.y * 16 * MB, rows_end = a.M;
+  if (a.z_off) {
+    if ((int)blockIdx.y >= *a.n_tiles) return;
+    z = a.tile_z[blockIdx.y]; m0 = a.tile_m0[blockIdx.y]; rows_end = a.z_off[z + 1];
+  }
+  stack_few_body<DT, EPI, DUAL, MB>(a, depth, z, m0, min(rows_end, m0 + 16 * MB));
+}
 // two products that do not need each other, of the same rows and contraction length, in one launch: blockIdx.z chooses (the low-rank pair of a channel-delta layer, sixteen rows of
 // 1024 x 128 each: 4.7 us and 4.7, 5.7 together)
 template <int DT, int MB>
 __global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_pair_kernel(const StackGemmArgs a, const StackGemmArgs b, const int depth) {
-  if (blockIdx.z == 0) stack_few_body<DT, SG_STORE, false, MB>(a, depth, 0);
-  else stack_few_body<DT, SG_STORE, false, MB>(b, depth, 0);
+  if (blockIdx.z == 0) stack_few_body<DT, SG_STORE, false, MB>(a, depth, 0, 0, a.M);      // (one tile of rows)
+  else stack_few_body<DT, SG_STORE, false, MB>(b, depth, 0, 0, b.M);
 }
 
 // Waves and ring depth: some eight waves a compute unit (2048 on the chip) and four a workgroup at least, never more than K has steps; two steps of each in flight, one

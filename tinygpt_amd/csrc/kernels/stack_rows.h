@@ -1,6 +1,7 @@
-// stack_rows.h — the products of layered models (stack_gemm.h) for the (token, expert) pairs of a step of few tokens: up to 128 pairs, grouped by expert in the kernel itself.
+// stack_rows.h — the products of layered models (stack_gemm.h) for the (token, expert) pairs of a step of few tokens, up to 128, grouped by expert in the kernel itself.  Made for a few
+// rows an expert: up to six on average (stack.hip sends more to a plan and sixteen-row tiles).
 //
-// What bounds it: the chosen experts' weights cross once (25 MB for four tokens of 1024 channels and two of eight experts of 1536: 4 us at the rate of a large read); beside
+// What bounds it: the weights of a chosen expert cross once for every eight rows that it has, so as a rule once (25 MB for four tokens of 1024 channels and two of eight experts of 1536: 4 us at the rate of a large read); beside
 // that stand a launch and whatever chain of loads comes before the first weight.  The form before it (moe_plan_kernel, then stack_few_kernel on sixteen-row tiles) paid a launch
 // for the plan, four dependent loads (number of tiles, tile, rows, activations) in each product, sixteen rows of activations for the one to four that an expert has and
 // sixteen-row matrix instructions for them.  Here every workgroup reads the choices themselves (one load, two ballots), and the products are v_mfma_f32_4x4x1_f32 in

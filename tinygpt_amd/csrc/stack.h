@@ -177,7 +177,7 @@ size_t mix_mfma_wg_lds(int heads, int kv_heads);      // LDS bytes of one of its
 bool stack_allow_lds(tgx_ctx* c, const void* kernel, size_t bytes);
 // stack_few.hip
 namespace tgx { struct StackGemmArgs; }
-void launch_stack_few(tgx_ctx* c, const tgx::StackGemmArgs& a, int epi, int nz, int dt);
+void launch_stack_few(tgx_ctx* c, const tgx::StackGemmArgs& a, int epi, int nz, int grouped_tiles, int dt);
 void launch_stack_few_pair(tgx_ctx* c, const tgx::StackGemmArgs& a, const tgx::StackGemmArgs& b, int dt);
 // stack_rows.hip
 void launch_stack_rows(tgx_ctx* c, const tgx::StackGemmArgs& a, int epi, int dt);

@@ -29,7 +29,7 @@ namespace tgx {
 // Four tokens, 8 heads of 256 x 128: 4.5 us and 4.4, 4.6 together.
 template <int DT>
 __global__ __launch_bounds__(64 * few_max_waves(1)) void latent_append_queries_kernel(StepMeta m, LatentAppendArgs la, StackGemmArgs a, const int depth, const int heads) {
-  if ((int)blockIdx.z < heads) stack_few_body<DT, SG_STORE, false, 1>(a, depth, blockIdx.z);
+  if ((int)blockIdx.z < heads) stack_few_body<DT, SG_STORE, false, 1>(a, depth, blockIdx.z, 0, a.M);
   else for (int t = blockIdx.x; t < m.T; t += gridDim.x) latent_append_body<DT>(m, la, t);
 }
 }  // namespace tgx
@@ -101,8 +101,13 @@ void launch_gemv_t(tgx_ctx* c, const tgx::StackGemmArgs& a, dim3 grid, int mr, b
   else if (ksplit) go(std::integral_constant<int, 2>{}, std::true_type{});
   else go(std::integral_constant<int, 2>{}, std::false_type{});
 }
-// steps of up to so many (token, expert) pairs take the experts' products without a plan (stack_rows_kernel); products of up to so many rows the few-row kernel
-constexpr int GROUPED_FEW_PAIRS = tgx::ROWS_MAX_PAIRS, FEW_ROWS_MAX = 64;
+// Steps of up to so many (token, expert) pairs: the experts' products on stack_rows_kernel, without a plan, while an expert has few rows on average, and on the few-row kernel by a plan
+// of tiles of sixteen rows beyond (the former reads an expert's weights again for every eight rows, and where six are the mean, some experts have more than eight).  A step of four
+// layers, pairs' kernel / planned tiles, us: two of eight experts of 1536 x 1024, 16 tokens 353 / 377, 24 413 / 416, 28 422 / 417, 42 512 / 475, 64 569 / 513 (fp32 storage 419 / 443,
+// 491 / 479, 524 / 481, 661 / 562, 772 / 603); four of sixteen of 2048 x 2048, 16 tokens 749 / 838, 24 889 / 911, 28 927 / 923, 32 971 / 922; with a shared expert riding, which has every
+// token's row, two of eight 16 tokens 333 / 344, 22 375 / 375, 42 468 / 436, four of sixteen 12 574 / 597, 16 605 / 605, 20 687 / 668, 24 719 / 671.
+// Products of up to so many rows: the few-row kernel.
+constexpr int GROUPED_FEW_PAIRS = tgx::ROWS_MAX_PAIRS, GROUPED_FEW_ROWS = 16, GROUPED_MEAN_ROWS = 6, FEW_ROWS_MAX = 64;
 // the vector kernel serves one and two rows (1024 x 1024, two rows: 4.4 us against 5.4; 3072 x 1024 gate and up: 6.8 against 7.7; four rows 6.0 against 5.5), stack_few_kernel
 // three to 64.  Where the line at 64 rows lies, us of the few-row kernel against the 64-wide tiles at 64 rows, bf16: 1024 x 3072 20 / 42, 2048 x 8192 39 / 92,
 // 2 x 3072 x 1024 17.5 / 26, four of 2048 x 2048 42 / 45; products whose tiles fill the chip are the faster ones on the tiles, in two 16-bit terms where the few-row kernel rounds
@@ -162,10 +167,10 @@ void scratch_sizes(tgx_ctx* c) {
   sm->terms_most = (size_t)std::max(cols, most);
 }
 // rows per tile of the two grouped products of an expert layer's plan (both must be able to take them: their contraction lengths are the width and the expert width); 0: no plan,
-// the pairs' kernel.  np: (token, expert) pairs, E: experts, up_n: columns of the first product (gate and up together)
+// the pairs' kernel (GROUPED_MEAN_ROWS).  np: (token, expert) pairs, E: experts, up_n: columns of the first product (gate and up together)
 int grouped_tile_rows(tgx_ctx* c, int np, int width, int ff, int E, int T, int up_n) {
   StackModel* sm = c->stack;
-  if (sm->gemv && np <= GROUPED_FEW_PAIRS && width % 8 == 0 && ff % 8 == 0) return 0;
+  if (sm->gemv && np <= GROUPED_FEW_PAIRS && width % 8 == 0 && ff % 8 == 0) return np <= GROUPED_MEAN_ROWS * E ? 0 : GROUPED_FEW_ROWS;
   if (sm->line && c->dt != tgx::DT_F32 && width % 64 == 0 && ff % 64 == 0 && E > 0) {
     const int tile = stack_line_tile_grouped(c, np, E, up_n);
     if (tile && ensure_terms(c, (size_t)T * 2 * width) && ensure_terms2(c, (size_t)np * 2 * ff)) return tile;
@@ -237,8 +242,9 @@ void launch_gemm(tgx_ctx* c, tgx::StackGemmArgs a, int epi, int nz, int grouped_
                    (!a.B2 || (uintptr_t)a.B2 % 16 == 0);
   const bool dual = tgx::sg_dual(epi);
   // few rows: the weight-streaming kernels
-  const bool few = sm->gemv && slices_ok(a) && !a.z_off && (a.M <= FEW_ROWS_MAX || a.N <= FEW_COLS_ANY_ROWS);
-  if (few && a.M > GEMV_ROWS_MAX) { launch_stack_few(c, a, epi, nz, dt); return; }
+  const bool few = sm->gemv && slices_ok(a) && (a.z_off ? grouped_tile == GROUPED_FEW_ROWS : (a.M <= FEW_ROWS_MAX || a.N <= FEW_COLS_ANY_ROWS));
+  if (a.z_off && grouped_tile == GROUPED_FEW_ROWS && !few) { c->launch_fault = "grouped product: the plan was made for the few-row kernel, which these operands cannot take"; return; }
+  if (few && (a.z_off || a.M > GEMV_ROWS_MAX)) { launch_stack_few(c, a, epi, nz, a.z_off ? grouped_rows / GROUPED_FEW_ROWS + std::min(groups, grouped_rows) : 0, dt); return; }
   if (few) {
     const int mr = a.M <= 1 ? 1 : 2;
     const bool ksplit = gemv_ksplit(c, a, nz);
@@ -392,8 +398,8 @@ int ensure_ws(tgx_ctx* c, int T) {
     const size_t np = std::max<size_t>(n * (size_t)sm->max_top, sm->hyper ? GROUPED_FEW_PAIRS : 0);      // (a shared expert that rides among the choices: at most that many pairs)
     if ((rc = dev_alloc(c, &sm->zr, n * (size_t)(sm->max_E + 1))) || (rc = dev_alloc(c, &sm->selw, np)) || (rc = dev_alloc(c, &sm->sel, np)) || (rc = dev_alloc(c, &sm->perm, np)) || (rc = dev_alloc(c, &sm->ptok, np)) ||
         (rc = dev_alloc(c, &sm->yh, np * (size_t)sm->max_ff + n * (size_t)sm->max_sff)) || (rc = dev_alloc(c, &sm->yd, np * W)) ||
-        (rc = dev_alloc(c, &sm->tile_e, np / 64 + (size_t)sm->max_E + 1)) ||
-        (rc = dev_alloc(c, &sm->tile_m0, np / 64 + (size_t)sm->max_E + 1))) return rc;
+        (rc = dev_alloc(c, &sm->tile_e, std::max<size_t>(np / 64, GROUPED_FEW_PAIRS / GROUPED_FEW_ROWS) + (size_t)sm->max_E + 1)) ||
+        (rc = dev_alloc(c, &sm->tile_m0, std::max<size_t>(np / 64, GROUPED_FEW_PAIRS / GROUPED_FEW_ROWS) + (size_t)sm->max_E + 1))) return rc;
   }
   sm->meta_cap = (size_t)9 * n + (size_t)4 * sm->d.max_seqs;
   if ((rc = dev_alloc(c, &sm->meta_dev, sm->meta_cap))) return rc;
@@ -1957,7 +1963,7 @@ void run_channel_delta(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T
 // the shared expert's product takes the wide tiles by itself.)
 bool shared_rides(const tgx_ctx* c, const StackLayerW& w, int T) {
   const int np = T * (w.d.top + 1);
-  return w.shared_slot && np <= GROUPED_FEW_PAIRS && c->stack->gemv && c->stack->d.width % 8 == 0 && w.d.ff % 8 == 0;      // (the pairs' kernel)
+  return w.shared_slot && np <= GROUPED_FEW_PAIRS && c->stack->gemv && c->stack->d.width % 8 == 0 && w.d.ff % 8 == 0;      // (the forms of few pairs)
 }
 tgx::RouterGroupArgs hyper_router(const tgx_ctx* c, const StackLayerW& w, int T) {
   const StackModel* sm = c->stack;

@@ -37,11 +37,12 @@ void launch_stack_few_pair(tgx_ctx* c, const tgx::StackGemmArgs& a, const tgx::S
     else launch_few_pair_mb<DT, 4>(c, a, b, grid);)
 }
 
-void launch_stack_few(tgx_ctx* c, const tgx::StackGemmArgs& a, int epi, int nz, int dt) {
+// grouped_tiles: upper bound of the tile list of a grouped product (a.z_off), 0 for plain and batched ones
+void launch_stack_few(tgx_ctx* c, const tgx::StackGemmArgs& a, int epi, int nz, int grouped_tiles, int dt) {
   // sixteen-row operands: all rows of a step in one workgroup up to 64 (the weights cross once); many rows of a narrow matrix (a router's) in sixteens, which spreads
   // them over the chip
-  const int mb = a.M <= 16 || a.M > 64 ? 1 : a.M <= 32 ? 2 : 4;
-  const dim3 grid((a.N + 15) / 16, (a.M + 16 * mb - 1) / (16 * mb), nz);
+  const int mb = a.z_off || a.M <= 16 || a.M > 64 ? 1 : a.M <= 32 ? 2 : 4;
+  const dim3 grid((a.N + 15) / 16, a.z_off ? grouped_tiles : (a.M + 16 * mb - 1) / (16 * mb), a.z_off ? 1 : nz);
   TGX_DT_SWITCH(dt,
     switch (epi) {
       case tgx::SG_STORE: launch_few_t<DT, tgx::SG_STORE, false>(c, a, grid, mb); break;
