@@ -52,6 +52,19 @@ def test_retention(dim, vdim, rot):
     stepped(tk, cfg, 7, dim)
 
 
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+def test_blocks_of_single_tokens_where_they_are_asked_for(dtype):
+    """ssd.min 1 sends single tokens of retention layers through the blocked recurrence whatever stack.rec_step says: the same bits, and others than the step kernel's"""
+    cfg = tk.config([tk.ret(dim=64, vdim=128), tk.ret(dim=32, vdim=32)], width=32)
+    out, toks = {}, tk.tokens(cfg, 9, 3)
+    for ssd_min, on in ((1, 1), (1, 0), (64, 1)):
+        eng, _ = tk.engine(cfg, dtype, 5, options={"ssd.min": ssd_min, "stack.rec_step": on})
+        out[ssd_min, on] = np.concatenate([eng.step([("r", toks[:3], [2])])] + [eng.step([("r", toks[i:i + 1], [0])]) for i in range(3, 9)])
+        eng.close()
+    np.testing.assert_array_equal(out[1, 1], out[1, 0])
+    assert (out[1, 1] != out[64, 1]).any()
+
+
 @pytest.mark.parametrize("dim,vdim", [(8, 6), (64, 32), (128, 128), (100, 65), (4, 200)])
 def test_channel_decays(dim, vdim):
     cfg = tk.config([tk.cd(dim=dim, vdim=vdim), tk.cd(tk.dense(16), dim=dim, vdim=vdim, conv=1)], width=24)

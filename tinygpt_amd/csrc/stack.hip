@@ -1893,13 +1893,14 @@ int run_retention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int
   oa.hs = sm->hs; oa.ldh = vd; oa.gate = sm->proj + vd + 2 * qd; oa.ldg = ldp; oa.silu_gate = 1; oa.out = sm->o; oa.ldo = vd; oa.vdim = ld.vdim; oa.eps = sm->d.norm_eps;
   tgx::RecStepArgs st{};
   st.s = ra; st.g = oa; st.rot_dims = ld.rot_dims; st.cs = w.rot >= 0 ? sm->rot[(size_t)w.rot].cs : nullptr;
-  if (!launch_rec_step(c, m, st, tgx::REC_SSD, S, max_count)) {
+  const bool blocks = sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && ensure_part(c, ssd_gram_elems(T, S, H), ssd_gram_elems(sm->cap_tokens, sm->d.max_seqs, H));
+  if (blocks || !launch_rec_step(c, m, st, tgx::REC_SSD, S, max_count)) {      // (blocks of single tokens only where ssd.min asks for them)
     if (w.rot >= 0) {      // q and k turn in place (2 H heads side by side)
       tgx::GqaAppendArgs ap{};
       ap.proj = sm->proj + vd; ap.ldp = ldp; ap.heads = 2 * H; ap.dim = ld.dim; ap.rot_dims = ld.rot_dims; ap.cs = sm->rot[(size_t)w.rot].cs;
       TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::gqa_append_kernel<DT>, dim3(T), dim3(256), 0, c->stream, m, ap))
     }
-    if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && ensure_part(c, ssd_gram_elems(T, S, H), ssd_gram_elems(sm->cap_tokens, sm->d.max_seqs, H))) {
+    if (blocks) {
       tgx::SsdArgs da{};
       da.row = sm->proj; da.ld = ldp; da.b0 = vd; da.c0 = vd + qd; da.heads = H; da.groups = H; da.N = ld.dim; da.E = ld.vdim; da.gram = sm->part; da.fixed = w.decays; da.dt0 = kscale; da.S = w.mS; da.out = sm->hs; da.ldo = vd;
       launch_ssd_mfma(c, m, da, S, max_count);
