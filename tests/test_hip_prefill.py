@@ -184,12 +184,14 @@ def test_gate_up_on_128_tiles_where_the_256_tiling_is_ragged(name, S):
 
 
 @pytest.mark.parametrize("name,S,dtype", [("llama-3.2-1b", 300, "bf16"), ("llama-3.2-1b", 777, "fp16"), ("qwen2.5-0.5b", 257, "bf16"),
-                                          ("mistral-7b-v0.3", 300, "bf16"), ("llama-3.2-3b", 200, "fp16"), ("qwen3-1.7b", 333, "bf16")])
+                                          ("mistral-7b-v0.3", 300, "bf16"), ("llama-3.2-3b", 200, "fp16"), ("qwen3-1.7b", 333, "bf16"),
+                                          ("llama-3.2-1b", 1100, "bf16"), ("mistral-7b-v0.3", 1061, "fp16")])
 def test_prefill_attention_forms_agree(name, S, dtype):
     """Round 5: the two other schedules of the prompt attention — K / V tiles by LDS-DMA with the next tile's scores under the current softmax (head_dim 64,
     kernels/attn_prefill_dma.h: the same matrix instructions on the same operands in the same order -> BIT-identical) and the key split inside the workgroup
     (attn_prefill_kernel KP = 2: the odd tiles' online-softmax stream merged once at the end -> another fp32 summation order, 2e-5 on one layer) — forced on prompts
-    that are ragged in the 128-query blocks and in the 64-key tiles.  The defaults take these forms only for long prompts / head_dim 128."""
+    that are ragged in the 128-query blocks and in the 64-key tiles.  The defaults take these forms only for long prompts / head_dim 128.  The key split runs in blocks of 64 queries
+    while those of 128 do not outnumber the compute units (up to 1024 rows of 32 heads), in blocks of 128 beyond: the two longest prompts."""
     d = copy.deepcopy(known_desc(name, dtype))
     d.layers, d.vocab, d.max_ctx = 1, 4096, S + 16
     m = Model(d, product_backend()).load_synthetic(1234, 0.02).finalize()
