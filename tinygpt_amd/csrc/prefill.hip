@@ -106,7 +106,7 @@ static void launch_gemm(tgx_ctx* c, int epi, const ebyte* B_, const ebyte* bias_
   const bool qkv_nosplit = qkv_bal && c->qkv_nosplit && qkv_wgs >= c->num_cus;
   const bool silu8 = epi == tgx::GEMM_SILU && (c->gemm_dma & 8) && K % 64 == 0 && !three_terms && tgx::gate_up_whole(M, N, K, c->num_cus, c->wide_8k_max);      // (whole: no slabs, no reduce launch)
   if (c->gemm_splitk && ntiles < c->num_cus && K % tgx::GBK == 0 && !qkv_nosplit && !silu8) nsplit = std::min(std::min(16, ktiles), (2 * c->num_cus + ntiles - 1) / ntiles);
-  // N = hidden products of a 129-1500-row prompt (round 4, option prefill.splitk_8k): their 128 x 128 tiles number less than a chip (Llama-3.2-1B S = 1024: 128 tiles on 256
+  // N = hidden products of a 129-1500-row prompt (option prefill.splitk_8k): their 128 x 128 tiles number less than a chip (Llama-3.2-1B S = 1024: 128 tiles on 256
   // CUs, 84 us per product against 104 at twice the rows) — the eight-wave LDS-DMA kernel over 2-8 K slabs instead of 64-row register-staged slabs or a half-empty chip
   bool part_8k = false;
   if (c->gemm_splitk && c->splitk_8k && (c->gemm_dma & 8) && K % 64 == 0 && !three_terms && (epi == tgx::GEMM_RESIDUAL || epi == tgx::GEMM_STORE) && M > 128) {

@@ -29,7 +29,7 @@ inline int eight_wave_slabs(int M, int N, int K, int num_cus) {
 // chip of tiles on, a longer one from half a chip on, where slabs would go into another round.  Whole / split, ms per prompt: Qwen3-0.6B (K 1024) 133 tokens (96 tiles) 2.68 / 2.78, 256
 // 2.98 / 3.21, 509 (192) 3.45 / 3.92; Qwen2.5-0.5B 133 (152) 2.07 / 2.27, 384 (228) 2.49 / 2.99.  Whole less split, us a layer: K 512 and 1024, 129 to 512 rows, 64 to 240 tiles -0.7 to
 // -21; K 2048, 129 to 512 rows, 64 tiles +5 to +7, 96 -4 to +2, 128 -3 to 0, 144 to 240 -14 to -28; K 2560, 3072 and 4096, 65 to 200 rows, 64 tiles +14 to +21, 96 -2 to +2, 128 +1 to
-// +7, 152 -8 to -18, 192 -17 to -33, 224 -20 to -37.  Up to 64 rows the slabs have tiles of 64 rows and nothing of it is padding.
+// +7, 152 -8 to -18, 192 -17 to -33, 224 -20 to -37 (profiles/prompt_gate_up_whole.txt).  Up to 64 rows the slabs have tiles of 64 rows and nothing of it is padding.
 inline bool gate_up_whole(int M, int N, int K, int num_cus, int most) {
   const long long tiles = (long long)((N + 127) / 128) * ((M + 127) / 128);
   if (M <= 64 || tiles >= num_cus || 2 * tiles > (long long)most * num_cus) return false;
