@@ -1,0 +1,106 @@
+"""The recurrences in blocks of 32 tokens (option rec.min) against the plain oracles and against the token by token scan: wkv and the delta rule (Vitudra), the delta rule with a decay
+per channel (Keronex), at the edges of blocks, of the matrix cores' tiles and of the state's tiles; portions that continue a state; several requests of unequal length in one step; decays
+of zero and products of decays that underflow inside a block; and without scratch.  fp32 storage, 1e-4 of the largest logit, as for these designs' other forms."""
+import numpy as np
+import pytest
+
+import test_hip_keronex as tk
+import test_hip_vitudra as tv
+
+pytestmark = pytest.mark.gpu
+HEADS = [(4, 5), (12, 16), (64, 17), (68, 64), (128, 33)]      # key and value channels
+
+
+def model(kind, dim, vdim, over=None, **kw):
+    """(engine, tokens -> wanted logits, config) of two layers of the recurrence around a plain one"""
+    if kind == "cdelta":
+        cfg = tk.config([tk.cd(tk.dense(), dim=dim, vdim=vdim), tk.ret(), tk.cd(dim=dim, vdim=vdim, heads=2, kv_heads=2)])
+        eng, w = tk.engine(cfg, "fp32", 3, over, **kw)
+        return eng, lambda t: tk.want_of(cfg, w, t), cfg
+    layers = ([tv.wkv(tv.ff(), heads=3, dim=dim), tv.attn(tv.ff()), tv.wkv(heads=2, dim=dim)] if kind == "wkv" else
+              [tv.par(tv.ff(), right=dict(dim=dim, vdim=vdim)), tv.attn(tv.ff()), tv.par(right=dict(dim=dim, vdim=vdim, heads=2, kv_heads=1))])
+    cfg = tv.config(layers)
+    eng, w = tv.engine(cfg, "fp32", 3, over, **kw)
+    return eng, lambda t: tv.want_of(cfg, w, t), cfg
+
+
+def close(got, want, what=""):
+    err = np.abs(got - want).max() / np.abs(want).max()
+    assert err < 1e-4, f"{what}: {err:.3e}"
+
+
+def by_portions(eng, rid, toks, sizes):
+    got, at = [], 0
+    for n in sizes:
+        got.append(eng.step([(rid, toks[at:at + n], list(range(n)))]))
+        at += n
+    return np.concatenate(got)
+
+
+@pytest.mark.parametrize("dim,vdim", HEADS)
+@pytest.mark.parametrize("kind", ["wkv", "delta", "cdelta"])
+def test_blocks_equal_the_oracle_and_the_scan(kind, dim, vdim):
+    """one portion over a few blocks, and the same tokens in portions that end in, on and behind a block's edge (a state that goes on, blocks of one token, tails of a block)"""
+    eng, want_of, cfg = model(kind, dim, vdim)
+    toks = tk.tokens(cfg, 131, seed=dim)
+    want = want_of(toks)
+    eng.model.set_option("rec.min", 0)
+    scan = by_portions(eng, "a", toks, [131])
+    eng.model.set_option("rec.min", 1)
+    blocks = by_portions(eng, "b", toks, [131])
+    close(scan, want, "scan")
+    close(blocks, want, "blocks")
+    assert not np.array_equal(scan, blocks)      # (another order of sums: both forms ran)
+    close(by_portions(eng, "c", toks, [33, 31, 1, 2, 63, 1]), want, "portions")
+    eng.close()
+
+
+@pytest.mark.parametrize("kind", ["wkv", "delta", "cdelta"])
+def test_requests_of_unequal_length_in_one_step(kind):
+    eng, want_of, cfg = model(kind, 64, 64)
+    eng.model.set_option("rec.min", 1)
+    sizes = [1, 97, 32, 45]
+    seqs = [tk.tokens(cfg, n + 40, seed=n) for n in sizes]
+    first = eng.step([("r%d" % i, s[:n], list(range(n))) for i, (s, n) in enumerate(zip(seqs, sizes))])
+    second = eng.step([("r%d" % i, s[n:], list(range(40))) for i, (s, n) in enumerate(zip(seqs, sizes))])
+    at = 0
+    for i, (s, n) in enumerate(zip(seqs, sizes)):
+        want = want_of(s)
+        close(first[at:at + n], want[:n], "first %d" % n)
+        close(second[40 * i:40 * i + 40], want[n:], "second %d" % n)
+        at += n
+    eng.close()
+
+
+@pytest.mark.parametrize("strength", [1.5, 3.0, 6.0])      # decays of 1e-2, 2e-9 (a block's product underflows) and zero a token
+@pytest.mark.parametrize("kind", ["wkv", "delta", "cdelta"])
+def test_strong_decays(kind, strength):
+    names = {"wkv": ("l0.mix.w0",), "delta": ("l0.mix.right.A_log",), "cdelta": ("l0.mix.A_log",)}[kind]
+    import keronex_oracle as ko
+    import vitudra_oracle as vo
+    eng, _, cfg = model(kind, 64, 32)
+    w0 = (ko.random_tensors(cfg, 3, None, 5, 7) if kind == "cdelta" else vo.random_tensors(cfg, 3))
+    eng.close()
+    over = {}
+    for n in names:
+        v = w0[n].copy()
+        v.reshape(-1)[::2] = strength      # every other channel or head keeps its own
+        over[n] = v
+    eng, want_of, cfg = model(kind, 64, 32, over)
+    eng.model.set_option("rec.min", 1)
+    toks = tk.tokens(cfg, 100, seed=9)
+    close(by_portions(eng, "r", toks, [70, 30]), want_of(toks))
+    eng.close()
+
+
+@pytest.mark.parametrize("kind", ["wkv", "delta", "cdelta"])
+def test_without_scratch_the_scan_takes_over(kind):
+    eng, want_of, cfg = model(kind, 64, 64)
+    toks = tk.tokens(cfg, 100, seed=2)
+    eng.model.set_option("ssd.min", 0)      # (the retention between takes scratch of its own)
+    eng.model.set_option("rec.min", 0)
+    scan = by_portions(eng, "a", toks, [100])
+    eng.model.set_option("stack.ws_max", 1)
+    eng.model.set_option("rec.min", 1)
+    assert np.array_equal(by_portions(eng, "b", toks, [100]), scan)
+    eng.close()

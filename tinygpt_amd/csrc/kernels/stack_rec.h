@@ -14,6 +14,7 @@
 // A sequence whose first token has position 0 starts from zero state whatever its slot held.
 #pragma once
 #include "stack.h"
+#include "stack_rec_args.h"
 
 namespace tgx {
 
@@ -143,20 +144,6 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(StepMeta m, DeltaPrepAr
 // fewer instructions in all; two tokens go without a branch between them, so that the one's sum over the groups lies under the other's arithmetic; and a column's outputs are kept by its
 // row groups, a token each, and leave in one store for as many tokens as there are groups.  2048 tokens, delta rule of 16 heads of 128 x 128: 632 us at eight row groups staged number
 // by number, 578 staged in vectors of four, 470 at sixteen with a store a token, 340 at thirty-two and stores by the block; wkv of 32 heads of 64 x 64 419, 409, 335, 257 (sixteen groups).
-enum { REC_WKV = 0, REC_DELTA = 1, REC_SSD = 2, REC_CDELTA = 3 };
-struct RecScanArgs {
-  const float* a; long long lda;     // per token and key head [dim]: the read vector (wkv: r, delta: q, ssd: C)
-  const float* k; long long ldk;     //                               k (ssd: B)
-  const float* w; long long ldw;     //                               wkv: the decay per channel; cdelta: per (query) head and channel
-  const float* v; long long ldv;     // per token and head [vdim]
-  const float* beta; const float* g; long long ldg;      // delta, ssd: per token and head (cdelta: beta alone)
-  const float* fixed; float beta0;   // ssd: [heads] decays that hold for every token, with beta0 as every token's beta (nullptr: beta and g)
-  const float* u;                    // wkv: [heads][dim] bonus
-  const float* skip;                 // ssd: [heads] (nullptr: none)
-  float* S;                          // [slots][heads][dim][vdim]
-  float* out; long long ldo;         // [T][heads * vdim]
-  int heads, kv_heads, dim, vdim;
-};
 constexpr int rec_cols(int rg) { return 4 * (64 / rg); }      // columns per workgroup
 template <int DPER, int KIND, int RG, bool VEC>
 __global__ __launch_bounds__(256) void rec_scan_kernel(StepMeta m, RecScanArgs a) {

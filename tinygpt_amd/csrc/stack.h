@@ -154,6 +154,7 @@ struct StackModel {
   int mlstm_narrow = -1;               // option mlstm.narrow: the matrix-memory scan's columns per wave (1: eight, 0: sixteen, -1: by the step's entries and heads)
   int rec_step = 1;                    // option stack.rec_step: 0 keeps a step's recurrences in their own launches (convolution, scan, norm and gate)
   int ssd_min = 64;                    // option ssd.min: portions from this many tokens on take the blocked form of the scalar-decay recurrence (0: never)
+  int rec_min = -1;                    // option rec.min: portions from this many tokens on take the blocked form of the other recurrences (0: never, -1: by the portions and heads)
   int mix_groups = 0;                  // option attn.mix_groups: key / value heads per workgroup of the matrix-core sigmoid attention: 1; 2 where their accumulators fit, whatever the grid; 0: 2 while the halved grid fills the chip
   std::set<const void*> lds_kernels;   // kernels that may take the whole LDS of a compute unit on this context's device
   size_t part_ask = 0, terms_cols = 0, terms2_cols = 0;      // what part can come to hold for divided keys; elements of one term that a token's row of terms and terms2 can come to hold (scratch_sizes)
@@ -193,6 +194,11 @@ bool ssd_mfma_shapes_ok(int heads, int groups, int N, int E, long long ld);
 size_t ssd_gram_elems(int T, int S, int groups);
 void launch_ssd_mfma(tgx_ctx* c, const tgx::StepMeta& m, const tgx::SsdArgs& a, int S, int max_count);
 void launch_gate_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::GateScanArgs& a, int S);
+
+// stack_recblk.hip
+namespace tgx { struct RecScanArgs; }
+size_t rec_block_elems(int T, int S, int heads, int dim, int vdim, bool solve);
+void launch_rec_blocks(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs& a, int kind, int S, int max_count, float* scratch);
 
 int stack_create(const tgx_stack_desc* desc, const tgx_layer_desc* layers, int device_ordinal, tgx_ctx** out_ctx);
 int stack_upload(tgx_ctx* c, const char* name, const void* host, const int64_t* shape, int nd, int src_dtype);

@@ -884,8 +884,12 @@ struct JointLayer {
   }
 };
 
+// whether a token's read, key and decay vectors are read four numbers at a time
+bool rec_vec(const tgx::RecScanArgs& a) {
+  return a.dim % 4 == 0 && a.lda % 4 == 0 && a.ldk % 4 == 0 && (uintptr_t)a.a % 16 == 0 && (uintptr_t)a.k % 16 == 0 && (!a.w || (a.ldw % 4 == 0 && (uintptr_t)a.w % 16 == 0));
+}
 void launch_rec_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs& a, int kind, int S) {
-  const bool vec = a.dim % 4 == 0 && a.lda % 4 == 0 && a.ldk % 4 == 0 && (uintptr_t)a.a % 16 == 0 && (uintptr_t)a.k % 16 == 0 && (!a.w || (a.ldw % 4 == 0 && (uintptr_t)a.w % 16 == 0));
+  const bool vec = rec_vec(a);
   // sixteen row groups per column while their workgroups, of sixteen columns, leave a compute unit with two at most: one prompt of 16 heads of 128 (kernels/stack_rec.h), a few
   // requests; thirty-two, of four rows, while there is a compute unit for each of theirs (one prompt of 16 heads of 128 x 128: 340 us against sixteen's 400 for 2048 tokens; a SIMD
   // with two of their waves would issue more than with one of sixteen groups'); a full chip issues fewer instructions with eight
@@ -912,6 +916,24 @@ void launch_rec_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs&
   else if (kind == tgx::REC_CDELTA) go(std::integral_constant<int, tgx::REC_CDELTA>{});
   else if (kind == tgx::REC_SSD) go(std::integral_constant<int, tgx::REC_SSD>{});
   else go(std::integral_constant<int, tgx::REC_DELTA>{});
+}
+
+// A recurrence over portions: in blocks of 32 tokens on the matrix cores (kernels/stack_rec_block.h) or token by token.  The blocks take the chain of a long portion, but move two to
+// three times the scan's bytes, so they are for portions of which the chain is what bounds them: long ones, while their workgroups (16 value channels each) are few to a compute unit.
+// us of a layer, blocks / scan.  wkv (heads of 64): one prompt of 96 tokens 16 / 15, 160 20 / 23, 2048 102 / 258; 2 workgroups a compute unit 66 / 80 and 39 / 42, 4 133 / 118 and
+// 70 / 62.  Delta rules (heads of 128 x 128): 96 tokens 25 / 20, 160 27 / 29, 2048 159 / 340; with a decay a channel 26 / 20, 28 / 31; 4 a compute unit 95 / 96, 177 / 189 and 98 / 107,
+// 8 209 / 181 and 222 / 201.
+constexpr int REC_WKV_BLOCK_MIN = 128, REC_DELTA_BLOCK_MIN = 160, REC_WKV_BLOCK_WGS = 2, REC_DELTA_BLOCK_WGS = 4;
+void launch_recurrence(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs& a, int kind, int T, int S, int max_count) {
+  StackModel* sm = c->stack;
+  const bool wkv = kind == tgx::REC_WKV;
+  const long long wgs = (long long)S * a.heads * ((a.vdim + 15) / 16);
+  const bool pays = sm->rec_min >= 0 ? sm->rec_min > 0 && max_count >= sm->rec_min
+                                     : max_count >= (wkv ? REC_WKV_BLOCK_MIN : REC_DELTA_BLOCK_MIN) && wgs <= (long long)(wkv ? REC_WKV_BLOCK_WGS : REC_DELTA_BLOCK_WGS) * c->num_cus;
+  if (pays && rec_vec(a) && a.dim <= 128 && a.vdim <= 256 &&
+      ensure_part(c, rec_block_elems(T, S, a.heads, a.dim, a.vdim, !wkv), rec_block_elems(sm->cap_tokens, sm->d.max_seqs, a.heads, a.dim, a.vdim, !wkv)))
+    launch_rec_blocks(c, m, a, kind, S, max_count, sm->part);
+  else launch_rec_scan(c, m, a, kind, S);
 }
 
 // a step of single tokens: the recurrence with what makes its inputs and finishes its outputs in one launch (kernels/stack_step.h), where the head's sizes allow; false: not launched
@@ -991,7 +1013,7 @@ void run_wkv(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer& jl,
     g = tgx::StackGemmArgs{};
     g.A = sm->lora; g.lda = R; g.B = w.w_w2; g.ldb = R; g.C = sm->proj + 4 * (size_t)HD; g.ldc = 5LL * HD; g.M = T; g.N = HD; g.K = R; g.scale = 1.f; g.bias = w.w0; g.act = tgx::SG_ACT_DECAY;
     launch_gemm(c, g, tgx::SG_STORE, 1);
-    launch_rec_scan(c, m, ra, tgx::REC_WKV, S);
+    launch_recurrence(c, m, ra, tgx::REC_WKV, T, S, max_count);
     hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, H), dim3(64), 0, c->stream, oa);
   }
   jl.add(c, to_stream(c, sm->o, HD, w.w_o, T, sm->d.residual_mult));
@@ -1043,7 +1065,7 @@ int run_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer&
     left_out();      // (unmerged layers' outputs are added here, before the right half takes their place)
     if (!launch_rec_step(c, m, st, tgx::REC_DELTA, S, max_count)) {
       hipLaunchKernelGGL(tgx::delta_prep_kernel, dim3(T, 2 * rG + rH + 1), dim3(256), 0, c->stream, m, dp);
-      launch_rec_scan(c, m, ra, tgx::REC_DELTA, S);
+      launch_recurrence(c, m, ra, tgx::REC_DELTA, T, S, max_count);
       hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, rH), dim3(64), 0, c->stream, oa);
     }
   }
@@ -1954,7 +1976,7 @@ void run_channel_delta(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T
   st.s = ra; st.p = dp; st.prep = 1; st.g = oa;
   if (!launch_rec_step(c, m, st, tgx::REC_CDELTA, S, max_count)) {
     hipLaunchKernelGGL(tgx::delta_prep_kernel, dim3(T, 2 * ld.kv_heads + ld.heads + 1), dim3(256), 0, c->stream, m, dp);
-    launch_rec_scan(c, m, ra, tgx::REC_CDELTA, S);
+    launch_recurrence(c, m, ra, tgx::REC_CDELTA, T, S, max_count);
     hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, ld.heads), dim3(64), 0, c->stream, oa);
   }
   sublayer_out(c, sm->o, k.HE, w.w_o, T);
