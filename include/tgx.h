@@ -486,7 +486,7 @@ TGX_API int tgx_set_logits(tgx_ctx* ctx, const float* logits, int batch);
  *                  tgx_reset_row / tgx_reset_cache; max_ctx stays the per-row limit.  A call that would need a block when none is free returns TGX_ERR_CONTEXT and
  *                  changes nothing (retire a row, retry).  Results are those of the unpaged cache, bit for bit on the same kernels (tests/test_hip_paged.py);
  *                  tgx_get_option "kv.free_tokens" = the unassigned blocks' worth of tokens (-1 when unpaged)
- *   "attn.split_min", "attn.gqa_split_min", "attn.mfma", "stack.gemv", "stack.rec_step", "stack.line", "stack.gemm_wt", "mlstm.narrow", "attn.mix_groups", "ssd.min", "rec.min"  (layered models) keys a workgroup walks from which a step of few
+ *   "attn.split_min", "attn.gqa_split_min", "attn.mfma", "stack.gemv", "stack.rec_step", "stack.line", "stack.gemm_wt", "mlstm.narrow", "attn.mix_groups", "ssd.min", "rec.min", "stack.conv_tiles"  (layered models) keys a workgroup walks from which a step of few
  *                  tokens divides them between workgroups (four thresholds: 128 on the matrix cores, 2048 on the lane kernels for latent rows, 1024 for grouped queries, counted in a
  *                  mask's span.  The first key sets all four, the second the grouped-query ones; a negative value brings the defaults back; tgx_get_option gives the
  *                  one in force, the matrix cores' where any layer's attention runs there);
@@ -494,7 +494,7 @@ TGX_API int tgx_set_logits(tgx_ctx* ctx, const float* logits, int batch);
  *                  0 = prompts' products on the register-staged tiles; forced product tile; the mLSTM scan's column split;
  *                  key / value heads per workgroup of the matrix-core sigmoid attention (1; 2 = two where their accumulators fit; 0 = two while the halved grid fills the chip);
  *                  tokens of a portion from which a scalar-decay recurrence runs in blocks on the matrix cores (0 = never); the same for delta rules and a decay per channel (-1 = by the
- *                  portions and heads)
+ *                  portions and heads); 1 / 0 = the recurrences' filters in tiles of tokens always / never (-1 = by the step's size)
  *   "stack.ws_max" (layered models) most KiB of each scratch buffer that divided keys, blocked recurrences and prompts' products ask for (-1: as memory allows); what would need more,
  *                  or finds no memory, takes its form without scratch; tgx_get_option "stack.ws_grown" = how often the context has allocated them
  *   "debug.refuse_lds"  (layered models, tests) the n-th product from now that asks for its LDS is refused it: its step fails half-way, TGX_ERR_UNSUPPORTED

@@ -1287,6 +1287,7 @@ int tgx_set_option(tgx_ctx* c, const char* key, int value) {
     if (!strcmp(key, "attn.mix_groups")) { c->stack->mix_groups = value == 1 || value == 2 ? value : 0; return TGX_OK; }      // key / value heads per workgroup of the matrix-core sigmoid attention: 1, 2 (where they fit, whatever the grid), 0 = by the grid
     if (!strcmp(key, "ssd.min")) { c->stack->ssd_min = value < 0 ? 0 : value; return TGX_OK; }      // tokens of a portion from which the scalar-decay recurrence runs in blocks on the matrix cores (0: never)
     if (!strcmp(key, "rec.min")) { c->stack->rec_min = value < 0 ? -1 : value; return TGX_OK; }      // ... from which a delta rule or a recurrence with a decay per channel does (0: never, -1: automatic)
+    if (!strcmp(key, "stack.conv_tiles")) { c->stack->conv_tiles = value < 0 ? -1 : (value != 0); return TGX_OK; }      // filters in front of the recurrences in tiles of tokens (-1: automatic)
     if (!strcmp(key, "stack.rec_step")) { c->stack->rec_step = value ? 1 : 0; return TGX_OK; }      // 0: single tokens in the launches of a longer portion
     if (!strcmp(key, "stack.gemv")) { c->stack->gemv = value != 0; return TGX_OK; }      // 0: products of few rows on the matrix-core tiles too
     if (!strcmp(key, "stack.line")) { c->stack->line = value != 0; return TGX_OK; }      // 0: prompts' products on the register-staged tiles

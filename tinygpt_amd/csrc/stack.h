@@ -155,6 +155,7 @@ struct StackModel {
   int rec_step = 1;                    // option stack.rec_step: 0 keeps a step's recurrences in their own launches (convolution, scan, norm and gate)
   int ssd_min = 64;                    // option ssd.min: portions from this many tokens on take the blocked form of the scalar-decay recurrence (0: never)
   int rec_min = -1;                    // option rec.min: portions from this many tokens on take the blocked form of the other recurrences (0: never, -1: by the portions and heads)
+  int conv_tiles = -1;                 // option stack.conv_tiles: 1 / 0 = convolutions in front of the recurrences in tiles of tokens always / never, -1 by the step's tokens and channels
   int mix_groups = 0;                  // option attn.mix_groups: key / value heads per workgroup of the matrix-core sigmoid attention: 1; 2 where their accumulators fit, whatever the grid; 0: 2 while the halved grid fills the chip
   std::set<const void*> lds_kernels;   // kernels that may take the whole LDS of a compute unit on this context's device
   size_t part_ask = 0, terms_cols = 0, terms2_cols = 0;      // what part can come to hold for divided keys; elements of one term that a token's row of terms and terms2 can come to hold (scratch_sizes)

@@ -21,6 +21,7 @@
 #include "kernels/stack_loop.h"
 #include "kernels/stack_mix_mfma.h"
 #include "kernels/stack_ssm.h"
+#include "kernels/stack_conv.h"
 #include "kernels/stack_ssd_mfma.h"
 #include "kernels/stack_hyper.h"
 
@@ -884,6 +885,35 @@ struct JointLayer {
   }
 };
 
+// Convolutions in tiles of eight tokens of four channels a lane (kernels/stack_conv.h) from so many (token, channel) numbers on, where rows and channels are whole fours; shorter steps keep
+// a channel a thread, whose workgroups then run all at once and whose waves have an eighth to do.  us, a channel a thread / in tiles: delta rule's inputs of 2048 channels 128 tokens 5.2 /
+// 8.8, 300 9.9 / 8.8, 1600 36 / 13, 2048 tokens of 4096 89 / 20; filters of 2048 channels 300 tokens 4.8 / 8.0, 2000 15.5 / 12.0, 10917 tokens of 4096 135 / 88
+constexpr long long DELTA_TILES_MIN = 1 << 19, CONV_TILES_MIN = 1 << 21;
+bool conv_tiles(const tgx_ctx* c, int T, int C, long long min) { const int o = c->stack->conv_tiles; return C % 4 == 0 && (o >= 0 ? o != 0 : (long long)T * C >= min); }
+bool fours(const void* p, long long ld) { return (uintptr_t)p % 16 == 0 && ld % 4 == 0; }
+template <class F>
+bool two_to_four_taps(int taps, F f) {
+  switch (taps) {
+    case 2: f(std::integral_constant<int, 2>{}); return true;
+    case 3: f(std::integral_constant<int, 3>{}); return true;
+    case 4: f(std::integral_constant<int, 4>{}); return true;
+    default: return false;
+  }
+}
+void launch_delta_prep(tgx_ctx* c, const tgx::StepMeta& m, const tgx::DeltaPrepArgs& a, int T) {
+  const int C = 2 * a.kv_heads * a.dim + a.heads * a.vdim;
+  if (conv_tiles(c, T, C, DELTA_TILES_MIN) && (a.dim == 32 || a.dim == 64 || a.dim == 128) && fours(a.proj + a.col0, a.ldp) && fours(a.out, a.ldo) && fours(a.cw, 0) && fours(a.state, (long long)a.state_buf)) {
+    const dim3 grid((T + tgx::CONV_WG_TOK - 1) / tgx::CONV_WG_TOK, (C + tgx::CONV_WG_CH - 1) / tgx::CONV_WG_CH + 1);
+    if (two_to_four_taps(a.taps, [&](auto TAPS) {
+          constexpr int N = decltype(TAPS)::value;
+          if (a.dim == 128) hipLaunchKernelGGL((tgx::delta_prep_tiles_kernel<N, 32>), grid, dim3(256), 0, c->stream, m, a);
+          else if (a.dim == 64) hipLaunchKernelGGL((tgx::delta_prep_tiles_kernel<N, 16>), grid, dim3(256), 0, c->stream, m, a);
+          else hipLaunchKernelGGL((tgx::delta_prep_tiles_kernel<N, 8>), grid, dim3(256), 0, c->stream, m, a);
+        })) return;
+  }
+  hipLaunchKernelGGL(tgx::delta_prep_kernel, dim3(T, 2 * a.kv_heads + a.heads + 1), dim3(256), 0, c->stream, m, a);
+}
+
 // whether a token's read, key and decay vectors are read four numbers at a time
 bool rec_vec(const tgx::RecScanArgs& a) {
   return a.dim % 4 == 0 && a.lda % 4 == 0 && a.ldk % 4 == 0 && (uintptr_t)a.a % 16 == 0 && (uintptr_t)a.k % 16 == 0 && (!a.w || (a.ldw % 4 == 0 && (uintptr_t)a.w % 16 == 0));
@@ -1064,7 +1094,7 @@ int run_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer&
     if (rc) return rc;
     left_out();      // (unmerged layers' outputs are added here, before the right half takes their place)
     if (!launch_rec_step(c, m, st, tgx::REC_DELTA, S, max_count)) {
-      hipLaunchKernelGGL(tgx::delta_prep_kernel, dim3(T, 2 * rG + rH + 1), dim3(256), 0, c->stream, m, dp);
+      launch_delta_prep(c, m, dp, T);
       launch_recurrence(c, m, ra, tgx::REC_DELTA, T, S, max_count);
       hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, rH), dim3(64), 0, c->stream, oa);
     }
@@ -1583,6 +1613,10 @@ void post_norm_add(tgx_ctx* c, const float* w, int T, const tgx::RowTerms& terms
 }
 void launch_conv_silu(tgx_ctx* c, const tgx::StepMeta& m, tgx::ConvSiluArgs a, int T) {
   const int cols = (a.C + 255) / 256 + (a.heads > 0 ? 1 : 0);
+  if (conv_tiles(c, T, a.C, CONV_TILES_MIN) && fours(a.proj + a.col0, a.ldp) && fours(a.out, a.ldo) && fours(a.cw, 0) && fours(a.cb, 0) && fours(a.state, (long long)a.state_buf)) {
+    const dim3 grid((T + tgx::CONV_WG_TOK - 1) / tgx::CONV_WG_TOK, cols);
+    if (two_to_four_taps(a.taps, [&](auto TAPS) { hipLaunchKernelGGL(tgx::conv_silu_tiles_kernel<decltype(TAPS)::value>, grid, dim3(256), 0, c->stream, m, a); })) return;
+  }
   a.tile = (long long)T * cols >= 16LL * c->num_cus ? 8 : 1;      // tokens per workgroup: rows are kept in registers from token to token once the grid fills the chip
   const dim3 grid((T + a.tile - 1) / a.tile, cols);
   switch (a.taps) {
@@ -1975,7 +2009,7 @@ void run_channel_delta(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T
   tgx::RecStepArgs st{};
   st.s = ra; st.p = dp; st.prep = 1; st.g = oa;
   if (!launch_rec_step(c, m, st, tgx::REC_CDELTA, S, max_count)) {
-    hipLaunchKernelGGL(tgx::delta_prep_kernel, dim3(T, 2 * ld.kv_heads + ld.heads + 1), dim3(256), 0, c->stream, m, dp);
+    launch_delta_prep(c, m, dp, T);
     launch_recurrence(c, m, ra, tgx::REC_CDELTA, T, S, max_count);
     hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, ld.heads), dim3(64), 0, c->stream, oa);
   }
