@@ -494,7 +494,7 @@ TGX_API int tgx_set_logits(tgx_ctx* ctx, const float* logits, int batch);
  *                  0 = prompts' products on the register-staged tiles; forced product tile; the mLSTM scan's column split;
  *                  key / value heads per workgroup of the matrix-core sigmoid attention (1; 2 = two where their accumulators fit; 0 = two while the halved grid fills the chip);
  *                  tokens of a portion from which a scalar-decay recurrence runs in blocks on the matrix cores (0 = never); the same for delta rules and a decay per channel (-1 = by the
- *                  portions and heads); 1 / 0 = the recurrences' filters in tiles of tokens always / never (-1 = by the step's size)
+ *                  portions and heads, 0 with stack.line 0); 1 / 0 = the recurrences' filters in tiles of tokens always / never (-1 = by the step's size)
  *   "stack.ws_max" (layered models) most KiB of each scratch buffer that divided keys, blocked recurrences and prompts' products ask for (-1: as memory allows); what would need more,
  *                  or finds no memory, takes its form without scratch; tgx_get_option "stack.ws_grown" = how often the context has allocated them
  *   "debug.refuse_lds"  (layered models, tests) the n-th product from now that asks for its LDS is refused it: its step fails half-way, TGX_ERR_UNSUPPORTED

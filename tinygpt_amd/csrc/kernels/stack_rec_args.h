@@ -17,5 +17,6 @@ struct RecScanArgs {
   float* out; long long ldo;         // [T][heads * vdim]
   int heads, kv_heads, dim, vdim;
 };
+constexpr int REC_BLOCK = 32, REC_BLOCK_MAX_DIM = 128, REC_BLOCK_MAX_VDIM = 256;      // tokens of a block; the largest head that blocks take
 
 }  // namespace tgx

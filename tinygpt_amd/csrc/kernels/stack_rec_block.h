@@ -23,7 +23,6 @@
 namespace tgx {
 
 typedef __attribute__((ext_vector_type(2))) float f32x2;
-constexpr int REC_BLOCK = 32;
 // a (block, head)'s part of the scratch, in floats.  Q, K, W: the matrix cores' fragments [16-channel tile][16-token tile][lane][4] (Q, W: lane = 16 (d % 16 / 4) + t % 16, four
 // channels; K: lane = 16 (t % 16 / 4) + d % 16, four tokens); U: [16-column tile][16-token tile][lane = 16 (t % 16 / 4) + e % 16][4 tokens]; P: [i % 4][lane = 16 (i % 16 / 4) + t % 16]
 // [2 (t / 16) + i / 16]; G: D(0, 32) per channel

@@ -159,6 +159,7 @@ struct StackModel {
   int mix_groups = 0;                  // option attn.mix_groups: key / value heads per workgroup of the matrix-core sigmoid attention: 1; 2 where their accumulators fit, whatever the grid; 0: 2 while the halved grid fills the chip
   std::set<const void*> lds_kernels;   // kernels that may take the whole LDS of a compute unit on this context's device
   size_t part_ask = 0, terms_cols = 0, terms2_cols = 0;      // what part can come to hold for divided keys; elements of one term that a token's row of terms and terms2 can come to hold (scratch_sizes)
+  size_t rec_block_most = 0;           // floats of scratch that a block of any layer's recurrence takes, all heads
   size_t terms_most = 0;               // ... of any product's input, whichever form it takes
   size_t ws_refused = SIZE_MAX;        // bytes that this step has asked for in vain
   int ws_grown = 0;                    // tgx_get_option stack.ws_grown: how often part, terms and terms2 were allocated
@@ -198,7 +199,7 @@ void launch_gate_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::GateScanArg
 
 // stack_recblk.hip
 namespace tgx { struct RecScanArgs; }
-size_t rec_block_elems(int T, int S, int heads, int dim, int vdim, bool solve);
+size_t rec_block_elems(size_t blocks, int heads, int dim, int vdim, bool solve);
 void launch_rec_blocks(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs& a, int kind, int S, int max_count, float* scratch);
 
 int stack_create(const tgx_stack_desc* desc, const tgx_layer_desc* layers, int device_ordinal, tgx_ctx** out_ctx);

@@ -150,7 +150,11 @@ bool ensure_terms(tgx_ctx* c, size_t need) {
   if (sm->in_terms) return sm->in_terms_elems + need <= sm->terms_elems;
   return ensure_scratch(c, sm->terms, sm->terms_elems, need, 2 * (size_t)sm->cap_tokens * (sm->joint || sm->post ? sm->terms_most + sm->d.width : sm->terms_cols));
 }
-bool ensure_terms2(tgx_ctx* c, size_t need) { StackModel* sm = c->stack; return ensure_scratch(c, sm->terms2, sm->terms2_elems, need, 2 * (size_t)sm->cap_tokens * sm->terms2_cols); }
+// (a feed-forward's hidden values, and before them a blocked recurrence's blocks: one buffer for the layer's two halves)
+bool ensure_terms2(tgx_ctx* c, size_t need) {
+  StackModel* sm = c->stack;
+  return ensure_scratch(c, sm->terms2, sm->terms2_elems, need, std::max(2 * (size_t)sm->cap_tokens * sm->terms2_cols, 2 * ((size_t)sm->cap_tokens / tgx::REC_BLOCK + (size_t)sm->d.max_seqs) * sm->rec_block_most));
+}
 // what those buffers can come to hold: the sums of the divided keys of any step (tiles of up to 32 rows on twice as many workgroups as there are compute units, a value or
 // latent row and two numbers each; or a token's outputs, heads in a row), and a token's widest product input and hidden row
 void scratch_sizes(tgx_ctx* c) {
@@ -162,6 +166,12 @@ void scratch_sizes(tgx_ctx* c) {
     if (sm->affine || w.pool) sm->part_ask = std::max(sm->part_ask, 2 * (size_t)c->num_cus * std::max(32 * row, (size_t)l.heads * l.vdim));
     cols = std::max(cols, l.mixer == TGX_MIXER_WKV ? 4 * sm->d.width : 0);      // (one split of four of the token shift's five mixes)
     most = std::max({most, l.heads * std::max(l.dim, l.kv_rank), l.heads * l.vdim + l.d_heads * l.d_vdim, l.inner, l.ff, l.shared_ff, l.decay_rank, l.gate_rank, l.dt_rank});
+    auto blocks = [&](int heads, int dim, int vdim, bool solve) {
+      if (dim <= tgx::REC_BLOCK_MAX_DIM && vdim <= tgx::REC_BLOCK_MAX_VDIM) sm->rec_block_most = std::max(sm->rec_block_most, rec_block_elems(1, heads, dim, vdim, solve));
+    };
+    if (l.mixer == TGX_MIXER_WKV) blocks(l.heads, l.dim, l.dim, false);
+    else if (l.mixer == TGX_MIXER_CHANNEL_DELTA) blocks(l.heads, l.dim, l.vdim, true);
+    else if (l.mixer == TGX_MIXER_PARALLEL && sm->joint) blocks(l.d_heads, l.d_dim, l.d_vdim, true);
     sm->terms2_cols = std::max(sm->terms2_cols, (size_t)(l.mlp == TGX_MLP_MOE ? std::max(l.top * l.ff, l.shared_ff) : l.ff));
   }
   sm->terms_cols = (size_t)cols;
@@ -948,21 +958,22 @@ void launch_rec_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs&
   else go(std::integral_constant<int, tgx::REC_DELTA>{});
 }
 
-// A recurrence over portions: in blocks of 32 tokens on the matrix cores (kernels/stack_rec_block.h) or token by token.  The blocks take the chain of a long portion, but move two to
-// three times the scan's bytes, so they are for portions of which the chain is what bounds them: long ones, while their workgroups (16 value channels each) are few to a compute unit.
-// us of a layer, blocks / scan.  wkv (heads of 64): one prompt of 96 tokens 16 / 15, 160 20 / 23, 2048 102 / 258; 2 workgroups a compute unit 66 / 80 and 39 / 42, 4 133 / 118 and
-// 70 / 62.  Delta rules (heads of 128 x 128): 96 tokens 25 / 20, 160 27 / 29, 2048 159 / 340; with a decay a channel 26 / 20, 28 / 31; 4 a compute unit 95 / 96, 177 / 189 and 98 / 107,
-// 8 209 / 181 and 222 / 201.
-constexpr int REC_WKV_BLOCK_MIN = 128, REC_DELTA_BLOCK_MIN = 160, REC_WKV_BLOCK_WGS = 2, REC_DELTA_BLOCK_WGS = 4;
+// A recurrence over portions: in blocks of 32 tokens on the matrix cores (kernels/stack_rec_block.h; their scratch is the hidden values', which come after) or token by token.  The blocks
+// shorten the chain of a long portion, but move two to three times the scan's bytes, so they are for portions of which the chain is what bounds them: long ones, while their workgroups
+// (16 value channels each) are few to a compute unit.  us of a layer, blocks / scan.  wkv (heads of 64): one prompt of 96 tokens 16 / 15, 160 20 / 23, 2048 102 / 258; 2 workgroups a compute
+// unit 66 / 80 and 39 / 42, 4 133 / 118 and 70 / 62.  Delta rules (heads of 128 x 128): 96 tokens 25 / 20, 160 27 / 29, 2048 159 / 340; with a decay a channel 26 / 20, 28 / 31; 4 a
+// compute unit 95 / 96, 177 / 189 and 98 / 107, 8 209 / 181 and 222 / 201.  More workgroups than compute units are bound by all requests' tokens: 4 a compute unit, 120 tokens a
+// request 57 / 55, 250 98 / 107.  Option stack.line 0, which brings the older forms of prompts' products back, brings the scan back as well unless rec.min says otherwise.
+constexpr int REC_WKV_BLOCK_MIN = 128, REC_DELTA_BLOCK_MIN = 160, REC_WKV_BLOCK_WGS = 2, REC_DELTA_BLOCK_WGS = 4, REC_BLOCK_FULL_MEAN = 192;
 void launch_recurrence(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs& a, int kind, int T, int S, int max_count) {
   StackModel* sm = c->stack;
   const bool wkv = kind == tgx::REC_WKV;
   const long long wgs = (long long)S * a.heads * ((a.vdim + 15) / 16);
   const bool pays = sm->rec_min >= 0 ? sm->rec_min > 0 && max_count >= sm->rec_min
-                                     : max_count >= (wkv ? REC_WKV_BLOCK_MIN : REC_DELTA_BLOCK_MIN) && wgs <= (long long)(wkv ? REC_WKV_BLOCK_WGS : REC_DELTA_BLOCK_WGS) * c->num_cus;
-  if (pays && rec_vec(a) && a.dim <= 128 && a.vdim <= 256 &&
-      ensure_part(c, rec_block_elems(T, S, a.heads, a.dim, a.vdim, !wkv), rec_block_elems(sm->cap_tokens, sm->d.max_seqs, a.heads, a.dim, a.vdim, !wkv)))
-    launch_rec_blocks(c, m, a, kind, S, max_count, sm->part);
+                                     : sm->line && max_count >= (wkv ? REC_WKV_BLOCK_MIN : REC_DELTA_BLOCK_MIN) && wgs <= (long long)(wkv ? REC_WKV_BLOCK_WGS : REC_DELTA_BLOCK_WGS) * c->num_cus &&
+                                           (wgs <= c->num_cus || T >= REC_BLOCK_FULL_MEAN * S);
+  if (pays && rec_vec(a) && a.dim <= tgx::REC_BLOCK_MAX_DIM && a.vdim <= tgx::REC_BLOCK_MAX_VDIM && ensure_terms2(c, 2 * rec_block_elems((size_t)T / tgx::REC_BLOCK + (size_t)S, a.heads, a.dim, a.vdim, !wkv)))
+    launch_rec_blocks(c, m, a, kind, S, max_count, reinterpret_cast<float*>(sm->terms2));
   else launch_rec_scan(c, m, a, kind, S);
 }
 

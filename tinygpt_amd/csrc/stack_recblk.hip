@@ -5,7 +5,7 @@
 
 #include "kernels/stack_rec_block.h"
 
-size_t rec_block_elems(int T, int S, int heads, int dim, int vdim, bool solve) { return ((size_t)T / tgx::REC_BLOCK + (size_t)S) * heads * tgx::RecBlockLayout(dim, vdim, solve).stride; }
+size_t rec_block_elems(size_t blocks, int heads, int dim, int vdim, bool solve) { return blocks * (size_t)heads * tgx::RecBlockLayout(dim, vdim, solve).stride; }
 
 void launch_rec_blocks(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs& a, int kind, int S, int max_count, float* scratch) {
   const int nblk = (max_count + tgx::REC_BLOCK - 1) / tgx::REC_BLOCK;
