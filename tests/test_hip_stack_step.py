@@ -167,3 +167,33 @@ def test_latents_beside_their_queries(slots, kv_rank, dim, heads):
     for i in {0, slots // 2, slots - 1}:
         want = so.forward(d, t, seqs[i].tolist())
         assert np.abs(got[i] - want).max() / np.abs(want).max() < 1e-4, (slots, i)
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("width", [24, 1016, 1032, 2056])      # one lane's slices, eight waves with a remainder, four waves, two passes and a remainder
+@pytest.mark.parametrize("rows", [1, 2])
+def test_norms_inside_the_products_of_one_and_two_rows(width, rows, dtype):
+    """the norms in front of a layer and of the output head in the products behind them, against the oracle and against the norms' own launches (stack.gemv 0): one row, two rows of one
+    sequence (the shift's row before is one of the step's) and two sequences of one row"""
+    cfg = tv.config([tv.wkv(tv.ff(16)), tv.par(tv.ff(16)), tv.attn(tv.ff(16))], width=width, vocab=4104)
+    tol = 1e-4 if dtype == "fp32" else 3e-2
+    eng, w = tv.engine(cfg, dtype, seed=4)
+    toks = [tv.tokens(cfg, 8, i) for i in range(2)]
+    want = [tv.want_of(cfg, w, t) for t in toks]
+    for one in (True, False):
+        got = {}
+        for on in (1, 0):
+            eng.model.set_option("stack.gemv", on)
+            out = []
+            for at in range(0, 8, rows if one else 1):
+                e = [("a", toks[0][at:at + rows], list(range(rows)))] if one else [(i, toks[i][at:at + 1], [0]) for i in range(rows)]
+                out.append(eng.step(e))
+            for r in (["a"] if one else range(rows)):
+                eng.release(r)
+            got[on] = np.concatenate(out)
+        ref = want[0] if one else np.stack(want[:rows], 1).reshape(-1, want[0].shape[1])
+        scale = np.abs(ref).max()
+        assert np.abs(got[1] - ref).max() / scale < tol
+        if dtype == "fp32":
+            assert np.abs(got[1] - got[0]).max() / scale < 1e-5
+    eng.close()

@@ -44,6 +44,8 @@ struct StackGemmArgs {
   // stack_line.h: the activations, or the outputs, as lines of two 16-bit terms [row][K / 32][hi 32 | lo 32] in the place of A, or of C (nullptr: fp32)
   const unsigned short* At; unsigned short* Ct;
   int a_count;                 // gathered products (a_rows): rows of A
+  // one- and two-row products (NORM): A's rows are normed on the way, A / sqrt(mean(A^2) + norm_eps) * (norm_offset + norm_w)
+  const float* norm_w; float norm_offset, norm_eps;
   // stack_rows.h: the choices of a step's pairs (an expert each; those from `experts` on have no product); pair p reads row p / pairs_per_row of A and writes row p of C
   const int* sel; int n_pairs, experts, pairs_per_row, tokens;
 };
@@ -295,7 +297,7 @@ __device__ __forceinline__ void stack_gemv_body(const StackGemmArgs& a, int bx, 
   constexpr int NC = STACK_GEMV_COLS, NB = DUAL ? 2 : 1;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int mbase = by * MR, mend = min(a.M, mbase + MR);
-  const int n0 = (KSPLIT ? bx : bx * 4 + wv) * NC;
+  const int n0 = (KSPLIT ? bx : bx * (int)(blockDim.x >> 6) + wv) * NC;
   if (n0 >= a.N) return;
   const float* Ab = a.A + (size_t)z * a.a_zoff;
   const float* arow[MR];
@@ -372,6 +374,94 @@ __device__ __forceinline__ void stack_gemv_body(const StackGemmArgs& a, int bx, 
   const int m = mbase + lane / NC, n = n0 + lane % NC;
   if (lane < MR * NC && m < mend && n < a.N) sg_finish<EPI>(a, z, m, n, v, v2);
 }
+// ---- the same where the rows are a stream in front of its RMS norm: rows / sqrt(mean(row^2) + norm_eps) * (norm_offset + norm_w).  A workgroup's first weights are on their way before
+// its threads read the rows, times the norm's weights, into LDS and sum their squares; the norm's factor multiplies the products at the end.  One launch less (2.3 to 3.6 us), and a row
+// is read once a workgroup instead of once a wave: the output product of 32000 x 1024 14.7 + 2.3 -> 12.8 us (5.1 TB/s), of 32000 x 2048 24.2 + 3.6 -> 22.5 (5.8).  Up to GEMV_NORM_MAX
+// channels.
+constexpr int GEMV_NORM_MAX = 4096;
+template <int DT, int EPI, bool DUAL, int MR, int NW>
+__device__ __forceinline__ void stack_gemv_norm_body(const StackGemmArgs& a, int bx) {
+  constexpr int NC = STACK_GEMV_COLS, NB = DUAL ? 2 : 1;
+  extern __shared__ __attribute__((aligned(16))) float s_row[];      // [MR][K]
+  __shared__ float s_ss[MR][NW];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, n0 = (bx * NW + wv) * NC, nsl = a.K >> 3;
+  const elem_t<DT>* wrow[NB][NC];
+#pragma unroll
+  for (int b = 0; b < NB; b++)
+#pragma unroll
+    for (int j = 0; j < NC; j++) wrow[b][j] = reinterpret_cast<const elem_t<DT>*>(b ? a.B2 : a.B) + (size_t)min(n0 + j, a.N - 1) * a.ldb;
+  Slice8<DT> w0[NB][NC], w1[NB][NC];
+  auto load = [&](int s0) {      // two slices per lane (past the end: the last again, dropped)
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int j = 0; j < NC; j++) { w0[b][j] = load_slice_nt<DT>(wrow[b][j], (size_t)min(s0, nsl - 1)); w1[b][j] = load_slice_nt<DT>(wrow[b][j], (size_t)min(s0 + 64, nsl - 1)); }
+  };
+  load(lane);
+#pragma unroll
+  for (int r = 0; r < MR; r++) {
+    const int mc = min(r, a.M - 1);
+    const float* row = a.A + (size_t)(a.a_rows ? a.a_rows[mc] : mc) * a.lda;
+    float ss = 0.f;
+    for (int c = 4 * threadIdx.x; c < a.K; c += 256 * NW) {
+      f32x4 x = *reinterpret_cast<const f32x4*>(row + c);
+      const f32x4 g = *reinterpret_cast<const f32x4*>(a.norm_w + c);
+#pragma unroll
+      for (int i = 0; i < 4; i++) { ss = fmaf(x[i], x[i], ss); x[i] *= a.norm_offset + g[i]; }
+      *reinterpret_cast<f32x4*>(s_row + (size_t)r * a.K + c) = x;
+    }
+    ss = group_sum<64>(ss);
+    if (lane == 0) s_ss[r][wv] = ss;
+  }
+  __syncthreads();
+  if (n0 >= a.N) return;
+  float acc[NB][NC][MR];
+#pragma unroll
+  for (int b = 0; b < NB; b++)
+#pragma unroll
+    for (int j = 0; j < NC; j++)
+#pragma unroll
+      for (int r = 0; r < MR; r++) acc[b][j][r] = 0.f;
+  for (int s0 = lane; s0 - lane < nsl; s0 += 128) {
+    if (s0 >= 128) load(s0);
+    const int s1 = s0 + 64;
+#pragma unroll
+    for (int r = 0; r < MR; r++) {
+      const f32x4* xp = reinterpret_cast<const f32x4*>(s_row + (size_t)r * a.K);
+      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+      const int c0 = min(s0, nsl - 1), c1 = min(s1, nsl - 1);
+      f32x4 xa = xp[2 * c0], xb = xp[2 * c0 + 1], ya = xp[2 * c1], yb = xp[2 * c1 + 1];
+      if (s0 >= nsl) xa = xb = zero;
+      if (s1 >= nsl) ya = yb = zero;
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int j = 0; j < NC; j++) { acc[b][j][r] = dot8<DT>(acc[b][j][r], w0[b][j], xa, xb); acc[b][j][r] = dot8<DT>(acc[b][j][r], w1[b][j], ya, yb); }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < MR; r++) {
+    float ss = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) ss += s_ss[r][w];
+    const float f = 1.0f / sqrtf(ss / (float)a.K + a.norm_eps);
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int j = 0; j < NC; j++) acc[b][j][r] = wave_sum(acc[b][j][r]) * f;
+  }
+  float v = acc[0][0][0], v2 = acc[NB - 1][0][0];
+#pragma unroll
+  for (int r = 0; r < MR; r++)
+#pragma unroll
+    for (int j = 0; j < NC; j++)
+      if (lane == r * NC + j) { v = acc[0][j][r]; v2 = acc[NB - 1][j][r]; }
+  const int m = lane / NC, n = n0 + lane % NC;
+  if (lane < MR * NC && m < a.M && n < a.N) sg_finish<EPI>(a, 0, m, n, v, v2);
+}
+// a plain product on rows in front of their norm (a model's last)
+template <int DT, int MR>
+__global__ __launch_bounds__(256) void stack_gemv_norm_kernel(const StackGemmArgs a) { stack_gemv_norm_body<DT, SG_STORE, false, MR, 4>(a, blockIdx.x); }
 template <int DT, int EPI, bool DUAL, int MR, bool KSPLIT>
 __global__ __launch_bounds__(256) void stack_gemv_kernel(const StackGemmArgs a) { stack_gemv_body<DT, EPI, DUAL, MR, KSPLIT>(a, blockIdx.x, blockIdx.y, blockIdx.z); }
 
@@ -382,13 +472,22 @@ __global__ __launch_bounds__(256) void stack_gemv_kernel(const StackGemmArgs a) 
 // Grid: the workgroups of the group's products one after the other; (N / 2) for the sum.  Eight layers of 1024 channels, one stream: 89 launches a step become 62, a step
 // 360 -> 283 us.
 struct StackGemvGroup { StackGemmArgs p0, p1, up; int z0, blocks0, blocks1; };      // blocks0: per member of the batch
-template <int DT, int MR>
-__global__ __launch_bounds__(256) void stack_gemv_group_kernel(const StackGemvGroup g) {
+// NORM: the rows are the stream in front of the layer's norm: 1 for the feed-forward, 2 for the mixer's first product as well.  NW: waves of a workgroup; with the norm eight up to
+// GEMV_GROUP_WIDE channels, whose weights are all on their way before the rows have been read (1024 channels, 24 MB: 6.9 us, four waves 7.7, without the norm 6.9 + 2.3), four beyond (2048
+// channels, 92 MB: 22.2, eight waves 23.9, without 20.0 + 3.6).
+constexpr int GEMV_GROUP_WIDE = 1024;
+template <int DT, int MR, int NORM, int NW>
+__global__ __launch_bounds__(64 * NW) void stack_gemv_group_kernel(const StackGemvGroup g) {
   int b = blockIdx.x;
-  if (b < g.blocks0 * g.z0) { stack_gemv_body<DT, SG_STORE, false, MR>(g.p0, b % g.blocks0, 0, b / g.blocks0); return; }
+  if (b < g.blocks0 * g.z0) {
+    if constexpr (NORM == 2) stack_gemv_norm_body<DT, SG_STORE, false, MR, NW>(g.p0, b);
+    else stack_gemv_body<DT, SG_STORE, false, MR>(g.p0, b % g.blocks0, 0, b / g.blocks0);
+    return;
+  }
   b -= g.blocks0 * g.z0;
   if (b < g.blocks1) { stack_gemv_body<DT, SG_STORE, false, MR>(g.p1, b, 0, 0); return; }
-  stack_gemv_body<DT, SG_SILU_MUL, true, MR>(g.up, b - g.blocks1, 0, 0);
+  if constexpr (NORM != 0) stack_gemv_norm_body<DT, SG_SILU_MUL, true, MR, NW>(g.up, b - g.blocks1);
+  else stack_gemv_body<DT, SG_SILU_MUL, true, MR>(g.up, b - g.blocks1, 0, 0);
 }
 // The four waves of a workgroup divide the slices of all sources of two columns between them, two in flight per lane and pass: W = 1024 would otherwise leave half of the
 // compute units without a wave and give the others five round trips.

@@ -864,10 +864,12 @@ tgx::StackGemmArgs to_stream(const tgx_ctx* c, const float* A, int K, const ebyt
 // product where it stands.
 struct JointLayer {
   bool merged = false;
+  bool norm = false;             // merged, and the norm in front rides in its products (and in the token shift) instead of a launch of its own
   tgx::StackGemmArgs up{};       // the feed-forward's first product (merged layers)
   tgx::StackGemvSum sum{};
   int n_sum = 0;
-  int blocks(int N) const { return (N + 4 * tgx::STACK_GEMV_COLS - 1) / (4 * tgx::STACK_GEMV_COLS); }
+  int waves() const { return norm && up.K <= tgx::GEMV_GROUP_WIDE ? 8 : 4; }
+  int blocks(int N) const { const int cols = waves() * tgx::STACK_GEMV_COLS; return (N + cols - 1) / cols; }
   // the mixer's first product (batched by nz) and, where it has one, a second that does not need it
   void first(tgx_ctx* c, const tgx::StackGemmArgs& p0, int nz, const tgx::StackGemmArgs* p1 = nullptr) {
     if (!merged) { launch_gemm(c, p0, tgx::SG_STORE, nz); if (p1) launch_gemm(c, *p1, tgx::SG_STORE, 1); return; }
@@ -876,9 +878,16 @@ struct JointLayer {
     if (p1) { g.p1 = *p1; g.blocks1 = blocks(p1->N); }
     g.p0.terms = g.p1.terms = g.up.terms = c->act16 ? 1 : 2;
     const dim3 grid(g.blocks0 * nz + g.blocks1 + blocks(up.N));
+    const size_t lds = norm ? (size_t)p0.M * up.K * 4 : 0;
     TGX_DT_SWITCH(c->dt,
-      if (p0.M == 1) hipLaunchKernelGGL((tgx::stack_gemv_group_kernel<DT, 1>), grid, dim3(256), 0, c->stream, g);
-      else hipLaunchKernelGGL((tgx::stack_gemv_group_kernel<DT, 2>), grid, dim3(256), 0, c->stream, g);)
+      auto go = [&](auto N, auto NW) {
+        constexpr int norms = decltype(N)::value, nw = decltype(NW)::value;
+        if (p0.M == 1) hipLaunchKernelGGL((tgx::stack_gemv_group_kernel<DT, 1, norms, nw>), grid, dim3(64 * nw), lds, c->stream, g);
+        else hipLaunchKernelGGL((tgx::stack_gemv_group_kernel<DT, 2, norms, nw>), grid, dim3(64 * nw), lds, c->stream, g);
+      };
+      auto normed = [&](auto NW) { if (p0.norm_w) go(std::integral_constant<int, 2>{}, NW); else go(std::integral_constant<int, 1>{}, NW); };
+      const std::integral_constant<int, 4> four{};
+      if (!norm) go(std::integral_constant<int, 0>{}, four); else if (waves() == 8) normed(std::integral_constant<int, 8>{}); else normed(four);)
   }
   // x += A . Wm^T * scale
   void add(tgx_ctx* c, const tgx::StackGemmArgs& p) { if (merged) sum.p[n_sum++] = p; else launch_gemm(c, p, tgx::SG_ADD, 1); }
@@ -1008,6 +1017,11 @@ bool launch_rec_step(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecStepArgs&
   return true;
 }
 
+// a product on a layer's normed rows, on the stream that they are made of
+tgx::StackGemmArgs before_norm(const StackModel* sm, const StackLayerW& w, tgx::StackGemmArgs g) {
+  g.A = sm->x; g.At = nullptr; g.norm_w = w.norm1; g.norm_offset = 1.0f; g.norm_eps = sm->d.norm_eps;
+  return g;
+}
 int run_joint_attention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer& jl, int T, int S, int max_keys, int max_count) {
   StackModel* sm = c->stack;
   const tgx_layer_desc& ld = w.d;
@@ -1015,7 +1029,7 @@ int run_joint_attention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, Join
   const int W = sm->d.width, H = ld.heads, G = ld.kv_heads, qd = H * ld.dim, vd = H * ld.vdim, nin = qd + (shared ? 0 : G * (ld.dim + ld.vdim));
   tgx::StackGemmArgs g{};
   g.A = sm->a; g.At = sm->in_terms; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = nin; g.M = T; g.N = nin; g.K = W; g.scale = 1.f;
-  jl.first(c, g, 1);
+  jl.first(c, jl.norm ? before_norm(sm, w, g) : g, 1);
   GqaSpec sp{};
   sp.proj = sm->proj; sp.ldp = nin; sp.heads = H; sp.kv_heads = G; sp.dim = ld.dim; sp.vdim = ld.vdim; sp.rot_dims = ld.rot_dims; sp.rot_pairs = ld.rot_pairs;
   sp.cs = w.rot >= 0 ? sm->rot[(size_t)w.rot].cs : nullptr; sp.poolK = w.pool; sp.poolV = w.poolV; sp.poolVT = w.poolVT; sp.append = !shared;
@@ -1033,7 +1047,10 @@ void run_wkv(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer& jl,
   const int W = sm->d.width, H = ld.heads, HD = H * ld.dim, R = ld.decay_rank;
   tgx::TokenShiftArgs ts{};
   ts.h = sm->a; ts.mu = w.mu; ts.out = sm->mixed; ts.state = w.shift; ts.state_buf = (size_t)sm->d.max_seqs * W; ts.W = W; ts.n = 5;
-  hipLaunchKernelGGL(tgx::token_shift_kernel, dim3(T, (W + 255) / 256), dim3(256), 0, c->stream, m, ts);
+  if (jl.norm) {
+    ts.h = sm->x; ts.w = w.norm1; ts.offset = 1.0f; ts.eps = sm->d.norm_eps;
+    hipLaunchKernelGGL(tgx::token_shift_kernel<true>, dim3(T, (W + 255) / 256), dim3(256), 0, c->stream, m, ts);
+  } else hipLaunchKernelGGL(tgx::token_shift_kernel<false>, dim3(T, (W + 255) / 256), dim3(256), 0, c->stream, m, ts);
   // proj row = [r | k | v | g | w]: the first four as one product batched over their mixes, the decay through its low-rank pair
   tgx::StackGemmArgs g{};
   g.A = sm->mixed; g.lda = 5LL * W; g.a_zoff = W; g.B = w.w_in; g.ldb = W; g.b_zstride = (long long)HD * W; g.C = sm->proj; g.ldc = 5LL * HD; g.c_zoff = HD;
@@ -1068,7 +1085,7 @@ int run_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer&
   // [left q | k | v | right q | k | v | b | a | g] = h . w_in^T: both halves read the same input
   tgx::StackGemmArgs g{};
   g.A = sm->a; g.At = sm->in_terms; g.lda = W; g.B = w.w_in; g.ldb = W; g.C = sm->proj; g.ldc = nin; g.M = T; g.N = nin; g.K = W; g.scale = 1.f;
-  jl.first(c, g, 1);
+  jl.first(c, jl.norm ? before_norm(sm, w, g) : g, 1);
   GqaSpec sp{};
   sp.proj = sm->proj; sp.ldp = nin; sp.heads = H; sp.kv_heads = G; sp.dim = ld.dim; sp.vdim = ld.vdim; sp.rot_dims = ld.rot_dims; sp.rot_pairs = ld.rot_pairs;
   sp.cs = w.rot >= 0 ? sm->rot[(size_t)w.rot].cs : nullptr; sp.poolK = w.pool; sp.poolV = w.poolV; sp.poolVT = w.poolVT; sp.append = true;
@@ -1123,18 +1140,23 @@ int run_layers_joint(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys,
     StackLayerW& w = sm->L[(size_t)li];
     const tgx_layer_desc& ld = w.d;
     sm->in_terms = nullptr;
-    const tgx::RowTerms terms = ld.mlp == TGX_MLP_DENSE ? norm_terms(c, T, ld.ff, true) : tgx::RowTerms{};      // (the feed-forward's first product, the mixer's where it reads these rows)
-    hipLaunchKernelGGL(tgx::offset_norm_kernel, dim3(T), dim3(256), 0, c->stream, sm->x, nullptr, w.norm1, 1.0f, sm->a, W, sm->d.norm_eps, terms);
     int rc = TGX_OK;
     JointLayer jl;
     tgx::StackGemmArgs g{};
-    if (ld.mlp == TGX_MLP_DENSE) {      // x += mult * down(silu(gate h) * (up h))
-      g.A = sm->a; g.At = sm->in_terms; g.lda = W; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.C = sm->yh; g.ldc = ld.ff; g.M = T; g.N = ld.ff; g.K = W;
-      jl.up = g;
+    if (ld.mlp == TGX_MLP_DENSE) {
       // every product that joins a launch must take the weight-streaming kernel by itself (one or two rows, whole slices)
       const int outs[] = {ld.heads * (ld.mixer == TGX_MIXER_WKV ? ld.dim : ld.vdim), ld.mixer == TGX_MIXER_PARALLEL ? ld.d_heads * ld.d_vdim : 0, ld.ff, W, ld.mixer == TGX_MIXER_PARALLEL ? sm->max_hv : 0};
       jl.merged = sm->gemv && T <= GEMV_ROWS_MAX;
       for (int k : outs) jl.merged = jl.merged && k % 8 == 0;
+      jl.norm = jl.merged && !c->act16 && W <= tgx::GEMV_NORM_MAX;      // (rounded activations are rounded behind the norm)
+    }
+    if (!jl.norm) {
+      const tgx::RowTerms terms = ld.mlp == TGX_MLP_DENSE ? norm_terms(c, T, ld.ff, true) : tgx::RowTerms{};      // (the feed-forward's first product, the mixer's where it reads these rows)
+      hipLaunchKernelGGL(tgx::offset_norm_kernel, dim3(T), dim3(256), 0, c->stream, sm->x, nullptr, w.norm1, 1.0f, sm->a, W, sm->d.norm_eps, terms);
+    }
+    if (ld.mlp == TGX_MLP_DENSE) {      // x += mult * down(silu(gate h) * (up h))
+      g.A = sm->a; g.At = sm->in_terms; g.lda = W; g.B = w.w_gate; g.B2 = w.w_up; g.ldb = W; g.C = sm->yh; g.ldc = ld.ff; g.M = T; g.N = ld.ff; g.K = W;
+      jl.up = jl.norm ? before_norm(sm, w, g) : g;
     }
     if (ld.mixer == TGX_MIXER_ATTENTION) rc = run_joint_attention(c, m, w, jl, T, S, max_keys, max_count);
     else if (ld.mixer == TGX_MIXER_WKV) run_wkv(c, m, w, jl, T, S, max_count);
@@ -2446,12 +2468,24 @@ int run_layers(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys, int m
 void run_logits(tgx_ctx* c, const int* want_dev, int nw, float* C, const int* c_rows) {
   StackModel* sm = c->stack;
   const int W = sm->d.width, V = sm->d.vocab;
-  if (sm->affine) hipLaunchKernelGGL(tgx::layer_norm_rows_kernel, dim3(nw), dim3(256), 0, c->stream, sm->x, want_dev, sm->final_norm, sm->final_norm + W, sm->xn, W, sm->d.norm_eps);
-  else if (sm->joint || sm->post || sm->hyper) hipLaunchKernelGGL(tgx::offset_norm_kernel, dim3(nw), dim3(256), 0, c->stream, sm->x, want_dev, sm->final_norm, sm->joint || sm->hyper ? 1.0f : 0.0f, sm->xn, W, sm->d.norm_eps, tgx::RowTerms{});
-  else if (sm->sandwich) hipLaunchKernelGGL(tgx::scalar_norm_kernel, dim3(nw), dim3(256), 0, c->stream, sm->x, want_dev, sm->norm_g + 4 * (size_t)sm->d.layers, sm->xn, W, sm->d.norm_eps);
-  else hipLaunchKernelGGL(tgx::final_norm_rows_kernel, dim3(nw), dim3(256), 0, c->stream, sm->x, want_dev, sm->final_norm, sm->xn, W, sm->d.norm_groups, sm->d.norm_eps);
   tgx::StackGemmArgs g{};
   g.A = sm->xn; g.lda = W; g.B = sm->head ? sm->head : c->embed; g.ldb = W; g.C = C; g.ldc = V; g.c_rows = c_rows; g.M = nw; g.N = V; g.K = W; g.scale = sm->d.logit_scale;
+  const bool rms = sm->joint || sm->post || sm->hyper;      // (rows / rms * (offset + w))
+  const float offset = sm->joint || sm->hyper ? 1.0f : 0.0f;
+  if (rms && sm->gemv && nw <= GEMV_ROWS_MAX && !c->act16 && W <= tgx::GEMV_NORM_MAX && slices_ok(g) && !gemv_ksplit(c, g, 1)) {      // one or two rows: the norm rides in the product
+    g.A = sm->x; g.a_rows = want_dev; g.norm_w = sm->final_norm; g.norm_offset = offset; g.norm_eps = sm->d.norm_eps; g.terms = 2;
+    constexpr int cols = 4 * tgx::STACK_GEMV_COLS;
+    const dim3 grid((V + cols - 1) / cols);
+    const size_t lds = (size_t)nw * W * 4;
+    TGX_DT_SWITCH(c->dt,
+      if (nw == 1) hipLaunchKernelGGL((tgx::stack_gemv_norm_kernel<DT, 1>), grid, dim3(256), lds, c->stream, g);
+      else hipLaunchKernelGGL((tgx::stack_gemv_norm_kernel<DT, 2>), grid, dim3(256), lds, c->stream, g);)
+    return;
+  }
+  if (sm->affine) hipLaunchKernelGGL(tgx::layer_norm_rows_kernel, dim3(nw), dim3(256), 0, c->stream, sm->x, want_dev, sm->final_norm, sm->final_norm + W, sm->xn, W, sm->d.norm_eps);
+  else if (rms) hipLaunchKernelGGL(tgx::offset_norm_kernel, dim3(nw), dim3(256), 0, c->stream, sm->x, want_dev, sm->final_norm, offset, sm->xn, W, sm->d.norm_eps, tgx::RowTerms{});
+  else if (sm->sandwich) hipLaunchKernelGGL(tgx::scalar_norm_kernel, dim3(nw), dim3(256), 0, c->stream, sm->x, want_dev, sm->norm_g + 4 * (size_t)sm->d.layers, sm->xn, W, sm->d.norm_eps);
+  else hipLaunchKernelGGL(tgx::final_norm_rows_kernel, dim3(nw), dim3(256), 0, c->stream, sm->x, want_dev, sm->final_norm, sm->xn, W, sm->d.norm_groups, sm->d.norm_eps);
   launch_gemm(c, g, tgx::SG_STORE, 1);
 }
 
