@@ -586,7 +586,8 @@ struct RouterGroupArgs {
   int E, top, groups, keep;
   float scale;
   int sigmoid_scores, group_top2, normalise;
-  int shared;                // 1: every token has one more choice behind its top: expert E with weight 1 (a shared expert that rides among the routed ones)
+  int shared, shared_at;     // 1: every token has one more choice behind its top, expert shared_at (the outputs from there on count one more) with weight 1 or, with sgw, that gate:
+                             // a shared expert that rides among the routed ones
 };
 template <bool PRODUCT>
 __device__ __forceinline__ void router_group_body(RouterGroupArgs a) {
@@ -644,9 +645,10 @@ __device__ __forceinline__ void router_group_body(RouterGroupArgs a) {
   }
   wave_fence();
   const float inv = a.normalise ? a.scale / (sum + 1e-20f * a.scale) : 1.f;
-  for (int k = lane; k < a.top; k += 64) { a.sel[(size_t)t * stride + k] = s_pick[k]; a.selw[(size_t)t * stride + k] = a.normalise ? s_pw[k] * inv : s_pw[k]; }
-  if (a.shared && lane == 0) { a.sel[(size_t)t * stride + a.top] = a.E; a.selw[(size_t)t * stride + a.top] = 1.f; }
-  if (a.sgw && lane == 0) a.sgw[t] = 1.0f / (1.0f + expf(-z[a.E]));
+  for (int k = lane; k < a.top; k += 64) { a.sel[(size_t)t * stride + k] = s_pick[k] + (a.shared && s_pick[k] >= a.shared_at ? 1 : 0); a.selw[(size_t)t * stride + k] = a.normalise ? s_pw[k] * inv : s_pw[k]; }
+  const float sg = a.sgw ? 1.0f / (1.0f + expf(-z[a.E])) : 1.f;
+  if (a.shared && lane == 0) { a.sel[(size_t)t * stride + a.top] = a.shared_at; a.selw[(size_t)t * stride + a.top] = sg; }
+  if (a.sgw && lane == 0) a.sgw[t] = sg;
 }
 __global__ __launch_bounds__(64) void router_group_kernel(RouterGroupArgs a) { router_group_body<false>(a); }
 // a few tokens' seam with the choice of experts behind it (as norm_conv_route_kernel)

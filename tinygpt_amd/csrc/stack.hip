@@ -406,7 +406,7 @@ int ensure_ws(tgx_ctx* c, int T) {
       (rc = dev_alloc(c, &sm->proj, n * (size_t)sm->max_in)) || (rc = dev_alloc(c, &sm->ql, n * (size_t)sm->max_hr)) || (rc = dev_alloc(c, &sm->lat, n * (size_t)sm->max_hr)) ||
       (rc = dev_alloc(c, &sm->o, n * (size_t)sm->max_hv)) || (rc = dev_alloc(c, &sm->xn, n * W)) || (rc = dev_alloc(c, &sm->lg, n * (size_t)sm->d.vocab))) return rc;
   if (sm->max_top > 0) {
-    const size_t np = std::max<size_t>(n * (size_t)sm->max_top, sm->hyper ? GROUPED_FEW_PAIRS : 0);      // (a shared expert that rides among the choices: at most that many pairs)
+    const size_t np = std::max<size_t>(n * (size_t)sm->max_top, sm->hyper || sm->affine || sm->sandwich ? GROUPED_FEW_PAIRS : 0);      // (a shared expert that rides among the choices: at most that many pairs)
     if ((rc = dev_alloc(c, &sm->zr, n * (size_t)(sm->max_E + 1))) || (rc = dev_alloc(c, &sm->selw, np)) || (rc = dev_alloc(c, &sm->sel, np)) || (rc = dev_alloc(c, &sm->perm, np)) || (rc = dev_alloc(c, &sm->ptok, np)) ||
         (rc = dev_alloc(c, &sm->yh, np * (size_t)sm->max_ff + n * (size_t)sm->max_sff)) || (rc = dev_alloc(c, &sm->yd, np * W)) ||
         (rc = dev_alloc(c, &sm->tile_e, std::max<size_t>(np / 64, GROUPED_FEW_PAIRS / GROUPED_FEW_ROWS) + (size_t)sm->max_E + 1)) ||
@@ -773,26 +773,33 @@ void run_dense_ff(tgx_ctx* c, StackLayerW& w, const float* hin, int T) {
   launch_gemm(c, g, tgx::SG_STORE, 1);
 }
 
+// whether the shared expert's products ride among the routed ones': steps of few pairs, where a product is a stream of weights and every launch counts.  (In long portions
+// the shared expert's product takes the wide tiles by itself.)  A step, us, its own two launches / among them: Zaluvik, two rows RIDE_Z; Modepel, one row RIDE_M
+bool shared_rides(const tgx_ctx* c, const StackLayerW& w, int T) {
+  const int np = T * (w.d.top + 1);
+  return w.shared_slot && np <= GROUPED_FEW_PAIRS && c->stack->gemv && c->stack->d.width % 8 == 0 && w.d.ff % 8 == 0;      // (the forms of few pairs)
+}
 // grouped-choice experts: the chosen pairs' rows land in yd (none for identity outputs), the shared expert's in ysh; the seam kernel sums them
 // products of a choice layer's router: its outputs and the shared expert's gate
 int choice_products(const tgx_layer_desc& ld) { return ld.experts + ld.identity + (ld.shared_ff > 0 ? 1 : 0); }
-tgx::RouterGroupArgs choice_router(const tgx_ctx* c, const StackLayerW& w, const float* hin) {
+tgx::RouterGroupArgs choice_router(const tgx_ctx* c, const StackLayerW& w, const float* hin, int T) {
   const StackModel* sm = c->stack;
   const tgx_layer_desc& ld = w.d;
   tgx::RouterGroupArgs ra{};
   ra.in = router_input(c, hin, w.w_router, choice_products(ld));
   ra.z = sm->zr; ra.ldz = choice_products(ld); ra.corr = w.b_router; ra.sel = sm->sel; ra.selw = sm->selw; ra.sgw = ld.shared_ff > 0 ? sm->sgw : nullptr;
   ra.E = ld.experts + ld.identity; ra.top = ld.top; ra.groups = ld.groups; ra.keep = ld.groups_keep; ra.scale = ld.router_scale;
+  ra.shared = shared_rides(c, w, T) ? 1 : 0; ra.shared_at = ld.experts;      // (between the experts and the identity outputs)
   return ra;
 }
 // routed: the choice stands already (it rode behind the seam)
 void run_choice_experts(tgx_ctx* c, StackLayerW& w, const float* hin, int T, bool routed) {
   StackModel* sm = c->stack;
   const tgx_layer_desc& ld = w.d;
-  const int W = sm->d.width, E = ld.experts + ld.identity, top = ld.top;
+  const int W = sm->d.width, ride = shared_rides(c, w, T) ? 1 : 0, E = ld.experts + ld.identity + ride, top = ld.top + ride;
   tgx::StackGemmArgs g{};
   if (!routed) {
-    tgx::RouterGroupArgs ra = choice_router(c, w, hin);
+    tgx::RouterGroupArgs ra = choice_router(c, w, hin, T);
     (void)route(c, ra.in, hin, w.w_router, choice_products(ld), T);
     hipLaunchKernelGGL(tgx::router_group_kernel, dim3(T), dim3(64), 0, c->stream, ra);
   }
@@ -803,9 +810,9 @@ void run_choice_experts(tgx_ctx* c, StackLayerW& w, const float* hin, int T, boo
     const tgx::StackGemmArgs gu = g;
     g = tgx::StackGemmArgs{};
     g.A = sm->yh; g.lda = ld.ff; g.B = w.w_down; g.ldb = ld.ff; g.b_zstride = (long long)W * ld.ff; g.C = sm->yd; g.ldc = W; g.N = W; g.K = ld.ff; g.rw = sm->selw;
-    launch_experts(c, gu, tgx::SG_SILU_MUL, g, tgx::SG_ROWSCALE, T, top, E, ld.experts);
+    launch_experts(c, gu, tgx::SG_SILU_MUL, g, tgx::SG_ROWSCALE, T, top, E, ld.experts + ride);
   }
-  if (ld.shared_ff > 0) {
+  if (ld.shared_ff > 0 && !ride) {
     float* hsh = sm->yh + (size_t)np * std::max(1, ld.ff);
     g = tgx::StackGemmArgs{};
     g.A = hin; g.lda = W; g.B = w.ws_gate; g.B2 = w.ws_up; g.ldb = W; g.C = hsh; g.ldc = ld.shared_ff; g.M = T; g.N = ld.shared_ff; g.K = W;
@@ -834,7 +841,7 @@ int run_layers_sandwich(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_ke
     tgx::SandwichArgs sa{};
     sa.x = sm->x; sa.y = sm->yd; sa.top = 1; sa.ytmp = sm->ytmp; sa.g_post = ng + 1; sa.g_next = ld.mlp != TGX_MLP_NONE ? ng + 2 : next_layer; sa.out = hout; sa.W = W; sa.eps = eps;
     const bool routed = ld.mlp == TGX_MLP_MOE && route_rides(c, choice_products(ld), T);
-    if (routed) launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::sandwich_route_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa, choice_router(c, w, hout)); });
+    if (routed) launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::sandwich_route_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa, choice_router(c, w, hout, T)); });
     else launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::sandwich_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa); });
     std::swap(hin, hout);
     if (ld.mlp == TGX_MLP_NONE) continue;
@@ -843,7 +850,8 @@ int run_layers_sandwich(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_ke
     if (ld.mlp == TGX_MLP_DENSE) run_dense_ff(c, w, hin, T);
     else {
       run_choice_experts(c, w, hin, T, routed);
-      sa.top = ld.top; sa.sel = sm->sel; sa.selw = sm->selw; sa.n_real = ld.experts; sa.h = hin; sa.ysh = ld.shared_ff > 0 ? sm->ysh : nullptr;
+      const int ride = shared_rides(c, w, T) ? 1 : 0;
+      sa.top = ld.top + ride; sa.sel = sm->sel; sa.selw = sm->selw; sa.n_real = ld.experts + ride; sa.h = hin; sa.ysh = ld.shared_ff > 0 && !ride ? sm->ysh : nullptr;
     }
     launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::sandwich_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa); });
     std::swap(hin, hout);
@@ -1355,13 +1363,14 @@ int run_affine_latent(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, const 
 }
 
 // the feed-forward of a layer-norm design into yd (one row per token, or `top` rows per token for experts) and ysh (the shared expert's row)
-tgx::RouterGroupArgs affine_router(const tgx_ctx* c, const StackLayerW& w) {
+tgx::RouterGroupArgs affine_router(const tgx_ctx* c, const StackLayerW& w, int T) {
   const StackModel* sm = c->stack;
   const tgx_layer_desc& ld = w.d;
   tgx::RouterGroupArgs ra{};
   ra.in = router_input(c, sm->a, w.w_router, ld.experts);
   ra.z = sm->zr; ra.ldz = ld.experts; ra.sel = sm->sel; ra.selw = sm->selw; ra.E = ld.experts; ra.top = ld.top; ra.groups = ld.groups; ra.keep = ld.groups_keep; ra.scale = 1.f;
   ra.sigmoid_scores = ld.router_fn == 1; ra.group_top2 = ld.group_score == 1; ra.normalise = ld.router_norm;
+  ra.shared = shared_rides(c, w, T) ? 1 : 0; ra.shared_at = ld.experts;
   return ra;
 }
 void run_affine_ff(tgx_ctx* c, StackLayerW& w, int T, bool routed) {
@@ -1374,10 +1383,10 @@ void run_affine_ff(tgx_ctx* c, StackLayerW& w, int T, bool routed) {
     launch_ff(c, g, tgx::SG_STORE, sublayer_product(c, sm->yh, ld.ff, w.w_down, T), tgx::SG_STORE);
     return;
   }
-  const int E = ld.experts, top = ld.top, np = T * top;
+  const int ride = shared_rides(c, w, T) ? 1 : 0, E = ld.experts + ride, top = ld.top + ride, np = T * top;
   if (!routed) {
-    tgx::RouterGroupArgs ra = affine_router(c, w);
-    (void)route(c, ra.in, sm->a, w.w_router, E, T);
+    tgx::RouterGroupArgs ra = affine_router(c, w, T);
+    (void)route(c, ra.in, sm->a, w.w_router, ld.experts, T);
     hipLaunchKernelGGL(tgx::router_group_kernel, dim3(T), dim3(64), 0, c->stream, ra);
   }
   g = tgx::StackGemmArgs{};
@@ -1386,7 +1395,7 @@ void run_affine_ff(tgx_ctx* c, StackLayerW& w, int T, bool routed) {
   g = tgx::StackGemmArgs{};
   g.A = sm->yh; g.lda = ld.ff; g.B = w.w_down; g.ldb = ld.ff; g.b_zstride = (long long)W * ld.ff; g.C = sm->yd; g.ldc = W; g.N = W; g.K = ld.ff; g.rw = sm->selw;
   launch_experts(c, gu, tgx::SG_SILU_MUL, g, tgx::SG_ROWSCALE, T, top, E, E);
-  if (ld.shared_ff > 0) {      // the shared expert runs for every token, without a gate of its own
+  if (ld.shared_ff > 0 && !ride) {      // the shared expert runs for every token, without a gate of its own
     float* hsh = sm->yh + (size_t)np * std::max(1, ld.ff);
     g = tgx::StackGemmArgs{};
     g.A = sm->a; g.lda = W; g.B = w.ws_gate; g.B2 = w.ws_up; g.ldb = W; g.C = hsh; g.ldc = ld.shared_ff; g.M = T; g.N = ld.shared_ff; g.K = W;
@@ -1429,13 +1438,14 @@ int run_layers_affine(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
     if (ld.mlp != TGX_MLP_NONE) { sa.w_next = ln + 4 * (size_t)W; sa.b_next = ln + 5 * (size_t)W; }
     else if (next_ln) { sa.w_next = next_ln; sa.b_next = next_ln + W; }
     const bool routed = ld.mlp == TGX_MLP_MOE && route_rides(c, ld.experts, T);
-    if (routed) launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::affine_seam_route_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa, affine_router(c, w)); });
+    if (routed) launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::affine_seam_route_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa, affine_router(c, w, T)); });
     else launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::affine_seam_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa); });
     normed = sa.w_next != nullptr;
     if (ld.mlp == TGX_MLP_NONE) continue;
     run_affine_ff(c, w, T, routed);
+    const int ride = ld.mlp == TGX_MLP_MOE && shared_rides(c, w, T) ? 1 : 0;
     sa = tgx::AffineSeamArgs{};
-    sa.x = sm->x; sa.y = sm->yd; sa.top = ld.mlp == TGX_MLP_MOE ? ld.top : 1; sa.ysh = ld.mlp == TGX_MLP_MOE && ld.shared_ff > 0 ? sm->ysh : nullptr; sa.ytmp = sm->ytmp;
+    sa.x = sm->x; sa.y = sm->yd; sa.top = ld.mlp == TGX_MLP_MOE ? ld.top + ride : 1; sa.ysh = ld.mlp == TGX_MLP_MOE && ld.shared_ff > 0 && !ride ? sm->ysh : nullptr; sa.ytmp = sm->ytmp;
     sa.w_post = ln + 6 * (size_t)W; sa.b_post = ln + 7 * (size_t)W; sa.mult = mult; sa.out = sm->a; sa.W = W; sa.eps = eps;
     if (next_ln) { sa.w_next = next_ln; sa.b_next = next_ln + W; }
     launch_seam(sa.W, [&](auto R) { hipLaunchKernelGGL(tgx::affine_seam_kernel<decltype(R)::value>, dim3(T), dim3(256), 0, c->stream, sa); });
@@ -1508,15 +1518,18 @@ int create_affine_layers(tgx_ctx* c, const tgx_layer_desc* layers) {
       continue;
     }
     const size_t E = (size_t)l.experts, F = (size_t)l.ff, SF = (size_t)l.shared_ff;
-    if ((rc = dev_alloc(c, &w.w_router, E * W)) || (rc = dev_alloc(c, &w.w_gate, E * F * W * es)) || (rc = dev_alloc(c, &w.w_up, E * F * W * es)) || (rc = dev_alloc(c, &w.w_down, E * W * F * es))) return rc;
+    w.shared_slot = SF == F;      // a shared expert of the routed ones' size stands behind them as one more
+    const size_t Es = E + (w.shared_slot ? 1 : 0);
+    if ((rc = dev_alloc(c, &w.w_router, E * W)) || (rc = dev_alloc(c, &w.w_gate, Es * F * W * es)) || (rc = dev_alloc(c, &w.w_up, Es * F * W * es)) || (rc = dev_alloc(c, &w.w_down, Es * W * F * es))) return rc;
     need(p, {"mlp.router"});
     for (int e = 0; e < l.experts; e++)
       for (const char* n : {".gate", ".up", ".down"}) sm->missing.insert(p + "mlp.e" + std::to_string(e) + n);
     if (SF > 0) {
-      if ((rc = dev_alloc(c, &w.ws_gate, SF * W * es)) || (rc = dev_alloc(c, &w.ws_up, SF * W * es)) || (rc = dev_alloc(c, &w.ws_down, W * SF * es))) return rc;
+      if (w.shared_slot) { w.ws_gate = w.w_gate + E * F * W * es; w.ws_up = w.w_up + E * F * W * es; w.ws_down = w.w_down + E * W * F * es; }
+      else if ((rc = dev_alloc(c, &w.ws_gate, SF * W * es)) || (rc = dev_alloc(c, &w.ws_up, SF * W * es)) || (rc = dev_alloc(c, &w.ws_down, W * SF * es))) return rc;
       need(p, {"mlp.shared.gate", "mlp.shared.up", "mlp.shared.down"});
     }
-    sm->max_top = std::max(sm->max_top, l.top); sm->max_ff = std::max(sm->max_ff, l.ff); sm->max_E = std::max(sm->max_E, l.experts); sm->max_sff = std::max(sm->max_sff, l.shared_ff);
+    sm->max_top = std::max(sm->max_top, l.top); sm->max_ff = std::max(sm->max_ff, l.ff); sm->max_E = std::max(sm->max_E, (int)Es); sm->max_sff = std::max(sm->max_sff, l.shared_ff);
   }
   return TGX_OK;
 }
@@ -2049,18 +2062,12 @@ void run_channel_delta(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T
   sublayer_out(c, sm->o, k.HE, w.w_o, T);
 }
 
-// whether the shared expert's products ride among the routed ones': steps of few pairs, where a product is a stream of weights and every launch counts.  (In long portions
-// the shared expert's product takes the wide tiles by itself.)
-bool shared_rides(const tgx_ctx* c, const StackLayerW& w, int T) {
-  const int np = T * (w.d.top + 1);
-  return w.shared_slot && np <= GROUPED_FEW_PAIRS && c->stack->gemv && c->stack->d.width % 8 == 0 && w.d.ff % 8 == 0;      // (the forms of few pairs)
-}
 tgx::RouterGroupArgs hyper_router(const tgx_ctx* c, const StackLayerW& w, int T) {
   const StackModel* sm = c->stack;
   const tgx_layer_desc& ld = w.d;
   tgx::RouterGroupArgs ra{};
   ra.in = router_input(c, sm->a, w.w_router, ld.experts);
-  ra.z = sm->zr; ra.ldz = ld.experts; ra.sel = sm->sel; ra.selw = sm->selw; ra.E = ld.experts; ra.top = ld.top; ra.shared = shared_rides(c, w, T) ? 1 : 0; ra.groups = 1; ra.keep = 1; ra.scale = 1.f;
+  ra.z = sm->zr; ra.ldz = ld.experts; ra.sel = sm->sel; ra.selw = sm->selw; ra.E = ld.experts; ra.top = ld.top; ra.shared = shared_rides(c, w, T) ? 1 : 0; ra.shared_at = ld.experts; ra.groups = 1; ra.keep = 1; ra.scale = 1.f;
   ra.sigmoid_scores = ld.router_fn == 1; ra.normalise = ld.router_norm;
   return ra;
 }
@@ -2593,16 +2600,19 @@ int create_sandwich_layers(tgx_ctx* c, const tgx_layer_desc* layers) {
     const size_t E = (size_t)l.experts, Et = E + (size_t)l.identity, F = (size_t)l.ff, SF = (size_t)l.shared_ff;
     if ((rc = dev_alloc(c, &w.w_router, (Et + 1) * W)) || (rc = dev_alloc(c, &w.b_router, Et))) return rc;
     for (const char* n : {"mlp.router", "mlp.correction"}) sm->missing.insert(p + n);
+    w.shared_slot = E > 0 && SF == F;      // a shared expert of the routed ones' size stands behind them as one more
+    const size_t Es = E + (w.shared_slot ? 1 : 0);
     if (E > 0) {
-      if ((rc = dev_alloc(c, &w.w_gate, E * F * W * es)) || (rc = dev_alloc(c, &w.w_up, E * F * W * es)) || (rc = dev_alloc(c, &w.w_down, E * W * F * es))) return rc;
+      if ((rc = dev_alloc(c, &w.w_gate, Es * F * W * es)) || (rc = dev_alloc(c, &w.w_up, Es * F * W * es)) || (rc = dev_alloc(c, &w.w_down, Es * W * F * es))) return rc;
       for (int e = 0; e < l.experts; e++)
         for (const char* n : {".gate", ".up", ".down"}) sm->missing.insert(p + "mlp.e" + std::to_string(e) + n);
     }
     if (SF > 0) {
-      if ((rc = dev_alloc(c, &w.ws_gate, SF * W * es)) || (rc = dev_alloc(c, &w.ws_up, SF * W * es)) || (rc = dev_alloc(c, &w.ws_down, W * SF * es))) return rc;
+      if (w.shared_slot) { w.ws_gate = w.w_gate + E * F * W * es; w.ws_up = w.w_up + E * F * W * es; w.ws_down = w.w_down + E * W * F * es; }
+      else if ((rc = dev_alloc(c, &w.ws_gate, SF * W * es)) || (rc = dev_alloc(c, &w.ws_up, SF * W * es)) || (rc = dev_alloc(c, &w.ws_down, W * SF * es))) return rc;
       for (const char* n : {"mlp.shared.gate", "mlp.shared.up", "mlp.shared.down", "mlp.shared.sg"}) sm->missing.insert(p + n);
     }
-    sm->max_top = std::max(sm->max_top, l.top); sm->max_ff = std::max(sm->max_ff, l.ff); sm->max_E = std::max(sm->max_E, (int)Et); sm->max_sff = std::max(sm->max_sff, l.shared_ff);
+    sm->max_top = std::max(sm->max_top, l.top); sm->max_ff = std::max(sm->max_ff, l.ff); sm->max_E = std::max(sm->max_E, (int)(Et + Es - E)); sm->max_sff = std::max(sm->max_sff, l.shared_ff);
   }
   return TGX_OK;
 }
@@ -3265,7 +3275,7 @@ void stack_destroy(tgx_ctx* c) {
       own.pool = w.pool; own.poolV = w.poolV; own.poolVT = w.poolVT; own.mS = w.mS; own.conv_state = w.conv_state;
       w = own;
     }
-    if (w.shared_slot) w.ws_up = w.ws_down = nullptr;      // (inside w_up / w_down)
+    if (w.shared_slot) w.ws_gate = w.ws_up = w.ws_down = nullptr;      // (inside w_gate / w_up / w_down)
     fr(w.hc); fr(w.decays); fr(w.w_b); fr(w.w_g1); fr(w.w_g2);
     fr(w.conv_b); fr(w.d_skip); fr(w.decay2); fr(w.q_norm); fr(w.k_norm); fr(w.dist);
     fr(w.w_o2); fr(w.w_w1); fr(w.w_w2); fr(w.mu); fr(w.w0); fr(w.ubonus); fr(w.conv_w); fr(w.a_log); fr(w.dt_bias); fr(w.shift);
