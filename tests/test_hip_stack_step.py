@@ -197,3 +197,62 @@ def test_norms_inside_the_products_of_one_and_two_rows(width, rows, dtype):
         if dtype == "fp32":
             assert np.abs(got[1] - got[0]).max() / scale < 1e-5
     eng.close()
+
+
+@pytest.mark.parametrize("rank,vdim,heads", [(64, 8, 3), (128, 33, 2), (320, 70, 2), (512, 16, 1), (72, 8, 2)])      # (72: merge and product apart)
+@pytest.mark.parametrize("keys,dtype", [(700, "fp32"), (1130, "bf16")])      # two or three records a token; eighteen
+def test_values_from_the_records_of_divided_keys(rank, vdim, heads, keys, dtype):
+    """a latent attention's merge and value product in one launch: one and three tokens over divided keys, against the oracle, and in fp32 against the two launches (act.round16, which
+    rounds nothing there, keeps them)"""
+    import stack_oracle as so
+    from tinygpt_amd.desc import LayerDesc, StackDesc
+    from tinygpt_amd.serving import SlotEngine
+    layers = [LayerDesc(heads=heads, dim=16, vdim=vdim, kv_rank=rank, scale=0.35, mlp=None) for _ in range(2)]
+    d = StackDesc(width=32, vocab=53, canon_taps=4, norm_groups=2, norm_eps=1e-6, max_seqs=3, max_ctx=1280, budget_tokens=3840, compute_dtype=dtype, layers=layers)
+    t = so.random_tensors(d, rank)
+    seqs = [np.random.default_rng(rank + i).integers(0, 53, keys - 9 * i) for i in range(3)]
+    eng = SlotEngine(desc=d, tensors={k: v.astype(np.float32) for k, v in t.items()})
+    eng.model.set_option("attn.split_min", 64)
+    got = {}
+    for apart in (0, 1):
+        eng.model.set_option("act.round16", apart if dtype == "fp32" else 0)
+        eng.step([(i, s[:-4], []) for i, s in enumerate(seqs)])
+        rows = [eng.step([(0, seqs[0][-4:-3], [0])])]
+        rows += [eng.step([(i, s[len(s) - 4 + j + (i == 0):len(s) - 3 + j + (i == 0)], [0]) for i, s in enumerate(seqs)]) for j in range(3)]
+        got[apart] = np.concatenate(rows)
+        for i in range(3):
+            eng.release(i)
+    eng.close()
+    want = [so.forward(d, t, s.tolist()) for s in seqs]
+    ref = np.concatenate([want[0][-4:-3]] + [np.stack([want[i][len(seqs[i]) - 4 + j + (i == 0)] for i in range(3)]) for j in range(3)])
+    scale = np.abs(ref).max()
+    assert np.abs(got[0] - ref).max() / scale < (1e-4 if dtype == "fp32" else 3e-2)
+    if dtype == "fp32":
+        assert np.abs(got[0] - got[1]).max() / scale < 1e-5
+
+
+@pytest.mark.parametrize("design", ["zaluvik", "modepel", "modepel_plain"])
+@pytest.mark.parametrize("tokens", [1, 2, 3, 16, 21, 40, 43, 90])      # pairs with the shared choice: up to 128 ride, of one to many rows an expert, more do not
+def test_shared_experts_among_the_routed_ones(design, tokens):
+    """a shared expert of the routed ones' size as one more choice (Modepel: between the experts and the identity outputs, weighted by its gate) against the oracle, and against its own
+    launches (a width of the experts that keeps the forms of few pairs away has none to compare: stack.gemv 0)"""
+    import test_hip_modepel as tm
+    import test_hip_zaluvik as tz
+    if design == "zaluvik":
+        t, cfg = tz, tz.config([tz.attn(tz.moe(ff=16, shared=16)), tz.lat(tz.moe(ff=16, shared=16, groups=None))], loop=None)
+    else:
+        identity = 2 if design == "modepel" else 0
+        t, cfg = tm, tm.config([tm.attn(tm.moe(ff=16, shared=16, identity=identity)), tm.rec(tm.moe(ff=16, shared=16, identity=identity, experts=8 - identity, top=3, keep=2))])
+    eng, w = t.engine(cfg, "fp32", 11)
+    toks = t.tokens(cfg, tokens, tokens)
+    got = {}
+    for on in (1, 0):
+        eng.model.set_option("stack.gemv", on)
+        got[on] = t.run_whole(eng, "r%d" % on, toks)
+    eng.close()
+    scale = np.abs(got[0]).max()
+    rows = np.abs(got[1] - got[0]).max(1) / scale
+    assert np.sort(rows)[-1 - tokens // 30] < 1e-4      # (a near tie of a router may send a token elsewhere)
+    want = t.want_of(cfg, w, toks)
+    rows = np.abs(got[1] - want).max(1) / np.abs(want).max()
+    assert np.sort(rows)[-1 - tokens // 30] < 1e-4

@@ -22,6 +22,7 @@
 #include "kernels/stack_mix_mfma.h"
 #include "kernels/stack_ssm.h"
 #include "kernels/stack_conv.h"
+#include "kernels/stack_latent.h"
 #include "kernels/stack_ssd_mfma.h"
 #include "kernels/stack_hyper.h"
 
@@ -420,6 +421,17 @@ int ensure_ws(tgx_ctx* c, int T) {
   return TGX_OK;
 }
 
+// the values of a latent attention from the records of its divided keys: merge and product in one launch in steps of few tokens (kernels/stack_latent.h), else the merge alone (false: the
+// product is still to come)
+bool latent_values(tgx_ctx* c, const tgx::LatentAttnArgs& aa, tgx::StackGemmArgs g, int T, int H) {
+  if (c->stack->gemv && !c->act16 && T <= 16 && g.K % 64 == 0 && g.K <= tgx::LATV_MAX_RANK && slices_ok(g)) {
+    const dim3 grid((g.N + tgx::LATV_COLS - 1) / tgx::LATV_COLS, H, T);
+    TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::latent_values_kernel<DT>, grid, dim3(256), 0, c->stream, aa, g))
+    return true;
+  }
+  hipLaunchKernelGGL(tgx::latent_attn_merge_kernel, dim3(T, H), dim3(256), 0, c->stream, aa);
+  return false;
+}
 // a filter's size by number where the kernels have it (kernels/stack.h)
 template <class F>
 void with_taps(int taps, F go) {
@@ -474,6 +486,11 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
       TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::latent_append_kernel<DT>, dim3(T), dim3(64), 0, c->stream, m, la))
       launch_gemm(c, g, tgx::SG_STORE, H);
     }
+    // o[t][h] = (lat[t][h] . uv[h]^T) * sigmoid(gate)
+    g = tgx::StackGemmArgs{};
+    g.A = sm->lat; g.lda = (long long)H * R; g.a_zoff = R; g.B = w.w_uv; g.ldb = R; g.b_zstride = (long long)ld.vdim * R; g.C = sm->o; g.ldc = vd; g.c_zoff = ld.vdim;
+    g.M = T; g.N = ld.vdim; g.K = R; g.G = sm->proj; g.ldg = nin; g.g_col0 = qd + R;
+    bool valued = false;
     tgx::LatentAttnArgs aa{};
     aa.q = sm->ql; aa.ldq = (long long)H * R; aa.pool = w.pool; aa.sink = w.sink; aa.out = sm->lat; aa.ldo = (long long)H * R; aa.rank = R; aa.heads = H;
     if (w.poolT && sm->attn_mfma) {
@@ -492,7 +509,7 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
         ma.part = sm->part; ma.nsplit = nsplit;
         aa.part = sm->part; aa.nsplit = nsplit;
         if (c->dt == tgx::DT_F16) launch_attn_mfma_t<tgx::DT_F16, true>(c, m, ma, dim3(tiles, S, nsplit)); else launch_attn_mfma_t<tgx::DT_BF16, true>(c, m, ma, dim3(tiles, S, nsplit));
-        hipLaunchKernelGGL(tgx::latent_attn_merge_kernel, dim3(T, H), dim3(256), 0, c->stream, aa);
+        valued = latent_values(c, aa, g, T, H);
       } else {
         if (c->dt == tgx::DT_F16) launch_attn_mfma_t<tgx::DT_F16, false>(c, m, ma, dim3(tiles, S)); else launch_attn_mfma_t<tgx::DT_BF16, false>(c, m, ma, dim3(tiles, S));
       }
@@ -507,16 +524,12 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
     if (nsplit > 1 && ensure_part(c, (size_t)T * H * nsplit * (size_t)(R + 2))) {
       aa.part = sm->part; aa.nsplit = nsplit;
       TGX_DT_SWITCH(c->dt, (launch_attn_t<DT, true>(c, m, aa, dim3(T, H, nsplit))))
-      hipLaunchKernelGGL(tgx::latent_attn_merge_kernel, dim3(T, H), dim3(256), 0, c->stream, aa);
+      valued = latent_values(c, aa, g, T, H);
     } else {
       TGX_DT_SWITCH(c->dt, (launch_attn_t<DT, false>(c, m, aa, dim3(T, H))))
     }
     }
-    // o[t][h] = (lat[t][h] . uv[h]^T) * sigmoid(gate)
-    g = tgx::StackGemmArgs{};
-    g.A = sm->lat; g.lda = (long long)H * R; g.a_zoff = R; g.B = w.w_uv; g.ldb = R; g.b_zstride = (long long)ld.vdim * R; g.C = sm->o; g.ldc = vd; g.c_zoff = ld.vdim;
-    g.M = T; g.N = ld.vdim; g.K = R; g.G = sm->proj; g.ldg = nin; g.g_col0 = qd + R;
-    launch_gemm(c, g, tgx::SG_GATE, H);
+    if (!valued) launch_gemm(c, g, tgx::SG_GATE, H);
     // x += o . w_o^T
     g = tgx::StackGemmArgs{};
     g.A = sm->o; g.lda = vd; g.B = w.w_o; g.ldb = vd; g.C = sm->x; g.ldc = W; g.M = T; g.N = W; g.K = vd; g.scale = 1.f;
@@ -774,7 +787,8 @@ void run_dense_ff(tgx_ctx* c, StackLayerW& w, const float* hin, int T) {
 }
 
 // whether the shared expert's products ride among the routed ones': steps of few pairs, where a product is a stream of weights and every launch counts.  (In long portions
-// the shared expert's product takes the wide tiles by itself.)  A step, us, its own two launches / among them: Zaluvik, two rows RIDE_Z; Modepel, one row RIDE_M
+// the shared expert's product takes the wide tiles by itself.)  The two launches / what the routed ones take more, us: 1536 x 1024 and two rows 6.3 + 4.6 / 1.1 + 1.0, 2048 x 2048
+// and one row 6.5 + 4.6 / 2.4 + 1.5
 bool shared_rides(const tgx_ctx* c, const StackLayerW& w, int T) {
   const int np = T * (w.d.top + 1);
   return w.shared_slot && np <= GROUPED_FEW_PAIRS && c->stack->gemv && c->stack->d.width % 8 == 0 && w.d.ff % 8 == 0;      // (the forms of few pairs)
@@ -1311,6 +1325,11 @@ int run_affine_latent(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, const 
   g.A = sm->proj; g.lda = nin; g.a_zoff = qs; g.B = w.w_ukT; g.ldb = ld.dim; g.b_zstride = (long long)R * ld.dim; g.C = sm->ql; g.ldc = (long long)H * RR; g.c_zoff = RR;
   g.M = T; g.N = R; g.K = ld.dim; g.scale = ld.scale;
   launch_gemm(c, g, tgx::SG_STORE, H);
+  // o[t][h] = (lat[t][h][0 .. R) . uv[h]^T) * sigmoid(gate of the head, or of the channel)
+  g = tgx::StackGemmArgs{};
+  g.A = sm->lat; g.lda = (long long)H * RR; g.a_zoff = RR; g.B = w.w_uv; g.ldb = R; g.b_zstride = (long long)ld.vdim * R; g.C = sm->o; g.ldc = vd; g.c_zoff = ld.vdim;
+  g.M = T; g.N = ld.vdim; g.K = R; g.G = sm->proj; g.ldg = nin; g.g_col0 = qd + RR; g.g_per_z = ld.gate_kind == 2;
+  bool valued = false;
   tgx::LatentAttnArgs aa{};
   aa.q = sm->ql; aa.ldq = (long long)H * RR; aa.pool = run.pool; aa.sink = nullptr; aa.out = sm->lat; aa.ldo = (long long)H * RR; aa.rank = RR; aa.heads = H;
   aa.mask_kind = ld.mask_kind; aa.mask_size = ld.mask_size;
@@ -1332,7 +1351,7 @@ int run_affine_latent(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, const 
       ma.part = sm->part; ma.nsplit = nsplit;
       aa.part = sm->part; aa.nsplit = nsplit;
       if (c->dt == tgx::DT_F16) launch_attn_mfma_t<tgx::DT_F16, true>(c, m, ma, dim3(tiles, S, nsplit)); else launch_attn_mfma_t<tgx::DT_BF16, true>(c, m, ma, dim3(tiles, S, nsplit));
-      hipLaunchKernelGGL(tgx::latent_attn_merge_kernel, dim3(T, H), dim3(256), 0, c->stream, aa);
+      valued = latent_values(c, aa, g, T, H);
     } else {
       if (c->dt == tgx::DT_F16) launch_attn_mfma_t<tgx::DT_F16, false>(c, m, ma, dim3(tiles, S)); else launch_attn_mfma_t<tgx::DT_BF16, false>(c, m, ma, dim3(tiles, S));
     }
@@ -1346,16 +1365,12 @@ int run_affine_latent(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, const 
   if (nsplit > 1 && ensure_part(c, (size_t)T * H * nsplit * (size_t)(RR + 2))) {
     aa.part = sm->part; aa.nsplit = nsplit;
     TGX_DT_SWITCH(c->dt, (launch_attn_t<DT, true>(c, m, aa, dim3(T, H, nsplit))))
-    hipLaunchKernelGGL(tgx::latent_attn_merge_kernel, dim3(T, H), dim3(256), 0, c->stream, aa);
+    valued = latent_values(c, aa, g, T, H);
   } else {
     TGX_DT_SWITCH(c->dt, (launch_attn_t<DT, false>(c, m, aa, dim3(T, H))))
   }
   }
-  // o[t][h] = (lat[t][h][0 .. R) . uv[h]^T) * sigmoid(gate of the head, or of the channel)
-  g = tgx::StackGemmArgs{};
-  g.A = sm->lat; g.lda = (long long)H * RR; g.a_zoff = RR; g.B = w.w_uv; g.ldb = R; g.b_zstride = (long long)ld.vdim * R; g.C = sm->o; g.ldc = vd; g.c_zoff = ld.vdim;
-  g.M = T; g.N = ld.vdim; g.K = R; g.G = sm->proj; g.ldg = nin; g.g_col0 = qd + RR; g.g_per_z = ld.gate_kind == 2;
-  launch_gemm(c, g, tgx::SG_GATE, H);
+  if (!valued) launch_gemm(c, g, tgx::SG_GATE, H);
   g = tgx::StackGemmArgs{};
   g.A = sm->o; g.lda = vd; g.B = w.w_o; g.ldb = vd; g.C = sm->yd; g.ldc = W; g.M = T; g.N = W; g.K = vd; g.scale = 1.f;
   launch_gemm(c, g, tgx::SG_STORE, 1);
