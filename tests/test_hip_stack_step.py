@@ -256,3 +256,18 @@ def test_shared_experts_among_the_routed_ones(design, tokens):
     want = t.want_of(cfg, w, toks)
     rows = np.abs(got[1] - want).max(1) / np.abs(want).max()
     assert np.sort(rows)[-1 - tokens // 30] < 1e-4
+
+
+@pytest.mark.parametrize("kv_rank,dim,rot_dim", [(16, 8, 8), (1032, 40, 16), (24, 136, 0)])
+@pytest.mark.parametrize("slots", [1, 2, 3, 16, 17])
+def test_rotated_latents_beside_their_queries(slots, kv_rank, dim, rot_dim):
+    """a rotated latent layer's append beside the queries' products into latent space (the vector kernel's up to two rows, the matrix cores' up to 16), token by token against the oracle"""
+    import test_hip_zaluvik as tz
+    cfg = tz.config([tz.lat(tz.dense(), heads=3, dim=dim, rot_dim=rot_dim, vdim=8, kv_rank=kv_rank, mask={"size": 4})], loop=None)
+    eng, w = tz.engine(cfg, "fp32", 2, max_seqs=slots, max_ctx=64, budget_tokens=64 * slots)
+    toks = [tz.tokens(cfg, 6, i) for i in range(slots)]
+    got = np.stack([eng.step([("s%d" % i, [s[j]], [0]) for i, s in enumerate(toks)]) for j in range(6)], 1)
+    eng.close()
+    for i in {0, slots // 2, slots - 1}:
+        want = tz.want_of(cfg, w, toks[i])
+        assert np.abs(got[i] - want).max() / np.abs(want).max() < 1e-4, (slots, i)

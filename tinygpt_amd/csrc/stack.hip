@@ -34,6 +34,12 @@ __global__ __launch_bounds__(64 * few_max_waves(1)) void latent_append_queries_k
   if ((int)blockIdx.z < heads) stack_few_body<DT, SG_STORE, false, 1>(a, depth, blockIdx.z, 0, a.M);
   else for (int t = blockIdx.x; t < m.T; t += gridDim.x) latent_append_body<DT>(m, la, t);
 }
+// ... beside the vector kernel's products (one and two tokens; a rotated key part's queries are turned by the append).  Two tokens, 8 heads of 192 x 128: 5.0 us and 4.7, 5.6 together.
+template <int DT, int MR, bool KSPLIT>
+__global__ __launch_bounds__(256) void latent_append_gemv_kernel(StepMeta m, LatentAppendArgs la, StackGemmArgs a, const int heads) {
+  if ((int)blockIdx.z < heads) stack_gemv_body<DT, SG_STORE, false, MR, KSPLIT>(a, blockIdx.x, 0, blockIdx.z);
+  else for (int t = blockIdx.x; t < m.T; t += gridDim.x) latent_append_body<DT>(m, la, t);
+}
 }  // namespace tgx
 
 int upload_param_ext(tgx_ctx* c, ebyte* dst, const void* host, int64_t n, int src_dtype);      // abi.hip
@@ -421,6 +427,29 @@ int ensure_ws(tgx_ctx* c, int T) {
   return TGX_OK;
 }
 
+// latents into the pool, and the queries into latent space (g, batched over the heads): in one launch in steps of few tokens
+void latent_in(tgx_ctx* c, const tgx::StepMeta& m, const tgx::LatentAppendArgs& la, tgx::StackGemmArgs g, int T, int H) {
+  if (c->stack->gemv && T <= 16 && slices_ok(g)) {
+    g.terms = c->act16 ? 1 : 2;
+    if (T <= GEMV_ROWS_MAX) {
+      const bool ksplit = gemv_ksplit(c, g, H);
+      const int cols = (ksplit ? 1 : 4) * tgx::STACK_GEMV_COLS;
+      const dim3 grid((g.N + cols - 1) / cols, 1, H + 1);
+      TGX_DT_SWITCH(c->dt,
+        auto go = [&](auto MR, auto KS) { hipLaunchKernelGGL((tgx::latent_append_gemv_kernel<DT, decltype(MR)::value, decltype(KS)::value>), grid, dim3(256), 0, c->stream, m, la, g, H); };
+        auto rows = [&](auto KS) { if (T == 1) go(std::integral_constant<int, 1>{}, KS); else go(std::integral_constant<int, 2>{}, KS); };
+        if (ksplit) rows(std::true_type{}); else rows(std::false_type{});)
+    } else {
+      const dim3 grid((g.N + 15) / 16, 1, H + 1);
+      TGX_DT_SWITCH(c->dt,
+        const tgx::FewPlan p = tgx::few_plan<DT, false, 1>(c->num_cus, (long long)grid.x * H, g.K);
+        if (stack_allow_lds(c, (const void*)&tgx::latent_append_queries_kernel<DT>, p.lds)) hipLaunchKernelGGL(tgx::latent_append_queries_kernel<DT>, grid, dim3(64 * p.nw), p.lds, c->stream, m, la, g, p.depth, H);)
+    }
+    return;
+  }
+  TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::latent_append_kernel<DT>, dim3(T), dim3(la.rot_dim > 0 ? 256 : 64), 0, c->stream, m, la))
+  launch_gemm(c, g, tgx::SG_STORE, H);
+}
 // the values of a latent attention from the records of its divided keys: merge and product in one launch in steps of few tokens (kernels/stack_latent.h), else the merge alone (false: the
 // product is still to come)
 bool latent_values(tgx_ctx* c, const tgx::LatentAttnArgs& aa, tgx::StackGemmArgs g, int T, int H) {
@@ -476,16 +505,7 @@ int run_layers_latent(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys
     g = tgx::StackGemmArgs{};
     g.A = sm->proj; g.lda = nin; g.a_zoff = ld.dim; g.B = w.w_ukT; g.ldb = ld.dim; g.b_zstride = (long long)R * ld.dim; g.C = sm->ql; g.ldc = (long long)H * R; g.c_zoff = R;
     g.M = T; g.N = R; g.K = ld.dim; g.scale = ld.scale;
-    if (sm->gemv && T > GEMV_ROWS_MAX && T <= 16 && slices_ok(g)) {
-      g.terms = c->act16 ? 1 : 2;
-      const dim3 grid((R + 15) / 16, 1, H + 1);
-      TGX_DT_SWITCH(c->dt,
-        const tgx::FewPlan p = tgx::few_plan<DT, false, 1>(c->num_cus, (long long)grid.x * H, g.K);
-        if (stack_allow_lds(c, (const void*)&tgx::latent_append_queries_kernel<DT>, p.lds)) hipLaunchKernelGGL(tgx::latent_append_queries_kernel<DT>, grid, dim3(64 * p.nw), p.lds, c->stream, m, la, g, p.depth, H);)
-    } else {
-      TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::latent_append_kernel<DT>, dim3(T), dim3(64), 0, c->stream, m, la))
-      launch_gemm(c, g, tgx::SG_STORE, H);
-    }
+    latent_in(c, m, la, g, T, H);
     // o[t][h] = (lat[t][h] . uv[h]^T) * sigmoid(gate)
     g = tgx::StackGemmArgs{};
     g.A = sm->lat; g.lda = (long long)H * R; g.a_zoff = R; g.B = w.w_uv; g.ldb = R; g.b_zstride = (long long)ld.vdim * R; g.C = sm->o; g.ldc = vd; g.c_zoff = ld.vdim;
@@ -1319,12 +1339,11 @@ int run_affine_latent(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, const 
   la.src = sm->proj; la.lds = nin; la.col0 = qd; la.nw = w.lat_norm; la.pool = run.pool; la.poolT = run.poolT; la.rank = R; la.eps = sm->d.norm_eps;
   la.rot_dim = ld.rot_dim; la.rot_dims = ld.rot_dims; la.cs = w.rot >= 0 ? sm->rot[(size_t)w.rot].cs : nullptr;
   la.q = sm->proj; la.heads = H; la.qstride = qs; la.qoff = ld.dim; la.qscale = ld.scale; la.ql = sm->ql;
-  TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::latent_append_kernel<DT>, dim3(T), dim3(256), 0, c->stream, m, la))
   // the plain part of every head's query into latent space: ql[t][h][0 .. R) = scale * q_plain[t][h] . ukT[h]^T
   g = tgx::StackGemmArgs{};
   g.A = sm->proj; g.lda = nin; g.a_zoff = qs; g.B = w.w_ukT; g.ldb = ld.dim; g.b_zstride = (long long)R * ld.dim; g.C = sm->ql; g.ldc = (long long)H * RR; g.c_zoff = RR;
   g.M = T; g.N = R; g.K = ld.dim; g.scale = ld.scale;
-  launch_gemm(c, g, tgx::SG_STORE, H);
+  latent_in(c, m, la, g, T, H);
   // o[t][h] = (lat[t][h][0 .. R) . uv[h]^T) * sigmoid(gate of the head, or of the channel)
   g = tgx::StackGemmArgs{};
   g.A = sm->lat; g.lda = (long long)H * RR; g.a_zoff = RR; g.B = w.w_uv; g.ldb = R; g.b_zstride = (long long)ld.vdim * R; g.C = sm->o; g.ldc = vd; g.c_zoff = ld.vdim;
