@@ -271,3 +271,22 @@ def test_rotated_latents_beside_their_queries(slots, kv_rank, dim, rot_dim):
     for i in {0, slots // 2, slots - 1}:
         want = tz.want_of(cfg, w, toks[i])
         assert np.abs(got[i] - want).max() / np.abs(want).max() < 1e-4, (slots, i)
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("kv_heads,dim,vdim,size", [(1, 8, 8, None), (2, 24, 40, 128), (4, 128, 512, 160), (4, 64, 16, 128)])
+def test_sigmoid_attention_appends_in_its_step(kv_heads, dim, vdim, size, dtype):
+    """single tokens whose keys are divided between workgroups: the last share stores the token's own row (one of its own, the last and the first of a tile and of a page), against the oracle"""
+    import test_hip_zaluvik as tz
+    cfg = tz.config([tz.attn(tz.dense(), heads=4, kv_heads=kv_heads, dim=dim, vdim=vdim, mask={"size": size} if size else None) for _ in range(2)], loop=None)
+    eng, w = tz.engine(cfg, dtype, 6)
+    toks = [tz.tokens(cfg, 200, i) for i in range(2)]
+    starts = [126, 188]      # keys that the steps see: 127 .. 131 and 189 .. 193, around a tile's and a page's first
+    got = [[], []]
+    eng.step([("s%d" % i, toks[i][:starts[i]], [0]) for i in range(2)])
+    for j in range(5):
+        step = eng.step([("s%d" % i, [toks[i][starts[i] + j]], [0]) for i in range(2)])
+        for i in range(2): got[i].append(step[i])
+    eng.close()
+    for i in range(2):
+        tz.check(np.stack(got[i]), tz.want_of(cfg, w, toks[i][:starts[i] + 5])[starts[i]:], dtype, f"sequence {i}")

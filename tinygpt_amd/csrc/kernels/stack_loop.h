@@ -167,6 +167,9 @@ struct MixAttnArgs {
   float scale;
   int mask_kind, mask_size;
   float* part; int nsplit, keys_per;    // split form: part [T][nsplit][heads * vdim]; split z takes keys_per keys from the first visible key on
+  // sigmoid_mix_step_kernel, single tokens: q holds the projections' row [q | k | v] as it comes, and the step appends the token itself (gqa_append_kernel's part): heads of q and k
+  // divided by sqrt(mean(head^2) + unit_eps) where that is positive, the row stored; poolVT: the values' transposed copy (nullptr: none)
+  int append; float unit_eps; void* poolVT;
 };
 inline size_t mix_attn_lds_bytes(int heads, int dim, int kt) { return ((size_t)heads * dim + 2 * (size_t)heads * kt + (size_t)heads * heads) * 4 + (size_t)kt * 4; }
 template <int DT, int NPT, bool VEC, bool SPLIT>
@@ -269,6 +272,7 @@ __global__ __launch_bounds__(256) void sigmoid_mix_attn_kernel(StepMeta m, MixAt
 // The split form of few tokens, whose workgroups each have a tile or two: bound by the chain of their loads (a key row a thread, four slices of it on their way, then the tile's value
 // rows four at a time: 18.5 us for two tokens over 1024 keys, 64 workgroups).  Here every load of a tile of 32 keys stands at once in whole lines: four keys a wave and turn, sixteen
 // lanes a key row, for the scores; a slice of eight value channels and every KG-th key a thread for the values, whose key groups meet in LDS.  9.0 us for the same (14.2 with runtime divisions in its index arithmetic and a sigmoid per head and lane).
+// Where every token is alone in its entry it also appends: 10.1 us in one launch where the walk was 9.1 and the append 5.3.
 // Rows of 16-byte slices, dim <= 128, at most 16 heads of at most four a key / value head, at most 256 value slices (mix_step_ok), rows of q at 16 bytes.
 constexpr int MIX_STEP_HEADS = 16, MIX_STEP_GROUP = 4, MIX_STEP_KEYS = 32;
 inline bool mix_step_ok(int heads, int kv_heads, int dim, int vdim) {
@@ -289,8 +293,39 @@ __global__ __launch_bounds__(256) void sigmoid_mix_step_kernel(StepMeta m, MixAt
   const elem_t<DT>* pk = reinterpret_cast<const elem_t<DT>*>(a.poolK);
   const elem_t<DT>* pv = reinterpret_cast<const elem_t<DT>*>(a.poolV);
   const int slices = vd >> 3, KG = 256 / slices, kg = tid / slices, sl = tid - kg * slices, vg = sl / (a.vdim >> 3);      // key groups; this thread's group, slice and key / value head
-  for (int h = tid >> 5; h < H; h += 8)
-    for (int c = 4 * (tid & 31); c < a.dim; c += 128) *reinterpret_cast<f32x4*>(&s_q[h][c]) = *reinterpret_cast<const f32x4*>(a.q + (size_t)t * a.ldq + (size_t)h * a.dim + c);
+  auto head = [&](const float* r) -> f32x4 {      // this lane's four channels of a head's 32, as the attention takes them
+    const int c = 4 * (tid & 31);
+    f32x4 x = {0.f, 0.f, 0.f, 0.f};
+    if (c < a.dim) x = *reinterpret_cast<const f32x4*>(r + c);
+    if (a.append && a.unit_eps > 0.f) {
+      const float ss = row_group_sum<32>(fmaf(x[0], x[0], x[1] * x[1]) + fmaf(x[2], x[2], x[3] * x[3]));
+      x *= 1.0f / sqrtf(ss / (float)a.dim + a.unit_eps);
+    }
+    return x;
+  };
+  const float* qr = a.q + (size_t)t * a.ldq;
+  if (a.append && k1 == pos + 1 && k0 < k1) {      // (uniform) the share that ends with the token's own key stores its row before any of its keys is read
+    const float *kr = qr + (size_t)H * a.dim, *vr = kr + kd;
+    elem_t<DT>*kdst = reinterpret_cast<elem_t<DT>*>(const_cast<void*>(a.poolK)) + slot_of(pos) * kd, *vdst = reinterpret_cast<elem_t<DT>*>(const_cast<void*>(a.poolV)) + slot_of(pos) * vd;
+    for (int g = tid >> 5; g < G; g += 8) {
+      const f32x4 x = head(kr + (size_t)g * a.dim);
+      if (4 * (tid & 31) < a.dim)
+#pragma unroll
+        for (int e = 0; e < 4; e++) kdst[(size_t)g * a.dim + 4 * (tid & 31) + e] = f32_to_elem<DT>(x[e]);
+    }
+    elem_t<DT>* vt = a.poolVT ? reinterpret_cast<elem_t<DT>*>(a.poolVT) + (((size_t)tbl[pos >> m.page_shift] * vd) << m.page_shift) + (size_t)(pos & pmask) : nullptr;
+    for (int c = tid; c < vd; c += 256) {
+      const elem_t<DT> e = f32_to_elem<DT>(vr[c]);
+      vdst[c] = e;
+      if (vt) vt[(size_t)c << m.page_shift] = e;
+    }
+    __threadfence_block();
+    __syncthreads();
+  }
+  for (int h = tid >> 5; h < H; h += 8) {
+    const f32x4 x = head(qr + (size_t)h * a.dim);
+    if (4 * (tid & 31) < a.dim) *reinterpret_cast<f32x4*>(&s_q[h][4 * (tid & 31)]) = x;
+  }
   if (a.talk && (tid >> 4) < H && (tid & 15) < H) s_t[tid >> 4][tid & 15] = a.talk[(tid >> 4) * H + (tid & 15)];
   float acc[MQ][8];
 #pragma unroll

@@ -1267,8 +1267,9 @@ int run_affine_attention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, con
   const bool mfma = run.poolT && sm->attn_mfma && max_count >= MIX_MFMA_MIN_COUNT;
   ap.poolVT = run.poolT;
   if (mfma) { ap.q_hi = sm->qplanes; ap.q_lo = sm->qplanes + (((size_t)sm->cap_tokens * sm->max_qd + 7) & ~(size_t)7); }      // (both planes 16-byte aligned)
-  TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::gqa_append_kernel<DT>, dim3(T), dim3(256), 0, c->stream, m, ap))
+  auto append = [&] { TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::gqa_append_kernel<DT>, dim3(T), dim3(256), 0, c->stream, m, ap)) };
   if (mfma) {
+    append();
     tgx::MixMfmaArgs ma{};
     ma.qh = ap.q_hi; ma.ql = ap.q_lo; ma.poolK = run.pool; ma.poolVT = run.poolT; ma.pb = w.pb; ma.talk = ld.head_mix ? w.talk : nullptr;
     ma.gate = ld.gate_kind == 1 ? sm->proj + qd + kd + kvv : nullptr; ma.ldg = nin; ma.out = sm->o; ma.ldo = vd;
@@ -1313,10 +1314,18 @@ int run_affine_attention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, con
   if (nsplit > 1 && ensure_part(c, (size_t)T * nsplit * (size_t)vd)) {
     aa.kt = std::min(aa.kt, aa.keys_per);
     aa.part = sm->part; aa.nsplit = nsplit;
-    if (nin % 4 == 0 && tgx::mix_step_ok(H, G, ld.dim, ld.vdim)) TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::sigmoid_mix_step_kernel<DT>, dim3(T, nsplit), dim3(256), 0, c->stream, m, aa))
-    else TGX_DT_SWITCH(c->dt, (launch_mix_attn_t<DT, true>(c, m, aa, dim3(T, nsplit), lds, vec)))
+    if (nin % 4 == 0 && tgx::mix_step_ok(H, G, ld.dim, ld.vdim)) {
+      // tokens alone in their entries: no other workgroup reads a row that the step appends
+      aa.append = max_count == 1; aa.unit_eps = ap.qk_unit_eps; aa.poolVT = ap.poolVT;
+      if (!aa.append) append();
+      TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::sigmoid_mix_step_kernel<DT>, dim3(T, nsplit), dim3(256), 0, c->stream, m, aa))
+    } else {
+      append();
+      TGX_DT_SWITCH(c->dt, (launch_mix_attn_t<DT, true>(c, m, aa, dim3(T, nsplit), lds, vec)))
+    }
     hipLaunchKernelGGL(tgx::sigmoid_mix_merge_kernel, dim3(T, std::min(8, (vd + 255) / 256)), dim3(256), 0, c->stream, aa);
   } else {
+    append();
     TGX_DT_SWITCH(c->dt, (launch_mix_attn_t<DT, false>(c, m, aa, dim3(T), lds, vec)))
   }
   // y = o . w_o^T
