@@ -391,48 +391,93 @@ __global__ __launch_bounds__(256) void latent_attn_merge_kernel(LatentAttnArgs a
 // choice kernels take the products themselves.
 struct RouterInput { const float* h; long long ldh; const float* w; int n, K; };      // h nullptr: the products are given
 constexpr int ROUTER_FUSED_MAX = 64;      // products a choice kernel takes itself
-__device__ __forceinline__ void router_products(const RouterInput& in, int t, float* s_z) {
+// What a choice kernel asks for before the work in front of it: a word of every line of the weights (up to 256 KB of them), which are then in L2 when the products want them, and a
+// lane's entry of what is added to the choice scores.
+struct RouterAhead { float add, touch[8]; };
+__device__ __forceinline__ RouterAhead router_ahead(const RouterInput& in, const float* add, int E) {
+  RouterAhead r;
+  const int tid = threadIdx.x, words = in.n * in.K;
+  r.add = add && tid < E ? add[tid] : 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; i++) r.touch[i] = 256 * 32 * i < words ? in.w[min(32 * (tid + 256 * i), words - 1)] : 0.f;
+  return r;
+}
+__device__ __forceinline__ void router_products(const RouterInput& in, int t, float* s_z, const RouterAhead& ahead) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const float* h = in.h + (size_t)t * in.ldh;
-  for (int e0 = 4 * wv; e0 < in.n; e0 += 16) {
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 4 * lane; k0 < in.K; k0 += 1024) {      // every load of 1024 channels and four products in flight at once; loads past the end repeat it and are dropped
-      f32x4 x[4], w[4][4];
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int k = min(k0 + 256 * i, in.K - 4);
-        x[i] = *reinterpret_cast<const f32x4*>(h + k);
+  for (int i = 0; i < 8; i++) asm volatile("" ::"v"(ahead.touch[i]));
+  // a wave's products in rounds of four and 1024 channels, the next round's loads in flight beside a round's sums; loads past the end repeat it and are dropped
+  struct Round { f32x4 x[4], w[4][4]; };
+  auto load = [&](Round& r, int e0, int k0) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) w[i][j] = *reinterpret_cast<const f32x4*>(in.w + (size_t)min(e0 + j, in.n - 1) * in.K + k);
-      }
-      __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < 4; i++) {
+      const int k = min(k0 + 256 * i, in.K - 4);
+      r.x[i] = *reinterpret_cast<const f32x4*>(h + k);
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const bool on = k0 + 256 * i < in.K;
+      for (int j = 0; j < 4; j++) r.w[i][j] = *reinterpret_cast<const f32x4*>(in.w + (size_t)min(e0 + j, in.n - 1) * in.K + k);
+    }
+  };
+  const int share = (in.n + 3) / 4, end = min(in.n, share * (wv + 1));
+  int e0 = share * wv, k0 = 4 * lane;      // (k0 - 4 lane is the same in every lane)
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  auto sums = [&](const Round& r) {
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
+    for (int i = 0; i < 4; i++) {
+      const bool on = k0 + 256 * i < in.K;
 #pragma unroll
-          for (int j = 0; j < 4; j++) acc[j] = on ? fmaf(x[i][u], w[i][j][u], acc[j]) : acc[j];
-        }
+      for (int u = 0; u < 4; u++) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[j] = on ? fmaf(r.x[i][u], r.w[i][j][u], acc[j]) : acc[j];
       }
     }
+  };
+  auto step = [&](Round& now, Round& next) -> bool {      // false: that was the last round
+    int e1 = e0, k1 = k0 + 1024;
+    if (k1 - 4 * lane >= in.K) { e1 += 4; k1 = 4 * lane; }
+    const bool more = e1 < end;
+    if (more) load(next, e1, k1);
+    __builtin_amdgcn_sched_barrier(0);
+    sums(now);
+    if (e1 != e0) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) { const float v = wave_sum(acc[j]); if (lane == 0 && e0 + j < in.n) s_z[e0 + j] = v; }
+      for (int j = 0; j < 4; j++) { const float v = wave_sum(acc[j]); if (lane == 0 && e0 + j < end) s_z[e0 + j] = v; acc[j] = 0.f; }
+    }
+    e0 = e1; k0 = k1;
+    return more;
+  };
+  if (e0 < end) {
+    Round a, b;
+    load(a, e0, k0);
+    while (step(a, b) && step(b, a)) {}
   }
   __syncthreads();
 }
 
-// the largest of s[0 .. n) and its index (ties: the lower; 0x7fffffff where all are -inf), in every lane of the wave.  ONE: n <= 64, a number per lane: the
-// maximum alone crosses the lanes and a ballot finds its first holder
-template <bool ONE>
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ float dpp_max(float v) {
+  const int b = __builtin_bit_cast(int, v);
+  return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(b, b, CTRL, ROW_MASK, 0xf, false)));
+}
+__device__ __forceinline__ float wave_max(float v) {      // wave_sum's steps
+  v = dpp_max<0xB1, 0xf>(v);
+  v = dpp_max<0x4E, 0xf>(v);
+  v = dpp_max<0x141, 0xf>(v);
+  v = dpp_max<0x140, 0xf>(v);
+  v = dpp_max<0x142, 0xa>(v);
+  v = dpp_max<0x143, 0xc>(v);
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+}
+// the first lane that holds the wave's largest value (-1: all are -inf), which is left in bv
+__device__ __forceinline__ int wave_first_max(float v, float& bv) {
+  bv = wave_max(v);
+  const unsigned long long mask = __ballot(v == bv && v > -INFINITY);
+  return mask ? (int)__builtin_ctzll(mask) : -1;
+}
+__device__ __forceinline__ float lane_value(float v, int lane) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane)); }
+// the largest of s[0 .. n) and its index (ties: the lower; 0x7fffffff where all are -inf), in every lane of the wave
 __device__ __forceinline__ int wave_pick(const float* s, int n, float& bv) {
   const int lane = threadIdx.x & 63;
-  if constexpr (ONE) {
-    const float v = lane < n ? s[lane] : -INFINITY;
-    bv = group_max<64>(v);
-    const unsigned long long mask = __ballot(v == bv && v > -INFINITY);
-    return mask ? (int)__builtin_ctzll(mask) : 0x7fffffff;
-  }
   int bi = 0x7fffffff;
   bv = -INFINITY;
   for (int e = lane; e < n; e += 64) { const float v = s[e]; if (v > bv) { bv = v; bi = e; } }
@@ -454,22 +499,17 @@ struct RouterArgs {
   int E, top;
 };
 constexpr int ROUTER_MAX_E = 1024, ROUTER_MAX_TOP = 64;
-template <bool PRODUCT>
-__device__ __forceinline__ void router_topk_body(RouterArgs a) {
+__global__ __launch_bounds__(64) void router_topk_kernel(RouterArgs a) {
   __shared__ float s_z[ROUTER_MAX_E];
   __shared__ float s_v[ROUTER_MAX_TOP];
   __shared__ int s_i[ROUTER_MAX_TOP];
   const int t = blockIdx.x, lane = threadIdx.x;
   // every lane owns the logits e = lane, lane + 64, ...: it alone writes, reads and retires them, so the loop needs no barrier; the butterfly leaves each
   // pick in all lanes, lane 0 keeps the list
-  if constexpr (PRODUCT) {
-    router_products(a.in, t, s_z);
-    if (lane >= 64) return;      // (no barrier below)
-    for (int e = lane; e < a.E; e += 64) s_z[e] += a.br[e];
-  } else for (int e = lane; e < a.E; e += 64) s_z[e] = a.z[(size_t)t * a.E + e] + a.br[e];
+  for (int e = lane; e < a.E; e += 64) s_z[e] = a.z[(size_t)t * a.E + e] + a.br[e];
   for (int k = 0; k < a.top; k++) {
     float bv;
-    const int bi = wave_pick<PRODUCT>(s_z, a.E, bv);
+    const int bi = wave_pick(s_z, a.E, bv);
     if (bi < a.E && (bi & 63) == lane) s_z[bi] = -INFINITY;
     if (lane == 0) { s_v[k] = bv; s_i[k] = bi < a.E ? bi : 0; }
   }
@@ -479,13 +519,31 @@ __device__ __forceinline__ void router_topk_body(RouterArgs a) {
   for (int k = 0; k < a.top; k++) den += expf(s_v[k] - mx);
   for (int k = lane; k < a.top; k += 64) { a.sel[(size_t)t * a.top + k] = s_i[k]; a.selw[(size_t)t * a.top + k] = expf(s_v[k] - mx) / den; }
 }
-__global__ __launch_bounds__(64) void router_topk_kernel(RouterArgs a) { router_topk_body<false>(a); }
-// A few tokens' norm and convolution with the choice of experts behind it, whose products a workgroup takes from the row that it has just written: a launch less (one of 2.6 us at least)
+// A few tokens' norm and convolution with the choice of experts behind it, whose products a workgroup takes from the row that it has just written: a launch less (one of 2.6 us at
+// least).  Up to 64 products, a lane each: scores, picks and weights never leave the registers.
+// Bound by a chain: the row's loads, its sums, the row and the weights from L2, the picks.  The weights were first asked for behind the row's barrier, and every pick went through LDS: one
+// token of 1024 channels 6.4 us, 5.8 now; the other seams 8.0 and 6.5 (two of 512, 16 experts in groups), 12.5 and 10.2 (one of 2048, 20), 6.8 and 6.5 (16 of four streams).
 template <int TAPS>
 __global__ __launch_bounds__(256) void norm_conv_route_kernel(StepMeta m, NormConvArgs a, RouterArgs r) {
+  __shared__ float s_z[ROUTER_FUSED_MAX];
+  const RouterAhead ahead = router_ahead(r.in, r.br, r.E);
   norm_conv_body<TAPS>(m, a);
   __syncthreads();
-  router_topk_body<true>(r);
+  const int t = blockIdx.x, lane = threadIdx.x;
+  router_products(r.in, t, s_z, ahead);
+  if (lane >= 64) return;      // (no barrier below)
+  float c = lane < r.E ? s_z[lane] + ahead.add : -INFINITY, v = -INFINITY;
+  int pick = 0;                // lane k: the k-th pick
+  for (int k = 0; k < r.top; k++) {
+    float bv;
+    const int bi = wave_first_max(c, bv);
+    if (bi == lane) c = -INFINITY;
+    if (lane == k) { v = bv; pick = max(bi, 0); }
+  }
+  const float mx = lane_value(v, 0), p = expf(v - mx);      // the first pick is the largest
+  float den = 0.f;
+  for (int k = 0; k < r.top; k++) den += lane_value(p, k);
+  if (lane < r.top) { r.sel[(size_t)t * r.top + lane] = pick; r.selw[(size_t)t * r.top + lane] = p / den; }
 }
 
 // ---- plan of the grouped expert products: pairs i = t * top + k grouped by expert.  One workgroup.

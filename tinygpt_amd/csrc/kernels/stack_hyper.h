@@ -167,9 +167,10 @@ template <int NS>
 __global__ __launch_bounds__(256) void hyper_seam_kernel(HyperSeamArgs a) { hyper_seam_body<NS>(a); }
 template <int NS>
 __global__ __launch_bounds__(256) void hyper_seam_route_kernel(HyperSeamArgs a, RouterGroupArgs r) {      // (as sandwich_route_kernel)
+  const RouterAhead ahead = router_ahead(r.in, r.corr, r.E);
   hyper_seam_body<NS>(a);
   __syncthreads();
-  router_group_body<true>(r);
+  router_group_lanes(r, ahead);
 }
 
 // ---- out[t][h] = d / sqrt(mean(d^2) + eps) * scale, d = o_1 - lambda o_2 of the head's two maps.  One wave per (token, head); vdim <= 64 GQA_MAX_RPL.

@@ -140,9 +140,10 @@ template <int NR>
 __global__ __launch_bounds__(256) void affine_seam_kernel(AffineSeamArgs a) { affine_seam_body<NR>(a); }
 template <int NR>
 __global__ __launch_bounds__(256) void affine_seam_route_kernel(AffineSeamArgs a, RouterGroupArgs r) {      // (as sandwich_route_kernel)
+  const RouterAhead ahead = router_ahead(r.in, r.corr, r.E);
   affine_seam_body<NR>(a);
   __syncthreads();
-  router_group_body<true>(r);
+  router_group_lanes(r, ahead);
 }
 
 // ---- sigmoid attention with mixed heads.  For the query token i and every key j it sees (a sliding window, a chunk, or all before it: stack_meta.h):

@@ -589,17 +589,11 @@ struct RouterGroupArgs {
   int shared, shared_at;     // 1: every token has one more choice behind its top, expert shared_at (the outputs from there on count one more) with weight 1 or, with sgw, that gate:
                              // a shared expert that rides among the routed ones
 };
-template <bool PRODUCT>
-__device__ __forceinline__ void router_group_body(RouterGroupArgs a) {
-  constexpr int ME = PRODUCT ? ROUTER_FUSED_MAX : ROUTER_MAX_E;
-  __shared__ float s_s[ME], s_c[ME], s_g[ME], s_z[PRODUCT ? ME : 1], s_pw[ROUTER_MAX_TOP];
+__global__ __launch_bounds__(64) void router_group_kernel(RouterGroupArgs a) {
+  __shared__ float s_s[ROUTER_MAX_E], s_c[ROUTER_MAX_E], s_g[ROUTER_MAX_E], s_pw[ROUTER_MAX_TOP];
   __shared__ int s_pick[ROUTER_MAX_TOP];
   const int t = blockIdx.x, lane = threadIdx.x, stride = a.top + a.shared;
-  const float* z = s_z;
-  if constexpr (PRODUCT) {
-    router_products(a.in, t, s_z);
-    if (threadIdx.x >= 64) return;      // one wave chooses: its barriers below are its own
-  } else z = a.z + (size_t)t * a.ldz;
+  const float* z = a.z + (size_t)t * a.ldz;
   if (a.sigmoid_scores) {
     for (int e = lane; e < a.E; e += 64) { s_s[e] = 1.0f / (1.0f + expf(-z[e])); s_c[e] = a.corr ? s_s[e] + a.corr[e] : s_s[e]; }
   } else {
@@ -637,7 +631,7 @@ __device__ __forceinline__ void router_group_body(RouterGroupArgs a) {
   float sum = 0.f;      // in choice order
   for (int k = 0; k < a.top; k++) {
     float bv;
-    const int bi = wave_pick<PRODUCT>(s_c, a.E, bv), pick = bi < a.E ? bi : 0;
+    const int bi = wave_pick(s_c, a.E, bv), pick = bi < a.E ? bi : 0;
     if (bi < a.E && (bi & 63) == lane) s_c[bi] = -INFINITY;
     const float v = bi < a.E ? s_s[pick] * a.scale : 0.f;
     sum += v;
@@ -650,13 +644,64 @@ __device__ __forceinline__ void router_group_body(RouterGroupArgs a) {
   if (a.shared && lane == 0) { a.sel[(size_t)t * stride + a.top] = a.shared_at; a.selw[(size_t)t * stride + a.top] = sg; }
   if (a.sgw && lane == 0) a.sgw[t] = sg;
 }
-__global__ __launch_bounds__(64) void router_group_kernel(RouterGroupArgs a) { router_group_body<false>(a); }
+// the same behind a seam: the workgroup takes the products itself (up to 64, a lane each), and scores, picks and weights stay in the registers of its first wave
+__device__ __forceinline__ void router_group_lanes(RouterGroupArgs a, const RouterAhead& ahead) {
+  __shared__ float s_z[ROUTER_FUSED_MAX], s_c[ROUTER_FUSED_MAX];
+  const int t = blockIdx.x, lane = threadIdx.x, stride = a.top + a.shared;
+  router_products(a.in, t, s_z, ahead);
+  if (threadIdx.x >= 64) return;
+  const bool own = lane < a.E;
+  const float z = own ? s_z[lane] : -INFINITY;
+  float s;
+  if (a.sigmoid_scores) s = 1.0f / (1.0f + expf(-z));
+  else {
+    const float mx = wave_max(z), p = own ? expf(z - mx) : 0.f;
+    s = p / wave_sum(p);
+  }
+  float c = own ? s + ahead.add : -INFINITY;
+  if (a.groups > 1) {
+    const int per = a.E / a.groups;
+    s_c[lane] = c;
+    wave_fence();
+    float g = -INFINITY, b2 = -INFINITY;      // a lane's group: the largest and the second largest
+    if (lane < a.groups) {
+#pragma unroll 4
+      for (int e = lane * per; e < (lane + 1) * per; e++) { const float v = s_c[e]; if (v > g) { b2 = g; g = v; } else b2 = fmaxf(b2, v); }
+      if (a.group_top2 && per > 1) g += b2;
+    }
+    unsigned long long kept = __ballot(g == INFINITY);      // the `keep` best groups (one of +inf in any case), a pick a round
+    if (g == INFINITY) g = -INFINITY;
+    for (int k = 0; k < a.keep; k++) {
+      float bv;
+      const int bi = wave_first_max(g, bv);
+      if (bi == lane) g = -INFINITY;
+      if (bi >= 0) kept |= 1ull << bi;
+    }
+    if (own && !(kept >> (lane / per) & 1)) c = -INFINITY;
+  }
+  float sum = 0.f, w = 0.f;      // sum in choice order; lane k: the k-th pick and its weight
+  int pick = 0;
+  for (int k = 0; k < a.top; k++) {
+    float bv;
+    const int bi = wave_first_max(c, bv);
+    if (bi == lane) c = -INFINITY;
+    const float v = bi >= 0 ? lane_value(s, bi) * a.scale : 0.f;
+    sum += v;
+    if (lane == k) { pick = max(bi, 0); w = v; }
+  }
+  if (a.normalise) w *= a.scale / (sum + 1e-20f * a.scale);
+  if (lane < a.top) { a.sel[(size_t)t * stride + lane] = pick + (a.shared && pick >= a.shared_at ? 1 : 0); a.selw[(size_t)t * stride + lane] = w; }
+  const float sg = a.sgw ? 1.0f / (1.0f + expf(-s_z[a.E])) : 1.f;
+  if (a.shared && lane == 0) { a.sel[(size_t)t * stride + a.top] = a.shared_at; a.selw[(size_t)t * stride + a.top] = sg; }
+  if (a.sgw && lane == 0) a.sgw[t] = sg;
+}
 // a few tokens' seam with the choice of experts behind it (as norm_conv_route_kernel)
 template <int NR>
 __global__ __launch_bounds__(256) void sandwich_route_kernel(SandwichArgs a, RouterGroupArgs r) {
+  const RouterAhead ahead = router_ahead(r.in, r.corr, r.E);
   sandwich_body<NR>(a);
   __syncthreads();
-  router_group_body<true>(r);
+  router_group_lanes(r, ahead);
 }
 
 }  // namespace tgx
