@@ -342,3 +342,27 @@ def test_terms_of_a_norm(design, width, dtype):
         got.append(eng.step([("p", ids, want)], ["p"]))
     eng.close()
     assert np.isfinite(got[0]).all() and (got[0] == got[1]).all()
+
+
+@pytest.mark.parametrize("dim,vdim", [(16, 16), (128, 40), (136, 33)])      # one and two tiles of state rows, ragged columns
+@pytest.mark.parametrize("sizes", [[384, 5], [385, 193, 64, 1], [700, 320], [320, 129]])      # portions of two blocks and more: whole and ragged ones, an entry of one portion, none at all
+@pytest.mark.parametrize("design", ["modepel", "keronex"])
+def test_scalar_decay_in_portions(design, sizes, dim, vdim):
+    """long entries' blocks in portions that run side by side, from the start of a sequence and from a state that it left, against the recurrence token by token (fp32 both)"""
+    if design == "modepel":
+        t, cfg = tm, tm.config([tm.rec(heads=2, dim=dim, vdim=vdim)], width=64)
+    else:
+        import test_hip_keronex as tk
+        t, cfg = tk, tk.config([tk.ret(heads=2, dim=dim, vdim=vdim, decay=[0.9, 0.99], rot=None)], width=64)
+    got = {}
+    for least in (64, 0):
+        eng, w = t.engine(cfg, seed=3, max_seqs=len(sizes), max_ctx=2048, budget_tokens=4096)
+        eng.model.set_option("ssd.min", least)
+        out = []
+        for step in range(2):      # (the second in reverse: the longest entry is not the first)
+            ids = list(range(len(sizes)))[::-1 if step else 1]
+            out.append(eng.step([("s%d" % i, t.tokens(cfg, sizes[i], 10 * step + i), [0, sizes[i] // 2, sizes[i] - 1]) for i in ids]))
+        out.append(eng.step([("s%d" % i, t.tokens(cfg, 1, i), [0]) for i in range(len(sizes))]))
+        got[least] = np.concatenate(out)
+        eng.close()
+    assert np.abs(got[64] - got[0]).max() / np.abs(got[0]).max() < 1e-4

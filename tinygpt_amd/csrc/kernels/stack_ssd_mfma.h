@@ -27,6 +27,8 @@ struct SsdArgs {
   float* out; long long ldo;           // [T][heads E]
   float* norm_S; size_t norm_buf;      // a second state N_t = g_t N_(t-1) + dt_t B_t, the sum that a matrix memory divides by: [2][slots][heads][N], norm_buf between the two (nullptr: none)
   float* norm_out; long long ldn;      // N_t . C_t: [T][heads]
+  int portion, portions;               // blocks of a portion (portions > 1: the longest entry's; an entry may have fewer)
+  float* states;                       // [entries][portions][heads][tiles][ssd_state_elems]: what the portions before leave (SSD_STATES)
 };
 // the first block of an entry in `gram`: entries never share a block
 __device__ __forceinline__ int ssd_first_block(int start, int e) { return start / SSD_BLOCK + e; }
@@ -71,12 +73,27 @@ __global__ __launch_bounds__(256) void ssd_gram_kernel(StepMeta m, SsdArgs a) {
 // NW: 32-row tiles of the state per wave (4 NW 32 >= N).  Wave w owns the state rows n of its tiles and 32 columns, in the accumulator layout: register r of a lane is
 // row (r & 3) + 8 (r >> 2) + 4 (lane / 32), column lane % 32.  Register r of the two half-waves is at the same time a B operand whose two contraction slots are those
 // two rows, so S^T C needs no transposition: its A operand takes C's channels in that order.  A wave contributes its rows' share of S^T C and the share of sixteen
-// keys j of the block's own product; the four waves' shares are added up in LDS.  Grid: (entries, heads, E / 32).
+// keys j of the block's own product; the four waves' shares are added up in LDS.  Grid: (heads, E / 32, entries portions).
 // Operands travel straight from memory to registers (every wave reads its own state rows only): B of a block is asked for at the block's start and used at its end,
 // C and the Gram rows of the next block replace the present ones as soon as these are used up, so nothing is held twice.  Rows past the
 // entry's end are clamped to its last one (what is read there twice meets dt = 0 or is not stored).
-// NORM: the grid's last z index carries the second state: the recurrence with x = 1 in one column.
-template <int NW, bool NORM = false>
+// NORM: the grid's last tile carries the second state: the recurrence with x = 1 in one column.
+// Entries and heads that leave the chip idle: a chain of blocks, 6.6 us each on 72 workgroups (2048 tokens, 8 heads of 128 x 256).  So an entry's blocks are cut into portions, which two
+// launches take at once: SSD_STATES the state that every portion but the last adds to a state of zero (the first: leaves behind the entry's own), and how much it decays; SSD_PORTIONS
+// every portion from its state, which is the first's and those after it in order: 27 us and 53 in seven portions where the chain took 212.
+// Entries that fill the chip are taken longest first, heads beside each other, so that no long one is left for the end: eight documents of up to 2048 tokens, 64 heads of 128 x 64,
+// 649 us a launch with the entries beside each other, 436 now.
+enum { SSD_WHOLE = 0, SSD_STATES = 1, SSD_PORTIONS = 2 };
+constexpr size_t ssd_state_elems(int NW) { return (size_t)NW * 16 * 256 + 4; }      // a workgroup's accumulators as it holds them, and the portion's decay
+// the entry of rank r by its tokens, longest first (the entry r itself where there are more than 64)
+__device__ __forceinline__ int entry_by_length(const StepMeta& m, int entries, int r) {
+  if (entries > 64) return r;
+  const int lane = threadIdx.x & 63, mine = lane < entries ? m.ent_count[lane] : -1;
+  int rank = 0;
+  for (int j = 0; j < entries; j++) { const int other = __builtin_amdgcn_readlane(mine, j); rank += other > mine || (other == mine && j < lane); }
+  return __builtin_ctzll(__ballot(lane < entries && rank == r));
+}
+template <int NW, bool NORM = false, int MODE = SSD_WHOLE>
 __global__ __launch_bounds__(256, NW == 1 ? 2 : 1) void ssd_block_kernel(StepMeta m, SsdArgs a) {
   constexpr int Q = SSD_BLOCK;
   constexpr double LOG2E = 1.4426950408889634;
@@ -84,10 +101,13 @@ __global__ __launch_bounds__(256, NW == 1 ? 2 : 1) void ssd_block_kernel(StepMet
   __shared__ double s_cs[2][Q];        // base-2 logarithms, summed from the block's start
   __shared__ float s_dt[2][Q], s_end[2][Q];      // dt_j, exp(cs_64 - cs_j) dt_j
   __shared__ float s_part[4][Q][33];
-  const int e = blockIdx.x, h = blockIdx.y, e0 = blockIdx.z * 32, tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), half = lane >> 5, l31 = lane & 31;
+  const int P = MODE == SSD_WHOLE ? 1 : a.portions, part = MODE == SSD_WHOLE ? 0 : blockIdx.z % P, tile = blockIdx.y, tiles = gridDim.y;
+  const int e = entry_by_length(m, gridDim.z / P, blockIdx.z / P), h = blockIdx.x, e0 = tile * 32, tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), half = lane >> 5, l31 = lane & 31;
   const int start = m.ent_start[e], cnt = m.ent_count[e], slot = m.ent_row[e], grp = h / (a.heads / a.groups);
+  const int nblk = (cnt + Q - 1) / Q, b0 = MODE == SSD_WHOLE ? 0 : part * a.portion, b1 = MODE == SSD_WHOLE ? nblk : min(nblk, b0 + a.portion);
+  if (MODE == SSD_STATES ? b1 >= nblk : b0 >= nblk) return;      // (the states of the last portion are nobody's start)
   const bool fresh = m.tok_pos[start] == 0;
-  const bool ones = NORM && blockIdx.z + 1 == gridDim.z;
+  const bool ones = NORM && tile + 1 == tiles;
   const int ld = (int)a.ld, ldg = (int)a.ldgate, oX = a.x0 + h * a.E + e0, oB = a.b0 + grp * a.N, oC = a.c0 + grp * a.N;
   const float* base = a.row + (size_t)start * ld;
   const float* gbase = a.gates + (size_t)start * ldg + h;
@@ -103,13 +123,31 @@ __global__ __launch_bounds__(256, NW == 1 ? 2 : 1) void ssd_block_kernel(StepMet
     Sg = a.norm_S + (size_t)par * a.norm_buf + at; Snew = a.norm_S + (size_t)(par ^ 1) * a.norm_buf + at;
   }
   f32x16 S[NW];
+  // slot 0: the entry's own state, slot p + 1: what portion p leaves
+  auto left = [&](int p) { return a.states + ((((size_t)e * P + p) * a.heads + h) * tiles + tile) * ssd_state_elems(NW); };
+  if (MODE != SSD_PORTIONS || nblk <= a.portion) {
 #pragma unroll
-  for (int w = 0; w < NW; w++)
+    for (int w = 0; w < NW; w++)
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int n = n0 + 32 * w + (r & 3) + 8 * (r >> 2) + 4 * half;
-      S[w][r] = (!fresh && n < a.N && colok) ? Sg[n * sn + sc] : 0.f;
+      for (int r = 0; r < 16; r++) {
+        const int n = n0 + 32 * w + (r & 3) + 8 * (r >> 2) + 4 * half;
+        S[w][r] = (!fresh && n < a.N && colok && (MODE != SSD_STATES || part == 0)) ? Sg[n * sn + sc] : 0.f;
+        if (MODE == SSD_STATES && part == 0) left(0)[(w * 16 + r) * 256 + tid] = S[w][r];      // (the last portion may have replaced it before the first one looks)
+      }
+  } else {
+#pragma unroll
+    for (int w = 0; w < NW; w++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) S[w][r] = left(min(part, 1))[(w * 16 + r) * 256 + tid];
+    for (int p = 2; p <= part; p++) {
+      const float* s = left(p);
+      const float g = s[NW * 4096];
+#pragma unroll
+      for (int w = 0; w < NW; w++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) S[w][r] = fmaf(S[w][r], g, s[(w * 16 + r) * 256 + tid]);
     }
+  }
   auto at = [](const float* p, unsigned int bytes) -> const float* { return reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + bytes); };
   // byte offset of row t0 + k of a block with `left` rows, clamped to its last one (ld < 2^21 floats: the factors fit 24 bits); the constant k stays out of registers
   auto row_at = [](int t0, int k, int left, int ld) -> unsigned int { return (unsigned int)(4 * (__mul24(t0, ld) + __mul24(min(k, left - 1 - t0), ld))); };
@@ -117,7 +155,7 @@ __global__ __launch_bounds__(256, NW == 1 ? 2 : 1) void ssd_block_kernel(StepMet
   float B[NW][32], x[8], dt = 0.f, la = 0.f;      // B[n][j]: j = kk + 32 half
   f32x4 C[NW][2][4], G[2][2];                     // C[i][n]: four channels at a time; the Gram rows of this wave's sixteen keys j = 16 wv + 8 half + 0 .. 7
   // (what stands in state rows beyond N is finite and meets a factor of zero)
-  auto fetch_B = [&](int b) {
+  auto fetch_B = [&](int b, float (*B)[32]) {
     const float* p = base + (size_t)b * Q * ld + oB;
     const int left = cnt - b * Q;
 #pragma unroll
@@ -170,14 +208,54 @@ __global__ __launch_bounds__(256, NW == 1 ? 2 : 1) void ssd_block_kernel(StepMet
   };
   if (a.fixed) { dt = a.dt0; la = a.fixed[a.heads + h]; }
   const float Dh = a.skip ? a.skip[h] : 0.f;
-  const int nblk = (cnt + Q - 1) / Q;
-  fetch_x(0); fetch_C(0); fetch_G(0);
-  stage(0);
-  for (int b = 0; b < nblk; b++) {
+  auto add_block = [&](int buf, float (*B)[32]) {      // S = exp(cs_64) S + sum_j B_j (exp(cs_64 - cs_j) dt_j x_j)^T
+    const float ge = __builtin_amdgcn_exp2f((float)s_cs[buf][Q - 1]);
+#pragma unroll
+    for (int w = 0; w < NW; w++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) S[w][r] *= ge;
+    if (n0 < a.N)
+#pragma unroll
+      for (int kk = 0; kk < 32; kk++) {
+        const int j = kk + 32 * half;
+        const float xs = s_x[buf][j][l31] * s_end[buf][j];
+#pragma unroll
+        for (int w = 0; w < NW; w++) S[w] = __builtin_amdgcn_mfma_f32_32x32x2f32(B[w][kk], xs, S[w], 0, 0, 0);
+      }
+  };
+  fetch_x(b0);
+  if constexpr (MODE == SSD_STATES) {
+    double decay = 0.0;
+    auto block = [&](int b, float (*now)[32], float (*next)[32]) {
+      const bool more = b + 1 < b1;
+      __syncthreads();      // the block's columns and sums stand; those of the block before have been read
+      if (more) { fetch_x(b + 1); fetch_B(b + 1, next); }
+      __builtin_amdgcn_sched_barrier(0);
+      decay += s_cs[b & 1][Q - 1];
+      add_block(b & 1, now);
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) stage(b + 1);
+      return more;
+    };
+    float B2[NW][32];
+    fetch_B(b0, B);
+    stage(b0);
+    for (int b = b0; block(b, B, B2) && block(b + 1, B2, B); b += 2) {}
+    float* s = left(part + 1);
+#pragma unroll
+    for (int w = 0; w < NW; w++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) s[(w * 16 + r) * 256 + tid] = S[w][r];
+    if (tid == 0) s[NW * 4096] = __builtin_amdgcn_exp2f((float)decay);
+    return;
+  }
+  fetch_C(b0); fetch_G(b0);
+  stage(b0);
+  for (int b = b0; b < b1; b++) {
     const int buf = b & 1, t0 = b * Q;
-    const bool more = b + 1 < nblk;
+    const bool more = b + 1 < b1;
     __syncthreads();      // the block's columns and sums stand; the shares of the block before have been read
-    fetch_B(b);
+    fetch_B(b, B);
     if (more) fetch_x(b + 1);
     __builtin_amdgcn_sched_barrier(0);      // (the phases stay apart: operands of a later one must not take registers early)
     f32x16 acc[2];
@@ -223,20 +301,7 @@ __global__ __launch_bounds__(256, NW == 1 ? 2 : 1) void ssd_block_kernel(StepMet
 #pragma unroll
       for (int r = 0; r < 16; r++) s_part[wv][32 * it + (r & 3) + 8 * (r >> 2) + 4 * half][l31] = acc[it][r];
     __builtin_amdgcn_sched_barrier(0);
-    // S_out
-    const float ge = __builtin_amdgcn_exp2f((float)s_cs[buf][Q - 1]);
-#pragma unroll
-    for (int w = 0; w < NW; w++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) S[w][r] *= ge;
-    if (n0 < a.N)
-#pragma unroll
-      for (int kk = 0; kk < 32; kk++) {
-        const int j = kk + 32 * half;
-        const float xs = s_x[buf][j][l31] * s_end[buf][j];
-#pragma unroll
-        for (int w = 0; w < NW; w++) S[w] = __builtin_amdgcn_mfma_f32_32x32x2f32(B[w][kk], xs, S[w], 0, 0, 0);
-      }
+    add_block(buf, B);
     __builtin_amdgcn_sched_barrier(0);
     if (more) stage(b + 1);
     __syncthreads();
@@ -247,6 +312,7 @@ __global__ __launch_bounds__(256, NW == 1 ? 2 : 1) void ssd_block_kernel(StepMet
         *(ones ? a.norm_out + (size_t)(start + t0 + t) * a.ldn + h : a.out + (size_t)(start + t0 + t) * a.ldo + h * a.E + e0 + l31) = fmaf(Dh, s_x[buf][t][l31], s_part[0][t][l31] + s_part[1][t][l31] + s_part[2][t][l31] + s_part[3][t][l31]);
     }
   }
+  if (b1 < nblk) return;
 #pragma unroll
   for (int w = 0; w < NW; w++)
 #pragma unroll
@@ -261,7 +327,7 @@ __global__ __launch_bounds__(256, NW == 1 ? 2 : 1) void ssd_block_kernel(StepMet
 // waves and portions of 1024 tokens gives every m_t from sums of the f alone (no difference of two long sums).  The maxima are kept in double: a thread takes the maximum
 // before its tokens from the composed maps and its neighbour's from its own steps, and in fp32 the two differed by a rounding, which is a factor on the whole memory.  The
 // maximum that the entry leaves is an fp32 number, so its last token's is rounded to that before its gates are made.  2048 tokens, 8 heads of 128 x 256: token by token 940 us a layer,
-// bound by each token's dependent step; 207 in blocks, a chain of 32 on 72 workgroups.  Grid: (entries, heads).
+// bound by each token's dependent step; 80 in blocks, their chain of 32 in seven portions.  Grid: (entries, heads).
 struct GateScanArgs {
   const float* proj; long long ldp; int i0, f0;      // the columns of the log gates
   float* mx; size_t mx_buf;                          // [2][slots][heads]

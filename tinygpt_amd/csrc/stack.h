@@ -194,7 +194,10 @@ void launch_stack_line(tgx_ctx* c, const tgx::StackGemmArgs& g, int epi, int nz,
 // stack_ssd.hip
 bool ssd_mfma_shapes_ok(int heads, int groups, int N, int E, long long ld);
 size_t ssd_gram_elems(int T, int S, int groups);
-void launch_ssd_mfma(tgx_ctx* c, const tgx::StepMeta& m, const tgx::SsdArgs& a, int S, int max_count);
+int ssd_portion(const tgx_ctx* c, int S, int heads, int N, int E, bool norm, int max_count);
+size_t ssd_portion_elems(int S, int heads, int N, int E, bool norm, int max_count, int portion);
+size_t ssd_portion_most(const tgx_ctx* c);
+void launch_ssd_mfma(tgx_ctx* c, const tgx::StepMeta& m, tgx::SsdArgs a, int S, int max_count);
 void launch_gate_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::GateScanArgs& a, int S);
 
 // stack_recblk.hip

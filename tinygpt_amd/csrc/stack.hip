@@ -151,6 +151,16 @@ bool ensure_scratch(tgx_ctx* c, E*& p, size_t& have, size_t need, size_t ask) {
   return true;
 }
 bool ensure_part(tgx_ctx* c, size_t need, size_t ask = 0) { StackModel* sm = c->stack; return ensure_scratch(c, sm->part, sm->part_elems, need, std::max(ask, sm->part_ask)); }
+// scratch of a blocked scalar-decay recurrence: its Gram rows, `more` numbers behind them and the states of its portions, for which there need not be room
+bool ensure_ssd(tgx_ctx* c, tgx::SsdArgs& a, int T, int S, int max_count, bool norm, size_t more = 0, size_t more_most = 0) {
+  StackModel* sm = c->stack;
+  const size_t need = ssd_gram_elems(T, S, a.groups) + more, most = ssd_gram_elems(sm->cap_tokens, sm->d.max_seqs, a.groups) + more_most + ssd_portion_most(c);
+  a.portion = ssd_portion(c, S, a.heads, a.N, a.E, norm, max_count);
+  if (a.portion && !ensure_part(c, need + ssd_portion_elems(S, a.heads, a.N, a.E, norm, max_count, a.portion), most)) a.portion = 0;
+  if (!a.portion && !ensure_part(c, need, most)) return false;
+  a.gram = sm->part; a.states = sm->part + need;
+  return true;
+}
 // (behind a norm's lines; the buffer does not grow while these stand in it: norm_terms asked for all that the step can come to need)
 bool ensure_terms(tgx_ctx* c, size_t need) {
   StackModel* sm = c->stack;
@@ -754,13 +764,14 @@ int run_mlstm(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, const float* h
   // portions: the recurrence with its maximum taken out is a scalar-decay recurrence and runs in blocks of 64 tokens (kernels/stack_ssd_mfma.h): from 64 tokens,
   // as the other families (a layer of 8 heads of 128 x 256, one prompt: 32 tokens 82 us by the scan and 86 in blocks, 64 tokens 115 and 107, 256 240 and 173, 1024 596 and 295)
   const size_t gram = ssd_gram_elems(T, S, H);
-  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && ensure_part(c, gram + (size_t)T * 4 * H, ssd_gram_elems(sm->cap_tokens, sm->d.max_seqs, H) + (size_t)sm->cap_tokens * 4 * H)) {
+  tgx::SsdArgs da{};
+  da.heads = H; da.groups = H; da.N = ld.dim; da.E = ld.vdim;
+  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && ensure_ssd(c, da, T, S, max_count, true, (size_t)T * 4 * H, (size_t)sm->cap_tokens * 4 * H)) {
     tgx::GateScanArgs ga{};
     ga.proj = sm->proj; ga.ldp = ldp; ga.i0 = 2 * qd + 2 * vd; ga.f0 = ga.i0 + H; ga.mx = w.mm; ga.mx_buf = (size_t)sm->d.max_seqs * H; ga.gates = sm->part + gram; ga.heads = H;
     launch_gate_scan(c, m, ga, S);
-    tgx::SsdArgs da{};
-    da.row = sm->proj; da.ld = ldp; da.x0 = 2 * qd; da.b0 = qd; da.c0 = 0; da.gates = ga.gates; da.ldgate = 3 * H; da.dt_col = 0; da.log_col = H; da.heads = H; da.groups = H; da.N = ld.dim; da.E = ld.vdim;
-    da.gram = sm->part; da.S = w.mS; da.out = sm->hs; da.ldo = vd; da.norm_S = w.mn; da.norm_buf = (size_t)sm->d.max_seqs * H * ld.dim; da.norm_out = ga.gates + (size_t)T * 3 * H; da.ldn = H;
+    da.row = sm->proj; da.ld = ldp; da.x0 = 2 * qd; da.b0 = qd; da.c0 = 0; da.gates = ga.gates; da.ldgate = 3 * H; da.dt_col = 0; da.log_col = H;
+    da.S = w.mS; da.out = sm->hs; da.ldo = vd; da.norm_S = w.mn; da.norm_buf = (size_t)sm->d.max_seqs * H * ld.dim; da.norm_out = ga.gates + (size_t)T * 3 * H; da.ldn = H;
     launch_ssd_mfma(c, m, da, S, max_count);
     oa.norm = da.norm_out; oa.ldnorm = H; oa.floor = ga.gates + 2 * H; oa.ldfloor = 3 * H; oa.scale = 1.0f / sqrtf((float)ld.dim);
   } else {
@@ -1781,9 +1792,10 @@ int run_ssm_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, 
   tgx::RecScanArgs ra{};
   ra.a = sm->rec_in + I + gn; ra.lda = ldr; ra.k = sm->rec_in + I; ra.ldk = ldr; ra.v = sm->rec_in; ra.ldv = ldr; ra.beta = sm->rec_in + C; ra.g = sm->rec_in + C + rH; ra.ldg = ldr;
   ra.skip = w.d_skip; ra.S = w.mS; ra.out = sm->hs; ra.ldo = I; ra.heads = rH; ra.kv_heads = ld.d_kv_heads; ra.dim = ld.d_dim; ra.vdim = ld.d_vdim;
-  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(rH, ld.d_kv_heads, ld.d_dim, ld.d_vdim, ldr) && ensure_part(c, ssd_gram_elems(T, S, ld.d_kv_heads), ssd_gram_elems(sm->cap_tokens, sm->d.max_seqs, ld.d_kv_heads))) {
-    tgx::SsdArgs da{};
-    da.row = sm->rec_in; da.ld = ldr; da.b0 = I; da.c0 = I + gn; da.gates = sm->rec_in; da.ldgate = ldr; da.dt_col = C; da.log_col = C + 2 * rH; da.heads = rH; da.groups = ld.d_kv_heads; da.N = ld.d_dim; da.E = ld.d_vdim; da.gram = sm->part; da.skip = w.d_skip; da.S = w.mS; da.out = sm->hs; da.ldo = I;
+  tgx::SsdArgs da{};
+  da.heads = rH; da.groups = ld.d_kv_heads; da.N = ld.d_dim; da.E = ld.d_vdim;
+  if (sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(rH, ld.d_kv_heads, ld.d_dim, ld.d_vdim, ldr) && ensure_ssd(c, da, T, S, max_count, false)) {
+    da.row = sm->rec_in; da.ld = ldr; da.b0 = I; da.c0 = I + gn; da.gates = sm->rec_in; da.ldgate = ldr; da.dt_col = C; da.log_col = C + 2 * rH; da.skip = w.d_skip; da.S = w.mS; da.out = sm->hs; da.ldo = I;
     launch_ssd_mfma(c, m, da, S, max_count);
   } else launch_rec_scan(c, m, ra, tgx::REC_SSD, S);
   tgx::PartNormArgs pa{};
@@ -2038,7 +2050,9 @@ int run_retention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int
   oa.hs = sm->hs; oa.ldh = vd; oa.gate = sm->proj + vd + 2 * qd; oa.ldg = ldp; oa.silu_gate = 1; oa.out = sm->o; oa.ldo = vd; oa.vdim = ld.vdim; oa.eps = sm->d.norm_eps;
   tgx::RecStepArgs st{};
   st.s = ra; st.g = oa; st.rot_dims = ld.rot_dims; st.cs = w.rot >= 0 ? sm->rot[(size_t)w.rot].cs : nullptr;
-  const bool blocks = sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && ensure_part(c, ssd_gram_elems(T, S, H), ssd_gram_elems(sm->cap_tokens, sm->d.max_seqs, H));
+  tgx::SsdArgs da{};
+  da.heads = H; da.groups = H; da.N = ld.dim; da.E = ld.vdim;
+  const bool blocks = sm->ssd_min > 0 && max_count >= sm->ssd_min && ssd_mfma_shapes_ok(H, H, ld.dim, ld.vdim, ldp) && ensure_ssd(c, da, T, S, max_count, false);
   if (blocks || !launch_rec_step(c, m, st, tgx::REC_SSD, S, max_count)) {      // (blocks of single tokens only where ssd.min asks for them)
     if (w.rot >= 0) {      // q and k turn in place (2 H heads side by side)
       tgx::GqaAppendArgs ap{};
@@ -2046,8 +2060,7 @@ int run_retention(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int
       TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::gqa_append_kernel<DT>, dim3(T), dim3(256), 0, c->stream, m, ap))
     }
     if (blocks) {
-      tgx::SsdArgs da{};
-      da.row = sm->proj; da.ld = ldp; da.b0 = vd; da.c0 = vd + qd; da.heads = H; da.groups = H; da.N = ld.dim; da.E = ld.vdim; da.gram = sm->part; da.fixed = w.decays; da.dt0 = kscale; da.S = w.mS; da.out = sm->hs; da.ldo = vd;
+      da.row = sm->proj; da.ld = ldp; da.b0 = vd; da.c0 = vd + qd; da.fixed = w.decays; da.dt0 = kscale; da.S = w.mS; da.out = sm->hs; da.ldo = vd;
       launch_ssd_mfma(c, m, da, S, max_count);
     } else launch_rec_scan(c, m, ra, tgx::REC_SSD, S);
     hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, H), dim3(64), 0, c->stream, oa);

@@ -7,16 +7,38 @@
 bool ssd_mfma_shapes_ok(int heads, int groups, int N, int E, long long ld) { return N % 4 == 0 && N <= 256 && (heads * E) % 4 == 0 && ld % 4 == 0 && ld < (1 << 21) && groups > 0; }
 size_t ssd_gram_elems(int T, int S, int groups) { return ((size_t)T / tgx::SSD_BLOCK + (size_t)S + 1) * groups * tgx::SSD_BLOCK * tgx::SSD_BLOCK; }
 
-void launch_ssd_mfma(tgx_ctx* c, const tgx::StepMeta& m, const tgx::SsdArgs& a, int S, int max_count) {
+namespace {
+int ssd_tiles(int E, bool norm) { return (E + 31) / 32 + (norm ? 1 : 0); }
+int ssd_state_tiles(int N) { return N <= 128 ? 1 : 2; }
+}  // namespace
+// Blocks of a portion (0: entries whole).  As many portions as the chip has room for beside the entries' heads (two workgroups a compute unit, one above 128 channels), of two blocks at least, from six blocks on.
+// A prompt of 8 heads of 128 x 256, whole and in two launches: four blocks 29.6 us and 29.4 with a launch more, eight 54 and 37, sixteen 105 and 54, 32 212 and 80.
+int ssd_portion(const tgx_ctx* c, int S, int heads, int N, int E, bool norm, int max_count) {
+  const long long room = (ssd_state_tiles(N) == 1 ? 2LL : 1LL) * c->num_cus, whole = (long long)S * heads * ssd_tiles(E, norm);
+  const int blocks = (max_count + tgx::SSD_BLOCK - 1) / tgx::SSD_BLOCK, P = blocks < 6 ? 1 : (int)std::min<long long>(room / whole, blocks / 2);
+  return P > 1 ? (blocks + P - 1) / P : 0;
+}
+size_t ssd_portion_elems(int S, int heads, int N, int E, bool norm, int max_count, int portion) {
+  const int blocks = (max_count + tgx::SSD_BLOCK - 1) / tgx::SSD_BLOCK;
+  return portion ? (size_t)S * ((blocks + portion - 1) / portion) * heads * ssd_tiles(E, norm) * tgx::ssd_state_elems(ssd_state_tiles(N)) : 0;
+}
+// the most that is: room for so many workgroups
+size_t ssd_portion_most(const tgx_ctx* c) { return 2 * (size_t)c->num_cus * tgx::ssd_state_elems(1); }
+
+void launch_ssd_mfma(tgx_ctx* c, const tgx::StepMeta& m, tgx::SsdArgs a, int S, int max_count) {
   if (!ssd_mfma_shapes_ok(a.heads, a.groups, a.N, a.E, a.ld) || a.b0 % 4 || a.c0 % 4) { c->launch_fault = "blocked state-space recurrence: sizes it does not take"; return; }
-  hipLaunchKernelGGL(tgx::ssd_gram_kernel<>, dim3((max_count + tgx::SSD_BLOCK - 1) / tgx::SSD_BLOCK, a.groups, S), dim3(256), 0, c->stream, m, a);
-  const dim3 grid(S, a.heads, (a.E + 31) / 32 + (a.norm_S ? 1 : 0));
-  auto go = [&](auto NORM) {
-    constexpr bool N = decltype(NORM)::value;
-    if (a.N <= 128) hipLaunchKernelGGL((tgx::ssd_block_kernel<1, N>), grid, dim3(256), 0, c->stream, m, a);
-    else hipLaunchKernelGGL((tgx::ssd_block_kernel<2, N>), grid, dim3(256), 0, c->stream, m, a);
+  const int blocks = (max_count + tgx::SSD_BLOCK - 1) / tgx::SSD_BLOCK;
+  hipLaunchKernelGGL(tgx::ssd_gram_kernel<>, dim3(blocks, a.groups, S), dim3(256), 0, c->stream, m, a);
+  a.portions = a.portion ? (blocks + a.portion - 1) / a.portion : 1;
+  const dim3 grid(a.heads, ssd_tiles(a.E, a.norm_S), S * a.portions);
+  auto go = [&](auto NW, auto NORM, auto MODE) { hipLaunchKernelGGL((tgx::ssd_block_kernel<decltype(NW)::value, decltype(NORM)::value, decltype(MODE)::value>), grid, dim3(256), 0, c->stream, m, a); };
+  auto mode = [&](auto NW, auto NORM) {
+    if (!a.portion) { go(NW, NORM, std::integral_constant<int, tgx::SSD_WHOLE>{}); return; }
+    go(NW, NORM, std::integral_constant<int, tgx::SSD_STATES>{});
+    go(NW, NORM, std::integral_constant<int, tgx::SSD_PORTIONS>{});
   };
-  if (a.norm_S) go(std::true_type{}); else go(std::false_type{});
+  auto norm = [&](auto NW) { if (a.norm_S) mode(NW, std::true_type{}); else mode(NW, std::false_type{}); };
+  if (ssd_state_tiles(a.N) == 1) norm(std::integral_constant<int, 1>{}); else norm(std::integral_constant<int, 2>{});
 }
 
 void launch_gate_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::GateScanArgs& a, int S) { hipLaunchKernelGGL(tgx::gate_scan_kernel<>, dim3(S, a.heads), dim3(256), 0, c->stream, m, a); }
