@@ -366,3 +366,22 @@ def test_scalar_decay_in_portions(design, sizes, dim, vdim):
         got[least] = np.concatenate(out)
         eng.close()
     assert np.abs(got[64] - got[0]).max() / np.abs(got[0]).max() < 1e-4
+
+
+# The scan's, the filter's, the attention's and the part norms' rows as terms that the product behind them reads, against the same step with fp32 rows and the other products (stack.line 0).
+# Both multiply weights of 16 bits by two 16-bit terms (2^-16 of an input, or 2^-22), layer by layer: 2^-12 of the largest logit holds what four layers make of it.
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("inner,rank,left,right", [(192, 160, 16, 16), (256, 168, 32, 16), (200, 160, 16, 12)])      # rows of whole lines, and (the last) none that are
+def test_rows_as_terms_of_the_product_behind(inner, rank, left, right, dtype):
+    import test_hip_nusovik as tn
+    mamba = tn.mamba(tn.ff(64), inner=inner, dt_rank=rank, state=16)
+    cfg = tn.config([mamba, tn.par(tn.ff(64), left=dict(heads=4, kv_heads=2, dim=left, mask={"size": 65}), right=dict(vdim=right))] * 2, width=320)
+    sizes = [3001, 1160]
+    got = []
+    for line in (1, 0):
+        eng, w = tn.engine(cfg, dtype, max_seqs=2, max_ctx=4096, budget_tokens=8192, options={"stack.line": line, "stack.conv_tiles": 1})
+        got.append(eng.step([("s%d" % i, tn.tokens(cfg, n, i), [0, 64, n // 2, n - 1]) for i, n in enumerate(sizes)]))
+        got[-1] = np.concatenate([got[-1], eng.step([("s%d" % i, tn.tokens(cfg, 1, i), [0]) for i in range(2)])])
+        eng.close()
+    assert np.abs(got[0] - got[1]).max() / np.abs(got[1]).max() < 2.0 ** -12
+    assert not (got[0] == got[1]).all()

@@ -13,6 +13,7 @@
 #pragma once
 #include "common.h"
 #include "stack_meta.h"
+#include "stack_terms.h"
 
 namespace tgx {
 
@@ -58,26 +59,10 @@ __device__ __forceinline__ void row_store(float* p, int k, int W, f32x4 v) {
 #pragma unroll
     for (int u = 0; u < 4; u++) { const int c = row_channel<false>(k, u); if (c < W) p[c] = v[u]; }
 }
-// The rows of a norm also as lines of two 16-bit terms, which the matrix-core products read (stack_line.h; row t at t * 2 W): what a launch of its own read and wrote again in front of
-// every product (2048 rows of 2048 channels 8.4 us and a launch each; here 1.2 us more).  W a multiple of 64, vectors of four.
-struct RowTerms { bf16_t* out; int half, one_term; };      // (half: fp16 terms; out nullptr: none)
+// the rows of a norm also as terms (stack_terms.h; 1.2 us more).  W a multiple of 64, vectors of four
 __device__ __forceinline__ void row_store_terms(const RowTerms& a, size_t t, int k, int W, f32x4 v) {
   const int c = row_channel<true>(k, 0);
-  if (c >= W) return;
-  unsigned int h[2], l[2];
-#pragma unroll
-  for (int i = 0; i < 2; i++) {
-    bf16_t hi[2], lo[2];
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-      if (a.half) split16<DT_F16>(v[2 * i + u], hi[u], lo[u]); else split16<DT_BF16>(v[2 * i + u], hi[u], lo[u]);
-    }
-    h[i] = (unsigned int)hi[0] | ((unsigned int)hi[1] << 16);
-    l[i] = a.one_term ? 0u : (unsigned int)lo[0] | ((unsigned int)lo[1] << 16);
-  }
-  bf16_t* line = a.out + t * 2 * W + (size_t)(c >> 5) * 64 + (c & 31);
-  *reinterpret_cast<uint2*>(line) = uint2{h[0], h[1]};
-  *reinterpret_cast<uint2*>(line + 32) = uint2{l[0], l[1]};
+  if (c < W) store_terms4(a, t, c, W, v);
 }
 // the sum over a workgroup of 256 with one barrier: every call of a kernel has its own four numbers of LDS
 __device__ __forceinline__ float block_sum_once(float v, float* own4) {

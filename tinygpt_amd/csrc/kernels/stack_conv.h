@@ -95,7 +95,12 @@ __global__ __launch_bounds__(256) void conv_silu_tiles_kernel(StepMeta m, ConvSi
   conv_taps<TAPS>(a.cw, c, w);
   conv_tile<TAPS>(m, a.proj + a.col0 + c, a.ldp, w, *reinterpret_cast<const f32x4*>(a.cb + c), a.state, a.state_buf, a.C, c, t0, n, f);
 #pragma unroll
-  for (int u = 0; u < CONV_TOK; u++) if (u < n) *reinterpret_cast<f32x4*>(a.out + (size_t)(t0 + u) * a.ldo + c) = silu4(f[u]);
+  for (int u = 0; u < CONV_TOK; u++) {
+    if (u >= n) break;
+    const f32x4 v = silu4(f[u]);
+    *reinterpret_cast<f32x4*>(a.out + (size_t)(t0 + u) * a.ldo + c) = v;
+    if (a.terms.out) store_terms4(a.terms, t0 + u, c, a.C, v);
+  }
 }
 
 // LPH: lanes of a q or k head (dim / 4).  Grid: (tokens / 32, C / 256 + 1 for the heads' gates)

@@ -16,6 +16,7 @@
 #pragma once
 #include "prefill.h"
 #include "stack_meta.h"
+#include "stack_terms.h"
 
 namespace tgx {
 
@@ -35,6 +36,7 @@ struct GqaMfmaArgs {
   const float* dist_tab; int dist_len;
   int gate_per_head;
   float out_scale;
+  RowTerms line;                       // undivided keys: the outputs as terms of rows of ldo channels, in place of out (stack_terms.h)
 };
 
 template <int DT, int ND, int NT, bool SPLIT>      // ND = dim / 64: 16-channel steps of a wave's share of the contraction; NT = ceil(vdim / 128): 32-column output tiles per wave
@@ -222,7 +224,8 @@ __global__ __launch_bounds__(256) void gqa_attn_mfma_kernel(StepMeta m, GqaMfmaA
         const size_t tok = (size_t)(start + gr / Gq), hc = (size_t)head(gr) * a.vdim + col;
         float v = s_l[ri] > 0.f ? acc[t][r] / s_l[ri] : 0.f;
         if (a.gate) v = v / (1.0f + expf(-a.gate[tok * a.ldg + (a.gate_per_head ? (size_t)head(gr) : hc)]));
-        a.out[tok * a.ldo + hc] = v * a.out_scale;
+        if (a.line.out) store_term(a.line, tok, (int)hc, (int)a.ldo, v * a.out_scale);
+        else a.out[tok * a.ldo + hc] = v * a.out_scale;
       }
     }
 }

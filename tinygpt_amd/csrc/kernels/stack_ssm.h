@@ -69,6 +69,7 @@ struct ConvSiluArgs {
   int C, taps, tile;
   int heads, dt_col;     // heads 0: no step sizes
   const float *dt_bias, *a_log;
+  RowTerms terms;        // conv_silu_tiles_kernel: the outputs also as terms of rows of C channels (stack_terms.h)
 };
 __device__ __forceinline__ float silu_f(float v) { return v / (1.0f + expf(-v)); }
 __device__ __forceinline__ float softplus_f(float v) { return v > 20.f ? v : log1pf(expf(v)); }
@@ -150,6 +151,7 @@ struct SelScanArgs {
   float* S;              // [slots][C][N]
   float* out; long long ldo;
   int C, N;
+  RowTerms terms;        // the outputs as terms of rows of C channels, in place of out (stack_terms.h)
 };
 template <int SPL, int LPC>
 __global__ __launch_bounds__(256) void selective_scan_kernel(StepMeta m, SelScanArgs a) {
@@ -172,6 +174,9 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(StepMeta m, SelScan
   }
   const float Dc = on ? a.D[c] : 0.f;
   float rdt[NX], rx[NX], rz[NX], rb[NB], rc[NB];
+  auto put = [&](int t, int cc, float v) {
+    if (a.terms.out) store_term(a.terms, start + t, cc, a.C, v); else a.out[(size_t)(start + t) * a.ldo + cc] = v;
+  };
   auto fetch = [&](int t0) {
     const int nb = min(TB, cnt - t0);
 #pragma unroll
@@ -198,7 +203,7 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(StepMeta m, SelScan
 #pragma unroll
       for (int u = 0; u < NX; u++) {
         const int i = tid + 256 * u, t = i / CPW, cc = i % CPW;
-        if (t < TB && c0 + cc < a.C) a.out[(size_t)(start + t0 - TB + t) * a.ldo + c0 + cc] = s_xz[t][cc].y;
+        if (t < TB && c0 + cc < a.C) put(t0 - TB + t, c0 + cc, s_xz[t][cc].y);
       }
       __syncthreads();
     }
@@ -260,14 +265,14 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(StepMeta m, SelScan
 #pragma unroll
   for (int u = 0; u < NX; u++) {
     const int i = tid + 256 * u, t = i / CPW, cc = i % CPW;
-    if (t < cnt - tl && c0 + cc < a.C) a.out[(size_t)(start + tl + t) * a.ldo + c0 + cc] = s_xz[t][cc].y;
+    if (t < cnt - tl && c0 + cc < a.C) put(tl + t, c0 + cc, s_xz[t][cc].y);
   }
 #pragma unroll
   for (int k = 0; k < SPL; k++) { const int n = l * SPL + k; if (on && n < a.N) Sg[n] = S[k]; }
 }
 
 // ---- u = y * silu(z) in `parts` equal parts of n channels; out = u / sqrt(mean over the part of u^2 + eps) * w * scale.  Grid: (tokens, parts).
-struct PartNormArgs { const float* y; long long ldy; const float* z; long long ldz; const float* w; float* out; long long ldo; int n; float eps, scale; };
+struct PartNormArgs { const float* y; long long ldy; const float* z; long long ldz; const float* w; float* out; long long ldo; int n; float eps, scale; RowTerms terms; int col0; };      // terms: in place of out, from column col0 of rows of ldo channels
 constexpr int PART_REG = 8;      // parts up to 256 * PART_REG channels stay in registers
 __global__ __launch_bounds__(256) void part_norm_gate_kernel(PartNormArgs a) {
   __shared__ float s4[4];
@@ -276,7 +281,7 @@ __global__ __launch_bounds__(256) void part_norm_gate_kernel(PartNormArgs a) {
   const float* __restrict__ y = a.y + t * a.ldy + c0;
   const float* __restrict__ z = a.z + t * a.ldz + c0;
   const float* __restrict__ w = a.w + c0;
-  float* __restrict__ out = a.out + t * a.ldo + c0;
+  auto put = [&](int c, float v) { if (a.terms.out) store_term(a.terms, t, a.col0 + c0 + c, (int)a.ldo, v); else a.out[t * a.ldo + c0 + c] = v; };
   float ss = 0.f;
   if (a.n <= 256 * PART_REG) {
     float u[PART_REG], g[PART_REG], wk[PART_REG];      // all loads first
@@ -290,13 +295,13 @@ __global__ __launch_bounds__(256) void part_norm_gate_kernel(PartNormArgs a) {
     ss = block_sum_256(ss, s4);
     const float r = a.scale / sqrtf(ss / (float)a.n + a.eps);
 #pragma unroll
-    for (int k = 0; k < PART_REG; k++) { const int c = threadIdx.x + 256 * k; if (c < a.n) out[c] = u[k] * r * wk[k]; }
+    for (int k = 0; k < PART_REG; k++) { const int c = threadIdx.x + 256 * k; if (c < a.n) put(c, u[k] * r * wk[k]); }
     return;
   }
   for (int c = threadIdx.x; c < a.n; c += 256) { const float u = y[c] * silu_f(z[c]); ss = fmaf(u, u, ss); }
   ss = block_sum_256(ss, s4);
   const float r = a.scale / sqrtf(ss / (float)a.n + a.eps);
-  for (int c = threadIdx.x; c < a.n; c += 256) out[c] = y[c] * silu_f(z[c]) * r * w[c];
+  for (int c = threadIdx.x; c < a.n; c += 256) put(c, y[c] * silu_f(z[c]) * r * w[c]);
 }
 
 }  // namespace tgx

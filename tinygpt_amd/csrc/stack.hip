@@ -232,6 +232,17 @@ tgx::RowTerms norm_terms(tgx_ctx* c, int T, int N, bool dual) {
   return t;
 }
 
+// where the kernel that makes the rows of a product writes them as terms in place of fp32 rows that a launch in front of the product would split (none: the product wants fp32 rows).
+// Eight Nusovik documents (10917 tokens of 2048 channels): seventeen splits of 55 us a step became five, the filter whose rows the scan reads too writes both (92 -> 126 us), the step
+// 27.7 -> 26.9 ms.
+tgx::RowTerms rows_as_terms(tgx_ctx* c, const tgx::StackGemmArgs& g) {
+  StackModel* sm = c->stack;
+  tgx::RowTerms t{};
+  if (!line_tile(c, g, tgx::SG_STORE, 1, c->dt) || !ensure_terms(c, 2 * (size_t)g.M * g.K)) return t;
+  t.out = sm->terms + (sm->in_terms ? sm->in_terms_elems : 0); t.half = c->dt == tgx::DT_F16; t.one_term = c->act16 ? 1 : 0;
+  return t;
+}
+
 // operands that the weight-streaming kernels' loads take: whole 8-element slices
 bool slices_ok(const tgx::StackGemmArgs& a) {
   return a.K % 8 == 0 && a.ldb % 8 == 0 && a.b_zstride % 8 == 0 && a.lda % 4 == 0 && a.a_zoff % 4 == 0 && (uintptr_t)a.A % 16 == 0 && (uintptr_t)a.B % 16 == 0 && (!a.B2 || (uintptr_t)a.B2 % 16 == 0);
@@ -627,6 +638,7 @@ struct GqaSpec {
   int maps = 1;                                                // score maps over the same values (heads and kv_heads count every map); with two, `out` takes the maps'
   float lambda = 0.f, diff_eps = 0.f, diff_scale = 0.f;        // normed difference (map_difference_kernel) and map_out their own outputs on the way there
   float* map_out = nullptr;
+  tgx::RowTerms line{}; bool* in_line = nullptr;               // where the outputs go as terms of rows of ldo channels, if the path taken can (*in_line: it did)
 };
 tgx::GqaAppendArgs append_args(const StackModel* sm, const GqaSpec& sp) {
   tgx::GqaAppendArgs ap{};
@@ -702,6 +714,7 @@ int run_gqa_core(tgx_ctx* c, const tgx::StepMeta& m, const GqaSpec& sp_, int T, 
       mg.gate_per_head = sp.gate_per_head; mg.out_scale = sp.out_scale;
       merge(mg);
     } else {
+      if (sp.in_line && sp.line.out) { ma.line = sp.line; *sp.in_line = true; }
       launch_gqa_mfma(c, m, ma, dim3(tiles, S * G), false);
       finish();
     }
@@ -1711,11 +1724,11 @@ void post_norm_add(tgx_ctx* c, const float* w, int T, const tgx::RowTerms& terms
   a.x = sm->x; a.y = sm->yd; a.w = w; a.W = sm->d.width; a.eps = sm->d.norm_eps; a.terms = terms;
   hipLaunchKernelGGL(tgx::post_norm_add_kernel, dim3(T), dim3(256), 0, c->stream, a);
 }
-void launch_conv_silu(tgx_ctx* c, const tgx::StepMeta& m, tgx::ConvSiluArgs a, int T) {
+bool launch_conv_silu(tgx_ctx* c, const tgx::StepMeta& m, tgx::ConvSiluArgs a, int T) {      // true: its rows stand as terms too, where `terms` asks for them
   const int cols = (a.C + 255) / 256 + (a.heads > 0 ? 1 : 0);
   if (conv_tiles(c, T, a.C, CONV_TILES_MIN) && fours(a.proj + a.col0, a.ldp) && fours(a.out, a.ldo) && fours(a.cw, 0) && fours(a.cb, 0) && fours(a.state, (long long)a.state_buf)) {
     const dim3 grid((T + tgx::CONV_WG_TOK - 1) / tgx::CONV_WG_TOK, cols);
-    if (two_to_four_taps(a.taps, [&](auto TAPS) { hipLaunchKernelGGL(tgx::conv_silu_tiles_kernel<decltype(TAPS)::value>, grid, dim3(256), 0, c->stream, m, a); })) return;
+    if (two_to_four_taps(a.taps, [&](auto TAPS) { hipLaunchKernelGGL(tgx::conv_silu_tiles_kernel<decltype(TAPS)::value>, grid, dim3(256), 0, c->stream, m, a); })) return a.terms.out != nullptr;
   }
   a.tile = (long long)T * cols >= 16LL * c->num_cus ? 8 : 1;      // tokens per workgroup: rows are kept in registers from token to token once the grid fills the chip
   const dim3 grid((T + a.tile - 1) / a.tile, cols);
@@ -1725,6 +1738,7 @@ void launch_conv_silu(tgx_ctx* c, const tgx::StepMeta& m, tgx::ConvSiluArgs a, i
     case 4: hipLaunchKernelGGL(tgx::conv_silu_kernel<4>, grid, dim3(256), 0, c->stream, m, a); break;
     default: hipLaunchKernelGGL(tgx::conv_silu_kernel<0>, grid, dim3(256), 0, c->stream, m, a); break;
   }
+  return false;
 }
 template <int SPL, int LPC>
 void launch_sel_scan_t(tgx_ctx* c, const tgx::StepMeta& m, const tgx::SelScanArgs& a, int S) {
@@ -1752,10 +1766,11 @@ void run_mamba1(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int S
   tgx::ConvSiluArgs ca{};
   ca.proj = sm->proj; ca.ldp = 2LL * I; ca.cw = w.conv_w; ca.cb = w.conv_b; ca.out = sm->rec_in; ca.ldo = I; ca.state = nb > 0 ? w.conv_state : nullptr;
   ca.state_buf = (size_t)sm->d.max_seqs * nb * I; ca.C = I; ca.taps = ld.conv_taps;
-  launch_conv_silu(c, m, ca, T);
   // [dt | B | C] = x . w_x^T, then the step sizes softplus(dt . w_dt^T + b), which take the place of the raw x columns
   g = tgx::StackGemmArgs{};
   g.A = sm->rec_in; g.lda = I; g.B = w.w_w1; g.ldb = I; g.C = sm->lora; g.ldc = ldq; g.M = T; g.N = R + 2 * N; g.K = I; g.scale = 1.f;
+  ca.terms = rows_as_terms(c, g);
+  if (launch_conv_silu(c, m, ca, T)) g.At = ca.terms.out;
   launch_gemm(c, g, tgx::SG_STORE, 1);
   g = tgx::StackGemmArgs{};
   g.A = sm->lora; g.lda = ldq; g.B = w.w_w2; g.ldb = R; g.C = sm->proj; g.ldc = 2LL * I; g.M = T; g.N = I; g.K = R; g.scale = 1.f; g.bias = w.w0; g.act = tgx::SG_ACT_SOFTPLUS;
@@ -1763,8 +1778,10 @@ void run_mamba1(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int S
   tgx::SelScanArgs sa{};
   sa.dt = sm->proj; sa.ldt = 2LL * I; sa.x = sm->rec_in; sa.ldx = I; sa.z = sm->proj + I; sa.ldz = 2LL * I; sa.bc = sm->lora + R; sa.ldbc = ldq; sa.ccol = N;
   sa.A2 = w.decay2; sa.D = w.d_skip; sa.S = w.mS; sa.out = sm->o; sa.ldo = I; sa.C = I; sa.N = N;
+  g = sublayer_product(c, sm->o, I, w.w_o, T);
+  sa.terms = rows_as_terms(c, g); g.At = sa.terms.out;
   launch_sel_scan(c, m, sa, S);
-  sublayer_out(c, sm->o, I, w.w_o, T);
+  launch_gemm(c, g, tgx::SG_STORE, 1);
 }
 
 int run_ssm_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int S, int max_keys, int max_count) {
@@ -1781,6 +1798,10 @@ int run_ssm_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, 
   sp.qk_eps = sm->d.norm_eps; sp.q_norm = w.q_norm; sp.k_norm = w.k_norm; sp.v_is_k = 1; sp.sinks = w.sink; sp.dist = w.dist; sp.dist_len = w.dist_len;
   sp.gate = sm->proj + r0 + I + C + rH; sp.ldg = ldp; sp.gate_per_head = 1; sp.scale = ld.scale; sp.mask_kind = ld.mask_kind; sp.mask_size = ld.mask_size;
   sp.out = sm->o; sp.ldo = ldo; sp.out_scale = ld.left_scale;
+  // both halves' outputs are the rows of one product: as terms where the left half's path can
+  tgx::StackGemmArgs go = sublayer_product(c, sm->o, ldo, w.w_o, T);
+  bool in_line = false;
+  sp.line = rows_as_terms(c, go); sp.in_line = &in_line;
   int rc = run_gqa_core(c, m, sp, T, S, max_keys, max_count);
   if (rc) return rc;
   // the right half: rec_in row = [x | B | C | dt | decay | log decay]
@@ -1800,8 +1821,9 @@ int run_ssm_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, 
   } else launch_rec_scan(c, m, ra, tgx::REC_SSD, S);
   tgx::PartNormArgs pa{};
   pa.y = sm->hs; pa.ldy = I; pa.z = sm->proj + r0; pa.ldz = ldp; pa.w = w.head_w; pa.out = sm->o + lvd; pa.ldo = ldo; pa.n = I / ld.part_norms; pa.eps = sm->d.norm_eps; pa.scale = ld.right_scale;
+  if (in_line) { pa.terms = sp.line; pa.col0 = lvd; go.At = sp.line.out; }
   hipLaunchKernelGGL(tgx::part_norm_gate_kernel, dim3(T, ld.part_norms), dim3(256), 0, c->stream, pa);
-  sublayer_out(c, sm->o, ldo, w.w_o, T);      // one product over both halves' outputs
+  launch_gemm(c, go, tgx::SG_STORE, 1);      // one product over both halves' outputs
   return TGX_OK;
 }
 
