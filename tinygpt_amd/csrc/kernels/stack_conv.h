@@ -3,7 +3,7 @@
 // What bounds them: their bytes, a row read and one written.  A token or a channel a thread, as those kernels have it for short portions, waits for a token's place in its entry and for its
 // rows at every turn.  Here a wave asks for the rows of eight tokens and the taps - 1 before them at once; the few tiles at an entry's ends take what is not among them from the slot's tails.
 // us: 2048 tokens of a delta rule's 4096 channels 89 -> 20 (67 MB), 10917 tokens of 4096 and 4608 channels 135 -> 88 and 146 -> 88 (358 and 402 MB; the silu's exponentials lie beside the bytes).
-// The sums are those kernels', term by term; a head's sum of squares runs over its lanes.
+// The sums are those kernels', term by term and in their order, a head's sum of squares too (head_squares): a model answers with the same bits whichever form its steps take.
 #pragma once
 #include "stack_rec.h"
 #include "stack_ssm.h"
@@ -103,6 +103,39 @@ __global__ __launch_bounds__(256) void conv_silu_tiles_kernel(StepMeta m, ConvSi
   }
 }
 
+__device__ __forceinline__ float lane_xor4(float v) {      // the lane 4 apart: row_shl:4 for the even banks of four lanes, row_shr:4 for the odd ones
+  const int b = __builtin_bit_cast(int, v);
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_amdgcn_update_dpp(0, b, 0x104, 0xf, 0x5, false), b, 0x114, 0xf, 0xa, false));
+}
+// the sum of a head's squares in the order of delta_prep_kernel, which has a channel a lane: over the channels 32 apart (the lower one's square is
+// added unrounded to the upper one's), 16, 8 and 4 apart, which are here lanes, 2 and 1 apart, which are a lane's components, and 64 apart.  Every lane of the head gets it.  (A sum in another order moves the
+// unit vectors in their last bits, which is enough to send a token with a near tie to another expert some layers on.)
+template <int LPH>
+__device__ __forceinline__ float head_squares(f32x4 v) {
+#pragma clang fp contract(off)
+  const bool upper = (threadIdx.x & 8) != 0;
+  float s[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const float x = v[k];
+    float y;
+    if constexpr (LPH >= 16) {
+      const float other = dpp_mov<0x128, 0xf>(x);          // row_ror:8: the lane 8 apart
+      const float lo = upper ? other : x, hi = upper ? x : other;
+      y = fmaf(lo, lo, hi * hi);
+    } else y = x * x;
+    y += lane_xor4(y);
+    y += dpp_mov<0x4E, 0xf>(y);
+    y += dpp_mov<0xB1, 0xf>(y);
+    s[k] = y;
+  }
+  float ss = (s[0] + s[2]) + (s[1] + s[3]);
+  if constexpr (LPH == 32) {
+    const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(ss), __float_as_uint(ss), false, false));
+    ss = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+  return ss;
+}
 // LPH: lanes of a q or k head (dim / 4).  Grid: (tokens / 32, C / 256 + 1 for the heads' gates)
 template <int TAPS, int LPH>
 __global__ __launch_bounds__(256) void delta_prep_tiles_kernel(StepMeta m, DeltaPrepArgs a) {
@@ -123,14 +156,16 @@ __global__ __launch_bounds__(256) void delta_prep_tiles_kernel(StepMeta m, Delta
   f32x4 w[TAPS], f[CONV_TOK];
   conv_taps<TAPS>(a.cw, c, w);
   conv_tile<TAPS>(m, a.proj + a.col0 + c, a.ldp, w, f32x4{0.f, 0.f, 0.f, 0.f}, a.state, a.state_buf, C, c, t0, n, f);
-  const bool qk = c < 2 * GD;
+  const bool qk = c < 2 * GD, any_qk = (int)blockIdx.y * CONV_WG_CH < 2 * GD;
   const float scale = c < GD ? a.q_scale : 1.0f;
 #pragma unroll
   for (int u = 0; u < CONV_TOK; u++) {
     if (u >= n) break;
     f32x4 v = silu4(f[u]);
-    const float ss = row_group_sum<LPH>(fmaf(v[0], v[0], v[1] * v[1]) + fmaf(v[2], v[2], v[3] * v[3]));      // (of a value channel: not used)
-    if (qk) v *= scale / sqrtf(ss + a.unit_eps);
+    if (any_qk) {
+      const float ss = head_squares<LPH>(v);      // (of value channels: not used)
+      if (qk) v *= scale / sqrtf(ss + a.unit_eps);
+    }
     *reinterpret_cast<f32x4*>(a.out + (size_t)(t0 + u) * a.ldo + c) = v;
   }
 }
