@@ -207,3 +207,30 @@ def test_a_prompt_allocates_its_scratch_once(dtype):
         eng.step([("a", ids[:n], [n - 1])], ["a"])
         assert eng.model.get_option("stack.ws_grown") == grown
     eng.close()
+
+
+def test_scratch_of_blocked_recurrences_only_where_they_run():
+    """a context whose recurrences run token by token asks for no more scratch with 1024 slots (their blocks: 148 MB) than with two"""
+    import ctypes
+    from tinygpt_amd.ffi import product_backend
+
+    def memory_left():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert product_backend().lib.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    cfg = dict(width=320, vocab=101, layers=[dict(type="wkv", mixer=dict(heads=5, dim=64), mlp=dict(ff=1088))] * 2)
+    w = {k: np.asarray(v, np.float32) for k, v in vo.random_tensors(cfg, 3, decay_rank=64).items()}
+    ids = np.random.default_rng(1).integers(0, 101, 4161)
+    took = []
+    for slots in (2, 1024):
+        d = wkv_model(320, 1088, "bf16", 4161)
+        d.max_seqs = slots
+        eng = SlotEngine(desc=d, tensors=w)
+        eng.model.set_option("rec.min", 0)
+        free = memory_left()
+        eng.step([("a", ids, [4160])], ["a"])
+        assert eng.model.get_option("stack.ws_grown") == 2      # (the products' terms and the hidden rows')
+        took.append(free - memory_left())
+        eng.close()
+    assert took[1] - took[0] < 32 << 20, took

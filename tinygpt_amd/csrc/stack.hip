@@ -167,10 +167,11 @@ bool ensure_terms(tgx_ctx* c, size_t need) {
   if (sm->in_terms) return sm->in_terms_elems + need <= sm->terms_elems;
   return ensure_scratch(c, sm->terms, sm->terms_elems, need, 2 * (size_t)sm->cap_tokens * (sm->joint || sm->post ? sm->terms_most + sm->d.width : sm->terms_cols));
 }
-// (a feed-forward's hidden values, and before them a blocked recurrence's blocks: one buffer for the layer's two halves)
-bool ensure_terms2(tgx_ctx* c, size_t need) {
+// (a feed-forward's hidden values, and before them a blocked recurrence's blocks: one buffer for the layer's two halves, which grows to what the blocks can come to need, rec_ask, once
+// a step takes them)
+bool ensure_terms2(tgx_ctx* c, size_t need, size_t rec_ask = 0) {
   StackModel* sm = c->stack;
-  return ensure_scratch(c, sm->terms2, sm->terms2_elems, need, std::max(2 * (size_t)sm->cap_tokens * sm->terms2_cols, 2 * ((size_t)sm->cap_tokens / tgx::REC_BLOCK + (size_t)sm->d.max_seqs) * sm->rec_block_most));
+  return ensure_scratch(c, sm->terms2, sm->terms2_elems, need, std::max(2 * (size_t)sm->cap_tokens * sm->terms2_cols, rec_ask));
 }
 // what those buffers can come to hold: the sums of the divided keys of any step (tiles of up to 32 rows on twice as many workgroups as there are compute units, a value or
 // latent row and two numbers each; or a token's outputs, heads in a row), and a token's widest product input and hidden row
@@ -1043,11 +1044,12 @@ constexpr int REC_WKV_BLOCK_MIN = 128, REC_DELTA_BLOCK_MIN = 160, REC_WKV_BLOCK_
 void launch_recurrence(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs& a, int kind, int T, int S, int max_count) {
   StackModel* sm = c->stack;
   const bool wkv = kind == tgx::REC_WKV;
-  const long long wgs = (long long)S * a.heads * ((a.vdim + 15) / 16);
+  const long long wgs = (long long)S * a.heads * ((a.vdim + 15) / 16), most_wgs = (long long)(wkv ? REC_WKV_BLOCK_WGS : REC_DELTA_BLOCK_WGS) * c->num_cus;
   const bool pays = sm->rec_min >= 0 ? sm->rec_min > 0 && max_count >= sm->rec_min
-                                     : sm->line && max_count >= (wkv ? REC_WKV_BLOCK_MIN : REC_DELTA_BLOCK_MIN) && wgs <= (long long)(wkv ? REC_WKV_BLOCK_WGS : REC_DELTA_BLOCK_WGS) * c->num_cus &&
+                                     : sm->line && max_count >= (wkv ? REC_WKV_BLOCK_MIN : REC_DELTA_BLOCK_MIN) && wgs <= most_wgs &&
                                            (wgs <= c->num_cus || T >= REC_BLOCK_FULL_MEAN * S);
-  if (pays && rec_vec(a) && a.dim <= tgx::REC_BLOCK_MAX_DIM && a.vdim <= tgx::REC_BLOCK_MAX_VDIM && ensure_terms2(c, 2 * rec_block_elems((size_t)T / tgx::REC_BLOCK + (size_t)S, a.heads, a.dim, a.vdim, !wkv)))
+  const size_t blocks = (size_t)T / tgx::REC_BLOCK + (size_t)S, most = (size_t)sm->cap_tokens / tgx::REC_BLOCK + (size_t)std::min<long long>(sm->d.max_seqs, most_wgs * S / wgs);      // (as many entries as the rule takes)
+  if (pays && rec_vec(a) && a.dim <= tgx::REC_BLOCK_MAX_DIM && a.vdim <= tgx::REC_BLOCK_MAX_VDIM && ensure_terms2(c, 2 * rec_block_elems(blocks, a.heads, a.dim, a.vdim, !wkv), 2 * most * sm->rec_block_most))
     launch_rec_blocks(c, m, a, kind, S, max_count, reinterpret_cast<float*>(sm->terms2));
   else launch_rec_scan(c, m, a, kind, S);
 }
