@@ -973,9 +973,16 @@ struct JointLayer {
 
 // Convolutions in tiles of eight tokens of four channels a lane (kernels/stack_conv.h) from so many (token, channel) numbers on, where rows and channels are whole fours; shorter steps keep
 // a channel a thread, whose workgroups then run all at once and whose waves have an eighth to do.  us, a channel a thread / in tiles: delta rule's inputs of 2048 channels 128 tokens 5.2 /
-// 8.8, 300 9.9 / 8.8, 1600 36 / 13, 2048 tokens of 4096 89 / 20; filters of 2048 channels 300 tokens 4.8 / 8.0, 2000 15.5 / 12.0, 10917 tokens of 4096 135 / 88
-constexpr long long DELTA_TILES_MIN = 1 << 19, CONV_TILES_MIN = 1 << 21;
-bool conv_tiles(const tgx_ctx* c, int T, int C, long long min) { const int o = c->stack->conv_tiles; return C % 4 == 0 && (o >= 0 ? o != 0 : (long long)T * C >= min); }
+// 8.8, 256 9.1 / 9.6, 512 14.3 / 10.0, 1600 36 / 13, 2048 tokens of 4096 89 / 21; filters of 2048 channels 300 tokens 4.8 / 8.0, 1024 10.4 / 10.2, 2000 15.5 / 12.0, 10917 tokens of 4096
+// 135 / 88.  A tile that an entry begins or ends in walks its tokens one by one, so entries shorter than two tiles on average take them from two and four times as much on: entries
+// of 2, 4 and 8 tokens, delta rule 256 tokens 9.2 / 12.4, 11.5 and 10.8, 512 tokens 15.2 / 14.2, 12.3 and 11.5, filters 1024 tokens 12.2 / 15.4, 10.9 / 14.1 and 10.4 / 12.0, 2048 tokens of
+// entries of 4 16.7 / 16.9, 4096 of 8 29.4 / 28.8.
+constexpr long long DELTA_TILES_MIN = 5 << 17, CONV_TILES_MIN = 1 << 21;
+constexpr int DELTA_TILES_SHORT = 2, CONV_TILES_SHORT = 4;
+bool conv_tiles(const tgx_ctx* c, int T, int S, int C, long long min, int short_entries) {
+  const int o = c->stack->conv_tiles;
+  return C % 4 == 0 && (o >= 0 ? o != 0 : (long long)T * C >= (T < 2 * tgx::CONV_TOK * S ? min * short_entries : min));
+}
 bool fours(const void* p, long long ld) { return (uintptr_t)p % 16 == 0 && ld % 4 == 0; }
 template <class F>
 bool two_to_four_taps(int taps, F f) {
@@ -986,9 +993,9 @@ bool two_to_four_taps(int taps, F f) {
     default: return false;
   }
 }
-void launch_delta_prep(tgx_ctx* c, const tgx::StepMeta& m, const tgx::DeltaPrepArgs& a, int T) {
+void launch_delta_prep(tgx_ctx* c, const tgx::StepMeta& m, const tgx::DeltaPrepArgs& a, int T, int S) {
   const int C = 2 * a.kv_heads * a.dim + a.heads * a.vdim;
-  if (conv_tiles(c, T, C, DELTA_TILES_MIN) && (a.dim == 32 || a.dim == 64 || a.dim == 128) && fours(a.proj + a.col0, a.ldp) && fours(a.out, a.ldo) && fours(a.cw, 0) && fours(a.state, (long long)a.state_buf)) {
+  if (conv_tiles(c, T, S, C, DELTA_TILES_MIN, DELTA_TILES_SHORT) && (a.dim == 32 || a.dim == 64 || a.dim == 128) && fours(a.proj + a.col0, a.ldp) && fours(a.out, a.ldo) && fours(a.cw, 0) && fours(a.state, (long long)a.state_buf)) {
     const dim3 grid((T + tgx::CONV_WG_TOK - 1) / tgx::CONV_WG_TOK, (C + tgx::CONV_WG_CH - 1) / tgx::CONV_WG_CH + 1);
     if (two_to_four_taps(a.taps, [&](auto TAPS) {
           constexpr int N = decltype(TAPS)::value;
@@ -1190,7 +1197,7 @@ int run_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer&
     if (rc) return rc;
     left_out();      // (unmerged layers' outputs are added here, before the right half takes their place)
     if (!launch_rec_step(c, m, st, tgx::REC_DELTA, S, max_count)) {
-      launch_delta_prep(c, m, dp, T);
+      launch_delta_prep(c, m, dp, T, S);
       launch_recurrence(c, m, ra, tgx::REC_DELTA, T, S, max_count);
       hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, rH), dim3(64), 0, c->stream, oa);
     }
@@ -1726,9 +1733,9 @@ void post_norm_add(tgx_ctx* c, const float* w, int T, const tgx::RowTerms& terms
   a.x = sm->x; a.y = sm->yd; a.w = w; a.W = sm->d.width; a.eps = sm->d.norm_eps; a.terms = terms;
   hipLaunchKernelGGL(tgx::post_norm_add_kernel, dim3(T), dim3(256), 0, c->stream, a);
 }
-bool launch_conv_silu(tgx_ctx* c, const tgx::StepMeta& m, tgx::ConvSiluArgs a, int T) {      // true: its rows stand as terms too, where `terms` asks for them
+bool launch_conv_silu(tgx_ctx* c, const tgx::StepMeta& m, tgx::ConvSiluArgs a, int T, int S) {      // true: its rows stand as terms too, where `terms` asks for them
   const int cols = (a.C + 255) / 256 + (a.heads > 0 ? 1 : 0);
-  if (conv_tiles(c, T, a.C, CONV_TILES_MIN) && fours(a.proj + a.col0, a.ldp) && fours(a.out, a.ldo) && fours(a.cw, 0) && fours(a.cb, 0) && fours(a.state, (long long)a.state_buf)) {
+  if (conv_tiles(c, T, S, a.C, CONV_TILES_MIN, CONV_TILES_SHORT) && fours(a.proj + a.col0, a.ldp) && fours(a.out, a.ldo) && fours(a.cw, 0) && fours(a.cb, 0) && fours(a.state, (long long)a.state_buf)) {
     const dim3 grid((T + tgx::CONV_WG_TOK - 1) / tgx::CONV_WG_TOK, cols);
     if (two_to_four_taps(a.taps, [&](auto TAPS) { hipLaunchKernelGGL(tgx::conv_silu_tiles_kernel<decltype(TAPS)::value>, grid, dim3(256), 0, c->stream, m, a); })) return a.terms.out != nullptr;
   }
@@ -1772,7 +1779,7 @@ void run_mamba1(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, int S
   g = tgx::StackGemmArgs{};
   g.A = sm->rec_in; g.lda = I; g.B = w.w_w1; g.ldb = I; g.C = sm->lora; g.ldc = ldq; g.M = T; g.N = R + 2 * N; g.K = I; g.scale = 1.f;
   ca.terms = rows_as_terms(c, g);
-  if (launch_conv_silu(c, m, ca, T)) g.At = ca.terms.out;
+  if (launch_conv_silu(c, m, ca, T, S)) g.At = ca.terms.out;
   launch_gemm(c, g, tgx::SG_STORE, 1);
   g = tgx::StackGemmArgs{};
   g.A = sm->lora; g.lda = ldq; g.B = w.w_w2; g.ldb = R; g.C = sm->proj; g.ldc = 2LL * I; g.M = T; g.N = I; g.K = R; g.scale = 1.f; g.bias = w.w0; g.act = tgx::SG_ACT_SOFTPLUS;
@@ -1811,7 +1818,7 @@ int run_ssm_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T, 
   tgx::ConvSiluArgs ca{};
   ca.proj = sm->proj; ca.ldp = ldp; ca.col0 = r0 + I; ca.cw = w.conv_w; ca.cb = w.conv_b; ca.out = sm->rec_in; ca.ldo = ldr; ca.state = nb > 0 ? w.conv_state : nullptr;
   ca.state_buf = (size_t)sm->d.max_seqs * nb * C; ca.C = C; ca.taps = ld.conv_taps; ca.heads = rH; ca.dt_col = r0 + I + C; ca.dt_bias = w.dt_bias; ca.a_log = w.a_log;
-  launch_conv_silu(c, m, ca, T);
+  launch_conv_silu(c, m, ca, T, S);
   tgx::RecScanArgs ra{};
   ra.a = sm->rec_in + I + gn; ra.lda = ldr; ra.k = sm->rec_in + I; ra.ldk = ldr; ra.v = sm->rec_in; ra.ldv = ldr; ra.beta = sm->rec_in + C; ra.g = sm->rec_in + C + rH; ra.ldg = ldr;
   ra.skip = w.d_skip; ra.S = w.mS; ra.out = sm->hs; ra.ldo = I; ra.heads = rH; ra.kv_heads = ld.d_kv_heads; ra.dim = ld.d_dim; ra.vdim = ld.d_vdim;
@@ -2135,7 +2142,7 @@ void run_channel_delta(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, int T
   tgx::RecStepArgs st{};
   st.s = ra; st.p = dp; st.prep = 1; st.g = oa;
   if (!launch_rec_step(c, m, st, tgx::REC_CDELTA, S, max_count)) {
-    launch_delta_prep(c, m, dp, T);
+    launch_delta_prep(c, m, dp, T, S);
     launch_recurrence(c, m, ra, tgx::REC_CDELTA, T, S, max_count);
     hipLaunchKernelGGL(tgx::head_norm_gate_kernel, dim3(T, ld.heads), dim3(64), 0, c->stream, oa);
   }
