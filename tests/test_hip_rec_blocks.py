@@ -9,6 +9,7 @@ import test_hip_vitudra as tv
 
 pytestmark = pytest.mark.gpu
 HEADS = [(4, 5), (12, 16), (64, 17), (68, 64), (128, 33)]      # key and value channels
+WIDE = [(128, 144), (128, 256), (64, 208)]                      # more columns than the preparation has threads: a second pass over them
 
 
 def model(kind, dim, vdim, over=None, **kw):
@@ -37,8 +38,7 @@ def by_portions(eng, rid, toks, sizes):
     return np.concatenate(got)
 
 
-@pytest.mark.parametrize("dim,vdim", HEADS)
-@pytest.mark.parametrize("kind", ["wkv", "delta", "cdelta"])
+@pytest.mark.parametrize("kind,dim,vdim", [(k, *h) for k in ("wkv", "delta", "cdelta") for h in HEADS + (WIDE if k != "wkv" else [])])
 def test_blocks_equal_the_oracle_and_the_scan(kind, dim, vdim):
     """one portion over a few blocks, and the same tokens in portions that end in, on and behind a block's edge (a state that goes on, blocks of one token, tails of a block)"""
     eng, want_of, cfg = model(kind, dim, vdim)
@@ -68,6 +68,41 @@ def test_requests_of_unequal_length_in_one_step(kind):
         want = want_of(s)
         close(first[at:at + n], want[:n], "first %d" % n)
         close(second[40 * i:40 * i + 40], want[n:], "second %d" % n)
+        at += n
+    eng.close()
+
+
+@pytest.mark.parametrize("kind,dim,vdim", [("wkv", 132, 132), ("delta", 132, 16), ("delta", 64, 260), ("cdelta", 132, 16), ("cdelta", 64, 260), ("delta", 6, 16)])
+def test_heads_beyond_the_blocks_take_the_scan(kind, dim, vdim):
+    eng, want_of, cfg = model(kind, dim, vdim)
+    toks = tk.tokens(cfg, 70, seed=5)
+    got = []
+    for least in (0, 1):
+        eng.model.set_option("rec.min", least)
+        got.append(by_portions(eng, "r%d" % least, toks, [70]))
+    close(got[1], want_of(toks))
+    assert np.array_equal(got[0], got[1])
+    eng.close()
+
+
+@pytest.mark.parametrize("kind,heads,dim,vdim", [("wkv", 17, 64, 64), ("wkv", 9, 128, 128), ("delta", 16, 64, 72), ("delta", 16, 128, 72), ("cdelta", 16, 64, 72), ("cdelta", 16, 128, 72)])
+def test_more_workgroups_than_compute_units(kind, heads, dim, vdim):
+    """four requests of one to ten blocks, odd and even counts, whose heads and columns are 272 to 320 workgroups, then all of them a second time from the states that they left"""
+    if kind == "cdelta":
+        cfg = tk.config([tk.cd(dim=dim, vdim=vdim, heads=heads, kv_heads=heads // 2)])
+        eng, w = tk.engine(cfg, "fp32", 3)
+        want_of = tk.want_of
+    else:
+        cfg = tv.config([tv.wkv(heads=heads, dim=dim) if kind == "wkv" else tv.par(right=dict(dim=dim, vdim=vdim, heads=heads, kv_heads=heads // 2))])
+        eng, w = tv.engine(cfg, "fp32", 3)
+        want_of = tv.want_of
+    eng.model.set_option("rec.min", 1)
+    sizes = [257, 64, 33, 320]
+    seqs = [tk.tokens(cfg, 2 * n, seed=n) for n in sizes]
+    halves = [eng.step([("r%d" % i, s[k * n:(k + 1) * n], list(range(n))) for i, (s, n) in enumerate(zip(seqs, sizes))]) for k in (0, 1)]
+    at = 0
+    for s, n in zip(seqs, sizes):
+        close(np.concatenate([h[at:at + n] for h in halves]), want_of(cfg, w, s), "%d" % n)
         at += n
     eng.close()
 

@@ -368,6 +368,26 @@ def test_scalar_decay_in_portions(design, sizes, dim, vdim):
     assert np.abs(got[64] - got[0]).max() / np.abs(got[0]).max() < 1e-4
 
 
+@pytest.mark.parametrize("slots", [64, 65])
+def test_order_of_many_entries(slots):
+    """blocks take up to 64 entries longest first and more as they stand: entries of equal and unequal length, every request's outputs and the state it leaves, against the scan"""
+    import test_hip_keronex as tk
+    cfg = tk.config([tk.ret(heads=2, dim=16, vdim=16, decay=[0.9, 0.99], rot=None)], width=64)
+    got = {}
+    for least in (1, 0):
+        eng, w = tk.engine(cfg, seed=3, max_seqs=slots, max_ctx=256, budget_tokens=256 * slots)
+        eng.model.set_option("ssd.min", least)
+        out = []
+        for step in range(2):
+            sizes = [[5, 70, 5, 64, 129, 1, 70][(i + step) % 7] for i in range(slots)]
+            out.append(eng.step([("s%d" % i, tk.tokens(cfg, n, 100 * step + i), [0, n // 2, n - 1]) for i, n in enumerate(sizes)]))
+        out.append(eng.step([("s%d" % i, tk.tokens(cfg, 1, i), [0]) for i in range(slots)]))
+        got[least] = np.concatenate(out)
+        eng.close()
+    assert np.abs(got[1] - got[0]).max() / np.abs(got[0]).max() < 1e-4
+    assert not np.array_equal(got[1], got[0])      # (both forms ran)
+
+
 # The scan's, the filter's, the attention's and the part norms' rows as terms that the product behind them reads, against the same step with fp32 rows and the other products (stack.line 0).
 # Both multiply weights of 16 bits by two 16-bit terms (2^-16 of an input, or 2^-22), layer by layer: 2^-12 of the largest logit holds what four layers make of it.
 @pytest.mark.parametrize("dtype", ["bf16", "fp16"])
