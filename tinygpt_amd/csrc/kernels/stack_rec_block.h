@@ -12,9 +12,10 @@
 // the entry's first token; a block past the entry's end is padded by tokens with q = k = v = beta = 0 and w = 1, which change nothing.
 //
 // What bounds it: the token by token scan is a chain of one dependent read-update step a token, of one wave's instructions (0.13 to 0.17 us each); here the chain has a 32nd of the steps, of
-// 1.8 us (delta) and 0.85 us (wkv).  A step's 44 to 68 KB of operands are as long in a compute unit's memory pipeline (1.3 us without the matrix instructions) as its matrix
-// instructions beside them (1.5 us without the loads).  Blocks of 32: longer ones have as many bytes and products a token and twice the pairs.  2048 tokens, us, scan -> preparation +
-// blocks: delta rule of 16 heads of 128 x 128 340 -> 43 + 116, with a decay a channel (8 heads) 345 -> 26 + 111, wkv of 32 heads of 64 x 64 257 -> 43 + 55.
+// 1.7 us (delta rules of up to 128 key channels; of 64 1.1) and 1.1 us (wkv; 0.75).  A block's operands are 68 KB a workgroup (40 KB) and 52 KB (32 KB), as long in a compute unit's memory
+// pipeline (delta, 128 channels: 1.3 us without the matrix instructions) as its matrix instructions beside them (1.5 us without the loads).  Blocks of 32: longer ones have as many bytes
+// and products a token and twice the pairs.  2048 tokens, us, scan -> preparation + blocks: delta rule of 16 heads of 128 x 128 337 -> 48 + 109, with a decay a channel (8 heads) 353 -> 30 + 106,
+// wkv of 32 heads of 64 x 64 251 -> 45 + 48.
 #pragma once
 #include <type_traits>
 
@@ -254,7 +255,12 @@ __global__ __launch_bounds__(256, KIND == REC_WKV ? 3 : 2) void rec_block_prep_k
 // 4 (l / 16) + r, column l % 16.  That is at the same time a B operand whose contraction slots are those rows, so W S and Q S need no transposition, and the same holds for u, whose
 // rows are tokens.  The four waves' shares of W S (and, a block later, of the outputs) meet in LDS; two buffers each, one barrier a block.  A block's operands are asked for a block
 // ahead, straight into registers: no wave reads another's.  Grid: (entries, heads, E / 16).
-template <int KIND, int NT, int DEPTH>
+// DEPTH: blocks whose operands are in registers or on their way.  Two, so that a compute unit has room for two workgroups; three for wkv heads of more than 64 channels, whose block has
+// the fewest matrix instructions for its bytes.  2048 tokens, two / three, us: wkv 64 x 64 48 / 54, 128 x 128 85 / 72, delta rules 128 x 128 109 / 112, eight entries of 300 tokens and 16
+// heads 60 / 84.
+template <int KIND, int NT>
+constexpr int rec_block_depth() { return KIND == REC_WKV && NT == 2 ? 3 : 2; }
+template <int KIND, int NT, int DEPTH = rec_block_depth<KIND, NT>()>
 __global__ __launch_bounds__(256, DEPTH > 2 ? 1 : 2) void rec_block_kernel(StepMeta m, RecScanArgs a, const float* scratch) {
   constexpr int Q = REC_BLOCK;
   constexpr bool SOLVE = KIND != REC_WKV;

@@ -13,8 +13,7 @@ void launch_rec_blocks(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArg
     constexpr int KIND = decltype(K)::value, NT = decltype(D)::value;
     hipLaunchKernelGGL((tgx::rec_block_prep_kernel<KIND, 64 * NT>), dim3(nblk, a.heads, S), dim3(256), 0, c->stream, m, a, scratch);
     const dim3 grid(S, a.heads, (a.vdim + 15) / 16);
-    if ((long long)grid.x * grid.y * grid.z <= c->num_cus) hipLaunchKernelGGL((tgx::rec_block_kernel<KIND, NT, 3>), grid, dim3(256), 0, c->stream, m, a, scratch);
-    else hipLaunchKernelGGL((tgx::rec_block_kernel<KIND, NT, 2>), grid, dim3(256), 0, c->stream, m, a, scratch);
+    hipLaunchKernelGGL((tgx::rec_block_kernel<KIND, NT>), grid, dim3(256), 0, c->stream, m, a, scratch);
   };
   auto dims = [&](auto K) { if (a.dim <= 64) go(K, std::integral_constant<int, 1>{}); else go(K, std::integral_constant<int, 2>{}); };
   if (kind == tgx::REC_WKV) dims(std::integral_constant<int, tgx::REC_WKV>{});
