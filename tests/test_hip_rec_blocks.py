@@ -107,6 +107,28 @@ def test_more_workgroups_than_compute_units(kind, heads, dim, vdim):
     eng.close()
 
 
+@pytest.mark.parametrize("kind,heads,dim,sizes,blocks", [
+    ("wkv", 16, 32, [96], False), ("wkv", 16, 32, [512], True), ("wkv", 16, 32, [130] * 8, False), ("wkv", 64, 32, [300] * 4, False), ("wkv", 8, 128, [300] * 2, True),
+    ("delta", 16, 32, [512], True), ("delta", 32, 32, [300] * 8, False), ("delta", 16, 64, [192] * 8, False), ("delta", 4, 64, [300] * 4, True),
+    ("cdelta", 16, 32, [200] * 16, False), ("cdelta", 8, 128, [512], True), ("cdelta", 8, 128, [200] * 16, False), ("cdelta", 8, 128, [700] + [3] * 7, True)])
+def test_the_form_follows_the_step(kind, heads, dim, sizes, blocks):
+    """steps of which one form takes at least a tenth less than the other: by themselves they take that one (its bits)"""
+    kw = dict(max_seqs=16, max_ctx=1024, budget_tokens=8192)
+    if kind == "cdelta":
+        cfg = tk.config([tk.cd(dim=dim, vdim=dim, heads=heads, kv_heads=heads)])
+        eng, _ = tk.engine(cfg, "fp32", 3, **kw)
+    else:
+        cfg = tv.config([tv.wkv(heads=heads, dim=dim) if kind == "wkv" else tv.par(right=dict(dim=dim, vdim=dim, heads=heads, kv_heads=heads // 2))])
+        eng, _ = tv.engine(cfg, "fp32", 3, **kw)
+    got = {}
+    for least in (-1, 0, 1):
+        eng.model.set_option("rec.min", least)
+        got[least] = eng.step([(i, tk.tokens(cfg, n, i), [n // 2, n - 1]) for i, n in enumerate(sizes)], range(len(sizes)))
+    eng.close()
+    assert not np.array_equal(got[0], got[1])
+    assert np.array_equal(got[-1], got[1 if blocks else 0])
+
+
 @pytest.mark.parametrize("strength", [1.5, 3.0, 6.0])      # decays of 1e-2, 2e-9 (a block's product underflows) and zero a token
 @pytest.mark.parametrize("kind", ["wkv", "delta", "cdelta"])
 def test_strong_decays(kind, strength):

@@ -1011,16 +1011,22 @@ void launch_delta_prep(tgx_ctx* c, const tgx::StepMeta& m, const tgx::DeltaPrepA
 bool rec_vec(const tgx::RecScanArgs& a) {
   return a.dim % 4 == 0 && a.lda % 4 == 0 && a.ldk % 4 == 0 && (uintptr_t)a.a % 16 == 0 && (uintptr_t)a.k % 16 == 0 && (!a.w || (a.ldw % 4 == 0 && (uintptr_t)a.w % 16 == 0));
 }
+// sixteen row groups per column while their workgroups, of sixteen columns, leave a compute unit with two at most: one prompt of 16 heads of 128 (kernels/stack_rec.h), a few
+// requests; thirty-two, of four rows, while there is a compute unit for each of theirs (one prompt of 16 heads of 128 x 128: 340 us against sixteen's 400 for 2048 tokens; a SIMD
+// with two of their waves would issue more than with one of sixteen groups'); a full chip issues fewer instructions with eight
+struct RecScanPlan { int rg, rows, cols; };      // row groups, rows per lane, workgroups of columns
+RecScanPlan rec_scan_plan(const tgx_ctx* c, const tgx::RecScanArgs& a, int S) {
+  auto cols = [&](int rg) { return (a.vdim + tgx::rec_cols(rg) - 1) / tgx::rec_cols(rg); };
+  const bool wide = rec_vec(a) && a.dim <= 256 && (long long)S * a.heads * cols(16) <= 2LL * c->num_cus;
+  const bool widest = wide && a.dim > 64 && a.dim <= 128 && (long long)S * a.heads * cols(32) <= c->num_cus;
+  const int rg = widest ? 32 : wide ? 16 : 8, dper = (a.dim + rg - 1) / rg;
+  return {rg, dper <= 4 ? 4 : dper <= 8 ? 8 : dper <= 16 ? 16 : 32, cols(rg)};
+}
 void launch_rec_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs& a, int kind, int S) {
   const bool vec = rec_vec(a);
-  // sixteen row groups per column while their workgroups, of sixteen columns, leave a compute unit with two at most: one prompt of 16 heads of 128 (kernels/stack_rec.h), a few
-  // requests; thirty-two, of four rows, while there is a compute unit for each of theirs (one prompt of 16 heads of 128 x 128: 340 us against sixteen's 400 for 2048 tokens; a SIMD
-  // with two of their waves would issue more than with one of sixteen groups'); a full chip issues fewer instructions with eight
-  auto cols = [&](int rg) { return (a.vdim + tgx::rec_cols(rg) - 1) / tgx::rec_cols(rg); };
-  const bool wide = vec && a.dim <= 256 && (long long)S * a.heads * cols(16) <= 2LL * c->num_cus;
-  const bool widest = wide && a.dim > 64 && a.dim <= 128 && (long long)S * a.heads * cols(32) <= c->num_cus;
-  const int rg = widest ? 32 : wide ? 16 : 8, dper = (a.dim + rg - 1) / rg;      // rows per lane
-  const dim3 grid(S, a.heads, cols(rg));
+  const RecScanPlan plan = rec_scan_plan(c, a, S);
+  const bool wide = plan.rg >= 16, widest = plan.rg == 32;
+  const dim3 grid(S, a.heads, plan.cols);
   auto go = [&](auto K) {
     constexpr int KIND = decltype(K)::value;
     auto rows = [&](auto D) {
@@ -1030,9 +1036,9 @@ void launch_rec_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs&
       if (vec) hipLaunchKernelGGL((tgx::rec_scan_kernel<DPER, KIND, 8, true>), grid, dim3(256), 0, c->stream, m, a);
       else hipLaunchKernelGGL((tgx::rec_scan_kernel<DPER, KIND, 8, false>), grid, dim3(256), 0, c->stream, m, a);
     };
-    if (dper <= 4) rows(std::integral_constant<int, 4>{});
-    else if (dper <= 8) rows(std::integral_constant<int, 8>{});
-    else if (dper <= 16) rows(std::integral_constant<int, 16>{});
+    if (plan.rows == 4) rows(std::integral_constant<int, 4>{});
+    else if (plan.rows == 8) rows(std::integral_constant<int, 8>{});
+    else if (plan.rows == 16) rows(std::integral_constant<int, 16>{});
     else rows(std::integral_constant<int, 32>{});
   };
   if (kind == tgx::REC_WKV) go(std::integral_constant<int, tgx::REC_WKV>{});
@@ -1041,20 +1047,36 @@ void launch_rec_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs&
   else go(std::integral_constant<int, tgx::REC_DELTA>{});
 }
 
-// A recurrence over portions: in blocks of 32 tokens on the matrix cores (kernels/stack_rec_block.h; their scratch is the hidden values', which come after) or token by token.  The blocks
-// shorten the chain of a long portion, but move two to three times the scan's bytes, so they are for portions of which the chain is what bounds them: long ones, while their workgroups
-// (16 value channels each) are few to a compute unit.  us of a layer, blocks / scan.  wkv (heads of 64): one prompt of 96 tokens 16 / 15, 160 20 / 23, 2048 102 / 258; 2 workgroups a compute
-// unit 66 / 80 and 39 / 42, 4 133 / 118 and 70 / 62.  Delta rules (heads of 128 x 128): 96 tokens 25 / 20, 160 27 / 29, 2048 159 / 340; with a decay a channel 26 / 20, 28 / 31; 4 a
-// compute unit 95 / 96, 177 / 189 and 98 / 107, 8 209 / 181 and 222 / 201.  More workgroups than compute units are bound by all requests' tokens: 4 a compute unit, 120 tokens a
-// request 57 / 55, 250 98 / 107.  Option stack.line 0, which brings the older forms of prompts' products back, brings the scan back as well unless rec.min says otherwise.
-constexpr int REC_WKV_BLOCK_MIN = 128, REC_DELTA_BLOCK_MIN = 160, REC_WKV_BLOCK_WGS = 2, REC_DELTA_BLOCK_WGS = 4, REC_BLOCK_FULL_MEAN = 192;
+// A recurrence over portions: in blocks of 32 tokens on the matrix cores (kernels/stack_rec_block.h; their scratch is the hidden values', which come after) or token by token, by what
+// either takes of this step, in us.  The line lies where it does because the two are bound by different things, and no one size tells them apart:
+//   token by token  the longest entry's chain, of a wave's instructions a token, which grow with the rows of a lane; or the rows of all entries that a compute unit has to issue
+//   blocks          their preparation, 12 to 19 us however short the step is and then so much for every block and head of a compute unit, whatever the head's size; the longest entry's
+//                   chain of blocks, or the blocks that a compute unit has from all of them; and a launch more
+// Measured on 17 shapes of 4 to 64 heads, 32 to 128 key and 32 to 256 value channels, each from one entry of 64 to 2048 tokens to sixteen of 200 (255 points), the two sums are within a tenth of
+// most kernels' times, and the form taken is at worst 1.05 times the other.  us, token by token / blocks: wkv 32 heads of 64 x 64 one entry of 96 tokens 14.6 / 17.9, 160 22.1 / 20.4,
+// 2048 251 / 93, four of 300 46.7 / 45.8, eight of 300 67 / 79; 64 heads of 32 x 32 four of 300 43 / 62; 16 of 128 x 128 eight of 300 113 / 86.  Delta rules of 16 heads of 128 x 128 one of 160
+// 30.9 / 31.2, 2048 338 / 157, eight of 300 107 / 121; 16 of 64 x 64 2048 276 / 109, eight of 300 55 / 69; 32 of 32 x 32 eight of 300 51 / 105; a decay a channel, 8 of 128 x 128, 2048 353 / 136,
+// eight of 300 79 / 74.  Option stack.line 0, which brings the older forms of prompts' products back, brings the scan back as well unless rec.min says otherwise.
+double rec_scan_us(const tgx_ctx* c, const tgx::RecScanArgs& a, bool wkv, int T, int S, int max_count) {
+  const RecScanPlan p = rec_scan_plan(c, a, S);
+  const double issued = (double)p.rows * S * a.heads * p.cols / c->num_cus;
+  const double chain = 0.075 + 0.013 * p.rows + (wkv ? 0.0 : 0.015) + (p.rg == 32 ? 0.02 : 0.0), full = wkv ? 0.065 + 0.01 * issued : 0.11 + 0.0081 * issued;
+  return 3.0 + std::max(max_count * chain, full * T / S);
+}
+double rec_blocks_us(const tgx_ctx* c, const tgx::RecScanArgs& a, bool wkv, int T, int S, int max_count) {
+  struct Cost { double least, some, block, step, step_full; };
+  const Cost k = wkv ? (a.dim <= 64 ? Cost{12.3, 9.5, 3.9, 0.74, 0.72} : Cost{14.5, 10.0, 6.8, 1.12, 1.04})
+                     : (a.dim <= 64 ? Cost{17.0, 10.5, 7.4, 1.08, 0.95} : Cost{19.0, 13.5, 9.1, 1.68, 1.46});
+  const double per_cu = (T / (double)tgx::REC_BLOCK + 0.5 * S) * a.heads / c->num_cus;      // (an entry's last block is half full on average)
+  return 4.0 + std::max(k.least, k.some + k.block * per_cu) + std::max(k.step * ((max_count + tgx::REC_BLOCK - 1) / tgx::REC_BLOCK), k.step_full * per_cu * ((a.vdim + 15) / 16));
+}
+constexpr int REC_BLOCK_WGS = 4;      // workgroups of the blocks a compute unit has at most (what their scratch is sized for; eight were never faster)
 void launch_recurrence(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs& a, int kind, int T, int S, int max_count) {
   StackModel* sm = c->stack;
   const bool wkv = kind == tgx::REC_WKV;
-  const long long wgs = (long long)S * a.heads * ((a.vdim + 15) / 16), most_wgs = (long long)(wkv ? REC_WKV_BLOCK_WGS : REC_DELTA_BLOCK_WGS) * c->num_cus;
+  const long long wgs = (long long)S * a.heads * ((a.vdim + 15) / 16), most_wgs = (long long)REC_BLOCK_WGS * c->num_cus;
   const bool pays = sm->rec_min >= 0 ? sm->rec_min > 0 && max_count >= sm->rec_min
-                                     : sm->line && max_count >= (wkv ? REC_WKV_BLOCK_MIN : REC_DELTA_BLOCK_MIN) && wgs <= most_wgs &&
-                                           (wgs <= c->num_cus || T >= REC_BLOCK_FULL_MEAN * S);
+                                     : sm->line && wgs <= most_wgs && rec_blocks_us(c, a, wkv, T, S, max_count) < rec_scan_us(c, a, wkv, T, S, max_count);
   const size_t blocks = (size_t)T / tgx::REC_BLOCK + (size_t)S, most = (size_t)sm->cap_tokens / tgx::REC_BLOCK + (size_t)std::min<long long>(sm->d.max_seqs, most_wgs * S / wgs);      // (as many entries as the rule takes)
   if (pays && rec_vec(a) && a.dim <= tgx::REC_BLOCK_MAX_DIM && a.vdim <= tgx::REC_BLOCK_MAX_VDIM && ensure_terms2(c, 2 * rec_block_elems(blocks, a.heads, a.dim, a.vdim, !wkv), 2 * most * sm->rec_block_most))
     launch_rec_blocks(c, m, a, kind, S, max_count, reinterpret_cast<float*>(sm->terms2));
