@@ -368,11 +368,26 @@ def test_scalar_decay_in_portions(design, sizes, dim, vdim):
     assert np.abs(got[64] - got[0]).max() / np.abs(got[0]).max() < 1e-4
 
 
+@pytest.mark.parametrize("heads,vdim,sizes", [(8, 256, [400] * 4), (8, 320, [500, 70]), (8, 320, [448, 70]), (40, 128, [500]), (40, 128, [448])])      # room for two portions, and for three or four
+def test_portions_only_where_they_pay(heads, vdim, sizes):
+    """entries whose portions would be too few, and as many as are enough, against the recurrence token by token (fp32 both)"""
+    import test_hip_keronex as tk
+    cfg = tk.config([tk.ret(heads=heads, dim=128, vdim=vdim, decay=[0.9, 0.99] * (heads // 2), rot=None)], width=64)
+    got = {}
+    for least in (64, 0):
+        eng, w = tk.engine(cfg, seed=3, max_seqs=len(sizes), max_ctx=2048, budget_tokens=4096)
+        eng.model.set_option("ssd.min", least)
+        out = [eng.step([("s%d" % i, tk.tokens(cfg, n, 10 * step + i), [0, n // 2, n - 1]) for i, n in enumerate(sizes)]) for step in range(2)]
+        got[least] = np.concatenate(out)
+        eng.close()
+    assert np.abs(got[64] - got[0]).max() / np.abs(got[0]).max() < 1e-4
+
+
 @pytest.mark.parametrize("slots", [64, 65])
 def test_order_of_many_entries(slots):
-    """blocks take up to 64 entries longest first and more as they stand: entries of equal and unequal length, every request's outputs and the state it leaves, against the scan"""
+    """blocks that more than fill the chip (576 workgroups) take up to 64 entries longest first and more as they stand: entries of equal and unequal length, every request's outputs and the state it leaves, against the scan"""
     import test_hip_keronex as tk
-    cfg = tk.config([tk.ret(heads=2, dim=16, vdim=16, decay=[0.9, 0.99], rot=None)], width=64)
+    cfg = tk.config([tk.ret(heads=9, dim=16, vdim=16, decay=[0.9, 0.99, 0.8] * 3, rot=None)], width=64)
     got = {}
     for least in (1, 0):
         eng, w = tk.engine(cfg, seed=3, max_seqs=slots, max_ctx=256, budget_tokens=256 * slots)

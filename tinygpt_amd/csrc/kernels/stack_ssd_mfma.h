@@ -28,6 +28,7 @@ struct SsdArgs {
   float* norm_S; size_t norm_buf;      // a second state N_t = g_t N_(t-1) + dt_t B_t, the sum that a matrix memory divides by: [2][slots][heads][N], norm_buf between the two (nullptr: none)
   float* norm_out; long long ldn;      // N_t . C_t: [T][heads]
   int portion, portions;               // blocks of a portion (portions > 1: the longest entry's; an entry may have fewer)
+  int ranked;                          // SSD_WHOLE: entries longest first
   float* states;                       // [entries][portions][heads][tiles][ssd_state_elems]: what the portions before leave (SSD_STATES)
 };
 // the first block of an entry in `gram`: entries never share a block
@@ -73,7 +74,7 @@ __global__ __launch_bounds__(256) void ssd_gram_kernel(StepMeta m, SsdArgs a) {
 // NW: 32-row tiles of the state per wave (4 NW 32 >= N).  Wave w owns the state rows n of its tiles and 32 columns, in the accumulator layout: register r of a lane is
 // row (r & 3) + 8 (r >> 2) + 4 (lane / 32), column lane % 32.  Register r of the two half-waves is at the same time a B operand whose two contraction slots are those
 // two rows, so S^T C needs no transposition: its A operand takes C's channels in that order.  A wave contributes its rows' share of S^T C and the share of sixteen
-// keys j of the block's own product; the four waves' shares are added up in LDS.  Grid: (heads, E / 32, entries portions).
+// keys j of the block's own product; the four waves' shares are added up in LDS.  Grid: (heads, E / 32, portions entries).
 // Operands travel straight from memory to registers (every wave reads its own state rows only): B of a block is asked for at the block's start and used at its end,
 // C and the Gram rows of the next block replace the present ones as soon as these are used up, so nothing is held twice.  Rows past the
 // entry's end are clamped to its last one (what is read there twice meets dt = 0 or is not stored).
@@ -81,8 +82,9 @@ __global__ __launch_bounds__(256) void ssd_gram_kernel(StepMeta m, SsdArgs a) {
 // Entries and heads that leave the chip idle: a chain of blocks, 6.6 us each on 72 workgroups (2048 tokens, 8 heads of 128 x 256).  So an entry's blocks are cut into portions, which two
 // launches take at once: SSD_STATES the state that every portion but the last adds to a state of zero (the first: leaves behind the entry's own), and how much it decays; SSD_PORTIONS
 // every portion from its state, which is the first's and those after it in order: 27 us and 53 in seven portions where the chain took 212.
-// Entries that fill the chip are taken longest first, heads beside each other, so that no long one is left for the end: eight documents of up to 2048 tokens, 64 heads of 128 x 64,
-// 649 us a launch with the entries beside each other, 436 now.
+// All entries' first portions come before their second ones, so that whole portions are dealt evenly and the short last ones behind them.
+// Entries that more than fill the chip are taken longest first, heads beside each other, so that no long one is left for the end: eight documents of up to 2048 tokens, 64 heads of 128 x 64,
+// 649 us a launch with the entries beside each other, 436 now.  (Where all run at once there is nothing to order, and finding the ranks is 1 us: sixteen entries of 200 tokens 27 and 28.)
 enum { SSD_WHOLE = 0, SSD_STATES = 1, SSD_PORTIONS = 2 };
 constexpr size_t ssd_state_elems(int NW) { return (size_t)NW * 16 * 256 + 4; }      // a workgroup's accumulators as it holds them, and the portion's decay
 // the entry of rank r by its tokens, longest first (the entry r itself where there are more than 64)
@@ -101,8 +103,8 @@ __global__ __launch_bounds__(256, NW == 1 ? 2 : 1) void ssd_block_kernel(StepMet
   __shared__ double s_cs[2][Q];        // base-2 logarithms, summed from the block's start
   __shared__ float s_dt[2][Q], s_end[2][Q];      // dt_j, exp(cs_64 - cs_j) dt_j
   __shared__ float s_part[4][Q][33];
-  const int P = MODE == SSD_WHOLE ? 1 : a.portions, part = MODE == SSD_WHOLE ? 0 : blockIdx.z % P, tile = blockIdx.y, tiles = gridDim.y;
-  const int e = entry_by_length(m, gridDim.z / P, blockIdx.z / P), h = blockIdx.x, e0 = tile * 32, tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), half = lane >> 5, l31 = lane & 31;
+  const int P = MODE == SSD_WHOLE ? 1 : a.portions, entries = gridDim.z / P, part = MODE == SSD_WHOLE ? 0 : blockIdx.z / entries, tile = blockIdx.y, tiles = gridDim.y;
+  const int e = MODE == SSD_WHOLE ? (a.ranked ? entry_by_length(m, entries, blockIdx.z) : blockIdx.z) : blockIdx.z - part * entries, h = blockIdx.x, e0 = tile * 32, tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), half = lane >> 5, l31 = lane & 31;
   const int start = m.ent_start[e], cnt = m.ent_count[e], slot = m.ent_row[e], grp = h / (a.heads / a.groups);
   const int nblk = (cnt + Q - 1) / Q, b0 = MODE == SSD_WHOLE ? 0 : part * a.portion, b1 = MODE == SSD_WHOLE ? nblk : min(nblk, b0 + a.portion);
   if (MODE == SSD_STATES ? b1 >= nblk : b0 >= nblk) return;      // (the states of the last portion are nobody's start)
