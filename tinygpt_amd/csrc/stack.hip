@@ -449,9 +449,13 @@ int ensure_ws(tgx_ctx* c, int T) {
   return TGX_OK;
 }
 
-// latents into the pool, and the queries into latent space (g, batched over the heads): in one launch in steps of few tokens
+// latents into the pool, and the queries into latent space (g, batched over the heads): in one launch in steps of few tokens.  From three tokens on a workgroup is a few waves, which are
+// slower at turning the rotated parts of many heads than the append's own launch, and has to find a workgroup a token; us, append + products / together, rotated parts of 64: 4 heads of 448
+// 5.6 + 4.8 / 9.0, 16 heads 7.8 + 4.8 / 16.7, 32 heads 10.5 + 4.8 / 25.0; sixteen tokens of 4 heads of 128 (eight workgroups) 4.5 + 4.8 / 10.0, of 16 heads 6.2 + 4.8 / 23.0
+constexpr int LATENT_IN_ROT_MAX = 640;      // rotated elements of a token (its key's part and every head's): ten a thread of one wave
 void latent_in(tgx_ctx* c, const tgx::StepMeta& m, const tgx::LatentAppendArgs& la, tgx::StackGemmArgs g, int T, int H) {
-  if (c->stack->gemv && T <= 16 && slices_ok(g)) {
+  const bool together = T <= GEMV_ROWS_MAX || la.rot_dim <= 0 || ((H + 1) * la.rot_dim <= LATENT_IN_ROT_MAX && T <= (g.N + 15) / 16);
+  if (c->stack->gemv && T <= 16 && together && slices_ok(g)) {
     g.terms = c->act16 ? 1 : 2;
     if (T <= GEMV_ROWS_MAX) {
       const bool ksplit = gemv_ksplit(c, g, H);
