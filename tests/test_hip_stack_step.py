@@ -308,6 +308,22 @@ def test_rotated_latents_beside_their_queries(slots, kv_rank, dim, rot_dim):
         assert np.abs(got[i] - want).max() / np.abs(want).max() < 1e-4, (slots, i)
 
 
+@pytest.mark.parametrize("slots,heads,kv_rank,rot_dim,vdim", [(3, 9, 64, 64, 8), (3, 10, 64, 64, 8), (4, 4, 64, 64, 8), (5, 4, 64, 64, 8), (16, 8, 64, 0, 256), (16, 8, 64, 0, 264)])
+def test_latent_steps_of_many_heads_and_tokens(slots, heads, kv_rank, rot_dim, vdim):
+    """both sides of where a latent layer's append and queries (rotated parts of 640 elements, four workgroups) and its merge and values (1024 workgroups) share a launch, against the oracle"""
+    import test_hip_zaluvik as tz
+    cfg = tz.config([tz.lat(tz.dense(), heads=heads, dim=16, rot_dim=rot_dim, vdim=vdim, kv_rank=kv_rank, mask=None) for _ in range(2)], loop=None)
+    eng, w = tz.engine(cfg, "fp32", 2, max_seqs=slots, max_ctx=384, budget_tokens=384 * slots)
+    eng.model.set_option("attn.split_min", 32)
+    toks = [tz.tokens(cfg, 134, i) for i in range(slots)]
+    for i, s in enumerate(toks): eng.step([(i, s[:130], [])])
+    got = np.stack([eng.step([(i, s[130 + j:131 + j], [0]) for i, s in enumerate(toks)]) for j in range(4)], 1)
+    eng.close()
+    for i in {0, slots // 2, slots - 1}:
+        want = tz.want_of(cfg, w, toks[i])
+        assert np.abs(got[i] - want[130:]).max() / np.abs(want).max() < 1e-4, (slots, i)
+
+
 @pytest.mark.parametrize("dtype", ["fp32", "bf16"])
 @pytest.mark.parametrize("kv_heads,dim,vdim,size", [(1, 8, 8, None), (2, 24, 40, 128), (4, 128, 512, 160), (4, 64, 16, 128)])
 def test_sigmoid_attention_appends_in_its_step(kv_heads, dim, vdim, size, dtype):

@@ -477,9 +477,12 @@ void latent_in(tgx_ctx* c, const tgx::StepMeta& m, const tgx::LatentAppendArgs& 
   launch_gemm(c, g, tgx::SG_STORE, H);
 }
 // the values of a latent attention from the records of its divided keys: merge and product in one launch in steps of few tokens (kernels/stack_latent.h), else the merge alone (false: the
-// product is still to come)
+// product is still to come).  Every workgroup of a head merges its records again, so up to four workgroups a compute unit: twelve records of rank 512, us, merge + product / together: 512
+// workgroups 6.5 + 4.2 / 7.4, 1024 6.7 + 4.7 / 11.4 (and a launch less), 2048 7.2 + 5.3 / 20.8, 4096 6.7 + 6.0 / 32.7; of rank 128 1024 4.7 + 4.8 / 5.0, 4096 4.8 + 4.8 / 13.0
+constexpr int LATENT_VALUES_WGS = 4;
 bool latent_values(tgx_ctx* c, const tgx::LatentAttnArgs& aa, tgx::StackGemmArgs g, int T, int H) {
-  if (c->stack->gemv && !c->act16 && T <= 16 && g.K % 64 == 0 && g.K <= tgx::LATV_MAX_RANK && slices_ok(g)) {
+  const long long wgs = (long long)T * H * ((g.N + tgx::LATV_COLS - 1) / tgx::LATV_COLS);
+  if (c->stack->gemv && !c->act16 && T <= 16 && wgs <= (long long)LATENT_VALUES_WGS * c->num_cus && g.K % 64 == 0 && g.K <= tgx::LATV_MAX_RANK && slices_ok(g)) {
     const dim3 grid((g.N + tgx::LATV_COLS - 1) / tgx::LATV_COLS, H, T);
     TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::latent_values_kernel<DT>, grid, dim3(256), 0, c->stream, aa, g))
     return true;
