@@ -473,8 +473,9 @@ __global__ __launch_bounds__(256) void stack_gemv_kernel(const StackGemmArgs a) 
 // 360 -> 283 us.
 struct StackGemvGroup { StackGemmArgs p0, p1, up; int z0, blocks0, blocks1; };      // blocks0: per member of the batch
 // NORM: the rows are the stream in front of the layer's norm: 1 for the feed-forward, 2 for the mixer's first product as well.  NW: waves of a workgroup; with the norm eight up to
-// GEMV_GROUP_WIDE channels, whose weights are all on their way before the rows have been read (1024 channels, 24 MB: 6.9 us, four waves 7.7, without the norm 6.9 + 2.3), four beyond (2048
-// channels, 92 MB: 22.2, eight waves 23.9, without 20.0 + 3.6).
+// GEMV_GROUP_WIDE channels, whose weights are all on their way before the rows have been read, four beyond.  One row, the group of a wkv and of an attention layer, eight / four waves, us: 512
+// channels 9.2 / 9.4, 1024 11.3 / 12.2, 1280 16.8 / 17.7, 1536 20.6 / 19.7, 2048 31 / 25, 3072 34.6 both; two rows are within 6 % of each other at every width.  With the
+// norms in launches of their own 1024 10.9 + 5.2, 1536 20.4 + 5.2, 2048 26.5 + 5.1.
 constexpr int GEMV_GROUP_WIDE = 1024;
 template <int DT, int MR, int NORM, int NW>
 __global__ __launch_bounds__(64 * NW) void stack_gemv_group_kernel(const StackGemvGroup g) {

@@ -14,8 +14,8 @@
 // What bounds it: the token by token scan is a chain of one dependent read-update step a token, of one wave's instructions (0.13 to 0.17 us each); here the chain has a 32nd of the steps, of
 // 1.7 us (delta rules of up to 128 key channels; of 64 1.1) and 1.1 us (wkv; 0.75).  A block's operands are 68 KB a workgroup (40 KB) and 52 KB (32 KB), as long in a compute unit's memory
 // pipeline (delta, 128 channels: 1.3 us without the matrix instructions) as its matrix instructions beside them (1.5 us without the loads).  Blocks of 32: longer ones have as many bytes
-// and products a token and twice the pairs.  2048 tokens, us, scan -> preparation + blocks: delta rule of 16 heads of 128 x 128 337 -> 48 + 109, with a decay a channel (8 heads) 353 -> 30 + 106,
-// wkv of 32 heads of 64 x 64 251 -> 45 + 48.
+// and products a token and twice the pairs.  2048 tokens, us, scan -> preparation + blocks: delta rule of 16 heads of 128 x 128 338 -> 48 + 109 (in a model's pass, its inputs not in the cache, 51 + 118),
+// with a decay a channel (8 heads) 353 -> 30 + 106, wkv of 32 heads of 64 x 64 251 -> 45 + 48 (50 + 50).
 #pragma once
 #include <type_traits>
 
