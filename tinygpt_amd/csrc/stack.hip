@@ -1059,14 +1059,14 @@ void launch_rec_scan(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs&
 //   token by token  the longest entry's chain, of a wave's instructions a token, which grow with the rows of a lane; or the rows of all entries that a compute unit has to issue
 //   blocks          their preparation, 12 to 19 us however short the step is and then so much for every block and head of a compute unit, whatever the head's size; the longest entry's
 //                   chain of blocks, or the blocks that a compute unit has from all of them; and a launch more
-// Measured on 17 shapes of 4 to 64 heads, 32 to 128 key and 32 to 256 value channels, each from one entry of 64 to 2048 tokens to sixteen of 200 (255 points), the two sums are within a tenth of
-// most kernels' times, and the form taken is at worst 1.05 times the other.  us, token by token / blocks: wkv 32 heads of 64 x 64 one entry of 96 tokens 14.6 / 17.9, 160 22.1 / 20.4,
-// 2048 251 / 93, four of 300 46.7 / 45.8, eight of 300 67 / 79; 64 heads of 32 x 32 four of 300 43 / 62; 16 of 128 x 128 eight of 300 113 / 86.  Delta rules of 16 heads of 128 x 128 one of 160
+// Measured on 33 shapes of 4 to 64 heads, 16 to 128 key and 16 to 256 value channels, each from one entry of 64 to 2048 tokens to sixteen of 200 (543 points), the two sums are within a tenth of
+// most kernels' times.  Blocks are taken from a twentieth less on: the form taken is then at worst 1.08 times the other, with the sums alone 1.18.
+// us, token by token / blocks: wkv 32 heads of 64 x 64 one entry of 96 tokens 14.6 / 17.9, 160 22.1 / 20.4, 2048 251 / 93, four of 300 46.7 / 45.8, eight of 300 67 / 79; 64 heads of 32 x 32 four of 300 43 / 62; 16 of 128 x 128 eight of 300 113 / 86.  Delta rules of 16 heads of 128 x 128 one of 160
 // 30.9 / 31.2, 2048 338 / 157, eight of 300 107 / 121; 16 of 64 x 64 2048 276 / 109, eight of 300 55 / 69; 32 of 32 x 32 eight of 300 51 / 105; a decay a channel, 8 of 128 x 128, 2048 353 / 136,
 // eight of 300 79 / 74.  Option stack.line 0, which brings the older forms of prompts' products back, brings the scan back as well unless rec.min says otherwise.
 double rec_scan_us(const tgx_ctx* c, const tgx::RecScanArgs& a, bool wkv, int T, int S, int max_count) {
   const RecScanPlan p = rec_scan_plan(c, a, S);
-  const double issued = (double)p.rows * S * a.heads * p.cols / c->num_cus;
+  const double issued = (double)p.rows * (((long long)S * a.heads * p.cols + c->num_cus - 1) / c->num_cus);      // (of the compute unit that has most workgroups)
   const double chain = 0.075 + 0.013 * p.rows + (wkv ? 0.0 : 0.015) + (p.rg == 32 ? 0.02 : 0.0), full = wkv ? 0.065 + 0.01 * issued : 0.11 + 0.0081 * issued;
   return 3.0 + std::max(max_count * chain, full * T / S);
 }
@@ -1077,13 +1077,13 @@ double rec_blocks_us(const tgx_ctx* c, const tgx::RecScanArgs& a, bool wkv, int 
   const double per_cu = (T / (double)tgx::REC_BLOCK + 0.5 * S) * a.heads / c->num_cus;      // (an entry's last block is half full on average)
   return 4.0 + std::max(k.least, k.some + k.block * per_cu) + std::max(k.step * ((max_count + tgx::REC_BLOCK - 1) / tgx::REC_BLOCK), k.step_full * per_cu * ((a.vdim + 15) / 16));
 }
-constexpr int REC_BLOCK_WGS = 4;      // workgroups of the blocks a compute unit has at most (what their scratch is sized for; eight were never faster)
+constexpr int REC_BLOCK_WGS = 4;      // workgroups of the blocks a compute unit has at most (what their scratch is sized for; with 4.5 to 8 between 0.8 and 3 times the scan's time)
 void launch_recurrence(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs& a, int kind, int T, int S, int max_count) {
   StackModel* sm = c->stack;
   const bool wkv = kind == tgx::REC_WKV;
   const long long wgs = (long long)S * a.heads * ((a.vdim + 15) / 16), most_wgs = (long long)REC_BLOCK_WGS * c->num_cus;
   const bool pays = sm->rec_min >= 0 ? sm->rec_min > 0 && max_count >= sm->rec_min
-                                     : sm->line && wgs <= most_wgs && rec_blocks_us(c, a, wkv, T, S, max_count) < rec_scan_us(c, a, wkv, T, S, max_count);
+                                     : sm->line && wgs <= most_wgs && rec_blocks_us(c, a, wkv, T, S, max_count) < 0.95 * rec_scan_us(c, a, wkv, T, S, max_count);
   const size_t blocks = (size_t)T / tgx::REC_BLOCK + (size_t)S, most = (size_t)sm->cap_tokens / tgx::REC_BLOCK + (size_t)std::min<long long>(sm->d.max_seqs, most_wgs * S / wgs);      // (as many entries as the rule takes)
   if (pays && rec_vec(a) && a.dim <= tgx::REC_BLOCK_MAX_DIM && a.vdim <= tgx::REC_BLOCK_MAX_VDIM && ensure_terms2(c, 2 * rec_block_elems(blocks, a.heads, a.dim, a.vdim, !wkv), 2 * most * sm->rec_block_most))
     launch_rec_blocks(c, m, a, kind, S, max_count, reinterpret_cast<float*>(sm->terms2));
