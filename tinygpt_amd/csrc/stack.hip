@@ -1077,7 +1077,7 @@ double rec_blocks_us(const tgx_ctx* c, const tgx::RecScanArgs& a, bool wkv, int 
   const double per_cu = (T / (double)tgx::REC_BLOCK + 0.5 * S) * a.heads / c->num_cus;      // (an entry's last block is half full on average)
   return 4.0 + std::max(k.least, k.some + k.block * per_cu) + std::max(k.step * ((max_count + tgx::REC_BLOCK - 1) / tgx::REC_BLOCK), k.step_full * per_cu * ((a.vdim + 15) / 16));
 }
-constexpr int REC_BLOCK_WGS = 4;      // workgroups of the blocks a compute unit has at most (what their scratch is sized for; with 4.5 to 8 between 0.8 and 3 times the scan's time)
+constexpr int REC_BLOCK_WGS = 4;      // workgroups of the blocks a compute unit has at most (what their scratch is sized for; with 4.5 to 8 between 0.8 and 3.6 times the scan's time)
 void launch_recurrence(tgx_ctx* c, const tgx::StepMeta& m, const tgx::RecScanArgs& a, int kind, int T, int S, int max_count) {
   StackModel* sm = c->stack;
   const bool wkv = kind == tgx::REC_WKV;
