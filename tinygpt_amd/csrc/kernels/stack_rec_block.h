@@ -10,6 +10,7 @@
 //   rec_block_kernel        one workgroup per (entry, head, 16 value channels) walks the entry's blocks: three products a block with the state in matrix-core accumulators
 // Every D is a product of decays as they are: no logarithms, no quotients, so decays of zero and blocks whose whole product underflows are nothing special.  Blocks are counted from
 // the entry's first token; a block past the entry's end is padded by tokens with q = k = v = beta = 0 and w = 1, which change nothing.
+// A number that is not finite reaches the outputs of the earlier tokens of its block too (a factor of zero times it), as in the scalar-decay blocks and the matrix-core attentions; never another request.
 //
 // What bounds it: the token by token scan is a chain of one dependent read-update step a token, of one wave's instructions (0.13 to 0.17 us each); here the chain has a 32nd of the steps, of
 // 1.7 us (delta rules of up to 128 key channels; of 64 1.1) and 1.1 us (wkv; 0.75).  A block's operands are 68 KB a workgroup (40 KB) and 52 KB (32 KB), as long in a compute unit's memory
