@@ -155,6 +155,43 @@ def test_prompt_products_of_experts_weighted_at_their_input(T, experts, top, ff,
     assert np.quantile(rows, 15 / 16) < 1e-4, (T, dtype, rows)
 
 
+# Tiles of a last, at most half full round as two halves of K (line_plan.h): width 1024, 6208 hidden values and 1700 tokens halve 87 tiles of 256 x 256 (16 steps of K; rows that end
+# inside) and 112 of 128 x 128 (97 steps: uneven halves); experts of 2112 hidden values halve what their plan leaves over.  Against whole tiles only the order of fp32 sums differs
+# (1e-4 as above); a pass repeats itself bit for bit, whichever half comes first.
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("T", [1700, 1537])
+def test_halved_tiles(T, dtype):
+    import vitudra_oracle as vo
+    W, ff = 1024, 6208
+    cfg = dict(width=W, vocab=101, layers=[dict(type="wkv", mixer=dict(heads=W // 64, dim=64), mlp=dict(ff=ff))] * 2)
+    eng = SlotEngine(desc=wkv_model(W, ff, dtype, T), tensors={k: np.asarray(v, np.float32) for k, v in vo.random_tensors(cfg, 3, decay_rank=64).items()})
+    ids, want = np.random.default_rng(T).integers(0, 101, T), [0, 127, 128, 255, 256, T - 2, T - 1]
+    halved = [eng.step([("p", ids, want)], ["p"]) for _ in range(3)]
+    eng.model.set_option("stack.line_share", 0)
+    whole = eng.step([("p", ids, want)], ["p"])
+    eng.model.set_option("stack.line_share", 1)
+    eng.model.set_option("stack.ws_max", 32 * 1024)      # (enough for the rows' terms, not for halves of 256 x 256)
+    eng.step([("p", ids, want)], ["p"])
+    eng.close()
+    assert (halved[0] == halved[1]).all() and (halved[0] == halved[2]).all() and not (halved[0] == whole).all()
+    assert np.abs(halved[0] - whole).max() / np.abs(whole).max() < 1e-4, (T, dtype)
+
+
+@pytest.mark.parametrize("T,experts,top", [(2100, 5, 2), (700, 3, 1)])
+def test_halved_tiles_of_experts(T, experts, top):
+    import test_hip_keronex as tk
+    layer = tk.ret(tk.moe(experts, top, 2112, 2112), heads=4, dim=32, vdim=64, decay=[0.875, 0.99, 0.5, 0.9])
+    cfg = tk.config([layer, layer], width=1024)
+    eng, _ = tk.engine(cfg, "bf16", max_seqs=1, max_ctx=T, budget_tokens=T + 64)
+    ids, want = np.array(tk.tokens(cfg, T)), sorted({*range(0, T, 17), 127, 128, T - 1})
+    halved = [eng.step([("p", ids, want)], ["p"]) for _ in range(3)]
+    eng.model.set_option("stack.line_share", 0)
+    whole = eng.step([("p", ids, want)], ["p"])
+    eng.close()
+    assert (halved[0] == halved[1]).all() and (halved[0] == halved[2]).all() and not (halved[0] == whole).all()
+    assert np.quantile(np.abs(halved[0] - whole).max(1) / np.abs(whole).max(), 15 / 16) < 1e-4, T      # (a near tie of the router)
+
+
 @pytest.mark.parametrize("vocab", [53, 96, 1028, 1030])
 def test_wanted_logits_reach_their_slots(vocab):
     """a step's last wanted logits are its slots' current logits (bit for bit) and their argmax is what the greedy pick starts from; slots whose last place is not wanted keep theirs"""

@@ -29,7 +29,7 @@ OBJDIR = os.path.join(LIBDIR, "obj")
 
 
 def _deps():
-    deps = [os.path.join(HERE, "..", "include", "tgx.h"), os.path.join(CSRC, "ctx.h"), os.path.join(CSRC, "stack.h"), os.path.join(CSRC, "prefill_plan.h")]
+    deps = [os.path.join(HERE, "..", "include", "tgx.h"), os.path.join(CSRC, "ctx.h"), os.path.join(CSRC, "stack.h"), os.path.join(CSRC, "prefill_plan.h"), os.path.join(CSRC, "line_plan.h")]
     kd = os.path.join(CSRC, "kernels")
     return deps + [os.path.join(kd, f) for f in sorted(os.listdir(kd))]
 

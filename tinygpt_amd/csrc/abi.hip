@@ -1291,6 +1291,7 @@ int tgx_set_option(tgx_ctx* c, const char* key, int value) {
     if (!strcmp(key, "stack.rec_step")) { c->stack->rec_step = value ? 1 : 0; return TGX_OK; }      // 0: single tokens in the launches of a longer portion
     if (!strcmp(key, "stack.gemv")) { c->stack->gemv = value != 0; return TGX_OK; }      // 0: products of few rows on the matrix-core tiles too
     if (!strcmp(key, "stack.line")) { c->stack->line = value != 0; return TGX_OK; }      // 0: prompts' products on the register-staged tiles
+    if (!strcmp(key, "stack.line_share")) { c->stack->line_share = value != 0; return TGX_OK; }      // 0: every tile of a prompt's products whole
     if (!strcmp(key, "stack.ws_max")) { c->stack->ws_max = value < 0 ? -1 : value; return TGX_OK; }      // most KiB of a scratch buffer (-1: as memory allows)
     if (!strcmp(key, "debug.refuse_lds")) { c->stack->refuse_lds = value; return TGX_OK; }
     if (!strcmp(key, "stack.gemm_wt")) { if (value < 0 || value > 2) return set_err(c, TGX_ERR_INVALID, "stack.gemm_wt: 0, 1 or 2"); c->stack->gemm_wt = value; return TGX_OK; }

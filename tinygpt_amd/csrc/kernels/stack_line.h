@@ -8,8 +8,10 @@
 //   128 x 128, eight waves = two row halves x the four k16 steps of a stage, a ring of three 48-KB stages (gemm_dma8k_kernel's): the others
 // The products of one output are summed in the same two-term form as before (small term first); only the order of the fp32 sums differs.
 // Dual products (gate and up) take their two matrices in alternate blocks of 32 columns of a tile, so that both values of an output meet in one lane.
+// A last round of tiles that is at most half full is halved over K (SHARED, line_plan.h).
 // Tiles are dealt to the XCDs in contiguous runs, each run walked eight row tiles at a time: an XCD's workgroups share row blocks and weight tiles in its L2.
 #pragma once
+#include "../line_plan.h"
 #include "gemm_dma.h"
 #include "stack_gemm.h"
 
@@ -19,6 +21,8 @@ struct LineArgs {
   StackGemmArgs g;                      // A is not read: the terms are
   const bf16_t* terms; long long ldt;   // [rows][ldt]: interleaved lines; batch member z starts z * 2 * a_zoff elements into a row
   int gm, gn;                           // row and column tiles (gm: upper bound for grouped products)
+  int cus;                              // SHARED: the last tiles are halved over K (line_plan.h, rounds of cus workgroups); [halved tile][2] who has come and whose sums lie ready
+  int* met; float* sums;                // (zero between launches), and the sums
 };
 
 constexpr size_t LINE256_LDS = 5 * 32 * 1024, LINE128_LDS = 3 * 48 * 1024;
@@ -46,25 +50,66 @@ __global__ __launch_bounds__(256) void split_terms_kernel(const float* a, long l
   }
 }
 
-// tile of a workgroup: runs of consecutive tiles per XCD (workgroup id mod 8), walked in bands of eight row tiles
-__device__ __forceinline__ void line_tile(int id, int gm, int gn, int& tm, int& tn) {
-  const int total = gm * gn, per = total >> 3, rest = total & 7, xcd = id & 7;
-  const int t = xcd * per + min(xcd, rest) + (id >> 3);
+// tile t in bands of eight row tiles
+__device__ __forceinline__ void line_at(int t, int gm, int gn, int& tm, int& tn) {
   const int band = t / (8 * gn), rows = min(8, gm - 8 * band), in = t - band * 8 * gn;
   tm = 8 * band + in % rows;
   tn = in / rows;
 }
+// the id-th of `total` workgroups to its tile: runs of consecutive tiles per XCD (workgroup ids mod 8)
+__device__ __forceinline__ int line_run(int id, int total) { return (id & 7) * (total >> 3) + min(id & 7, total & 7) + (id >> 3); }
 
 // rows of the tile and where its operands lie
-struct LineTile { int z, mbase, mend, tn; };
+struct LineTile { int z, mbase, mend, tn, k0, nk, rest; };      // its steps of 64 from k0 on; the number of a halved one (-1: whole)
+template <bool SHARED>
 __device__ __forceinline__ bool line_place(const LineArgs& a, int TM, LineTile& t) {
-  int tm, gm = a.gm;
-  if (a.g.z_off) gm = min(gm, *a.g.n_tiles);
-  if ((int)blockIdx.x >= gm * a.gn) return false;
-  line_tile((int)blockIdx.x, gm, a.gn, tm, t.tn);
+  int tm;
+  const int id = (int)blockIdx.x, gm = a.g.z_off ? min(a.gm, *a.g.n_tiles) : a.gm, nk = a.g.K >> 6;
+  const LineShare sh = SHARED ? line_share(gm * a.gn, TM, nk, a.cus) : LineShare{gm * a.gn, 0};
+  t.k0 = 0; t.nk = nk; t.rest = -1;
+  if (id < sh.whole) line_at(line_run(id, sh.whole), gm, a.gn, tm, t.tn);
+  else if (!SHARED || id >= sh.whole + 2 * sh.rest) return false;
+  else {      // first halves of all, then the second ones: neighbours share operands in an XCD's L2
+    const int at = id - sh.whole, half = at >= sh.rest;
+    t.rest = line_run(half ? at - sh.rest : at, sh.rest);
+    line_at(sh.whole + t.rest, gm, a.gn, tm, t.tn);
+    t.k0 = half ? nk >> 1 : 0;
+    t.nk = half ? nk - t.k0 : nk >> 1;
+  }
   if (a.g.z_off) { t.z = a.g.tile_z[tm]; t.mbase = a.g.tile_m0[tm]; t.mend = min(a.g.z_off[t.z + 1], t.mbase + TM); }
   else { t.z = blockIdx.y; t.mbase = tm * TM; t.mend = min(a.g.M, t.mbase + TM); }
   return true;
+}
+// A halved tile's workgroups meet in memory: the first to have its sums writes them (numbers in pairs, past the L2 of its XCD, which the other's does not see) and is done; the
+// second adds them to its own, whichever half that is, and goes on to the epilogue.  What it waits for at most is the first one's writes, which nothing holds up.
+__device__ __forceinline__ void line_give(float* at, float x, float y) {
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(at), (unsigned long long)__float_as_uint(x) | ((unsigned long long)__float_as_uint(y) << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+typedef __attribute__((ext_vector_type(2))) float f32x2;
+__device__ __forceinline__ f32x2 line_take(const float* at) {
+  const unsigned long long v = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(at), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return f32x2{__uint_as_float((unsigned)v), __uint_as_float((unsigned)(v >> 32))};
+}
+// whether this workgroup is the first of its tile (the same in all threads; lds: an int that nobody else uses)
+__device__ __forceinline__ bool line_first(const LineArgs& a, const LineTile& t, int* lds) {
+  if (threadIdx.x == 0) *lds = __hip_atomic_fetch_add(a.met + 2 * t.rest, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const bool first = *lds == 0;
+  __syncthreads();
+  return first;
+}
+__device__ __forceinline__ void line_ready(const LineArgs& a, const LineTile& t) {      // behind the first one's last line_give
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's sums are in memory
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(a.met + 2 * t.rest + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void line_await(const LineArgs& a, const LineTile& t) {      // in front of the second one's first line_take
+  if (threadIdx.x == 0) {
+    while (!__hip_atomic_load(a.met + 2 * t.rest + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) __builtin_amdgcn_s_sleep(1);
+    __hip_atomic_store(a.met + 2 * t.rest, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // for the next launch
+    __hip_atomic_store(a.met + 2 * t.rest + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
 }
 __device__ __forceinline__ const bf16_t* line_row(const LineArgs& a, const LineTile& t, int row) {
   const int m = min(t.mbase + row, t.mend - 1);      // rows past the end are computed on a clamped row, never stored
@@ -134,12 +179,12 @@ __device__ __forceinline__ void line_epilogue(const LineArgs& a, const LineTile&
   else loop(std::false_type{}, std::integral_constant<int, EPI == SG_ADD || EPI == SG_ROWSCALE ? 4 : 1>{});
 }
 
-template <int DT, int EPI, bool DUAL>
+template <int DT, int EPI, bool DUAL, bool SHARED>
 __global__ __launch_bounds__(512) void stack_line256_kernel(const LineArgs a) {
   constexpr int TMN = 256, NSLOT = 5, UNIT = TMN * 64;     // 16-bit elements per unit: 256 rows x 128 bytes
   extern __shared__ __attribute__((aligned(1024))) bf16_t dma_lds[];
   LineTile t;
-  if (!line_place(a, TMN, t)) return;
+  if (!line_place<SHARED>(a, TMN, t)) return;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wv >> 1, wn = wv & 1;
   const unsigned lds_base = (unsigned)(size_t)dma_lds;
@@ -157,10 +202,10 @@ __global__ __launch_bounds__(512) void stack_line256_kernel(const LineArgs a) {
 #pragma unroll
   for (int p = 0; p < 4; p++) {
     const int row = (wv + 8 * p) * 8 + prow, chunk = pslot ^ ((row >> 1) & 7);
-    srcA[p] = line_row(a, t, row) + chunk * 8;
-    srcB[p] = line_col<DUAL, TMN>(a, t, row) + chunk * 8;
+    srcA[p] = line_row(a, t, row) + (size_t)t.k0 * 128 + chunk * 8;
+    srcB[p] = line_col<DUAL, TMN>(a, t, row) + (size_t)t.k0 * 64 + chunk * 8;
   }
-  const int nblk = a.g.K >> 6;
+  const int nblk = t.nk;
   // unit u = 3 b + j: j = 0 the A lines of step 2b, 1 the B lines of block b, 2 the A lines of step 2b + 1 (units past the end reload the last block)
   auto issue = [&](int b, int j, int p) {
     const int bb = min(b, nblk - 1);
@@ -224,7 +269,32 @@ __global__ __launch_bounds__(512) void stack_line256_kernel(const LineArgs a) {
     mfma_step(fa1, fb1, b + 2, 0, 0, 4);                        // unit 3b+6 = A of step 2b+4
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();                                 // the ring is free: every wave stages its block, 32 rows at a time, in a slice of its own
+  __builtin_amdgcn_s_barrier();                                 // the ring is free
+  if (SHARED && t.rest >= 0) {
+    float* at = a.sums + (size_t)t.rest * TMN * TMN + 2 * tid;
+    if (line_first(a, t, reinterpret_cast<int*>(dma_lds))) {
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+          for (int r = 0; r < 8; r++) line_give(at + ((i * 4 + j) * 8 + r) * 1024, acc[i][j][2 * r], acc[i][j][2 * r + 1]);
+      line_ready(a, t);
+      return;
+    }
+    line_await(a, t);
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+          const f32x2 v = line_take(at + ((i * 4 + j) * 8 + r) * 1024);
+          acc[i][j][2 * r] += v[0];
+          acc[i][j][2 * r + 1] += v[1];
+        }
+  }
+  // every wave stages its block, 32 rows at a time, in a slice of its own
   float* st = reinterpret_cast<float*>(dma_lds) + (size_t)wv * 32 * LINE_RS;
 #pragma unroll
   for (int i = 0; i < 2; i++) {
@@ -238,12 +308,12 @@ __global__ __launch_bounds__(512) void stack_line256_kernel(const LineArgs a) {
   }
 }
 
-template <int DT, int EPI, bool DUAL>
+template <int DT, int EPI, bool DUAL, bool SHARED>
 __global__ __launch_bounds__(512) void stack_line128_kernel(const LineArgs a) {
   constexpr int TMN = 128, NS = 3, T_A = TMN * 64, STAGE = 3 * T_A;      // a stage: A lines of two k32 steps | B lines, 128 rows x 128 bytes each
   extern __shared__ __attribute__((aligned(1024))) bf16_t dma_lds[];
   LineTile t;
-  if (!line_place(a, TMN, t)) return;
+  if (!line_place<SHARED>(a, TMN, t)) return;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kq = wv >> 1, wm = wv & 1;                         // k16 step of every stage, row half
   const unsigned lds_base = (unsigned)(size_t)dma_lds;
@@ -260,13 +330,13 @@ __global__ __launch_bounds__(512) void stack_line128_kernel(const LineArgs a) {
 #pragma unroll
   for (int p = 0; p < 2; p++) {
     const int piece = wv + 8 * p, row = piece * 8 + prow, chunk = pslot ^ ((row >> 1) & 7);
-    const bf16_t* ar = line_row(a, t, row) + chunk * 8;
-    gsrc[3 * p] = ar; gsrc[3 * p + 1] = ar + 64; gsrc[3 * p + 2] = line_col<DUAL, TMN>(a, t, row) + chunk * 8;
+    const bf16_t* ar = line_row(a, t, row) + (size_t)t.k0 * 128 + chunk * 8;
+    gsrc[3 * p] = ar; gsrc[3 * p + 1] = ar + 64; gsrc[3 * p + 2] = line_col<DUAL, TMN>(a, t, row) + (size_t)t.k0 * 64 + chunk * 8;
     ldst[3 * p] = (unsigned)(piece * 1024); ldst[3 * p + 1] = ldst[3 * p] + (unsigned)(T_A * 2); ldst[3 * p + 2] = ldst[3 * p] + (unsigned)(2 * T_A * 2);
   }
   // stage k: A lines advance by two (128 elements), B lines by one (64)
   auto issue_piece = [&](int q, int k, int stage) { dma_1k(gsrc[q] + (size_t)k * (q % 3 == 2 ? 64 : 128), lds_base + (unsigned)(stage * STAGE * 2) + ldst[q]); };
-  const int nk = a.g.K >> 6;
+  const int nk = t.nk;
 #pragma unroll
   for (int q = 0; q < 6; q++) issue_piece(q, 0, 0);
   if (nk > 1) {
@@ -333,6 +403,28 @@ __global__ __launch_bounds__(512) void stack_line128_kernel(const LineArgs a) {
         for (int r = 0; r < 16; r++) dst[(wm * 64 + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5)) * LINE_RS + j * 32 + (lane & 31)] = acc[i][j][r];
   }
   __syncthreads();
+  if (SHARED && t.rest >= 0) {
+    float* at = a.sums + (size_t)t.rest * TMN * TMN + 2 * tid;
+    auto cell = [&](int q) { return reinterpret_cast<f32x4*>(red + (size_t)(q * 16 + (tid >> 5)) * LINE_RS + 4 * (tid & 31)); };      // a thread's four columns of eight rows
+    if (line_first(a, t, reinterpret_cast<int*>(red + (size_t)2 * TMN * LINE_RS))) {
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const f32x4 v = *cell(q) + cell(q)[TMN * LINE_RS / 4];
+        line_give(at + (2 * q) * 1024, v[0], v[1]);
+        line_give(at + (2 * q + 1) * 1024, v[2], v[3]);
+      }
+      line_ready(a, t);
+      return;
+    }
+    line_await(a, t);
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const f32x2 u = line_take(at + (2 * q) * 1024), v = line_take(at + (2 * q + 1) * 1024);
+      *cell(q) = (*cell(q) + cell(q)[TMN * LINE_RS / 4]) + f32x4{u[0], u[1], v[0], v[1]};      // (the same whichever half is second)
+      cell(q)[TMN * LINE_RS / 4] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    __syncthreads();
+  }
   line_epilogue<DT, EPI, DUAL, TMN, true>(a, t, red, red + (size_t)TMN * LINE_RS, TMN, 0, t.tn * (DUAL ? 64 : 128), tid, 512);
 }
 

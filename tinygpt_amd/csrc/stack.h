@@ -165,6 +165,8 @@ struct StackModel {
   int ws_grown = 0;                    // tgx_get_option stack.ws_grown: how often part, terms and terms2 were allocated
   int ws_max = -1;                     // option stack.ws_max: most KiB of each of part, terms and terms2 (-1: as memory allows); products, attention and recurrences that would need more take their forms without scratch
   int refuse_lds = 0;                  // option debug.refuse_lds: the n-th product from now that asks for its LDS is refused it, as a device could (tests of a step that fails half-way)
+  void* share = nullptr; size_t share_bytes = 0, share_refused = SIZE_MAX;      // divided tiles of prompts' products (stack_line.hip)
+  int line_share = 1;                  // option stack.line_share: 0 keeps every tile of a prompt's products whole
   int line = 1;                        // option stack.line: 0 keeps prompts' products on the register-staged tiles
   int gemm_wt = 0;                     // option stack.gemm_wt: force the product's tile (1: 64 x 64, 2: 128 x 128); 0 = by the number of tiles
 };

@@ -5,13 +5,18 @@
 #include "kernels/stack_line.h"
 
 namespace {
-template <int DT, int EPI, bool DUAL>
+template <int DT, int EPI, bool DUAL, bool SHARED>
 void launch_line_t(tgx_ctx* c, const tgx::LineArgs& a, dim3 grid, int tile) {
   if (tile == 256) {
-    if (stack_allow_lds(c, (const void*)&tgx::stack_line256_kernel<DT, EPI, DUAL>, tgx::LINE256_LDS))
-      hipLaunchKernelGGL((tgx::stack_line256_kernel<DT, EPI, DUAL>), grid, dim3(512), tgx::LINE256_LDS, c->stream, a);
-  } else if (stack_allow_lds(c, (const void*)&tgx::stack_line128_kernel<DT, EPI, DUAL>, tgx::LINE128_LDS))
-    hipLaunchKernelGGL((tgx::stack_line128_kernel<DT, EPI, DUAL>), grid, dim3(512), tgx::LINE128_LDS, c->stream, a);
+    if (stack_allow_lds(c, (const void*)&tgx::stack_line256_kernel<DT, EPI, DUAL, SHARED>, tgx::LINE256_LDS))
+      hipLaunchKernelGGL((tgx::stack_line256_kernel<DT, EPI, DUAL, SHARED>), grid, dim3(512), tgx::LINE256_LDS, c->stream, a);
+  } else if (stack_allow_lds(c, (const void*)&tgx::stack_line128_kernel<DT, EPI, DUAL, SHARED>, tgx::LINE128_LDS))
+    hipLaunchKernelGGL((tgx::stack_line128_kernel<DT, EPI, DUAL, SHARED>), grid, dim3(512), tgx::LINE128_LDS, c->stream, a);
+}
+template <int DT, int EPI, bool DUAL>
+void launch_line_t(tgx_ctx* c, const tgx::LineArgs& a, dim3 grid, int tile) {
+  if (a.cus) launch_line_t<DT, EPI, DUAL, true>(c, a, grid, tile);
+  else launch_line_t<DT, EPI, DUAL, false>(c, a, grid, tile);
 }
 // 256-row or 128-row tiles for t256 / t128 of them: a compute unit takes 2.8 times as long for the large one (2048 x 2048 x 2048: 89 us for one round of 256 x 256, 38 for one of
 // 128 x 128; 11264 x 8192 x 2048: 652 us for six rounds against 768 for 22).  Fewer than 64 small ones leave most of the chip idle either way: the 64-wide tiles
@@ -20,6 +25,24 @@ int tile_of(const tgx_ctx* c, long long t256, long long t128) {
   if (t128 < 64) return 0;
   const long long r256 = (t256 + c->num_cus - 1) / c->num_cus, r128 = (t128 + c->num_cus - 1) / c->num_cus;
   return r256 * 28 <= r128 * 10 ? 256 : 128;
+}
+// memory of halved tiles (half a round at most): two numbers for each, then the sums of a half.  false: there is none, or option stack.ws_max forbids it, and every tile is whole
+bool share_scratch(tgx_ctx* c, int tile) {
+  StackModel* sm = c->stack;
+  const size_t need = (size_t)c->num_cus * 4 + (size_t)(c->num_cus / 2) * tile * tile * 4;
+  if (sm->ws_max >= 0 && need > (size_t)sm->ws_max * 1024) return false;
+  if (need <= sm->share_bytes) return true;
+  if (need >= sm->share_refused || hipStreamSynchronize(c->stream) != hipSuccess) return false;
+  void* p = nullptr;
+  if (hipMalloc(&p, need) != hipSuccess || hipMemsetAsync(p, 0, (size_t)c->num_cus * 4, c->stream) != hipSuccess) {
+    (void)hipGetLastError();
+    if (p) (void)hipFree(p);
+    sm->share_refused = need;
+    return false;
+  }
+  if (sm->share) (void)hipFree(sm->share);
+  sm->share = p; sm->share_bytes = need;
+  return true;
 }
 }  // namespace
 
@@ -43,7 +66,15 @@ void launch_stack_line(tgx_ctx* c, const tgx::StackGemmArgs& g, int epi, int nz,
   tgx::LineArgs a{};
   a.g = g; a.terms = terms; a.ldt = ldt; a.gm = row_tiles;
   a.gn = tgx::sg_dual(epi) ? (g.N + tile / 2 - 1) / (tile / 2) : (g.N + tile - 1) / tile;
-  const dim3 grid((unsigned)a.gm * (unsigned)a.gn, g.z_off ? 1 : nz);
+  int wgs = a.gm * a.gn;
+  if (nz == 1 && c->stack->line_share) {
+    const tgx::LineShare sh = tgx::line_share(g.z_off ? 1 : wgs, tile, g.K >> 6, c->num_cus);      // (a plan's tiles are counted on the device: half a round at most that are halved)
+    if (sh.rest && share_scratch(c, tile)) {
+      a.cus = c->num_cus; a.met = (int*)c->stack->share; a.sums = (float*)c->stack->share + c->num_cus;
+      wgs += g.z_off ? c->num_cus / 2 : sh.rest;
+    }
+  }
+  const dim3 grid((unsigned)wgs, g.z_off ? 1 : nz);
   TGX_DT16_SWITCH(c->dt,
     switch (epi) {
       case tgx::SG_STORE: launch_line_t<DT, tgx::SG_STORE, false>(c, a, grid, tile); break;
