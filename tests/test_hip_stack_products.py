@@ -47,6 +47,19 @@ def test_rows_of_a_step(slots, width, ff, vdim):
         assert np.abs(got[i] - want).max() / np.abs(want).max() < 2e-5, (slots, width, i)
 
 
+# (where the few-row kernel brings another four rows of a tile; the bound above)
+@pytest.mark.parametrize("width,ff", [(72, 24), (264, 40), (1024, 64)])
+@pytest.mark.parametrize("slots", [4, 5, 7, 8, 9, 12])
+def test_rows_of_a_tile(slots, width, ff):
+    d = desc(width, "fp32", slots, ff, 8)
+    t = so.random_tensors(d, slots)
+    seqs = np.random.default_rng(slots).integers(0, d.vocab, (slots, 2))
+    got = both(d, t, seqs)
+    for i in range(slots):
+        want = so.forward(d, t, seqs[i].tolist())
+        assert np.abs(got[i] - want).max() / np.abs(want).max() < 2e-5, (slots, width, i)
+
+
 @pytest.mark.parametrize("dtype,bound", [("bf16", 2.0 ** -8), ("fp16", 2.0 ** -11)])
 @pytest.mark.parametrize("slots", [2, 3, 16, 33, 64, 65])
 def test_rows_of_a_step_in_half_storage(slots, dtype, bound):

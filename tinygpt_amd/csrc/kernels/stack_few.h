@@ -26,20 +26,25 @@ namespace tgx {
 
 constexpr int few_max_waves(int mb) { return mb == 1 ? 16 : 8; }      // 128 / 256 registers a wave
 
-template <int DT, bool DUAL, int MB> constexpr int few_step_bytes() { return (DUAL ? 2 : 1) * (DT == DT_F32 ? 4096 : 2048) + MB * 4096; }
+// XP: the pieces (four activation rows each) of a tile of sixteen that are brought: 1 or 2 where the step has no more than four or eight rows (the rest of the operand repeats them and is
+// not stored).  A step of 64 k is 2 KB of weights and XP KB of activations, which cross from L2 for every sixteen columns.  us a launch, XP 4 -> as many as there are rows, four rows:
+// 2304 x 1024 5.7 -> 5.1, 8192 x 1024 8.3 -> 7.2, 32000 x 1024 20.8 -> 17.8, 2 x 8192 x 2048 21.5 -> 18.6; eight: 2048 x 4096 11.6 -> 10.5, 8192 x 2048 13.3 -> 11.9, 2048 x 8192
+// 18.8 -> 16.7, 32000 x 2048 35.0 -> 33.7
+template <int DT, bool DUAL, int MB, int XP> constexpr int few_step_bytes() { return (DUAL ? 2 : 1) * (DT == DT_F32 ? 4096 : 2048) + MB * XP * 1024; }
 // LDS of a workgroup: the waves' rings, which the sums use again at the end
-template <int DT, bool DUAL, int MB> constexpr size_t few_lds_bytes(int waves, int depth) {
-  const size_t ring = (size_t)waves * depth * few_step_bytes<DT, DUAL, MB>(), sums = (size_t)waves * (DUAL ? 2 : 1) * MB * 1024;
+template <int DT, bool DUAL, int MB, int XP> constexpr size_t few_lds_bytes(int waves, int depth) {
+  const size_t ring = (size_t)waves * depth * few_step_bytes<DT, DUAL, MB, XP>(), sums = (size_t)waves * (DUAL ? 2 : 1) * MB * 1024;
   return ring > sums ? ring : sums;
 }
 
 // what a lane reads whose place lies past the end of K (the last step of a K that is no multiple of 64)
 __device__ const u32x4 few_zeros = {0u, 0u, 0u, 0u};
 
-template <int DT, int EPI, bool DUAL, int MB>
+template <int DT, int EPI, bool DUAL, int MB, int XP>
 __device__ __forceinline__ void stack_few_body(const StackGemmArgs& a, const int depth, const int z, const int mbase, const int mend) {
   constexpr int NB = DUAL ? 2 : 1, WP = DT == DT_F32 ? 4 : 2;       // 1-KB pieces of a step's weight rows (per matrix)
-  constexpr int PIECES = NB * WP + MB * 4, STEP = few_step_bytes<DT, DUAL, MB>();
+  constexpr int PIECES = NB * WP + MB * XP, STEP = few_step_bytes<DT, DUAL, MB, XP>();
+  static_assert(XP == 4 || MB == 1, "all rows of a tile but the only one");
   extern __shared__ __attribute__((aligned(1024))) unsigned char few_lds[];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
   const int li = lane & 15, q = lane >> 4;                          // row (column) of the operands, quarter of a half step's k
@@ -50,7 +55,7 @@ __device__ __forceinline__ void stack_few_body(const StackGemmArgs& a, const int
 
   // DMA map: rows and slots of this lane in every piece; a slot past the end of K takes zeros
   const elem_t<DT>* wsrc[NB][WP];
-  const float* xsrc[MB][4];
+  const float* xsrc[MB][XP];
   constexpr int WROWS = 16 / WP;                                    // weight rows per piece
   const int wslot = lane % (64 / WROWS), xslot = lane & 15;
 #pragma unroll
@@ -61,7 +66,7 @@ __device__ __forceinline__ void stack_few_body(const StackGemmArgs& a, const int
 #pragma unroll
   for (int i = 0; i < MB; i++)
 #pragma unroll
-    for (int p = 0; p < 4; p++) {
+    for (int p = 0; p < XP; p++) {
       const int mc = min(mbase + 16 * i + 4 * p + q, mend - 1);
       xsrc[i][p] = a.A + (size_t)z * a.a_zoff + (size_t)(a.a_rows ? a.a_rows[mc] : mc) * a.lda;
     }
@@ -78,7 +83,7 @@ __device__ __forceinline__ void stack_few_body(const StackGemmArgs& a, const int
 #pragma unroll
     for (int i = 0; i < MB; i++)
 #pragma unroll
-      for (int p = 0; p < 4; p++, dst += 1024) {
+      for (int p = 0; p < XP; p++, dst += 1024) {
         const int k = 64 * c + 4 * (xslot ^ ((4 * p + q) & 7));
         dma_1k(k < a.K ? (const void*)(xsrc[i][p] + k) : (const void*)&few_zeros, dst);
       }
@@ -118,8 +123,9 @@ __device__ __forceinline__ void stack_few_body(const StackGemmArgs& a, const int
       }
 #pragma unroll
       for (int i = 0; i < MB; i++) {
-        const unsigned char* rx = st + NB * WP * 1024 + i * 4096 + li * 256;
-        const f32x4 x0 = *reinterpret_cast<const f32x4*>(rx + (((2 * sl) ^ (li & 7)) << 4)), x1 = *reinterpret_cast<const f32x4*>(rx + (((2 * sl + 1) ^ (li & 7)) << 4));
+        const int xr = li & (4 * XP - 1);
+        const unsigned char* rx = st + NB * WP * 1024 + i * 4096 + xr * 256;
+        const f32x4 x0 = *reinterpret_cast<const f32x4*>(rx + (((2 * sl) ^ (xr & 7)) << 4)), x1 = *reinterpret_cast<const f32x4*>(rx + (((2 * sl + 1) ^ (xr & 7)) << 4));
 #pragma unroll
         for (int e = 0; e < 8; e++) {
           const float v = e < 4 ? x0[e & 3] : x1[e & 3], x = R16.value ? round_storage_if<DT>(v, 1) : v;
@@ -179,36 +185,38 @@ __device__ __forceinline__ void stack_few_body(const StackGemmArgs& a, const int
   }
 }
 
-template <int DT, int EPI, bool DUAL, int MB>
+template <int DT, int EPI, bool DUAL, int MB, int XP>
 __global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_kernel(const StackGemmArgs a, const int depth) {
   int z = blockIdx.z, m0 = blockIdx.y * 16 * MB, rows_end = a.M;
   if (a.z_off) {
     if ((int)blockIdx.y >= *a.n_tiles) return;
     z = a.tile_z[blockIdx.y]; m0 = a.tile_m0[blockIdx.y]; rows_end = a.z_off[z + 1];
   }
-  stack_few_body<DT, EPI, DUAL, MB>(a, depth, z, m0, min(rows_end, m0 + 16 * MB));
+  stack_few_body<DT, EPI, DUAL, MB, XP>(a, depth, z, m0, min(rows_end, m0 + 16 * MB));
 }
 // two products that do not need each other, of the same rows and contraction length, in one launch: blockIdx.z chooses (the low-rank pair of a channel-delta layer, sixteen rows of
 // 1024 x 128 each: 4.7 us and 4.7, 5.7 together)
-template <int DT, int MB>
+template <int DT, int MB, int XP>
 __global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_pair_kernel(const StackGemmArgs a, const StackGemmArgs b, const int depth) {
-  if (blockIdx.z == 0) stack_few_body<DT, SG_STORE, false, MB>(a, depth, 0, 0, a.M);      // (one tile of rows)
-  else stack_few_body<DT, SG_STORE, false, MB>(b, depth, 0, 0, b.M);
+  if (blockIdx.z == 0) stack_few_body<DT, SG_STORE, false, MB, XP>(a, depth, 0, 0, a.M);      // (one tile of rows)
+  else stack_few_body<DT, SG_STORE, false, MB, XP>(b, depth, 0, 0, b.M);
 }
 
+// pieces of four activation rows that the tiles of sixteen need (a plan's rows are counted on the device)
+inline int few_pieces(const StackGemmArgs& a) { return a.z_off || a.M > 8 ? 4 : a.M > 4 ? 2 : 1; }
 // Waves and ring depth: some eight waves a compute unit (2048 on the chip) and four a workgroup at least, never more than K has steps; two steps of each in flight, one
 // where the launch has a thousand workgroups that cover for each other.  Measured, us at waves / depth 4/1, 4/2, 8/1, 8/2, 16/1: sixteen rows 1024 x 1024 (64 workgroups):
 // 6.7, 5.9, 5.6, 5.6, 5.5; eight rows 2048 x 8192 (128): 36.6, 22.7, 23.3, 18.5, 18.8; 4096 x 2048 (256): 12.8, 9.3, 9.8, 8.8, 9.3; 8192 x 2048 (512): 15.1, 13.0, 14.0, 15.5,
 // 15.7; sixteen rows 24576 x 1024 (1536): 16.8, 17.7, 18.1, 26.7, 26.8
 struct FewPlan { int nw, depth; size_t lds; };
-template <int DT, bool DUAL, int MB>
+template <int DT, bool DUAL, int MB, int XP>
 inline FewPlan few_plan(int num_cus, long long wgs, int K) {
   const int steps = (K + 63) / 64;
   FewPlan p{4, 1, 0};
   while (p.nw < few_max_waves(MB) && wgs * p.nw < 8LL * num_cus) p.nw *= 2;
   while (p.nw > 1 && p.nw > steps) p.nw /= 2;
   p.depth = wgs >= 4LL * num_cus || p.nw >= steps ? 1 : 2;
-  while ((p.lds = few_lds_bytes<DT, DUAL, MB>(p.nw, p.depth)) > 160 * 1024) { if (p.depth > 1) p.depth--; else p.nw /= 2; }
+  while ((p.lds = few_lds_bytes<DT, DUAL, MB, XP>(p.nw, p.depth)) > 160 * 1024) { if (p.depth > 1) p.depth--; else p.nw /= 2; }
   return p;
 }
 

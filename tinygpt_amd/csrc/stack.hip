@@ -29,9 +29,9 @@
 namespace tgx {
 // A few tokens: the latents into the pool beside the queries into latent space (a product batched over the heads, kernels/stack_few.h): neither needs the other, attention needs both.
 // Four tokens, 8 heads of 256 x 128: 4.5 us and 4.4, 4.6 together.
-template <int DT>
+template <int DT, int XP>
 __global__ __launch_bounds__(64 * few_max_waves(1)) void latent_append_queries_kernel(StepMeta m, LatentAppendArgs la, StackGemmArgs a, const int depth, const int heads) {
-  if ((int)blockIdx.z < heads) stack_few_body<DT, SG_STORE, false, 1>(a, depth, blockIdx.z, 0, a.M);
+  if ((int)blockIdx.z < heads) stack_few_body<DT, SG_STORE, false, 1, XP>(a, depth, blockIdx.z, 0, a.M);
   else for (int t = blockIdx.x; t < m.T; t += gridDim.x) latent_append_body<DT>(m, la, t);
 }
 // ... beside the vector kernel's products (one and two tokens; a rotated key part's queries are turned by the append).  Two tokens, 8 heads of 192 x 128: 5.0 us and 4.7, 5.6 together.
@@ -468,8 +468,14 @@ void latent_in(tgx_ctx* c, const tgx::StepMeta& m, const tgx::LatentAppendArgs& 
     } else {
       const dim3 grid((g.N + 15) / 16, 1, H + 1);
       TGX_DT_SWITCH(c->dt,
-        const tgx::FewPlan p = tgx::few_plan<DT, false, 1>(c->num_cus, (long long)grid.x * H, g.K);
-        if (stack_allow_lds(c, (const void*)&tgx::latent_append_queries_kernel<DT>, p.lds)) hipLaunchKernelGGL(tgx::latent_append_queries_kernel<DT>, grid, dim3(64 * p.nw), p.lds, c->stream, m, la, g, p.depth, H);)
+        auto go = [&](auto Xc) {
+          constexpr int XP = decltype(Xc)::value;
+          const tgx::FewPlan p = tgx::few_plan<DT, false, 1, XP>(c->num_cus, (long long)grid.x * H, g.K);
+          if (stack_allow_lds(c, (const void*)&tgx::latent_append_queries_kernel<DT, XP>, p.lds))
+            hipLaunchKernelGGL((tgx::latent_append_queries_kernel<DT, XP>), grid, dim3(64 * p.nw), p.lds, c->stream, m, la, g, p.depth, H);
+        };
+        const int xp = tgx::few_pieces(g);
+        if (xp == 1) go(std::integral_constant<int, 1>{}); else if (xp == 2) go(std::integral_constant<int, 2>{}); else go(std::integral_constant<int, 4>{});)
     }
     return;
   }

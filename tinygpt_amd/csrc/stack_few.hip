@@ -5,24 +5,30 @@
 #include "kernels/stack_few.h"
 
 namespace {
-template <int DT, int EPI, bool DUAL, int MB>
+template <int DT, int EPI, bool DUAL, int MB, int XP>
 void launch_few_mb(tgx_ctx* c, const tgx::StackGemmArgs& a, dim3 grid) {
-  const tgx::FewPlan p = tgx::few_plan<DT, DUAL, MB>(c->num_cus, (long long)grid.x * grid.y * grid.z, a.K);
-  if (!stack_allow_lds(c, (const void*)&tgx::stack_few_kernel<DT, EPI, DUAL, MB>, p.lds)) return;
-  hipLaunchKernelGGL((tgx::stack_few_kernel<DT, EPI, DUAL, MB>), grid, dim3(64 * p.nw), p.lds, c->stream, a, p.depth);
+  const tgx::FewPlan p = tgx::few_plan<DT, DUAL, MB, XP>(c->num_cus, (long long)grid.x * grid.y * grid.z, a.K);
+  if (!stack_allow_lds(c, (const void*)&tgx::stack_few_kernel<DT, EPI, DUAL, MB, XP>, p.lds)) return;
+  hipLaunchKernelGGL((tgx::stack_few_kernel<DT, EPI, DUAL, MB, XP>), grid, dim3(64 * p.nw), p.lds, c->stream, a, p.depth);
 }
-template <int DT, int MB>
+template <int DT, int MB, int XP>
 void launch_few_pair_mb(tgx_ctx* c, const tgx::StackGemmArgs& a, const tgx::StackGemmArgs& b, dim3 grid) {
-  const tgx::FewPlan p = tgx::few_plan<DT, false, MB>(c->num_cus, (long long)grid.x * grid.y * grid.z, a.K);
-  if (!stack_allow_lds(c, (const void*)&tgx::stack_few_pair_kernel<DT, MB>, p.lds)) return;
-  hipLaunchKernelGGL((tgx::stack_few_pair_kernel<DT, MB>), grid, dim3(64 * p.nw), p.lds, c->stream, a, b, p.depth);
+  const tgx::FewPlan p = tgx::few_plan<DT, false, MB, XP>(c->num_cus, (long long)grid.x * grid.y * grid.z, a.K);
+  if (!stack_allow_lds(c, (const void*)&tgx::stack_few_pair_kernel<DT, MB, XP>, p.lds)) return;
+  hipLaunchKernelGGL((tgx::stack_few_pair_kernel<DT, MB, XP>), grid, dim3(64 * p.nw), p.lds, c->stream, a, b, p.depth);
 }
 template <int DT, int EPI, bool DUAL>
 void launch_few_t(tgx_ctx* c, const tgx::StackGemmArgs& a, dim3 grid, int mb) {
   switch (mb) {
-    case 1: launch_few_mb<DT, EPI, DUAL, 1>(c, a, grid); break;
-    case 2: launch_few_mb<DT, EPI, DUAL, 2>(c, a, grid); break;
-    default: launch_few_mb<DT, EPI, DUAL, 4>(c, a, grid); break;
+    case 1: {
+      const int xp = tgx::few_pieces(a);
+      if (xp == 1) launch_few_mb<DT, EPI, DUAL, 1, 1>(c, a, grid);
+      else if (xp == 2) launch_few_mb<DT, EPI, DUAL, 1, 2>(c, a, grid);
+      else launch_few_mb<DT, EPI, DUAL, 1, 4>(c, a, grid);
+      break;
+    }
+    case 2: launch_few_mb<DT, EPI, DUAL, 2, 4>(c, a, grid); break;
+    default: launch_few_mb<DT, EPI, DUAL, 4, 4>(c, a, grid); break;
   }
 }
 }  // namespace
@@ -32,9 +38,11 @@ void launch_stack_few_pair(tgx_ctx* c, const tgx::StackGemmArgs& a, const tgx::S
   const int mb = a.M <= 16 ? 1 : a.M <= 32 ? 2 : 4;
   const dim3 grid((std::max(a.N, b.N) + 15) / 16, 1, 2);
   TGX_DT_SWITCH(dt,
-    if (mb == 1) launch_few_pair_mb<DT, 1>(c, a, b, grid);
-    else if (mb == 2) launch_few_pair_mb<DT, 2>(c, a, b, grid);
-    else launch_few_pair_mb<DT, 4>(c, a, b, grid);)
+    if (mb == 1 && tgx::few_pieces(a) == 1) launch_few_pair_mb<DT, 1, 1>(c, a, b, grid);
+    else if (mb == 1 && tgx::few_pieces(a) == 2) launch_few_pair_mb<DT, 1, 2>(c, a, b, grid);
+    else if (mb == 1) launch_few_pair_mb<DT, 1, 4>(c, a, b, grid);
+    else if (mb == 2) launch_few_pair_mb<DT, 2, 4>(c, a, b, grid);
+    else launch_few_pair_mb<DT, 4, 4>(c, a, b, grid);)
 }
 
 // grouped_tiles: upper bound of the tile list of a grouped product (a.z_off), 0 for plain and batched ones
