@@ -246,6 +246,25 @@ def test_short_prompt_blocks_equal_steps(name, S, dtype):
         assert rel_err(k1, k0) < ulp and rel_err(v1, v0) < ulp
 
 
+# blocks of 32 queries whose keys four waves divide (up to a chip of them; head_dim 128 from seven tiles of keys on): the last block of one, 31 and 32 rows, streams without a tile, keys
+# that end at and beside four tiles.  Against the undivided form on one layer: another order of fp32 sums, 2e-5 as for two streams
+@pytest.mark.parametrize("name,S", [("qwen2.5-0.5b", 129), ("qwen2.5-0.5b", 160), ("qwen2.5-0.5b", 191), ("qwen2.5-0.5b", 257), ("llama-3.2-1b", 256), ("qwen3-0.6b", 385), ("qwen3-0.6b", 449), ("qwen3-0.6b", 512)])
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+def test_four_streams_of_keys(name, S, dtype):
+    d = copy.deepcopy(known_desc(name, dtype))
+    d.layers, d.vocab, d.max_ctx = 1, 4096, S + 16
+    m = Model(d, product_backend()).load_synthetic(1234, 0.02).finalize()
+    prompt = synth.synth_prompt(d.vocab, S, 80)[None, :]
+    outs = []
+    for ksplit in (0, 1, 1):
+        m.set_option("prefill.attn_ksplit", ksplit)
+        m.reset_cache(); m.forward(prompt)
+        outs.append(m.logits(rounded=False).copy())
+    np.testing.assert_array_equal(outs[1], outs[2])
+    assert not (outs[0] == outs[1]).all()
+    assert rel_err(outs[1], outs[0]) < 2e-5, rel_err(outs[1], outs[0])
+
+
 # N = hidden products whose steps of 64 do not fill six or seven slabs (25 and 29 steps; tests/test_prefill_plan.py has the rule): the counts that do are taken.  Bound as above
 @pytest.mark.parametrize("heads,S,dtype", [(25, 129, "bf16"), (25, 245, "fp16"), (29, 200, "bf16"), (29, 131, "fp16")])
 def test_products_that_fill_no_six_slabs(heads, S, dtype):

@@ -520,7 +520,8 @@ struct AttnPrefillArgs {
 // query meet once, through LDS, after the loop ((m, l, O) merged as flash-decoding does).  One workgroup per CU instead of two, the same matrix work per CU and
 // cycle, half the chain; blocks are dispatched heaviest first (AttnPrefillArgs.heavy_first) so that the second round fills the CUs as they free up.
 // QW = waves of queries (32 each).  A short prompt's blocks of 128 queries leave most of the chip idle (509 tokens, sixteen heads: 64 workgroups, two waves a SIMD walking four
-// pairs of tiles); blocks of 64 are twice as many workgroups of four waves.
+// pairs of tiles); blocks of 64 are twice as many workgroups of four waves, and blocks of 32 with KP = 4 as many again of four waves with a quarter of the tiles each: two steps where
+// there were four (509 tokens, sixteen heads of 128: 19.5 -> 17.4 us; 192 tokens, 32 heads of 64 8.9 -> 8.4).
 // PAGED (round 6): the workgroup copies the part of the sequence's block table it needs (<= 1024 entries) into LDS first; a K / V row's address then takes one LDS
 // read (it does not touch the counted vmcnt waits of the tile pipeline) — a 64-key tile never straddles a 128-token page.
 template <int DT, int HD, int LA = 2, int KP = 1, bool PAGED = false, int QW = 4>
@@ -750,12 +751,12 @@ __global__ __launch_bounds__(64 * QW * KP, QW < 4 ? 1 : KP == 2 ? 2 : (LA == 1 ?
   // 2-byte writes 4 KB apart (64 cache lines per instruction: ~20 µs of the kernel at S = 2048); instead each wave transposes its 32 x HD block
   // through LDS (rows of 2 HD + 8 bytes: conflict-free 4-byte column writes) and stores whole rows, 16 bytes per lane.
   __syncthreads();                              // every wave is done with the last K / V tile
-  if constexpr (KP == 2) {
-    // the odd-tile stream of every query joins the even-tile one: lane-to-lane (the two waves hold the same queries in the same layout)
+  if constexpr (KP >= 2) {
+    // the other streams of every query join the first one: lane-to-lane (the waves hold the same queries in the same layout)
     constexpr int NV = NB * 16 + 2;
-    static_assert(QW * NV * 64 * 4 <= KP * REG * 2, "the merge buffer exceeds the K / V tiles");
-    float* const mo = reinterpret_cast<float*>(smem) + (size_t)wv * NV * 64 + lane;
-    if (kp == 1) {
+    static_assert((KP - 1) * QW * NV * 64 * 4 <= KP * REG * 2, "the merge buffer exceeds the K / V tiles");
+    if (kp > 0) {
+      float* const mo = reinterpret_cast<float*>(smem) + (size_t)((kp - 1) * QW + wv) * NV * 64 + lane;
 #pragma unroll
       for (int b = 0; b < NB; b++)
 #pragma unroll
@@ -764,19 +765,23 @@ __global__ __launch_bounds__(64 * QW * KP, QW < 4 ? 1 : KP == 2 ? 2 : (LA == 1 ?
     }
     __syncthreads();
     if (kp == 0) {
-      const float m_b = mo[(NB * 16) * 64], l_b = mo[(NB * 16 + 1) * 64];
-      const float m_new = fmaxf(m_run, m_b);
-      const bool dead = m_new == -INFINITY;
-      const float fa = dead ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new), fb = dead ? 1.f : __builtin_amdgcn_exp2f(m_b - m_new);
-      l_run = l_run * fa + l_b * fb;
-      m_run = m_new;
 #pragma unroll
-      for (int b = 0; b < NB; b++)
+      for (int s = 0; s < KP - 1; s++) {
+        const float* const mo = reinterpret_cast<const float*>(smem) + (size_t)(s * QW + wv) * NV * 64 + lane;
+        const float m_b = mo[(NB * 16) * 64], l_b = mo[(NB * 16 + 1) * 64];
+        const float m_new = fmaxf(m_run, m_b);
+        const bool dead = m_new == -INFINITY;
+        const float fa = dead ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new), fb = dead ? 1.f : __builtin_amdgcn_exp2f(m_b - m_new);
+        l_run = l_run * fa + l_b * fb;
+        m_run = m_new;
 #pragma unroll
-        for (int r = 0; r < 16; r++) oacc[b][r] = oacc[b][r] * fa + mo[(b * 16 + r) * 64] * fb;
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) oacc[b][r] = oacc[b][r] * fa + mo[(b * 16 + r) * 64] * fb;
+      }
     }
     __syncthreads();                            // the merge buffer is read: the staging rows below reuse it
-    if (kp == 1) return;
+    if (kp > 0) return;
   }
   constexpr int RS = HD + 4;                    // staged row stride in 16-bit elements
   static_assert(QW * 32 * RS <= 64 * LQ + 64 * LV, "output staging exceeds the K / V tiles");

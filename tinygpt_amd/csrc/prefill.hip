@@ -318,12 +318,20 @@ void launch_attn_prefill(tgx_ctx* c, const tgx::AttnPrefillArgs& a_, bool allow_
   // below a chip of workgroups: blocks of 64 queries, twice as many of half the waves (QW = 2).  ms per prompt, 64 / 128: Qwen3-0.6B 256 tokens 2.72 / 2.82, 509 3.43 / 3.53, 1000
   // 4.86 / 5.03, 1300 6.05 / 6.15; Llama-3.2-1B fp16 256 2.22 / 2.26, 700 4.53 / 4.57
   const bool half = ksplit && nwg <= c->num_cus;
+  // ... and of 32, whose keys four waves divide, while those do not outnumber the compute units: at head_dim 128 only from seven tiles of keys on (below, the same or one step less, and
+  // half of what a wave stages at a time).  us a prompt, 32 / 64: Qwen3-0.6B 133 tokens 2523 / 2490, 256 2713 / 2730, 384 3146 / 3132, 509 3206 / 3288; Qwen2.5-0.5B 200 2010 / 2035, 509
+  // 2869 / 2926; Llama-3.2-1B 256 2243 / 2253; beyond a chip Llama-3.2-1B 384 tokens 2962 / 2910, 1000 5148 / 4913
+  const bool quarter = half && a.heads * ((a.S + 31) / 32) <= c->num_cus && (hd == 64 || a.past + a.S > 6 * 64);
   a.heavy_first = ksplit ? 1 : 0;
   const dim3 gridk(a.heads, nqb), blkk(512), grid(nqb, a.heads), blk(256);
   auto go = [&](auto paged) {        // (paged KV: the same forms through the sequence's block table)
     constexpr bool P = decltype(paged)::value;
     TGX_DT16_SWITCH(c->dt,
-      if (half) {
+      if (quarter) {
+        const dim3 gridq(a.heads, (a.S + 31) / 32);
+        if (hd == 64) hipLaunchKernelGGL((tgx::attn_prefill_kernel<DT, 64, 1, 4, P, 1>), gridq, dim3(256), 4 * lds1, c->stream, a);
+        else hipLaunchKernelGGL((tgx::attn_prefill_kernel<DT, 128, 1, 4, P, 1>), gridq, dim3(256), 4 * lds1, c->stream, a);
+      } else if (half) {
         const dim3 gridh(a.heads, (a.S + 63) / 64);
         if (hd == 64) hipLaunchKernelGGL((tgx::attn_prefill_kernel<DT, 64, 2, 2, P, 2>), gridh, dim3(256), 2 * lds1, c->stream, a);
         else hipLaunchKernelGGL((tgx::attn_prefill_kernel<DT, 128, 1, 2, P, 2>), gridh, dim3(256), 2 * lds1, c->stream, a);
@@ -456,6 +464,14 @@ int prefill_set_attrs(tgx_ctx* c) {
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma_qkv8_kernel<tgx::DT_F16>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (3 * 128 + 128 + 64) * 64 * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8i_kernel<tgx::DT_BF16, tgx::GEMM_SILU>), hipFuncAttributeMaxDynamicSharedMemorySize, 5 * 256 * 128));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8i_kernel<tgx::DT_F16, tgx::GEMM_SILU>), hipFuncAttributeMaxDynamicSharedMemorySize, 5 * 256 * 128));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_BF16, 64, 1, 4, false, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, 4 * (64 * 72 + 64 * 96) * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_BF16, 128, 1, 4, false, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, 4 * (64 * 136 + 64 * 160) * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_BF16, 64, 1, 4, true, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, 4 * (64 * 72 + 64 * 96) * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_BF16, 128, 1, 4, true, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, 4 * (64 * 136 + 64 * 160) * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_F16, 64, 1, 4, false, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, 4 * (64 * 72 + 64 * 96) * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_F16, 128, 1, 4, false, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, 4 * (64 * 136 + 64 * 160) * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_F16, 64, 1, 4, true, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, 4 * (64 * 72 + 64 * 96) * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_F16, 128, 1, 4, true, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, 4 * (64 * 136 + 64 * 160) * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_BF16, 128, 1, 2, false, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_BF16, 128, 1, 2, true, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_F16, 128, 1, 2, false, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
