@@ -265,6 +265,23 @@ def test_four_streams_of_keys(name, S, dtype):
     assert rel_err(outs[1], outs[0]) < 2e-5, rel_err(outs[1], outs[0])
 
 
+# the eight-wave 128 x 128 tiles with a stage's k16 steps in halves (chains of up to 32 stages; 33 and 34 take quarters): the last row tile of one row, 32 and 127, column tiles that end
+# inside, gate_up whole, N = hidden products in slabs and (700 rows) whole.  Against the steps as above
+@pytest.mark.parametrize("S", [129, 160, 255, 257, 700])
+@pytest.mark.parametrize("heads,inter,dtype", [(7, 1472, "bf16"), (32, 2048, "fp16"), (33, 2176, "bf16")])
+def test_eight_wave_tiles_in_halves(heads, inter, dtype, S):
+    d = copy.deepcopy(known_desc("llama-3.2-1b", dtype))
+    d.hidden, d.heads, d.kv_heads, d.inter, d.layers, d.vocab, d.max_ctx = 64 * heads, heads, 1 if heads < 32 else heads // 8 if heads % 8 == 0 else 3, inter, 1, 1024, 704
+    gpu = Model(d, product_backend()).load_synthetic(23, 0.02).finalize()
+    prompt = synth.synth_prompt(d.vocab, S, 5)[None, :]
+    l1, _, _, kv1 = run(gpu, prompt, mfma=True)
+    l0, _, _, kv0 = run(gpu, prompt, mfma=False)
+    assert rel_err(l1, l0) < 1e-3
+    ulp = {"bf16": 8e-3, "fp16": 1e-3}[dtype]
+    for (k1, v1), (k0, v0) in zip(kv1, kv0):
+        assert rel_err(k1, k0) < ulp and rel_err(v1, v0) < ulp
+
+
 # N = hidden products whose steps of 64 do not fill six or seven slabs (25 and 29 steps; tests/test_prefill_plan.py has the rule): the counts that do are taken.  Bound as above
 @pytest.mark.parametrize("heads,S,dtype", [(25, 129, "bf16"), (25, 245, "fp16"), (29, 200, "bf16"), (29, 131, "fp16")])
 def test_products_that_fill_no_six_slabs(heads, S, dtype):

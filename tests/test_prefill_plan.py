@@ -21,6 +21,7 @@ extern "C" int empty_slab(int cus, int k_lo, int k_hi, int* out) {
 }
 extern "C" int whole(int m, int n, int k, int cus, int most) { return tgx::gate_up_whole(m, n, k, cus, most); }
 extern "C" int slabs(int m, int n, int k, int cus) { return tgx::eight_wave_slabs(m, n, k, cus); }
+extern "C" int halves(int stages) { return tgx::eight_wave_halves(stages); }
 extern "C" int steps(int k, int z) { return tgx::slab_steps(k, z); }
 """
 
@@ -63,3 +64,12 @@ def test_gate_up_is_whole_only_where_the_eight_wave_kernel_takes_it(plan):
         for tiles in range(1, 300):
             assert not (plan.whole(100, 128 * tiles, 512, 256, most) and 2 * tiles > most * 256)
     assert not plan.whole(133, 128 * 48, 1024, 256, 0) and plan.whole(133, 128 * 48, 1024, 256, 1)
+
+
+def test_short_chains_of_stages_are_halved(plan):
+    assert [plan.halves(n) for n in (1, 4, 32, 33, 128)] == [1, 1, 1, 0, 0]
+
+
+@pytest.mark.parametrize("rows,columns,K,slabs", [(384, 1024, 3072, 8), (385, 1024, 3072, 7), (509, 1024, 3072, 5), (600, 1024, 3072, 5), (509, 896, 4864, 8)])
+def test_slabs_of_more_than_three_row_tiles(plan, rows, columns, K, slabs):
+    assert plan.slabs(rows, columns, K, 256) == slabs

@@ -793,4 +793,132 @@ __global__ __launch_bounds__(512) void gemm_dma8k_kernel(const GemmArgs a) {
     }
 }
 
+// ---- the same tile, waves = 2 x 2 quadrants x TWO k halves of every stage, for short chains of stages (K slabs, K up to 2048) ------------------------
+// A launch of few stages is what stands around its loop: the quarters above meet in 384 KB of LDS traffic over three barriers, half of the waves idle from the first on, and four waves store
+// a tile four bytes a lane: 5.7 of the 14.5 us of 200 x 2048 x 2048 in eight slabs (2.1 to the first stage, 0.83 a stage).  Two halves exchange a quarter of that over one barrier and
+// all eight waves store: 2.3 us.  The price are twelve fragment reads a stage and wave for eight.  us quarters / halves: 200 x 2048 x 2048 in eight slabs (four stages) 14.5 / 12.1, in
+// four (eight) 15.2 / 12.3; 509 x 1024 x 3072, eight (six) 17.4 / 14.8; 200 x 2048 x 8192, eight (sixteen) 28.0 / 26.8; 300 x 2048 x 8192, five (26) 34.8 / 34.3; 2048 x 2048 x 2048, whole
+// (32) 40.7 / 40.1; 1000 x 2048 x 8192, two (64) 68.4 / 70.1; 2048 x 2048 x 8192, whole (128) 124 / 129: up to 32 stages (prefill_plan.h).
+template <int DT, int EPI, bool LO = true>
+__global__ __launch_bounds__(512) void gemm_dma8h_kernel(const GemmArgs a) {
+  constexpr int DBK = 64, TMN = 128, NS = 3, STAGE = 3 * TMN * DBK;
+  extern __shared__ __attribute__((aligned(1024))) bf16_t dma_lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kh = wv >> 2, wm = (wv >> 1) & 1, wn = wv & 1;
+  int tile_m, tile_n;
+  xcd_tile(a, tile_m, tile_n);
+  const int m0 = tile_m * TMN, n0 = tile_n * TMN;
+  const unsigned lds_base = (unsigned)(size_t)dma_lds;
+  f32x16 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+
+  const int prow = lane >> 3, pslot = lane & 7;
+  const int k_begin = EPI == GEMM_PARTIAL ? (int)blockIdx.z * a.k_per : 0;
+  const int k_end = EPI == GEMM_PARTIAL ? min(a.K, k_begin + a.k_per) : a.K;
+  const bf16_t* gsrc[6];
+  unsigned ldst[6];
+#pragma unroll
+  for (int p = 0; p < 2; p++) {
+    const int piece = wv + 8 * p, row = piece * 8 + prow;
+    const int chunk = pslot ^ ((row >> 1) & 7);
+    const size_t g = (size_t)min(m0 + row, a.M - 1) * a.K + chunk * 8;
+    const int nb = min(n0 + row, a.N - 1);
+    const size_t brow = EPI == GEMM_SILU ? (size_t)((nb & 1) ? a.inter : 0) + (size_t)(nb >> 1) : (size_t)nb;
+    gsrc[3 * p] = a.A_hi + g + k_begin; gsrc[3 * p + 1] = a.A_lo + g + k_begin; gsrc[3 * p + 2] = a.B + brow * a.K + chunk * 8 + k_begin;
+    ldst[3 * p] = (unsigned)(piece * 1024); ldst[3 * p + 1] = ldst[3 * p] + (unsigned)(TMN * DBK * 2); ldst[3 * p + 2] = ldst[3 * p] + (unsigned)(2 * TMN * DBK * 2);
+  }
+  auto issue_piece = [&](int q, int k, int stage) { if (!LO && q % 3 == 1) return; dma_1k(gsrc[q] + k * DBK, lds_base + (unsigned)(stage * STAGE * 2) + ldst[q]); };
+  auto frag = [&](const bf16_t* tile, int row, int kchunk) -> bf16x8 {
+    return *reinterpret_cast<const bf16x8*>(tile + row * DBK + ((kchunk ^ ((row >> 1) & 7)) << 3));
+  };
+  const int nk = (k_end - k_begin) / DBK;      // (one at least: slabs_hold_k)
+#pragma unroll
+  for (int q = 0; q < 6; q++) issue_piece(q, 0, 0);
+  if (nk > 1) {
+#pragma unroll
+    for (int q = 0; q < 6; q++) issue_piece(q, 1, 1);
+  }
+  bf16x8 fah[2][2], fal[2][2], fb[2][2];
+  for (int k = 0; k < nk; k++) {
+    // stage k landed: only this wave's pieces of stage k + 1 may fly
+    if (k + 1 < nk) { if (LO) asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); else asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); }
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    const bool more = k + 2 < nk;
+    const int nst = (k + 2) % NS;
+    const bf16_t* st = dma_lds + (size_t)(k % NS) * STAGE;
+    const bf16_t *tAh = st, *tAl = st + TMN * DBK, *tB = st + 2 * TMN * DBK;
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      const int kchunk = (kh * 2 + s) * 2 + (lane >> 5);      // this wave's k16 steps of the stage
+#pragma unroll
+      for (int j = 0; j < 2; j++) fb[s][j] = frag(tB, wn * 64 + j * 32 + (lane & 31), kchunk);
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const int row = wm * 64 + i * 32 + (lane & 31);
+        fah[s][i] = frag(tAh, row, kchunk);
+        if (LO) fal[s][i] = frag(tAl, row, kchunk);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+          if (LO) acc[i][j] = mfma16<DT>(fal[s][i], fb[s][j], acc[i][j]);   // small term first
+          acc[i][j] = mfma16<DT>(fah[s][i], fb[s][j], acc[i][j]);
+          const int q = s * 4 + i * 2 + j;
+          if (more && q < 6) issue_piece(q, k + 2, nst);            // one DMA per two MFMAs
+        }
+  }
+
+  // a wave hands the other half's wave the column block that that one finishes (kh 0: j 0, kh 1: j 1); first half + second half on both sides
+  __builtin_amdgcn_s_barrier();                               // every wave is done with the ring
+  float* red = reinterpret_cast<float*>(dma_lds);
+  auto give = [&](auto J) {                                   // (constant block indices: a run-time one would send the accumulators to scratch memory)
+    float* dst = red + (size_t)wv * 2 * 16 * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) dst[(i * 16 + r) * 64] = acc[i][J.value][r];
+  };
+  if (kh == 0) give(std::integral_constant<int, 1>{}); else give(std::integral_constant<int, 0>{});
+  __syncthreads();
+  const float* other = red + (size_t)(wv ^ 4) * 2 * 16 * 64 + lane;
+  f32x16 fin[2];                                              // the wave's final 64 x 32
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const float o = other[(i * 16 + r) * 64];
+      fin[i][r] = kh == 0 ? acc[i][0][r] + o : o + acc[i][1][r];
+    }
+  const int col = n0 + wn * 64 + kh * 32 + (lane & 31), row0 = m0 + wm * 64;
+  if constexpr (EPI == GEMM_SILU) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) silu_block_store<DT>(fin[i], lane, col, row0 + i * 32, a);
+  } else {
+    if (col >= a.N) return;
+    const float bv = EPI != GEMM_PARTIAL && a.bias ? elem_to_f32<DT>(a.bias[col]) : 0.f;
+    float* out = EPI == GEMM_PARTIAL ? a.part + ((size_t)blockIdx.z * a.M + row0) * a.N + col : a.C + (size_t)row0 * a.ldc + col;
+    const unsigned ld = EPI == GEMM_PARTIAL ? (unsigned)a.N : (unsigned)a.ldc;
+    const int rows = a.M - row0;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const int row = i * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
+        if (row >= rows) continue;
+        float* dst = out + (size_t)((unsigned)row * ld);
+        *dst = EPI == GEMM_PARTIAL ? fin[i][r] : EPI == GEMM_RESIDUAL ? *dst + (fin[i][r] + bv) : fin[i][r] + bv;
+      }
+  }
+}
+
 }  // namespace tgx

@@ -68,6 +68,18 @@ static bool gemm_full_lines(const tgx_ctx* c, int epi, int M, int N, int K) {
   return t256 >= c->num_cus && !ragged256;
 }
 
+// the eight-wave 128 x 128 kernels: k16 steps of a stage in halves or quarters between the waves (prefill_plan.h); one: the first term of the activations alone
+template <int DT, int EPI, bool LO>
+static void launch_dma8k_t(tgx_ctx* c, const tgx::GemmArgs& g, dim3 grid, int stages) {
+  const size_t lds = (size_t)3 * 3 * 128 * 64 * 2;
+  if (tgx::eight_wave_halves(stages)) hipLaunchKernelGGL((tgx::gemm_dma8h_kernel<DT, EPI, LO>), grid, dim3(512), lds, c->stream, g);
+  else hipLaunchKernelGGL((tgx::gemm_dma8k_kernel<DT, EPI, LO>), grid, dim3(512), lds, c->stream, g);
+}
+template <int DT, int EPI>
+static void launch_dma8k(tgx_ctx* c, const tgx::GemmArgs& g, dim3 grid, int stages, bool one) {
+  if (one) launch_dma8k_t<DT, EPI, false>(c, g, grid, stages);
+  else launch_dma8k_t<DT, EPI, true>(c, g, grid, stages);
+}
 static void launch_gemm(tgx_ctx* c, int epi, const ebyte* B_, const ebyte* bias_, float* C, int M, int N, int K, int ldc, bool three_terms = false,
                  const bf16_t* a_hi = nullptr, const bf16_t* a_lo = nullptr, int three_from = 0, int* defer = nullptr, bool a_inter = false) {
   if (defer) *defer = 1;
@@ -151,9 +163,8 @@ static void launch_gemm(tgx_ctx* c, int epi, const ebyte* B_, const ebyte* bias_
   }
   if (store_slab && c->ws_part_bytes >= (size_t)M * N * 4) {
     g.part = c->ws_part; g.nsplit = 1; g.interleave = 0; g.k_per = K;
-    const dim3 g8((N + 127) / 128, (M + 127) / 128, 1), b8(512);
-    const size_t lds8 = (size_t)3 * 3 * 128 * 64 * 2;
-    TGX_DT16_SWITCH(c->dt, if (one_k) hipLaunchKernelGGL((tgx::gemm_dma8k_kernel<DT, tgx::GEMM_PARTIAL, false>), g8, b8, lds8, c->stream, g); else hipLaunchKernelGGL((tgx::gemm_dma8k_kernel<DT, tgx::GEMM_PARTIAL>), g8, b8, lds8, c->stream, g);)
+    const dim3 g8((N + 127) / 128, (M + 127) / 128, 1);
+    TGX_DT16_SWITCH(c->dt, (launch_dma8k<DT, tgx::GEMM_PARTIAL>(c, g, g8, K / 64, one_k));)
     *defer = -1;
     return;
   }
@@ -168,9 +179,8 @@ static void launch_gemm(tgx_ctx* c, int epi, const ebyte* B_, const ebyte* bias_
     // measured (Llama-3.2-1B, ms per prompt, DMA vs register-staged slabs): S = 40 1.61 / 1.79, 48 1.65 / 1.76, 64 1.71 / 1.87; 96 2.08 / 1.99, 128 2.12 / 2.09,
     // 256 2.65 / 2.68; Mistral-7B S = 48 5.40 / 6.23 — the 64-row tile wins, the 128-row one does not: prompts of <= 64 rows only (value 2 = always)
     if (part_8k) {
-      const dim3 g8((N + 127) / 128, (M + 127) / 128, nsplit), b8(512);
-      const size_t lds8 = (size_t)3 * 3 * 128 * 64 * 2;
-      TGX_DT16_SWITCH(c->dt, if (one_k) hipLaunchKernelGGL((tgx::gemm_dma8k_kernel<DT, tgx::GEMM_PARTIAL, false>), g8, b8, lds8, c->stream, g); else hipLaunchKernelGGL((tgx::gemm_dma8k_kernel<DT, tgx::GEMM_PARTIAL>), g8, b8, lds8, c->stream, g);)
+      const dim3 g8((N + 127) / 128, (M + 127) / 128, nsplit);
+      TGX_DT16_SWITCH(c->dt, (launch_dma8k<DT, tgx::GEMM_PARTIAL>(c, g, g8, g.k_per / 64, one_k));)
     }
     const bool dma_part = !part_8k && M <= 64 && (c->gemm_dma & 3) && g.k_per % 64 == 0 && K % 64 == 0;
     if (dma_part) {
@@ -223,9 +233,8 @@ static void launch_gemm(tgx_ctx* c, int epi, const ebyte* B_, const ebyte* bias_
     // wave pairs instead of the four-wave one (option prefill.wide_8k: Llama-3.2-1B S = 256 gate_up 61 us per layer)
     const int t128 = ((N + 127) / 128) * ((M + 127) / 128);
     if ((silu8 || 2 * t128 >= c->num_cus) && (2 * t128 <= c->wide_8k_max * c->num_cus || ragged256)) {
-      const dim3 g8((N + 127) / 128, (M + 127) / 128), b8(512);
-      const size_t lds8 = (size_t)3 * 3 * 128 * 64 * 2;
-      TGX_DT16_SWITCH(c->dt, if (one_k) hipLaunchKernelGGL((tgx::gemm_dma8k_kernel<DT, tgx::GEMM_SILU, false>), g8, b8, lds8, c->stream, g); else hipLaunchKernelGGL((tgx::gemm_dma8k_kernel<DT, tgx::GEMM_SILU>), g8, b8, lds8, c->stream, g);)
+      const dim3 g8((N + 127) / 128, (M + 127) / 128);
+      TGX_DT16_SWITCH(c->dt, (launch_dma8k<DT, tgx::GEMM_SILU>(c, g, g8, K / 64, one_k));)
       return;
     }
   }
@@ -233,11 +242,10 @@ static void launch_gemm(tgx_ctx* c, int epi, const ebyte* B_, const ebyte* bias_
     // N = hidden products whose 128 x 128 tiles number between half a chip and a chip and a half: eight waves per tile, K step split between wave pairs
     const int t128 = ((N + 127) / 128) * ((M + 127) / 128);
     if (2 * t128 >= c->num_cus && 2 * t128 <= 3 * c->num_cus) {
-      const dim3 g8((N + 127) / 128, (M + 127) / 128), b8(512);
-      const size_t lds8 = (size_t)3 * 3 * 128 * 64 * 2;
+      const dim3 g8((N + 127) / 128, (M + 127) / 128);
       TGX_DT16_SWITCH(c->dt,
-        if (epi == tgx::GEMM_RESIDUAL) { if (one_k) hipLaunchKernelGGL((tgx::gemm_dma8k_kernel<DT, tgx::GEMM_RESIDUAL, false>), g8, b8, lds8, c->stream, g); else hipLaunchKernelGGL((tgx::gemm_dma8k_kernel<DT, tgx::GEMM_RESIDUAL>), g8, b8, lds8, c->stream, g); }
-        else { if (one_k) hipLaunchKernelGGL((tgx::gemm_dma8k_kernel<DT, tgx::GEMM_STORE, false>), g8, b8, lds8, c->stream, g); else hipLaunchKernelGGL((tgx::gemm_dma8k_kernel<DT, tgx::GEMM_STORE>), g8, b8, lds8, c->stream, g); })
+        if (epi == tgx::GEMM_RESIDUAL) launch_dma8k<DT, tgx::GEMM_RESIDUAL>(c, g, g8, K / 64, one_k);
+        else launch_dma8k<DT, tgx::GEMM_STORE>(c, g, g8, K / 64, one_k);)
       return;
     }
   }
@@ -480,6 +488,22 @@ int prefill_set_attrs(tgx_ctx* c) {
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_BF16, 128, 1, 2, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_F16, 128, 1, 2, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_F16, 128, 1, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_BF16, tgx::GEMM_SILU, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_BF16, tgx::GEMM_SILU, false>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_BF16, tgx::GEMM_RESIDUAL, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_BF16, tgx::GEMM_RESIDUAL, false>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_BF16, tgx::GEMM_STORE, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_BF16, tgx::GEMM_STORE, false>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_BF16, tgx::GEMM_PARTIAL, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_BF16, tgx::GEMM_PARTIAL, false>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_F16, tgx::GEMM_SILU, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_F16, tgx::GEMM_SILU, false>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_F16, tgx::GEMM_RESIDUAL, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_F16, tgx::GEMM_RESIDUAL, false>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_F16, tgx::GEMM_STORE, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_F16, tgx::GEMM_STORE, false>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_F16, tgx::GEMM_PARTIAL, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_F16, tgx::GEMM_PARTIAL, false>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8k_kernel<tgx::DT_BF16, tgx::GEMM_SILU>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8k_kernel<tgx::DT_F16, tgx::GEMM_SILU>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8k_kernel<tgx::DT_BF16, tgx::GEMM_RESIDUAL>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));

@@ -11,13 +11,14 @@ inline bool slabs_hold_k(int K, int z) { return (z - 1) * slab_steps(K, z) < K /
 // round of whole tiles (160 tiles on 256 CUs: z = 3 -> 2 rounds of a third = 0.67; 128 tiles: z = 2 -> 0.5); taken from 0.8 down (the slabs cost a pass over z x M x N floats).  More
 // than four where all of them run at once and the steps of K that they save (0.6 us each) outweigh their floats (written and read at 5 TB/s): eight / four, ms per prompt,
 // Llama-3.2-1B 133 tokens 2.14 / 2.25, 256 2.28 / 2.39, Qwen2.5-0.5B 256 2.51 / 2.67; with eight in two rounds or for K 2048 at 509 rows and N 1024 it is slower
-// (Qwen3-0.6B 3.53 / 3.45).  Every slab has four steps on average and one at least.
+// (Qwen3-0.6B 3.53 / 3.45).  From 385 rows on the sixth to eighth slab costs its reader more (Qwen3-0.6B, K 3072, eight / as few as that takes: 400 tokens 3.03 / 2.97, 450 3.13 / 2.95,
+// 509 3.22 / 3.08, 600 3.58 / 3.53; 330 2.84 / 2.87).  Every slab has four steps on average and one at least.
 inline int eight_wave_slabs(int M, int N, int K, int num_cus) {
   const int tiles = ((N + 127) / 128) * ((M + 127) / 128);
   int z = 1;
   double best = 0.8001;
   for (int zz = 2; zz <= 8 && tiles < num_cus; zz++) {
-    if (zz > 4 && (zz * tiles > num_cus || K < 6.8e-4 * zz * M * N)) break;
+    if (zz > 4 && (zz * tiles > num_cus || K < (zz > 5 && M > 384 ? 1e-3 : 6.8e-4) * zz * M * N)) break;
     const double cost = (double)((zz * tiles + num_cus - 1) / num_cus) / zz;
     if (cost < best - 1e-9 && K / 64 >= 4 * zz && slabs_hold_k(K, zz)) { best = cost; z = zz; }
   }
@@ -35,5 +36,9 @@ inline bool gate_up_whole(int M, int N, int K, int num_cus, int most) {
   if (M <= 64 || tiles >= num_cus || 2 * tiles > (long long)most * num_cus) return false;
   return K <= 1024 && M > 128 ? 4 * tiles >= num_cus : 2 * tiles > num_cus;
 }
+
+// Whether the eight waves of a 128 x 128 tile divide a stage of K into halves (gemm_dma8h_kernel, both sides' times there) and not into quarters: chains of few stages, which are mostly
+// what stands in front of and behind them.
+inline bool eight_wave_halves(int stages) { return stages <= 32; }
 
 }  // namespace tgx
