@@ -5,7 +5,7 @@
 // ONCE into lines [row][K / 32][32 first terms | 32 second terms] (split_terms_kernel, the norm in front, or the epilogue of the product in front), so that the two terms of a k32 block are one
 // line, weights come as whole k64 lines, and the tiles are those of gemm_dma.h:
 //   256 x 256, eight waves of 64 x 128, a ring of five 32-KB units (gemm_dma8i_kernel's schedule): products that fill the chip with such tiles
-//   128 x 128, eight waves = two row halves x the four k16 steps of a stage, a ring of three 48-KB stages (gemm_dma8k_kernel's): the others
+//   128 x 128, eight waves = two row halves x the four k16 steps of a stage, or quadrants x two of them, a ring of three 48-KB stages (gemm_dma8k_kernel's): the others
 // The products of one output are summed in the same two-term form as before (small term first); only the order of the fp32 sums differs.
 // Dual products (gate and up) take their two matrices in alternate blocks of 32 columns of a tile, so that both values of an output meet in one lane.
 // A last round of tiles that is at most half full is halved over K (SHARED, line_plan.h).
@@ -308,20 +308,24 @@ __global__ __launch_bounds__(512) void stack_line256_kernel(const LineArgs a) {
   }
 }
 
-template <int DT, int EPI, bool DUAL, bool SHARED>
+// HALF: the waves are 2 x 2 quadrants x two halves of a stage's k16 steps, not two row halves x four quarters, for chains of up to 32 stages, as in gemm_dma8h_kernel (gemm_dma.h): the sums
+// meet in the epilogue, with no exchange in front of it.  us quarters / halves: 1999 x 1024 x 512 13.7 / 12.5, K 1024 19.6 / 18.9, K 2048 halved tiles 28.5 / 27.4; 2397 x 2304 x 1024 37.4 /
+// 35.5; 2397 x 8192 x 1024 93.7 / 88.8; 2048 x 2048 x 2048 37.2 / 37.1, K 4096 62.4 / 63.5
+template <int DT, int EPI, bool DUAL, bool SHARED, bool HALF>
 __global__ __launch_bounds__(512) void stack_line128_kernel(const LineArgs a) {
   constexpr int TMN = 128, NS = 3, T_A = TMN * 64, STAGE = 3 * T_A;      // a stage: A lines of two k32 steps | B lines, 128 rows x 128 bytes each
   extern __shared__ __attribute__((aligned(1024))) bf16_t dma_lds[];
   LineTile t;
   if (!line_place<SHARED>(a, TMN, t)) return;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int kq = wv >> 1, wm = wv & 1;                         // k16 step of every stage, row half
+  constexpr int NJ = HALF ? 2 : 4, NSTEP = HALF ? 2 : 1;       // blocks of 32 columns, k16 steps of a stage
+  const int kq = HALF ? wv >> 2 : wv >> 1, wm = HALF ? (wv >> 1) & 1 : wv & 1, wn = HALF ? wv & 1 : 0;      // half or quarter of every stage's k16 steps, row half, column half
   const unsigned lds_base = (unsigned)(size_t)dma_lds;
-  f32x16 acc[2][4];
+  f32x16 acc[2][NJ];
 #pragma unroll
   for (int i = 0; i < 2; i++)
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int j = 0; j < NJ; j++)
 #pragma unroll
       for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
   const int prow = lane >> 3, pslot = lane & 7;
@@ -343,8 +347,8 @@ __global__ __launch_bounds__(512) void stack_line128_kernel(const LineArgs a) {
 #pragma unroll
     for (int q = 0; q < 6; q++) issue_piece(q, 1, 1);
   }
-  const int swz = ((lane & 31) >> 1) & 7, ca = (kq & 1) * 2 + (lane >> 5), cb = kq * 2 + (lane >> 5);
-  bf16x8 fah[2], fal[2], fb[4];
+  const int swz = ((lane & 31) >> 1) & 7;
+  bf16x8 fah[NSTEP][2], fal[NSTEP][2], fb[NSTEP][NJ];
   for (int k = 0; k < nk; k++) {
     if (k + 1 < nk) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");      // stage k landed: only this wave's pieces of stage k + 1 may fly
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -352,55 +356,65 @@ __global__ __launch_bounds__(512) void stack_line128_kernel(const LineArgs a) {
     const bool more = k + 2 < nk;
     const int nst = (k + 2) % NS;
     const bf16_t* st = dma_lds + (size_t)(k % NS) * STAGE;
-    const bf16_t *tA = st + (kq >> 1) * T_A, *tB = st + 2 * T_A;
+    const bf16_t *tA = st + (HALF ? kq : kq >> 1) * T_A, *tB = st + 2 * T_A;
 #pragma unroll
-    for (int j = 0; j < 4; j++) fb[j] = *reinterpret_cast<const bf16x8*>(tB + (j * 32 + (lane & 31)) * 64 + ((cb ^ swz) << 3));
+    for (int s = 0; s < NSTEP; s++) {
+      const int ca = (HALF ? s : kq & 1) * 2 + (lane >> 5), cb = (HALF ? kq * 2 + s : kq) * 2 + (lane >> 5);
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-      const bf16_t* row = tA + (wm * 64 + i * 32 + (lane & 31)) * 64;
-      fah[i] = *reinterpret_cast<const bf16x8*>(row + ((ca ^ swz) << 3));
-      fal[i] = *reinterpret_cast<const bf16x8*>(row + (((4 + ca) ^ swz) << 3));
+      for (int j = 0; j < NJ; j++) fb[s][j] = *reinterpret_cast<const bf16x8*>(tB + (wn * 64 + j * 32 + (lane & 31)) * 64 + ((cb ^ swz) << 3));
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const bf16_t* row = tA + (wm * 64 + i * 32 + (lane & 31)) * 64;
+        fah[s][i] = *reinterpret_cast<const bf16x8*>(row + ((ca ^ swz) << 3));
+        fal[s][i] = *reinterpret_cast<const bf16x8*>(row + (((4 + ca) ^ swz) << 3));
+      }
     }
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int s = 0; s < NSTEP; s++)
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        acc[i][j] = mfma16<DT>(fal[i], fb[j], acc[i][j]);   // small term first
-        acc[i][j] = mfma16<DT>(fah[i], fb[j], acc[i][j]);
-        if (more && (i * 4 + j) < 6) issue_piece(i * 4 + j, k + 2, nst);
-      }
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+          acc[i][j] = mfma16<DT>(fal[s][i], fb[s][j], acc[i][j]);   // small term first
+          acc[i][j] = mfma16<DT>(fah[s][i], fb[s][j], acc[i][j]);
+          const int q = (s * 2 + i) * NJ + j;
+          if (more && q < 6) issue_piece(q, k + 2, nst);
+        }
   }
-  // (q0 + q2) + (q1 + q3): quarters 2, 3 -> LDS -> added by quarters 0, 1 (same row half), whose sums are staged as rows and added by the epilogue, in which all waves take part
+  // halves: both are staged as rows and added by the epilogue.  Quarters: (q0 + q2) + (q1 + q3): quarters 2, 3 -> LDS -> added by quarters 0, 1 (same row half), whose sums are
+  // staged so.  All waves take part in the epilogue
   __builtin_amdgcn_s_barrier();
   float* red = reinterpret_cast<float*>(dma_lds);
-  if (kq >= 2) {
-    float* dst = red + (size_t)(wv - 4) * 8 * 16 * 64;
+  if constexpr (!HALF) {
+    if (kq >= 2) {
+      float* dst = red + (size_t)(wv - 4) * 8 * 16 * 64;
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+      for (int i = 0; i < 2; i++)
 #pragma unroll
-      for (int j = 0; j < 4; j++)
+        for (int j = 0; j < 4; j++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) dst[((i * 4 + j) * 16 + r) * 64 + lane] = acc[i][j][r];
+          for (int r = 0; r < 16; r++) dst[((i * 4 + j) * 16 + r) * 64 + lane] = acc[i][j][r];
+    }
+    __syncthreads();
+    if (kq < 2) {
+      const float* src = red + (size_t)wv * 8 * 16 * 64;
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) acc[i][j][r] += src[((i * 4 + j) * 16 + r) * 64 + lane];
+    }
+    __syncthreads();
   }
-  __syncthreads();
-  if (kq < 2) {
-    const float* src = red + (size_t)wv * 8 * 16 * 64;
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[i][j][r] += src[((i * 4 + j) * 16 + r) * 64 + lane];
-  }
-  __syncthreads();
   if (kq < 2) {
     float* dst = red + (size_t)kq * TMN * LINE_RS;
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
-      for (int j = 0; j < 4; j++)
+      for (int j = 0; j < NJ; j++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) dst[(wm * 64 + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5)) * LINE_RS + j * 32 + (lane & 31)] = acc[i][j][r];
+        for (int r = 0; r < 16; r++) dst[(wm * 64 + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5)) * LINE_RS + wn * 64 + j * 32 + (lane & 31)] = acc[i][j][r];
   }
   __syncthreads();
   if (SHARED && t.rest >= 0) {

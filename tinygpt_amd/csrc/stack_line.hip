@@ -2,6 +2,7 @@
 // beside stack.hip.
 #include "stack.h"
 
+#include "prefill_plan.h"
 #include "kernels/stack_line.h"
 
 namespace {
@@ -10,8 +11,11 @@ void launch_line_t(tgx_ctx* c, const tgx::LineArgs& a, dim3 grid, int tile) {
   if (tile == 256) {
     if (stack_allow_lds(c, (const void*)&tgx::stack_line256_kernel<DT, EPI, DUAL, SHARED>, tgx::LINE256_LDS))
       hipLaunchKernelGGL((tgx::stack_line256_kernel<DT, EPI, DUAL, SHARED>), grid, dim3(512), tgx::LINE256_LDS, c->stream, a);
-  } else if (stack_allow_lds(c, (const void*)&tgx::stack_line128_kernel<DT, EPI, DUAL, SHARED>, tgx::LINE128_LDS))
-    hipLaunchKernelGGL((tgx::stack_line128_kernel<DT, EPI, DUAL, SHARED>), grid, dim3(512), tgx::LINE128_LDS, c->stream, a);
+  } else if (tgx::eight_wave_halves(a.g.K >> 6)) {
+    if (stack_allow_lds(c, (const void*)&tgx::stack_line128_kernel<DT, EPI, DUAL, SHARED, true>, tgx::LINE128_LDS))
+      hipLaunchKernelGGL((tgx::stack_line128_kernel<DT, EPI, DUAL, SHARED, true>), grid, dim3(512), tgx::LINE128_LDS, c->stream, a);
+  } else if (stack_allow_lds(c, (const void*)&tgx::stack_line128_kernel<DT, EPI, DUAL, SHARED, false>, tgx::LINE128_LDS))
+    hipLaunchKernelGGL((tgx::stack_line128_kernel<DT, EPI, DUAL, SHARED, false>), grid, dim3(512), tgx::LINE128_LDS, c->stream, a);
 }
 template <int DT, int EPI, bool DUAL>
 void launch_line_t(tgx_ctx* c, const tgx::LineArgs& a, dim3 grid, int tile) {
