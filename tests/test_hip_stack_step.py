@@ -6,7 +6,10 @@ import numpy as np
 import pytest
 
 import test_hip_keronex as tk
+import test_hip_modepel as tm
+import test_hip_nusovik as tn
 import test_hip_vitudra as tv
+from tinygpt_amd.ffi import GREEDY, SamplerCfg
 
 pytestmark = pytest.mark.gpu
 
@@ -341,3 +344,32 @@ def test_sigmoid_attention_appends_in_its_step(kv_heads, dim, vdim, size, dtype)
     eng.close()
     for i in range(2):
         tz.check(np.stack(got[i]), tz.want_of(cfg, w, toks[i][:starts[i] + 5])[starts[i]:], dtype, f"sequence {i}")
+
+
+# The launch between two greedy steps (kernels/stack_next.h) goes through the logits of a row itself up to 65536 columns and starts from their partials beyond; a slot that was given back, and one
+# that was never taken, ride along.  The same kernels run in steps that are fed those tokens, so that the logits are the same numbers.
+@pytest.mark.parametrize("t,vocab", [(tv, 1), (tv, 67), (tv, 4100), (tv, 32772), (tv, 65536), (tv, 65540), (tm, 67), (tn, 131)])
+def test_between_greedy_steps(t, vocab):
+    cfg = t.config(vocab=vocab)
+    first = [t.tokens(cfg, 3 + i, i) for i in range(3)]
+    eng, _ = t.engine(cfg, seed=5)
+    m = eng.model
+    eng.step([(i, s, [len(s) - 1]) for i, s in enumerate(first)])
+    eng.release(1)
+    start = m.sample(GREEDY)
+    toks = np.concatenate([m.decode(5, GREEDY), m.decode(1, GREEDY)])
+    last, again = m.logits(rounded=False), m.sample(GREEDY)
+    drawn = m.sample(SamplerCfg(temperature=0.7, top_k=1), seed=3)      # the sampler's maximum comes from the partials that the launch left
+    eng.close()
+    eng, _ = t.engine(cfg, seed=5)
+    want = eng.step([(i, s, [len(s) - 1]) for i, s in enumerate(first)])
+    eng.release(1)
+    live, fed = [0, 2], start
+    assert (np.argmax(want, 1)[live] == start[live]).all()
+    for row in toks:
+        want = eng.step([(i, [int(fed[i])], [0]) for i in live])
+        assert (np.argmax(want, 1) == row[live]).all()
+        fed = row
+    assert np.array_equal(last[live], want) and (again[live] == toks[-1][live]).all()
+    assert (drawn[live] == toks[-1][live]).all()
+    eng.close()

@@ -79,6 +79,23 @@ struct FinalizeArgs {
   int n_pos;
 };
 
+// a row's next token into its slot, the rings and the counters (one thread); s_pos: the position it will stand at
+__device__ __forceinline__ void publish_token(const FinalizeArgs& a, int best, int& s_tok, int& s_pos) {
+  const int t = (unsigned)best < (unsigned)a.V ? best : 0;   // all-NaN logits leave the sentinel index: never gather out of the table
+  s_tok = t;
+  *a.tok = t;
+  const int np = *a.pos + (a.advance_pos ? 1 : 0);
+  if (a.advance_pos) *a.pos = np;
+  s_pos = np < a.n_pos ? np : a.n_pos - 1;    // a full context takes no further step: stay inside wpe
+  if (a.log) {
+    const int st = *a.step;
+    a.tok_log[(st % a.log_cap) * a.rows + a.row] = t;
+    if (a.host_ring) a.host_ring[(st % a.ring_cap) * a.rows + a.row] = t;
+    if (a.done) { if (atomicAdd(a.done, 1) == a.done_total - 1) { *a.done = 0; *a.step = st + 1; } }
+    else if (a.bump_step) *a.step = st + 1;
+  }
+}
+
 // the body of the greedy finalize for one row, run by all 256 threads of a workgroup: finalize_greedy_kernel (tgx_sample after a
 // prefill, sampled steps' pick kernel) and the lm_head launch's last-arriving workgroup (greedy decode steps) share it
 template <int DT>
@@ -101,21 +118,7 @@ __device__ __forceinline__ void finalize_row(const FinalizeArgs& a) {
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    const int t = (unsigned)si[0] < (unsigned)a.V ? si[0] : 0;   // all-NaN logits leave the sentinel index: never gather out of the table
-    s_tok = t;
-    *a.tok = t;
-    const int np = *a.pos + (a.advance_pos ? 1 : 0);
-    if (a.advance_pos) *a.pos = np;
-    s_pos = np < a.n_pos ? np : a.n_pos - 1;    // a full context takes no further step: stay inside wpe
-    if (a.log) {
-      const int st = *a.step;
-      a.tok_log[(st % a.log_cap) * a.rows + a.row] = t;
-      if (a.host_ring) a.host_ring[(st % a.ring_cap) * a.rows + a.row] = t;
-      if (a.done) { if (atomicAdd(a.done, 1) == a.done_total - 1) { *a.done = 0; *a.step = st + 1; } }
-      else if (a.bump_step) *a.step = st + 1;
-    }
-  }
+  if (threadIdx.x == 0) publish_token(a, si[0], s_tok, s_pos);
   __syncthreads();
   gather_embedding<DT>(a.embed, s_tok, a.x, a.H, a.wpe, a.wpe ? s_pos : 0);
 }

@@ -130,6 +130,7 @@ struct StackModel {
   size_t part_elems = 0;
   unsigned short *terms = nullptr, *terms2 = nullptr;      // prompt products: the activations as lines of two 16-bit terms, and a feed-forward's hidden values (grown to the largest product seen)
   size_t terms_elems = 0, terms2_elems = 0;
+  bool x_ready = false;                // the step's stream already holds its tokens' embedding rows (greedy decode, kernels/stack_next.h)
   const unsigned short* in_terms = nullptr; size_t in_terms_elems = 0;      // the rows that the last norm wrote as such lines, at the start of terms (nullptr: it did not; norms in front of such products set it anew)
   int *sel = nullptr, *moe_off = nullptr, *perm = nullptr, *ptok = nullptr, *tile_e = nullptr, *tile_m0 = nullptr, *n_tiles = nullptr;
   int max_in = 0, max_hr = 0, max_hv = 0, max_top = 0, max_ff = 0, max_E = 0, max_rank = 0;

@@ -25,6 +25,7 @@
 #include "kernels/stack_latent.h"
 #include "kernels/stack_ssd_mfma.h"
 #include "kernels/stack_hyper.h"
+#include "kernels/stack_next.h"
 
 namespace tgx {
 // A few tokens: the latents into the pool beside the queries into latent space (a product batched over the heads, kernels/stack_few.h): neither needs the other, attention needs both.
@@ -900,7 +901,7 @@ int run_layers_sandwich(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_ke
   const tgx::StepMeta m = step_meta(sm, mp, T, S);
   const int W = sm->d.width, L = sm->d.layers;
   const float eps = sm->d.norm_eps;
-  TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::embed_rows_kernel<DT>, dim3(T), dim3(256), 0, c->stream, m, reinterpret_cast<const tgx::elem_t<DT>*>(c->embed), sm->x, W))
+  if (!sm->x_ready) { TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::embed_rows_kernel<DT>, dim3(T), dim3(256), 0, c->stream, m, reinterpret_cast<const tgx::elem_t<DT>*>(c->embed), sm->x, W)) }
   hipLaunchKernelGGL(tgx::scalar_norm_kernel, dim3(T), dim3(256), 0, c->stream, sm->x, nullptr, sm->norm_g, sm->a, W, eps);
   float *hin = sm->a, *hout = sm->a2;
   for (int li = 0; li < L; li++) {
@@ -1245,7 +1246,7 @@ int run_layers_joint(tgx_ctx* c, const MetaPtrs& mp, int T, int S, int max_keys,
   StackModel* sm = c->stack;
   const tgx::StepMeta m = step_meta(sm, mp, T, S);
   const int W = sm->d.width;
-  TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::embed_rows_kernel<DT>, dim3(T), dim3(256), 0, c->stream, m, reinterpret_cast<const tgx::elem_t<DT>*>(c->embed), sm->x, W))
+  if (!sm->x_ready) { TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::embed_rows_kernel<DT>, dim3(T), dim3(256), 0, c->stream, m, reinterpret_cast<const tgx::elem_t<DT>*>(c->embed), sm->x, W)) }
   for (int li = 0; li < sm->d.layers; li++) {
     StackLayerW& w = sm->L[(size_t)li];
     const tgx_layer_desc& ld = w.d;
@@ -2618,10 +2619,27 @@ void run_logits(tgx_ctx* c, const int* want_dev, int nw, float* C, const int* c_
   launch_gemm(c, g, tgx::SG_STORE, 1);
 }
 
+// most columns of a head whose rows one workgroup each goes through behind a greedy step; more are reduced to partials by a launch in front
+constexpr int NEXT_SCAN = 65536;
 // n rows of logits into the slots rows_dev names, with their argmax partials (src nullptr: the logits stand there already)
 void launch_slot_logits(tgx_ctx* c, const float* src, const int* rows_dev, int n) {
   const int V = c->d.vocab, gx = std::min(c->lm_grid, std::max(1, (V / 4 + 255) / 256));
   hipLaunchKernelGGL(tgx::slot_logits_kernel, dim3(gx, n), dim3(256), 0, c->stream, src, rows_dev, c->slab_logits, V, c->slab_part_val, c->slab_part_idx, c->lm_grid);
+}
+
+// designs whose stream begins as the plain embedding row
+bool next_embeds(const StackModel* sm) { return sm->joint || sm->sandwich; }
+// behind a greedy decode step's logits: every slot's token and the next step's inputs (kernels/stack_next.h)
+void launch_next(tgx_ctx* c, const MetaPtrs& dp, int S) {
+  StackModel* sm = c->stack;
+  tgx::StackNextArgs a{};
+  a.f = make_finalize_args(c, 0, /*advance_pos=*/true, /*log_step=*/true);
+  a.part_stride = c->lm_grid; a.part_val = c->slab_part_val; a.part_idx = c->slab_part_idx;
+  a.logits = c->slab_logits; a.scan = c->d.vocab <= NEXT_SCAN ? 1 : 0;
+  a.tok_id = dp.tok_id; a.tok_pos = dp.tok_pos; a.tok_par = dp.tok_par; a.ent_par = dp.ent_par; a.ent_row = dp.ent_row; a.S = S;
+  a.x = next_embeds(sm) ? sm->x : nullptr; a.W = sm->d.width;
+  if (!a.scan) launch_slot_logits(c, nullptr, dp.want_row, S);
+  TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::stack_next_kernel<DT>, dim3(c->batch), dim3(1024), 0, c->stream, a))
 }
 
 // pages for `tokens` tokens of a slot; the caller has checked that enough are free
@@ -3519,7 +3537,6 @@ int stack_step(tgx_ctx* c, int S, const int32_t* rows, const int32_t* counts, co
 // n decode steps of every live slot: its device-resident current token in, logits into its row, the shared sampler picks the next token
 int stack_decode(tgx_ctx* c, const tgx_sampler_cfg& cfg, uint64_t seed, int n) {
   StackModel* sm = c->stack;
-  const tgx_stack_desc& d = sm->d;
   if (n <= 0) return TGX_OK;
   std::vector<int> live;
   long long need_pages = 0;
@@ -3558,11 +3575,17 @@ int stack_decode(tgx_ctx* c, const tgx_sampler_cfg& cfg, uint64_t seed, int n) {
   c->have_probs = !is_greedy(&cfg);
   for (int s = 0; s < n; s++) {
     if (s == 0) hipLaunchKernelGGL(tgx::stack_gather_tok_kernel, dim3((S + 63) / 64), dim3(64), 0, c->stream, dp.tok_id, dp.ent_row, c->slab_tok, S);
-    if ((rc = run_layers(c, dp, S, S, max_keys + s + 1, 1))) return half_way(c, rc);
+    sm->x_ready = s > 0 && is_greedy(&cfg) && next_embeds(sm);
+    rc = run_layers(c, dp, S, S, max_keys + s + 1, 1);
+    sm->x_ready = false;
+    if (rc) return half_way(c, rc);
     run_logits(c, dp.want, S, c->slab_logits, dp.want_row);
-    launch_slot_logits(c, nullptr, dp.want_row, S);
-    launch_sample(c, 0, c->batch, cfg, /*advance_pos=*/true, /*log_step=*/true);
-    hipLaunchKernelGGL(tgx::stack_advance_kernel, dim3((S + 63) / 64), dim3(64), 0, c->stream, dp.tok_id, dp.ent_row, c->slab_tok, dp.tok_pos, dp.ent_par, dp.tok_par, S);
+    if (is_greedy(&cfg)) launch_next(c, dp, S);
+    else {
+      launch_slot_logits(c, nullptr, dp.want_row, S);
+      launch_sample(c, 0, c->batch, cfg, /*advance_pos=*/true, /*log_step=*/true);
+      hipLaunchKernelGGL(tgx::stack_advance_kernel, dim3((S + 63) / 64), dim3(64), 0, c->stream, dp.tok_id, dp.ent_row, c->slab_tok, dp.tok_pos, dp.ent_par, dp.tok_par, S);
+    }
     c->steps_issued++;
     if (c->launch_fault) return half_way(c, TGX_OK);
   }
