@@ -57,6 +57,32 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const long long* ids, c
   }
 }
 
+// ---- two vectors of four of a row summed over the nsplit slabs of K that a product left, in z order.  Eight (four) slabs of both are on their way at once, past the last one the last
+// again (from L1, not added): a slab after the other was a chain of round trips to L2, and the readers are launches of a row a workgroup that do little else.
+// 509 rows, us: norm of 1024 channels behind five slabs 6.5 -> 5.8; rotation and cache append of 32 heads of 128 behind four 9.6 -> 8.1 (with both halves of a head, the angles and the bias
+// asked for together, and a unit a thread).
+__device__ __forceinline__ void slab_sums(const float* p0, const float* p1, int nsplit, long long slab, f32x4& s0, f32x4& s1) {
+  s0 = f32x4{0.f, 0.f, 0.f, 0.f}; s1 = s0;
+  auto group = [&](auto Nc, int z) {
+    constexpr int N = decltype(Nc)::value;
+    f32x4 a0[N], a1[N];
+#pragma unroll
+    for (int u = 0; u < N; u++) {
+      const size_t at = (size_t)min(z + u, nsplit - 1) * slab;
+      a0[u] = *reinterpret_cast<const f32x4*>(p0 + at); a1[u] = *reinterpret_cast<const f32x4*>(p1 + at);
+    }
+#pragma unroll
+    for (int u = 0; u < N; u++)
+#pragma unroll
+      for (int t = 0; t < 4; t++) { s0[t] += z + u < nsplit ? a0[u][t] : 0.f; s1[t] += z + u < nsplit ? a1[u][t] : 0.f; }
+  };
+  if (nsplit == 1) { group(std::integral_constant<int, 1>{}, 0); return; }
+  if (nsplit == 2) { group(std::integral_constant<int, 2>{}, 0); return; }
+  int z = 0;
+  for (; z + 4 < nsplit; z += 8) group(std::integral_constant<int, 8>{}, z);
+  if (z < nsplit) group(std::integral_constant<int, 4>{}, z);
+}
+
 // ---- row-wise RMSNorm, output as bf16 hi/lo ---------------------------------------------------------------------
 // `lo2` (optional) receives a third term: x = hi + lo + lo2 carries ~24 mantissa bits.  The QKV projection uses it,
 // because its output is the only one that is rounded to bf16 again (the KV cache): with two terms (2^-18) a few
@@ -78,22 +104,8 @@ __global__ __launch_bounds__(256) void rmsnorm_split_kernel(float* X, const bf16
     v0 = *reinterpret_cast<const f32x4*>(x + 8 * c); v1 = *reinterpret_cast<const f32x4*>(x + 8 * c + 4);
     if (part) {
       const float* p = part + (size_t)blockIdx.x * H + 8 * c;
-      f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
-      int z = 0;
-      for (; z + 8 <= nsplit; z += 8) {          // eight slabs in flight together (a batched step has one workgroup per row: the loop was a chain of L2 round trips); summed in z order
-        f32x4 a0[8], a1[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) { a0[u] = *reinterpret_cast<const f32x4*>(p + (size_t)(z + u) * slab); a1[u] = *reinterpret_cast<const f32x4*>(p + (size_t)(z + u) * slab + 4); }
-#pragma unroll
-        for (int u = 0; u < 8; u++)
-#pragma unroll
-          for (int t = 0; t < 4; t++) { s0[t] += a0[u][t]; s1[t] += a1[u][t]; }
-      }
-      for (; z < nsplit; z++) {
-        const f32x4 a0 = *reinterpret_cast<const f32x4*>(p + (size_t)z * slab), a1 = *reinterpret_cast<const f32x4*>(p + (size_t)z * slab + 4);
-#pragma unroll
-        for (int t = 0; t < 4; t++) { s0[t] += a0[t]; s1[t] += a1[t]; }
-      }
+      f32x4 s0, s1;
+      slab_sums(p, p + 4, nsplit, slab, s0, s1);
       if (bias) {
         const u32x4 bv = *reinterpret_cast<const u32x4*>(bias + 8 * c);
 #pragma unroll
@@ -175,51 +187,33 @@ struct RopeKvArgs {
   const int* blk_tbl;      // paged KV (common.h kv_paged_off): this sequence's block table, k_cache / v_cache = the layer's pools — or nullptr
 };
 template <int DT>
-__global__ __launch_bounds__(256) void rope_kv_split_kernel(const RopeKvArgs a) {
+__global__ __launch_bounds__(512) void rope_kv_split_kernel(const RopeKvArgs a) {
   // one workgroup per position; a thread owns FOUR adjacent RoPE pairs (p..p+3, p+half..p+half+3) of one head: 16-byte loads, 8-byte stores
   const int s = blockIdx.x, pos = a.past + s, half = a.hd >> 1, q4 = half >> 2;
   const int qd = a.heads * a.hd, kvd = a.kv_heads * a.hd;
   const float* row = (a.QKV ? a.QKV : a.part) + (size_t)s * (qd + 2 * kvd);
   const int units = (a.heads + 2 * a.kv_heads) * q4;
-  auto fetch4 = [&](int col) {
-    if (a.QKV) return *reinterpret_cast<const f32x4*>(row + col);
-    f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-    int z = 0;
-    for (; z + 8 <= a.nsplit; z += 8) {        // eight slabs in flight together, summed in z order (as rmsnorm_split_kernel)
-      f32x4 t[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) t[u] = *reinterpret_cast<const f32x4*>(row + (size_t)(z + u) * a.slab + col);
-#pragma unroll
-      for (int u = 0; u < 8; u++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) v[e] += t[u][e];
-    }
-    if (z + 4 <= a.nsplit) {
-      f32x4 t[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++) t[u] = *reinterpret_cast<const f32x4*>(row + (size_t)(z + u) * a.slab + col);
-#pragma unroll
-      for (int u = 0; u < 4; u++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) v[e] += t[u][e];
-      z += 4;
-    }
-    for (; z < a.nsplit; z++) {
-      const f32x4 t = *reinterpret_cast<const f32x4*>(row + (size_t)z * a.slab + col);
-#pragma unroll
-      for (int e = 0; e < 4; e++) v[e] += t[e];
-    }
+  auto fetch8 = [&](int c0, int c1, f32x4& v0, f32x4& v1) {
+    if (a.QKV) { v0 = *reinterpret_cast<const f32x4*>(row + c0); v1 = *reinterpret_cast<const f32x4*>(row + c1); return; }
+    u32x2 b0 = {0u, 0u}, b1 = b0;
+    if (a.bias) { b0 = *reinterpret_cast<const u32x2*>(a.bias + c0); b1 = *reinterpret_cast<const u32x2*>(a.bias + c1); }
+    slab_sums(row + c0, row + c1, a.nsplit, a.slab, v0, v1);
     if (a.bias) {
 #pragma unroll
-      for (int e = 0; e < 4; e++) v[e] += elem_to_f32<DT>(a.bias[col + e]);
+      for (int e = 0; e < 2; e++) {
+        v0[2 * e] += pair_lo<DT>(b0[e]); v0[2 * e + 1] += pair_hi<DT>(b0[e]);
+        v1[2 * e] += pair_lo<DT>(b1[e]); v1[2 * e + 1] += pair_hi<DT>(b1[e]);
+      }
     }
-    return v;
   };
   auto pack4 = [](const bf16_t* e) { return u32x2{(unsigned int)e[0] | ((unsigned int)e[1] << 16), (unsigned int)e[2] | ((unsigned int)e[3] << 16)}; };
-  for (int u = threadIdx.x; u < units; u += 256) {
+  for (int u = threadIdx.x; u < units; u += blockDim.x) {
     const int hh = u / q4, p = 4 * (u - hh * q4);
-    f32x4 x0 = fetch4(hh * a.hd + p), x1 = fetch4(hh * a.hd + p + half);
-    if (a.q_norm_w != nullptr && hh < a.heads + a.kv_heads) {
+    const bool turned = hh < a.heads + a.kv_heads;
+    f32x4 cs = {1.f, 1.f, 1.f, 1.f}, sn = {0.f, 0.f, 0.f, 0.f}, x0, x1;      // (asked for in front of the slabs)
+    if (turned) { cs = *reinterpret_cast<const f32x4*>(a.rope_cos + (size_t)pos * half + p); sn = *reinterpret_cast<const f32x4*>(a.rope_sin + (size_t)pos * half + p); }
+    fetch8(hh * a.hd + p, hh * a.hd + p + half, x0, x1);
+    if (a.q_norm_w != nullptr && turned) {
       // AttentionWithQKNorm (Attention.h:156-163): RMSNorm over head_dim; the hd/8 lanes of one head are adjacent and
       // aligned (8 or 16), so the mean of squares is a sub-wave butterfly
       float ss = 0.f;
@@ -234,8 +228,7 @@ __global__ __launch_bounds__(256) void rope_kv_split_kernel(const RopeKvArgs a) 
         x1[t] = elem_to_f32<DT>(w[p + t + half]) * (x1[t] * inv);
       }
     }
-    if (hh < a.heads + a.kv_heads) {
-      const f32x4 cs = *reinterpret_cast<const f32x4*>(a.rope_cos + (size_t)pos * half + p), sn = *reinterpret_cast<const f32x4*>(a.rope_sin + (size_t)pos * half + p);
+    if (turned) {
 #pragma unroll
       for (int t = 0; t < 4; t++) {
         float r0 = x0[t], r1 = x1[t];

@@ -354,7 +354,7 @@ void launch_attn_prefill(tgx_ctx* c, const tgx::AttnPrefillArgs& a_, bool allow_
 }
 // RoPE + cache append + q split of S prompt rows of one batch row
 void launch_rope_kv_split(tgx_ctx* c, const tgx::RopeKvArgs& a, int S) {
-  TGX_DT16_SWITCH(c->dt, hipLaunchKernelGGL(tgx::rope_kv_split_kernel<DT>, dim3(S), dim3(256), 0, c->stream, a))
+  TGX_DT16_SWITCH(c->dt, hipLaunchKernelGGL(tgx::rope_kv_split_kernel<DT>, dim3(S), dim3((a.heads + 2 * a.kv_heads) * (a.hd >> 3) > 256 ? 512 : 256), 0, c->stream, a))
 }
 // RMSNorm of the rows of x into 16-bit terms (ws_ah / ws_al), first adding a pending split-K residual (nsplit > 1: the slabs in ws_part)
 void launch_norm_terms(tgx_ctx* c, float* x, const ebyte* norm_w, int M, int H, int nsplit, bool third) {
