@@ -313,3 +313,20 @@ def test_gate_up_whole_equals_slabs(name, S, dtype):
     assert rel_err(outs[1][0], outs[0][0]) < 2e-5, rel_err(outs[1][0], outs[0][0])
     np.testing.assert_array_equal(outs[1][1], outs[0][1])
     np.testing.assert_array_equal(outs[2][0], outs[0][0])
+
+
+# the QKV product of a bf16 prompt in slabs of the eight-wave tiles, columns from the keys on with a third term: chains of one, four and more stages, a tile that holds queries and keys, the
+# last tile of one row.  What the cache holds are sums rounded to bf16 (2^-9): with three terms (2^-25) and fp32 sums of at most 3072 terms (2^-24 each, some 2^-20 of the result) one entry
+# in a thousand rounds to the other neighbour, with two (2^-17) one in a hundred and more
+@pytest.mark.parametrize("name,S", [("qwen3-0.6b", 129), ("qwen3-0.6b", 384), ("qwen3-0.6b", 509), ("llama-3.2-1b", 133), ("llama-3.2-1b", 257), ("qwen2.5-0.5b", 640), ("wide", 129), ("wide", 255)])
+def test_third_term_in_slabs(name, S):
+    d = copy.deepcopy(known_desc("llama-3.2-1b" if name == "wide" else name, "bf16"))
+    if name == "wide":      # 33 heads: keys begin inside a tile
+        d.hidden, d.heads, d.kv_heads, d.inter = 2112, 33, 3, 2048
+    d.layers, d.vocab, d.max_ctx = 1, 1024, 704
+    m = Model(d, product_backend()).load_synthetic(29, 0.02).finalize()
+    prompt = synth.synth_prompt(d.vocab, S, 6)[None, :]
+    (k1, v1), = run(m, prompt, mfma=True, n_decode=1)[3]
+    (k0, v0), = run(m, prompt, mfma=False, n_decode=1)[3]
+    assert np.mean(k1 != k0) < 3e-3 and np.mean(v1 != v0) < 3e-3, (np.mean(k1 != k0), np.mean(v1 != v0))
+    assert rel_err(k1, k0) < 8e-3 and rel_err(v1, v0) < 8e-3

@@ -799,7 +799,9 @@ __global__ __launch_bounds__(512) void gemm_dma8k_kernel(const GemmArgs a) {
 // all eight waves store: 2.3 us.  The price are twelve fragment reads a stage and wave for eight.  us quarters / halves: 200 x 2048 x 2048 in eight slabs (four stages) 14.5 / 12.1, in
 // four (eight) 15.2 / 12.3; 509 x 1024 x 3072, eight (six) 17.4 / 14.8; 200 x 2048 x 8192, eight (sixteen) 28.0 / 26.8; 300 x 2048 x 8192, five (26) 34.8 / 34.3; 2048 x 2048 x 2048, whole
 // (32) 40.7 / 40.1; 1000 x 2048 x 8192, two (64) 68.4 / 70.1; 2048 x 2048 x 8192, whole (128) 124 / 129: up to 32 stages (prefill_plan.h).
-template <int DT, int EPI, bool LO = true>
+// T3: columns from three_from on take a third term of the activations (the QKV product of a bf16 model).  It comes first, in stages of its own of one A tile beside B and half the matrix
+// work, through the same ring, so that the other columns' tiles cost what they cost without it.
+template <int DT, int EPI, bool LO = true, bool T3 = false>
 __global__ __launch_bounds__(512) void gemm_dma8h_kernel(const GemmArgs a) {
   constexpr int DBK = 64, TMN = 128, NS = 3, STAGE = 3 * TMN * DBK;
   extern __shared__ __attribute__((aligned(1024))) bf16_t dma_lds[];
@@ -837,21 +839,66 @@ __global__ __launch_bounds__(512) void gemm_dma8h_kernel(const GemmArgs a) {
     return *reinterpret_cast<const bf16x8*>(tile + row * DBK + ((kchunk ^ ((row >> 1) & 7)) << 3));
   };
   const int nk = (k_end - k_begin) / DBK;      // (one at least: slabs_hold_k)
-#pragma unroll
-  for (int q = 0; q < 6; q++) issue_piece(q, 0, 0);
-  if (nk > 1) {
-#pragma unroll
-    for (int q = 0; q < 6; q++) issue_piece(q, 1, 1);
-  }
   bf16x8 fah[2][2], fal[2][2], fb[2][2];
+  int base = 0;                                // stages of the ring in front of the loop's own
+  if (T3 && n0 + TMN > a.three_from) {
+    base = nk;
+    const bf16_t* third[2];
+#pragma unroll
+    for (int p = 0; p < 2; p++) third[p] = a.A_lo2 + (gsrc[3 * p] - a.A_hi);
+    auto issue_third = [&](int q, int k, int stage) { if (q % 3 != 1) dma_1k((q % 3 == 0 ? third[q / 3] : gsrc[q]) + k * DBK, lds_base + (unsigned)(stage * STAGE * 2) + ldst[q]); };
+#pragma unroll
+    for (int q = 0; q < 6; q++) issue_third(q, 0, 0);
+    if (nk > 1) {
+#pragma unroll
+      for (int q = 0; q < 6; q++) issue_third(q, 1, 1);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 6; q++) issue_piece(q, 0, 1);
+    }
+    for (int k = 0; k < nk; k++) {
+      if (k + 1 < nk) asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); else asm volatile("s_waitcnt vmcnt(6)" ::: "memory");      // only this wave's pieces of the next stage, the last of them a whole one, may fly
+      __builtin_amdgcn_s_barrier();
+      const bf16_t* st = dma_lds + (size_t)(k % NS) * STAGE;
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        const int kchunk = (kh * 2 + s) * 2 + (lane >> 5);
+#pragma unroll
+        for (int j = 0; j < 2; j++) fb[s][j] = frag(st + 2 * TMN * DBK, wn * 64 + j * 32 + (lane & 31), kchunk);
+#pragma unroll
+        for (int i = 0; i < 2; i++) fah[s][i] = frag(st, wm * 64 + i * 32 + (lane & 31), kchunk);
+      }
+      const int nst = (k + 2) % NS;
+      if (k + 2 < nk) {
+#pragma unroll
+        for (int q = 0; q < 6; q++) issue_third(q, k + 2, nst);
+      } else if (k + 2 < 2 * nk) {
+#pragma unroll
+        for (int q = 0; q < 6; q++) issue_piece(q, k + 2 - nk, nst);
+      }
+#pragma unroll
+      for (int s = 0; s < 2; s++)
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int j = 0; j < 2; j++) acc[i][j] = mfma16<DT>(fah[s][i], fb[s][j], acc[i][j]);
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 6; q++) issue_piece(q, 0, 0);
+    if (nk > 1) {
+#pragma unroll
+      for (int q = 0; q < 6; q++) issue_piece(q, 1, 1);
+    }
+  }
   for (int k = 0; k < nk; k++) {
     // stage k landed: only this wave's pieces of stage k + 1 may fly
     if (k + 1 < nk) { if (LO) asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); else asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); }
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     const bool more = k + 2 < nk;
-    const int nst = (k + 2) % NS;
-    const bf16_t* st = dma_lds + (size_t)(k % NS) * STAGE;
+    const int nst = (base + k + 2) % NS;
+    const bf16_t* st = dma_lds + (size_t)((base + k) % NS) * STAGE;
     const bf16_t *tAh = st, *tAl = st + TMN * DBK, *tB = st + 2 * TMN * DBK;
 #pragma unroll
     for (int s = 0; s < 2; s++) {

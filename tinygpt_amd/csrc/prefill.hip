@@ -72,6 +72,8 @@ static bool gemm_full_lines(const tgx_ctx* c, int epi, int M, int N, int K) {
 template <int DT, int EPI, bool LO>
 static void launch_dma8k_t(tgx_ctx* c, const tgx::GemmArgs& g, dim3 grid, int stages) {
   const size_t lds = (size_t)3 * 3 * 128 * 64 * 2;
+  if constexpr (DT == tgx::DT_BF16 && EPI == tgx::GEMM_PARTIAL && LO)
+    if (g.A_lo2) { hipLaunchKernelGGL((tgx::gemm_dma8h_kernel<DT, EPI, true, true>), grid, dim3(512), lds, c->stream, g); return; }
   if (tgx::eight_wave_halves(stages)) hipLaunchKernelGGL((tgx::gemm_dma8h_kernel<DT, EPI, LO>), grid, dim3(512), lds, c->stream, g);
   else hipLaunchKernelGGL((tgx::gemm_dma8k_kernel<DT, EPI, LO>), grid, dim3(512), lds, c->stream, g);
 }
@@ -120,10 +122,13 @@ static void launch_gemm(tgx_ctx* c, int epi, const ebyte* B_, const ebyte* bias_
   if (c->gemm_splitk && ntiles < c->num_cus && K % tgx::GBK == 0 && !qkv_nosplit && !silu8) nsplit = std::min(std::min(16, ktiles), (2 * c->num_cus + ntiles - 1) / ntiles);
   // N = hidden products of a 129-1500-row prompt (option prefill.splitk_8k): their 128 x 128 tiles number less than a chip (Llama-3.2-1B S = 1024: 128 tiles on 256
   // CUs, 84 us per product against 104 at twice the rows) — the eight-wave LDS-DMA kernel over 2-8 K slabs instead of 64-row register-staged slabs or a half-empty chip
+  // The QKV product of a bf16 model as well (its keys' and values' columns with a third term), while its slabs are half a chip: two to four slabs where the register-staged tiles are four to
+  // fourteen, which the rotation's launch reads.  us a prompt, register-staged / here (slab_sums with it): Qwen3-0.6B 133 tokens 2260 / 2203, 320 2799 / 2639, 509 3030 / 2875, 1000 4606 / 4591;
+  // Llama-3.2-1B 133 2014 / 1911, 256 2172 / 2032, 509 3185 / 3119; Qwen2.5-0.5B 384 tokens 2154 / 2118, 700 3059 / 2970
   bool part_8k = false;
-  if (c->gemm_splitk && c->splitk_8k && (c->gemm_dma & 8) && K % 64 == 0 && !three_terms && (epi == tgx::GEMM_RESIDUAL || epi == tgx::GEMM_STORE) && M > 128) {
+  if (c->gemm_splitk && (c->splitk_8k || three_terms) && (c->gemm_dma & 8) && K % 64 == 0 && (!three_terms || c->dt == tgx::DT_BF16) && !qkv_nosplit && (epi == tgx::GEMM_RESIDUAL || epi == tgx::GEMM_STORE) && M > 128) {
     const int z = tgx::eight_wave_slabs(M, N, K, c->num_cus);
-    if (z >= 2) { part_8k = true; nsplit = z; }
+    if (z >= 2 && (!three_terms || (2 * z * ntiles >= c->num_cus && tgx::eight_wave_halves(tgx::slab_steps(K, z))))) { part_8k = true; nsplit = z; }
   }
   // K >> N (`down`) on 128 x 256 tiles x 2 K slabs: a third fewer operand lines per output than the 128 x 128 kernel, which waits for them (kernels/gemm_dma.h
   // gemm_dma8n_kernel).  Needs a consumer that sums pending slabs (`defer`) and two rounds of workgroups (prefill.wide_n_min, in chips): at one
@@ -488,6 +493,7 @@ int prefill_set_attrs(tgx_ctx* c) {
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_BF16, 128, 1, 2, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_F16, 128, 1, 2, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::attn_prefill_kernel<tgx::DT_F16, 128, 1, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * (64 * 136 + 64 * 160) * 2));
+  HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_BF16, tgx::GEMM_PARTIAL, true, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_BF16, tgx::GEMM_SILU, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_BF16, tgx::GEMM_SILU, false>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
   HIP_OK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&tgx::gemm_dma8h_kernel<tgx::DT_BF16, tgx::GEMM_RESIDUAL, true>), hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 128 * 64 * 2));
