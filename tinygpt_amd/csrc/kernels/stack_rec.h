@@ -51,7 +51,7 @@ __global__ __launch_bounds__(256) void offset_norm_kernel(const float* x, const 
 // the slot's kept row for an entry's first token, zero at position 0.  The kept row is double-buffered with the slot's step parity (the entry's last
 // token writes buffer par ^ 1 while its first reads buffer par).  Grid: (tokens, width / 256).
 // NORM: h is the stream in front of the layer's RMS norm (eps, offset + w), which every workgroup makes for itself: one launch where the norm and the shift were two (a decoded row of
-// 1024 channels: 2.3 + 2.9 us, here 3.9).
+// 1024 channels: 2.3 + 2.9 us, here 3.2; 3.7 with a channel, then a mix, after the other).
 struct TokenShiftArgs {
   const float* h;        // [T][W]
   const float* mu;       // [n][W]
@@ -63,20 +63,34 @@ struct TokenShiftArgs {
 };
 template <bool NORM>
 __global__ __launch_bounds__(256) void token_shift_kernel(StepMeta m, TokenShiftArgs a) {
+  constexpr int MU = 8, RV = 8;      // mixes, and channels a thread of a row's sum, that are on their way at once, the row's and the mixes' in front of what the tables say
   __shared__ float s_now[4], s_before[4];
   const int t = blockIdx.x, c = blockIdx.y * 256 + threadIdx.x;
   if (!NORM && c >= a.W) return;
   const int cc = min(c, a.W - 1);
-  const int i = m.tok_idx[t], cnt = m.tok_cnt[t], pos = m.tok_pos[t], row = m.tok_row[t], par = m.tok_par[t];
   const float* __restrict__ cur = a.h + (size_t)t * a.W;
-  const float* __restrict__ before = i > 0 ? cur - a.W : a.state + (size_t)par * a.state_buf + (size_t)row * a.W;
+  const float* __restrict__ mus = a.mu + cc;
   float* __restrict__ outp = a.out + (size_t)t * a.n * a.W;
-  float x = cur[cc], b = pos == 0 ? 0.f : before[cc];
+  float mu[MU];
+#pragma unroll
+  for (int s = 0; s < MU; s++) mu[s] = mus[(size_t)min(s, a.n - 1) * a.W];
+  float x = cur[cc];
+  const float w = NORM ? a.offset + a.w[cc] : 1.f;
+  auto squares = [&](const float* __restrict__ r, int k0) {
+    float v[RV], ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < RV; k++) v[k] = r[min(k0 + 256 * k, a.W - 1)];
+#pragma unroll
+    for (int k = 0; k < RV; k++) if (k0 + 256 * k < a.W) ss = fmaf(v[k], v[k], ss);
+    return ss;
+  };
+  const int i = m.tok_idx[t], cnt = m.tok_cnt[t], pos = m.tok_pos[t], row = m.tok_row[t], par = m.tok_par[t];
+  const float* __restrict__ before = i > 0 ? cur - a.W : a.state + (size_t)par * a.state_buf + (size_t)row * a.W;
+  float b = pos == 0 ? 0.f : before[cc];
   if constexpr (NORM) {
-    const float w = a.offset + a.w[cc];
     auto factor = [&](const float* r, float* s4) {
       float ss = 0.f;
-      for (int k = threadIdx.x; k < a.W; k += 256) ss = fmaf(r[k], r[k], ss);
+      for (int k0 = threadIdx.x; k0 < a.W; k0 += 256 * RV) ss += squares(r, k0);
       return 1.0f / sqrtf(block_sum_once(ss, s4) / (float)a.W + a.eps);
     };
     x = x * factor(cur, s_now) * w;
@@ -84,7 +98,13 @@ __global__ __launch_bounds__(256) void token_shift_kernel(StepMeta m, TokenShift
     if (c >= a.W) return;
   }
   const float d = b - x;
-  for (int s = 0; s < a.n; s++) outp[(size_t)s * a.W + c] = fmaf(d, a.mu[(size_t)s * a.W + c], x);
+  for (int s0 = 0; s0 < a.n; s0 += MU) {
+    if (s0 > 0)
+#pragma unroll
+      for (int s = 0; s < MU; s++) mu[s] = mus[(size_t)min(s0 + s, a.n - 1) * a.W];
+#pragma unroll
+    for (int s = 0; s < MU; s++) if (s0 + s < a.n) outp[(size_t)(s0 + s) * a.W + c] = fmaf(d, mu[s], x);
+  }
   if (i == cnt - 1) a.state[(size_t)(par ^ 1) * a.state_buf + (size_t)row * a.W + c] = x;
 }
 

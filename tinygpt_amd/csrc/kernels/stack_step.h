@@ -6,16 +6,19 @@
 // The arithmetic is that of the kernels it stands for (stack_rec.h, stack_seq.h), fp32 throughout; sums over the key channels and over a head's outputs meet in another order.
 //
 // Threads: column j = tid & (CP - 1) (CP: vdim rounded up to a power of two), row group tid / CP with DPER rows each.
-// Measured, us a launch in a decoded step's trace (before: the launches that it stands for): one stream, delta rule of 8 heads of 128 x 128 7.4 (convolution 3.9, scan 5.3, norm 2.6),
-// wkv of 16 heads of 64 x 64 with its decays 5.2 (3.8, 4.1, 2.5); sixteen entries, channel decays of 8 heads of 128 x 128 9.7 (5.4, 11.7, 3.3), retention of 4 heads of 128 x 256 with
-// its rotation 9.3 (3.7, 9.3, 3.0; with the inputs held in registers, which spill at 32 rows a lane, 17.5).
+// Measured, us a launch in a decoded step's trace (the launches that it stands for): one stream, wkv of 16 heads of 64 x 64 with its decays 5.2 (3.8, 4.1, 2.5); sixteen entries, channel
+// decays of 8 heads of 128 x 128 8.8 (convolution 5.4, scan 11.7, norm 3.3), retention of 4 heads of 128 x 256 with its rotation 8.8 (3.7, 9.3, 3.0).
+// What bounds it is latency: the launch, the step's tables, the loads that depend on them, three meetings of the waves.  So no load waits for another that it does not depend on: all of them, the state last,
+// are asked for before anything is computed, with clamped places in place of branches.  A convolution's taps one after the other, four slices of a decay's product, and conditional loads, whose registers
+// the compiler waits for where branches meet, were up to ten round trips: channel decays 9.2 -> 8.8, retention 9.4 -> 8.8, a delta rule beside attention 8.9 -> 8.2 (with attention as below).  Eight waves
+// with twice the rows each are no faster (9.6, 8.7; retention's rows do not fit them).
 #pragma once
 #include "stack_rec.h"
 #include "stack_seq.h"
 
 namespace tgx {
 
-constexpr int STEP_MAX_DIM = 256, STEP_MAX_TAPS = 8;
+constexpr int STEP_MAX_DIM = 256, STEP_MAX_TAPS = 8, STEP_THREADS = 1024;
 struct RecStepArgs {
   RecScanArgs s;             // the recurrence (rec_scan_kernel); with prep its a, k, v, beta and g are made here instead
   DeltaPrepArgs p; int prep; // the convolved inputs (delta_prep_kernel)
@@ -27,54 +30,86 @@ struct RecStepArgs {
 
 template <int DT, int KIND, int DPER>
 __device__ __forceinline__ void rec_step_body(const StepMeta& m, const RecStepArgs& a, const int log_cp, const int e, const int h) {
+  constexpr int NT = STEP_THREADS;
   __shared__ __attribute__((aligned(16))) float s_q[STEP_MAX_DIM + 8], s_k[STEP_MAX_DIM + 8], s_w[STEP_MAX_DIM + 8];      // (zeros behind dim)
   __shared__ float s_v[STEP_MAX_DIM], s_b[2], s_n[16], s_unit[2];
-  __shared__ float s_pk[1024], s_po[1024];
+  __shared__ float s_pk[NT], s_po[NT];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int t = e, row = m.tok_row[t], pos = m.tok_pos[t], par = m.tok_par[t];      // (an entry is a token)
   const int dim = a.s.dim, vdim = a.s.vdim, share = a.s.heads / a.s.kv_heads, kh = h / share;
-  const int cp = 1 << log_cp, RG = 1024 >> log_cp, j = tid & (cp - 1), rg = tid >> log_cp, d0 = rg * DPER;
+  const int cp = 1 << log_cp, RG = NT >> log_cp, j = tid & (cp - 1), rg = tid >> log_cp, d0 = rg * DPER;
   const bool col = j < vdim;
+  // What a thread needs beside the state is asked for here, all of it, in front of the state: the first slices of a wkv head's decay product (sixteen lanes a channel, four elements a lane), the
+  // output's gate and norm weight.  (A slice after the other they were four round trips.)
+  const bool mine = tid < vdim;
+  const int out_c = min(tid, vdim - 1);
+  const float* gp = a.g.gate + (size_t)t * a.g.ldg + (size_t)h * vdim;
+  const float gate = gp[out_c], w_out = (a.g.w ? a.g.w + (size_t)h * a.g.w_hstride : gp)[out_c];
+  constexpr bool W2 = KIND == REC_WKV;
+  typename std::conditional<DT == DT_F32, float, unsigned>::type w2r[W2 ? 4 : 1];      // (as they lie in memory: widened where they are used)
+  float lor[W2 ? 4 : 1], w0 = 0.f;
+  auto decay_slices = [&](int c0, int r0) {
+    const size_t at = (size_t)h * dim + min(c0 + (tid >> 4), dim - 1);
+#pragma unroll
+    for (int i = 0; i < (W2 ? 4 : 0); i++) { const int k = min(r0 + (tid & 15) + 16 * i, a.rank - 1); w2r[i] = reinterpret_cast<const elem_t<DT>*>(a.w2)[at * a.rank + k]; lor[i] = a.lora[(size_t)t * a.ldlora + k]; }
+    if (r0 == 0) w0 = a.w0[at];
+  };
+  if (W2 && a.w2) decay_slices(0, 0);
+  // ... and the raw row, taps and tails of a convolved channel (of the last one again in the threads that have none)
+  constexpr bool PREP = KIND == REC_DELTA || KIND == REC_CDELTA;
+  const DeltaPrepArgs& p = a.p;
+  const int GD = p.kv_heads * dim, C = 2 * GD + p.heads * vdim, nb = p.taps - 1, ct = min(tid, 2 * dim + vdim - 1), part = ct < dim ? 0 : ct < 2 * dim ? 1 : 2, cc = ct - part * dim;
+  const int c = part == 0 ? kh * dim + cc : part == 1 ? GD + kh * dim + cc : 2 * GD + h * vdim + cc;
+  const size_t tail = (size_t)row * nb * C + c;
+  float zb = 0.f, za_raw = 0.f, za_bias = 0.f, al = 0.f;
+  if (PREP && a.prep) {
+    const float* pr = p.proj + (size_t)t * p.ldp + p.col0 + p.b_col + h;
+    zb = pr[0];
+    if (p.a_log) { za_raw = pr[p.heads]; za_bias = p.dt_bias[h]; al = p.a_log[h]; }
+  }
+  float x0 = 0.f, cw[PREP ? STEP_MAX_TAPS : 1], old[PREP ? STEP_MAX_TAPS : 1];      // old[d]: the row d positions back
+  if (PREP && a.prep) {
+    x0 = p.proj[(size_t)t * p.ldp + p.col0 + c];
+#pragma unroll
+    for (int d = 0; d < (PREP ? STEP_MAX_TAPS : 0); d++) cw[d] = p.cw[(size_t)c * p.taps + max(nb - d, 0)];
+    if (nb > 0)
+#pragma unroll
+      for (int d = 1; d < (PREP ? STEP_MAX_TAPS : 0); d++) old[d] = p.state[(size_t)par * p.state_buf + tail + (size_t)max(nb - d, 0) * C];
+  }
   float* Sg = a.s.S + ((size_t)row * a.s.heads + h) * (size_t)dim * vdim;
   float S[DPER], ub[KIND == REC_WKV ? DPER : 1];
 #pragma unroll
   for (int dd = 0; dd < DPER; dd++) {
     const int d = d0 + dd;
-    S[dd] = (pos != 0 && d < dim && col) ? Sg[(size_t)d * vdim + j] : 0.f;
-    if (KIND == REC_WKV) ub[dd] = d < dim ? a.s.u[(size_t)h * dim + d] : 0.f;
+    S[dd] = Sg[(size_t)min(d, dim - 1) * vdim + min(j, vdim - 1)];      // (rows and columns that are not there: below)
+    if (KIND == REC_WKV) ub[dd] = a.s.u[(size_t)h * dim + min(d, dim - 1)];
   }
   // ---- the head's inputs
   if (tid < 8) s_q[dim + tid] = s_k[dim + tid] = s_w[dim + tid] = 0.f;
-  if (KIND != REC_WKV && a.prep) {
-    const DeltaPrepArgs& p = a.p;
-    const int GD = p.kv_heads * dim, C = 2 * GD + p.heads * vdim, nb = p.taps - 1;
+  if (PREP && a.prep) {
     if (tid < 2 * dim + vdim) {
-      const int part = tid < dim ? 0 : tid < 2 * dim ? 1 : 2, cc = tid - part * dim, c = part == 0 ? kh * dim + cc : part == 1 ? GD + kh * dim + cc : 2 * GD + h * vdim + cc;
-      const float* st_old = p.state + (size_t)par * p.state_buf + (size_t)row * nb * C + c;
-      float* st_new = p.state + (size_t)(par ^ 1) * p.state_buf + (size_t)row * nb * C + c;
-      const float* cw = p.cw + (size_t)c * p.taps;
-      const float x0 = p.proj[(size_t)t * p.ldp + p.col0 + c];
-      float old[STEP_MAX_TAPS - 1];                                // old[d - 1]: the row d positions back
+      float acc = cw[0] * x0;
 #pragma unroll
-      for (int d = 1; d < STEP_MAX_TAPS; d++) old[d - 1] = d <= nb && pos - d >= 0 ? st_old[(size_t)(nb - d) * C] : 0.f;
-      float acc = cw[nb] * x0;
-#pragma unroll
-      for (int d = 1; d < STEP_MAX_TAPS; d++) if (d <= nb) acc = fmaf(cw[nb - d], old[d - 1], acc);
+      for (int d = 1; d < (PREP ? STEP_MAX_TAPS : 0); d++) {
+        if (d > nb) continue;
+        if (pos - d < 0) old[d] = 0.f;
+        acc = fmaf(cw[d], old[d], acc);
+      }
       const float act = acc / (1.0f + expf(-acc));
       if (part == 0) s_q[cc] = act; else if (part == 1) s_k[cc] = act; else s_v[cc] = act;
       if (nb > 0 && (part == 2 || h == kh * share)) {              // (heads that share keys: the first of them moves the tails)
+        float* st_new = p.state + (size_t)(par ^ 1) * p.state_buf + tail;
         st_new[(size_t)(nb - 1) * C] = x0;
 #pragma unroll
-        for (int d = 1; d < STEP_MAX_TAPS - 1; d++) if (d < nb) st_new[(size_t)(nb - 1 - d) * C] = old[d - 1];
+        for (int d = 1; d < (PREP ? STEP_MAX_TAPS : 0) - 1; d++) if (d < nb) st_new[(size_t)(nb - 1 - d) * C] = old[d];
       }
     }
-    if (tid == 1023) {
-      const float* pr = p.proj + (size_t)t * p.ldp + p.col0;
-      s_b[0] = 1.0f / (1.0f + expf(-pr[p.b_col + h]));
+    if (tid == NT - 1) {
+      const float za = za_raw + za_bias;
+      s_b[0] = 1.0f / (1.0f + expf(-zb));
       if (p.a_log) {
-        const float za = pr[p.b_col + p.heads + h] + p.dt_bias[h];
         const float sp = za > 20.f ? za : log1pf(expf(za));
-        s_b[1] = expf(-expf(p.a_log[h]) * sp);
+        s_b[1] = expf(-expf(al) * sp);
       }
     }
     if (KIND == REC_CDELTA && tid < dim) s_w[tid] = a.s.w[(size_t)t * a.s.ldw + (size_t)h * dim + tid];
@@ -101,21 +136,25 @@ __device__ __forceinline__ void rec_step_body(const StepMeta& m, const RecStepAr
       }
       s_q[tid] = qv; s_k[tid] = kv;
       if ((KIND == REC_CDELTA || KIND == REC_WKV) && !a.w2) s_w[tid] = a.s.w[(size_t)t * a.s.ldw + (size_t)(KIND == REC_WKV ? kh : h) * dim + tid];
-    } else if (tid >= 512 && tid < 512 + vdim) s_v[tid - 512] = a.s.v[(size_t)t * a.s.ldv + (size_t)h * vdim + tid - 512];
-    if (KIND != REC_WKV && tid == 1023) {
+    }
+    if (tid >= NT - vdim) s_v[tid - (NT - vdim)] = a.s.v[(size_t)t * a.s.ldv + (size_t)h * vdim + tid - (NT - vdim)];      // (in other threads than q and k where there are enough)
+    if (KIND != REC_WKV && tid == NT - 1) {
       const size_t at = (size_t)t * a.s.ldg + h;
       if (KIND == REC_SSD && a.s.fixed) { s_b[0] = a.s.beta0; s_b[1] = a.s.fixed[h]; }
       else { s_b[0] = a.s.beta[at]; if (KIND != REC_CDELTA) s_b[1] = a.s.g[at]; }
     }
-    if (KIND == REC_WKV && a.w2) {                                 // sixteen lanes a channel
-      const elem_t<DT>* w2 = reinterpret_cast<const elem_t<DT>*>(a.w2);
-      for (int c0 = 0; c0 < dim; c0 += 64) {
+    if (W2 && a.w2) {
+      for (int c0 = 0; c0 < dim; c0 += NT / 16) {
         const int c = c0 + (tid >> 4);
         float acc = 0.f;
-        for (int r = tid & 15; r < a.rank; r += 16)
-          acc = fmaf(elem_to_f32<DT>(w2[((size_t)h * dim + min(c, dim - 1)) * a.rank + r]), round_storage_if<DT>(a.lora[(size_t)t * a.ldlora + r], a.terms == 1), acc);
+        for (int r0 = 0; r0 < a.rank; r0 += 64) {
+          if (c0 + r0 > 0) decay_slices(c0, r0);
+#pragma unroll
+          for (int i = 0; i < (W2 ? 4 : 0); i++)
+            if (r0 + (tid & 15) + 16 * i < a.rank) acc = fmaf(elem_to_f32<DT>((elem_t<DT>)w2r[i]), round_storage_if<DT>(lor[i], a.terms == 1), acc);
+        }
         acc = row_group_sum<16>(acc);
-        if ((tid & 15) == 0 && c < dim) s_w[c] = expf(-expf(acc + a.w0[(size_t)h * dim + c]));
+        if ((tid & 15) == 0 && c < dim) s_w[c] = expf(-expf(acc + w0));
       }
     }
     if (tid < 2) s_unit[tid] = 1.f;
@@ -135,6 +174,11 @@ __device__ __forceinline__ void rec_step_body(const StepMeta& m, const RecStepAr
     return x;
   };
   float po = 0.f;
+#pragma unroll
+  for (int dd = 0; dd < DPER; dd++) {
+    if (pos == 0 || d0 + dd >= dim || !col) S[dd] = 0.f;
+    if (KIND == REC_WKV && d0 + dd >= dim) ub[dd] = 0.f;
+  }
   if (KIND == REC_WKV) {
 #pragma unroll
     for (int dd = 0; dd < DPER; dd += 4) {
@@ -178,8 +222,6 @@ __device__ __forceinline__ void rec_step_body(const StepMeta& m, const RecStepAr
 #pragma unroll
   for (int dd = 0; dd < DPER; dd++) { const int d = d0 + dd; if (d < dim && col) Sg[(size_t)d * vdim + j] = S[dd]; }
   // the outputs, their norm and gate: one thread a column
-  const bool mine = tid < vdim;
-  const float gate = mine ? a.g.gate[(size_t)t * a.g.ldg + (size_t)h * vdim + tid] : 0.f, w = mine && a.g.w ? a.g.w[(size_t)h * a.g.w_hstride + tid] : 1.f;
   __syncthreads();
   float o = 0.f;
   if (mine) {
@@ -193,20 +235,22 @@ __device__ __forceinline__ void rec_step_body(const StepMeta& m, const RecStepAr
   float ss = 0.f;
   for (int i = 0; i < (vdim + 63) >> 6; i++) ss += s_n[i];
   const float rinv = 1.0f / sqrtf(ss / (float)vdim + a.g.eps), sg = 1.0f / (1.0f + expf(-gate));
-  a.g.out[(size_t)t * a.g.ldo + (size_t)h * vdim + tid] = o * rinv * w * (a.g.silu_gate ? gate * sg : sg);
+  a.g.out[(size_t)t * a.g.ldo + (size_t)h * vdim + tid] = o * rinv * (a.g.w ? w_out : 1.f) * (a.g.silu_gate ? gate * sg : sg);
 }
 
 template <int DT, int KIND, int DPER>
-__global__ __launch_bounds__(1024) void rec_step_kernel(StepMeta m, RecStepArgs a, const int log_cp) { rec_step_body<DT, KIND, DPER>(m, a, log_cp, blockIdx.x, blockIdx.y); }
+__global__ __launch_bounds__(STEP_THREADS) void rec_step_kernel(StepMeta m, RecStepArgs a, const int log_cp) { rec_step_body<DT, KIND, DPER>(m, a, log_cp, blockIdx.x, blockIdx.y); }
 
 // ---- attention of single tokens over up to STEP_MAX_KEYS keys, the token's own among them.  The divided form took three launches for this (append, a walk of key tiles by matrix
-// instructions, merge), the undivided one two, its walk a chain of 1.3 us a tile on a workgroup per key / value head.  Here a workgroup of sixteen waves owns an entry and a key /
-// value head with its (up to four) query heads: it finishes the token's queries, key and value in LDS (gqa_append_kernel) and stores the latter two, then
+// instructions, merge), the undivided one two, its walk a chain of 1.3 us a tile on a workgroup per key / value head.  Here a workgroup of eight waves owns an entry and a
+// query head (those that share a key / value head read its rows from L2): it finishes the token's queries, key and value in LDS (gqa_append_kernel), the first head of a group stores
+// the latter two, then
 //   scores   four keys a wave at a time, sixteen lanes a key with eight channels each; every wave's keys are on their way at once
-//   softmax  a wave per query head, base 2, as in gqa_attn_mfma_kernel (cap, distance slope, sink, mask)
-//   values   a key per wave at a time, a lane's channels of all query heads; the waves' sums meet in LDS
+//   softmax  every wave for itself, base 2, as in gqa_attn_mfma_kernel (cap, distance slope, sink, mask)
+//   values   a key per wave at a time; the waves' sums meet in LDS
 // Queries and probabilities stay fp32 (the matrix forms take them as two 16-bit terms).
-// Measured, us: one stream of 50 to 95 keys, two key / value heads of 128 x 128 7.9 (append 3.0, undivided walk 7.9; 8.4 with the columns of a row found by divisions); beside a delta rule in one launch 9.0 (7.4 of the rule's own).
+// Measured, us: one stream of 50 to 95 keys, eight query heads on two key / value heads of 128 x 128 7.9 (append 3.0, undivided walk 7.9); beside a delta rule in one launch 8.2 (a workgroup of sixteen
+// waves a key / value head 8.0 and 8.9).
 constexpr int STEP_MAX_KEYS = 256, STEP_MAX_GROUP = 4, STEP_MAX_VDIM = 128;
 struct GqaStepArgs {
   GqaAppendArgs ap;          // the token's row (maps 1, no q_hi, no qk_unit_eps)
@@ -217,82 +261,111 @@ struct GqaStepArgs {
   float softcap; int dist_bias;
   const void *poolK, *poolV; // the pools that are read (those of ap where the layer appends)
 };
-template <int DT>
-__device__ __forceinline__ void gqa_step_body(const StepMeta& m, const GqaStepArgs& a, const int e, const int g) {
-  constexpr int MG = STEP_MAX_GROUP, KW = STEP_MAX_KEYS / 16;      // keys of a wave
+template <int DT, int NT>
+__device__ __forceinline__ void gqa_step_body(const StepMeta& m, const GqaStepArgs& a, const int e, const int h) {
+  constexpr int NW = NT / 64, KU = STEP_MAX_KEYS / (4 * NW), VU = STEP_MAX_KEYS / NW;      // turns of a wave over keys (four at a time) and over values
   constexpr float LOG2E = 1.4426950408889634f;
-  __shared__ __attribute__((aligned(16))) float s_qr[MG][STEP_MAX_DIM], s_kn[STEP_MAX_DIM];
-  __shared__ float s_vn[STEP_MAX_VDIM], s_s[MG][STEP_MAX_KEYS], s_l[MG], s_acc[16][MG][STEP_MAX_VDIM];
+  __shared__ __attribute__((aligned(16))) float s_qr[STEP_MAX_DIM], s_kn[STEP_MAX_DIM];
+  __shared__ float s_vn[STEP_MAX_VDIM], s_s[STEP_MAX_KEYS], s_acc[NW][STEP_MAX_VDIM];
   const GqaAppendArgs& ap = a.ap;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int row = m.tok_row[e], pos = m.tok_pos[e], dim = ap.dim, vdim = ap.vdim, Gq = ap.heads / ap.kv_heads;
+  const int row = m.tok_row[e], pos = m.tok_pos[e], dim = ap.dim, vdim = ap.vdim, Gq = ap.heads / ap.kv_heads, g = h / Gq;
   const int lo = first_key(pos, a.mask_kind, a.mask_size), n = pos - lo + 1, kd = ap.kv_heads * dim, vd = ap.kv_heads * vdim;
   const int* tbl = m.tbl + (size_t)row * m.tbl_stride;
   const bool fresh_key = ap.poolK != nullptr;                      // (a layer that reads another layer's pool appends nothing: its last key stands there)
+  const bool appends = fresh_key && h == g * Gq;                   // (one of a group's workgroups stores the token's key and value; all of them make them)
   const int stored = fresh_key ? n - 1 : n, pmask = (1 << m.page_shift) - 1;
   const float* prow = ap.proj + (size_t)e * ap.ldp;
-  // keys and values of this wave, on their way before anything is computed: four keys a turn, sixteen lanes a key; then a key a turn for the values
+  // Everything that a thread needs of the token's row is asked for first, then the pages, all of them, then rows, and values as they lie in memory: a page asked for between two rows, or a value
+  // widened where it is loaded, waits for every load before it.  Keys: four a wave and turn, sixteen lanes a key; values: a key a wave and turn.
+  const int out_c = min(tid, vdim - 1);
+  const float gate = a.gate ? a.gate[(size_t)e * a.ldg + (a.gate_per_head ? (size_t)h : (size_t)h * vdim + out_c)] : 0.f;
+  const int half = ap.rot_dims >> 1, what = wv >> 1;               // waves 0 and 1: the head's queries, 2 and 3: the key, then the value
+  const float* qrow = prow + (what == 0 ? (size_t)h * dim : (size_t)ap.heads * dim + (size_t)g * dim);
+  const bool turns = what == 0 || (what == 1 && fresh_key);
+  float qv[2] = {0.f, 0.f}, qo[2] = {0.f, 0.f}, qc[2] = {1.f, 1.f}, qs[2] = {0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int c = lane + 64 * (wv & 1) + 128 * i;
+    if (!turns || c >= dim) break;
+    qv[i] = qrow[c];
+    if (c < ap.rot_dims) {
+      const int p = ap.rot_pairs ? c >> 1 : c < half ? c : c - half;
+      qo[i] = qrow[ap.rot_pairs ? c ^ 1 : c < half ? c + half : c - half];
+      qc[i] = ap.cs[((size_t)pos * half + p) * 2]; qs[i] = ap.cs[((size_t)pos * half + p) * 2 + 1];
+    }
+  }
+  const int vc = tid - 256;
+  const bool own_v = fresh_key && vc >= 0 && vc < vdim;
+  const size_t vat0 = (size_t)e * vd + (size_t)g * vdim + vc;
+  float own = own_v ? prow[(size_t)ap.heads * dim + kd + (size_t)g * vdim + vc] : 0.f;
+  const float first = own_v && ap.vmode == 2 ? ap.vfirst[vat0] : 0.f, lam = own_v && ap.vmode == 2 ? ap.lam[0] : 0.f;
+  const size_t own_page = appends ? (size_t)tbl[pos >> m.page_shift] : 0;
   const int sub = lane >> 4, ch = 8 * (lane & 15);
   const elem_t<DT>* pK = reinterpret_cast<const elem_t<DT>*>(a.poolK) + (size_t)g * dim;
   const elem_t<DT>* pV = reinterpret_cast<const elem_t<DT>*>(a.poolV) + (size_t)g * vdim;
-  auto slot_of = [&](int i) -> size_t { const int key = lo + min(i, max(stored - 1, 0)); return ((size_t)tbl[key >> m.page_shift] << m.page_shift) + (size_t)(key & pmask); };
-  Slice8<DT> kr[KW / 4][2];
+  auto key_of = [&](int i) { return lo + min(i, max(stored - 1, 0)); };
+  auto slot_of = [&](int page, int i) -> size_t { return ((size_t)page << m.page_shift) + (size_t)(key_of(i) & pmask); };
+  int kat[KU], vat[VU];
 #pragma unroll
-  for (int u = 0; u < KW / 4; u++) {
-    const int i = 4 * (wv + 16 * u) + sub;
-    if (64 * u >= n) break;                                        // (uniform)
-    const elem_t<DT>* kp = pK + slot_of(i) * kd;
+  for (int u = 0; u < KU; u++) { if (4 * NW * u >= n) break; kat[u] = tbl[key_of(4 * (wv + NW * u) + sub) >> m.page_shift]; }      // (uniform; past the last key: the last one's again)
+#pragma unroll
+  for (int u = 0; u < VU; u++) { if (NW * u >= n) break; vat[u] = tbl[key_of(wv + NW * u) >> m.page_shift]; }
+  __builtin_amdgcn_sched_barrier(0);
+  Slice8<DT> kr[KU][2];
+#pragma unroll
+  for (int u = 0; u < KU; u++) {
+    if (4 * NW * u >= n) break;
+    const elem_t<DT>* kp = pK + slot_of(kat[u], 4 * (wv + NW * u) + sub) * kd;
 #pragma unroll
     for (int c = 0; c < 2; c++) if (128 * c < dim) kr[u][c] = load_slice<DT>(kp + min(ch + 128 * c, dim - 8), 0);
   }
-  float vr[KW][2];
+  typename std::conditional<DT == DT_F32, float, unsigned>::type vr[VU][2];      // (a register each: packed in pairs they would be waited for)
 #pragma unroll
-  for (int u = 0; u < KW; u++) {
-    if (16 * u >= n) break;
-    const elem_t<DT>* vp = pV + slot_of(wv + 16 * u) * vd;
-#pragma unroll
-    for (int c = 0; c < 2; c++) vr[u][c] = 64 * c < vdim ? elem_to_f32<DT>(vp[min(lane + 64 * c, vdim - 1)]) : 0.f;
+  for (int u = 0; u < VU; u++) {
+    if (NW * u >= n) break;
+    const elem_t<DT>* vp = pV + slot_of(vat[u], wv + NW * u) * vd;
+    vr[u][0] = vp[min(lane, vdim - 1)];
+    if (vdim > 64) vr[u][1] = vp[min(lane + 64, vdim - 1)];
   }
   // the token's queries (score scale and log2 e folded in), key and value
   const bool capped = a.softcap > 0.f;
   const float temp = ap.q_temp_coef != 0.f ? fmaf(ap.q_temp_coef, logf((float)((pos + 1) / ap.q_temp_every) + 1.0f), 1.0f) : 1.0f, qscale = capped ? a.scale : a.scale * LOG2E;
-  const int nq = Gq + (fresh_key ? 1 : 0);
-  if (wv < 2 * nq)                                                 // two waves a row
-    for (int c = lane + 64 * (wv & 1); c < dim; c += 128) {
-      const int r = wv >> 1;
-      const float* u = prow + (r < Gq ? (size_t)(g * Gq + r) * dim : (size_t)ap.heads * dim + (size_t)g * dim);
-      float v = u[c];
+  if (turns) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int c = lane + 64 * (wv & 1) + 128 * i;
+      if (c >= dim) break;
+      float v = qv[i];
       if (c < ap.rot_dims) {
-        const int half = ap.rot_dims >> 1, p = ap.rot_pairs ? c >> 1 : c < half ? c : c - half;
-        const bool first = ap.rot_pairs ? (c & 1) == 0 : c < half;
-        const float cs = ap.cs[((size_t)pos * half + p) * 2], sn = ap.cs[((size_t)pos * half + p) * 2 + 1], o = u[ap.rot_pairs ? c ^ 1 : first ? c + half : c - half];
-        v = first ? __fsub_rn(__fmul_rn(v, cs), __fmul_rn(o, sn)) : __fadd_rn(__fmul_rn(v, cs), __fmul_rn(o, sn));
+        const bool first_half = ap.rot_pairs ? (c & 1) == 0 : c < half;
+        v = first_half ? __fsub_rn(__fmul_rn(v, qc[i]), __fmul_rn(qo[i], qs[i])) : __fadd_rn(__fmul_rn(v, qc[i]), __fmul_rn(qo[i], qs[i]));
       }
-      if (r < Gq) s_qr[r][c] = v * temp * qscale;
+      if (what == 0) s_qr[c] = v * temp * qscale;
       else {
         const elem_t<DT> k = f32_to_elem<DT>(v);
-        reinterpret_cast<elem_t<DT>*>(ap.poolK)[(((size_t)tbl[pos >> m.page_shift] << m.page_shift) + (size_t)(pos & pmask)) * kd + (size_t)g * dim + c] = k;
+        if (appends) reinterpret_cast<elem_t<DT>*>(ap.poolK)[((own_page << m.page_shift) + (size_t)(pos & pmask)) * kd + (size_t)g * dim + c] = k;
         s_kn[c] = elem_to_f32<DT>(k);
       }
     }
-  if (fresh_key && tid < vdim) {
-    const size_t at = (size_t)e * vd + (size_t)g * vdim + tid;
-    float v = prow[(size_t)ap.heads * dim + kd + (size_t)g * vdim + tid];
-    if (ap.vmode == 1) ap.vfirst[at] = v;
-    if (ap.vmode == 2) { const float lam = ap.lam[0]; v = fmaf(lam, ap.vfirst[at], __fmul_rn(1.0f - lam, v)); }
-    const elem_t<DT> sv = f32_to_elem<DT>(v);
-    const size_t pg = (size_t)tbl[pos >> m.page_shift];
-    reinterpret_cast<elem_t<DT>*>(ap.poolV)[((pg << m.page_shift) + (size_t)(pos & pmask)) * vd + (size_t)g * vdim + tid] = sv;
-    if (ap.poolVT) reinterpret_cast<elem_t<DT>*>(ap.poolVT)[((pg * vd + (size_t)g * vdim + tid) << m.page_shift) + (size_t)(pos & pmask)] = sv;
-    s_vn[tid] = elem_to_f32<DT>(sv);
+  }
+  if (own_v) {
+    if (ap.vmode == 1 && appends) ap.vfirst[vat0] = own;
+    if (ap.vmode == 2) own = fmaf(lam, first, __fmul_rn(1.0f - lam, own));
+    const elem_t<DT> sv = f32_to_elem<DT>(own);
+    if (appends) {
+      reinterpret_cast<elem_t<DT>*>(ap.poolV)[((own_page << m.page_shift) + (size_t)(pos & pmask)) * vd + (size_t)g * vdim + vc] = sv;
+      if (ap.poolVT) reinterpret_cast<elem_t<DT>*>(ap.poolVT)[((own_page * vd + (size_t)g * vdim + vc) << m.page_shift) + (size_t)(pos & pmask)] = sv;
+    }
+    s_vn[vc] = elem_to_f32<DT>(sv);
   }
   __syncthreads();
   // scores
 #pragma unroll
-  for (int u = 0; u < KW / 4; u++) {
-    if (64 * u >= n) break;
-    const int i = 4 * (wv + 16 * u) + sub;
-    float sc[MG] = {0.f, 0.f, 0.f, 0.f};
+  for (int u = 0; u < KU; u++) {
+    if (4 * NW * u >= n) break;
+    const int i = 4 * (wv + NW * u) + sub;
+    float sc = 0.f;
 #pragma unroll
     for (int c = 0; c < 2; c++) {
       if (128 * c >= dim) break;
@@ -304,81 +377,69 @@ __device__ __forceinline__ void gqa_step_body(const StepMeta& m, const GqaStepAr
         for (int x = 0; x < 8; x++) k[x] = s_kn[min(at + x, dim - 1)];
       }
       if (at < dim) {
+        const f32x4 q0 = *reinterpret_cast<const f32x4*>(&s_qr[at]), q1 = *reinterpret_cast<const f32x4*>(&s_qr[at + 4]);
 #pragma unroll
-        for (int r = 0; r < MG; r++) {
-          const f32x4 q0 = *reinterpret_cast<const f32x4*>(&s_qr[min(r, Gq - 1)][at]), q1 = *reinterpret_cast<const f32x4*>(&s_qr[min(r, Gq - 1)][at + 4]);
-#pragma unroll
-          for (int x = 0; x < 8; x++) sc[r] = fmaf(k[x], x < 4 ? q0[x & 3] : q1[x & 3], sc[r]);
-        }
+        for (int x = 0; x < 8; x++) sc = fmaf(k[x], x < 4 ? q0[x & 3] : q1[x & 3], sc);
       }
     }
-#pragma unroll
-    for (int r = 0; r < MG; r++) { sc[r] = row_group_sum<16>(sc[r]); if ((lane & 15) == r && r < Gq && i < n) s_s[r][i] = sc[r]; }
+    sc = row_group_sum<16>(sc);
+    if ((lane & 15) == 0 && i < n) s_s[i] = sc;
   }
   __syncthreads();
-  if (wv < Gq) {
-    const int h = g * Gq + wv;
-    const float slope2 = a.dist_bias ? distance_slope(h, ap.heads) * LOG2E : 0.f;
-    float s[STEP_MAX_KEYS / 64], mx = a.has_sink ? a.sink * LOG2E : -INFINITY, l = 0.f;
+  // softmax: every wave for itself, keys lane, lane + 64, ..
+  const float slope2 = a.dist_bias ? distance_slope(h, ap.heads) * LOG2E : 0.f;
+  float p[STEP_MAX_KEYS / 64], mx = a.has_sink ? a.sink * LOG2E : -INFINITY, l = 0.f;
 #pragma unroll
-    for (int u = 0; u < STEP_MAX_KEYS / 64; u++) {
-      const int i = lane + 64 * u;
-      float v = i < n ? s_s[wv][i] : -INFINITY;
-      if (capped && i < n) v = a.softcap * tanhf(v / a.softcap) * LOG2E;
-      s[u] = i < n ? fmaf(-slope2, (float)(n - 1 - i), v) : -INFINITY;
-      mx = fmaxf(mx, s[u]);
-    }
-    mx = group_max<64>(mx);
-    const bool dead = mx == -INFINITY;
-#pragma unroll
-    for (int u = 0; u < STEP_MAX_KEYS / 64; u++) { const float p = dead ? 0.f : __builtin_amdgcn_exp2f(s[u] - mx); l += p; if (lane + 64 * u < n) s_s[wv][lane + 64 * u] = p; }
-    l = wave_sum(l);
-    if (a.has_sink) l += __builtin_amdgcn_exp2f(a.sink * LOG2E - mx);
-    if (lane == 0) s_l[wv] = l;
+  for (int u = 0; u < STEP_MAX_KEYS / 64; u++) {
+    p[u] = -INFINITY;
+    if (64 * u >= n) continue;                                     // (uniform)
+    const int i = lane + 64 * u;
+    float v = i < n ? s_s[i] : -INFINITY;
+    if (capped && i < n) v = a.softcap * tanhf(v / a.softcap) * LOG2E;
+    p[u] = i < n ? fmaf(-slope2, (float)(n - 1 - i), v) : -INFINITY;
+    mx = fmaxf(mx, p[u]);
   }
-  __syncthreads();
+  mx = group_max<64>(mx);
+  const bool dead = mx == -INFINITY;
+#pragma unroll
+  for (int u = 0; u < STEP_MAX_KEYS / 64; u++) { p[u] = dead ? 0.f : __builtin_amdgcn_exp2f(p[u] - mx); l += p[u]; }
+  l = wave_sum(l);
+  if (a.has_sink) l += __builtin_amdgcn_exp2f(a.sink * LOG2E - mx);
   // values
-  float acc[MG][2];
+  float acc[2] = {0.f, 0.f};
 #pragma unroll
-  for (int r = 0; r < MG; r++) acc[r][0] = acc[r][1] = 0.f;
-#pragma unroll
-  for (int u = 0; u < KW; u++) {
-    if (16 * u >= n) break;
-    const int i = wv + 16 * u;
+  for (int u = 0; u < VU; u++) {
+    if (NW * u >= n) break;
+    const int i = wv + NW * u;
     if (i >= n) break;                                             // (wave-uniform)
-    const bool own = fresh_key && i == n - 1;
-    const float v0 = own ? s_vn[min(lane, vdim - 1)] : vr[u][0], v1 = own ? s_vn[min(lane + 64, vdim - 1)] : vr[u][1];
-#pragma unroll
-    for (int r = 0; r < MG; r++) { const float p = s_s[min(r, Gq - 1)][i]; acc[r][0] = fmaf(p, v0, acc[r][0]); acc[r][1] = fmaf(p, v1, acc[r][1]); }
+    const float w = __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(p[NW * u / 64]), i & 63));      // (NW divides 64)
+    const bool last = fresh_key && i == n - 1;
+    acc[0] = fmaf(w, last ? s_vn[min(lane, vdim - 1)] : elem_to_f32<DT>((elem_t<DT>)vr[u][0]), acc[0]);
+    if (vdim > 64) acc[1] = fmaf(w, last ? s_vn[min(lane + 64, vdim - 1)] : elem_to_f32<DT>((elem_t<DT>)vr[u][1]), acc[1]);
   }
-#pragma unroll
-  for (int r = 0; r < MG; r++)
-#pragma unroll
-    for (int c = 0; c < 2; c++) if (lane + 64 * c < STEP_MAX_VDIM) s_acc[wv][r][lane + 64 * c] = acc[r][c];
+  s_acc[wv][lane] = acc[0]; s_acc[wv][lane + 64] = acc[1];
   __syncthreads();
-  const int r = tid >> 7, c = tid & 127;                           // (STEP_MAX_VDIM columns a head)
-  if (r < Gq && c < vdim) {
-    const size_t hc = (size_t)(g * Gq + r) * vdim + c;
-    float t[16];
+  if (tid < vdim) {
+    float t[NW];
 #pragma unroll
-    for (int w = 0; w < 16; w++) t[w] = s_acc[w][r][c];
+    for (int w = 0; w < NW; w++) t[w] = s_acc[w][tid];
 #pragma unroll
-    for (int o = 8; o > 0; o >>= 1)
+    for (int o = NW / 2; o > 0; o >>= 1)
 #pragma unroll
       for (int w = 0; w < o; w++) t[w] += t[w + o];
-    float v = s_l[r] > 0.f ? t[0] / s_l[r] : 0.f;
-    if (a.gate) v = v / (1.0f + expf(-a.gate[(size_t)e * a.ldg + (a.gate_per_head ? (size_t)(g * Gq + r) : hc)]));
-    a.out[(size_t)e * a.ldo + hc] = v * a.out_scale;
+    float v = l > 0.f ? t[0] / l : 0.f;
+    if (a.gate) v = v / (1.0f + expf(-gate));
+    a.out[(size_t)e * a.ldo + (size_t)h * vdim + tid] = v * a.out_scale;
   }
 }
 template <int DT>
-__global__ __launch_bounds__(1024) void gqa_step_kernel(StepMeta m, GqaStepArgs a) { gqa_step_body<DT>(m, a, blockIdx.x, blockIdx.y); }
+__global__ __launch_bounds__(512) void gqa_step_kernel(StepMeta m, GqaStepArgs a) { gqa_step_body<DT, 512>(m, a, blockIdx.x, blockIdx.y); }
 
-// both halves of a parallel mixer (attention beside a delta rule) in one launch: grid (entries, key / value heads of the one + heads of the other)
+// both halves of a parallel mixer (attention beside a delta rule) in one launch: grid (entries, heads of the one + heads of the other)
 template <int DT, int DPER>
-__global__ __launch_bounds__(1024) void parallel_step_kernel(StepMeta m, GqaStepArgs a, RecStepArgs r, const int log_cp) {
-  if ((int)blockIdx.y < a.ap.kv_heads) gqa_step_body<DT>(m, a, blockIdx.x, blockIdx.y);
-  else rec_step_body<DT_F32, REC_DELTA, DPER>(m, r, log_cp, blockIdx.x, blockIdx.y - a.ap.kv_heads);
+__global__ __launch_bounds__(STEP_THREADS) void parallel_step_kernel(StepMeta m, GqaStepArgs a, RecStepArgs r, const int log_cp) {
+  if ((int)blockIdx.y < a.ap.heads) gqa_step_body<DT, STEP_THREADS>(m, a, blockIdx.x, blockIdx.y);
+  else rec_step_body<DT_F32, REC_DELTA, DPER>(m, r, log_cp, blockIdx.x, blockIdx.y - a.ap.heads);
 }
 
 }  // namespace tgx

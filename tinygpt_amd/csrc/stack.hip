@@ -679,7 +679,7 @@ int run_gqa_core(tgx_ctx* c, const tgx::StepMeta& m, const GqaSpec& sp_, int T, 
   GqaSpec sp = sp_;
   tgx::GqaStepArgs sa{};
   if (gqa_step(sm, sp, max_keys, max_count, sa)) {
-    TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::gqa_step_kernel<DT>, dim3(S, sp.kv_heads), dim3(1024), 0, c->stream, m, sa))
+    TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::gqa_step_kernel<DT>, dim3(S, sp.heads), dim3(512), 0, c->stream, m, sa))
     return TGX_OK;
   }
   if (sp.maps == 2) { sp.out = sp_.map_out; sp.ldo = (long long)sp.heads * sp.vdim; }
@@ -1222,7 +1222,7 @@ int run_parallel(tgx_ctx* c, const tgx::StepMeta& m, StackLayerW& w, JointLayer&
   const RecStepPlan sp1 = rec_step_plan(c, st, max_count);
   tgx::GqaStepArgs sa{};
   if (jl.merged && sp1.ok && sp1.dper <= 16 && gqa_step(sm, sp, max_keys, max_count, sa)) {      // both halves' outputs stay until the layer's sum: one launch for the two
-    const dim3 grid(S, G + rH);
+    const dim3 grid(S, ld.heads + rH);
     TGX_DT_SWITCH(c->dt,
       if (sp1.dper <= 4) hipLaunchKernelGGL((tgx::parallel_step_kernel<DT, 4>), grid, dim3(1024), 0, c->stream, m, sa, st, sp1.log_cp);
       else if (sp1.dper <= 8) hipLaunchKernelGGL((tgx::parallel_step_kernel<DT, 8>), grid, dim3(1024), 0, c->stream, m, sa, st, sp1.log_cp);
