@@ -19,6 +19,7 @@
 // Measured against the vector form (us, medians of a step's launches, bf16): sixteen rows 2 x 3072 x 1024 19.0 -> 8.5, 32000 x 1024 82 -> 24; eight rows 2 x 8192 x 2048 35 -> 20,
 // 2048 x 8192 26 -> 14; four rows 2 x 8192 x 2048 22.7 -> 19.8 (3.4 TB/s), 2048 x 8192 13.0 -> 14.2; against the 64-wide tiles, 47 rows: 2 x 3072 x 1024 27 -> 17, 1024 x 3072 42 -> 20.
 #pragma once
+#include "args_ahead.h"
 #include "gemm_dma.h"
 #include "stack_gemm.h"
 
@@ -48,8 +49,8 @@ __device__ __forceinline__ void stack_few_body(const StackGemmArgs& a, const int
   extern __shared__ __attribute__((aligned(1024))) unsigned char few_lds[];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
   const int li = lane & 15, q = lane >> 4;                          // row (column) of the operands, quarter of a half step's k
-  const int n0 = blockIdx.x * 16, steps = (a.K + 63) >> 6;
-  if (n0 >= a.N) return;                                            // (the narrower product of a pair)
+  const int n0 = blockIdx.x * 16, N = args_ahead(a.N, a, (int)blockDim.x), steps = (a.K + 63) >> 6;
+  if (n0 >= N) return;                                            // (the narrower product of a pair)
   unsigned char* ring = few_lds + (size_t)wv * depth * STEP;
   const unsigned ring_lds = (unsigned)(size_t)ring;
 
@@ -62,7 +63,7 @@ __device__ __forceinline__ void stack_few_body(const StackGemmArgs& a, const int
   for (int b = 0; b < NB; b++)
 #pragma unroll
     for (int p = 0; p < WP; p++)
-      wsrc[b][p] = reinterpret_cast<const elem_t<DT>*>(b ? a.B2 : a.B) + (size_t)z * a.b_zstride + (size_t)min(n0 + p * WROWS + lane / (64 / WROWS), a.N - 1) * a.ldb;
+      wsrc[b][p] = reinterpret_cast<const elem_t<DT>*>(b ? a.B2 : a.B) + (size_t)z * a.b_zstride + (size_t)min(n0 + p * WROWS + lane / (64 / WROWS), N - 1) * a.ldb;
 #pragma unroll
   for (int i = 0; i < MB; i++)
 #pragma unroll
@@ -188,7 +189,7 @@ __device__ __forceinline__ void stack_few_body(const StackGemmArgs& a, const int
 template <int DT, int EPI, bool DUAL, int MB, int XP>
 __global__ __launch_bounds__(64 * few_max_waves(MB)) void stack_few_kernel(const StackGemmArgs a, const int depth) {
   int z = blockIdx.z, m0 = blockIdx.y * 16 * MB, rows_end = a.M;
-  if (a.z_off) {
+  if (args_ahead(a.z_off, a, (int)blockDim.x)) {
     if ((int)blockIdx.y >= *a.n_tiles) return;
     z = a.tile_z[blockIdx.y]; m0 = a.tile_m0[blockIdx.y]; rows_end = a.z_off[z + 1];
   }

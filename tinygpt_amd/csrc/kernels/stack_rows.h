@@ -18,6 +18,7 @@
 // 2 x 2048 x 2048 15.6 (18.4; 4.3 TB/s), 2048 x 2048 10.0 (11.3).
 // Any N and pairs; K a multiple of 8, 16-byte aligned rows (launch_gemm's condition).
 #pragma once
+#include "args_ahead.h"
 #include "stack_gemm.h"
 
 namespace tgx {
@@ -35,8 +36,9 @@ __global__ __launch_bounds__(64 * ROWS_MAX_WAVES, 3) void stack_rows_kernel(cons
   extern __shared__ __attribute__((aligned(16))) float s_sum[];     // rows_lds()
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
   // the pairs of this workgroup's expert: blockIdx.y is the expert, or, where there are fewer pairs than experts, a pair that stands for its expert if none before it does
-  const int c0 = lane < a.n_pairs ? a.sel[lane] : -1, c1 = lane + 64 < a.n_pairs ? a.sel[lane + 64] : -1;
-  const bool by_pair = a.n_pairs < a.experts;
+  const int n_pairs = args_ahead(a.n_pairs, a, (int)blockDim.x);
+  const int c0 = lane < n_pairs ? a.sel[lane] : -1, c1 = lane + 64 < n_pairs ? a.sel[lane + 64] : -1;
+  const bool by_pair = n_pairs < a.experts;
   const int y = blockIdx.y, z = by_pair ? __builtin_amdgcn_readlane(y < 64 ? c0 : c1, y & 63) : y;
   if (z >= a.experts) return;                                       // (an identity output: no product)
   const unsigned long long m0 = __ballot(c0 == z), m1 = __ballot(c1 == z);
