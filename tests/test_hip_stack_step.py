@@ -373,3 +373,15 @@ def test_between_greedy_steps(t, vocab):
     assert np.array_equal(last[live], want) and (again[live] == toks[-1][live]).all()
     assert (drawn[live] == toks[-1][live]).all()
     eng.close()
+
+
+# a dense feed-forward's PolyNorm: rows of fours up to 8192 channels stay in registers, others pass through memory; prompts and single tokens.  fp32 sums over the row: 1e-4 as in the design's tests
+@pytest.mark.parametrize("ff", [1, 3, 4, 1020, 1022, 1024, 1028, 8188, 8192, 8196])
+def test_poly_norm_rows(ff):
+    cfg = tm.config([tm.rec(tm.dense(ff)), tm.rec(tm.dense(ff))])
+    eng, w = tm.engine(cfg, seed=ff)
+    toks = tm.tokens(cfg, 6, ff)
+    got = np.concatenate([eng.step([(0, toks[:4], [0, 1, 2, 3])])] + [eng.step([(0, toks[i:i + 1], [0])]) for i in (4, 5)])
+    want = tm.want_of(cfg, w, toks)
+    eng.close()
+    assert np.abs(got - want).max() / np.abs(want).max() < 1e-4
