@@ -346,8 +346,8 @@ def test_sigmoid_attention_appends_in_its_step(kv_heads, dim, vdim, size, dtype)
         tz.check(np.stack(got[i]), tz.want_of(cfg, w, toks[i][:starts[i] + 5])[starts[i]:], dtype, f"sequence {i}")
 
 
-# The launch between two greedy steps (kernels/stack_next.h) goes through the logits of a row itself up to 65536 columns and starts from their partials beyond; a slot that was given back, and one
-# that was never taken, ride along.  The same kernels run in steps that are fed those tokens, so that the logits are the same numbers.
+# The launch between two greedy steps (kernels/stack_next.h): heads of one column, of fewer and of more than there are partials; a slot that was given back, and one that was never taken, ride
+# along.  The same kernels run in steps that are fed those tokens, so that the logits are the same numbers.
 @pytest.mark.parametrize("t,vocab", [(tv, 1), (tv, 67), (tv, 4100), (tv, 32772), (tv, 65536), (tv, 65540), (tm, 67), (tn, 131)])
 def test_between_greedy_steps(t, vocab):
     cfg = t.config(vocab=vocab)

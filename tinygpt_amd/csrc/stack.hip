@@ -2619,8 +2619,6 @@ void run_logits(tgx_ctx* c, const int* want_dev, int nw, float* C, const int* c_
   launch_gemm(c, g, tgx::SG_STORE, 1);
 }
 
-// most columns of a head whose rows one workgroup each goes through behind a greedy step; more are reduced to partials by a launch in front
-constexpr int NEXT_SCAN = 65536;
 // n rows of logits into the slots rows_dev names, with their argmax partials (src nullptr: the logits stand there already)
 void launch_slot_logits(tgx_ctx* c, const float* src, const int* rows_dev, int n) {
   const int V = c->d.vocab, gx = std::min(c->lm_grid, std::max(1, (V / 4 + 255) / 256));
@@ -2634,11 +2632,10 @@ void launch_next(tgx_ctx* c, const MetaPtrs& dp, int S) {
   StackModel* sm = c->stack;
   tgx::StackNextArgs a{};
   a.f = make_finalize_args(c, 0, /*advance_pos=*/true, /*log_step=*/true);
-  a.part_stride = c->lm_grid; a.part_val = c->slab_part_val; a.part_idx = c->slab_part_idx;
-  a.logits = c->slab_logits; a.scan = c->d.vocab <= NEXT_SCAN ? 1 : 0;
+  a.part_stride = c->lm_grid;
   a.tok_id = dp.tok_id; a.tok_pos = dp.tok_pos; a.tok_par = dp.tok_par; a.ent_par = dp.ent_par; a.ent_row = dp.ent_row; a.S = S;
   a.x = next_embeds(sm) ? sm->x : nullptr; a.W = sm->d.width;
-  if (!a.scan) launch_slot_logits(c, nullptr, dp.want_row, S);
+  launch_slot_logits(c, nullptr, dp.want_row, S);
   TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::stack_next_kernel<DT>, dim3(c->batch), dim3(1024), 0, c->stream, a))
 }
 
