@@ -282,6 +282,43 @@ def test_eight_wave_tiles_in_halves(heads, inter, dtype, S):
         assert rel_err(k1, k0) < ulp and rel_err(v1, v0) < ulp
 
 
+# A stage's four k16 steps keep sums of their own, (0 + 2) + (1 + 3) at the end, whichever waves have them.  Weights of one large number in step 0 of every stage, its negative in step 2 and
+# small multiples of 1/8 in steps 1 and 3, on an activation row of one value: sums of 0 and 2 cancel to nothing, those of 1 and 3 are exact to 2^-20; where 0 and 1 shared a sum, the large
+# numbers (2^15 a stage) took the small ones' last bits, 1e-3 of the result and more.  What remains is a hidden value stored as two 16-bit terms (2^-17) through one product.
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("S", [129, 300])
+@pytest.mark.parametrize("which", ["up", "down"])
+def test_steps_of_a_stage_keep_their_own_sums(which, S, dtype):
+    d = copy.deepcopy(known_desc("llama-3.2-1b", dtype))
+    d.hidden, d.heads, d.kv_heads, d.inter, d.layers, d.vocab, d.max_ctx, d.tied = 1024, 16, 4, 2048, 1, 1024, 320, False
+    rng = np.random.default_rng(3)
+    w = {n: np.zeros(s, np.float32) for n, s in d.tensor_shapes().items()}
+    for n in w:
+        if "norm" in n:
+            w[n][:] = 1
+    w["model.embed_tokens.weight"][:] = 1
+    w["lm_head.weight"][:] = np.eye(1024)
+    gate, up, down = (w["model.layers.0.mlp.%s_proj.weight" % n] for n in ("gate", "up", "down"))
+    gate[:, 0] = up[:, 0] = 1
+    down[:, :1024] = np.eye(1024)
+    m = up if which == "up" else down
+    m[:] = rng.integers(-8, 9, m.shape) / 8
+    k = np.arange(m.shape[1]) % 64
+    m[:, (k < 16) | ((k >= 32) & (k < 48))] = 0
+    m[:, k == 0], m[:, k == 32] = 2.0 ** 15, -2.0 ** 15
+    gpu = Model(d, product_backend())
+    for n, v in w.items():
+        gpu.upload(n, v)
+    gpu.finalize()
+    gpu.set_option("prefill.mfma", 1)
+    gpu.forward(rng.integers(0, 1024, S)[None, :])
+    x = 1 / np.sqrt(1 + np.float64(d.norm_eps))
+    g, u = gate.astype(np.float64).sum(1) * x, up.astype(np.float64).sum(1) * x
+    y = 1 + down.astype(np.float64) @ (g / (1 + np.exp(-g)) * u)
+    want = y / np.sqrt((y * y).mean() + d.norm_eps)
+    assert rel_err(gpu.logits(rounded=False)[0], want) < 5e-5
+
+
 # N = hidden products whose steps of 64 do not fill six or seven slabs (25 and 29 steps; tests/test_prefill_plan.py has the rule): the counts that do are taken.  Bound as above
 @pytest.mark.parametrize("heads,S,dtype", [(25, 129, "bf16"), (25, 245, "fp16"), (29, 200, "bf16"), (29, 131, "fp16")])
 def test_products_that_fill_no_six_slabs(heads, S, dtype):

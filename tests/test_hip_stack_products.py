@@ -168,6 +168,28 @@ def test_prompt_products_of_experts_weighted_at_their_input(T, experts, top, ff,
     assert np.quantile(rows, 15 / 16) < 1e-4, (T, dtype, rows)
 
 
+# The steps of a stage keep sums of their own on the 128 x 128 tiles too (tests/test_hip_prefill.py has the same of the flat families' kernel): every token the same row of one value, the
+# head's rows a large number in step 0 of a stage, its negative in step 2, small ones in steps 1 and 3
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+def test_steps_of_a_stage_keep_their_own_sums(dtype):
+    W, V, T = 1024, 4096, 300
+    rng = np.random.default_rng(4)
+    d = wkv_model(W, 64, dtype, T)
+    d.vocab = V
+    w = {n: np.zeros(s, np.float32) for n, s in d.tensor_shapes().items()}
+    w["embed"][:] = 1
+    head = rng.integers(-8, 9, (V, W)) / 8
+    k = np.arange(W) % 64
+    head[:, (k < 16) | ((k >= 32) & (k < 48))] = 0
+    head[:, k == 0], head[:, k == 32] = 2.0 ** 15, -2.0 ** 15
+    w["head"][:] = head
+    eng = SlotEngine(desc=d, tensors=w)
+    got = eng.step([("p", rng.integers(0, V, T), list(range(T)))], ["p"])
+    eng.close()
+    want = head.sum(1) / np.sqrt(1 + 1e-5)
+    assert np.abs(got - want).max() / np.abs(want).max() < 1e-5
+
+
 # Tiles of a last, at most half full round as two halves of K (line_plan.h): width 1024, 6208 hidden values and 1700 tokens halve 87 tiles of 256 x 256 (16 steps of K; rows that end
 # inside) and 112 of 128 x 128 (97 steps: uneven halves); experts of 2112 hidden values halve what their plan leaves over.  Against whole tiles only the order of fp32 sums differs
 # (1e-4 as above); a pass repeats itself bit for bit, whichever half comes first.

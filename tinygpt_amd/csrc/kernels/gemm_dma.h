@@ -796,7 +796,9 @@ __global__ __launch_bounds__(512) void gemm_dma8k_kernel(const GemmArgs a) {
 // ---- the same tile, waves = 2 x 2 quadrants x TWO k halves of every stage, for short chains of stages (K slabs, K up to 2048) ------------------------
 // A launch of few stages is what stands around its loop: the quarters above meet in 384 KB of LDS traffic over three barriers, half of the waves idle from the first on, and four waves store
 // a tile four bytes a lane: 5.7 of the 14.5 us of 200 x 2048 x 2048 in eight slabs (2.1 to the first stage, 0.83 a stage).  Two halves exchange a quarter of that over one barrier and
-// all eight waves store: 2.3 us.  The price are twelve fragment reads a stage and wave for eight.  us quarters / halves: 200 x 2048 x 2048 in eight slabs (four stages) 14.5 / 12.1, in
+// all eight waves store: 2.3 us.  A half is the k16 steps kh and kh + 2, each with a sum of its own until the loop is over, so that an output is the same number as above, bit for bit (in
+// one sum for both the chains were twice as long: Llama-3.2-1B fp16 300 tokens 1.03 +- 0.02 of the error against 64 bits, Zaluvik's two requests 1.06 +- 0.02); it costs 64 registers
+// (198 of 256) and no time.  The price are twelve fragment reads a stage and wave for eight.  us quarters / halves: 200 x 2048 x 2048 in eight slabs (four stages) 14.5 / 12.1, in
 // four (eight) 15.2 / 12.3; 509 x 1024 x 3072, eight (six) 17.4 / 14.8; 200 x 2048 x 8192, eight (sixteen) 28.0 / 26.8; 300 x 2048 x 8192, five (26) 34.8 / 34.3; 2048 x 2048 x 2048, whole
 // (32) 40.7 / 40.1; 1000 x 2048 x 8192, two (64) 68.4 / 70.1; 2048 x 2048 x 8192, whole (128) 124 / 129: up to 32 stages (prefill_plan.h).
 // T3: columns from three_from on take a third term of the activations (the QKV product of a bf16 model).  It comes first, in stages of its own of one A tile beside B and half the matrix
@@ -811,13 +813,15 @@ __global__ __launch_bounds__(512) void gemm_dma8h_kernel(const GemmArgs a) {
   xcd_tile(a, tile_m, tile_n);
   const int m0 = tile_m * TMN, n0 = tile_n * TMN;
   const unsigned lds_base = (unsigned)(size_t)dma_lds;
-  f32x16 acc[2][2];
+  f32x16 acc[2][2][2];                         // [k16 step of a stage: kh, kh + 2]
 #pragma unroll
-  for (int i = 0; i < 2; i++)
+  for (int s = 0; s < 2; s++)
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int i = 0; i < 2; i++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[s][i][j][r] = 0.f;
 
   const int prow = lane >> 3, pslot = lane & 7;
   const int k_begin = EPI == GEMM_PARTIAL ? (int)blockIdx.z * a.k_per : 0;
@@ -862,7 +866,7 @@ __global__ __launch_bounds__(512) void gemm_dma8h_kernel(const GemmArgs a) {
       const bf16_t* st = dma_lds + (size_t)(k % NS) * STAGE;
 #pragma unroll
       for (int s = 0; s < 2; s++) {
-        const int kchunk = (kh * 2 + s) * 2 + (lane >> 5);
+        const int kchunk = (kh + 2 * s) * 2 + (lane >> 5);
 #pragma unroll
         for (int j = 0; j < 2; j++) fb[s][j] = frag(st + 2 * TMN * DBK, wn * 64 + j * 32 + (lane & 31), kchunk);
 #pragma unroll
@@ -881,7 +885,7 @@ __global__ __launch_bounds__(512) void gemm_dma8h_kernel(const GemmArgs a) {
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
-          for (int j = 0; j < 2; j++) acc[i][j] = mfma16<DT>(fah[s][i], fb[s][j], acc[i][j]);
+          for (int j = 0; j < 2; j++) acc[s][i][j] = mfma16<DT>(fah[s][i], fb[s][j], acc[s][i][j]);
     }
   } else {
 #pragma unroll
@@ -902,7 +906,7 @@ __global__ __launch_bounds__(512) void gemm_dma8h_kernel(const GemmArgs a) {
     const bf16_t *tAh = st, *tAl = st + TMN * DBK, *tB = st + 2 * TMN * DBK;
 #pragma unroll
     for (int s = 0; s < 2; s++) {
-      const int kchunk = (kh * 2 + s) * 2 + (lane >> 5);      // this wave's k16 steps of the stage
+      const int kchunk = (kh + 2 * s) * 2 + (lane >> 5);      // this wave's k16 steps of the stage
 #pragma unroll
       for (int j = 0; j < 2; j++) fb[s][j] = frag(tB, wn * 64 + j * 32 + (lane & 31), kchunk);
 #pragma unroll
@@ -918,14 +922,20 @@ __global__ __launch_bounds__(512) void gemm_dma8h_kernel(const GemmArgs a) {
       for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-          if (LO) acc[i][j] = mfma16<DT>(fal[s][i], fb[s][j], acc[i][j]);   // small term first
-          acc[i][j] = mfma16<DT>(fah[s][i], fb[s][j], acc[i][j]);
+          if (LO) acc[s][i][j] = mfma16<DT>(fal[s][i], fb[s][j], acc[s][i][j]);   // small term first
+          acc[s][i][j] = mfma16<DT>(fah[s][i], fb[s][j], acc[s][i][j]);
           const int q = s * 4 + i * 2 + j;
           if (more && q < 6) issue_piece(q, k + 2, nst);            // one DMA per two MFMAs
         }
   }
 
-  // a wave hands the other half's wave the column block that that one finishes (kh 0: j 0, kh 1: j 1); first half + second half on both sides
+  // the wave's two quarters; then it hands the other half's wave the column block that that one finishes (kh 0: j 0, kh 1: j 1): (q0 + q2) + (q1 + q3) on both sides
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[0][i][j][r] += acc[1][i][j][r];
   __builtin_amdgcn_s_barrier();                               // every wave is done with the ring
   float* red = reinterpret_cast<float*>(dma_lds);
   auto give = [&](auto J) {                                   // (constant block indices: a run-time one would send the accumulators to scratch memory)
@@ -933,7 +943,7 @@ __global__ __launch_bounds__(512) void gemm_dma8h_kernel(const GemmArgs a) {
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) dst[(i * 16 + r) * 64] = acc[i][J.value][r];
+      for (int r = 0; r < 16; r++) dst[(i * 16 + r) * 64] = acc[0][i][J.value][r];
   };
   if (kh == 0) give(std::integral_constant<int, 1>{}); else give(std::integral_constant<int, 0>{});
   __syncthreads();
@@ -944,7 +954,7 @@ __global__ __launch_bounds__(512) void gemm_dma8h_kernel(const GemmArgs a) {
 #pragma unroll
     for (int r = 0; r < 16; r++) {
       const float o = other[(i * 16 + r) * 64];
-      fin[i][r] = kh == 0 ? acc[i][0][r] + o : o + acc[i][1][r];
+      fin[i][r] = kh == 0 ? acc[0][i][0][r] + o : o + acc[0][i][1][r];
     }
   const int col = n0 + wn * 64 + kh * 32 + (lane & 31), row0 = m0 + wm * 64;
   if constexpr (EPI == GEMM_SILU) {

@@ -309,7 +309,7 @@ __global__ __launch_bounds__(512) void stack_line256_kernel(const LineArgs a) {
 }
 
 // HALF: the waves are 2 x 2 quadrants x two halves of a stage's k16 steps, not two row halves x four quarters, for chains of up to 32 stages, as in gemm_dma8h_kernel (gemm_dma.h): the sums
-// meet in the epilogue, with no exchange in front of it.  us quarters / halves: 1999 x 1024 x 512 13.7 / 12.5, K 1024 19.6 / 18.9, K 2048 halved tiles 28.5 / 27.4; 2397 x 2304 x 1024 37.4 /
+// meet in the epilogue, with no exchange in front of it.  Each k16 step has a sum of its own, as there: the same numbers either way.  us quarters / halves: 1999 x 1024 x 512 13.7 / 12.5, K 1024 19.6 / 18.9, K 2048 halved tiles 28.5 / 27.4; 2397 x 2304 x 1024 37.4 /
 // 35.5; 2397 x 8192 x 1024 93.7 / 88.8; 2048 x 2048 x 2048 37.2 / 37.1, K 4096 62.4 / 63.5
 template <int DT, int EPI, bool DUAL, bool SHARED, bool HALF>
 __global__ __launch_bounds__(512) void stack_line128_kernel(const LineArgs a) {
@@ -321,13 +321,15 @@ __global__ __launch_bounds__(512) void stack_line128_kernel(const LineArgs a) {
   constexpr int NJ = HALF ? 2 : 4, NSTEP = HALF ? 2 : 1;       // blocks of 32 columns, k16 steps of a stage
   const int kq = HALF ? wv >> 2 : wv >> 1, wm = HALF ? (wv >> 1) & 1 : wv & 1, wn = HALF ? wv & 1 : 0;      // half or quarter of every stage's k16 steps, row half, column half
   const unsigned lds_base = (unsigned)(size_t)dma_lds;
-  f32x16 acc[2][NJ];
+  f32x16 acc[NSTEP][2][NJ];                                    // (halves: steps kq and kq + 2)
 #pragma unroll
-  for (int i = 0; i < 2; i++)
+  for (int s = 0; s < NSTEP; s++)
 #pragma unroll
-    for (int j = 0; j < NJ; j++)
+    for (int i = 0; i < 2; i++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+      for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[s][i][j][r] = 0.f;
   const int prow = lane >> 3, pslot = lane & 7;
   const bf16_t* gsrc[6];
   unsigned ldst[6];
@@ -356,10 +358,11 @@ __global__ __launch_bounds__(512) void stack_line128_kernel(const LineArgs a) {
     const bool more = k + 2 < nk;
     const int nst = (k + 2) % NS;
     const bf16_t* st = dma_lds + (size_t)(k % NS) * STAGE;
-    const bf16_t *tA = st + (HALF ? kq : kq >> 1) * T_A, *tB = st + 2 * T_A;
+    const bf16_t* tB = st + 2 * T_A;
 #pragma unroll
     for (int s = 0; s < NSTEP; s++) {
-      const int ca = (HALF ? s : kq & 1) * 2 + (lane >> 5), cb = (HALF ? kq * 2 + s : kq) * 2 + (lane >> 5);
+      const bf16_t* tA = st + (HALF ? s : kq >> 1) * T_A;
+      const int ca = (kq & 1) * 2 + (lane >> 5), cb = (kq + 2 * s) * 2 + (lane >> 5);
 #pragma unroll
       for (int j = 0; j < NJ; j++) fb[s][j] = *reinterpret_cast<const bf16x8*>(tB + (wn * 64 + j * 32 + (lane & 31)) * 64 + ((cb ^ swz) << 3));
 #pragma unroll
@@ -375,17 +378,24 @@ __global__ __launch_bounds__(512) void stack_line128_kernel(const LineArgs a) {
       for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
-          acc[i][j] = mfma16<DT>(fal[s][i], fb[s][j], acc[i][j]);   // small term first
-          acc[i][j] = mfma16<DT>(fah[s][i], fb[s][j], acc[i][j]);
+          acc[s][i][j] = mfma16<DT>(fal[s][i], fb[s][j], acc[s][i][j]);   // small term first
+          acc[s][i][j] = mfma16<DT>(fah[s][i], fb[s][j], acc[s][i][j]);
           const int q = (s * 2 + i) * NJ + j;
           if (more && q < 6) issue_piece(q, k + 2, nst);
         }
   }
-  // halves: both are staged as rows and added by the epilogue.  Quarters: (q0 + q2) + (q1 + q3): quarters 2, 3 -> LDS -> added by quarters 0, 1 (same row half), whose sums are
-  // staged so.  All waves take part in the epilogue
+  // (q0 + q2) + (q1 + q3).  Halves: q0 + q2 and q1 + q3 lie in one wave, are staged as rows and added by the epilogue.  Quarters: 2, 3 -> LDS -> added by 0, 1 (same row half), whose
+  // sums are staged so.  All waves take part in the epilogue
   __builtin_amdgcn_s_barrier();
   float* red = reinterpret_cast<float*>(dma_lds);
-  if constexpr (!HALF) {
+  if constexpr (HALF) {
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[0][i][j][r] += acc[1][i][j][r];
+  } else {
     if (kq >= 2) {
       float* dst = red + (size_t)(wv - 4) * 8 * 16 * 64;
 #pragma unroll
@@ -393,7 +403,7 @@ __global__ __launch_bounds__(512) void stack_line128_kernel(const LineArgs a) {
 #pragma unroll
         for (int j = 0; j < 4; j++)
 #pragma unroll
-          for (int r = 0; r < 16; r++) dst[((i * 4 + j) * 16 + r) * 64 + lane] = acc[i][j][r];
+          for (int r = 0; r < 16; r++) dst[((i * 4 + j) * 16 + r) * 64 + lane] = acc[0][i][j][r];
     }
     __syncthreads();
     if (kq < 2) {
@@ -403,7 +413,7 @@ __global__ __launch_bounds__(512) void stack_line128_kernel(const LineArgs a) {
 #pragma unroll
         for (int j = 0; j < 4; j++)
 #pragma unroll
-          for (int r = 0; r < 16; r++) acc[i][j][r] += src[((i * 4 + j) * 16 + r) * 64 + lane];
+          for (int r = 0; r < 16; r++) acc[0][i][j][r] += src[((i * 4 + j) * 16 + r) * 64 + lane];
     }
     __syncthreads();
   }
@@ -414,7 +424,7 @@ __global__ __launch_bounds__(512) void stack_line128_kernel(const LineArgs a) {
 #pragma unroll
       for (int j = 0; j < NJ; j++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) dst[(wm * 64 + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5)) * LINE_RS + wn * 64 + j * 32 + (lane & 31)] = acc[i][j][r];
+        for (int r = 0; r < 16; r++) dst[(wm * 64 + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5)) * LINE_RS + wn * 64 + j * 32 + (lane & 31)] = acc[0][i][j][r];
   }
   __syncthreads();
   if (SHARED && t.rest >= 0) {
