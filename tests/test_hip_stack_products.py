@@ -191,7 +191,7 @@ def test_steps_of_a_stage_keep_their_own_sums(dtype):
 
 
 # Tiles of a last, at most half full round as two halves of K (line_plan.h): width 1024, 6208 hidden values and 1700 tokens halve 87 tiles of 256 x 256 (16 steps of K; rows that end
-# inside) and 112 of 128 x 128 (97 steps: uneven halves); experts of 2112 hidden values halve what their plan leaves over.  Against whole tiles only the order of fp32 sums differs
+# inside) and 112 of 128 x 128 (97 steps: uneven halves).  Against whole tiles only the order of fp32 sums differs
 # (1e-4 as above); a pass repeats itself bit for bit, whichever half comes first.
 @pytest.mark.parametrize("dtype", ["bf16", "fp16"])
 @pytest.mark.parametrize("T", [1700, 1537])
@@ -212,19 +212,19 @@ def test_halved_tiles(T, dtype):
     assert np.abs(halved[0] - whole).max() / np.abs(whole).max() < 1e-4, (T, dtype)
 
 
+# ... and experts' tiles stay whole: their rows stand in any order (the plan takes them as they come), so that a row that is summed in halves in one pass would be summed whole in the next
 @pytest.mark.parametrize("T,experts,top", [(2100, 5, 2), (700, 3, 1)])
-def test_halved_tiles_of_experts(T, experts, top):
+def test_experts_tiles_stay_whole(T, experts, top):
     import test_hip_keronex as tk
     layer = tk.ret(tk.moe(experts, top, 2112, 2112), heads=4, dim=32, vdim=64, decay=[0.875, 0.99, 0.5, 0.9])
     cfg = tk.config([layer, layer], width=1024)
     eng, _ = tk.engine(cfg, "bf16", max_seqs=1, max_ctx=T, budget_tokens=T + 64)
     ids, want = np.array(tk.tokens(cfg, T)), sorted({*range(0, T, 17), 127, 128, T - 1})
-    halved = [eng.step([("p", ids, want)], ["p"]) for _ in range(3)]
+    passes = [eng.step([("p", ids, want)], ["p"]) for _ in range(3)]
     eng.model.set_option("stack.line_share", 0)
     whole = eng.step([("p", ids, want)], ["p"])
     eng.close()
-    assert (halved[0] == halved[1]).all() and (halved[0] == halved[2]).all() and not (halved[0] == whole).all()
-    assert np.quantile(np.abs(halved[0] - whole).max(1) / np.abs(whole).max(), 15 / 16) < 1e-4, T      # (a near tie of the router)
+    assert all((p == whole).all() for p in passes)
 
 
 @pytest.mark.parametrize("vocab", [53, 96, 1028, 1030])

@@ -8,7 +8,8 @@
 //   128 x 128, eight waves = two row halves x the four k16 steps of a stage, or quadrants x two of them, a ring of three 48-KB stages (gemm_dma8k_kernel's): the others
 // The products of one output are summed in the same two-term form as before (small term first); only the order of the fp32 sums differs.
 // Dual products (gate and up) take their two matrices in alternate blocks of 32 columns of a tile, so that both values of an output meet in one lane.
-// A last round of tiles that is at most half full is halved over K (SHARED, line_plan.h).
+// A last round of tiles that is at most half full is halved over K (SHARED, line_plan.h); not in grouped products, whose plan deals an expert's rows to its tiles in any order: a row
+// would be summed whole in one pass and in halves in the next.
 // Tiles are dealt to the XCDs in contiguous runs, each run walked eight row tiles at a time: an XCD's workgroups share row blocks and weight tiles in its L2.
 #pragma once
 #include "../line_plan.h"
@@ -64,7 +65,7 @@ struct LineTile { int z, mbase, mend, tn, k0, nk, rest; };      // its steps of 
 template <bool SHARED>
 __device__ __forceinline__ bool line_place(const LineArgs& a, int TM, LineTile& t) {
   int tm;
-  const int id = (int)blockIdx.x, gm = a.g.z_off ? min(a.gm, *a.g.n_tiles) : a.gm, nk = a.g.K >> 6;
+  const int id = (int)blockIdx.x, gm = !SHARED && a.g.z_off ? min(a.gm, *a.g.n_tiles) : a.gm, nk = a.g.K >> 6;
   const LineShare sh = SHARED ? line_share(gm * a.gn, TM, nk, a.cus) : LineShare{gm * a.gn, 0};
   t.k0 = 0; t.nk = nk; t.rest = -1;
   if (id < sh.whole) line_at(line_run(id, sh.whole), gm, a.gn, tm, t.tn);
@@ -76,7 +77,7 @@ __device__ __forceinline__ bool line_place(const LineArgs& a, int TM, LineTile& 
     t.k0 = half ? nk >> 1 : 0;
     t.nk = half ? nk - t.k0 : nk >> 1;
   }
-  if (a.g.z_off) { t.z = a.g.tile_z[tm]; t.mbase = a.g.tile_m0[tm]; t.mend = min(a.g.z_off[t.z + 1], t.mbase + TM); }
+  if (!SHARED && a.g.z_off) { t.z = a.g.tile_z[tm]; t.mbase = a.g.tile_m0[tm]; t.mend = min(a.g.z_off[t.z + 1], t.mbase + TM); }
   else { t.z = blockIdx.y; t.mbase = tm * TM; t.mend = min(a.g.M, t.mbase + TM); }
   return true;
 }

@@ -71,11 +71,11 @@ void launch_stack_line(tgx_ctx* c, const tgx::StackGemmArgs& g, int epi, int nz,
   a.g = g; a.terms = terms; a.ldt = ldt; a.gm = row_tiles;
   a.gn = tgx::sg_dual(epi) ? (g.N + tile / 2 - 1) / (tile / 2) : (g.N + tile - 1) / tile;
   int wgs = a.gm * a.gn;
-  if (nz == 1 && c->stack->line_share) {
-    const tgx::LineShare sh = tgx::line_share(g.z_off ? 1 : wgs, tile, g.K >> 6, c->num_cus);      // (a plan's tiles are counted on the device: half a round at most that are halved)
+  if (nz == 1 && !g.z_off && c->stack->line_share) {      // (experts' rows stand in any order in their tiles: whole ones give a row the same sum wherever it stands)
+    const tgx::LineShare sh = tgx::line_share(wgs, tile, g.K >> 6, c->num_cus);
     if (sh.rest && share_scratch(c, tile)) {
       a.cus = c->num_cus; a.met = (int*)c->stack->share; a.sums = (float*)c->stack->share + c->num_cus;
-      wgs += g.z_off ? c->num_cus / 2 : sh.rest;
+      wgs += sh.rest;
     }
   }
   const dim3 grid((unsigned)wgs, g.z_off ? 1 : nz);
