@@ -498,7 +498,8 @@ TGX_API int tgx_set_logits(tgx_ctx* ctx, const float* logits, int batch);
  *   "stack.ws_max" (layered models) most KiB of each scratch buffer that divided keys, blocked recurrences and prompts' products ask for (-1: as memory allows); what would need more,
  *                  or finds no memory, takes its form without scratch; tgx_get_option "stack.ws_grown" = how often the context has allocated them
  *   "stack.line_share"  (layered models) 0 = every tile of a prompt's products whole; 1 [default] = a last round that is at most half full as two halves of K (memory for a half's
- *                  sums, up to 32 MB, within stack.ws_max; not counted by stack.ws_grown)
+ *                  sums, 128 KiB a compute unit at most, 32 MiB of 256, within stack.ws_max and counted by stack.ws_grown; tgx_get_option "stack.line_share_kib" = what the context
+ *                  holds of it; where there is none every tile is whole)
  *   "debug.refuse_lds"  (layered models, tests) the n-th product from now that asks for its LDS is refused it: its step fails half-way, TGX_ERR_UNSUPPORTED
  *   "debug.*"      experiment switches (tools/gemv_dissect.py, tools/attn_dissect.py; live only in a -DTGX_DISSECT=1 build) */
 TGX_API int tgx_set_option(tgx_ctx* ctx, const char* key, int value);

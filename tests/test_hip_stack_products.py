@@ -205,11 +205,55 @@ def test_halved_tiles(T, dtype):
     eng.model.set_option("stack.line_share", 0)
     whole = eng.step([("p", ids, want)], ["p"])
     eng.model.set_option("stack.line_share", 1)
-    eng.model.set_option("stack.ws_max", 32 * 1024)      # (enough for the rows' terms, not for halves of 256 x 256)
-    eng.step([("p", ids, want)], ["p"])
+    eng.model.set_option("stack.ws_max", 32 * 1024)      # (enough for the rows' terms and for halves of 128 x 128, not for halves of 256 x 256)
+    some = [eng.step([("p", ids, want)], ["p"]) for _ in range(2)]
     eng.close()
+    assert (some[0] == some[1]).all() and not (some[0] == whole).all() and not (some[0] == halved[0]).all()
+    assert np.abs(some[0] - whole).max() / np.abs(whole).max() < 1e-4, (T, dtype)
     assert (halved[0] == halved[1]).all() and (halved[0] == halved[2]).all() and not (halved[0] == whole).all()
     assert np.abs(halved[0] - whole).max() / np.abs(whole).max() < 1e-4, (T, dtype)
+
+
+def test_memory_of_halved_tiles():
+    """taken once, in front of a context's first step of more than 64 rows and of the size that its steps can come to need; where it is not to be had every tile is whole, and the next step asks
+    again"""
+    import vitudra_oracle as vo
+    W, ff, T = 1024, 6208, 1700
+    cfg = dict(width=W, vocab=101, layers=[dict(type="wkv", mixer=dict(heads=W // 64, dim=64), mlp=dict(ff=ff))] * 2)
+    w = {k: np.asarray(v, np.float32) for k, v in vo.random_tensors(cfg, 3, decay_rank=64).items()}
+    ids, want = np.random.default_rng(T).integers(0, 101, T), [0, 255, T - 1]
+
+    def engine(**options):
+        eng = SlotEngine(desc=wkv_model(W, ff, "bf16", T), tensors=w)
+        for k, v in options.items():
+            eng.model.set_option("stack." + k, v)
+        return eng
+
+    eng = engine()
+    held = lambda: eng.model.get_option("stack.line_share_kib")      # noqa: E731
+    eng.step([("p", ids[:64], [63])], ["p"])
+    assert held() == 0
+    halved = eng.step([("p", ids, want)], ["p"])
+    kib, grown = held(), eng.model.get_option("stack.ws_grown")
+    assert kib % 128 <= 1 and kib >= 128 * 200      # (128 KiB and a number a compute unit)
+    assert (eng.step([("p", ids, want)], ["p"]) == halved).all() and (held(), eng.model.get_option("stack.ws_grown")) == (kib, grown)
+    eng.close()
+    got = []
+    for line_share in (0, 1):
+        eng = engine(line_share=line_share, ws_max=8 * 1024 - 1)      # (neither tile's halves fit; the rows' terms do not either, so that products go through the staged tiles)
+        got.append(eng.step([("p", ids, want)], ["p"]))
+        assert held() == 0
+        if line_share:
+            eng.model.set_option("stack.ws_max", -1)
+            assert (eng.step([("p", ids, want)], ["p"]) == halved).all() and held() == kib
+        eng.close()
+    assert (got[0] == got[1]).all()
+    eng = engine(ws_max=32 * 1024)      # (halves of 128 x 128 alone)
+    some = eng.step([("p", ids, want)], ["p"])
+    assert 0 < held() < kib and not (some == halved).all()
+    eng.model.set_option("stack.ws_max", -1)
+    assert (eng.step([("p", ids, want)], ["p"]) == halved).all() and held() == kib
+    eng.close()
 
 
 # ... and experts' tiles stay whole: their rows stand in any order (the plan takes them as they come), so that a row that is summed in halves in one pass would be summed whole in the next

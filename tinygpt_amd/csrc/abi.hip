@@ -1262,6 +1262,7 @@ int tgx_get_option(const tgx_ctx* c, const char* key, int* out_value) {
     if (!strcmp(key, "kv.page_tokens")) { *out_value = c->stack->page; return TGX_OK; }
     if (!strcmp(key, "act.round16")) { *out_value = c->act16; return TGX_OK; }
     if (!strcmp(key, "stack.ws_grown")) { *out_value = c->stack->ws_grown; return TGX_OK; }
+    if (!strcmp(key, "stack.line_share_kib")) { *out_value = (int)(c->stack->share_elems / 256); return TGX_OK; }
     if (!strcmp(key, "attn.split_min")) { *out_value = c->stack->on_matrix_cores() ? c->stack->latent_split_min_keys : c->stack->attn_split_min_keys; return TGX_OK; }
     if (!strcmp(key, "attn.gqa_split_min")) { *out_value = c->stack->on_matrix_cores() ? c->stack->gqa_split_min_keys : c->stack->gqa_lane_split_min_keys; return TGX_OK; }
     return TGX_ERR_INVALID;

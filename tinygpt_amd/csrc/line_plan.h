@@ -1,6 +1,7 @@
 // line_plan.h — how the last tiles of a prompt's product (kernels/stack_line.h) are divided between the compute units, as plain arithmetic on their number (no HIP call: tests go
 // through it on the CPU, the kernels through the same function).
 #pragma once
+#include <cstddef>
 
 #if defined(__HIPCC__)
 #define TGX_HD __host__ __device__ inline
@@ -23,6 +24,14 @@ constexpr int LINE_SHARE_STEPS256 = 16, LINE_SHARE_STEPS128 = 32;
 TGX_HD LineShare line_share(int tiles, int tile, int nk, int cus) {
   const int rest = cus > 0 ? tiles % cus : 0;
   return rest && 2 * rest <= cus && nk >= (tile == 256 ? LINE_SHARE_STEPS256 : LINE_SHARE_STEPS128) ? LineShare{tiles - rest, rest} : LineShare{tiles, 0};
+}
+// floats of a launch's halved tiles: who has come and whose sums lie ready, two numbers for each of half a round at most, then the sums (256 x 256: 128 KB a compute unit)
+TGX_HD size_t line_share_elems(int tile, int cus) { return (size_t)cus + (size_t)(cus / 2) * tile * tile; }
+// the larger tile of which products of up to `rows` rows, `cols` columns (of both matrices of a dual one) and nk steps can come to halve a round; 0: none.  256 x 256 tiles are taken only
+// where those of 128 x 128 are more than two rounds (tile_of, stack_line.hip)
+TGX_HD int line_share_tile(long long rows, long long cols, int nk, int cus) {
+  if (nk >= LINE_SHARE_STEPS256 && ((rows + 127) / 128) * ((cols + 127) / 128) > 2LL * cus) return 256;
+  return nk >= LINE_SHARE_STEPS128 ? 128 : 0;
 }
 
 }  // namespace tgx

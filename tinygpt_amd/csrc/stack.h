@@ -163,10 +163,11 @@ struct StackModel {
   size_t rec_block_most = 0;           // floats of scratch that a block of any layer's recurrence takes, all heads
   size_t terms_most = 0;               // ... of any product's input, whichever form it takes
   size_t ws_refused = SIZE_MAX;        // bytes that this step has asked for in vain
-  int ws_grown = 0;                    // tgx_get_option stack.ws_grown: how often part, terms and terms2 were allocated
-  int ws_max = -1;                     // option stack.ws_max: most KiB of each of part, terms and terms2 (-1: as memory allows); products, attention and recurrences that would need more take their forms without scratch
+  int ws_grown = 0;                    // tgx_get_option stack.ws_grown: how often part, terms, terms2 and share were allocated
+  int ws_max = -1;                     // option stack.ws_max: most KiB of each of part, terms, terms2 and share (-1: as memory allows); products, attention and recurrences that would need more take their forms without scratch
   int refuse_lds = 0;                  // option debug.refuse_lds: the n-th product from now that asks for its LDS is refused it, as a device could (tests of a step that fails half-way)
-  void* share = nullptr; size_t share_bytes = 0, share_refused = SIZE_MAX;      // divided tiles of prompts' products (stack_line.hip)
+  float* share = nullptr; size_t share_elems = 0;      // halved tiles of prompts' products (line_share_elems, line_plan.h; reserve_share)
+  long long cols_most = 0;             // columns of the widest product of the stream's rows (of both matrices of a dual one)
   int line_share = 1;                  // option stack.line_share: 0 keeps every tile of a prompt's products whole
   int line = 1;                        // option stack.line: 0 keeps prompts' products on the register-staged tiles
   int gemm_wt = 0;                     // option stack.gemm_wt: force the product's tile (1: 64 x 64, 2: 128 x 128); 0 = by the number of tiles

@@ -26,6 +26,7 @@
 #include "kernels/stack_ssd_mfma.h"
 #include "kernels/stack_hyper.h"
 #include "kernels/stack_next.h"
+#include "line_plan.h"
 
 namespace tgx {
 // A few tokens: the latents into the pool beside the queries into latent space (a product batched over the heads, kernels/stack_few.h): neither needs the other, attention needs both.
@@ -192,9 +193,32 @@ void scratch_sizes(tgx_ctx* c) {
     else if (l.mixer == TGX_MIXER_CHANNEL_DELTA) blocks(l.heads, l.dim, l.vdim, true);
     else if (l.mixer == TGX_MIXER_PARALLEL && sm->joint) blocks(l.d_heads, l.d_dim, l.d_vdim, true);
     sm->terms2_cols = std::max(sm->terms2_cols, (size_t)(l.mlp == TGX_MLP_MOE ? std::max(l.top * l.ff, l.shared_ff) : l.ff));
+    sm->cols_most = std::max<long long>(sm->cols_most, 2LL * (l.mlp == TGX_MLP_MOE ? l.shared_ff : l.ff));
   }
+  sm->cols_most = std::max<long long>({sm->cols_most, sm->max_in, sm->d.vocab});
   sm->terms_cols = (size_t)cols;
   sm->terms_most = (size_t)std::max(cols, most);
+}
+// memory of halved tiles (kernels/stack_line.h), in front of a step's launches and not by one of its products: of the size that this context's steps can come to need, by the products of
+// the stream's rows and those into the stream; a smaller one where that cannot be had, none where every tile is whole
+void reserve_share(tgx_ctx* c, long long rows) {
+  StackModel* sm = c->stack;
+  if (rows <= FEW_ROWS_MAX || !sm->line || !sm->line_share || sm->gemm_wt || c->dt == tgx::DT_F32) return;
+  const int W = sm->d.width;
+  const int most = std::max(tgx::line_share_tile(sm->cap_tokens, sm->cols_most, W / 64, c->num_cus), tgx::line_share_tile(sm->cap_tokens, W, (int)(sm->terms_most / 64), c->num_cus));
+  const size_t refused = sm->ws_refused;
+  for (int tile = most; tile >= 128; tile /= 2) {
+    const size_t need = tgx::line_share_elems(tile, c->num_cus);
+    const bool grows = need > sm->share_elems;
+    const bool ok = ensure_scratch(c, sm->share, sm->share_elems, need, need);
+    if (grows && sm->share && hipMemsetAsync(sm->share, 0, (size_t)c->num_cus * 4, c->stream) != hipSuccess) {      // (nobody has come to any tile)
+      (void)hipGetLastError();
+      (void)hipFree(sm->share);
+      sm->share = nullptr; sm->share_elems = 0;
+    }
+    if (ok) break;
+  }
+  sm->ws_refused = refused;      // (what the terms ask for may be found by giving back what they hold)
 }
 // rows per tile of the two grouped products of an expert layer's plan (both must be able to take them: their contraction lengths are the width and the expert width); 0: no plan,
 // the pairs' kernel (GROUPED_MEAN_ROWS).  np: (token, expert) pairs, E: experts, up_n: columns of the first product (gate and up together)
@@ -3488,6 +3512,7 @@ int stack_step(tgx_ctx* c, int S, const int32_t* rows, const int32_t* counts, co
   int rc;
   sm->ws_refused = SIZE_MAX;
   if ((rc = ensure_ws(c, (int)std::max<long long>(T, n_want)))) return rc;
+  reserve_share(c, std::max<long long>(T, n_want));
   if (max_count == 1) reserve_part(c);
   if ((rc = meta_host_free(c))) return rc;
   const MetaPtrs hp = meta_layout(sm->meta_host, (int)T, S, n_want), dp = meta_layout(sm->meta_dev, (int)T, S, n_want);
@@ -3558,6 +3583,7 @@ int stack_decode(tgx_ctx* c, const tgx_sampler_cfg& cfg, uint64_t seed, int n) {
   int rc;
   sm->ws_refused = SIZE_MAX;
   if ((rc = ensure_ws(c, S)) || (rc = meta_host_free(c))) return rc;
+  reserve_share(c, S);
   reserve_part(c);
   const MetaPtrs hp = meta_layout(sm->meta_host, S, S, S), dp = meta_layout(sm->meta_dev, S, S, S);
   for (int e = 0; e < S; e++) {

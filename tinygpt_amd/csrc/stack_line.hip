@@ -30,23 +30,11 @@ int tile_of(const tgx_ctx* c, long long t256, long long t128) {
   const long long r256 = (t256 + c->num_cus - 1) / c->num_cus, r128 = (t128 + c->num_cus - 1) / c->num_cus;
   return r256 * 28 <= r128 * 10 ? 256 : 128;
 }
-// memory of halved tiles (half a round at most): two numbers for each, then the sums of a half.  false: there is none, or option stack.ws_max forbids it, and every tile is whole
-bool share_scratch(tgx_ctx* c, int tile) {
-  StackModel* sm = c->stack;
-  const size_t need = (size_t)c->num_cus * 4 + (size_t)(c->num_cus / 2) * tile * tile * 4;
-  if (sm->ws_max >= 0 && need > (size_t)sm->ws_max * 1024) return false;
-  if (need <= sm->share_bytes) return true;
-  if (need >= sm->share_refused || hipStreamSynchronize(c->stream) != hipSuccess) return false;
-  void* p = nullptr;
-  if (hipMalloc(&p, need) != hipSuccess || hipMemsetAsync(p, 0, (size_t)c->num_cus * 4, c->stream) != hipSuccess) {
-    (void)hipGetLastError();
-    if (p) (void)hipFree(p);
-    sm->share_refused = need;
-    return false;
-  }
-  if (sm->share) (void)hipFree(sm->share);
-  sm->share = p; sm->share_bytes = need;
-  return true;
+// whether there is memory for halved tiles (the step asked for it, reserve_share); option stack.ws_max can forbid what is there
+bool share_scratch(const tgx_ctx* c, int tile) {
+  const StackModel* sm = c->stack;
+  const size_t need = tgx::line_share_elems(tile, c->num_cus);
+  return need <= sm->share_elems && (sm->ws_max < 0 || need * sizeof(float) <= (size_t)sm->ws_max * 1024);
 }
 }  // namespace
 
@@ -74,7 +62,7 @@ void launch_stack_line(tgx_ctx* c, const tgx::StackGemmArgs& g, int epi, int nz,
   if (nz == 1 && !g.z_off && c->stack->line_share) {      // (experts' rows stand in any order in their tiles: whole ones give a row the same sum wherever it stands)
     const tgx::LineShare sh = tgx::line_share(wgs, tile, g.K >> 6, c->num_cus);
     if (sh.rest && share_scratch(c, tile)) {
-      a.cus = c->num_cus; a.met = (int*)c->stack->share; a.sums = (float*)c->stack->share + c->num_cus;
+      a.cus = c->num_cus; a.met = reinterpret_cast<int*>(c->stack->share); a.sums = c->stack->share + c->num_cus;
       wgs += sh.rest;
     }
   }
