@@ -367,3 +367,20 @@ def test_third_term_in_slabs(name, S):
     (k0, v0), = run(m, prompt, mfma=False, n_decode=1)[3]
     assert np.mean(k1 != k0) < 3e-3 and np.mean(v1 != v0) < 3e-3, (np.mean(k1 != k0), np.mean(v1 != v0))
     assert rel_err(k1, k0) < 8e-3 and rel_err(v1, v0) < 8e-3
+
+
+@pytest.mark.parametrize("name,S", [("llama-3.2-1b", 257), ("qwen3-0.6b", 384)])
+def test_qkv_slabs_by_option(name, S):
+    """option prefill.qkv_8k 0: the QKV product on the register-staged tiles, as where the eight-wave kernels are off (prefill.gemm_dma without 8); prefill.splitk_8k leaves it alone"""
+    d = copy.deepcopy(known_desc(name, "bf16"))
+    d.layers, d.vocab, d.max_ctx = 1, 1024, S + 16
+    m = Model(d, product_backend()).load_synthetic(31, 0.02).finalize()
+    prompt = synth.synth_prompt(d.vocab, S, 7)[None, :]
+    kv = {}
+    for key, options in (("default", {}), ("slabs", {"splitk_8k": 0}), ("staged", {"qkv_8k": 0}), ("off", {"gemm_dma": 543 - 8})):
+        for o, v in {"splitk_8k": 1, "qkv_8k": 1, "gemm_dma": 543, **options}.items():
+            m.set_option("prefill." + o, v)
+        kv[key] = np.concatenate([x.ravel() for x in run(m, prompt, mfma=True, n_decode=1)[3][0]])
+    np.testing.assert_array_equal(kv["staged"], kv["off"])
+    np.testing.assert_array_equal(kv["slabs"], kv["default"])
+    assert (kv["staged"] != kv["default"]).any()

@@ -122,11 +122,11 @@ static void launch_gemm(tgx_ctx* c, int epi, const ebyte* B_, const ebyte* bias_
   if (c->gemm_splitk && ntiles < c->num_cus && K % tgx::GBK == 0 && !qkv_nosplit && !silu8) nsplit = std::min(std::min(16, ktiles), (2 * c->num_cus + ntiles - 1) / ntiles);
   // N = hidden products of a 129-1500-row prompt (option prefill.splitk_8k): their 128 x 128 tiles number less than a chip (Llama-3.2-1B S = 1024: 128 tiles on 256
   // CUs, 84 us per product against 104 at twice the rows) — the eight-wave LDS-DMA kernel over 2-8 K slabs instead of 64-row register-staged slabs or a half-empty chip
-  // The QKV product of a bf16 model as well (its keys' and values' columns with a third term), while its slabs are half a chip: two to four slabs where the register-staged tiles are four to
+  // The QKV product of a bf16 model as well (option prefill.qkv_8k; its keys' and values' columns with a third term), while its slabs are half a chip: two to four slabs where the register-staged tiles are four to
   // fourteen, which the rotation's launch reads.  us a prompt, register-staged / here (slab_sums with it): Qwen3-0.6B 133 tokens 2260 / 2203, 320 2799 / 2639, 509 3030 / 2875, 1000 4606 / 4591;
   // Llama-3.2-1B 133 2014 / 1911, 256 2172 / 2032, 509 3185 / 3119; Qwen2.5-0.5B 384 tokens 2154 / 2118, 700 3059 / 2970
   bool part_8k = false;
-  if (c->gemm_splitk && (c->splitk_8k || three_terms) && (c->gemm_dma & 8) && K % 64 == 0 && (!three_terms || c->dt == tgx::DT_BF16) && !qkv_nosplit && (epi == tgx::GEMM_RESIDUAL || epi == tgx::GEMM_STORE) && M > 128) {
+  if (c->gemm_splitk && (three_terms ? c->qkv_8k : c->splitk_8k) && (c->gemm_dma & 8) && K % 64 == 0 && (!three_terms || c->dt == tgx::DT_BF16) && !qkv_nosplit && (epi == tgx::GEMM_RESIDUAL || epi == tgx::GEMM_STORE) && M > 128) {
     const int z = tgx::eight_wave_slabs(M, N, K, c->num_cus);
     if (z >= 2 && (!three_terms || (2 * z * ntiles >= c->num_cus && tgx::eight_wave_halves(tgx::slab_steps(K, z))))) { part_8k = true; nsplit = z; }
   }
