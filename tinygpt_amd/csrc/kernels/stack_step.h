@@ -10,7 +10,7 @@
 // decays of 8 heads of 128 x 128 8.8 (convolution 5.4, scan 11.7, norm 3.3), retention of 4 heads of 128 x 256 with its rotation 8.8 (3.7, 9.3, 3.0).
 // What bounds it is latency: the launch, the step's tables, the loads that depend on them, three meetings of the waves.  So no load waits for another that it does not depend on: all of them, the state last,
 // are asked for before anything is computed, with clamped places in place of branches.  A convolution's taps one after the other, four slices of a decay's product, and conditional loads, whose registers
-// the compiler waits for where branches meet, were up to ten round trips: channel decays 9.2 -> 8.8, retention 9.4 -> 8.8, a delta rule beside attention 8.9 -> 8.2 (with attention as below).  Eight waves
+// the compiler waits for where branches meet, were up to ten round trips: channel decays 9.2 -> 8.9, retention 9.4 -> 8.8, a delta rule beside attention 8.9 -> 7.9 (with attention as below).  Eight waves
 // with twice the rows each are no faster (9.6, 8.7; retention's rows do not fit them).
 #pragma once
 #include "stack_rec.h"
@@ -41,10 +41,16 @@ __device__ __forceinline__ void rec_step_body(const StepMeta& m, const RecStepAr
   const bool col = j < vdim;
   // What a thread needs beside the state is asked for here, all of it, in front of the state: the first slices of a wkv head's decay product (sixteen lanes a channel, four elements a lane), the
   // output's gate and norm weight.  (A slice after the other they were four round trips.)
+  // A convolution in front of 32 rows a lane has no registers for that (they spilled: 256 x 128, sixteen entries 15.6 us, 13.7 so): there everything is asked for where it is used.
+  constexpr bool PREP = KIND == REC_DELTA || KIND == REC_CDELTA, AHEAD = !PREP || DPER <= 16;
   const bool mine = tid < vdim;
-  const int out_c = min(tid, vdim - 1);
-  const float* gp = a.g.gate + (size_t)t * a.g.ldg + (size_t)h * vdim;
-  const float gate = gp[out_c], w_out = (a.g.w ? a.g.w + (size_t)h * a.g.w_hstride : gp)[out_c];
+  float gate = 0.f, w_out = 1.f;
+  auto out_operands = [&] {
+    const int out_c = min(tid, vdim - 1);
+    const float* gp = a.g.gate + (size_t)t * a.g.ldg + (size_t)h * vdim;
+    gate = gp[out_c]; w_out = (a.g.w ? a.g.w + (size_t)h * a.g.w_hstride : gp)[out_c];
+  };
+  if (AHEAD) out_operands();
   constexpr bool W2 = KIND == REC_WKV;
   typename std::conditional<DT == DT_F32, float, unsigned>::type w2r[W2 ? 4 : 1];      // (as they lie in memory: widened where they are used)
   float lor[W2 ? 4 : 1], w0 = 0.f;
@@ -55,39 +61,44 @@ __device__ __forceinline__ void rec_step_body(const StepMeta& m, const RecStepAr
     if (r0 == 0) w0 = a.w0[at];
   };
   if (W2 && a.w2) decay_slices(0, 0);
-  // ... and the raw row, taps and tails of a convolved channel (of the last one again in the threads that have none)
-  constexpr bool PREP = KIND == REC_DELTA || KIND == REC_CDELTA;
+  // ... and the raw row, taps and tails of a convolved channel, in the waves that have any: taps that the filter has not and channels again in idle waves were 15 loads a thread more than
+  // their data, in line with the state's (8 heads of 128 x 128, one / four / sixteen entries: delta rule 7.9 / 8.5 / 9.5 us, so 7.1 / 7.6 / 8.8)
   const DeltaPrepArgs& p = a.p;
   const int GD = p.kv_heads * dim, C = 2 * GD + p.heads * vdim, nb = p.taps - 1, ct = min(tid, 2 * dim + vdim - 1), part = ct < dim ? 0 : ct < 2 * dim ? 1 : 2, cc = ct - part * dim;
   const int c = part == 0 ? kh * dim + cc : part == 1 ? GD + kh * dim + cc : 2 * GD + h * vdim + cc;
   const size_t tail = (size_t)row * nb * C + c;
   float zb = 0.f, za_raw = 0.f, za_bias = 0.f, al = 0.f;
-  if (PREP && a.prep) {
+  auto gates = [&] {
     const float* pr = p.proj + (size_t)t * p.ldp + p.col0 + p.b_col + h;
     zb = pr[0];
     if (p.a_log) { za_raw = pr[p.heads]; za_bias = p.dt_bias[h]; al = p.a_log[h]; }
-  }
+  };
   float x0 = 0.f, cw[PREP ? STEP_MAX_TAPS : 1], old[PREP ? STEP_MAX_TAPS : 1];      // old[d]: the row d positions back
-  if (PREP && a.prep) {
+  auto channel = [&] {
     x0 = p.proj[(size_t)t * p.ldp + p.col0 + c];
 #pragma unroll
-    for (int d = 0; d < (PREP ? STEP_MAX_TAPS : 0); d++) cw[d] = p.cw[(size_t)c * p.taps + max(nb - d, 0)];
-    if (nb > 0)
+    for (int d = 0; d < (PREP ? STEP_MAX_TAPS : 0); d++) if (d <= nb) cw[d] = p.cw[(size_t)c * p.taps + nb - d];
 #pragma unroll
-      for (int d = 1; d < (PREP ? STEP_MAX_TAPS : 0); d++) old[d] = p.state[(size_t)par * p.state_buf + tail + (size_t)max(nb - d, 0) * C];
+    for (int d = 1; d < (PREP ? STEP_MAX_TAPS : 0); d++) if (d <= nb) old[d] = p.state[(size_t)par * p.state_buf + tail + (size_t)(nb - d) * C];
+  };
+  if (PREP && AHEAD && a.prep) {
+    gates();
+    if (64 * __builtin_amdgcn_readfirstlane(wv) < 2 * dim + vdim) channel();
   }
   float* Sg = a.s.S + ((size_t)row * a.s.heads + h) * (size_t)dim * vdim;
   float S[DPER], ub[KIND == REC_WKV ? DPER : 1];
 #pragma unroll
   for (int dd = 0; dd < DPER; dd++) {
     const int d = d0 + dd;
-    S[dd] = Sg[(size_t)min(d, dim - 1) * vdim + min(j, vdim - 1)];      // (rows and columns that are not there: below)
+    if (AHEAD) S[dd] = Sg[(size_t)min(d, dim - 1) * vdim + min(j, vdim - 1)];      // (rows and columns that are not there: below)
+    else S[dd] = (pos != 0 && d < dim && col) ? Sg[(size_t)d * vdim + j] : 0.f;
     if (KIND == REC_WKV) ub[dd] = a.s.u[(size_t)h * dim + min(d, dim - 1)];
   }
   // ---- the head's inputs
   if (tid < 8) s_q[dim + tid] = s_k[dim + tid] = s_w[dim + tid] = 0.f;
   if (PREP && a.prep) {
     if (tid < 2 * dim + vdim) {
+      if (!AHEAD) channel();
       float acc = cw[0] * x0;
 #pragma unroll
       for (int d = 1; d < (PREP ? STEP_MAX_TAPS : 0); d++) {
@@ -105,6 +116,7 @@ __device__ __forceinline__ void rec_step_body(const StepMeta& m, const RecStepAr
       }
     }
     if (tid == NT - 1) {
+      if (!AHEAD) gates();
       const float za = za_raw + za_bias;
       s_b[0] = 1.0f / (1.0f + expf(-zb));
       if (p.a_log) {
@@ -176,7 +188,7 @@ __device__ __forceinline__ void rec_step_body(const StepMeta& m, const RecStepAr
   float po = 0.f;
 #pragma unroll
   for (int dd = 0; dd < DPER; dd++) {
-    if (pos == 0 || d0 + dd >= dim || !col) S[dd] = 0.f;
+    if (AHEAD && (pos == 0 || d0 + dd >= dim || !col)) S[dd] = 0.f;
     if (KIND == REC_WKV && d0 + dd >= dim) ub[dd] = 0.f;
   }
   if (KIND == REC_WKV) {
@@ -222,6 +234,7 @@ __device__ __forceinline__ void rec_step_body(const StepMeta& m, const RecStepAr
 #pragma unroll
   for (int dd = 0; dd < DPER; dd++) { const int d = d0 + dd; if (d < dim && col) Sg[(size_t)d * vdim + j] = S[dd]; }
   // the outputs, their norm and gate: one thread a column
+  if (!AHEAD) out_operands();
   __syncthreads();
   float o = 0.f;
   if (mine) {
@@ -249,7 +262,7 @@ __global__ __launch_bounds__(STEP_THREADS) void rec_step_kernel(StepMeta m, RecS
 //   softmax  every wave for itself, base 2, as in gqa_attn_mfma_kernel (cap, distance slope, sink, mask)
 //   values   a key per wave at a time; the waves' sums meet in LDS
 // Queries and probabilities stay fp32 (the matrix forms take them as two 16-bit terms).
-// Measured, us: one stream of 50 to 95 keys, eight query heads on two key / value heads of 128 x 128 7.9 (append 3.0, undivided walk 7.9); beside a delta rule in one launch 8.2 (a workgroup of sixteen
+// Measured, us: one stream of 50 to 95 keys, eight query heads on two key / value heads of 128 x 128 7.9 (append 3.0, undivided walk 7.9); beside a delta rule in one launch 7.9 (a workgroup of sixteen
 // waves a key / value head 8.0 and 8.9).
 constexpr int STEP_MAX_KEYS = 256, STEP_MAX_GROUP = 4, STEP_MAX_VDIM = 128;
 struct GqaStepArgs {
