@@ -1,6 +1,6 @@
 """Single tokens through a mixer's one launch (kernels/stack_step.h): recurrences whose heads fill, exceed and fall short of the columns and row groups of a workgroup,
 convolutions of one tap to the most that the kernel takes and one more, attention over one key up to the most that it takes and past that, masks, caps, slopes, rotations and
-groups of one to four query heads.  fp32 storage against the plain oracles of the designs: fp32 sums over at most 256 channels and keys, 1e-4 of the largest logit as in the
+groups of one to eight query heads.  fp32 storage against the plain oracles of the designs: fp32 sums over at most 256 channels and keys, 1e-4 of the largest logit as in the
 designs' own tests; and against the same steps in the launches that it stands for, whose sums meet in another order (1e-5: a thousand roundings of 2^-24)."""
 import numpy as np
 import pytest
@@ -75,7 +75,8 @@ def test_channel_decays(dim, vdim):
 
 
 @pytest.mark.parametrize("n", [1, 2, 62, 63, 64, 127, 128, 255, 256, 257])
-@pytest.mark.parametrize("shape", [dict(heads=4, kv_heads=1, dim=8, vdim=6), dict(heads=2, kv_heads=2, dim=64, vdim=64), dict(heads=3, kv_heads=1, dim=136, vdim=128), dict(heads=8, kv_heads=2, dim=256, vdim=100)])
+@pytest.mark.parametrize("shape", [dict(heads=4, kv_heads=1, dim=8, vdim=6), dict(heads=2, kv_heads=2, dim=64, vdim=64), dict(heads=3, kv_heads=1, dim=136, vdim=128), dict(heads=8, kv_heads=2, dim=256, vdim=100), dict(heads=5, kv_heads=1, dim=16, vdim=24),
+                                   dict(heads=16, kv_heads=2, dim=64, vdim=64)])
 def test_attention_of_so_many_keys(n, shape):
     layers = [tv.attn(mask=None, **shape), tv.attn(tv.ff(16), kv_from=0, mask=None, **shape), tv.par(tv.ff(16), left=dict(shape, mask=None, softcap=3.0, rot={"base": 300.0, "dims": 8}))]
     cfg = tv.config(layers, width=24)

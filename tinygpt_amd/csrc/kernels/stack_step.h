@@ -263,8 +263,9 @@ __global__ __launch_bounds__(STEP_THREADS) void rec_step_kernel(StepMeta m, RecS
 //   values   a key per wave at a time; the waves' sums meet in LDS
 // Queries and probabilities stay fp32 (the matrix forms take them as two 16-bit terms).
 // Measured, us: one stream of 50 to 95 keys, eight query heads on two key / value heads of 128 x 128 7.9 (append 3.0, undivided walk 7.9); beside a delta rule in one launch 7.9 (a workgroup of sixteen
-// waves a key / value head 8.0 and 8.9).
-constexpr int STEP_MAX_KEYS = 256, STEP_MAX_GROUP = 4, STEP_MAX_VDIM = 128;
+// waves a key / value head 8.0 and 8.9).  The group's size does not matter to it: eight or sixteen query heads a key / value head, 50 to 85 keys, one entry 7.4 (append 3.2, walk 7.8 to 9.5), sixteen
+// 8.0 (4.2, 10.5 to 12.4), beside a delta rule 7.4 (with the rule's launch 19); 220 to 240 keys 14.8 in one launch and 13.2 to 15.7 in three, beside a delta rule 13.1 and 21.
+constexpr int STEP_MAX_KEYS = 256, STEP_MAX_VDIM = 128;
 struct GqaStepArgs {
   GqaAppendArgs ap;          // the token's row (maps 1, no q_hi, no qk_unit_eps)
   const float* gate; long long ldg; int gate_per_head;

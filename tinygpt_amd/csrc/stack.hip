@@ -690,7 +690,7 @@ tgx::GqaAppendArgs append_args(const StackModel* sm, const GqaSpec& sp) {
 bool gqa_step(const StackModel* sm, const GqaSpec& sp, int max_keys, int max_count, tgx::GqaStepArgs& a) {
   const int span = sp.mask_kind == tgx::MASK_CAUSAL ? max_keys : std::min(max_keys, sp.mask_size);
   if (max_count != 1 || !sm->rec_step || !sm->attn_mfma || sm->gqa_split_min_keys != StackModel::MFMA_SPLIT_MIN || span > tgx::STEP_MAX_KEYS) return false;
-  if (sp.maps != 1 || sp.v_is_k || sp.sinks || sp.dist || sp.dim % 8 || sp.dim > tgx::STEP_MAX_DIM || sp.vdim > tgx::STEP_MAX_VDIM || sp.heads > tgx::STEP_MAX_GROUP * sp.kv_heads) return false;
+  if (sp.maps != 1 || sp.v_is_k || sp.sinks || sp.dist || sp.dim % 8 || sp.dim > tgx::STEP_MAX_DIM || sp.vdim > tgx::STEP_MAX_VDIM) return false;
   a.ap = append_args(sm, sp);
   a.gate = sp.gate; a.ldg = sp.ldg; a.gate_per_head = sp.gate_per_head; a.out = sp.out; a.ldo = sp.ldo; a.out_scale = sp.out_scale;
   a.scale = sp.scale; a.sink = sp.sink; a.has_sink = sp.has_sink; a.mask_kind = sp.mask_kind; a.mask_size = sp.mask_size; a.softcap = sp.softcap; a.dist_bias = sp.dist_bias;
