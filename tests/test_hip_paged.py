@@ -175,7 +175,8 @@ def test_paged_needs_16_bit_storage_and_is_set_before_finalize(hip):
 
 
 @pytest.mark.parametrize("name,S,dtype", [("llama-3.2-1b", 40, "bf16"), ("llama-3.2-1b", 300, "bf16"), ("llama-3.2-1b", 1100, "bf16"), ("llama-3.2-1b", 3500, "bf16"), ("llama-3.2-1b", 6500, "bf16"),
-                                          ("mistral-7b-v0.3", 200, "fp16"), ("qwen2.5-0.5b", 700, "bf16"), ("qwen3-1.7b", 150, "bf16")])
+                                          ("mistral-7b-v0.3", 200, "fp16"), ("qwen2.5-0.5b", 700, "bf16"), ("qwen3-1.7b", 150, "bf16"),
+                                          ("llama-3.2-1b", 256, "bf16"), ("qwen3-0.6b", 449, "bf16"), ("qwen3-0.6b", 512, "fp16")])      # (blocks of 32 queries, keys in four streams)
 def test_matrix_core_prefill_into_a_paged_cache(name, S, dtype, hip):
     """Prompts of 40 .. 6500 rows (the last: the 20 decode steps run the long-context matrix-core attention) at real layer shapes (2 layers) through the skinny and the tiled matrix-core prefill of a paged context: RoPE + cache append
     (the QKV GEMM's epilogue at head_dim 64, else rope_kv_split_kernel) and the causal prompt attention (attn_prefill_kernel<.., PAGED> plain / key-split /

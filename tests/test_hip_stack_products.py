@@ -207,11 +207,14 @@ def test_halved_tiles(T, dtype):
     eng.model.set_option("stack.line_share", 1)
     eng.model.set_option("stack.ws_max", 32 * 1024)      # (enough for the rows' terms and for halves of 128 x 128, not for halves of 256 x 256)
     some = [eng.step([("p", ids, want)], ["p"]) for _ in range(2)]
+    eng.model.set_option("stack.line", 0)
+    plain = eng.step([("p", ids, want)], ["p"])
     eng.close()
     assert (some[0] == some[1]).all() and not (some[0] == whole).all() and not (some[0] == halved[0]).all()
     assert np.abs(some[0] - whole).max() / np.abs(whole).max() < 1e-4, (T, dtype)
     assert (halved[0] == halved[1]).all() and (halved[0] == halved[2]).all() and not (halved[0] == whole).all()
-    assert np.abs(halved[0] - whole).max() / np.abs(whole).max() < 1e-4, (T, dtype)
+    for other in (whole, plain):
+        assert np.abs(halved[0] - other).max() / np.abs(other).max() < 1e-4, (T, dtype)
 
 
 def test_memory_of_halved_tiles():
