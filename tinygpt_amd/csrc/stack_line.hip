@@ -19,8 +19,9 @@ void launch_line_t(tgx_ctx* c, const tgx::LineArgs& a, dim3 grid, int tile) {
 }
 template <int DT, int EPI, bool DUAL>
 void launch_line_t(tgx_ctx* c, const tgx::LineArgs& a, dim3 grid, int tile) {
-  if (a.cus) launch_line_t<DT, EPI, DUAL, true>(c, a, grid, tile);
-  else launch_line_t<DT, EPI, DUAL, false>(c, a, grid, tile);
+  if constexpr (EPI != tgx::SG_EXPERT_ACT)      // (of experts alone, whose tiles are whole)
+    if (a.cus) { launch_line_t<DT, EPI, DUAL, true>(c, a, grid, tile); return; }
+  launch_line_t<DT, EPI, DUAL, false>(c, a, grid, tile);
 }
 // 256-row or 128-row tiles for t256 / t128 of them: a compute unit takes 2.8 times as long for the large one (2048 x 2048 x 2048: 89 us for one round of 256 x 256, 38 for one of
 // 128 x 128; 11264 x 8192 x 2048: 652 us for six rounds against 768 for 22).  Fewer than 64 small ones leave most of the chip idle either way: the 64-wide tiles
