@@ -798,9 +798,10 @@ __global__ __launch_bounds__(512) void gemm_dma8k_kernel(const GemmArgs a) {
 // a tile four bytes a lane: 5.7 of the 14.5 us of 200 x 2048 x 2048 in eight slabs (2.1 to the first stage, 0.83 a stage).  Two halves exchange a quarter of that over one barrier and
 // all eight waves store: 2.3 us.  A half is the k16 steps kh and kh + 2, each with a sum of its own until the loop is over, so that an output is the same number as above, bit for bit (in
 // one sum for both the chains were twice as long: Llama-3.2-1B fp16 300 tokens 1.03 +- 0.02 of the error against 64 bits, Zaluvik's two requests 1.06 +- 0.02); it costs 64 registers
-// (198 of 256) and no time.  The price are twelve fragment reads a stage and wave for eight.  us quarters / halves: 200 x 2048 x 2048 in eight slabs (four stages) 14.5 / 12.1, in
-// four (eight) 15.2 / 12.3; 509 x 1024 x 3072, eight (six) 17.4 / 14.8; 200 x 2048 x 8192, eight (sixteen) 28.0 / 26.8; 300 x 2048 x 8192, five (26) 34.8 / 34.3; 2048 x 2048 x 2048, whole
-// (32) 40.7 / 40.1; 1000 x 2048 x 8192, two (64) 68.4 / 70.1; 2048 x 2048 x 8192, whole (128) 124 / 129: up to 32 stages (prefill_plan.h).
+// (198 of 256) and no time.  The price are twelve fragment reads a stage and wave for eight.  us quarters / halves: 200 x 2048 x 2048 in
+// seven slabs (four or five stages) 14.5 / 12.9, 509 x 1024 x 2048, five (seven) 14.8 / 12.1, 509 x 1024 x 3072, five (ten) 17.1 / 14.6; 200 x 2048 x 8192, eight (sixteen) 29.0 / 22.8; 300 x
+// 2048 x 8192, five (26) 31.5 / 30.5; 2048 x 2048 x 2048, whole (32) 41.5 / 40.8; 1000 x 2048 x 8192, two (64) 67.3 / 66.3; 2048 x 2048 x 8192, whole (128) 139 / 142: up to 32 stages
+// (prefill_plan.h).
 // T3: columns from three_from on take a third term of the activations (the QKV product of a bf16 model).  It comes first, in stages of its own of one A tile beside B and half the matrix
 // work, through the same ring, so that the other columns' tiles cost what they cost without it.
 template <int DT, int EPI, bool LO = true, bool T3 = false>

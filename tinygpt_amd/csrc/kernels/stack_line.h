@@ -310,8 +310,9 @@ __global__ __launch_bounds__(512) void stack_line256_kernel(const LineArgs a) {
 }
 
 // HALF: the waves are 2 x 2 quadrants x two halves of a stage's k16 steps, not two row halves x four quarters, for chains of up to 32 stages, as in gemm_dma8h_kernel (gemm_dma.h): the sums
-// meet in the epilogue, with no exchange in front of it.  Each k16 step has a sum of its own, as there: the same numbers either way.  us quarters / halves: 1999 x 1024 x 512 13.7 / 12.5, K 1024 19.6 / 18.9, K 2048 halved tiles 28.5 / 27.4; 2397 x 2304 x 1024 37.4 /
-// 35.5; 2397 x 8192 x 1024 93.7 / 88.8; 2048 x 2048 x 2048 37.2 / 37.1, K 4096 62.4 / 63.5
+// meet in the epilogue, with no exchange in front of it.  Each k16 step has a sum of its own, as there: the same numbers either way.  us quarters / halves: 1999 rows, gate and up of 512
+// (K 1024) 21.2 / 20.5, of 2048 45.0 / 43.8, into 1024 columns K 1024 23.1 / 22.4, K 2048 in halved tiles 33.1 / 32.7; 2397 rows, gate and up of 4096 (K 1024) 107.8 / 104.6, into 1024 columns
+// K 1024 26.1 / 25.3, K 4096 62.0 / 62.1; 2048 x 2048 x 2048 44.3 / 44.0
 template <int DT, int EPI, bool DUAL, bool SHARED, bool HALF>
 __global__ __launch_bounds__(512) void stack_line128_kernel(const LineArgs a) {
   constexpr int TMN = 128, NS = 3, T_A = TMN * 64, STAGE = 3 * T_A;      // a stage: A lines of two k32 steps | B lines, 128 rows x 128 bytes each

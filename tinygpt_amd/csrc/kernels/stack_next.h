@@ -1,9 +1,9 @@
 // stack_next.h — what stands between two greedy decode steps of a layered model, in one launch behind the logits' argmax partials (slot_logits_kernel): a row's argmax, the token published as
 // finalize_row does (gemv.h), and the next step's inputs: its token, position and state buffer, and in designs whose stream begins as the plain embedding row that row.
 //
-// The launch is latency alone: it replaces one a row for the token, one for the step's tables and one for the embedding, each 2.2 to 4.6 us of which 2.2 is an empty launch.  A workgroup of sixteen
-// waves owns a row.  (One that goes through the row's logits itself, without the partials' launch, is slower, since one compute unit reads them: a step of a small model of 8192 columns 38.9 us so,
-// 47.8 with it, 32768 42.2 and 49.8, 65536 46.3 and 54.3.)
+// The launch is latency alone: it replaces one a row for the token, one for the step's tables and one for the embedding, each 2.4 to 4.6 us where an empty launch is 2.4.  A workgroup of sixteen
+// waves owns a row.  (It could go through the row's logits itself and save the partials' launch, but one compute unit would read them.  A step of a small model, us, partials' launch and this
+// one / this one over the logits: 8192 columns 38.9 / 47.8, 32768 42.2 / 49.8, 65536 46.3 / 54.3.)
 #pragma once
 #include "gemv.h"
 #include "stack_meta.h"

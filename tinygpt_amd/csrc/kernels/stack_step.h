@@ -1,4 +1,4 @@
-// stack_step.h — one decoded token of a mixer in ONE launch: what stands between the mixer's products.  First the recurrences, then attention over a short context.  A step of single tokens is bound by its launches (2.6 us for an
+// stack_step.h — one decoded token of a mixer in ONE launch: what stands between the mixer's products.  First the recurrences, then attention over a short context.  A step of single tokens is bound by its launches (2.4 us for an
 // empty one), and a recurrence took three to five of them: the low-rank decay's second product or the convolution with its norms and gates, the rotation, the scan, the norm and gate
 // behind it.  Here a workgroup owns a head of one entry with all of its value columns, so that nothing crosses workgroups: the head's inputs are made in LDS, the state [dim][vdim]
 // passes through the registers of 1024 threads once (rows of it are read and written whole, 256 bytes a wave and row; the scan's workgroups of sixteen columns take 64-byte

@@ -16,8 +16,8 @@ struct LineShare { int whole, rest; };
 
 // Halving takes half of a tile's steps off the last round and costs a pass of the first half's sums through memory (256 KB a tile of 256 x 256) and a ring filled anew.  From these steps
 // on it was faster, us halved / whole: 256 x 256, 10917 x 2048 (88 tiles of 344 halved) K 1024 104 / 108, 2048 170 / 189, 4096 315 / 357, 8192 589 / 685; 10917 x 8192 (96 of 1376)
-// K 2048 587 / 602; 2048 x 10240 (64 of 320) 169 / 189.  128 x 128, 1999 x 1024 (128 of 128) K 1024 21.8 / 19.9, 1536 24.9 / 26.3, 2048 28.9 / 32.0, 4096 42.7 / 58.5; 1999 x 3072
-// (128 of 384) K 1024 43.2 / 40.1, 2048 64.8 / 65.7, 3072 87.3 / 92.2.  Beyond half a round two halves are two rounds, and thirds to sevenths lose to the sums' way through memory what
+// K 2048 587 / 602; 2048 x 10240 (64 of 320) 169 / 189.  128 x 128, 1999 x 1024 (128 of 128) K 1024 25.0 / 22.4, 1536 28.1 / 28.6, 2048 31.8 / 34.0, 3072 40.0 / 47.5, 4096 46.2 / 59.1;
+// 1999 rows, gate and up of 1536 (128 of 384) K 1024 43.2 / 41.2, 1536 55.2 / 56.2, 2048 66.0 / 70.3, 3072 91.4 / 97.6: at 24 steps the two are within two runs of one.  Beyond half a round two halves are two rounds, and thirds to sevenths lose to the sums' way through memory what
 // they save (344 tiles, K 8192: thirds 663, fifths 626; 200 tiles, K 2048: 98 whole, 149 and 174).  The card's power sets the rate of full rounds, so that a half-empty one is not
 // half lost.
 constexpr int LINE_SHARE_STEPS256 = 16, LINE_SHARE_STEPS128 = 32;

@@ -23,8 +23,9 @@ void launch_line_t(tgx_ctx* c, const tgx::LineArgs& a, dim3 grid, int tile) {
     if (a.cus) { launch_line_t<DT, EPI, DUAL, true>(c, a, grid, tile); return; }
   launch_line_t<DT, EPI, DUAL, false>(c, a, grid, tile);
 }
-// 256-row or 128-row tiles for t256 / t128 of them: a compute unit takes 2.8 times as long for the large one (2048 x 2048 x 2048: 89 us for one round of 256 x 256, 38 for one of
-// 128 x 128; 11264 x 8192 x 2048: 652 us for six rounds against 768 for 22).  Fewer than 64 small ones leave most of the chip idle either way: the 64-wide tiles
+// 256-row or 128-row tiles for t256 / t128 of them: a compute unit takes 2.8 times as long for the large one, between what a lone round shows (2048 x 2048 x 2048: 113 us on 64 tiles of
+// 256 x 256, 95 with them halved, 48 on 256 of 128 x 128) and what full ones do (K 2048, gate and up of 8192, 2048 rows: 229 us for two rounds, 290 for eight; of 4096 118 and 149).  A last
+// round counts whole where it is halved too (line_plan.h): 2048 x 9344 x 2048, 296 tiles with 40 halved 174 us, 1168 small ones 178.  Fewer than 64 small ones leave most of the chip idle either way: the 64-wide tiles
 // (0) spread further (130 rows, 1024 x 1024: 18.7 us against 20.4 with the split)
 int tile_of(const tgx_ctx* c, long long t256, long long t128) {
   if (t128 < 64) return 0;
