@@ -83,6 +83,34 @@ def test_attention_of_so_many_keys(n, shape):
     stepped(tv, cfg, n + 2, n, max(1, n - 1))
 
 
+# as many entries as give a workgroup a query head (256 compute units), and one more: four heads of a key / value head a workgroup from there on, the last of a group fewer (9 on 1: four, four,
+# one), a layer that reads another's pool, caps, rotations, slopes, values mixed with the first layer's; keys from one to the most that the kernels take
+@pytest.mark.parametrize("t", [tv, tm])
+@pytest.mark.parametrize("shape", [dict(heads=8, kv_heads=2, dim=128, vdim=128), dict(heads=9, kv_heads=3, dim=16, vdim=24), dict(heads=9, kv_heads=1, dim=8, vdim=6), dict(heads=8, kv_heads=4, dim=136, vdim=100),
+                                   dict(heads=16, kv_heads=1, dim=64, vdim=72)])
+@pytest.mark.parametrize("more", [0, 1])
+def test_attention_of_many_entries(t, shape, more):
+    if t is tv:
+        cfg = tv.config([tv.attn(mask=None, **shape), tv.attn(tv.ff(16), kv_from=0, mask=None, **shape), tv.par(tv.ff(16), left=dict(shape, mask=None, softcap=3.0, rot={"base": 300.0, "dims": 8}))], width=24)
+    else:
+        cfg = tm.config([tm.attn(tm.dense(), **shape), tm.attn(tm.dense(), **shape), tm.attn(v_mix=False, **shape)], width=24)
+    n = 256 // shape["heads"] + more
+    lens = [1, 2, 15, 16, 17, 63, 64, 65, 127, 128, 129, 252]
+    toks = [t.tokens(cfg, lens[i % len(lens)] + 3, i) for i in range(n)]
+    out = []
+    for on in (1, 0):
+        eng, w = t.engine(cfg, seed=shape["dim"], max_seqs=n, max_ctx=256, budget_tokens=256 * n)
+        eng.model.set_option("stack.rec_step", on)
+        got = [eng.step([(i, s[:-3], [len(s) - 4]) for i, s in enumerate(toks)])]
+        got += [eng.step([(i, s[len(s) - j:len(s) - j + 1], [0]) for i, s in enumerate(toks)]) for j in (3, 2, 1)]
+        eng.close()
+        out.append(np.stack(got, 1))
+    assert np.abs(out[0] - out[1]).max() / np.abs(out[1]).max() < 1e-5
+    for i in (*range(min(n, len(lens))), n - 1):
+        want = t.want_of(cfg, w, toks[i])
+        assert np.abs(out[0][i] - want[-4:]).max() / np.abs(want).max() < 1e-4, i
+
+
 @pytest.mark.parametrize("mask", [{"size": 1}, {"size": 64}, {"size": 200}, {"size": 256}, {"size": 300}])
 def test_attention_behind_masks(mask):
     cfg = tv.config([tv.attn(mask=mask), tv.par(tv.ff(16), left=dict(mask=mask))], width=24)

@@ -449,6 +449,173 @@ __device__ __forceinline__ void gqa_step_body(const StepMeta& m, const GqaStepAr
 template <int DT>
 __global__ __launch_bounds__(512) void gqa_step_kernel(StepMeta m, GqaStepArgs a) { gqa_step_body<DT, 512>(m, a, blockIdx.x, blockIdx.y); }
 
+// The same for steps of more query heads than compute units: a workgroup of sixteen waves takes up to STEP_GROUP query heads of a key / value head, whose rows come once for all of them.  A
+// workgroup a query head holds all that a wave loads in registers, so that a compute unit takes one at a time, and the second round costs what the first did.  us, a query head a workgroup /
+// this form, 60, 120 and 245 keys: 32 entries of eight heads on two of 128 x 128 (256 heads) 7.6, 10.6, 15.5 / 9.4, 13.4, 20.7, 48 entries 12.3, 17.3, 27.4 / 9.3, 12.7, 20.7; sixteen heads on four of
+// 64 x 64, sixteen entries (256) 7.2, 9.3, 14.4 / 8.2, 10.0, 15.4, 24 entries 12.2, 16.1, 25.2 / 8.1, 10.2, 15.8, 64 entries 21.3, 29.5, 48.0 / 8.1, 11.2, 16.6; eight heads on four, 48 entries 12.8, 17.5,
+// 28.0 / 10.5, 13.2, 21.4, on one 12.2, 17.0, 27.6 / 8.5, 11.6, 19.4.  With a key / value head a query head there is nothing to share: 48 entries of eight 13.1, 17.7, 29.4 / 17.5, 24.0, 39.9.
+constexpr int STEP_GROUP = 4;
+template <int DT>
+__device__ __forceinline__ void gqa_group_step_body(const StepMeta& m, const GqaStepArgs& a, const int e, const int blk) {
+  constexpr int MG = STEP_GROUP, KW = STEP_MAX_KEYS / 16;      // keys of a wave
+  constexpr float LOG2E = 1.4426950408889634f;
+  __shared__ __attribute__((aligned(16))) float s_qr[MG][STEP_MAX_DIM], s_kn[STEP_MAX_DIM];
+  __shared__ float s_vn[STEP_MAX_VDIM], s_s[MG][STEP_MAX_KEYS], s_l[MG], s_acc[16][MG][STEP_MAX_VDIM];
+  const GqaAppendArgs& ap = a.ap;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row = m.tok_row[e], pos = m.tok_pos[e], dim = ap.dim, vdim = ap.vdim, Gq = ap.heads / ap.kv_heads;
+  const int blocks = (Gq + MG - 1) / MG, g = blk / blocks, hb = MG * (blk - g * blocks), h0 = g * Gq + hb, nh = min(MG, Gq - hb);      // its key / value head and its query heads
+  const int lo = first_key(pos, a.mask_kind, a.mask_size), n = pos - lo + 1, kd = ap.kv_heads * dim, vd = ap.kv_heads * vdim;
+  const int* tbl = m.tbl + (size_t)row * m.tbl_stride;
+  const bool fresh_key = ap.poolK != nullptr;                      // (a layer that reads another layer's pool appends nothing: its last key stands there)
+  const bool appends = fresh_key && hb == 0;                       // (one of a key / value head's workgroups stores the token's key and value; all of them make them)
+  const int stored = fresh_key ? n - 1 : n, pmask = (1 << m.page_shift) - 1;
+  const float* prow = ap.proj + (size_t)e * ap.ldp;
+  // keys and values of this wave, on their way before anything is computed: four keys a turn, sixteen lanes a key; then a key a turn for the values
+  const int sub = lane >> 4, ch = 8 * (lane & 15);
+  const elem_t<DT>* pK = reinterpret_cast<const elem_t<DT>*>(a.poolK) + (size_t)g * dim;
+  const elem_t<DT>* pV = reinterpret_cast<const elem_t<DT>*>(a.poolV) + (size_t)g * vdim;
+  auto slot_of = [&](int i) -> size_t { const int key = lo + min(i, max(stored - 1, 0)); return ((size_t)tbl[key >> m.page_shift] << m.page_shift) + (size_t)(key & pmask); };
+  Slice8<DT> kr[KW / 4][2];
+#pragma unroll
+  for (int u = 0; u < KW / 4; u++) {
+    const int i = 4 * (wv + 16 * u) + sub;
+    if (64 * u >= n) break;                                        // (uniform)
+    const elem_t<DT>* kp = pK + slot_of(i) * kd;
+#pragma unroll
+    for (int c = 0; c < 2; c++) if (128 * c < dim) kr[u][c] = load_slice<DT>(kp + min(ch + 128 * c, dim - 8), 0);
+  }
+  float vr[KW][2];
+#pragma unroll
+  for (int u = 0; u < KW; u++) {
+    if (16 * u >= n) break;
+    const elem_t<DT>* vp = pV + slot_of(wv + 16 * u) * vd;
+#pragma unroll
+    for (int c = 0; c < 2; c++) vr[u][c] = 64 * c < vdim ? elem_to_f32<DT>(vp[min(lane + 64 * c, vdim - 1)]) : 0.f;
+  }
+  // the token's queries (score scale and log2 e folded in), key and value
+  const bool capped = a.softcap > 0.f;
+  const float temp = ap.q_temp_coef != 0.f ? fmaf(ap.q_temp_coef, logf((float)((pos + 1) / ap.q_temp_every) + 1.0f), 1.0f) : 1.0f, qscale = capped ? a.scale : a.scale * LOG2E;
+  const int nq = nh + (fresh_key ? 1 : 0);
+  if (wv < 2 * nq)                                                 // two waves a row
+    for (int c = lane + 64 * (wv & 1); c < dim; c += 128) {
+      const int r = wv >> 1;
+      const float* u = prow + (r < nh ? (size_t)(h0 + r) * dim : (size_t)ap.heads * dim + (size_t)g * dim);
+      float v = u[c];
+      if (c < ap.rot_dims) {
+        const int half = ap.rot_dims >> 1, p = ap.rot_pairs ? c >> 1 : c < half ? c : c - half;
+        const bool first = ap.rot_pairs ? (c & 1) == 0 : c < half;
+        const float cs = ap.cs[((size_t)pos * half + p) * 2], sn = ap.cs[((size_t)pos * half + p) * 2 + 1], o = u[ap.rot_pairs ? c ^ 1 : first ? c + half : c - half];
+        v = first ? __fsub_rn(__fmul_rn(v, cs), __fmul_rn(o, sn)) : __fadd_rn(__fmul_rn(v, cs), __fmul_rn(o, sn));
+      }
+      if (r < nh) s_qr[r][c] = v * temp * qscale;
+      else {
+        const elem_t<DT> k = f32_to_elem<DT>(v);
+        if (appends) reinterpret_cast<elem_t<DT>*>(ap.poolK)[(((size_t)tbl[pos >> m.page_shift] << m.page_shift) + (size_t)(pos & pmask)) * kd + (size_t)g * dim + c] = k;
+        s_kn[c] = elem_to_f32<DT>(k);
+      }
+    }
+  if (fresh_key && tid < vdim) {
+    const size_t at = (size_t)e * vd + (size_t)g * vdim + tid;
+    float v = prow[(size_t)ap.heads * dim + kd + (size_t)g * vdim + tid];
+    if (ap.vmode == 1 && appends) ap.vfirst[at] = v;
+    if (ap.vmode == 2) { const float lam = ap.lam[0]; v = fmaf(lam, ap.vfirst[at], __fmul_rn(1.0f - lam, v)); }
+    const elem_t<DT> sv = f32_to_elem<DT>(v);
+    if (appends) {
+      const size_t pg = (size_t)tbl[pos >> m.page_shift];
+      reinterpret_cast<elem_t<DT>*>(ap.poolV)[((pg << m.page_shift) + (size_t)(pos & pmask)) * vd + (size_t)g * vdim + tid] = sv;
+      if (ap.poolVT) reinterpret_cast<elem_t<DT>*>(ap.poolVT)[((pg * vd + (size_t)g * vdim + tid) << m.page_shift) + (size_t)(pos & pmask)] = sv;
+    }
+    s_vn[tid] = elem_to_f32<DT>(sv);
+  }
+  __syncthreads();
+  // scores
+#pragma unroll
+  for (int u = 0; u < KW / 4; u++) {
+    if (64 * u >= n) break;
+    const int i = 4 * (wv + 16 * u) + sub;
+    float sc[MG] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      if (128 * c >= dim) break;
+      const int at = ch + 128 * c;
+      float k[8];
+      slice_unpack<DT>(kr[u][c], k);
+      if (fresh_key && i == n - 1) {
+#pragma unroll
+        for (int x = 0; x < 8; x++) k[x] = s_kn[min(at + x, dim - 1)];
+      }
+      if (at < dim) {
+#pragma unroll
+        for (int r = 0; r < MG; r++) {
+          const f32x4 q0 = *reinterpret_cast<const f32x4*>(&s_qr[min(r, nh - 1)][at]), q1 = *reinterpret_cast<const f32x4*>(&s_qr[min(r, nh - 1)][at + 4]);
+#pragma unroll
+          for (int x = 0; x < 8; x++) sc[r] = fmaf(k[x], x < 4 ? q0[x & 3] : q1[x & 3], sc[r]);
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < MG; r++) { sc[r] = row_group_sum<16>(sc[r]); if ((lane & 15) == r && r < nh && i < n) s_s[r][i] = sc[r]; }
+  }
+  __syncthreads();
+  if (wv < nh) {
+    const int h = h0 + wv;
+    const float slope2 = a.dist_bias ? distance_slope(h, ap.heads) * LOG2E : 0.f;
+    float s[STEP_MAX_KEYS / 64], mx = a.has_sink ? a.sink * LOG2E : -INFINITY, l = 0.f;
+#pragma unroll
+    for (int u = 0; u < STEP_MAX_KEYS / 64; u++) {
+      const int i = lane + 64 * u;
+      float v = i < n ? s_s[wv][i] : -INFINITY;
+      if (capped && i < n) v = a.softcap * tanhf(v / a.softcap) * LOG2E;
+      s[u] = i < n ? fmaf(-slope2, (float)(n - 1 - i), v) : -INFINITY;
+      mx = fmaxf(mx, s[u]);
+    }
+    mx = group_max<64>(mx);
+    const bool dead = mx == -INFINITY;
+#pragma unroll
+    for (int u = 0; u < STEP_MAX_KEYS / 64; u++) { const float p = dead ? 0.f : __builtin_amdgcn_exp2f(s[u] - mx); l += p; if (lane + 64 * u < n) s_s[wv][lane + 64 * u] = p; }
+    l = wave_sum(l);
+    if (a.has_sink) l += __builtin_amdgcn_exp2f(a.sink * LOG2E - mx);
+    if (lane == 0) s_l[wv] = l;
+  }
+  __syncthreads();
+  // values
+  float acc[MG][2];
+#pragma unroll
+  for (int r = 0; r < MG; r++) acc[r][0] = acc[r][1] = 0.f;
+#pragma unroll
+  for (int u = 0; u < KW; u++) {
+    if (16 * u >= n) break;
+    const int i = wv + 16 * u;
+    if (i >= n) break;                                             // (wave-uniform)
+    const bool own = fresh_key && i == n - 1;
+    const float v0 = own ? s_vn[min(lane, vdim - 1)] : vr[u][0], v1 = own ? s_vn[min(lane + 64, vdim - 1)] : vr[u][1];
+#pragma unroll
+    for (int r = 0; r < MG; r++) { const float p = s_s[min(r, nh - 1)][i]; acc[r][0] = fmaf(p, v0, acc[r][0]); acc[r][1] = fmaf(p, v1, acc[r][1]); }
+  }
+#pragma unroll
+  for (int r = 0; r < MG; r++)
+#pragma unroll
+    for (int c = 0; c < 2; c++) if (lane + 64 * c < STEP_MAX_VDIM) s_acc[wv][r][lane + 64 * c] = acc[r][c];
+  __syncthreads();
+  const int r = tid >> 7, c = tid & 127;                           // (STEP_MAX_VDIM columns a head)
+  if (r < nh && c < vdim) {
+    const size_t hc = (size_t)(h0 + r) * vdim + c;
+    float t[16];
+#pragma unroll
+    for (int w = 0; w < 16; w++) t[w] = s_acc[w][r][c];
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1)
+#pragma unroll
+      for (int w = 0; w < o; w++) t[w] += t[w + o];
+    float v = s_l[r] > 0.f ? t[0] / s_l[r] : 0.f;
+    if (a.gate) v = v / (1.0f + expf(-a.gate[(size_t)e * a.ldg + (a.gate_per_head ? (size_t)(h0 + r) : hc)]));
+    a.out[(size_t)e * a.ldo + hc] = v * a.out_scale;
+  }
+}
+template <int DT>
+__global__ __launch_bounds__(1024) void gqa_group_step_kernel(StepMeta m, GqaStepArgs a) { gqa_group_step_body<DT>(m, a, blockIdx.x, blockIdx.y); }
+
 // both halves of a parallel mixer (attention beside a delta rule) in one launch: grid (entries, heads of the one + heads of the other)
 template <int DT, int DPER>
 __global__ __launch_bounds__(STEP_THREADS) void parallel_step_kernel(StepMeta m, GqaStepArgs a, RecStepArgs r, const int log_cp) {

@@ -703,7 +703,13 @@ int run_gqa_core(tgx_ctx* c, const tgx::StepMeta& m, const GqaSpec& sp_, int T, 
   GqaSpec sp = sp_;
   tgx::GqaStepArgs sa{};
   if (gqa_step(sm, sp, max_keys, max_count, sa)) {
-    TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::gqa_step_kernel<DT>, dim3(S, sp.heads), dim3(512), 0, c->stream, m, sa))
+    const int group = sp.heads / sp.kv_heads;
+    if (group > 1 && (long long)S * sp.heads > c->num_cus) {      // (both sides' times: gqa_group_step_body)
+      const dim3 grid(S, sp.kv_heads * ((group + tgx::STEP_GROUP - 1) / tgx::STEP_GROUP));
+      TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::gqa_group_step_kernel<DT>, grid, dim3(1024), 0, c->stream, m, sa))
+    } else {
+      TGX_DT_SWITCH(c->dt, hipLaunchKernelGGL(tgx::gqa_step_kernel<DT>, dim3(S, sp.heads), dim3(512), 0, c->stream, m, sa))
+    }
     return TGX_OK;
   }
   if (sp.maps == 2) { sp.out = sp_.map_out; sp.ldo = (long long)sp.heads * sp.vdim; }
